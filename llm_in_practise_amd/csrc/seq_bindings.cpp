@@ -93,6 +93,12 @@ void seq_delta_scan(int, const void*, int, const void*, int, const void*, int, c
 void seq_talk_attention(int, const void*, int, const void*, const void*, float*, float*, float*, const float*,
                         const void*, int, void*, int, int, int, int, int, int, float, const int*, const int*, int,
                         SeqDesc, hipStream_t);
+size_t seq_chunk_floats(int, const void*, int, const void*, int, const void*, int, int, int, int, int, int);
+void seq_chunk_ssd(const void*, int, const void*, int, const void*, int, const void*, int, const float*, const float*,
+                   const float*, float*, float*, float*, int, int, int, int, SeqDesc, hipStream_t);
+void seq_chunk_mlstm(const void*, int, const void*, int, const void*, int, const float*, const float*, const float*,
+                     const float*, float, float, float*, float*, float*, float*, float*, float*, float*, int, int, int, SeqDesc,
+                     hipStream_t);
 int seq_scan_max_dk();
 int seq_conv_max_head();
 int seq_conv_max_taps();
@@ -332,6 +338,15 @@ std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H, dv}, S.options());
   auto den = at::empty({T, H}, S.options()), efl = at::empty({T, H}, S.options());
+  if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), (int)T, d.B, (int)H,
+                                        (int)dk, (int)dv)) {
+    auto ws = at::empty({(int64_t)n}, S.options());
+    seq_chunk_mlstm(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
+                    fpre.data_ptr<float>(), ib.data_ptr<float>(), fb.data_ptr<float>(), (float)cap, (float)qscale,
+                    S.data_ptr<float>(), N.data_ptr<float>(), M.data_ptr<float>(), out.data_ptr<float>(), den.data_ptr<float>(),
+                    efl.data_ptr<float>(), ws.data_ptr<float>(), (int)H, (int)dk, (int)dv, d, stream());
+    return {out, den, efl};
+  }
   seq_mlstm_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
                  fpre.data_ptr<float>(), ib.data_ptr<float>(), fb.data_ptr<float>(), (float)cap, (float)qscale,
                  S.data_ptr<float>(), N.data_ptr<float>(), M.data_ptr<float>(), out.data_ptr<float>(),
@@ -426,6 +441,14 @@ Tensor ssd_scan(Tensor q, Tensor k, Tensor v, Tensor dtraw, Tensor dt_bias, Tens
   check_state(S, H, dv, dk);
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H * dv}, S.options());
+  if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), (int)T, d.B, (int)H,
+                                        (int)dk, (int)dv)) {
+    auto ws = at::empty({(int64_t)n}, S.options());
+    seq_chunk_ssd(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), dtraw.data_ptr(), ld(dtraw),
+                  dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), dskip.data_ptr<float>(), S.data_ptr<float>(),
+                  out.data_ptr<float>(), ws.data_ptr<float>(), (int)H, (int)G, (int)dk, (int)dv, d, stream());
+    return out;
+  }
   seq_ssd_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), dtraw.data_ptr(), ld(dtraw),
                dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), dskip.data_ptr<float>(), S.data_ptr<float>(),
                out.data_ptr<float>(), (int)H, (int)G, (int)dk, (int)dv, d, stream());

@@ -1,0 +1,108 @@
+"""The chunked scans (csrc/kernels/seq/seq_chunk.hip) against the token-by-token reference ops, at the sizes where a chunk, a
+tile or the choice between the two forms ends."""
+import pytest
+import torch
+
+from llm_in_practise_amd.models.common import SeqBatch, SeqStateCache
+from llm_in_practise_amd.ops import recurrent as R
+
+# float sums of up to a few hundred products of order 1, and of decayed states: a few hundred roundings of 2^-24 each, taken
+# from both sides and relative to the outputs' norm
+TOL = 1e-5
+
+
+def _batch(spec, lens, starts, device, live=None):
+    cache = SeqStateCache([spec], len(lens), max(n + s for n, s in zip(lens, starts)) + 1, torch.bfloat16, device)
+    sb = SeqBatch.packed(cache, list(range(len(lens)))[::-1], lens, starts)
+    if live is not None:
+        sb.live = torch.tensor(live, dtype=torch.int32, device=device)
+    return cache.layers[0], sb
+
+
+def _close(got, want, names):
+    for name, a, b in zip(names, got, want):
+        a, b = a.detach().cpu().double(), b.detach().cpu().double()
+        assert torch.isfinite(a).all(), name
+        assert (a - b).norm() <= TOL * b.norm() + 1e-12, (name, ((a - b).norm() / b.norm()).item())
+
+
+LENS = [([64], [0]), ([128], [0]), ([127, 129, 1, 128, 65], [0, 0, 0, 3, 0]), ([300, 20, 257], [7, 0, 512]), ([63], [5])]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,starts", LENS)
+@pytest.mark.parametrize("H,G,dk,dv", [(4, 2, 128, 64), (2, 1, 32, 36), (3, 3, 96, 100), (2, 2, 64, 4), (2, 1, 48, 64)])
+def test_ssd_chunks(lens, starts, H, G, dk, dv):
+    g = torch.Generator().manual_seed(dk + dv + len(lens))
+    T = sum(lens)
+    xbc = torch.randn(T, H * dv + 2 * G * dk, generator=g).bfloat16()
+    dt, dtb = torch.randn(T, H, generator=g).bfloat16(), torch.randn(H, generator=g) - 2
+    a_log, skip = torch.randn(H, generator=g), torch.randn(H, generator=g)
+    a_log[-1] = 60.0 if T % 2 else 2.0                  # a head that forgets everything at once
+    S0 = 0.3 * torch.randn(len(lens), H, dv, dk, generator=g)
+    res = []
+    for dev in ("cpu", "cuda"):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, starts, dev)
+        st["S"].copy_(S0)
+        x, p = xbc.to(dev), [t.to(dev) for t in (dt, dtb, a_log, skip)]
+        y = R.ssd_scan(x[:, H * dv + G * dk:], x[:, H * dv:H * dv + G * dk], x[:, :H * dv], *p, st["S"], H, G, sb)
+        res.append((y.view(T, H, dv), st["S"]))
+    _close(res[1], res[0], ("y", "state"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,starts", LENS)
+@pytest.mark.parametrize("H,dk,dv", [(2, 128, 192), (2, 64, 96), (3, 32, 36), (1, 96, 4), (2, 160, 32)])
+def test_mlstm_chunks(lens, starts, H, dk, dv):
+    g = torch.Generator().manual_seed(dk + dv + len(lens))
+    T = sum(lens)
+    P = torch.randn(T, 2 * H * dk + H * dv, generator=g).bfloat16()
+    i, f = 4 * torch.randn(T, H, generator=g), 3 * torch.randn(T, H, generator=g)
+    i[::50] += 20.0                                     # the running maximum jumps
+    ib, fb = torch.randn(H, generator=g), torch.randn(H, generator=g) + 3
+    old = [torch.randn(len(lens), H, dv, dk, generator=g), torch.randn(len(lens), H, dk, generator=g),
+           torch.rand(len(lens), H, generator=g)]
+    st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lens, starts, "cuda")
+    for t, o in zip(st.values(), old):
+        t.copy_(o)
+    p, gt = P.cuda(), [t.cuda() for t in (i, f, ib, fb)]
+    got = R.mlstm_scan(p[:, :H * dk], p[:, H * dk:2 * H * dk], p[:, 2 * H * dk:], *gt, 15.0, dk ** -0.5, st["S"], st["N"],
+                       st["M"], H, sb)
+    # numerators, normaliser and floor of the reference's recurrence in 64 bits (their quotient is ill-conditioned where the
+    # normaliser crosses 0)
+    q, k, v = (x.double().view(T, H, -1) for x in P.split([H * dk, H * dk, H * dv], 1))
+    ig = 15.0 * torch.tanh((i + ib).double() / 15.0)
+    fg = torch.nn.functional.logsigmoid(15.0 * torch.tanh((f + fb).double() / 15.0))
+    o, den, floor = torch.empty(T, H, dv).double(), torch.empty(T, H).double(), torch.empty(T, H).double()
+    S, N, M = (x.double().clone() for x in old)
+    off, slots, pos0 = sb.host()
+    for b, slot in enumerate(slots):
+        if pos0[b] == 0:
+            S[slot], N[slot], M[slot] = 0, 0, 0
+        for t in range(off[b], off[b + 1]):
+            m = torch.maximum(fg[t] + M[slot], ig[t])
+            a, c = torch.exp(fg[t] + M[slot] - m), torch.exp(ig[t] - m)
+            M[slot] = m
+            S[slot] = a[:, None, None] * S[slot] + c[:, None, None] * v[t][:, :, None] * k[t][:, None, :]
+            N[slot] = a[:, None] * N[slot] + c[:, None] * k[t]
+            o[t], den[t] = (S[slot] * q[t][:, None]).sum(-1) * dk ** -0.5, (N[slot] * q[t]).sum(-1) * dk ** -0.5
+            floor[t] = torch.exp(-m)
+    _close((*got, *st.values()), (o, den, floor, S, N, M), ("o", "den", "floor", "S", "N", "M"))
+
+
+@pytest.mark.gpu
+def test_idle_sequences_keep_their_state():
+    lens, H, dk, dv = [130, 200, 70], 2, 64, 32
+    g = torch.Generator().manual_seed(0)
+    xbc = torch.randn(sum(lens), H * dv + 2 * dk, generator=g).bfloat16().cuda()
+    dt, dtb, a_log, skip = (torch.randn(*s, generator=g).cuda() for s in ((sum(lens), H), (H,), (H,), (H,)))
+    out = []
+    for live in (None, [1, 0, 1]):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, [0, 0, 0], "cuda", live)
+        st["S"].fill_(7.0)
+        y = R.ssd_scan(xbc[:, H * dv + dk:], xbc[:, H * dv:H * dv + dk], xbc[:, :H * dv], dt.bfloat16(), dtb, a_log, skip, st["S"],
+                       H, 1, sb)
+        out.append((y, st["S"]))
+    assert (out[1][1][1] == 7.0).all()                  # slot 1 belongs to sequence 1
+    assert torch.equal(out[0][1][[0, 2]], out[1][1][[0, 2]])
+    assert torch.equal(out[0][0][:130], out[1][0][:130]) and torch.equal(out[0][0][330:], out[1][0][330:])
