@@ -1,0 +1,341 @@
+// Prompts through the recurrences whose decay differs per key channel - the gated delta rule and gated linear attention - in
+// blocks of 16 tokens.  With G_t the product of the decays from the block's first token up to t (per key channel) and S the
+// state in front of the block,
+//   u_t = beta_t (v_t - (k_t G_t)^T S - sum_{j<t} A_tj u_j),   A_tj = sum_d k_td k_jd G_td / G_jd     (linear attention: u = v)
+//   o_t = (q_t G_t)^T S + sum_{j<=t} B_tj u_j,                 B_tj = sum_d q_td k_jd G_td / G_jd
+//   S  <- G_16 S + sum_j (k_j G_16 / G_j) u_j^T.
+// A first kernel forms, for all blocks at once, everything that does not read the state: the scaled rows, B, and
+// T = (I + beta A)^-1 beta, with which u = T (v - (k G)^T S).  The ratios G_t / G_j are running products of the decays
+// themselves, never quotients, so a decay of 0 (or any other value) is what it is in the token-by-token scan.  The second
+// kernel walks a sequence's blocks with the state in registers; all its products are float on the float matrix units
+// (v_mfma_f32_16x16x4_f32), whose result layout is also its operand layout: the state, u and the outputs never move
+// between lanes.
+//
+// Measured, token by token -> blocks: three sequences of 1500, 700 and 97 tokens, 8 delta heads of 128 x 128: 576 -> 110 us (25
+// for the first kernel, 88 for the walk); eight sequences of 512 tokens, 16 linear-attention heads of 64 x 128: 119 -> 69 us.
+// Error against 64 bits as before (2e-7).  Ten inputs a lane two or three blocks ahead gave 2.0 -> 0.94 us a block of the longest
+// sequence.
+#include "seq_common.h"
+
+using namespace lipa;
+
+namespace {
+
+constexpr int BT = 16;      // tokens of a block
+
+// what the first kernel leaves per (block, head): [k G | q G | k G_16 / G] in operand order, G_16, T, B
+__host__ __device__ constexpr int cell_floats(int dk) { return 3 * BT * dk + dk + 2 * BT * BT; }
+
+__device__ __forceinline__ float row16_sum(float v) {       // over the 16 lanes of a row, in all of them
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));    // quad_perm [1, 0, 3, 2]
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));    // quad_perm [2, 3, 0, 1]
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true));   // row_half_mirror
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xF, 0xF, true));   // row_mirror
+  return v;
+}
+
+__device__ __forceinline__ f32x4 row4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ f32x4 row4(const bf16* p) {
+  const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
+  return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+}
+
+struct DecayArgs {
+  const float* g;           // [T, H * dk]: decays (delta rule) or their pre-activations (linear attention)
+  const float* bias;        // linear attention: [H * dk]
+  const float* beta;        // delta rule: [T, H] pre-activations
+  float inv_tau, qscale;
+};
+
+// 256 threads: token j = tid / 16, and the four channels 4 x .. of every 64 (x = tid % 16).  A thread carries its token's key
+// times the decays of the tokens behind it; at token s the 16 threads of a row sum k_s and q_s against it, and lane s keeps
+// the sums.
+template <typename T, int NS, bool DELTA>
+__global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk,
+                                                    DecayArgs a, float* __restrict__ ws, int H, int G, SeqDesc d) {
+  constexpr int DK = 64 * NS;
+  __shared__ __attribute__((aligned(16))) float sg[BT * DK];
+  __shared__ __attribute__((aligned(16))) float sk[BT * DK];
+  __shared__ __attribute__((aligned(16))) float sq[BT * DK];
+  __shared__ float sA[BT * BT];
+  __shared__ float sb[BT];
+  int lo = 0, hi = d.B - 1;
+  const int slot = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x;
+  while (lo < hi) {                              // sequence s owns the slots from seq_off[s] / 16 + s on
+    const int mid = (lo + hi + 1) >> 1;
+    if (d.seq_off[mid] / BT + mid <= slot)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  const int o0 = d.seq_off[lo], t0 = o0 + (slot - (o0 / BT + lo)) * BT, n = min(BT, d.seq_off[lo + 1] - t0);
+  if (t0 < o0 || n <= 0 || (d.live && !d.live[lo])) return;
+  const int j = tid >> 4, x = tid & 15, kh = hd / (H / G);
+  const bool on = j < n;
+  const size_t t = t0 + (on ? j : 0);
+  f32x4 kj[NS], qj[NS], W[NS], Gm[NS];
+#pragma unroll
+  for (int c = 0; c < NS; ++c) {
+    const int D = 64 * c + 4 * x;
+    f32x4 g = row4(a.g + (t * H + hd) * DK + D);
+    kj[c] = row4(k + t * ldk + kh * DK + D);
+    qj[c] = row4(q + t * ldq + kh * DK + D);
+    if (!DELTA) {
+      const f32x4 z = g + row4(a.bias + hd * DK + D);        // ln sigmoid(z) = min(z, 0) - ln(1 + e^-|z|)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        g[e] = __builtin_amdgcn_exp2f((fminf(z[e], 0.f) - log1p_exp_neg(fabsf(z[e]))) * (a.inv_tau * 1.4426950408889634f));
+      qj[c] *= a.qscale;
+    }
+    if (!on) {                                               // past the end: tokens that change nothing
+      kj[c] = qj[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      g = f32x4{1.f, 1.f, 1.f, 1.f};
+    }
+    *reinterpret_cast<f32x4*>(sg + j * DK + D) = g;
+    *reinterpret_cast<f32x4*>(sk + j * DK + D) = kj[c];
+    *reinterpret_cast<f32x4*>(sq + j * DK + D) = qj[c];
+    W[c] = kj[c];
+    Gm[c] = f32x4{1.f, 1.f, 1.f, 1.f};
+  }
+  if (DELTA && tid < BT) sb[tid] = tid < n ? sigmoidf_(a.beta[(size_t)(t0 + tid) * H + hd]) : 0.f;
+  __syncthreads();
+  float ra = 0.f, rb = 0.f;                                  // A and B of (token x, token j)
+#pragma unroll
+  for (int s = 0; s < BT; ++s) {
+    float pa = 0.f, pb = 0.f;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      const int D = s * DK + 64 * c + 4 * x;
+      const f32x4 g = row4(sg + D);
+      if (s <= j)
+        Gm[c] *= g;
+      else
+        W[c] *= g;
+      const f32x4 qs = row4(sq + D);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pb += qs[e] * W[c][e];
+      if (DELTA) {
+        const f32x4 ks = row4(sk + D);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pa += ks[e] * W[c][e];
+      }
+    }
+    pb = row16_sum(pb);
+    if (DELTA) pa = row16_sum(pa);
+    if (x == s) {
+      rb = pb;
+      ra = pa;
+    }
+  }
+  float* cell = ws + ((size_t)slot * H + hd) * cell_floats(DK);
+  float *ck = cell, *cq = cell + BT * DK, *cp = cell + 2 * BT * DK, *cg = cell + 3 * BT * DK, *cT = cg + DK, *cB = cT + BT * BT;
+#pragma unroll
+  for (int c = 0; c < NS; ++c) {
+    // operand order of the 16x16x4 products: [tile of 16 channels][4 channels][token][channel of the 4] for the rows, and
+    // [tile][4 tokens][channel][token of the 4] for the keys that are written to the state
+    const int tile = 4 * c + (x >> 2), base = (tile * 64 + (x & 3) * 16 + j) * 4;
+    if (DELTA) *reinterpret_cast<f32x4*>(ck + base) = kj[c] * Gm[c];
+    *reinterpret_cast<f32x4*>(cq + base) = qj[c] * Gm[c];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) cp[(tile * 64 + (j >> 2) * 16 + 4 * (x & 3) + e) * 4 + (j & 3)] = W[c][e];
+    if (j == BT - 1) *reinterpret_cast<f32x4*>(cg + 64 * c + 4 * x) = Gm[c];
+  }
+  cB[x * BT + j] = x >= j ? rb : 0.f;
+  if (DELTA) {
+    sA[x * BT + j] = ra;
+    __syncthreads();
+    if (tid < BT) {                                          // column tid of (I + beta A)^-1 beta, row after row
+      float r[BT];
+#pragma unroll
+      for (int s = 0; s < BT; ++s) {
+        float acc = s == tid ? 1.f : 0.f;
+#pragma unroll
+        for (int i = 0; i < s; ++i) acc -= sA[s * BT + i] * r[i];
+        r[s] = sb[s] * acc;
+        cT[s * BT + tid] = r[s];
+      }
+    }
+  }
+}
+
+// A block owns 16 value columns of one (sequence, head); its four waves own a quarter of the key rows each, with the state in
+// registers in operand layout.  Per 16 tokens a wave runs its share of the key products, the four shares meet in LDS (two
+// buffers, one barrier), every wave finishes u for itself and updates its rows; the query products run under the LDS round trip
+// and the waves take turns at summing them into outputs, one block of tokens later.  Bound by the chain of a block of tokens
+// (key products, LDS round trip, u, update); what it reads is on its way two or three blocks ahead, since it comes from memory
+// or another die's cache.
+template <typename T, int NS, bool DELTA>
+__global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float* __restrict__ ws, const T* __restrict__ v, int ldv,
+                                                                    float* __restrict__ S, float* __restrict__ out, int H, int dv,
+                                                                    SeqDesc d) {
+  constexpr int DK = 64 * NS, CELL = cell_floats(DK), RING = NS == 1 ? 4 : 3;
+  __shared__ __attribute__((aligned(16))) f32x4 red[2][4][2][64];
+  const int s = blockIdx.x / H, hd = blockIdx.x % H, tid = threadIdx.x;
+  if (d.live && !d.live[s]) return;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, col = blockIdx.y * 16 + (lane & 15);
+  const bool colok = col < dv;
+  const int t0 = d.seq_off[s], t1 = d.seq_off[s + 1], steps = (t1 - t0 + BT - 1) / BT;
+  if (steps <= 0) return;
+  const float* cell = ws + ((size_t)(t0 / BT + s) * H + hd) * CELL;
+  const size_t step = (size_t)H * CELL;
+  const T* vp = v + (size_t)t0 * ldv + (size_t)hd * dv;
+  const unsigned vcol = colok ? col : 0, m = 3 * BT * DK + DK + (lane & 15) * BT + 4 * g;
+  float* Sp = S + (((size_t)d.slots[s] * H + hd) * dv + (colok ? col : 0)) * DK + 16 * NS * w + 4 * g;
+  f32x4 St[NS];
+  const bool old = d.pos0[s] > 0 && colok;
+#pragma unroll
+  for (int c = 0; c < NS; ++c) St[c] = old ? row4(Sp + 16 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
+  struct In {
+    f32x4 k[NS], q[NS], p[NS], g[NS], tm, bm;
+    T v[4];
+  } in[RING];
+  auto load = [&](int i, In& x) {
+    const float* c0 = cell + (size_t)i * step;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      const unsigned o = ((NS * w + c) * 64 + lane) * 4;
+      if (DELTA) x.k[c] = row4(c0 + o);
+      x.q[c] = row4(c0 + BT * DK + o);
+      x.p[c] = row4(c0 + 2 * BT * DK + o);
+      x.g[c] = row4(c0 + 3 * BT * DK + 16 * (NS * w + c) + (unsigned)(4 * g));
+    }
+    if (DELTA) x.tm = row4(c0 + m);
+    x.bm = row4(c0 + m + BT * BT);
+    // (values are not looked at before their turn: that would wait for every load issued before them)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      x.v[e] = (vp + (size_t)i * BT * ldv)[(unsigned)min(4 * g + e, t1 - t0 - i * BT - 1) * (unsigned)ldv + vcol];
+  };
+  f32x4 uo, bo;                                   // u and B of the block of tokens before
+  auto outputs = [&](int i) {
+    const auto& r = red[i & 1];
+    f32x4 o = (r[0][1][lane] + r[1][1][lane]) + (r[2][1][lane] + r[3][1][lane]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(bo[e], uo[e], o, 0, 0, 0);
+    // (a store that has no place goes past the end of its window and is dropped: with a branch around it the compiler waits for
+    // every load in flight)
+    const int b0 = t0 + i * BT;
+    const auto win = __builtin_amdgcn_make_buffer_rsrc(out + (size_t)b0 * H * dv, 0, min(BT, t1 - b0) * H * dv * 4, 0x00020000);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[e]), win, colok ? (((4 * g + e) * H + hd) * dv + col) * 4 : -4, 0, 0);
+  };
+  auto run = [&](int i, const In& x) {
+    auto& r = red[i & 1];
+    if (DELTA) {                                  // two chains of products: one alone waits for its own results
+      f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NS; ++c) {
+        x0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[c][0], St[c][0], x0, 0, 0, 0);
+        x1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[c][1], St[c][1], x1, 0, 0, 0);
+        x0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[c][2], St[c][2], x0, 0, 0, 0);
+        x1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[c][3], St[c][3], x1, 0, 0, 0);
+      }
+      r[w][0][lane] = x0 + x1;
+    }
+    __syncthreads();
+    f32x4 xq = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NS; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xq = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[c][e], St[c][e], xq, 0, 0, 0);
+    f32x4 u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) u[e] = t0 + i * BT + 4 * g + e < t1 ? (float)x.v[e] : 0.f;
+    if (DELTA) {
+      const f32x4 e = u - ((r[0][0][lane] + r[1][0][lane]) + (r[2][0][lane] + r[3][0][lane]));
+      u = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.tm[j], e[j], u, 0, 0, 0);
+    }
+    r[w][1][lane] = xq;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      St[c] *= x.g[c];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) St[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[c][e], u[e], St[c], 0, 0, 0);
+    }
+    if (w == (i & 3) && i > 0) outputs(i - 1);    // its query products were written in front of this barrier
+    uo = u;
+    bo = x.bm;
+  };
+#pragma unroll
+  for (int x = 0; x < RING - 1; ++x) load(min(x, steps - 1), in[x]);
+  int i = 0;
+  for (; i + RING <= steps; i += RING) {
+#pragma unroll
+    for (int x = 0; x < RING; ++x) {
+      load(min(i + x + RING - 1, steps - 1), in[(x + RING - 1) % RING]);
+      run(i + x, in[x]);
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < RING - 1; ++x)
+    if (i + x < steps) run(i + x, in[x]);
+  __syncthreads();                                // the last query products stand
+  if (w == (steps & 3)) outputs(steps - 1);
+  if (colok)
+#pragma unroll
+    for (int c = 0; c < NS; ++c) *reinterpret_cast<f32x4*>(Sp + 16 * c) = St[c];
+}
+
+size_t slots_of(int T_, int B) { return (size_t)T_ / BT + B; }
+
+template <typename T, int NS, bool DELTA>
+void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const DecayArgs& a, float* S, float* out,
+            float* ws, int H, int G, int dv, const SeqDesc& d, hipStream_t st) {
+  hipLaunchKernelGGL((k_block_prep<T, NS, DELTA>), dim3((unsigned)slots_of(d.Ttot, d.B), H), dim3(256), 0, st, (const T*)q, ldq,
+                     (const T*)k, ldk, a, ws, H, G, d);
+  hipLaunchKernelGGL((k_block_scan<T, NS, DELTA>), dim3(d.B * H, (dv + 15) / 16), dim3(256), 0, st, ws, (const T*)v, ldv, S, out,
+                     H, dv, d);
+  LIPA_CHECK_LAUNCH();
+}
+
+template <bool DELTA>
+void dispatch(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const DecayArgs& a, float* S,
+              float* out, float* ws, int H, int G, int dk, int dv, const SeqDesc& d, hipStream_t st) {
+  SEQ_DISPATCH_T(code, {
+    switch (dk / 64) {
+      case 1: launch<T, 1, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dv, d, st); break;
+      case 2: launch<T, 2, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dv, d, st); break;
+      case 3: launch<T, 3, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dv, d, st); break;
+      default: launch<T, 4, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dv, d, st); break;
+    }
+  });
+}
+
+}  // namespace
+
+// Floats of workspace of the blocked form, or 0 where the token-by-token scan is the one to run: key sizes that are no multiple
+// of 64 or above 256, rows that vector loads of four channels cannot take, and steps of few tokens a sequence.
+size_t seq_block_floats(int code, bool delta, const void* q, int ldq, const void* k, int ldk, const void* g, const void* bias,
+                        const void* S, int T_, int B, int H, int dk, int dv) {
+  const int bytes = code == 0 ? 8 : 16;
+  const auto fits = [](const void* p, int ld, int b) { return ld % 4 == 0 && ((uintptr_t)p & (b - 1)) == 0; };
+  if (dk % 64 != 0 || dk > 256 || !fits(q, ldq, bytes) || !fits(k, ldk, bytes) || !fits(g, 4, 16) || !fits(bias, 4, 16) ||
+      !fits(S, 4, 16) || B == 0)
+    return 0;
+  // Two launches and a block's chain of 0.5 to 0.9 us per 16 tokens, against 0.23 (linear attention) and 0.39 us a token; with
+  // many (sequence, head, 16 columns) to run at once both are bound by issue, and linear attention's token form is then the
+  // cheaper one.  us, tokens -> blocks, heads of 128 x 128 (delta) and 64 x 128: 64 delta heads (512 blocks) at 32 tokens 19 -> 16,
+  // at 512 201 -> 83; 384 heads at 48 tokens 69 -> 73, at 64 88 -> 85, at 256 318 -> 290.  Linear attention: 64 heads at 32
+  // tokens 11 -> 12, at 48 15 -> 12, at 512 119 -> 44; 128 heads at 48 16 -> 17, at 64 20 -> 19; 384 heads at 256 100 -> 120.
+  const long blocks = (long)B * H * ((dv + 15) / 16);
+  const long least = delta ? (blocks <= 1024 ? 32 : 64) : blocks <= 512 ? 40 : blocks <= 1536 ? 64 : 1L << 40;
+  if (T_ < least * B) return 0;
+  return slots_of(T_, B) * H * cell_floats(dk);
+}
+
+void seq_block_delta(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g,
+                     const float* bpre, float* S, float* out, float* ws, int H, int G, int dk, int dv, SeqDesc d,
+                     hipStream_t st) {
+  const DecayArgs a = {g, nullptr, bpre, 1.f, 1.f};
+  dispatch<true>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dk, dv, d, st);
+}
+
+void seq_block_gla(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* z,
+                   const float* zb, float inv_tau, float qscale, float* S, float* out, float* ws, int H, int dk, int dv,
+                   SeqDesc d, hipStream_t st) {
+  const DecayArgs a = {z, zb, nullptr, inv_tau, qscale};
+  dispatch<false>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, H, H, dk, dv, d, st);
+}

@@ -27,6 +27,21 @@ __device__ __forceinline__ float gelu_tanhf_(float v) {
 }
 __device__ __forceinline__ float logsigmoidf_(float x) { return fminf(x, 0.f) - log1pf(expf(-fabsf(x))); }
 
+// ln(1 + e^-a) for a >= 0 as 2 atanh(e / (2 + e)), e = e^-a: the argument stays below 1/3, so eight terms of the odd series
+// reach float accuracy without a table or a branch (the staging of a chunk evaluates one per element).
+__device__ __forceinline__ float log1p_exp_neg(float a) {
+  const float e = __builtin_amdgcn_exp2f(a * -1.4426950408889634f), s = e * __builtin_amdgcn_rcpf(2.f + e), q = s * s;
+  float p = 1.f / 17.f;
+  p = p * q + 1.f / 15.f;
+  p = p * q + 1.f / 13.f;
+  p = p * q + 1.f / 11.f;
+  p = p * q + 1.f / 9.f;
+  p = p * q + 1.f / 7.f;
+  p = p * q + 1.f / 5.f;
+  p = p * q + 1.f / 3.f;
+  return 2.f * s * (p * q + 1.f);
+}
+
 // Entry c of a vector whose first `dims` entries are rotated by pos * inv_freq[pair]: neighbours (2i, 2i+1) form pair
 // i, or with `half` entries (i, i + dims/2) do; the rest pass unchanged.  Sine and cosine are multiplied by mag.
 // The pair (u, v) becomes (u cos - v sin, v cos + u sin); the angle is a float product.

@@ -12,20 +12,6 @@ namespace {
 
 constexpr int CT = 16;      // tokens staged per chunk
 
-// ln(1 + e^-a) for a >= 0 as 2 atanh(e / (2 + e)), e = e^-a: the argument stays below 1/3, so eight terms of the odd series
-// reach float accuracy without a table or a branch (the staging of a chunk evaluates one per element).
-__device__ __forceinline__ float log1p_exp_neg(float a) {
-  const float e = __builtin_amdgcn_exp2f(a * -1.4426950408889634f), s = e * __builtin_amdgcn_rcpf(2.f + e), q = s * s;
-  float p = 1.f / 17.f;
-  p = p * q + 1.f / 15.f;
-  p = p * q + 1.f / 13.f;
-  p = p * q + 1.f / 11.f;
-  p = p * q + 1.f / 9.f;
-  p = p * q + 1.f / 7.f;
-  p = p * q + 1.f / 5.f;
-  p = p * q + 1.f / 3.f;
-  return 2.f * s * (p * q + 1.f);
-}
 __device__ __forceinline__ float softplus_fast(float x) { return fmaxf(x, 0.f) + log1p_exp_neg(fabsf(x)); }
 __device__ __forceinline__ float silu_fast(float z) {
   return z * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(z * -1.4426950408889634f));

@@ -99,6 +99,12 @@ void seq_chunk_ssd(const void*, int, const void*, int, const void*, int, const v
 void seq_chunk_mlstm(const void*, int, const void*, int, const void*, int, const float*, const float*, const float*,
                      const float*, float, float, float*, float*, float*, float*, float*, float*, float*, int, int, int, SeqDesc,
                      hipStream_t);
+size_t seq_block_floats(int, bool, const void*, int, const void*, int, const void*, const void*, const void*, int, int, int, int,
+                        int);
+void seq_block_delta(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float*, float*, float*,
+                     int, int, int, int, SeqDesc, hipStream_t);
+void seq_block_gla(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float, float*,
+                   float*, float*, int, int, int, SeqDesc, hipStream_t);
 int seq_scan_max_dk();
 int seq_conv_max_head();
 int seq_conv_max_taps();
@@ -371,6 +377,14 @@ Tensor delta_scan(Tensor q, Tensor k, Tensor v, Tensor g, Tensor bpre, Tensor S,
   check_state(S, H, dv, dk);
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H, dv}, S.options());
+  if (const size_t n = seq_block_floats(code, true, q.data_ptr(), ld(q), k.data_ptr(), ld(k), g.data_ptr(), nullptr,
+                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv)) {
+    auto ws = at::empty({(int64_t)n}, S.options());
+    seq_block_delta(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), g.data_ptr<float>(),
+                    bpre.data_ptr<float>(), S.data_ptr<float>(), out.data_ptr<float>(), ws.data_ptr<float>(), (int)H, (int)G,
+                    (int)dk, (int)dv, d, stream());
+    return out;
+  }
   seq_delta_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), g.data_ptr<float>(),
                  bpre.data_ptr<float>(), S.data_ptr<float>(), out.data_ptr<float>(), (int)H, (int)G, (int)dk, (int)dv, d,
                  stream());
@@ -1116,6 +1130,14 @@ Tensor gated_linear_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, 
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H, dv}, S.options());
   if (T == 0) return out;
+  if (const size_t n = seq_block_floats(code, false, q.data_ptr(), ld(q), k.data_ptr(), ld(k), z.data_ptr(), z_bias.data_ptr(),
+                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv)) {
+    auto ws = at::empty({(int64_t)n}, S.options());
+    seq_block_gla(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), z.data_ptr<float>(),
+                  z_bias.data_ptr<float>(), (float)(1.0 / tau), (float)q_scale, S.data_ptr<float>(), out.data_ptr<float>(),
+                  ws.data_ptr<float>(), (int)H, (int)dk, (int)dv, d, stream());
+    return out;
+  }
   seq_gla_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), z.data_ptr<float>(),
                z_bias.data_ptr<float>(), (float)(1.0 / tau), (float)q_scale, S.data_ptr<float>(), out.data_ptr<float>(), (int)H,
                (int)dk, (int)dv, d, stream());

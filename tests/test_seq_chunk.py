@@ -1,5 +1,5 @@
-"""The chunked scans (csrc/kernels/seq/seq_chunk.hip) against the token-by-token reference ops, at the sizes where a chunk, a
-tile or the choice between the two forms ends."""
+"""The chunked and blocked scans (csrc/kernels/seq/seq_chunk.hip, seq_block.hip) against the token-by-token reference ops, at the
+sizes where a chunk, a tile or the choice between two forms ends."""
 import pytest
 import torch
 
@@ -106,3 +106,54 @@ def test_idle_sequences_keep_their_state():
     assert (out[1][1][1] == 7.0).all()                  # slot 1 belongs to sequence 1
     assert torch.equal(out[0][1][[0, 2]], out[1][1][[0, 2]])
     assert torch.equal(out[0][0][:130], out[1][0][:130]) and torch.equal(out[0][0][330:], out[1][0][330:])
+
+
+BLOCK_LENS = [([32], [0]), ([31], [3]), ([48, 15, 1, 128, 65, 33], [0, 0, 9, 5, 0, 0]), ([100, 47], [512, 0])]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,starts", BLOCK_LENS)
+@pytest.mark.parametrize("H,G,dk,dv,dt", [(4, 2, 128, 64, torch.float32), (2, 1, 64, 20, torch.bfloat16),
+                                          (1, 1, 256, 16, torch.float32), (2, 2, 192, 33, torch.bfloat16),
+                                          (2, 1, 96, 32, torch.float32)])
+def test_delta_blocks(lens, starts, H, G, dk, dv, dt):
+    g = torch.Generator().manual_seed(dk + dv + len(lens))
+    T = sum(lens)
+    P = torch.randn(T, 2 * G * dk + H * dv, generator=g)
+    for j in (0, 1):
+        x = P[:, j * G * dk:(j + 1) * G * dk].view(T, G, dk)
+        x.copy_(torch.nn.functional.normalize(x, dim=-1))
+    P, decay, beta = P.to(dt), torch.rand(T, H * dk, generator=g) ** 0.2, 2 * torch.randn(T, H, generator=g)
+    decay[::7, ::3] = 0.0                               # channels that forget everything
+    S0 = torch.randn(len(lens), H, dv, dk, generator=g)
+    res = []
+    for dev in ("cpu", "cuda"):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, starts, dev)
+        st["S"].copy_(S0)
+        p = P.to(dev)
+        o = R.gated_delta_scan(p[:, :G * dk], p[:, G * dk:2 * G * dk], p[:, 2 * G * dk:], decay.to(dev), beta.to(dev), st["S"], H,
+                               G, sb)
+        res.append((o, st["S"]))
+    _close(res[1], res[0], ("o", "state"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,starts", BLOCK_LENS)
+@pytest.mark.parametrize("H,dk,dv,dt", [(4, 64, 128, torch.bfloat16), (2, 128, 20, torch.float32), (1, 256, 33, torch.bfloat16),
+                                        (2, 72, 32, torch.float32)])
+def test_gla_blocks(lens, starts, H, dk, dv, dt):
+    g = torch.Generator().manual_seed(dk + dv + len(lens))
+    T = sum(lens)
+    P = torch.randn(T, 2 * H * dk + H * dv, generator=g).to(dt)
+    z, zb = 3 * torch.randn(T, H * dk, generator=g), torch.randn(H * dk, generator=g)
+    z[::9, ::5] = -4000.0                               # channels that forget everything
+    S0 = torch.randn(len(lens), H, dv, dk, generator=g)
+    res = []
+    for dev in ("cpu", "cuda"):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, starts, dev)
+        st["S"].copy_(S0)
+        p = P.to(dev)
+        o = R.gated_linear_scan(p[:, :H * dk], p[:, H * dk:2 * H * dk], p[:, 2 * H * dk:], z.to(dev), zb.to(dev), 16.0,
+                                dk ** -0.5, st["S"], H, sb)
+        res.append((o, st["S"]))
+    _close(res[1], res[0], ("o", "state"))
