@@ -90,33 +90,64 @@ __device__ __forceinline__ void store_state(float* p, int i0, int len, const flo
 // NC = 256 / R * CH channels of one sequence.  dt and dt x of the chunk go through LDS, a thread keeps the x and z it
 // fetched for the read-out of the same (token, channel) pairs.  Two tokens per turn: their four read-outs are summed over
 // the lanes together, and the next pair's inputs are read while the current pair is computed.
+//
+// One prompt keeps C / NC blocks busy for as long as it has tokens (0.23 us each), so a step whose sequences do not fill the
+// chip is cut over time (k_selective_walk and the two cut modes): every segment of 32 or 64 tokens first runs from a zero state for
+// the state it leaves and the sum of its step sizes (its decay is e^{A sum dt}), a walk over a sequence's segments turns those
+// into the states in front of the segments, and every segment then runs from its own.  Two prompts of 2048 and 1337 tokens, 4096
+// channels of 16 states: 464 -> 125 us (49 for what segments leave, 15, 72: bound by one
+// quarter-rate exponential per channel, state and token).
 constexpr int CH = 2;
+enum { WHOLE, LEAVES, FROM };       // a sequence; a segment from zero (state and step sizes); a segment from the state before it
 
-template <typename T, int NS, int R>
+// segment slots: sequence s owns slots seq_off[s] / seg + s, .. (consecutive sequences never overlap)
+__device__ __forceinline__ int find_segment(const SeqDesc& d, int seg, int slot, int& first) {
+  int lo = 0, hi = d.B - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (d.seq_off[mid] / seg + mid <= slot)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  first = d.seq_off[lo] + (slot - (d.seq_off[lo] / seg + lo)) * seg;
+  return lo;
+}
+
+template <typename T, int NS, int R, int MODE>
 __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x, int ldx, const float* __restrict__ dtp,
                                                         const float* __restrict__ dtb, const T* __restrict__ bm, int ldb,
                                                         const T* __restrict__ cm, int ldc, const float* __restrict__ a_log,
                                                         const float* __restrict__ dskip, const T* __restrict__ z, int ldz,
                                                         float* __restrict__ S, T* __restrict__ out, int ldo, float scale,
-                                                        int C, int N, SeqDesc d) {
+                                                        int C, int N, float* __restrict__ ws, float* __restrict__ wdt,
+                                                        int seg, SeqDesc d) {
   constexpr int NC = 256 / R * CH, PER = CT * NC / 256, NP = NS * R, PB = (CT * NP + 255) / 256;
   __shared__ __attribute__((aligned(16))) float sdt[CT * NC];
   __shared__ __attribute__((aligned(16))) float sdx[CT * NC];     // dt x
   __shared__ __attribute__((aligned(16))) float sy[CT * NC];      // the tokens' read-outs
   __shared__ __attribute__((aligned(16))) float sB[CT * NP];
   __shared__ __attribute__((aligned(16))) float sC[CT * NP];
-  const int s = blockIdx.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   const int lane = tid & 63, grp = (tid >> 6) * (64 / R) + lane_group<R>(lane), row = lane >> 4;
   const int cb = blockIdx.y * NC, c0 = cb + grp * CH, n0 = lane_part<R>(lane) * NS;
+  int s = blockIdx.x, first = 0;
+  if (MODE != WHOLE) s = find_segment(d, seg, blockIdx.x, first);
   if (d.live && !d.live[s]) return;
-  const int t0 = d.seq_off[s], t1 = d.seq_off[s + 1], p0 = d.pos0[s], slot = d.slots[s];
-  float Sr[CH][NS], A[CH][NS];
+  const int end = d.seq_off[s + 1], t0 = MODE == WHOLE ? d.seq_off[s] : first, t1 = MODE == WHOLE ? end : min(end, first + seg);
+  // (behind a sequence's last segment stands nothing that a leaving state would serve)
+  if (MODE != WHOLE && (t0 < d.seq_off[s] || t0 >= end || (MODE == LEAVES && t1 == end))) return;
+  const int p0 = d.pos0[s], slot = d.slots[s];
+  float Sr[CH][NS], A[CH][NS], sum[CH] = {0.f, 0.f};
 #pragma unroll
   for (int h = 0; h < CH; ++h) {
     const bool ok = c0 + h < C;
     const size_t ch = ok ? c0 + h : 0;
     load_state<NS>(a_log + ch * N, n0, N, ok, A[h]);
-    load_state<NS>(S + ((size_t)slot * C + ch) * N, n0, N, ok && p0 > 0, Sr[h]);
+    if (MODE == FROM)
+      load_state<NS>(ws + ((size_t)blockIdx.x * C + ch) * N, n0, N, ok, Sr[h]);
+    else
+      load_state<NS>(S + ((size_t)slot * C + ch) * N, n0, N, MODE == WHOLE && ok && p0 > 0, Sr[h]);
 #pragma unroll
     for (int i = 0; i < NS; ++i) A[h][i] = -expf(A[h][i]) * 1.4426950408889634f;    // decays as powers of two
   }
@@ -133,14 +164,14 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
     for (int i = 0; i < PER; ++i) {
       const size_t t = min(tb + ft + 256 / NC * i, t1 - 1);
       fx[i] = x[t * ldx + fcc];
-      fz[i] = z[t * ldz + fcc];
+      if (MODE != LEAVES) fz[i] = z[t * ldz + fcc];
       fd[i] = dtp[t * C + fcc];
     }
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
       const size_t t = min(tb + bt + 256 / NP * i, t1 - 1);
       fB[i] = bm[t * ldb + brc];
-      fC[i] = cm[t * ldc + brc];
+      if (MODE != LEAVES) fC[i] = cm[t * ldc + brc];
     }
   };
   if (t0 < t1) fetch(t0);
@@ -152,14 +183,16 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
       const float dt = softplus_fast(fd[i] + bias);
       sdt[tid + 256 * i] = dt;
       sdx[tid + 256 * i] = dt * (float)fx[i];
-      gx[i] = fx[i];
-      gz[i] = fz[i];
+      if (MODE != LEAVES) {
+        gx[i] = fx[i];
+        gz[i] = fz[i];
+      }
     }
 #pragma unroll
     for (int i = 0; i < PB; ++i)
       if (CT * NP >= 256 || tid < CT * NP) {
         sB[tid + 256 * i] = br < N ? (float)fB[i] : 0.f;          // a padded state never leaves zero
-        sC[tid + 256 * i] = br < N ? (float)fC[i] : 0.f;
+        if (MODE != LEAVES) sC[tid + 256 * i] = br < N ? (float)fC[i] : 0.f;
       }
     __syncthreads();
     if (tb + CT < t1) fetch(tb + CT);
@@ -171,7 +204,7 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
 #pragma unroll
       for (int i4 = 0; i4 < NS / 4; ++i4) {
         in.B[i4] = *reinterpret_cast<const f32x4*>(sB + tt * NP + n0 + 4 * i4);
-        in.C[i4] = *reinterpret_cast<const f32x4*>(sC + tt * NP + n0 + 4 * i4);
+        if (MODE != LEAVES) in.C[i4] = *reinterpret_cast<const f32x4*>(sC + tt * NP + n0 + 4 * i4);
       }
 #pragma unroll
       for (int h = 0; h < CH; ++h) {
@@ -186,9 +219,12 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
           Sr[h][i] = __builtin_amdgcn_exp2f(in.dt[h] * A[h][i]) * Sr[h][i] + in.dx[h] * in.B[i >> 2][i & 3];
-          p[i & 1] += Sr[h][i] * in.C[i >> 2][i & 3];
+          if (MODE != LEAVES) p[i & 1] += Sr[h][i] * in.C[i >> 2][i & 3];
         }
-        y[h] = p[0] + p[1];
+        if (MODE == LEAVES)
+          sum[h] += in.dt[h];
+        else
+          y[h] = p[0] + p[1];
       }
     };
     In a0, a1;
@@ -200,14 +236,16 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
       step(a0, ya);
       load(min(tt + 2, n - 1), a0);
       step(a1, yb);
+      if (MODE == LEAVES) continue;
       const float v = sum_four<R>(ya[0], ya[1], yb[0], yb[1]);     // row i of the wave: token tt + i / 2, channel i % 2
       if (R == 4 || (lane & (R == 8 ? 1 : 3)) == 0) sy[(tt + (row >> 1)) * NC + grp * CH + (row & 1)] = v;
     }
     if (tt < n) {
       step(a0, ya);
-      const float v = sum_four<R>(ya[0], ya[1], yb[0], yb[1]);
-      if ((R == 4 || (lane & (R == 8 ? 1 : 3)) == 0) && row < 2) sy[tt * NC + grp * CH + row] = v;
+      const float v = MODE == LEAVES ? 0.f : sum_four<R>(ya[0], ya[1], yb[0], yb[1]);
+      if (MODE != LEAVES && (R == 4 || (lane & (R == 8 ? 1 : 3)) == 0) && row < 2) sy[tt * NC + grp * CH + row] = v;
     }
+    if (MODE == LEAVES) continue;
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -220,7 +258,49 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
   }
 #pragma unroll
   for (int h = 0; h < CH; ++h)
-    if (c0 + h < C) store_state<NS>(S + ((size_t)slot * C + c0 + h) * N, n0, N, Sr[h]);
+    if (c0 + h < C) {
+      if (MODE == LEAVES) {
+        store_state<NS>(ws + ((size_t)blockIdx.x * C + c0 + h) * N, n0, N, Sr[h]);
+        if (n0 == 0) wdt[(size_t)blockIdx.x * C + c0 + h] = sum[h];
+      } else if (MODE == WHOLE || t1 == end) {
+        store_state<NS>(S + ((size_t)slot * C + c0 + h) * N, n0, N, Sr[h]);
+      }
+    }
+}
+
+// The states in front of a sequence's segments, one (channel, state) per thread: they replace the states that the segments left.
+__global__ __launch_bounds__(256) void k_selective_walk(const float* __restrict__ a_log, const float* __restrict__ S,
+                                                        float* __restrict__ ws, const float* __restrict__ wdt, int C, int N,
+                                                        int seg, SeqDesc d) {
+  const int s = blockIdx.x;
+  const size_t e = (size_t)blockIdx.y * 256 + threadIdx.x, size = (size_t)C * N;
+  if ((d.live && !d.live[s]) || e >= size) return;
+  const int t0 = d.seq_off[s], n = (d.seq_off[s + 1] - t0 + seg - 1) / seg, first = t0 / seg + s;
+  const float A = -expf(a_log[e]) * 1.4426950408889634f;
+  float x = d.pos0[s] > 0 ? S[(size_t)d.slots[s] * size + e] : 0.f;
+  float* u = ws + (size_t)first * size + e;
+  const float* dt = wdt + (size_t)first * C + e / N;
+  constexpr int AHEAD = 16;                         // segments in flight (the last one left nothing)
+  float f[AHEAD], g[AHEAD];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i)
+    if (i < n - 1) {
+      f[i] = u[i * size];
+      g[i] = dt[(size_t)i * C];
+    }
+  for (int c0 = 0; c0 < n; c0 += AHEAD)
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int c = c0 + i;
+      if (c < n) {
+        u[c * size] = x;
+        if (c < n - 1) x = __builtin_amdgcn_exp2f(g[i] * A) * x + f[i];
+        if (c + AHEAD < n - 1) {
+          f[i] = u[(c + AHEAD) * size];
+          g[i] = dt[(size_t)(c + AHEAD) * C];
+        }
+      }
+    }
 }
 
 // ------------------------------------------------------------------------------------------ gated linear attention
@@ -338,14 +418,40 @@ __global__ __launch_bounds__(256) void k_gla_scan(const T* __restrict__ q, int l
 int seq_selective_max_states() { return 256; }
 int seq_gla_max_dk() { return 256; }
 
+// Tokens of a segment of the scan cut over time, or 0 where sequences run whole.  Whole, the longest sequence takes 0.226 us a
+// token as long as the chip is not full; cut, a step takes 8.5 us per 1000 tokens and 1000 channels and about 25 us.  Segments
+// of 32 tokens where those of 64 would leave the chip idle, else 64: their states pass through memory four times.
+int seq_selective_segment(int T_, int B, int C) {
+  if (B == 0 || 0.226f * T_ / B < 8.5e-6f * T_ * C + 25.f) return 0;
+  return (long)T_ * C < (1L << 22) ? 32 : 64;
+}
+size_t seq_selective_floats(int T_, int B, int C, int N) {
+  const int seg = seq_selective_segment(T_, B, C);
+  return seg == 0 ? 0 : ((size_t)T_ / seg + B) * C * (N + 1);
+}
+
 void seq_selective_scan(int code, const void* x, int ldx, const float* dtp, const float* dtb, const void* b, int ldb,
                         const void* c, int ldc, const float* a_log, const float* dskip, const void* z, int ldz, float* S,
-                        void* out, int ldo, float scale, int C, int N, SeqDesc d, hipStream_t st) {
+                        void* out, int ldo, float scale, int C, int N, float* ws, SeqDesc d, hipStream_t st) {
   if (d.B == 0) return;
-#define SEL_LAUNCH(NS_, R_)                                                                                           \
-  hipLaunchKernelGGL((k_selective_scan<T, NS_, R_>), dim3(d.B, (C + 256 / R_ * CH - 1) / (256 / R_ * CH)), dim3(256), \
-                     0, st, (const T*)x, ldx, dtp, dtb, (const T*)b, ldb, (const T*)c, ldc, a_log, dskip, (const T*)z, ldz, \
-                     S, (T*)out, ldo, scale, C, N, d)
+  const int seg = ws != nullptr ? seq_selective_segment(d.Ttot, d.B, C) : 1;
+  const size_t slots = (size_t)d.Ttot / seg + d.B;
+  float* wdt = ws != nullptr ? ws + slots * C * N : nullptr;
+#define SEL_LAUNCH_(NS_, R_, MODE_, X_)                                                                                     \
+  hipLaunchKernelGGL((k_selective_scan<T, NS_, R_, MODE_>), dim3((unsigned)(X_), (C + 256 / R_ * CH - 1) / (256 / R_ * CH)), \
+                     dim3(256), 0, st, (const T*)x, ldx, dtp, dtb, (const T*)b, ldb, (const T*)c, ldc, a_log, dskip,        \
+                     (const T*)z, ldz, S, (T*)out, ldo, scale, C, N, ws, wdt, seg, d)
+#define SEL_LAUNCH(NS_, R_)                                                                                              \
+  do {                                                                                                                   \
+    if (ws == nullptr) {                                                                                                 \
+      SEL_LAUNCH_(NS_, R_, WHOLE, d.B);                                                                                  \
+    } else {                                                                                                             \
+      SEL_LAUNCH_(NS_, R_, LEAVES, slots);                                                                               \
+      hipLaunchKernelGGL(k_selective_walk, dim3(d.B, (unsigned)(((size_t)C * N + 255) / 256)), dim3(256), 0, st, a_log, S, ws, \
+                         wdt, C, N, seg, d);                                                                                  \
+      SEL_LAUNCH_(NS_, R_, FROM, slots);                                                                                 \
+    }                                                                                                                    \
+  } while (0)
   SEQ_DISPATCH_T(code, {
     if (N <= 16)
       SEL_LAUNCH(4, 4);
@@ -359,6 +465,7 @@ void seq_selective_scan(int code, const void* x, int ldx, const float* dtp, cons
       SEL_LAUNCH(16, 16);
   });
 #undef SEL_LAUNCH
+#undef SEL_LAUNCH_
   LIPA_CHECK_LAUNCH();
 }
 

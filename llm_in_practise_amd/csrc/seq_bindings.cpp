@@ -70,7 +70,8 @@ void seq_residual_dyt(int, int, const float*, const void*, int, float, float*, i
                       SeqDesc, hipStream_t);
 void seq_softcap(float*, size_t, float, hipStream_t);
 void seq_selective_scan(int, const void*, int, const float*, const float*, const void*, int, const void*, int, const float*,
-                        const float*, const void*, int, float*, void*, int, float, int, int, SeqDesc, hipStream_t);
+                        const float*, const void*, int, float*, void*, int, float, int, int, float*, SeqDesc, hipStream_t);
+size_t seq_selective_floats(int, int, int, int);
 void seq_gla_scan(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float,
                   float*, float*, int, int, int, SeqDesc, hipStream_t);
 int seq_dyt_max_taps();
@@ -1106,9 +1107,12 @@ Tensor selective_scan(Tensor x, Tensor dt_pre, Tensor dt_bias, Tensor b, Tensor 
     out = at::empty({T, C}, x.options());
   }
   if (T == 0) return out;
+  Tensor ws;
+  if (const size_t n = seq_selective_floats((int)T, d.B, (int)C, (int)N)) ws = at::empty({(int64_t)n}, S.options());
   seq_selective_scan(code, x.data_ptr(), ld(x), dt_pre.data_ptr<float>(), dt_bias.data_ptr<float>(), b.data_ptr(), ld(b),
                      c.data_ptr(), ld(c), a_log.data_ptr<float>(), d_skip.data_ptr<float>(), z.data_ptr(), ld(z),
-                     S.data_ptr<float>(), out.data_ptr(), ld(out), (float)scale, (int)C, (int)N, d, stream());
+                     S.data_ptr<float>(), out.data_ptr(), ld(out), (float)scale, (int)C, (int)N,
+                     ws.defined() ? ws.data_ptr<float>() : nullptr, d, stream());
   return out;
 }
 

@@ -157,3 +157,29 @@ def test_gla_blocks(lens, starts, H, dk, dv, dt):
                                 dk ** -0.5, st["S"], H, sb)
         res.append((o, st["S"]))
     _close(res[1], res[0], ("o", "state"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,starts,C,N,dt", [([160], [0], 40, 16, torch.bfloat16), ([129, 256, 1, 320], [0, 7, 0, 0], 33, 5, torch.float32),
+                                                ([127, 130], [0, 3], 130, 40, torch.bfloat16), ([200], [0], 64, 200, torch.float32),
+                                                ([1089], [0], 4096, 16, torch.bfloat16), ([60, 64], [0, 0], 64, 16, torch.float32)])
+def test_selective_cut_over_time(lens, starts, C, N, dt):
+    g = torch.Generator().manual_seed(C + N)
+    T = sum(lens)
+    x, z, bc = (torch.randn(T, n, generator=g).to(dt) for n in (C, C, 2 * N))
+    dtp, dtb, skip = torch.randn(T, C, generator=g), torch.randn(C, generator=g) - 2, torch.randn(C, generator=g)
+    a_log = torch.randn(C, N, generator=g)
+    a_log[:, 0], a_log[0] = -30.0, 40.0                 # states that keep everything, a channel that forgets everything
+    S0 = torch.randn(len(lens), C, N, generator=g)
+    res = []
+    for dev in ("cpu", "cuda"):
+        st, sb = _batch({"S": ((C, N), "f32")}, lens, starts, dev)
+        st["S"].copy_(S0)
+        p = [t.to(dev) for t in (x, dtp, dtb, bc[:, :N], bc[:, N:], a_log, skip, z)]
+        y = R.selective_scan(*p, st["S"], sb)
+        res.append((y.float(), st["S"]))
+    # (bf16 outputs: both sides round, to at most one unit of 2^-8 apart)
+    (y1, s1), (y0, s0) = res[1], res[0]
+    _close((s1,), (s0,), ("state",))
+    tol = TOL if dt == torch.float32 else 2.0 ** -8
+    assert torch.isfinite(y1).all() and (y1.cpu() - y0).norm() <= tol * y0.norm()
