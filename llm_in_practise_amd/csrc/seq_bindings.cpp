@@ -52,6 +52,9 @@ void seq_route_fused(int, const void*, int, const float*, const float*, int*, fl
                      int, int, float*, int, hipStream_t);
 void seq_moe_pairs(int, const void*, int, const void*, const void*, const int*, const float*, const void*, const float*,
                    void*, float*, int, int, int, int, int, float, int, int, hipStream_t);
+bool seq_moe_tiles_ok(int, const void*, const void*, const void*, long, int, int, int, int);
+void seq_moe_tiles(const void*, const void*, const void*, const int*, const float*, int*, int*, long*, void*, void*, int, int, int,
+                   int, int, float, int, hipStream_t);
 void seq_moe_combine(int, const void*, const long*, const int*, const float*, const void*, int, const void*, const float*,
                      float*, int, int, int, int, hipStream_t);
 void seq_embed_learned(int, const long*, const int*, const void*, const void*, float*, int, int, int, int, int,
@@ -763,6 +766,42 @@ Tensor moe_pairs(Tensor h, Tensor wgu, Tensor wd, Tensor idx, Tensor w, optional
   return out;
 }
 
+// prompts: the pairs ordered by expert, every expert's products in tiles of its run.  As moe_pairs; none where the kernels do not
+// take the shapes.
+optional<Tensor> moe_tiles(Tensor h, Tensor wgu, Tensor wd, Tensor idx, Tensor w, optional<Tensor> shared, double limit, int64_t mode,
+                           optional<Tensor> shared_gate, bool weight_input) {
+  TORCH_CHECK(mode == 1 || mode == 2, "expert activation: 1 clipped GLU, 2 SiLU GLU");
+  const int code = code_of(h);
+  TORCH_CHECK(h.is_cuda() && h.dim() == 2, "h: [T, W]");
+  const int64_t T = h.size(0), W = h.size(1);
+  if (!h.is_contiguous() || !wgu.is_cuda() || !wgu.is_contiguous() || wgu.dim() != 4 || wgu.size(1) != 2 || wgu.size(3) != W ||
+      code_of(wgu) != code || !wd.is_cuda() || !wd.is_contiguous() || wd.dim() != 3 || wd.size(0) != wgu.size(0) ||
+      wd.size(1) != W || wd.size(2) != wgu.size(2) || code_of(wd) != code)
+    return optional<Tensor>();
+  const int64_t E = wgu.size(0), F = wgu.size(2);
+  check_route(idx, w, T);
+  const int64_t top = idx.size(1);
+  if (T == 0 || top == 0 || !seq_moe_tiles_ok(code, h.data_ptr(), wgu.data_ptr(), wd.data_ptr(), T, (int)top, (int)E, (int)F, (int)W))
+    return optional<Tensor>();
+  const void* sp = nullptr;
+  if (shared && shared->defined()) {
+    TORCH_CHECK(shared->is_cuda() && shared->is_contiguous() && shared->dim() == 2 && shared->size(0) == T &&
+                    shared->size(1) == W && code_of(*shared) == code, "shared: [T, W]");
+    sp = shared->data_ptr();
+  }
+  auto ints = at::empty({E + 1 + T * top}, idx.options());
+  auto pos = at::empty({T * top}, idx.options().dtype(at::kLong));
+  auto a = at::empty({T * top, F}, h.options()), ys = at::empty({T * top, W}, h.options());
+  auto out = at::empty({T, W}, h.options().dtype(at::kFloat));
+  const Tensor ones = weight_input ? at::ones_like(w) : w;
+  seq_moe_tiles(h.data_ptr(), wgu.data_ptr(), wd.data_ptr(), idx.data_ptr<int>(), weight_input ? w.data_ptr<float>() : nullptr,
+                ints.data_ptr<int>(), ints.data_ptr<int>() + E + 1, pos.data_ptr<long>(), a.data_ptr(), ys.data_ptr(), (int)T,
+                (int)top, (int)E, (int)F, (int)W, (float)limit, (int)mode, stream());
+  seq_moe_combine(code, ys.data_ptr(), pos.data_ptr<long>(), idx.data_ptr<int>(), ones.data_ptr<float>(), h.data_ptr(), (int)W, sp,
+                  shared_gate_of(shared_gate, T), out.data_ptr<float>(), (int)T, (int)top, (int)E, (int)W, stream());
+  return out;
+}
+
 // ys [rows, W]: expert outputs in expert-sorted order; pos [T, top] int64: the row of every pair
 Tensor moe_combine_sorted(Tensor ys, Tensor pos, Tensor idx, Tensor w, Tensor h, optional<Tensor> shared, int64_t E,
                           optional<Tensor> shared_gate) {
@@ -1250,6 +1289,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("route_grouped", &route_grouped);
   m.def("route_fused", &route_fused);
   m.def("moe_pairs", &moe_pairs);
+  m.def("moe_tiles", &moe_tiles);
   m.def("moe_combine_sorted", &moe_combine_sorted);
   m.def("ff_act", &ff_act, py::arg("z"), py::arg("mode"), py::arg("limit"), py::arg("row_scale") = py::none());
   m.def("embed_learned", &embed_learned);

@@ -208,8 +208,9 @@ def moe_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tens
     expert's output is multiplied by its sigmoid).  ``w_gate_up`` ``[E, 2, F, W]``,
     ``w_down`` ``[E, W, F]``; ids ``>= E`` are identity experts (their output is ``h``); ``shared`` ``[T, W]`` is
     added.  ``few_tokens`` (decode steps, captured graphs): every (token, expert) pair streams its expert's rows in
-    two kernels with no sort and no host round trip.  Otherwise rows are sorted by expert, every expert runs one
-    vendor matrix product pair over its run of rows (one host read of the run lengths; long runs are rounded up to a
+    two kernels with no sort and no host round trip.  Otherwise the pairs are ordered by expert and every expert's
+    products run over tiles of its run (bf16, ``F`` and ``W`` multiples of 64: csrc/kernels/seq/seq_moe_gemm.hip; else one
+    vendor matrix product pair per expert, with one host read of the run lengths and long runs rounded up to a
     multiple of ``PAD_ROWS`` rows), and a kernel combines.  ``weight_input`` (``act="silu"``): a pair's weight multiplies
     the expert's input instead of its output, ``sum_e expert_e(w_e h)``; it is applied in float to the gate and up
     products, which are linear in the input."""
@@ -228,6 +229,11 @@ def moe_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tens
     if use_seq(h) and few_tokens:
         return native_seq().moe_pairs(h.contiguous(), w_gate_up, w_down, idx, weights, shared, limit, mode, shared_gate,
                                       weight_input)
+    if use_seq(h):
+        out = native_seq().moe_tiles(h.contiguous(), w_gate_up, w_down, idx, weights, shared, limit, mode, shared_gate,
+                                     weight_input)
+        if out is not None:
+            return out
     flat = idx.reshape(-1).long()
     order = torch.sort(flat, stable=True).indices
     counts = torch.bincount(flat, minlength=E).tolist()[:E]

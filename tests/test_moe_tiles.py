@@ -1,0 +1,52 @@
+"""Routed experts of prompts: the kernels that order pairs by expert and run every expert's products in tiles
+(csrc/kernels/seq/seq_moe_gemm.hip), and the routing kernel of prompts, against the reference ops."""
+import pytest
+import torch
+
+from llm_in_practise_amd.ops import moe as M
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,top,E,F,W,kind", [
+    (40, 2, 8, 64, 64, "even"), (129, 2, 5, 192, 192, "even"), (300, 4, 8, 128, 320, "identity"), (257, 1, 1, 64, 128, "even"),
+    (700, 3, 9, 448, 256, "skewed"), (33, 2, 16, 384, 64, "skewed"), (2100, 2, 3, 64, 64, "even")])
+@pytest.mark.parametrize("act,weight_input,gate", [("silu", False, True), ("silu", True, False), ("clipped", False, False)])
+def test_expert_tiles(T, top, E, F, W, kind, act, weight_input, gate):
+    g = torch.Generator().manual_seed(T + F)
+    h = torch.randn(T, W, generator=g).bfloat16()
+    gu = (torch.randn(E, 2, F, W, generator=g) * W ** -0.5).bfloat16()
+    d = (torch.randn(E, W, F, generator=g) * F ** -0.5).bfloat16()
+    n = E + 2 if kind == "identity" else E
+    idx = torch.rand(T, max(n, top), generator=g).argsort(1)[:, :top]
+    if kind == "skewed":                                # one expert takes nearly all, others nothing
+        idx = torch.where(torch.rand(T, top, generator=g) < 0.9, torch.full_like(idx, E - 2), idx)
+    idx, w = (idx % n).int().contiguous(), torch.rand(T, top, generator=g)
+    sh, sg = torch.randn(T, W, generator=g).bfloat16(), torch.randn(T, generator=g) if gate else None
+    on = [t.cuda() for t in (h, gu, d, idx, w)]
+    got = M.moe_glu_experts(*on, 7.0, sh.cuda(), False, act=act, shared_gate=None if sg is None else sg.cuda(),
+                            weight_input=weight_input)
+    want = M.moe_glu_experts(h.float(), gu.float(), d.float(), idx, w, 7.0, sh.float(), False, act=act, shared_gate=sg,
+                             weight_input=weight_input)
+    # the activation and an expert's output are rounded to bf16 once each: two relative errors of at most 2^-9
+    assert torch.isfinite(got).all() and (got.cpu() - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("T", [256, 259, 1000])
+@pytest.mark.parametrize("n,W,top,groups,keep,kw", [
+    (8, 2048, 2, 1, 1, dict(normalize=True)), (10, 1024, 4, 2, 1, dict(scale=2.0)), (16, 72, 3, 4, 2, dict(score="sigmoid", group_rank="top2")),
+    (3, 64, 1, 1, 1, dict(extra=2)), (7, 516, 7, 1, 1, dict(always=1)), (1, 4, 1, 1, 1, {}), (13, 260, 2, 1, 1, dict(extra=3, always=2))])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_routing_of_prompts(T, n, W, top, groups, keep, kw, dt):
+    g = torch.Generator().manual_seed(T + n + W)
+    h = torch.randn(T, W, generator=g).to(dt)
+    router = torch.randn(n + kw.get("extra", 0), W, generator=g) * W ** -0.5
+    corr = 0.1 * torch.randn(n, generator=g)
+    got = M.route_tokens(h.cuda(), router.cuda(), corr.cuda(), top, groups, keep, **kw)
+    want = M.route_tokens(h, router, corr, top, groups, keep, **kw)
+    # float products of W terms in another order; a choice can only differ where two scores are that close
+    same = (got[0].cpu() == want[0]).all(1)
+    assert same.float().mean() >= 0.995
+    assert (got[1].cpu() - want[1])[same].abs().max() <= 1e-5 * max(1.0, kw.get("scale", 1.0))
+    if kw.get("extra"):
+        torch.testing.assert_close(got[2].cpu(), want[2], rtol=1e-5, atol=1e-5)
