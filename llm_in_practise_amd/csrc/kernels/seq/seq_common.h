@@ -42,6 +42,16 @@ __device__ __forceinline__ float log1p_exp_neg(float a) {
   return 2.f * s * (p * q + 1.f);
 }
 
+// sums of two values over exchanged lanes
+__device__ __forceinline__ float swap32_add(float a, float b) {       // lanes 0-31: sum of a, lanes 32-63: sum of b
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap16_add(float a, float b) {       // even rows: sum of a over a pair of rows, odd: of b
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // Entry c of a vector whose first `dims` entries are rotated by pos * inv_freq[pair]: neighbours (2i, 2i+1) form pair
 // i, or with `half` entries (i, i + dims/2) do; the rest pass unchanged.  Sine and cosine are multiplied by mag.
 // The pair (u, v) becomes (u cos - v sin, v cos + u sin); the angle is a float product.

@@ -12,51 +12,65 @@ using namespace lipa;
 
 constexpr int RPL = 4;   // router outputs per lane: experts + identity experts <= 64 * RPL
 
-// (value, index) maximum over a wave; ties go to the lower index
-__device__ __forceinline__ void wave_argmax(float& v, int& i) {
+// (value, index) maximum over GW lanes; ties go to the lower index
+template <int GW>
+__device__ __forceinline__ void group_argmax(float& v, int& i) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o, 64);
-    const int oi = __shfl_xor(i, o, 64);
+  for (int o = GW / 2; o > 0; o >>= 1) {
+    const float ov = __shfl_xor(v, o, GW);
+    const int oi = __shfl_xor(i, o, GW);
     if (ov > v || (ov == v && oi < i)) {
       v = ov;
       i = oi;
     }
   }
 }
+template <int GW>
+__device__ __forceinline__ float group_max(float v) {
+#pragma unroll
+  for (int o = GW / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, GW));
+  return v;
+}
+template <int GW>
+__device__ __forceinline__ float group_add(float v) {
+#pragma unroll
+  for (int o = GW / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, GW);
+  return v;
+}
 
-// One wave routes one token from its n router logits z (global or LDS).  s = softmax(z) over all n outputs;
+// GW lanes route one token from its n router logits, RP a lane (z[i]: output lane + GW i).  s = softmax(z) over all n outputs;
 // choice = s + corr; the n outputs form `groups` equal runs of neighbours, a group's score is its largest choice and
 // only the `keep` best groups stay eligible; the `top` largest eligible choices are taken and weighted by s * scale
 // (s without the correction, not renormalised).  `always` more ids n, n + 1, .. of weight 1 follow the chosen ones (experts
 // that every token uses).
-__device__ __forceinline__ void route_wave(const float* z, const float* __restrict__ corr, int* __restrict__ idx,
+template <int GW, int RP>
+__device__ __forceinline__ void route_lanes(const float (&z)[RP], const float* __restrict__ corr, int* __restrict__ idx,
                                            float* __restrict__ wout, int lane, int n, int top, int groups, int keep,
                                            float scale, int kind, int always) {
-  float s[RPL], ch[RPL];
+  float s[RP], ch[RP];
   float mx = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < RPL; ++i) {
-    const int e = lane + 64 * i;
+  for (int i = 0; i < RP; ++i) {
+    const int e = lane + GW * i;
     // a row nobody reads (an idle decode row) may carry anything, NaN included: it still gets ids inside [0, n)
-    s[i] = e < n ? (isfinite(z[e]) ? z[e] : 0.f) : -INFINITY;
+    s[i] = e < n ? (isfinite(z[i]) ? z[i] : 0.f) : -INFINITY;
     if ((kind & 8) && e < n && corr != nullptr) s[i] += corr[e];
     mx = fmaxf(mx, s[i]);
   }
-  mx = wave_max(mx);
+  mx = group_max<GW>(mx);
   float sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < RPL; ++i) {
+  for (int i = 0; i < RP; ++i) {
     if (kind & 1)
-      s[i] = lane + 64 * i < n ? sigmoidf_(s[i]) : 0.f;
+      s[i] = lane + GW * i < n ? sigmoidf_(s[i]) : 0.f;
     else
-      s[i] = lane + 64 * i < n ? expf(s[i] - mx) : 0.f;
+      s[i] = lane + GW * i < n ? expf(s[i] - mx) : 0.f;
     sum += s[i];
   }
-  sum = (kind & 1) ? 1.f : wave_sum(sum);
+  sum = (kind & 1) ? 1.f : group_add<GW>(sum);
 #pragma unroll
-  for (int i = 0; i < RPL; ++i) {
-    const int e = lane + 64 * i;
+  for (int i = 0; i < RP; ++i) {
+    const int e = lane + GW * i;
     s[i] /= sum;
     ch[i] = e < n ? s[i] + (corr != nullptr && !(kind & 8) ? corr[e] : 0.f) : -INFINITY;
   }
@@ -68,83 +82,83 @@ __device__ __forceinline__ void route_wave(const float* z, const float* __restri
       float b1 = -INFINITY;
       int e1 = 1 << 30;
 #pragma unroll
-      for (int i = 0; i < RPL; ++i) {
-        const int e = lane + 64 * i;
+      for (int i = 0; i < RP; ++i) {
+        const int e = lane + GW * i;
         if (e < n && e / gs == g && (ch[i] > b1 || (ch[i] == b1 && e < e1))) {
           b1 = ch[i];
           e1 = e;
         }
       }
-      wave_argmax(b1, e1);
+      group_argmax<GW>(b1, e1);
       float b2 = -INFINITY;
 #pragma unroll
-      for (int i = 0; i < RPL; ++i) {
-        const int e = lane + 64 * i;
+      for (int i = 0; i < RP; ++i) {
+        const int e = lane + GW * i;
         if (e < n && e / gs == g && e != e1) b2 = fmaxf(b2, ch[i]);
       }
-      b2 = wave_max(b2);
+      b2 = group_max<GW>(b2);
       if (lane == g) rank = b1 + (b2 == -INFINITY ? 0.f : b2);
     }
-    unsigned long long kept = 0ull;               // groups <= 64
+    unsigned long long kept = 0ull;               // groups <= GW
     for (int r = 0; r < keep; ++r) {
       float bv = rank;
       int bg = lane < groups ? lane : 1 << 30;
-      wave_argmax(bv, bg);
+      group_argmax<GW>(bv, bg);
       if (bg < groups) kept |= 1ull << bg;
       if (lane == bg) rank = -INFINITY;
     }
 #pragma unroll
-    for (int i = 0; i < RPL; ++i) {
-      const int e = lane + 64 * i;
+    for (int i = 0; i < RP; ++i) {
+      const int e = lane + GW * i;
       if (e < n && !((kept >> (e / gs)) & 1ull)) ch[i] = -INFINITY;
     }
   } else if (groups > 1 && keep < groups) {
     const int gs = n / groups;
     // a lane's outputs may lie in different groups: the kept-group mask is built by `keep` rounds of
     // "best remaining group", each an argmax over (choice, group) pairs
-    unsigned long long kept = 0ull;               // groups <= 64
+    unsigned long long kept = 0ull;               // groups <= GW
     for (int r = 0; r < keep; ++r) {
       float bv = -INFINITY;
       int bg = 1 << 30;
 #pragma unroll
-      for (int i = 0; i < RPL; ++i) {
-        const int e = lane + 64 * i, g = e / gs;
+      for (int i = 0; i < RP; ++i) {
+        const int e = lane + GW * i, g = e / gs;
         if (e < n && !((kept >> g) & 1ull) && (ch[i] > bv || (ch[i] == bv && g < bg))) {
           bv = ch[i];
           bg = g;
         }
       }
-      wave_argmax(bv, bg);
+      group_argmax<GW>(bv, bg);
       if (bg < groups) kept |= 1ull << bg;
     }
 #pragma unroll
-    for (int i = 0; i < RPL; ++i) {
-      const int e = lane + 64 * i;
+    for (int i = 0; i < RP; ++i) {
+      const int e = lane + GW * i;
       if (e < n && !((kept >> (e / gs)) & 1ull)) ch[i] = -INFINITY;
     }
   }
   unsigned taken = 0u;                            // bit i: this lane's output i is already chosen
-  float tot = 0.f, myw = 0.f;                     // lane r keeps the r-th choice (top <= 64)
+  float tot = 0.f, myw = 0.f;                     // lane r keeps the r-th choice (top <= GW)
   int myid = 0;
   for (int r = 0; r < top; ++r) {
     float bv = -INFINITY;
     int be = 1 << 30;
 #pragma unroll
-    for (int i = 0; i < RPL; ++i) {
-      const int e = lane + 64 * i;
+    for (int i = 0; i < RP; ++i) {
+      const int e = lane + GW * i;
       if (e < n && !((taken >> i) & 1u) && (ch[i] > bv || (ch[i] == bv && e < be))) {
         bv = ch[i];
         be = e;
       }
     }
-    wave_argmax(bv, be);
+    group_argmax<GW>(bv, be);
     be = min(be, n - 1);                          // (only when fewer than `top` outputs are eligible)
     float cand = 0.f;
 #pragma unroll
-    for (int i = 0; i < RPL; ++i)
-      if (i == (be >> 6)) cand = s[i];
-    const float bs = __shfl(cand, be & 63, 64);
-    if ((be & 63) == lane) taken |= 1u << (be >> 6);
+    for (int i = 0; i < RP; ++i)
+      if (i == (be / GW)) cand = s[i];
+    const float bs = __shfl(cand, be % GW, GW);
+    if ((be % GW) == lane) taken |= 1u << (be / GW);
     tot += bs;
     if (lane == r) {
       myw = bs;
@@ -158,6 +172,16 @@ __device__ __forceinline__ void route_wave(const float* z, const float* __restri
     idx[lane] = n + lane - top;
     wout[lane] = 1.f;
   }
+}
+
+// one wave per token, logits in memory or LDS
+__device__ __forceinline__ void route_wave(const float* z, const float* __restrict__ corr, int* __restrict__ idx,
+                                           float* __restrict__ wout, int lane, int n, int top, int groups, int keep,
+                                           float scale, int kind, int always) {
+  float v[RPL];
+#pragma unroll
+  for (int i = 0; i < RPL; ++i) v[i] = lane + 64 * i < n ? z[lane + 64 * i] : 0.f;
+  route_lanes<64, RPL>(v, corr, idx, wout, lane, n, top, groups, keep, scale, kind, always);
 }
 
 // routing from given logits: one wave per token
@@ -230,6 +254,55 @@ __global__ __launch_bounds__(64 * NW) void k_route_fused(const T* __restrict__ h
   if (wv == 0)
     route_wave(sz, corr, idx + (size_t)t * (top + always), wout + (size_t)t * (top + always), lane, n - extra, top, groups,
                keep, scale, kind, always);
+}
+
+// The same for prompts and up to 16 outputs: a block takes four tokens, a wave a quarter of their columns, so that a router row
+// read from the cache serves four tokens; the 4 x 16 sums over a wave's lanes leave (token, output) in lane 16 token + output, and
+// after the four waves' sums meet in LDS each 16 lanes of the first route their token.  8000 tokens of width 2048, 8 outputs: 41
+// -> 18 us (a block per token read the whole router from L2, 0.6 GB in all, and routed with 64 lanes).
+template <typename T, int NG>
+__global__ __launch_bounds__(256) void k_route_rows(const T* __restrict__ h, int ldh, const float* __restrict__ router,
+                                                    const float* __restrict__ corr, int* __restrict__ idx,
+                                                    float* __restrict__ wout, int T_, int n, int W, int top, int groups, int keep,
+                                                    float scale, int kind, int extra, float* __restrict__ xout, int always) {
+  __shared__ float part[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, t0 = blockIdx.x * 4;
+  float v[64];
+#pragma unroll
+  for (int i = 0; i < 64; ++i) v[i] = 0.f;
+#pragma unroll 2
+  for (int c = 4 * lane + 256 * w; c < W; c += 1024) {
+    f32x4 x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = load4(h + (size_t)min(t0 + i, T_ - 1) * ldh + c);
+#pragma unroll
+    for (int o = 0; o < 4 * NG; ++o) {
+      const f32x4 r = load4(router + (size_t)min(o, n - 1) * W + c);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[16 * i + o] += r[0] * x[i][0] + r[1] * x[i][1] + r[2] * x[i][2] + r[3] * x[i][3];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 32; ++i) v[i] = swap32_add(v[i], v[i + 32]);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = swap16_add(v[i], v[i + 16]);
+#pragma unroll
+  for (int half = 8; half > 0; half >>= 1) {
+    const bool up = lane & half;
+#pragma unroll
+    for (int i = 0; i < half; ++i) {
+      const float keep_ = up ? v[i + half] : v[i], send = up ? v[i] : v[i + half];
+      v[i] = keep_ + __shfl_xor(send, half, 64);
+    }
+  }
+  part[w][lane] = v[0];
+  __syncthreads();
+  const int t = t0 + (lane >> 4), o = lane & 15;
+  if (w != 0 || t >= T_) return;
+  const float z[1] = {(part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane])};
+  if (o >= n - extra && o < n) xout[(size_t)t * extra + o - (n - extra)] = z[0];
+  route_lanes<16, 1>(z, corr, idx + (size_t)t * (top + always), wout + (size_t)t * (top + always), o, n - extra, top, groups, keep,
+                     scale, kind, always);
 }
 
 // g = min(g, limit), u = clamp(u, -limit, limit): g * sigmoid(1.702 g) * (u + 1)
@@ -397,6 +470,24 @@ void seq_route_fused(int code, const void* h, int ldh, const float* router, cons
                      int T_, int n, int W, int top, int groups, int keep, float scale, int kind, int extra, float* xout,
                      int always, hipStream_t st) {
   if (T_ == 0) return;
+  const auto fits = [](const void* p, int b) { return ((uintptr_t)p & (b - 1)) == 0; };
+  // (below 256 tokens a block of 16 waves per token fills the chip better: 8 us at any number up to 200)
+  if (T_ >= 256 && n <= 16 && top + always <= 16 && W % 4 == 0 && ldh % 4 == 0 && fits(h, code == 0 ? 8 : 16) && fits(router, 16)) {
+#define ROUTE_ROWS(NG_)                                                                                                      \
+  hipLaunchKernelGGL((k_route_rows<T, NG_>), dim3((T_ + 3) / 4), dim3(256), 0, st, (const T*)h, ldh, router, corr, idx, w, T_, n,    \
+                     W, top, groups, keep, scale, kind, extra, xout, always)
+    SEQ_DISPATCH_T(code, {
+      switch ((n + 3) / 4) {
+        case 1: ROUTE_ROWS(1); break;
+        case 2: ROUTE_ROWS(2); break;
+        case 3: ROUTE_ROWS(3); break;
+        default: ROUTE_ROWS(4); break;
+      }
+    });
+#undef ROUTE_ROWS
+    LIPA_CHECK_LAUNCH();
+    return;
+  }
   SEQ_DISPATCH_T(code, {
     if (T_ < 256)
       hipLaunchKernelGGL((k_route_fused<T, 16>), dim3(T_), dim3(1024), 0, st, (const T*)h, ldh, router, corr, idx, w, n,

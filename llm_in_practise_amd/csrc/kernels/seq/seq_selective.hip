@@ -34,14 +34,6 @@ __device__ __forceinline__ float dpp_quad_add(float v, int which) {
                            : __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true);    // quad_perm [2, 3, 0, 1]
   return v + __int_as_float(o);
 }
-__device__ __forceinline__ float swap32_add(float a, float b) {       // lanes 0-31: sum of a, lanes 32-63: sum of b
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float swap16_add(float a, float b) {       // even rows: sum of a over a pair of rows, odd: of b
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 template <int R>
 __device__ __forceinline__ float sum_four(float v0, float v1, float v2, float v3) {
   float v = swap16_add(swap32_add(v0, v2), swap32_add(v1, v3));
