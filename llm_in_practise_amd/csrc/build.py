@@ -73,7 +73,7 @@ def build_hip_extension(jobs: int | None = None, verbose: bool = True) -> str:
     kdir = os.path.join(HERE, "kernels")
     headers = sorted(glob.glob(os.path.join(kdir, "*.h")))
     kflags = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-munsafe-fp-atomics",
-              "-ffp-contract=fast", f"-I{kdir}"]
+              "-ffp-contract=fast", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", f"-I{kdir}"]
     # LIPA_HIP_DEFINES="-DNAME ...": A/B builds of kernel variants (scripts/gpu_r6_ab_build.sh); never set by default
     kflags += [d for d in os.environ.get("LIPA_HIP_DEFINES", "").split() if d.startswith("-D")]
     bflags = ["-O3", "-std=c++17", "-fPIC", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-D__HIP_PLATFORM_AMD__=1",
