@@ -37,12 +37,11 @@ void launch_unscale(int, void*, size_t, const float*, float*, hipStream_t);
 void launch_nf4_quantize(const void*, uint8_t*, float*, size_t, hipStream_t);
 void launch_nf4_dequant2(const uint8_t*, const float*, void*, size_t, hipStream_t);
 void launch_int4_dequant(const uint8_t*, const float*, const float*, void*, size_t, int, hipStream_t);
-int skinny_splits(int, int);
 bool lt_gemm(bool, bool, long, long, long, const void*, long, const void*, long, const void*, void*, long, int, long,
              long, long, void*, size_t, hipStream_t, bool);
 void lt_reset();
 void launch_sum_slices(const void*, void*, int, size_t, size_t, hipStream_t);
-void launch_gemm_skinny(const void*, int, const void*, const void*, void*, float*, int, int, int, int, hipStream_t);
+void launch_gemm_skinny(const void*, int, const void*, const void*, void*, int, int, int, bool, hipStream_t);
 bool w4mm_supported(int, int, int, int);
 bool w4g_supported(int, int, int, int);
 int w4g_splits(int, int, int);
@@ -506,7 +505,7 @@ Tensor lt_dx(Tensor dy, Tensor w, int64_t split, bool tune, optional<Tensor> c) 
   return out;
 }
 
-Tensor gemm_skinny(Tensor x, Tensor w, optional<Tensor> residual) {
+static void check_skinny(const Tensor& x, const Tensor& w) {
   CHECK_CUDA(x);
   CHECK_BF16(x);
   CHECK_BF16(w);
@@ -517,6 +516,11 @@ Tensor gemm_skinny(Tensor x, Tensor w, optional<Tensor> residual) {
   TORCH_CHECK(w.dim() == 2 && w.size(1) == K && K % 64 == 0 && N % 16 == 0, "gemm_skinny: W [N%16, K%64]");
   TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
               "gemm_skinny: 16-B aligned operands");
+}
+
+Tensor gemm_skinny(Tensor x, Tensor w, optional<Tensor> residual) {
+  check_skinny(x, w);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   const void* rp = nullptr;
   if (residual.has_value() && residual->defined()) {
     CHECK_BF16((*residual));
@@ -524,11 +528,18 @@ Tensor gemm_skinny(Tensor x, Tensor w, optional<Tensor> residual) {
     TORCH_CHECK(residual->size(0) == M && residual->size(1) == N, "gemm_skinny: residual shape");
     rp = residual->data_ptr();
   }
-  const int S = skinny_splits(N, K);
-  Tensor part = at::empty({S, M, N}, x.options().dtype(at::kFloat));
   Tensor out = at::empty({M, N}, x.options());
-  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), rp, out.data_ptr(), part.data_ptr<float>(), M, N, K, S,
-                     stream());
+  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), rp, out.data_ptr(), M, N, K, false, stream());
+  return out;
+}
+
+// h [M, F] = silu(x Wgᵀ) (x Wuᵀ), w [2F, K] = [gate | up] rows
+Tensor gemm_skinny_swiglu(Tensor x, Tensor w) {
+  check_skinny(x, w);
+  const int64_t M = x.size(0), K = x.size(1), F = w.size(0) / 2;
+  TORCH_CHECK(w.size(0) % 32 == 0, "gemm_skinny_swiglu: W [2F, K], F % 16 == 0");
+  Tensor out = at::empty({M, F}, x.options());
+  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), nullptr, out.data_ptr(), M, F, K, true, stream());
   return out;
 }
 
@@ -1699,6 +1710,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("nf4_dequant", &nf4_dequant);
   m.def("nf4_dequant_fast", &nf4_dequant_fast);
   m.def("gemm_skinny", &gemm_skinny);
+  m.def("gemm_skinny_swiglu", &gemm_skinny_swiglu);
   m.def("lt_linear", &lt_linear);
   m.def("lt_dx", &lt_dx);
   m.def("lt_reset", &lt_reset);

@@ -1,125 +1,170 @@
-// Decode-shaped bf16 GEMM (SURVEY.md K8 at serving sizes): y[M, N] = x[M, K] · W[N, K]ᵀ (+ residual)
-// for M <= 64 — the weight-streaming regime, where the whole cost is reading W once from HBM.
+// Decode-shaped bf16 GEMM: y[M, N] = x[M, K] · W[N, K]ᵀ (+ residual) for few rows, and the same with the gated activation
+// h[M, F] = silu(x·Wgᵀ)·(x·Wuᵀ) as its end — the weight-streaming regime, where the whole cost is reading W once from HBM and
+// every launch beside it.
 //
-// hipBLASLt reaches 2-4.7 TB/s on these shapes (profiles/decode_skinny_gemm.txt: 128-column
-// tiles give N/128 workgroups, too few loads in flight).  Here:
-//  * grid (N/128, S): a workgroup owns 128 rows of W (4 waves x 32) and 1/S of K (split-K, S chosen
-//    on the host so that >= ~512 workgroups stream W); XCD-aware remap so the S splits of one
-//    N-block share an L2;
-//  * a wave's two 16-row W fragments are the MFMA A operands, loaded straight from HBM (16 B per
-//    lane, eight k-steps in flight); x (tiny, L2-resident) supplies the B operands of up to four
-//    16-column m-tiles, so every W byte feeds MT MFMAs (v_mfma_f32_16x16x32_bf16);
-//  * split-K partials go to an fp32 [S, M, N] buffer; a second kernel sums the S slices, adds the
-//    residual and writes bf16 (deterministic — no atomics).
+//  * a workgroup owns 16·CT rows of W and ALL of K, shared out to its NW waves; the partial sums meet in LDS and the one launch
+//    ends in the residual (or the activation) and bf16.  (Split-K partials through memory took a second launch: 5.7 µs of the
+//    18 of a 6144 × 4096 product.)
+//  * up to 16 rows K is cut into the S pieces of skinny_splits, whose sums are added in order: the order, and so every bit of a
+//    product, does not depend on how the pieces are shared out.  The gated form and more rows take 64-deep units in turns.
+//  * W fragments are the MFMA A operands, loaded straight from HBM (16 B per lane, whole 128-byte lines per row); one batch
+//    of steps per wave is in flight while another is multiplied.  x (tiny, L2-resident) supplies the B operands.
+//  * no load sits behind a branch: a partial batch loads its last step again and multiplies it by zero.
 #include "common.h"
 
 using namespace lipa;
 
 namespace {
 
-constexpr int SK_NB = 128;      // W rows per workgroup
-constexpr int SK_KS = 8;        // k-steps (of 32) per load batch
-
-template <int MT>
-__global__ __launch_bounds__(256) void gemm_skinny_k(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W,
-                                                     float* __restrict__ part, int M, int N, int K, int kc) {
-  const int nblk = gridDim.x, S = gridDim.y;
-  const int id = xcd_remap(blockIdx.x * S + blockIdx.y, nblk * S);
-  const int bn = id / S, sp = id % S;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
-  const int n0 = bn * SK_NB + 32 * w;
-  const int k0 = sp * kc, k1 = min(K, k0 + kc);
-  const bf16* wr0 = W + (size_t)min(n0 + li, N - 1) * K + 8 * g;
-  const bf16* wr1 = W + (size_t)min(n0 + 16 + li, N - 1) * K + 8 * g;
-  const bf16* xr[MT];
+// CUT: S pieces of kc, each with its own sum (red: S tiles); else units of 64 in turns, a sum per wave (red: NW tiles).
+// B: 32-deep steps per batch; FULL: every piece is whole batches.
+template <int CT, int MT, int NW, int B, bool GLU, bool CUT, bool FULL>
+__global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W,
+                                                         const bf16* __restrict__ res, bf16* __restrict__ out, int M, int N,
+                                                         int K, int S) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  f32x4(*red)[CT * MT][64] = reinterpret_cast<f32x4(*)[CT * MT][64]>(smem);
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16 * (GLU ? CT / 2 : CT);
+  const bf16 *wr[CT], *xr[MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) xr[mt] = X + (size_t)min(16 * mt + li, M - 1) * ldx + 8 * g;
-  f32x4 acc[2][MT];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int kb = k0; kb < k1; kb += 32 * SK_KS) {
-    const int ns = min(SK_KS, (k1 - kb) / 32);
-    bf16x8 a0[SK_KS], a1[SK_KS];
-#pragma unroll
-    for (int s = 0; s < SK_KS; ++s)
-      if (s < ns) {
-        a0[s] = *reinterpret_cast<const bf16x8*>(wr0 + kb + 32 * s);
-        a1[s] = *reinterpret_cast<const bf16x8*>(wr1 + kb + 32 * s);
-      }
-#pragma unroll
-    for (int s = 0; s < SK_KS; ++s)
-      if (s < ns) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const bf16x8 b = *reinterpret_cast<const bf16x8*>(xr[mt] + kb + 32 * s);
-          acc[0][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[s], b, acc[0][mt], 0, 0, 0);
-          acc[1][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[s], b, acc[1][mt], 0, 0, 0);
-        }
-      }
+  for (int t = 0; t < CT; ++t) {
+    const int n = GLU ? (t < CT / 2 ? 0 : N) + min(n0 + 16 * (t % (CT / 2 > 0 ? CT / 2 : 1)) + li, N - 1) : min(n0 + 16 * t + li, N - 1);
+    wr[t] = W + (size_t)n * K + 8 * g;
   }
-  // lane holds C[n = n0 + 16t + 4g + i][m = 16mt + li]
-  float* pp = part + (size_t)sp * M * N;
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int m = 16 * mt + li;
-    if (m >= M) continue;
+  for (int m = 0; m < MT; ++m) xr[m] = X + (size_t)min(16 * m + li, M - 1) * ldx + 8 * g;
+  f32x4 acc[CT][MT];
+  auto clear = [&] {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int n = n0 + 16 * t + 4 * g;
-      if (n < N) *reinterpret_cast<f32x4*>(pp + (size_t)m * N + n) = acc[t][mt];
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto leave = [&](int slot) {
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) red[slot][t * MT + m][lane] = acc[t][m];
+  };
+  struct Batch {
+    bf16x8 a[B][CT], b[B][MT];
+  };
+  // steps of one piece (of the whole wave, if not CUT), batches of one piece, batches of this wave
+  const int kc = CUT ? K / S : K, steps = CUT ? kc / 32 : 2 * ((K / 64 - w + NW - 1) / NW), per = (steps + B - 1) / B;
+  const int nb = CUT ? (S - w + NW - 1) / NW * per : per;
+  int lp = w, lb = 0;                            // the next batch to load: its piece, its place in it
+  auto load = [&](Batch& s) {
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int e = FULL ? lb * B + u : min(lb * B + u, steps - 1);
+      const int k = CUT ? lp * kc + 32 * e : 64 * (w + NW * (e >> 1)) + 32 * (e & 1);
+#pragma unroll
+      for (int t = 0; t < CT; ++t) s.a[u][t] = *reinterpret_cast<const bf16x8*>(wr[t] + k);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) s.b[u][m] = *reinterpret_cast<const bf16x8*>(xr[m] + k);
+    }
+    if (++lb == per) lb = 0, lp += NW;
+  };
+  int rp = w, rb = 0;                            // the next batch to multiply
+  auto run = [&](const Batch& s) {
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        u32x4 b = __builtin_bit_cast(u32x4, s.b[u][m]);
+        if (!FULL && rb * B + u >= steps) b = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+          acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.a[u][t], __builtin_bit_cast(bf16x8, b), acc[t][m], 0, 0, 0);
+      }
+    if (++rb == per && CUT) {
+      leave(rp);
+      clear();
+      rb = 0, rp += NW;
+    }
+  };
+  clear();
+  if (nb > 0) {
+    Batch p, q;
+    load(p);
+    int i = 0;
+    for (; i + 2 < nb; i += 2) {
+      load(q);
+      run(p);
+      load(p);
+      run(q);
+    }
+    if (i + 1 < nb) {
+      load(q);
+      run(p);
+      run(q);
+    } else {
+      run(p);
     }
   }
-}
-
-
-// out[m, n] = Σ_s part[s, m, n] (+ residual) → bf16; 8 outputs per thread
-__global__ __launch_bounds__(256) void skinny_reduce_k(const float* __restrict__ part, const bf16* __restrict__ res,
-                                                       bf16* __restrict__ out, int S, size_t MN) {
-  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
-  if (i >= MN) return;
-  float v[8];
-  {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(part + i), b = *reinterpret_cast<const f32x4*>(part + i + 4);
-    v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3]; v[4] = b[0]; v[5] = b[1]; v[6] = b[2]; v[7] = b[3];
-  }
-  for (int s = 1; s < S; ++s) {
-    const float* p = part + (size_t)s * MN + i;
-    const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
-    v[0] += a[0]; v[1] += a[1]; v[2] += a[2]; v[3] += a[3]; v[4] += b[0]; v[5] += b[1]; v[6] += b[2]; v[7] += b[3];
-  }
-  if (res) {
-    const bf16x8 r = *reinterpret_cast<const bf16x8*>(res + i);
+  if (!CUT) leave(w);
+  const int parts = CUT ? S : NW;
+  __syncthreads();
+  // lane holds C[n = n0 + 16 t + 4 g + i][m = 16 mt + li]
+  for (int c = w; c < (GLU ? CT / 2 : CT) * MT; c += NW) {
+    const int t = c / MT, m = 16 * (c % MT) + li, n = n0 + 16 * t + 4 * g;
+    f32x4 v = red[0][c][lane], up = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 1; s < parts; ++s) v += red[s][c][lane];
+    if (GLU) {
+      for (int s = 0; s < parts; ++s) up += red[s][c + CT / 2 * MT][lane];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] += (float)r[j];
-  }
-  bf16x8 o;
+      for (int e = 0; e < 4; ++e) {          // (rounded like the products they would have been)
+        const float gt = (float)(bf16)v[e], ut = (float)(bf16)up[e];
+        v[e] = gt / (1.f + __expf(-gt)) * ut;
+      }
+    }
+    if (m >= M || n >= N) continue;
+    if (res != nullptr) {
+      const bf16x4 r = *reinterpret_cast<const bf16x4*>(res + (size_t)m * N + n);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) o[j] = (bf16)v[j];
-  *reinterpret_cast<bf16x8*>(out + i) = o;
+      for (int e = 0; e < 4; ++e) v[e] += (float)r[e];
+    }
+    *reinterpret_cast<bf16x4*>(out + (size_t)m * N + n) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+  }
 }
 
 }  // namespace
 
-// Split count: >= ~512 workgroups, K-slice a multiple of 32·SK_KS where possible.
-int skinny_splits(int N, int K) {
-  const int nblk = (N + SK_NB - 1) / SK_NB;
+// Pieces of K: about 512 pairs of 128 rows and a piece, each piece 256 or more.
+static int skinny_splits(int N, int K) {
+  const int nblk = (N + 127) / 128;
   int s = 1;
   while (nblk * s < 512 && K % (64 * s) == 0 && K / (2 * s) >= 256) s *= 2;
   return s;
 }
 
-void launch_gemm_skinny(const void* X, int ldx, const void* W, const void* res, void* out, float* part, int M, int N,
-                        int K, int S, hipStream_t st) {
-  const int kc = K / S;
-  dim3 grid((N + SK_NB - 1) / SK_NB, S);
-#define L(MT) gemm_skinny_k<MT><<<grid, 256, 0, st>>>((const bf16*)X, ldx, (const bf16*)W, part, M, N, K, kc)
-  if (M <= 16) L(1);
-  else if (M <= 32) L(2);
-  else L(4);
+// Column tiles and waves per workgroup, us at 1 / 8 / 16 rows: two tiles of 8 waves take 13.2 / 13.9 / 15.1 for 6144 x 4096 (one tile
+// of 4 waves 13.7 / 15.5 / 17.5) and 9.7 / 10.8 / 12.3 for 6144 x 2560 (10.7 / 12.3 / 14.4), but 4096 rows of W fill half the CUs with
+// them: 11.9 / 13.2 / 14.9 for K = 4096 against 9.0 / 9.7 / 10.9.  The gated form pairs 16 gate with 16 up rows: 38.2 / 39.4 / 44.0
+// for 2 x 12288 x 4096, 5.3 TB/s.  Batches of 5 steps where the pieces divide by them (2560: whole batches 9.7, partial ones 11.8).
+void launch_gemm_skinny(const void* X, int ldx, const void* W, const void* res, void* out, int M, int N, int K, bool glu,
+                        hipStream_t st) {
+  const int S = skinny_splits(N, K);             // (one tile of 1 KB of LDS each: up to 32)
+  const bool cut = S <= 32 && M <= 16 && !glu;
+#define L(CT_, MT_, NW_, B_, GLU_, CUT_, FULL_)                                                                             \
+  gemm_skinny_k<CT_, MT_, NW_, B_, GLU_, CUT_, FULL_>                                                                       \
+      <<<(N + 16 * (GLU_ ? CT_ / 2 : CT_) - 1) / (16 * (GLU_ ? CT_ / 2 : CT_)), 64 * NW_, (CUT_ ? S : NW_) * CT_ * MT_ * 1024, \
+         st>>>((const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, S)
+#define LM(CT_, NW_, B_, GLU_)                                                                 \
+  do {                                                                                         \
+    if (cut && (K / S) % (32 * B_) == 0) L(CT_, 1, NW_, B_, GLU_, !GLU_, true);                \
+    else if (cut && (K / S) % 160 == 0) L(CT_, 1, NW_, 5, GLU_, !GLU_, true);                  \
+    else if (cut) L(CT_, 1, NW_, 4, GLU_, !GLU_, false);                                       \
+    else if (M <= 16 && K % (32 * B_ * NW_) == 0) L(CT_, 1, NW_, B_, GLU_, false, true);       \
+    else if (M <= 16) L(CT_, 1, NW_, 4, GLU_, false, false);                                   \
+    else if (M <= 32) L(CT_, 2, NW_, 4, GLU_, false, false);                                   \
+    else L(CT_, 4, NW_, 4, GLU_, false, false);                                                \
+  } while (0)
+  if (glu) LM(2, 4, 4, true);
+  else if (N >= 6144) LM(2, 8, 4, false);
+  else LM(1, 4, 8, false);
+#undef LM
 #undef L
-  const size_t MN = (size_t)M * N;
-  skinny_reduce_k<<<(MN / 8 + 255) / 256, 256, 0, st>>>(part, (const bf16*)res, (bf16*)out, S, MN);
   LIPA_CHECK_LAUNCH();
 }

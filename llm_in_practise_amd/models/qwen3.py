@@ -26,7 +26,7 @@ import torch.nn as nn
 
 from ..ops import reference as ref
 from ..ops.activation import swiglu_fused
-from ..ops.mlp import fusable as mlp_fusable, swiglu_mlp
+from ..ops.mlp import fusable as mlp_fusable, skinny_swiglu, swiglu_mlp
 from ..ops.attention import flash_attention, flash_attention_prefix
 from ..ops.decode import decode_attention_append
 from ..ops.linear import checkpoint as lora_checkpoint
@@ -236,15 +236,25 @@ class Qwen3MLP(nn.Module):
             return None
         return self._gu.base, down_base
 
+    def _few_rows(self, x):
+        """The activated gate|up product of a decode step in one launch, or None (adapters, other weights, more rows)."""
+        if self._gu is None or self._gu.bias is not None or any(
+                (isinstance(m, LoraLayer) and not m.merged) or getattr(_leaf_linear(m), "_mlora", None) is not None
+                for m in (self.gate_proj, self.up_proj)):
+            return None
+        return skinny_swiglu(x, self._gu.base)
+
     def forward(self, x, residual=None):
         tr = self.training
         bases = self._fused_bases(x)
         if bases is not None:
             return swiglu_mlp(x, bases[0], bases[1], residual)
-        gu = project([self.gate_proj, self.up_proj], x, None, tr, self._gu)
+        h = self._few_rows(x)
+        if h is None:
+            h = swiglu_fused(project([self.gate_proj, self.up_proj], x, None, tr, self._gu))
         if self.tp_group is None:
-            return project([self.down_proj], swiglu_fused(gu), residual, tr)
-        y = project([self.down_proj], swiglu_fused(gu), residual if self.tp_rank == 0 else None, tr)
+            return project([self.down_proj], h, residual, tr)
+        y = project([self.down_proj], h, residual if self.tp_rank == 0 else None, tr)
         return tp_all_reduce(y, self.tp_group)
 
 

@@ -172,9 +172,9 @@ def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
     N = base.shape[0]
     if (x.is_cuda and M <= 16 and N <= 8192 and K <= 8192 and N % 16 == 0 and K % 64 == 0 and x.stride(0) % 8 == 0
             and x.stride(1) == 1 and base.is_contiguous()):
-        # decode-sized q|k|v / o projections: the split-K weight-streaming MFMA kernel
-        # (csrc/kernels/skinny.hip) beats hipBLASLt's latency-bound 23 µs by 25-45 % and fuses
-        # the residual; the wide gate|up / long-K down stay on hipBLASLt (≥ 5 TB/s there)
+        # decode-sized q|k|v / o projections: the weight-streaming MFMA kernel (csrc/kernels/skinny.hip) takes 9-11 µs for
+        # 4096 × 4096 and 1-16 rows, residual included, where hipBLASLt takes 15.5 (13.2-15.1 against 14.2 for 6144 rows of W).
+        # A long K re-reads x in every workgroup: 4096 × 12288 is even at 1-8 rows and 25.6 against 21.6 µs at 16
         _count("decode")
         y = native().gemm_skinny(x, base, residual)
         return y if ext_a is None else y.addmm_(ext_a, ext_b.t())

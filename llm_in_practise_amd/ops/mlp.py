@@ -24,7 +24,7 @@ from __future__ import annotations
 import torch
 
 from ..quant.nf4 import NF4Weight
-from ._native import native, fn_apply
+from ._native import force_reference, native, fn_apply
 from .checkpoint import _sac_recording, sac_put, sac_take, saves_discarded, tail_skippable
 from .gemm import _MIN_M, _count, _nf4_expand, _nf4_w4
 
@@ -110,3 +110,26 @@ def swiglu_mlp(x: torch.Tensor, gu_base, down_base, residual: torch.Tensor | Non
     r2 = residual.reshape(-1, residual.shape[-1]).contiguous() if residual is not None else None
     y = fn_apply(_SwiGLUMLPFn, x2, r2, (gu_base, down_base))
     return y.view(*shape[:-1], y.shape[-1])
+
+
+class _SkinnySwiGLUFn(torch.autograd.Function):
+    """(No backward: skinny_swiglu leaves what needs a gradient to the differentiable ops.)"""
+    @staticmethod
+    def forward(ctx, x, w):
+        return native().gemm_skinny_swiglu(x, w)
+
+
+def skinny_swiglu(x: torch.Tensor, gu_base) -> torch.Tensor | None:
+    """``silu(x·W_gateᵀ)·(x·W_upᵀ)`` of up to 16 decode rows in one launch (csrc/kernels/skinny.hip), or None where that kernel
+    does not serve: a bf16 [gate | up] weight, no gradient.  The products are rounded to bf16 before the activation, as the
+    separate kernels round them.  4096 → 2 × 12288, product and activation: 50 → 38 µs at 1 row, 48 → 44 at 16; above that a
+    library product pulls ahead (24 rows 44 + 5 against 52)."""
+    x2 = x.reshape(-1, x.shape[-1])
+    if (torch.is_grad_enabled() and x.requires_grad) or not (
+            x.is_cuda and x.dtype == torch.bfloat16 and isinstance(gu_base, torch.Tensor) and gu_base.dtype == torch.bfloat16
+            and not gu_base.requires_grad and gu_base.is_contiguous() and 1 <= x2.shape[0] <= 16 and x2.stride(1) == 1
+            and x2.stride(0) % 8 == 0 and x2.shape[1] % 64 == 0 and gu_base.shape[0] % 32 == 0
+            and x2.data_ptr() % 16 == 0 and gu_base.data_ptr() % 16 == 0 and not force_reference()):
+        return None
+    _count("decode")
+    return fn_apply(_SkinnySwiGLUFn, x2, gu_base).view(*x.shape[:-1], gu_base.shape[0] // 2)

@@ -141,3 +141,26 @@ def test_gemm_skinny_matches_fp32(native_ext, M, N, K):
     y = native_ext.gemm_skinny(x, w, res)
     want = ref + res.float()
     assert ((y.float() - want).abs().max() / want.abs().max()).item() < 1e-2
+
+
+@pytest.mark.parametrize("M", [1, 3, 16, 17, 40])
+@pytest.mark.parametrize("N,K", [(6144, 2560), (4096, 4096), (48, 64), (1040, 576), (6160, 1984), (80, 20480)])
+def test_gemm_skinny_pieces(native_ext, M, N, K):
+    """The cuts of K (pieces of whole and of partial batches, more pieces than the LDS form takes) and the gated end against 64
+    bits: sums of K products in float lie within (K + 1) half-ulps of the absolute sum, then one rounding to bf16."""
+    torch.manual_seed(N + M)
+    x, w = torch.randn(M, K, device=DEV).to(torch.bfloat16), (torch.randn(N, K, device=DEV) * 0.02).to(torch.bfloat16)
+    res = torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    exact = x.double() @ w.double().t()
+    slack = (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    for r in (None, res):
+        want = exact if r is None else exact + r.double()
+        got = native_ext.gemm_skinny(x, w, r).double()
+        assert ((got - want).abs() <= 2 * slack + 2.0 ** -8 * want.abs()).all()
+    if N % 32 == 0:                                 # both products rounded to bf16, the activation, and rounded again
+        F = N // 2
+        g, u = exact[:, :F], exact[:, F:]
+        eg, eu = 2.0 ** -8 * g.abs() + 2 * slack[:, :F], 2.0 ** -8 * u.abs() + 2 * slack[:, F:]
+        want = g * torch.sigmoid(g) * u             # |d silu| <= 1.1
+        bound = 1.1 * eg * (u.abs() + eu) + (g * torch.sigmoid(g)).abs() * eu + 2.0 ** -7 * want.abs() + 1e-6
+        assert ((native_ext.gemm_skinny_swiglu(x, w).double() - want).abs() <= bound).all()
