@@ -48,6 +48,7 @@ int w4g_splits(int, int, int);
 void launch_w4g(const void*, int, const uint8_t*, const float*, int, const void*, void*, float*, int, int, int, int,
                 hipStream_t);
 int w4mm_nkb(int, int, int);
+bool launch_w4row(const void*, int, const uint8_t*, const float*, int, const void*, void*, int, int, int, int, bool, hipStream_t);
 void launch_w4mm(const void*, int, const uint8_t*, const float*, int, const void*, void*, float*, int, int, int, int,
                  hipStream_t);
 void set_dequant_variant(int);
@@ -547,10 +548,10 @@ Tensor gemm_skinny_swiglu(Tensor x, Tensor w) {
 // sc2 fp32 [N, K/gs, 2] = (scale, bias − 128·scale)
 bool w4mm_ok(int64_t M, int64_t N, int64_t K, int64_t gs) { return w4mm_supported((int)M, (int)N, (int)K, (int)gs); }
 
-Tensor w4mm(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, optional<Tensor> residual, int64_t nkb) {
+static void check_w4mm(const Tensor& x, const Tensor& codes, const Tensor& sc2, int64_t N, int64_t gs) {
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_CONTIG(codes); CHECK_CONTIG(sc2);
-  const int64_t M = x.size(0), K = x.size(1);
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0, "w4mm: x row-major, 16-B aligned rows");
+  const int64_t M = x.size(0), K = x.size(1);
   TORCH_CHECK(w4mm_supported((int)M, (int)N, (int)K, (int)gs), "w4mm: M<=64, N%128, K%128, gs%128");
   TORCH_CHECK(codes.scalar_type() == at::kByte && codes.numel() == N * K / 2, "w4mm: codes [N, K/2] uint8");
   TORCH_CHECK(sc2.scalar_type() == at::kFloat && sc2.numel() == N * (K / gs) * 2, "w4mm: sc2 fp32 [N, K/gs, 2]");
@@ -558,6 +559,11 @@ Tensor w4mm(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, optional<
                   reinterpret_cast<uintptr_t>(sc2.data_ptr()) % 8 == 0,
               "w4mm: aligned operands");
   TORCH_CHECK((size_t)N * K / 2 < (1ull << 31) * 2, "w4mm: codes too large");
+}
+
+Tensor w4mm(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, optional<Tensor> residual, int64_t nkb) {
+  check_w4mm(x, codes, sc2, N, gs);
+  const int64_t M = x.size(0), K = x.size(1);
   const void* rp = nullptr;
   if (residual.has_value() && residual->defined()) {
     CHECK_BF16((*residual));
@@ -570,10 +576,25 @@ Tensor w4mm(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, optional<
   TORCH_CHECK((K / 128) % nb == 0, "w4mm: K/128 divisible by nkb");
   const int KS = (int)(K / (128 * nb));
   Tensor out = at::empty({M, N}, x.options());
+  if (launch_w4row(x.data_ptr(), (int)x.stride(0), codes.data_ptr<uint8_t>(), sc2.data_ptr<float>(), (int)gs, rp,
+                   out.data_ptr(), (int)M, (int)N, (int)K, nb, false, stream()))
+    return out;
   Tensor part;
   if (KS > 1) part = at::empty({KS, M, N}, x.options().dtype(at::kFloat));
   launch_w4mm(x.data_ptr(), (int)x.stride(0), codes.data_ptr<uint8_t>(), sc2.data_ptr<float>(), (int)gs, rp,
               out.data_ptr(), KS > 1 ? part.data_ptr<float>() : nullptr, (int)M, (int)N, (int)K, nb, stream());
+  return out;
+}
+
+// h [M, N/2] = silu(g) u of the products [g | u] = x deq(W)^T, rounded to bf16 as w4mm rounds them; None where one launch does not serve
+optional<Tensor> w4mm_swiglu(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs) {
+  check_w4mm(x, codes, sc2, N, gs);
+  const int64_t M = x.size(0), K = x.size(1);
+  const int nb = w4mm_nkb((int)M, (int)N, (int)K);
+  Tensor out = at::empty({M, N / 2}, x.options());
+  if (!launch_w4row(x.data_ptr(), (int)x.stride(0), codes.data_ptr<uint8_t>(), sc2.data_ptr<float>(), (int)gs, nullptr,
+                    out.data_ptr(), (int)M, (int)N / 2, (int)K, nb, true, stream()))
+    return {};
   return out;
 }
 
@@ -1717,6 +1738,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("w4mm", &w4mm, py::arg("x"), py::arg("codes"), py::arg("sc2"), py::arg("N"), py::arg("gs"),
         py::arg("residual") = py::none(), py::arg("nkb") = 0);
   m.def("w4mm_ok", &w4mm_ok);
+  m.def("w4mm_swiglu", &w4mm_swiglu);
   m.def("w4g", &w4g, py::arg("x"), py::arg("codes"), py::arg("sc2"), py::arg("N"), py::arg("gs"),
         py::arg("residual") = py::none(), py::arg("ks") = 0);
   m.def("w4g_ok", &w4g_ok);

@@ -194,6 +194,183 @@ __global__ __launch_bounds__(256) void w4mm_reduce_k(const float* __restrict__ p
   *reinterpret_cast<bf16x2*>(out + i) = o;
 }
 
+// ============================================================================ w4row: M <= 32, one launch
+// w4mm's slices and sums with all of K in one workgroup: it owns 16·CT columns at a time, its waves take the 128·NKB-deep slices, and
+// the slices' tiles meet in LDS, added in order — the bits of w4mm and its reduce without the second launch, and with the
+// residual or SwiGLU (GLU: CT/2 gate and CT/2 up tiles of W [2N, K], products rounded to bf16 first) in the end.
+//  * ONE: as many waves as slices.  A wave keeps its slice of x in MFMA order, with its sums, in registers and walks column tiles,
+//    the codes of the next tile in flight while it multiplies this one: x is read once per workgroup, not per 16 columns.
+//  * else (long K): 8 waves take the slices of one tile in turns, the next slice's codes and x in flight.
+// x comes in whole rows of 256 B and turns through 4 KB of LDS per wave (as fragments straight from memory, 64 lines a load, the 16
+// rows of 4096 x 12288 took 20 µs, not 16).  Rows past M repeat row M - 1 and are not stored.  4.0 TB/s of codes at 24576 x 4096;
+// smaller products are the chain of launch, x, its turn and the sums: 8.3 µs for 4096 x 4096, 1.6 for each further tile.
+template <int RT, int NKB, int CT, bool GLU, bool ONE, int NT>
+__global__ __launch_bounds__(NT) void w4row_k(const bf16* __restrict__ X, int ldx, const uint8_t* __restrict__ codes,
+                                              const float2* __restrict__ sc, int gs, const bf16* __restrict__ residual,
+                                              bf16* __restrict__ out, int M, int N, int K) {
+  constexpr int CO = GLU ? CT / 2 : CT;
+  extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, q = lane >> 4;
+  const int nw = blockDim.x >> 6, KS = K / (128 * NKB), G = K / gs, nt = N / (16 * CO);
+  char* xw = lds_raw + w * 4096;                                     // (ONE: the sums take its place afterwards)
+  char* sums = lds_raw + (ONE ? 0 : nw * 4096);
+  struct Codes {
+    u32x4 c[NKB][CT];
+    float2 s[NKB][CT];
+  };
+  struct Rows {
+    u32x4 x[NKB][RT][4];
+  };
+  auto load_codes = [&](Codes& s, int tile, int slice) {
+#pragma unroll
+    for (int b = 0; b < NKB; ++b)
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        const size_t n = (size_t)((GLU && t >= CO ? N : 0) + tile * 16 * CO + 16 * (t % CO) + li);
+        const int kb = slice * NKB + b;
+        s.c[b][t] = *reinterpret_cast<const u32x4*>(codes + n * (K / 2) + 16 * q + kb * 64);
+        s.s[b][t] = sc[n * G + kb * 128 / gs];
+      }
+  };
+  auto load_rows = [&](Rows& s, int slice) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const bf16* xp = X + (size_t)min(16 * rt + 4 * p + q, M - 1) * ldx + slice * 128 * NKB + 8 * li;
+#pragma unroll
+        for (int b = 0; b < NKB; ++b) s.x[b][rt][p] = *reinterpret_cast<const u32x4*>(xp + 128 * b);
+      }
+  };
+  bf16x8 xa[NKB][RT][4];
+  f32x4 ax[NKB][RT];                             // Σx of rows 4q .. 4q+3
+  auto turn = [&](const Rows& s) {
+#pragma unroll
+    for (int b = 0; b < NKB; ++b)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        asm volatile("" ::: "memory");           // (a wave's LDS accesses are in order)
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          *reinterpret_cast<u32x4*>(xw + (4 * p + q) * 256 + 16 * (li ^ (4 * p + q))) = s.x[b][rt][p];
+        asm volatile("" ::: "memory");
+        float t[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const u32x4 d = *reinterpret_cast<const u32x4*>(xw + li * 256 + 16 * ((4 * q + j) ^ li));
+          const bf16x8 v = __builtin_bit_cast(bf16x8, d);
+          t[j] = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[j] += (float)v[e];
+          xa[b][rt][j] = __builtin_bit_cast(bf16x8, x_perm(d));
+        }
+        float sum = (t[0] + t[1]) + (t[2] + t[3]);                   // (the pairs of w4mm_k's staging: same bits)
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ax[b][rt][i] = __shfl(sum, 4 * q + i, 64);
+      }
+  };
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](const Codes& s, char* to) {
+    f32x4 acc[CT][RT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = zero;
+#pragma unroll
+    for (int b = 0; b < NKB; ++b)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        bf16x8 bq[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bq[j] = i4_bf16(s.c[b][ct][j]);
+        const float sv = s.s[b][ct].x, cc = s.s[b][ct].y;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          f32x4 g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[b][rt][0], bq[0], zero, 0, 0, 0);
+#pragma unroll
+          for (int j = 1; j < 4; ++j) g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[b][rt][j], bq[j], g, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[ct][rt][i] = fmaf(sv, g[i], fmaf(cc, ax[b][rt][i], acc[ct][rt][i]));
+        }
+      }
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) *reinterpret_cast<f32x4*>(to + ((ct * RT + rt) * 64 + lane) * 16) = acc[ct][rt];
+  };
+  constexpr int TILE = CT * RT * 256;            // floats of one slice's sums
+  auto finish = [&](const char* from, int tile) {                    // element e: y[m = 16·rt + 4q + i][its column]
+    const float* rf = reinterpret_cast<const float*>(from);
+    for (int e = tid; e < CO * RT * 256; e += blockDim.x) {
+      const int i = e & 3, l = (e >> 2) & 63, c = e >> 8, m = 16 * (c % RT) + 4 * (l >> 4) + i;
+      const int n = tile * 16 * CO + 16 * (c / RT) + (l & 15);
+      float v = 0.f, up = 0.f;
+#pragma unroll 8
+      for (int s = 0; s < KS; ++s) {
+        v += rf[s * TILE + e];
+        if (GLU) up += rf[s * TILE + CO * RT * 256 + e];
+      }
+      if (m >= M) continue;
+      if (GLU) {
+        const float gt = (float)(bf16)v, ut = (float)(bf16)up;
+        v = gt / (1.f + __expf(-gt)) * ut;
+      } else if (residual) {
+        v += (float)residual[(size_t)m * N + n];
+      }
+      out[(size_t)m * N + n] = (bf16)v;
+    }
+  };
+  if constexpr (ONE) {
+    Codes p, r;
+    {
+      Rows x;
+      load_rows(x, w);
+      load_codes(p, blockIdx.x, w);
+      turn(x);
+    }
+    __syncthreads();
+    int buf = 0;
+    auto step = [&](const Codes& now, Codes& next, int tile) {
+      load_codes(next, min(tile + (int)gridDim.x, nt - 1), w);
+      char* to = sums + buf * KS * TILE * 4;
+      multiply(now, to + w * TILE * 4);
+      __syncthreads();                           // (the other buffer is read before the next of these)
+      finish(to, tile);
+      buf ^= 1;
+    };
+    for (int tile = blockIdx.x; tile < nt; tile += 2 * gridDim.x) {
+      step(p, r, tile);
+      if (tile + (int)gridDim.x < nt) step(r, p, tile + gridDim.x);
+    }
+  } else {
+    const int tile = blockIdx.x;
+    Codes p, r;
+    Rows xp, xr;
+    int s = w;
+    if (s < KS) {
+      load_rows(xp, s);
+      load_codes(p, tile, s);
+    }
+    auto step = [&](const Codes& now, const Rows& xn, Codes& next, Rows& xt) {
+      const int n = min(s + nw, KS - 1);
+      load_rows(xt, n);
+      load_codes(next, tile, n);
+      turn(xn);
+      multiply(now, sums + s * TILE * 4);
+      s += nw;
+    };
+    while (s < KS) {
+      step(p, xp, r, xr);
+      if (s >= KS) break;
+      step(r, xr, p, xp);
+    }
+    __syncthreads();
+    finish(sums, tile);
+  }
+}
+
 // ============================================================================ w4g: 32 < M <= 64
 // The same dequant and group fold, tiled for decode batches: a workgroup owns BM = 16·RT rows × BN = 64·CT
 // columns (4 waves × 16·CT, each wave every row) over a K slice of nkb 128-deep blocks.  x is streamed per
@@ -369,6 +546,39 @@ int w4mm_nkb(int M, int N, int K) {
   const int ncs = N / W4_COLS, kb = K / 128;
   if (kb % 4 == 0 && !(M <= 8 && ncs * (kb / 4) < 512)) return 4;
   return kb % 2 == 0 ? 2 : 1;
+}
+
+// One launch of w4row_k, or false where it does not serve (w4mm_k then does).  Against w4mm_k and its reduce, us at 12 / 24 rows:
+// 6144 x 4096 9.9 / 12.9 (13.4 / 17.1), 4096 x 4096 8.3 / 11.1 (10.1 / 13.3), 24576 x 4096 19.0 / 24.1 (26.9 / 37.0; ended in SwiGLU
+// 19.9 at 12 rows, but 31.5 at 24, where 32 rows of x and two tiles of sums leave the registers), 4096 x 12288 15.6 at 12 rows (17.7;
+// its 24 slices of 32 rows do not fit the LDS).  Tiles of 32 columns lose everywhere (6144 x 4096 11.7 at 12 rows).
+bool launch_w4row(const void* X, int ldx, const uint8_t* codes, const float* sc2, int gs, const void* res, void* out, int M,
+                  int N, int K, int nkb, bool glu, hipStream_t st) {
+  const int KS = K / (128 * nkb), RT = M <= 16 ? 1 : 2, CT = glu ? 2 : 1, tiles = N / 16;
+  const bool one = KS * nkb <= 32;               // (8 waves of 4 blocks or 16 of 2 hold x)
+  const size_t sums = (size_t)KS * CT * RT * 1024, lds = one ? std::max(2 * sums, (size_t)KS * 4096) : sums + 8 * 4096;
+  if (M > (glu ? 16 : 32) || (nkb != 2 && nkb != 4) || ((RT == 2 || glu) && !one) || lds > 65536) return false;
+  const int per = (tiles + 255) / 256, grid = one ? (tiles + per - 1) / per : tiles;   // tiles of a workgroup: even shares
+#define L(RT_, NKB_, CT_, GLU_, ONE_, NT_)                                                                       \
+  w4row_k<RT_, NKB_, CT_, GLU_, ONE_, NT_><<<grid, ONE_ ? 64 * KS : 512, lds, st>>>(                             \
+      (const bf16*)X, ldx, codes, (const float2*)sc2, gs, (const bf16*)res, (bf16*)out, M, N, K)
+  if (one && glu) {
+    if (nkb == 4) L(1, 4, 2, true, true, 512);
+    else L(1, 2, 2, true, true, 1024);
+  } else if (one && RT == 1) {
+    if (nkb == 4) L(1, 4, 1, false, true, 512);
+    else L(1, 2, 1, false, true, 1024);
+  } else if (one) {
+    if (nkb == 4) L(2, 4, 1, false, true, 512);
+    else L(2, 2, 1, false, true, 1024);
+  } else if (nkb == 4) {
+    L(1, 4, 1, false, false, 512);
+  } else {
+    L(1, 2, 1, false, false, 512);
+  }
+#undef L
+  LIPA_CHECK_LAUNCH();
+  return true;
 }
 
 void launch_w4mm(const void* X, int ldx, const uint8_t* codes, const float* sc2, int gs, const void* res, void* out,

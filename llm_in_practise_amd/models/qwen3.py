@@ -35,7 +35,7 @@ from ..ops.norm import RMSNorm, rms_norm, rms_norm_residual
 from ..ops.rope import apply_rope, qk_norm_rope
 from ..parallel.tensor_parallel import tp_all_reduce
 from ..peft.lora import LoraLayer, base_of
-from ..quant.int4 import Int4Linear
+from ..quant.int4 import Int4Linear, Int4Weight, int4_swiglu
 from ..ops.embedding import Embedding
 from .common import CausalLMOutput, FusedProjection, KVCache, PackedPrefill, _leaf_linear, can_fuse, project
 
@@ -242,7 +242,8 @@ class Qwen3MLP(nn.Module):
                 (isinstance(m, LoraLayer) and not m.merged) or getattr(_leaf_linear(m), "_mlora", None) is not None
                 for m in (self.gate_proj, self.up_proj)):
             return None
-        return skinny_swiglu(x, self._gu.base)
+        base = self._gu.base
+        return int4_swiglu(x, base) if isinstance(base, Int4Weight) else skinny_swiglu(x, base)
 
     def forward(self, x, residual=None):
         tr = self.training

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from llm_in_practise_amd.quant.int4 import int4_linear, quantize_rtn
+from llm_in_practise_amd.quant.int4 import int4_linear, int4_swiglu, quantize_rtn
 from llm_in_practise_amd.quant.nf4 import dequantize_nf4, quantize_nf4
 
 pytestmark = pytest.mark.gpu
@@ -58,6 +58,27 @@ def test_w4g_decode_batches(native_ext, M, N, K, gs):
             continue
         y = native_ext.w4g(x, w.codes, w.w4mm_table(), N, gs, res, ks)
         assert y.shape == (M, N) and rel(y, want) < 1e-2, (ks, rel(y, want))
+
+
+@pytest.mark.parametrize("M", [3, 8, 12, 16])
+@pytest.mark.parametrize("N,K,gs", [(6144, 4096, 128), (24576, 4096, 128), (512, 1024, 256), (4096, 12288, 128), (768, 2560, 128),
+                                    (256, 384, 128), (256, 7680, 128)])
+def test_w4mm_one_launch_keeps_the_sums(native_ext, M, N, K, gs):
+    """All of K in one workgroup (x held by as many waves as slices, or slices in turns; even and ragged shares of tiles) against
+    64 bits, and the end in SwiGLU bit for bit the product and the activation."""
+    torch.manual_seed(M)
+    w = quantize_rtn(torch.randn(N, K, device=DEV), gs, False)
+    x, res = torch.randn(M, K, device=DEV).to(torch.bfloat16), torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    want = x.double() @ w.dequantize(torch.float32).double().t()
+    # the offset form sums 128 + q for q, so its float sums err with (136 |s|) sum |x|
+    big = 144 * w.scales.double().abs().max() * x.double().abs().sum(1, keepdim=True)
+    y = int4_linear(x, w)
+    assert ((y.double() - want).abs() <= (K / 128 + 132) * 2.0 ** -24 * big + 2.0 ** -8 * want.abs()).all()
+    wr = want + res.double()
+    assert ((int4_linear(x, w, residual=res).double() - wr).abs() <= (K / 128 + 132) * 2.0 ** -24 * big + 2.0 ** -8 * wr.abs()).all()
+    h = int4_swiglu(x, w)
+    assert h is None or torch.equal(h, native_ext.swiglu_fwd(y))
+    assert (h is not None) == (K in (4096, 1024, 2560))
 
 
 @pytest.mark.parametrize("N,K,gs,sym", [(256, 512, 128, False), (384, 1024, 64, True)])
