@@ -70,6 +70,9 @@ void launch_gemm4w_lora(const void*, int, const void*, int, const float*, const 
                         int, int, int, hipStream_t);
 void launch_gemm4w_loradx(const void*, int, const void*, int, const float*, const void*, void*, const LoraDx&, int, int,
                           int, int, int, hipStream_t);
+void launch_attn_fwd_packed(const void*, const void*, const void*, int, int, int, const int*, void*, int, int, int, int, int,
+                            float, hipStream_t);
+void launch_cache_rows(const void*, const void*, int, int, const int64_t*, void*, void*, int, int, int64_t, hipStream_t);
 void launch_attn_fwd(const void*, const void*, const void*, int, int, int, const int*, const int*, void*, float*, int,
                      int, int, int, int, int, int, int, float, float, uint64_t, hipStream_t);
 void launch_attn_bwd(const void*, const void*, const void*, const void*, const void*, const float*, const int*, int,
@@ -999,6 +1002,44 @@ std::vector<Tensor> attn_fwd_ext(Tensor q, Tensor k, Tensor v, optional<Tensor> 
   return {o, lse};
 }
 
+// Causal attention of prompts packed back to back: q [T, hq*128], k / v [T, hkv*128], off int32 [B + 1] (each prompt's first
+// token, then T), lengths up to S.
+Tensor attn_fwd_packed(Tensor q, Tensor k, Tensor v, Tensor off, int64_t S, int64_t hq, int64_t hkv, double scale) {
+  const int64_t T = q.size(0), B = off.numel() - 1;
+  TORCH_CHECK(hkv > 0 && hq % hkv == 0, "attn: GQA group");
+  TORCH_CHECK(T > 0 && B > 0 && S > 0 && S <= T && off.is_contiguous() && off.scalar_type() == at::kInt &&
+                  off.device() == q.device(), "attn: packed offsets int32 [B + 1] on the device");
+  TORCH_CHECK(((B * hkv + 7) / 8) * 8 * (hq / hkv) * ((S + 127) / 128) < (1ll << 31), "attn: packed grid");
+  attn_check(q, T, hq, 128, "q");
+  attn_check(k, T, hkv, 128, "k");
+  attn_check(v, T, hkv, 128, "v");
+  auto o = at::empty({T, hq * 128}, q.options());
+  launch_attn_fwd_packed(q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0),
+                         off.data_ptr<int>(), o.data_ptr(), T, B, S, hq, hkv, scale, stream());
+  return o;
+}
+
+// k / v rows [T, W] into rows idx of the caches [rows, W]
+void cache_rows(Tensor k, Tensor v, Tensor idx, Tensor kc, Tensor vc) {
+  const int64_t T = k.size(0), W = kc.size(-1), rows = W > 0 ? kc.numel() / W : 0;
+  for (const Tensor* t : {&k, &v, &kc, &vc}) {
+    CHECK_CUDA((*t));
+    CHECK_BF16((*t));
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "cache_rows: 16-byte aligned rows");
+  }
+  CHECK_CONTIG(kc);
+  CHECK_CONTIG(vc);
+  CHECK_CONTIG(idx);
+  TORCH_CHECK(k.dim() == 2 && v.dim() == 2 && v.size(0) == T && k.size(1) == W && v.size(1) == W && W % 8 == 0 &&
+                  k.stride(1) == 1 && v.stride(1) == 1 && k.stride(0) % 8 == 0 && v.stride(0) % 8 == 0 &&
+                  kc.sizes() == vc.sizes(), "cache_rows: k / v [T, W] rows for caches of W columns");
+  TORCH_CHECK(idx.scalar_type() == at::kLong && idx.numel() == T && idx.device() == k.device(), "cache_rows: idx int64 [T]");
+  TORCH_CHECK(T * (W / 8) < (1ll << 31) && k.stride(0) < (1ll << 31) && v.stride(0) < (1ll << 31), "cache_rows: size");
+  if (T == 0) return;
+  launch_cache_rows(k.data_ptr(), v.data_ptr(), k.stride(0), v.stride(0), idx.data_ptr<int64_t>(), kc.data_ptr(),
+                    vc.data_ptr(), T, W, rows, stream());
+}
+
 std::vector<Tensor> attn_fwd(Tensor q, Tensor k, Tensor v, optional<Tensor> kv_lens, int64_t B, int64_t S, int64_t hq,
                              int64_t hkv, int64_t d, bool causal, double scale) {
   return attn_fwd_ext(q, k, v, kv_lens, c10::nullopt, B, S, S, S, hq, hkv, d, causal, scale, 0.0, 0);
@@ -1757,6 +1798,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("f_w4") = 0, py::arg("want_gu") = true, py::arg("want_h") = true);
   m.def("mlora_apply", &mlora_apply);
   m.def("gemm4w_dswiglu", &gemm4w_dswiglu, py::arg("dy"), py::arg("w"), py::arg("gu"), py::arg("wscale") = py::none());
+  m.def("attn_fwd_packed", &attn_fwd_packed);
+  m.def("cache_rows", &cache_rows);
   m.def("attn_fwd", &attn_fwd);
   m.def("attn_fwd_ext", &attn_fwd_ext);
   m.def("attn_bwd", &attn_bwd);

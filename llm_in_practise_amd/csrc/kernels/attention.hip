@@ -369,7 +369,11 @@ __device__ __forceinline__ void attn_dma16(const rsrc_t& rs, uint32_t m0v, uint3
       : "memory");
 }
 
-template <bool DROP>
+// VAR: prompts packed back to back, kv_lens = the offsets [B + 1] of their first tokens in the kv_rows rows of Q, K, V and O; Sq and
+// Skv bound the lengths.  The grid is flat: block id % 8 is its XCD, which takes every 8th (prompt, kv head) with all its query
+// heads, long blocks first, so that each XCD's L2 holds few keys and a long prompt is spread over all of them.  Six prompts of 2451 tokens,
+// longest 1023, 32 heads over 8: 29 µs, where the padded form takes 64 and its copies 75.
+template <bool DROP, bool VAR>
 __global__ __launch_bounds__(256, 2) void attn_fwd128_k(const bf16* __restrict__ Q, const bf16* __restrict__ K,
                                                      const bf16* __restrict__ V, int ldq, int ldk, int ldv,
                                                      const int* __restrict__ kv_lens, const int* __restrict__ q_offs,
@@ -379,16 +383,28 @@ __global__ __launch_bounds__(256, 2) void attn_fwd128_k(const bf16* __restrict__
   constexpr int D = 128, TB = 64 * 256;   // bytes per K or V tile image
   __shared__ __attribute__((aligned(16))) char smem[4 * TB];   // K0 V0 K1 V1
   const int nqb = (Sq + 127) / 128;
-  int i0, h, b;
-  xcd_grid3_lpt(i0, h, b, causal >> 1);
+  int i0, h, b, row0 = 0;
+  if constexpr (VAR) {
+    const int G = hq / hkv, groups = (Skv * hkv + 7) / 8;            // (Skv: the prompts, until it is their tokens)
+    const int x = blockIdx.x & 7, s = blockIdx.x >> 3, t = s % (groups * G), p = t / G * 8 + x;
+    if (p >= Skv * hkv) return;
+    i0 = s / (groups * G);
+    b = p / hkv;
+    h = p % hkv * G + t % G;
+    row0 = min(max(kv_lens[b], 0), kv_rows);
+    Sq = Skv = min(max(kv_lens[b + 1], row0), kv_rows) - row0;       // this prompt's tokens
+    if ((nqb - 1 - i0) * 128 >= Sq) return;
+  } else {
+    xcd_grid3_lpt(i0, h, b, causal >> 1);
+  }
   const int qb = nqb - 1 - i0;   // heavy (late, causal) blocks first
   const int hk = h / (hq / hkv);
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, r32 = lane & 31, hi = lane >> 5;
   const int q0w = qb * 128 + 32 * w;   // this wave's first query
   const int qa = q0w + r32;            // this lane's query
-  const int qoff = q_offs ? q_offs[b] : 0;
-  const int kvlen = min(kv_lens ? kv_lens[b] : Skv, Skv);
-  const size_t tok0 = (size_t)b * Sq, ktok0 = (size_t)b * kv_rows;
+  const int qoff = !VAR && q_offs ? q_offs[b] : 0;
+  const int kvlen = min(!VAR && kv_lens ? kv_lens[b] : Skv, Skv);
+  const size_t tok0 = VAR ? row0 : (size_t)b * Sq, ktok0 = VAR ? row0 : (size_t)b * kv_rows;
 
   // Q as the B operand of Sᵀ = K·Qᵀ: lane (q, hi) holds Q[q][16ds + 8hi + j]
   bf16x8 qf[8];
@@ -556,7 +572,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd128_k(const bf16* __restrict__
         *reinterpret_cast<bf16x8*>(orow + 32 * dt + 16 * hf) =
             bf16x8{(bf16)a[0], (bf16)a[1], (bf16)a[2], (bf16)a[3], (bf16)c[0], (bf16)c[1], (bf16)c[2], (bf16)c[3]};
     }
-  if (hi == 0 && qa < Sq)
+  if (!VAR && hi == 0 && qa < Sq)
     lse[((size_t)b * hq + h) * Sq + qa] = lt > 0.f ? (m_run * scale_log2 + log2f(lt)) * 0.6931471805599453f : INFINITY;
 }
 
@@ -1461,7 +1477,7 @@ void launch_attn_fwd(const void* q, const void* k, const void* v, int ldq, int l
   const float sl2 = scale * LOG2E;
   if (D == 128) {   // the 32x32x16 form with LDS-DMA K / V tiles (attn_fwd128_k); other head dims: attn_fwd_k
 #define F128(DR)                                                                                              \
-  attn_fwd128_k<DR><<<grid, blk, 0, st>>>((const bf16*)q, (const bf16*)k, (const bf16*)v, ldq, ldk, ldv, kv_lens, \
+  attn_fwd128_k<DR, false><<<grid, blk, 0, st>>>((const bf16*)q, (const bf16*)k, (const bf16*)v, ldq, ldk, ldv, kv_lens, \
                                           q_offs, (bf16*)o, lse, Sq, Skv, kv_rows, hq, hkv,                    \
                                           causal ? 1 | (attn_lpt() << 1) : 0, sl2, dp)
     if (dp.thresh) F128(true); else F128(false);
@@ -1475,6 +1491,37 @@ void launch_attn_fwd(const void* q, const void* k, const void* v, int ldq, int l
                                                 kv_rows, hq, hkv, causal ? 1 | (attn_lpt() << 1) : 0, sl2, dp)
   LIPA_ATTN_D3(D, FWD(1, 2));
 #undef FWD
+  LIPA_CHECK_LAUNCH();
+}
+
+// Causal attention of prompts packed back to back (head dim 128); off [B + 1], lengths up to S.
+void launch_attn_fwd_packed(const void* q, const void* k, const void* v, int ldq, int ldk, int ldv, const int* off, void* o,
+                            int T, int B, int S, int hq, int hkv, float scale, hipStream_t st) {
+  const int nqb = (S + 127) / 128, groups = (B * hkv + 7) / 8;
+  attn_fwd128_k<false, true><<<8 * groups * (hq / hkv) * nqb, 256, 0, st>>>(
+      (const bf16*)q, (const bf16*)k, (const bf16*)v, ldq, ldk, ldv, off, nullptr, (bf16*)o, nullptr, S, B, T, hq, hkv, 1,
+      scale * LOG2E, DropParams{});
+  LIPA_CHECK_LAUNCH();
+}
+
+// K and V rows of a prefill into their cache rows: 16 bytes a thread, both in one launch.
+__global__ __launch_bounds__(256) void cache_rows_k(const bf16* __restrict__ k, const bf16* __restrict__ v, int ldk, int ldv,
+                                                    const int64_t* __restrict__ idx, bf16* __restrict__ kc,
+                                                    bf16* __restrict__ vc, int T, int W, int64_t rows) {
+  const int cw = W / 8, i = blockIdx.x * 256 + threadIdx.x, t = i / cw, c = i % cw;
+  if (t >= T) return;
+  const int64_t r = idx[t];
+  if (r < 0 || r >= rows) return;
+  const u32x4 a = *reinterpret_cast<const u32x4*>(k + (size_t)t * ldk + 8 * c);
+  const u32x4 b = *reinterpret_cast<const u32x4*>(v + (size_t)t * ldv + 8 * c);
+  *reinterpret_cast<u32x4*>(kc + (size_t)r * W + 8 * c) = a;
+  *reinterpret_cast<u32x4*>(vc + (size_t)r * W + 8 * c) = b;
+}
+
+void launch_cache_rows(const void* k, const void* v, int ldk, int ldv, const int64_t* idx, void* kc, void* vc, int T, int W,
+                       int64_t rows, hipStream_t st) {
+  const unsigned blocks = (unsigned)(((int64_t)T * (W / 8) + 255) / 256);
+  cache_rows_k<<<blocks, 256, 0, st>>>((const bf16*)k, (const bf16*)v, ldk, ldv, idx, (bf16*)kc, (bf16*)vc, T, W, rows);
   LIPA_CHECK_LAUNCH();
 }
 

@@ -3,11 +3,13 @@ from __future__ import annotations
 
 import dataclasses
 import functools
+import itertools
 
 import torch
 import torch.nn as nn
 
 from ..ops.activation import softcap
+from ..ops.attention import flash_attention, packed_attention, write_cache_rows
 from ..ops.gemm import matmul_f32
 from ..ops.linear import LoraBranch, fused_linear
 from ..peft.lora import Linear4bit, LoraLayer, base_of
@@ -187,9 +189,9 @@ class PackedPrefill:
     """Prefill of several prompts packed back to back — ``[1, T]`` tokens, no padding — straight
     into their KV-cache slots (the serving engine's admission path).
 
-    Every token-wise op (projections, norms, SwiGLU: nearly all prefill FLOPs) runs on the
-    packed tokens only; attention scatters q/k/v into a right-padded ``[B, S]`` view for the
-    flash kernel (causal, per-row ``kv_lens``) and gathers the valid rows back, and each
+    Every token-wise op (projections, norms, SwiGLU: nearly all prefill FLOPs) and, at head_dim 128 on
+    the GPU, attention runs on the packed tokens only; elsewhere attention scatters q/k/v into a
+    right-padded ``[B, S]`` view (causal, per-row ``kv_lens``) and gathers the valid rows back.  Each
     layer's K/V rows are written into the cache slots with one indexed copy.  Against padding
     every prompt to the longest one this removes the padded GEMM work (≈ 40 % on chat-length
     prompts) and the scratch-cache → slot copy."""
@@ -200,17 +202,26 @@ class PackedPrefill:
         tb = torch.cat([torch.full((n,), b, dtype=torch.long) for b, n in enumerate(lens)])
         tp = torch.cat([torch.arange(n, dtype=torch.long) for n in lens])
         sl = torch.tensor(slots, dtype=torch.long)
+        if any(s < 0 or s * cache.max_len + n > cache.batch * cache.max_len for s, n in zip(slots, lens)):
+            raise IndexError(f"slots {slots} of {lens} tokens pass the cache's {cache.batch} rows of {cache.max_len}")
         self.positions = tp.to(device)[None]
-        self.pad_idx = (tb * self.S + tp).to(device)
+        self._pad = tb * self.S + tp
         self.cache_idx = (sl[tb] * cache.max_len + tp).to(device)
+        self.off = torch.tensor([0, *itertools.accumulate(lens)], dtype=torch.int32, device=device)
         self.kv_lens = torch.tensor(lens, dtype=torch.int32, device=device)
         self.last = (torch.cumsum(torch.tensor(lens), 0) - 1).to(device)
 
+    @functools.cached_property
+    def pad_idx(self) -> torch.Tensor:
+        return self._pad.to(self.cache_idx.device)
+
     def attend(self, layer: int, q, k, v, hq: int, hkv: int, d: int, attention_fn):
-        self.cache.k[layer].view(-1, hkv * d).index_copy_(0, self.cache_idx, k)
-        self.cache.v[layer].view(-1, hkv * d).index_copy_(0, self.cache_idx, v)
+        write_cache_rows(self.cache.k[layer], self.cache.v[layer], self.cache_idx, k, v)
         if self.B == 1:
             return attention_fn(q, k, v, 1, self.S, hq, hkv, d, causal=True, kv_lens=None)
+        o = packed_attention(q, k, v, self.off, self.S, hq, hkv, d) if attention_fn is flash_attention else None
+        if o is not None:
+            return o
         n = self.B * self.S
 
         def pad(t):

@@ -1058,3 +1058,33 @@ def test_mlora_apply_per_row_adapter(native_ext):
     base_rows = ids == 0
     assert torch.equal(y[base_rows].float(), want[base_rows])           # base rows untouched
     assert torch.equal(y[:, :c0].float(), want[:, :c0])                 # other columns untouched
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (32, 8), (5, 5), (12, 3)])
+@pytest.mark.parametrize("lens", [[1, 64, 65], [129, 1, 128, 127, 300, 33, 31, 32, 5], [700, 37], [256] * 3])
+def test_packed_attention_matches_padded(native_ext, hq, hkv, lens):
+    """Prompts packed back to back: bit for bit the right-padded form (v a strided view of the fused projection), and the cache
+    rows of K and V."""
+    from llm_in_practise_amd.models.common import KVCache
+    from llm_in_practise_amd.ops.attention import flash_attention, packed_attention
+    torch.manual_seed(sum(lens))
+    T, d = sum(lens), 128
+    q, k = torch.randn(T, hq * d, device=DEV).bfloat16(), torch.randn(T, hkv * d, device=DEV).bfloat16()
+    v = torch.randn(T, (hq + 2 * hkv) * d, device=DEV).bfloat16()[:, (hq + hkv) * d:]
+    B, S = len(lens), max(lens)
+    cache = KVCache(1, B + 2, S + 3, hkv, d, torch.bfloat16, DEV)
+    slots = list(range(B + 1, 1, -1))
+    pp = cache.packed(slots, lens)
+    assert packed_attention(q, k, v, pp.off, pp.S, hq, hkv, d) is not None
+    with torch.no_grad():
+        got = pp.attend(0, q, k, v, hq, hkv, d, flash_attention)
+        want = pp.attend(0, q, k, v, hq, hkv, d, lambda *a, **kw: flash_attention(*a, **kw))      # (another function: padded)
+    assert torch.equal(got, want)
+    t = 0
+    for s, n in zip(slots, lens):
+        assert torch.equal(cache.k[0][s, :n], k[t:t + n]) and torch.equal(cache.v[0][s, :n], v[t:t + n])
+        assert not cache.k[0][s, n:].any() and not cache.v[0][s, n:].any()
+        t += n
+    assert not cache.k[0][:2].any()
+    with pytest.raises(IndexError):
+        cache.packed([B + 1], [S + 4])
