@@ -147,6 +147,28 @@ G4wCfg gemm4w_cfg(int M, int N, int K, bool bt, int bn_req, int sp_req, int bm_r
     }
   }
   if (sp_req > 0) best.splits = std::min(sp_req, 8);
+  if (w4) return best;
+  // The tile again for those splits (they fix the order of a product's sums, the tile does not), at what the tiles take over
+  // several rounds: the 128-high ones 0.62 of the 256-high, the 128-wide ones 0.97 µs a K-tile, and 6 µs a round to fill and empty it.  Of 216
+  // shapes of 256 .. 8192 rows none gets slower by more than 2 %; 4700 rows of 24576 × 4096 894 → 775 µs, 2451 of
+  // 4096 × 12288 (4 splits) 291 → 272, 700 of it (8) 112 → 100.
+  best_t = 1e30;
+  const int s = best.splits;
+  for (int bm : {256, 128}) {
+    if (bm_req && bm != bm_req) continue;
+    for (int bn : {256, 192, 128}) {
+      if (bn == 192 && bt && bm != 256) continue;
+      if (bn_req > 0 ? bn != bn_req : bn_req < 0 && bn == 192) continue;
+      double kt_us = bn == 256 ? (bt ? 1.52 : 1.5) : bn == 192 ? (bt ? 1.24 : 1.22) : 0.97;
+      if (bm == 128) kt_us *= 0.62;
+      const double t = (double)((tiles_of(M, N, bm, bn) * s + 255) / 256) * ((nk + s - 1) / s * kt_us + 6.0);
+      if (t < best_t - 1e-9) {
+        best_t = t;
+        best.bm = bm;
+        best.bn = bn;
+      }
+    }
+  }
   return best;
 }
 
