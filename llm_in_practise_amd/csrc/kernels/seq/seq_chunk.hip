@@ -11,8 +11,8 @@
 // numbers, which hold its 24 bits: three products with float sums, at five times the rate of the float matrix units.  Log
 // decays are summed in 64 bits and kept as two floats, so that the difference of two large sums is exact.
 //
-// Measured, token by token -> chunks: state space, one prompt of 4093 tokens, 64 heads of 128 x 64: 2344 -> 154 us (state 56,
-// walk 24, outputs 78); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 94 us (40, 18, 39).  Error against
+// Measured, token by token -> chunks: state space, one prompt of 4093 tokens, 64 heads of 128 x 64: 2344 -> 144 us (state 45,
+// walk 24, outputs 78); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 92 us (38, 18, 38).  Error against
 // 64 bits 1.5e-7 -> 1.0e-7 and 4.8e-7 -> 2.0e-7: fewer roundings stand between a token and the outputs far behind it.
 // Chunks of 128 tokens: the states of a step pass through memory once per chunk (69 MB of the first case, three times), and a
 // chunk's scores grow with its square.
@@ -156,9 +156,11 @@ __device__ __forceinline__ void load_4x4(const bf16* __restrict__ p, size_t ld, 
 __device__ __forceinline__ int c_row(int i, int half) { return (i & 3) + 8 * (i >> 2) + 4 * half; }   // 32x32 tile: row of register i
 
 // (1) U[slot, head, dv, dk] = sum_j w_j v_j k_j^T over a chunk, w_j = e^{F_C - F_j} c_j (mLSTM: against the chunk's largest),
-// for 64 value columns.  Bound by splitting the weighted values (once per element, into LDS) and the products, about equal.
+// for 64 value columns.  Bound by latency: a wave of a SIMD's three waits in turn for the gates, k and v, and the LDS, so the loads
+// stand before the gates and the second half's before the first half's products (56 -> 45 us for 4093 tokens of 64 heads, with
+// the registers held to three workgroups a CU; 40 -> 38 for the mLSTM's).
 template <int NK, bool MLSTM>
-__global__ __launch_bounds__(256) void k_chunk_state(const bf16* __restrict__ k, int ldk, const bf16* __restrict__ v,
+__global__ __launch_bounds__(256, 3) void k_chunk_state(const bf16* __restrict__ k, int ldk, const bf16* __restrict__ v,
                                                      int ldv, GateArgs ga, float* __restrict__ U, float* __restrict__ NU,
                                                      double* __restrict__ meta, int H, int G, int dv, SeqDesc d) {
   constexpr int DK = 32 * NK;
@@ -171,6 +173,20 @@ __global__ __launch_bounds__(256) void k_chunk_state(const bf16* __restrict__ k,
   if (!find_chunk(d, slot, c)) return;
   const int w = tid >> 6, lane = tid & 63, l32 = lane & 31, half = lane >> 5, kh = hd / (H / G);
   const size_t cell = (size_t)slot * H + hd;
+  const bf16* kp = k + (size_t)c.t0 * ldk + kh * DK;
+  const bf16* vp = v + (size_t)c.t0 * ldv + (size_t)hd * dv + cb;
+  constexpr int KL = (DK / 4 * 16 + 255) / 256;
+  bf16x4 rk[KL][4], rv[4];
+  const int c4 = tid & 15, vt = tid >> 4;
+  auto load = [&](int j0) {                    // (the second half over the products of the first)
+#pragma unroll
+    for (int i = 0; i < KL; ++i) {
+      const int e = tid + 256 * i, d4 = e % (DK / 4), t4 = j0 + 4 * (e / (DK / 4));
+      load_4x4(kp + (size_t)t4 * ldk + 4 * d4, ldk, c.n - t4, e < DK / 4 * 16, rk[i]);
+    }
+    load_4x4(vp + (size_t)(j0 + 4 * vt) * ldv + 4 * c4, ldv, c.n - j0 - 4 * vt, cb + 4 * c4 < dv, rv);
+  };
+  load(0);
   if (w == 0) {
     const Gate g = gates<MLSTM>(ga, c, hd, lane);
     double top = 0.0, add = g.Fc;
@@ -193,20 +209,10 @@ __global__ __launch_bounds__(256) void k_chunk_state(const bf16* __restrict__ k,
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
   float nsum = 0.f;
-  const bf16* kp = k + (size_t)c.t0 * ldk + kh * DK;
-  const bf16* vp = v + (size_t)c.t0 * ldv + (size_t)hd * dv + cb;
   for (int j0 = 0; j0 < c.n; j0 += 64) {
-    bf16x4 rk[(DK / 4 * 16 + 255) / 256][4], rv[4];
-#pragma unroll
-    for (int i = 0; i < (DK / 4 * 16 + 255) / 256; ++i) {
-      const int e = tid + 256 * i, d4 = e % (DK / 4), t4 = j0 + 4 * (e / (DK / 4));
-      load_4x4(kp + (size_t)t4 * ldk + 4 * d4, ldk, c.n - t4, e < DK / 4 * 16, rk[i]);
-    }
-    const int c4 = tid & 15, vt = tid >> 4;
-    load_4x4(vp + (size_t)(j0 + 4 * vt) * ldv + 4 * c4, ldv, c.n - j0 - 4 * vt, cb + 4 * c4 < dv, rv);
     __syncthreads();                           // the last turn's reads are done; the weights stand
 #pragma unroll
-    for (int i = 0; i < (DK / 4 * 16 + 255) / 256; ++i) {
+    for (int i = 0; i < KL; ++i) {
       const int e = tid + 256 * i, d4 = e % (DK / 4), t4 = e / (DK / 4);
       if (e < DK / 4 * 16)
 #pragma unroll
@@ -229,6 +235,7 @@ __global__ __launch_bounds__(256) void k_chunk_state(const bf16* __restrict__ k,
       *reinterpret_cast<bf16x4*>(row + 64 * KP) = m;
       *reinterpret_cast<bf16x4*>(row + 2 * 64 * KP) = l;
     }
+    if (j0 + 64 < c.n) load(j0 + 64);
     __syncthreads();
     const int vrow = (w & 1) * 32 + l32;
     if (cb + (w & 1) * 32 < dv) {
