@@ -351,8 +351,9 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
 }
 
 // One workgroup per (sequence, head): a lane takes a split's maximum and weight, then every thread sums its column, in the order of
-// the splits, with the loads of eight in flight.  (With the splits' maxima, weights and columns as one dependent chain a merge of 30 splits took 10.5 µs.)
-template <int D>
+// the splits.  Bound by latency: the first NP partial rows, maxima and sums are loaded before the length says which of them count.
+// 30 splits of one row: 4.35 µs (10.5 as one dependent chain of maxima, weights and columns, 5.2 behind the length).
+template <int D, int NP>
 __global__ __launch_bounds__(D) void decode_attn_merge2_k(const float* __restrict__ opart,
                                                           const float* __restrict__ mpart,
                                                           const float* __restrict__ lpart,
@@ -362,28 +363,35 @@ __global__ __launch_bounds__(D) void decode_attn_merge2_k(const float* __restric
   __shared__ float scratch[D / 64];
   const size_t h = blockIdx.x;  // b*hq + head
   const int d = threadIdx.x;
+  const float* op = opart + h * nsplit * D + d;
+  float v[NP];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) v[j] = op[(size_t)min(j, nsplit - 1) * D];
+  const float m0 = mpart[h * nsplit + min(d, nsplit - 1)], l0 = lpart[h * nsplit + min(d, nsplit - 1)];
   const int len = (int)pos[h / hq] + 1;
   const int chunk = split_chunk32(len, nsplit);
   const int nv = min(nsplit, (len + chunk - 1) / chunk);
-  float m = -INFINITY;
-  for (int s = d; s < nv; s += D) m = fmaxf(m, mpart[h * nsplit + s]);
+  float m = d < nv ? m0 : -INFINITY;
+  for (int s = d + D; s < nv; s += D) m = fmaxf(m, mpart[h * nsplit + s]);
   const float M = block_max<D / 64>(m, scratch);
   for (int s = d; s < nv; s += D) {
-    sc[s] = __expf(mpart[h * nsplit + s] - M);
-    sc[nsplit + s] = lpart[h * nsplit + s];
+    sc[s] = __expf((s == d ? m0 : mpart[h * nsplit + s]) - M);
+    sc[nsplit + s] = s == d ? l0 : lpart[h * nsplit + s];
   }
   __syncthreads();
   float L = 0.f;
   for (int s = 0; s < nv; ++s) L += sc[nsplit + s] * sc[s];
   float A = 0.f;
-  const float* op = opart + h * nsplit * D + d;
-  int s = 0;
+#pragma unroll
+  for (int j = 0; j < NP; ++j)
+    if (j < nv) A += v[j] * sc[j];
+  int s = NP;
   for (; s + 8 <= nv; s += 8) {
-    float v[8];
+    float u[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = op[(size_t)(s + j) * D];
+    for (int j = 0; j < 8; ++j) u[j] = op[(size_t)(s + j) * D];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) A += v[j] * sc[s + j];
+    for (int j = 0; j < 8; ++j) A += u[j] * sc[s + j];
   }
   for (; s < nv; ++s) A += op[(size_t)s * D] * sc[s];
   out[h * D + d] = (bf16)(L > 0.f ? A / L : 0.f);
@@ -565,13 +573,16 @@ void launch_decode_attention2(const void* q, int ldq, const void* knew, int ldkn
                               int Smax, int hq, int hkv, int d, int nsplit, float scale, hipStream_t st) {
   dim3 grid(nsplit, hkv, B);
   const float sl2 = scale * 1.4426950408889634f;
+#define M(D_, NP_) \
+  decode_attn_merge2_k<D_, NP_><<<B * hq, D_, 2 * nsplit * sizeof(float), st>>>(opart, mpart, lpart, pos, (bf16*)out, hq, nsplit)
 #define P(D_)                                                                                                          \
   decode_attn_mfma_k<D_><<<grid, 256, 0, st>>>((const bf16*)q, ldq, (const bf16*)knew, ldkn, (const bf16*)vnew, ldvn, \
                                                (bf16*)kc, (bf16*)vc, pos, opart, mpart, lpart, Smax, hq, hkv, nsplit, \
                                                sl2);                                                                   \
-  decode_attn_merge2_k<D_><<<B * hq, D_, 2 * nsplit * sizeof(float), st>>>(opart, mpart, lpart, pos, (bf16*)out, hq, nsplit)
+  if (nsplit > 8) M(D_, 32); else if (nsplit > 4) M(D_, 8); else M(D_, 4)
   if (d == 128) { P(128); } else { P(64); }
 #undef P
+#undef M
   LIPA_CHECK_LAUNCH();
 }
 
