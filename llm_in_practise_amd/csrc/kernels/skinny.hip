@@ -16,9 +16,9 @@ using namespace lipa;
 
 namespace {
 
-// CUT: S pieces of kc, each with its own sum (red: S tiles); else units of 64 in turns, a sum per wave (red: NW tiles).
+// CUT: S pieces of kc, each with its own sum (red: S tiles); else units of UNIT in turns, a sum per wave (red: NW tiles).
 // B: 32-deep steps per batch; FULL: every piece is whole batches.
-template <int CT, int MT, int NW, int B, bool GLU, bool CUT, bool FULL>
+template <int CT, int MT, int NW, int B, bool GLU, bool CUT, bool FULL, int UNIT>
 __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W,
                                                          const bf16* __restrict__ res, bf16* __restrict__ out, int M, int N,
                                                          int K, int S) {
@@ -51,14 +51,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict_
     bf16x8 a[B][CT], b[B][MT];
   };
   // steps of one piece (of the whole wave, if not CUT), batches of one piece, batches of this wave
-  const int kc = CUT ? K / S : K, steps = CUT ? kc / 32 : 2 * ((K / 64 - w + NW - 1) / NW), per = (steps + B - 1) / B;
+  const int kc = CUT ? K / S : K, steps = CUT ? kc / 32 : UNIT / 32 * ((K / UNIT - w + NW - 1) / NW), per = (steps + B - 1) / B;
   const int nb = CUT ? (S - w + NW - 1) / NW * per : per;
   int lp = w, lb = 0;                            // the next batch to load: its piece, its place in it
   auto load = [&](Batch& s) {
 #pragma unroll
     for (int u = 0; u < B; ++u) {
       const int e = FULL ? lb * B + u : min(lb * B + u, steps - 1);
-      const int k = CUT ? lp * kc + 32 * e : 64 * (w + NW * (e >> 1)) + 32 * (e & 1);
+      const int k = CUT ? lp * kc + 32 * e : UNIT * (w + NW * (e / (UNIT / 32))) + 32 * (e % (UNIT / 32));
 #pragma unroll
       for (int t = 0; t < CT; ++t) s.a[u][t] = *reinterpret_cast<const bf16x8*>(wr[t] + k);
 #pragma unroll
@@ -142,28 +142,31 @@ static int skinny_splits(int N, int K) {
 // Column tiles and waves per workgroup, us at 1 / 8 / 16 rows: two tiles of 8 waves take 13.2 / 13.9 / 15.1 for 6144 x 4096 (one tile
 // of 4 waves 13.7 / 15.5 / 17.5) and 9.7 / 10.8 / 12.3 for 6144 x 2560 (10.7 / 12.3 / 14.4), but 4096 rows of W fill half the CUs with
 // them: 11.9 / 13.2 / 14.9 for K = 4096 against 9.0 / 9.7 / 10.9.  The gated form pairs 16 gate with 16 up rows: 38.2 / 39.4 / 44.0
-// for 2 x 12288 x 4096, 5.3 TB/s.  Batches of 5 steps where the pieces divide by them (2560: whole batches 9.7, partial ones 11.8).
+// for 2 x 12288 x 4096, 5.3 TB/s, with 4 waves of 64-deep units (2 of 128: 46 / 46 / 48), but 61 / 65 / 73 for 2 x 13824 x 5120 with 2 of
+// 128 (64 / 70 / 79), which are even at 2 x 9728 x 2560 (24): the orders of sums that the library's products have for those K.  Batches of 5 steps where the pieces divide by them (2560: whole batches 9.7, partial ones 11.8).
 void launch_gemm_skinny(const void* X, int ldx, const void* W, const void* res, void* out, int M, int N, int K, bool glu,
                         hipStream_t st) {
-  const int S = skinny_splits(N, K);             // (one tile of 1 KB of LDS each: up to 32)
-  const bool cut = S <= 32 && M <= 16 && !glu;
-#define L(CT_, MT_, NW_, B_, GLU_, CUT_, FULL_)                                                                             \
-  gemm_skinny_k<CT_, MT_, NW_, B_, GLU_, CUT_, FULL_>                                                                       \
-      <<<(N + 16 * (GLU_ ? CT_ / 2 : CT_) - 1) / (16 * (GLU_ ? CT_ / 2 : CT_)), 64 * NW_, (CUT_ ? S : NW_) * CT_ * MT_ * 1024, \
-         st>>>((const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, S)
-#define LM(CT_, NW_, B_, GLU_)                                                                 \
-  do {                                                                                         \
-    if (cut && (K / S) % (32 * B_) == 0) L(CT_, 1, NW_, B_, GLU_, !GLU_, true);                \
-    else if (cut && (K / S) % 160 == 0) L(CT_, 1, NW_, 5, GLU_, !GLU_, true);                  \
-    else if (cut) L(CT_, 1, NW_, 4, GLU_, !GLU_, false);                                       \
-    else if (M <= 16 && K % (32 * B_ * NW_) == 0) L(CT_, 1, NW_, B_, GLU_, false, true);       \
-    else if (M <= 16) L(CT_, 1, NW_, 4, GLU_, false, false);                                   \
-    else if (M <= 32) L(CT_, 2, NW_, 4, GLU_, false, false);                                   \
-    else L(CT_, 4, NW_, 4, GLU_, false, false);                                                \
+  const int pieces = skinny_splits(N, K);        // (one tile of 1 KB of LDS each: up to 32)
+  const bool cut = pieces <= 32 && M <= 16 && !glu;
+#define L(CT_, MT_, NW_, B_, GLU_, CUT_, FULL_, UNIT_)                                                                          \
+  gemm_skinny_k<CT_, MT_, NW_, B_, GLU_, CUT_, FULL_, UNIT_>                                                                       \
+      <<<(N + 16 * (GLU_ ? CT_ / 2 : CT_) - 1) / (16 * (GLU_ ? CT_ / 2 : CT_)), 64 * NW_, (CUT_ ? pieces : NW_) * CT_ * MT_ * 1024, \
+         st>>>((const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, pieces)
+#define LM(CT_, NW_, B_, GLU_, UNIT_)                                                                \
+  do {                                                                                               \
+    const int kc = K / pieces;                                                                       \
+    if (cut && kc % (32 * B_) == 0) L(CT_, 1, NW_, B_, GLU_, !GLU_, true, UNIT_);                   \
+    else if (cut && kc % 160 == 0) L(CT_, 1, NW_, 5, GLU_, !GLU_, true, UNIT_);                     \
+    else if (cut) L(CT_, 1, NW_, 4, GLU_, !GLU_, false, UNIT_);                                     \
+    else if (M <= 16 && K % (UNIT_ * NW_) == 0 && K % (32 * B_ * NW_) == 0) L(CT_, 1, NW_, B_, GLU_, false, true, UNIT_); \
+    else if (M <= 16) L(CT_, 1, NW_, 4, GLU_, false, false, UNIT_);                                  \
+    else if (M <= 32) L(CT_, 2, NW_, 4, GLU_, false, false, UNIT_);                                  \
+    else L(CT_, 4, NW_, 4, GLU_, false, false, UNIT_);                                               \
   } while (0)
-  if (glu) LM(2, 4, 4, true);
-  else if (N >= 6144) LM(2, 8, 4, false);
-  else LM(1, 4, 8, false);
+  if (glu && (K % 1024 || K > 4096) && K % 128 == 0) LM(2, 2, 4, true, 128);
+  else if (glu) LM(2, 4, 4, true, 64);
+  else if (N >= 6144) LM(2, 8, 4, false, 64);
+  else LM(1, 4, 8, false, 64);
 #undef LM
 #undef L
   LIPA_CHECK_LAUNCH();
