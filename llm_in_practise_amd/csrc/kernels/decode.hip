@@ -196,6 +196,11 @@ __device__ __forceinline__ bf16x4 dec_tr_read(const bf16* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p));
 }
 __device__ __forceinline__ int split_chunk32(int len, int nsplit) { return ((len + nsplit - 1) / nsplit + 31) & ~31; }
+// x as the float it is rounded to: the compiler fuses no product with a sum across this
+__device__ __forceinline__ float rounded(float x) {
+  asm("" : "+v"(x));
+  return x;
+}
 
 template <int D>
 __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict__ q, int ldq,
@@ -338,8 +343,9 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
 #pragma unroll
     for (int s2 = 0; s2 < 4; ++s2) {
       const float c = __builtin_amdgcn_exp2f(sm[s2][hh] - M);   // -inf (idle wave) → 0
-      L += sl[s2][hh] * c;
-      A += sacc[(s2 * 16 + hh) * D + d] * c;
+      // (products are rounded before they are summed: a step's bits do not depend on what the compiler fuses)
+      L += rounded(sl[s2][hh] * c);
+      A += rounded(sacc[(s2 * 16 + hh) * D + d] * c);
     }
     const size_t hrow = ((size_t)b * hq + kh * G + hh) * nsplit + split;
     opart[hrow * D + d] = A;

@@ -143,6 +143,34 @@ def test_gemm_skinny_matches_fp32(native_ext, M, N, K):
     assert ((y.float() - want).abs().max() / want.abs().max()).item() < 1e-2
 
 
+@pytest.mark.parametrize("d", [64, 128])
+def test_decode_attention_append_rounds_products_before_sums(native_ext, d):
+    """The sums over a workgroup's tiles of keys round each product before it is added: a tile whose weighted value is the exact
+    negative of the rounded product of the other cancels it to 0 (a fused multiply-add would leave the rounding error)."""
+    scale, n = 0.3, 64                                   # two tiles of 32 keys in one split (the cache is too short for more)
+    k, v = torch.zeros(1, 2 * n, d), torch.zeros(1, 2 * n, d)
+    k[0, 32:n, 0] = -1.0                                 # scores 0 in the first tile, -scale in the second: weights 1 and c
+    q = torch.zeros(1, d, device=DEV)
+    q[0, 0] = 1.0
+    c = torch.exp2(torch.tensor([-1.0], device=DEV) * torch.tensor([scale * 1.4426950408889634], device=DEV)).cpu()
+    g = torch.Generator().manual_seed(d)
+
+    def parts(x):                                        # a float as the sum of three bf16
+        out = []
+        for _ in range(3):
+            out.append(x.bfloat16().float())
+            x = x - out[-1]
+        return torch.stack(out)
+    b = parts(torch.rand(d, generator=g) + 0.5)
+    product = b.sum(0) * c                               # one float rounding
+    assert (product.double() != b.double().sum(0) * c.double()).any()
+    v[0, 32:35], v[0, :3] = b, -parts(product)
+    kc, vc = k.bfloat16().to(DEV), v.bfloat16().to(DEV)
+    o = native_ext.decode_attention_append(q.bfloat16(), kc[:, n - 1].contiguous(), vc[:, n - 1].contiguous(), kc, vc,
+                                           torch.tensor([n - 1], device=DEV), 1, 1, d, n, scale)
+    assert not o.any()
+
+
 @pytest.mark.parametrize("M", [1, 3, 16, 17, 40])
 @pytest.mark.parametrize("N,K", [(6144, 2560), (4096, 4096), (48, 64), (1040, 576), (6160, 1984), (80, 20480)])
 def test_gemm_skinny_pieces(native_ext, M, N, K):
