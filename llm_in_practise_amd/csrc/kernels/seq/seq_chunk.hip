@@ -119,7 +119,8 @@ __device__ __forceinline__ Gate gates(const GateArgs& g, const Chunk& c, int hd,
     if (lane >= o) sum += t;
   }
   r.F1 = sum;
-  r.F0 = sum - l[1];
+  const double before = shfl_up_d(sum, 1);
+  r.F0 = l[1] == l[1] ? sum - l[1] : lane ? before + l[0] : l[0];      // (a NaN decay starts at its own token)
   r.Fc = last_lane_d(sum);
   r.a0 = ig[0] - r.F0;
   r.a1 = ig[1] - r.F1;
@@ -368,6 +369,7 @@ __global__ __launch_bounds__(256, 2) void k_chunk_out(const bf16* __restrict__ q
   __shared__ __attribute__((aligned(16))) bf16 sv[32 * VP];              // values: [dv][token]
   __shared__ __attribute__((aligned(16))) float sah[CK], sal[CK], sc[CK], sbh[CK], sbl[CK], sx[CK];
   __shared__ float sN[DK];
+  __shared__ int sbad[2][32];                              // per column the first token whose value is no number
   Chunk c;
   const int slot = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x;
   if (!find_chunk(d, slot, c)) return;
@@ -407,6 +409,7 @@ __global__ __launch_bounds__(256, 2) void k_chunk_out(const bf16* __restrict__ q
     sx[j] = exp2f((float)x0);
     sx[j + 1] = exp2f((float)x1);
   }
+  if (tid < 64) sbad[tid >> 5][tid & 31] = CK;
   if (MLSTM && tid >= 256 - DK) sN[tid - (256 - DK)] = old ? NU[cell * DK + tid - (256 - DK)] : 0.f;
   const bool work = 32 * w < c.n;
   const int qi = 32 * w + l32;                              // this lane's query
@@ -480,6 +483,25 @@ __global__ __launch_bounds__(256, 2) void k_chunk_out(const bf16* __restrict__ q
       }
     }
     if (cb) __syncthreads();                                // the last columns' reads are done
+    // A masked score is a 0 that multiplies a later token's value: an infinite or NaN value would reach the queries in front of
+    // it.  It counts as 0 in the products, and its column is NaN from its token on.
+    int* const bad = sbad[(cb >> 5) & 1];
+    unsigned m[2] = {0u, 0u};
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const u32x2 u = __builtin_bit_cast(u32x2, rv[x]);
+      m[0] |= (u[0] & 0x7f807f80u) + 0x00800080u;           // bit 15 of a half: its exponent is all ones
+      m[1] |= (u[1] & 0x7f807f80u) + 0x00800080u;
+    }
+    if ((m[0] | m[1]) & 0x80008000u)
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (!isfinite((float)rv[x][t])) {
+            rv[x][t] = (bf16)0.f;
+            atomicMin(bad + 4 * c4 + x, 4 * vt + t);
+          }
 #pragma unroll
     for (int x = 0; x < 4; ++x) *reinterpret_cast<bf16x4*>(sv + (4 * c4 + x) * VP + 4 * vt) = rv[x];
     if (old) {
@@ -529,14 +551,16 @@ __global__ __launch_bounds__(256, 2) void k_chunk_out(const bf16* __restrict__ q
           for (int part = 2; part >= 0; --part) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf[kt][ks][part], b, acc, 0, 0, 0);
         }
       }
+    if (tid < 32) sbad[(~cb >> 5) & 1][tid] = CK;           // (for the next columns; this one's last readers are past a barrier)
     const int col = cb + l32;
+    const int first = bad[l32];
     if (col < dv) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int r = 32 * w + c_row(i, half);
         if (r < c.n) {
           const float y = MLSTM ? acc[i] * ga.qscale : acc[i] + skip * (float)sv[l32 * VP + r];
-          out[((size_t)(c.t0 + r) * H + hd) * dv + col] = y;
+          out[((size_t)(c.t0 + r) * H + hd) * dv + col] = r >= first ? NAN : y;
         }
       }
     }

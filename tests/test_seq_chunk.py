@@ -108,6 +108,58 @@ def test_idle_sequences_keep_their_state():
     assert torch.equal(out[0][0][:130], out[1][0][:130]) and torch.equal(out[0][0][330:], out[1][0][330:])
 
 
+def _planted(run, inputs, name, t, at, value, lens):
+    """Outputs [T, heads, columns] with and without an infinite or NaN entry of one token: every output in front of it, and of the
+    other sequences, is what it was; the token's own is no number somewhere."""
+    clean = run(inputs)
+    x = inputs[name].clone()
+    x[t][at] = value
+    got = run({**inputs, name: x})
+    end = next(e for e in torch.tensor(lens).cumsum(0).tolist() if e > t)
+    for a, b in zip(got, clean):
+        other = torch.cat([a[:t], a[end:]]), torch.cat([b[:t], b[end:]])
+        _close(other[:1], other[1:], (name,))
+    assert not torch.isfinite(got[0][t]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,value", [("v", float("inf")), ("v", float("nan")), ("k", float("-inf")), ("q", float("nan")),
+                                        ("dt", float("nan")), ("dt", float("inf"))])
+@pytest.mark.parametrize("t", [150, 203, 268, 383])
+def test_ssd_token_that_is_no_number(name, value, t):
+    lens, H, dk, dv = [120, 264], 2, 128, 40
+    g = torch.Generator().manual_seed(t)
+    T = sum(lens)
+    inputs = {n: torch.randn(T, w, generator=g).bfloat16().cuda() for n, w in (("q", dk), ("k", dk), ("v", H * dv), ("dt", H))}
+    dtb, a_log, skip = (torch.randn(H, generator=g).cuda() for _ in range(3))
+
+    def run(x):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, [0, 5], "cuda")
+        st["S"].fill_(0.5)
+        return (R.ssd_scan(x["q"], x["k"], x["v"], x["dt"], dtb, a_log, skip, st["S"], H, 1, sb).view(T, H, dv),)
+    _planted(run, inputs, name, t, 1, value, lens)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,value", [("v", float("-inf")), ("v", float("nan")), ("k", float("inf")), ("q", float("nan")),
+                                        ("i", float("nan")), ("f", float("nan"))])
+@pytest.mark.parametrize("t", [129, 204, 299])
+def test_mlstm_token_that_is_no_number(name, value, t):
+    lens, H, dk, dv = [70, 230], 2, 64, 96
+    g = torch.Generator().manual_seed(t)
+    T = sum(lens)
+    inputs = {n: torch.randn(T, H * w, generator=g).bfloat16().cuda() for n, w in (("q", dk), ("k", dk), ("v", dv))}
+    inputs |= {n: 2 * torch.randn(T, H, generator=g).cuda() for n in "if"}
+    ib, fb = torch.randn(H, generator=g).cuda(), (torch.randn(H, generator=g) + 3).cuda()
+
+    def run(x):
+        st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lens, [9, 0], "cuda")
+        for s in st.values():
+            s.fill_(0.25)
+        return R.mlstm_scan(x["q"], x["k"], x["v"], x["i"], x["f"], ib, fb, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb)
+    _planted(run, inputs, name, t, 1, value, lens)
+
+
 BLOCK_LENS = [([32], [0]), ([31], [3]), ([48, 15, 1, 128, 65, 33], [0, 0, 9, 5, 0, 0]), ([100, 47], [512, 0])]
 
 
