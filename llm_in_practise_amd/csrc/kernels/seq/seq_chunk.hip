@@ -108,10 +108,11 @@ __device__ __forceinline__ Gate gates(const GateArgs& g, const Chunk& c, int hd,
       w[e] = on ? dt : 0.f;
     }
   }
-  // a token that forgets everything (down to -inf) counts as 2^-512, which is 0 in every float it meets: the sums behind it
-  // keep their bits
+  // state space: a token that forgets everything (down to -inf) counts as 2^-512, which is 0 in every float it meets: the sums
+  // behind it keep their bits.  (The mLSTM weighs its inputs against the log decays: those stay as they are, and above -cap - 1.)
+  if (!MLSTM)
 #pragma unroll
-  for (int e = 0; e < 2; ++e) l[e] = l[e] < -512.0 ? -512.0 : l[e];
+    for (int e = 0; e < 2; ++e) l[e] = l[e] < -512.0 ? -512.0 : l[e];
   double sum = l[0] + l[1];
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {

@@ -91,6 +91,26 @@ def test_mlstm_chunks(lens, starts, H, dk, dv):
 
 
 @pytest.mark.gpu
+def test_mlstm_chunks_keep_decays_of_a_wide_cap():
+    """Caps beyond 512 ln 2: a token may forget more than a float holds while its input weighs still less, or more."""
+    lens, H, dk, dv, cap = [131], 3, 32, 32, 2000.0
+    g = torch.Generator().manual_seed(0)
+    T = sum(lens)
+    i, f = torch.zeros(T, H), torch.full((T, H), 5.0)
+    f[-2], i[-2] = torch.tensor([-900.0, -900.0, -300.0]), torch.tensor([-500.0, -950.0, -500.0])
+    i[-1] = -5000.0
+    P = [torch.randn(T, H * n, generator=g).bfloat16().cuda() for n in (dk, dk, dv)]
+    st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lens, [0], "cuda")
+    zero = torch.zeros(H).cuda()
+    R.mlstm_scan(*P, i.cuda(), f.cuda(), zero, zero, cap, dk ** -0.5, st["S"], st["N"], st["M"], H, sb)
+    ig, fg = cap * torch.tanh(i.double() / cap), torch.nn.functional.logsigmoid(cap * torch.tanh(f.double() / cap))
+    M = torch.zeros(H, dtype=torch.float64)
+    for t in range(T):
+        M = torch.maximum(fg[t] + M, ig[t])
+    torch.testing.assert_close(st["M"][0].cpu().double(), M, rtol=1e-5, atol=1e-3)
+
+
+@pytest.mark.gpu
 def test_idle_sequences_keep_their_state():
     lens, H, dk, dv = [130, 200, 70], 2, 64, 32
     g = torch.Generator().manual_seed(0)
