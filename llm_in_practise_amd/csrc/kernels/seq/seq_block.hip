@@ -17,13 +17,16 @@
 // sequence.
 #include "seq_common.h"
 
+#include <type_traits>
+
 using namespace lipa;
 
 namespace {
 
 constexpr int BT = 16;      // tokens of a block
 
-// what the first kernel leaves per (block, head): [k G | q G | k G_16 / G] in operand order, G_16, T, B
+// what the first kernel leaves per (block, head): [k G | q G | k G_16 / G] in operand order, G_16, T, B; and behind these, per
+// (block, head) and of each of its four waves, whether a value of its tokens is infinite or NaN
 __host__ __device__ constexpr int cell_floats(int dk) { return 3 * BT * dk + dk + 2 * BT * BT; }
 
 __device__ __forceinline__ float row16_sum(float v) {       // over the 16 lanes of a row, in all of them
@@ -52,13 +55,15 @@ struct DecayArgs {
 // the sums.
 template <typename T, int NS, bool DELTA>
 __global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk,
-                                                    DecayArgs a, float* __restrict__ ws, int H, int G, SeqDesc d) {
+                                                    const T* __restrict__ v, int ldv, int dv, DecayArgs a,
+                                                    float* __restrict__ ws, unsigned* __restrict__ seen, int H, int G, SeqDesc d) {
   constexpr int DK = 64 * NS;
   __shared__ __attribute__((aligned(16))) float sg[BT * DK];
   __shared__ __attribute__((aligned(16))) float sk[BT * DK];
   __shared__ __attribute__((aligned(16))) float sq[BT * DK];
   __shared__ float sA[BT * BT];
   __shared__ float sb[BT];
+  __shared__ int sbad[BT];
   int lo = 0, hi = d.B - 1;
   const int slot = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x;
   while (lo < hi) {                              // sequence s owns the slots from seq_off[s] / 16 + s on
@@ -97,6 +102,9 @@ __global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int
     W[c] = kj[c];
     Gm[c] = f32x4{1.f, 1.f, 1.f, 1.f};
   }
+  float vz = 0.f;
+#pragma unroll 8
+  for (int c = x; c < dv; c += 16) vz += 0.f * (float)v[t * ldv + (size_t)hd * dv + c];
   if (DELTA && tid < BT) sb[tid] = tid < n ? sigmoidf_(a.beta[(size_t)(t0 + tid) * H + hd]) : 0.f;
   __syncthreads();
   float ra = 0.f, rb = 0.f;                                  // A and B of (token x, token j)
@@ -127,23 +135,42 @@ __global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int
       ra = pa;
     }
   }
+  // Delta rule: from the first token on whose key, decays or beta are no numbers everything is NaN.  In front of it T and B are 0
+  // there, and 0 x NaN is NaN: such rows of k G and T are 0, and NaN stands in B's rows, which reach the outputs of these tokens,
+  // and in the key that is written to the state.
+  bool bad = false;
+  if (DELTA) {
+    float z = 0.f;
+#pragma unroll
+    for (int c = 0; c < NS; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z += 0.f * (kj[c][e] * Gm[c][e]);
+    bad = !(row16_sum(z) == 0.f && isfinite(sb[j]));
+    if (x == 0) sbad[j] = bad ? j : BT;
+  }
   float* cell = ws + ((size_t)slot * H + hd) * cell_floats(DK);
+  const bool odd = __any(vz != 0.f);
+  if ((tid & 63) == 0) seen[((size_t)slot * H + hd) * 4 + (tid >> 6)] = odd;
   float *ck = cell, *cq = cell + BT * DK, *cp = cell + 2 * BT * DK, *cg = cell + 3 * BT * DK, *cT = cg + DK, *cB = cT + BT * BT;
 #pragma unroll
   for (int c = 0; c < NS; ++c) {
     // operand order of the 16x16x4 products: [tile of 16 channels][4 channels][token][channel of the 4] for the rows, and
     // [tile][4 tokens][channel][token of the 4] for the keys that are written to the state
     const int tile = 4 * c + (x >> 2), base = (tile * 64 + (x & 3) * 16 + j) * 4;
-    if (DELTA) *reinterpret_cast<f32x4*>(ck + base) = kj[c] * Gm[c];
+    if (DELTA) *reinterpret_cast<f32x4*>(ck + base) = bad ? f32x4{0.f, 0.f, 0.f, 0.f} : kj[c] * Gm[c];
     *reinterpret_cast<f32x4*>(cq + base) = qj[c] * Gm[c];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) cp[(tile * 64 + (j >> 2) * 16 + 4 * (x & 3) + e) * 4 + (j & 3)] = W[c][e];
+    for (int e = 0; e < 4; ++e) cp[(tile * 64 + (j >> 2) * 16 + 4 * (x & 3) + e) * 4 + (j & 3)] = bad ? NAN : W[c][e];
     if (j == BT - 1) *reinterpret_cast<f32x4*>(cg + 64 * c + 4 * x) = Gm[c];
   }
-  cB[x * BT + j] = x >= j ? rb : 0.f;
+  if (!DELTA) cB[x * BT + j] = x >= j ? rb : 0.f;
   if (DELTA) {
     sA[x * BT + j] = ra;
     __syncthreads();
+    int first = sbad[x];
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, 16));
+    cB[x * BT + j] = x >= first ? NAN : x >= j ? rb : 0.f;
     if (tid < BT) {                                          // column tid of (I + beta A)^-1 beta, row after row
       float r[BT];
 #pragma unroll
@@ -151,7 +178,7 @@ __global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int
         float acc = s == tid ? 1.f : 0.f;
 #pragma unroll
         for (int i = 0; i < s; ++i) acc -= sA[s * BT + i] * r[i];
-        r[s] = sb[s] * acc;
+        r[s] = s >= first ? 0.f : sb[s] * acc;
         cT[s * BT + tid] = r[s];
       }
     }
@@ -165,9 +192,9 @@ __global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int
 // (key products, LDS round trip, u, update); what it reads is on its way two or three blocks ahead, since it comes from memory
 // or another die's cache.
 template <typename T, int NS, bool DELTA>
-__global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float* __restrict__ ws, const T* __restrict__ v, int ldv,
-                                                                    float* __restrict__ S, float* __restrict__ out, int H, int dv,
-                                                                    SeqDesc d) {
+__global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float* __restrict__ ws, const unsigned* __restrict__ seen,
+                                                                    const T* __restrict__ v, int ldv, float* __restrict__ S,
+                                                                    float* __restrict__ out, int H, int dv, SeqDesc d) {
   constexpr int DK = 64 * NS, CELL = cell_floats(DK), RING = NS == 1 ? 4 : 3;
   __shared__ __attribute__((aligned(16))) f32x4 red[2][4][2][64];
   const int s = blockIdx.x / H, hd = blockIdx.x % H, tid = threadIdx.x;
@@ -207,11 +234,24 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
       x.v[e] = (vp + (size_t)i * BT * ldv)[(unsigned)min(4 * g + e, t1 - t0 - i * BT - 1) * (unsigned)ldv + vcol];
   };
   f32x4 uo, bo;                                   // u and B of the block of tokens before
-  auto outputs = [&](int i) {
+  unsigned long long fo[4];                       // lanes whose value of token e of 4 there is a number
+  // A value that is infinite or NaN: T and B are 0 in front of their diagonals, and 0 x inf is NaN, so it counts as 0 in the
+  // products, its column of the state is NaN, and its column of the outputs from its token on.  (This costs a tenth of the time: a
+  // sequence without such values runs the loop that does not look at them.)
+  auto outputs = [&](int i, auto odd) {
     const auto& r = red[i & 1];
     f32x4 o = (r[0][1][lane] + r[1][1][lane]) + (r[2][1][lane] + r[3][1][lane]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(bo[e], uo[e], o, 0, 0, 0);
+    if constexpr (odd) {
+      int first = BT;
+#pragma unroll
+      for (int e = 3; e >= 0; --e) first = (fo[e] >> lane) & 1 ? first : 4 * g + e;
+      first = min(first, __shfl_xor(first, 16, 64));
+      first = min(first, __shfl_xor(first, 32, 64));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = 4 * g + e >= first ? NAN : o[e];
+    }
     // (a store that has no place goes past the end of its window and is dropped: with a branch around it the compiler waits for
     // every load in flight)
     const int b0 = t0 + i * BT;
@@ -220,7 +260,7 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
     for (int e = 0; e < 4; ++e)
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[e]), win, colok ? (((4 * g + e) * H + hd) * dv + col) * 4 : -4, 0, 0);
   };
-  auto run = [&](int i, const In& x) {
+  auto run = [&](int i, const In& x, auto odd) {
     auto& r = red[i & 1];
     if (DELTA) {                                  // two chains of products: one alone waits for its own results
       f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = {0.f, 0.f, 0.f, 0.f};
@@ -242,6 +282,13 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
     f32x4 u;
 #pragma unroll
     for (int e = 0; e < 4; ++e) u[e] = t0 + i * BT + 4 * g + e < t1 ? (float)x.v[e] : 0.f;
+    bool fin[4];
+    if constexpr (odd)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        fin[e] = isfinite(u[e]);
+        u[e] = fin[e] ? u[e] : 0.f;
+      }
     if (DELTA) {
       const f32x4 e = u - ((r[0][0][lane] + r[1][0][lane]) + (r[2][0][lane] + r[3][0][lane]));
       u = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -249,31 +296,51 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
       for (int j = 0; j < 4; ++j) u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.tm[j], e[j], u, 0, 0, 0);
     }
     r[w][1][lane] = xq;
+    f32x4 us = u;
+    if constexpr (odd)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) us[e] = fin[e] ? u[e] : NAN;
 #pragma unroll
     for (int c = 0; c < NS; ++c) {
       St[c] *= x.g[c];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) St[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[c][e], u[e], St[c], 0, 0, 0);
+      for (int e = 0; e < 4; ++e) St[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[c][e], us[e], St[c], 0, 0, 0);
     }
-    if (w == (i & 3) && i > 0) outputs(i - 1);    // its query products were written in front of this barrier
+    if (w == (i & 3) && i > 0) outputs(i - 1, odd);    // its query products were written in front of this barrier
     uo = u;
     bo = x.bm;
+    if constexpr (odd)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) fo[e] = __ballot(fin[e]);
   };
 #pragma unroll
   for (int x = 0; x < RING - 1; ++x) load(min(x, steps - 1), in[x]);
-  int i = 0;
-  for (; i + RING <= steps; i += RING) {
-#pragma unroll
-    for (int x = 0; x < RING; ++x) {
-      load(min(i + x + RING - 1, steps - 1), in[(x + RING - 1) % RING]);
-      run(i + x, in[x]);
+  u32x4 any = {0u, 0u, 0u, 0u};
+  for (int i = lane; i < steps; i += 64) any |= reinterpret_cast<const u32x4*>(seen)[((size_t)(t0 / BT + s) + i) * H + hd];
+  if (__any((any[0] | any[1]) | (any[2] | any[3]))) {
+#pragma unroll 1
+    for (int i = 0; i < steps; ++i) {
+      load(i, in[0]);
+      run(i, in[0], std::true_type{});
     }
-  }
+    __syncthreads();                              // the last query products stand
+    if (w == (steps & 3)) outputs(steps - 1, std::true_type{});
+  } else {
+    constexpr std::false_type odd{};
+    int i = 0;
+    for (; i + RING <= steps; i += RING) {
 #pragma unroll
-  for (int x = 0; x < RING - 1; ++x)
-    if (i + x < steps) run(i + x, in[x]);
-  __syncthreads();                                // the last query products stand
-  if (w == (steps & 3)) outputs(steps - 1);
+      for (int x = 0; x < RING; ++x) {
+        load(min(i + x + RING - 1, steps - 1), in[(x + RING - 1) % RING]);
+        run(i + x, in[x], odd);
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < RING - 1; ++x)
+      if (i + x < steps) run(i + x, in[x], odd);
+    __syncthreads();
+    if (w == (steps & 3)) outputs(steps - 1, odd);
+  }
   if (colok)
 #pragma unroll
     for (int c = 0; c < NS; ++c) *reinterpret_cast<f32x4*>(Sp + 16 * c) = St[c];
@@ -284,10 +351,12 @@ size_t slots_of(int T_, int B) { return (size_t)T_ / BT + B; }
 template <typename T, int NS, bool DELTA>
 void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const DecayArgs& a, float* S, float* out,
             float* ws, int H, int G, int dv, const SeqDesc& d, hipStream_t st) {
-  hipLaunchKernelGGL((k_block_prep<T, NS, DELTA>), dim3((unsigned)slots_of(d.Ttot, d.B), H), dim3(256), 0, st, (const T*)q, ldq,
-                     (const T*)k, ldk, a, ws, H, G, d);
-  hipLaunchKernelGGL((k_block_scan<T, NS, DELTA>), dim3(d.B * H, (dv + 15) / 16), dim3(256), 0, st, ws, (const T*)v, ldv, S, out,
-                     H, dv, d);
+  const size_t slots = slots_of(d.Ttot, d.B);
+  unsigned* seen = reinterpret_cast<unsigned*>(ws + slots * H * cell_floats(64 * NS));
+  hipLaunchKernelGGL((k_block_prep<T, NS, DELTA>), dim3((unsigned)slots, H), dim3(256), 0, st, (const T*)q, ldq, (const T*)k, ldk,
+                     (const T*)v, ldv, dv, a, ws, seen, H, G, d);
+  hipLaunchKernelGGL((k_block_scan<T, NS, DELTA>), dim3(d.B * H, (dv + 15) / 16), dim3(256), 0, st, ws, seen, (const T*)v, ldv, S,
+                     out, H, dv, d);
   LIPA_CHECK_LAUNCH();
 }
 
@@ -323,7 +392,7 @@ size_t seq_block_floats(int code, bool delta, const void* q, int ldq, const void
   const long blocks = (long)B * H * ((dv + 15) / 16);
   const long least = delta ? (blocks <= 1024 ? 32 : 64) : blocks <= 512 ? 40 : blocks <= 1536 ? 64 : 1L << 40;
   if (T_ < least * B) return 0;
-  return slots_of(T_, B) * H * cell_floats(dk);
+  return slots_of(T_, B) * H * (cell_floats(dk) + 4);
 }
 
 void seq_block_delta(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g,

@@ -232,6 +232,44 @@ def test_gla_blocks(lens, starts, H, dk, dv, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name,value", [("v", float("inf")), ("v", float("nan")), ("k", float("nan")), ("q", float("inf")),
+                                        ("g", float("nan")), ("b", float("nan"))])
+@pytest.mark.parametrize("t", [53, 68, 95, 96, 110])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_delta_token_that_is_no_number(name, value, t, dt):
+    lens, H, dk, dv = [50, 70], 2, 128, 20
+    g = torch.Generator().manual_seed(t)
+    T = sum(lens)
+    inputs = {n: torch.nn.functional.normalize(torch.randn(T, dk, generator=g), dim=-1).to(dt).cuda() for n in "qk"}
+    inputs |= {"v": torch.randn(T, H * dv, generator=g).to(dt).cuda(), "g": (torch.rand(T, H * dk, generator=g) ** 0.2).cuda(),
+               "b": torch.randn(T, H, generator=g).cuda()}
+
+    def run(x):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, [3, 0], "cuda")
+        st["S"].fill_(0.5)
+        return (R.gated_delta_scan(x["q"], x["k"], x["v"], x["g"], x["b"], st["S"], H, 1, sb),)
+    _planted(run, inputs, name, t, 1, value, lens)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,value", [("v", float("-inf")), ("v", float("nan")), ("k", float("inf")), ("q", float("nan")),
+                                        ("z", float("nan"))])
+@pytest.mark.parametrize("t", [53, 68, 95, 96, 110])
+def test_gla_token_that_is_no_number(name, value, t):
+    lens, H, dk, dv = [50, 70], 2, 64, 40
+    g = torch.Generator().manual_seed(t)
+    T = sum(lens)
+    inputs = {n: torch.randn(T, H * w, generator=g).cuda() for n, w in (("q", dk), ("k", dk), ("v", dv), ("z", dk))}
+    zb = torch.randn(H * dk, generator=g).cuda()
+
+    def run(x):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, [0, 4], "cuda")
+        st["S"].fill_(0.5)
+        return (R.gated_linear_scan(x["q"], x["k"], x["v"], x["z"], zb, 16.0, dk ** -0.5, st["S"], H, sb),)
+    _planted(run, inputs, name, t, 1, value, lens)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("lens,starts,C,N,dt", [([160], [0], 40, 16, torch.bfloat16), ([129, 256, 1, 320], [0, 7, 0, 0], 33, 5, torch.float32),
                                                 ([127, 130], [0, 3], 130, 40, torch.bfloat16), ([200], [0], 64, 200, torch.float32),
                                                 ([1089], [0], 4096, 16, torch.bfloat16), ([60, 64], [0, 0], 64, 16, torch.float32)])
