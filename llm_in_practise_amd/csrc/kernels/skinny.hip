@@ -9,7 +9,7 @@
 //    product, does not depend on how the pieces are shared out.  The gated form and more rows take 64-deep units in turns.
 //  * W fragments are the MFMA A operands, loaded straight from HBM (16 B per lane, whole 128-byte lines per row); one batch
 //    of steps per wave is in flight while another is multiplied.  x (tiny, L2-resident) supplies the B operands.
-//  * no load sits behind a branch: a partial batch loads its last step again and multiplies it by zero.
+//  * no load sits behind a branch: a partial batch loads its last step again and does not multiply it.
 #include "common.h"
 
 using namespace lipa;
@@ -69,15 +69,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict_
   int rp = w, rb = 0;                            // the next batch to multiply
   auto run = [&](const Batch& s) {
 #pragma unroll
-    for (int u = 0; u < B; ++u)
+    for (int u = 0; u < B; ++u) {
+      if (!FULL && rb * B + u >= steps) break;
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        u32x4 b = __builtin_bit_cast(u32x4, s.b[u][m]);
-        if (!FULL && rb * B + u >= steps) b = u32x4{0u, 0u, 0u, 0u};
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int t = 0; t < CT; ++t)
-          acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.a[u][t], __builtin_bit_cast(bf16x8, b), acc[t][m], 0, 0, 0);
-      }
+          acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.a[u][t], s.b[u][m], acc[t][m], 0, 0, 0);
+    }
     if (++rb == per && CUT) {
       leave(rp);
       clear();

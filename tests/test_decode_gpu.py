@@ -192,3 +192,18 @@ def test_gemm_skinny_pieces(native_ext, M, N, K):
         want = g * torch.sigmoid(g) * u             # |d silu| <= 1.1
         bound = 1.1 * eg * (u.abs() + eu) + (g * torch.sigmoid(g)).abs() * eu + 2.0 ** -7 * want.abs() + 1e-6
         assert ((native_ext.gemm_skinny_swiglu(x, w).double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 40])
+@pytest.mark.parametrize("N,K", [(32, 64), (1056, 192), (6144, 1088), (64, 1984), (96, 20480)])
+def test_gemm_skinny_infinite_weights(native_ext, M, N, K):
+    """A partial batch of steps repeats loads: an infinite weight in its last step is an infinite product, not NaN."""
+    x, w = torch.ones(M, K, device=DEV).bfloat16(), torch.full((N, K), 2.0 ** -6, device=DEV).bfloat16()
+    for j in range(0, K, 32):                           # one infinite weight of every step, in a row of its own
+        w[j // 32 % N, j + 31] = float("inf")
+    want = x.float() @ w.float().t()
+    assert want.isinf().any() and not want.isnan().any()
+    y = native_ext.gemm_skinny(x, w, None).float()
+    assert torch.equal(y.isinf(), want.isinf()) and not y.isnan().any()
+    h = native_ext.gemm_skinny_swiglu(x, w).float()
+    assert torch.equal(h.isinf(), want[:, :N // 2].isinf() | want[:, N // 2:].isinf()) and not h.isnan().any()
