@@ -6,7 +6,7 @@
 //    ends in the residual (or the activation) and bf16.  (Split-K partials through memory took a second launch: 5.7 µs of the
 //    18 of a 6144 × 4096 product.)
 //  * up to 16 rows K is cut into the S pieces of skinny_splits, whose sums are added in order: the order, and so every bit of a
-//    product, does not depend on how the pieces are shared out.  The gated form and more rows take 64-deep units in turns.
+//    product, does not depend on how the pieces are shared out.  The gated form and more rows take units of 64 or 128 in turns.
 //  * W fragments are the MFMA A operands, loaded straight from HBM (16 B per lane, whole 128-byte lines per row); one batch
 //    of steps per wave is in flight while another is multiplied.  x (tiny, L2-resident) supplies the B operands.
 //  * no load sits behind a branch: a partial batch loads its last step again and does not multiply it.
@@ -140,33 +140,45 @@ static int skinny_splits(int N, int K) {
 
 // Column tiles and waves per workgroup, us at 1 / 8 / 16 rows: two tiles of 8 waves take 13.2 / 13.9 / 15.1 for 6144 x 4096 (one tile
 // of 4 waves 13.7 / 15.5 / 17.5) and 9.7 / 10.8 / 12.3 for 6144 x 2560 (10.7 / 12.3 / 14.4), but 4096 rows of W fill half the CUs with
-// them: 11.9 / 13.2 / 14.9 for K = 4096 against 9.0 / 9.7 / 10.9.  The gated form pairs 16 gate with 16 up rows: 38.2 / 39.4 / 44.0
-// for 2 x 12288 x 4096, 5.3 TB/s, with 4 waves of 64-deep units (2 of 128: 46 / 46 / 48), but 61 / 65 / 73 for 2 x 13824 x 5120 with 2 of
-// 128 (64 / 70 / 79), which are even at 2 x 9728 x 2560 (24): the orders of sums that the library's products have for those K.  Batches of 5 steps where the pieces divide by them (2560: whole batches 9.7, partial ones 11.8).
+// them: 11.9 / 13.2 / 14.9 for K = 4096 against 9.0 / 9.7 / 10.9.  Batches of 5 steps where the pieces divide by them (2560: whole
+// batches 9.7, partial ones 11.8).
+// The gated form pairs 16 gate with 16 up rows.  4 waves of 64-deep units against 2 of 128-deep ones: with few workgroups the
+// waves count, 2 x 3072 x 1024 5.3 / 5.7 / 6.0 against 6.1 / 6.3 / 6.4, 2 x 2048 x 4096 12.4 / 13.7 / 14.9 against 15.7 / 16.5 / 17.2; with
+// many, the longer units: 2 x 8192 x 3072 20.7 / 22.5 / 24.9 against 19.8 / 20.5 / 22.4, 2 x 6912 x 2304 16.2 / 18.7 / 20.7 against 14.6 / 15.3
+// / 16.6.  Where K is a multiple of 2048 the four waves are ahead at one row all the same (2 x 12288 x 4096 39.1 / 40.8 / 45.7 against
+// 40.2 / 39.4 / 42.1, 2 x 8192 x 2048 16.5 / 17.6 / 17.9 against 17.1 / 17.3 / 16.5) and stay, since one row is where latency counts.
 void launch_gemm_skinny(const void* X, int ldx, const void* W, const void* res, void* out, int M, int N, int K, bool glu,
                         hipStream_t st) {
-  const int pieces = skinny_splits(N, K);        // (one tile of 1 KB of LDS each: up to 32)
-  const bool cut = pieces <= 32 && M <= 16 && !glu;
+  const int pieces = skinny_splits(N, K), kc = K / pieces;        // (one tile of 1 KB of LDS each: up to 32)
 #define L(CT_, MT_, NW_, B_, GLU_, CUT_, FULL_, UNIT_)                                                                          \
   gemm_skinny_k<CT_, MT_, NW_, B_, GLU_, CUT_, FULL_, UNIT_>                                                                       \
       <<<(N + 16 * (GLU_ ? CT_ / 2 : CT_) - 1) / (16 * (GLU_ ? CT_ / 2 : CT_)), 64 * NW_, (CUT_ ? pieces : NW_) * CT_ * MT_ * 1024, \
          st>>>((const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, pieces)
-#define LM(CT_, NW_, B_, GLU_, UNIT_)                                                                \
+#define PIECES(CT_, NW_, B_)                                                                         \
   do {                                                                                               \
-    const int kc = K / pieces;                                                                       \
-    if (cut && kc % (32 * B_) == 0) L(CT_, 1, NW_, B_, GLU_, !GLU_, true, UNIT_);                   \
-    else if (cut && kc % 160 == 0) L(CT_, 1, NW_, 5, GLU_, !GLU_, true, UNIT_);                     \
-    else if (cut) L(CT_, 1, NW_, 4, GLU_, !GLU_, false, UNIT_);                                     \
-    else if (M <= 16 && K % (UNIT_ * NW_) == 0 && K % (32 * B_ * NW_) == 0) L(CT_, 1, NW_, B_, GLU_, false, true, UNIT_); \
+    if (kc % (32 * B_) == 0) L(CT_, 1, NW_, B_, false, true, true, 64);                              \
+    else if (kc % 160 == 0) L(CT_, 1, NW_, 5, false, true, true, 64);                                \
+    else L(CT_, 1, NW_, 4, false, true, false, 64);                                                  \
+  } while (0)
+#define TURNS(CT_, NW_, B_, GLU_, UNIT_)                                                             \
+  do {                                                                                               \
+    if (M <= 16 && K % (UNIT_ * NW_) == 0 && K % (32 * B_ * NW_) == 0) L(CT_, 1, NW_, B_, GLU_, false, true, UNIT_); \
     else if (M <= 16) L(CT_, 1, NW_, 4, GLU_, false, false, UNIT_);                                  \
     else if (M <= 32) L(CT_, 2, NW_, 4, GLU_, false, false, UNIT_);                                  \
     else L(CT_, 4, NW_, 4, GLU_, false, false, UNIT_);                                               \
   } while (0)
-  if (glu && (K % 1024 || K > 4096) && K % 128 == 0) LM(2, 2, 4, true, 128);
-  else if (glu) LM(2, 4, 4, true, 64);
-  else if (N >= 6144) LM(2, 8, 4, false, 64);
-  else LM(1, 4, 8, false, 64);
-#undef LM
+  if (glu) {
+    if (N > 4096 && K % 2048 && K % 128 == 0) TURNS(2, 2, 4, true, 128);
+    else TURNS(2, 4, 4, true, 64);
+  } else if (pieces <= 32 && M <= 16) {
+    if (N >= 6144) PIECES(2, 8, 4);
+    else PIECES(1, 4, 8);
+  } else {
+    if (N >= 6144) TURNS(2, 8, 4, false, 64);
+    else TURNS(1, 4, 8, false, 64);
+  }
+#undef TURNS
+#undef PIECES
 #undef L
   LIPA_CHECK_LAUNCH();
 }

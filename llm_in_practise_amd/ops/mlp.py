@@ -122,12 +122,15 @@ class _SkinnySwiGLUFn(torch.autograd.Function):
 def skinny_swiglu(x: torch.Tensor, gu_base) -> torch.Tensor | None:
     """``silu(x·W_gateᵀ)·(x·W_upᵀ)`` of up to 16 decode rows in one launch (csrc/kernels/skinny.hip), or None where that kernel
     does not serve: a bf16 [gate | up] weight, no gradient.  The products are rounded to bf16 before the activation, as the
-    separate kernels round them.  4096 → 2 × 12288, product and activation: 50 → 38 µs at 1 row, 48 → 44 at 16; above that a
-    library product pulls ahead (24 rows 44 + 5 against 52)."""
+    separate kernels round them.  4096 → 2 × 12288, product and activation: 45 → 39 µs at 1 row, 46 → 46 at 16; above that a
+    library product pulls ahead (24 rows 44 + 5 against 52), and so it does for wider or deeper weights: 5120 → 2 × 17408 75 against
+    81 µs at 1 row and 77 against 98 at 16, 2560 → 2 × 27648 53 against 55 and 54 against 67, 5120 → 2 × 5120 25 against 28 and 26
+    against 36.  Up to 2 × 14336 and 4096 no width is slower (14336 × 4096 62 → 49 and 63 → 58, 3072 × 1024 10.1 → 5.3 and 10.4 → 6.0)."""
     x2 = x.reshape(-1, x.shape[-1])
     if (torch.is_grad_enabled() and x.requires_grad) or not (
             x.is_cuda and x.dtype == torch.bfloat16 and isinstance(gu_base, torch.Tensor) and gu_base.dtype == torch.bfloat16
             and not gu_base.requires_grad and gu_base.is_contiguous() and 1 <= x2.shape[0] <= 16 and x2.stride(1) == 1
+            and x2.shape[1] <= 4096 and gu_base.shape[0] <= 2 * 14336
             and x2.stride(0) % 8 == 0 and x2.shape[1] % 64 == 0 and gu_base.shape[0] % 32 == 0
             and x2.data_ptr() % 16 == 0 and gu_base.data_ptr() % 16 == 0 and not force_reference()):
         return None

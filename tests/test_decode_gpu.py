@@ -207,3 +207,17 @@ def test_gemm_skinny_infinite_weights(native_ext, M, N, K):
     assert torch.equal(y.isinf(), want.isinf()) and not y.isnan().any()
     h = native_ext.gemm_skinny_swiglu(x, w).float()
     assert torch.equal(h.isinf(), want[:, :N // 2].isinf() | want[:, N // 2:].isinf()) and not h.isnan().any()
+
+
+@pytest.mark.parametrize("F,K,own", [(14336, 128, True), (14352, 128, False), (17408, 5120, False), (32, 4096, True), (32, 4160, False)])
+def test_gated_product_of_wide_weights_stays_with_the_library(native_ext, F, K, own):
+    """One launch for gate, up and activation only up to the widths where it is not the slower form."""
+    from llm_in_practise_amd.ops.mlp import skinny_swiglu
+    x, w = torch.randn(4, K, device=DEV).bfloat16(), (torch.randn(2 * F, K, device=DEV) * K ** -0.5).bfloat16()
+    with torch.no_grad():
+        h = skinny_swiglu(x, w)
+    assert (h is not None) == own
+    if own:
+        g, u = (x.float() @ w.float().t()).split(F, 1)
+        want = torch.nn.functional.silu(g) * u
+        assert (h.float() - want).norm() <= 2.0 ** -7 * want.norm()      # three roundings to bf16 of 2^-9 each
