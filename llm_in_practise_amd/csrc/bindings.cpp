@@ -48,6 +48,7 @@ int w4g_splits(int, int, int);
 void launch_w4g(const void*, int, const uint8_t*, const float*, int, const void*, void*, float*, int, int, int, int,
                 hipStream_t);
 int w4mm_nkb(int, int, int);
+bool w4row_serves(int, int, int, int, bool);
 bool launch_w4row(const void*, int, const uint8_t*, const float*, int, const void*, void*, int, int, int, int, bool, hipStream_t);
 void launch_w4mm(const void*, int, const uint8_t*, const float*, int, const void*, void*, float*, int, int, int, int,
                  hipStream_t);
@@ -564,7 +565,8 @@ static void check_w4mm(const Tensor& x, const Tensor& codes, const Tensor& sc2, 
   TORCH_CHECK((size_t)N * K / 2 < (1ull << 31) * 2, "w4mm: codes too large");
 }
 
-Tensor w4mm(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, optional<Tensor> residual, int64_t nkb) {
+// one: in one launch where that serves (false: the slices' partial sums through memory; the same bits)
+Tensor w4mm(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, optional<Tensor> residual, int64_t nkb, bool one) {
   check_w4mm(x, codes, sc2, N, gs);
   const int64_t M = x.size(0), K = x.size(1);
   const void* rp = nullptr;
@@ -579,8 +581,8 @@ Tensor w4mm(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, optional<
   TORCH_CHECK((K / 128) % nb == 0, "w4mm: K/128 divisible by nkb");
   const int KS = (int)(K / (128 * nb));
   Tensor out = at::empty({M, N}, x.options());
-  if (launch_w4row(x.data_ptr(), (int)x.stride(0), codes.data_ptr<uint8_t>(), sc2.data_ptr<float>(), (int)gs, rp,
-                   out.data_ptr(), (int)M, (int)N, (int)K, nb, false, stream()))
+  if (one && launch_w4row(x.data_ptr(), (int)x.stride(0), codes.data_ptr<uint8_t>(), sc2.data_ptr<float>(), (int)gs, rp,
+                          out.data_ptr(), (int)M, (int)N, (int)K, nb, false, stream()))
     return out;
   Tensor part;
   if (KS > 1) part = at::empty({KS, M, N}, x.options().dtype(at::kFloat));
@@ -599,6 +601,11 @@ optional<Tensor> w4mm_swiglu(Tensor x, Tensor codes, Tensor sc2, int64_t N, int6
                     out.data_ptr(), (int)M, (int)N / 2, (int)K, nb, true, stream()))
     return {};
   return out;
+}
+
+// Does one launch serve w4mm (glu: w4mm_swiglu)?
+bool w4mm_one(int64_t M, int64_t N, int64_t K, bool glu) {
+  return w4row_serves((int)M, (int)(glu ? N / 2 : N), (int)K, w4mm_nkb((int)M, (int)N, (int)K), glu);
 }
 
 // The decode-batch tiling of the same W4A16 GEMM (w4mm.hip w4g_k): 1 <= M <= 64, same operands as w4mm.
@@ -1777,8 +1784,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("lt_dx", &lt_dx);
   m.def("lt_reset", &lt_reset);
   m.def("w4mm", &w4mm, py::arg("x"), py::arg("codes"), py::arg("sc2"), py::arg("N"), py::arg("gs"),
-        py::arg("residual") = py::none(), py::arg("nkb") = 0);
+        py::arg("residual") = py::none(), py::arg("nkb") = 0, py::arg("one") = true);
   m.def("w4mm_ok", &w4mm_ok);
+  m.def("w4mm_one", &w4mm_one);
   m.def("w4mm_swiglu", &w4mm_swiglu);
   m.def("w4g", &w4g, py::arg("x"), py::arg("codes"), py::arg("sc2"), py::arg("N"), py::arg("gs"),
         py::arg("residual") = py::none(), py::arg("ks") = 0);

@@ -548,16 +548,31 @@ int w4mm_nkb(int M, int N, int K) {
   return kb % 2 == 0 ? 2 : 1;
 }
 
-// One launch of w4row_k, or false where it does not serve (w4mm_k then does).  Against w4mm_k and its reduce, us at 12 / 24 rows:
+// Does w4row_k serve (N: columns of the result)?  Against w4mm_k and its reduce, us in a captured graph at 12 / 24 rows:
 // 6144 x 4096 9.9 / 12.9 (13.4 / 17.1), 4096 x 4096 8.3 / 11.1 (10.1 / 13.3), 24576 x 4096 19.0 / 24.1 (26.9 / 37.0; ended in SwiGLU
-// 19.9 at 12 rows, but 31.5 at 24, where 32 rows of x and two tiles of sums leave the registers), 4096 x 12288 15.6 at 12 rows (17.7;
-// its 24 slices of 32 rows do not fit the LDS).  Tiles of 32 columns lose everywhere (6144 x 4096 11.7 at 12 rows).
-bool launch_w4row(const void* X, int ldx, const uint8_t* codes, const float* sc2, int gs, const void* res, void* out, int M,
-                  int N, int K, int nkb, bool glu, hipStream_t st) {
-  const int KS = K / (128 * nkb), RT = M <= 16 ? 1 : 2, CT = glu ? 2 : 1, tiles = N / 16;
+// 19.9 at 12 rows, but 31.5 at 24, where 32 rows of x and two tiles of sums leave the registers).  Where w4mm_k is the better one, us of
+// w4row_k against it:
+//  * one workgroup holds all of x: a single slice is a single wave, too few for the codes of 3 tiles or more (28672 x 512, 12 rows, 11.2
+//    against 6.6); 32 blocks over few tiles are a chain of 16 waves' sums (1024 x 4096, 3 rows, 7.8 against 7.0; ended in SwiGLU
+//    11.1 against 8.9 at 3 rows, 11.3 against 10.8 at 12).
+//  * slices in turns: from the second tile on x is read and turned again (5120 x 5120 11.1 against 10.9 at 3 rows, 27648 x 5120 41.0
+//    against 29.7, 5120 x 13824 25.3 against 20.0; 4096 x 12288 13.8 against 15.2); few tiles of a long K leave the chip idle (1024 x
+//    12288, 16 rows, 13.2 against 10.6; 1024 x 6144 8.4 against 9.7).
+bool w4row_serves(int M, int N, int K, int nkb, bool glu) {
+  const int KS = K / (128 * nkb), RT = M <= 16 ? 1 : 2, CT = glu ? 2 : 1, tiles = N / 16, per = (tiles + 255) / 256;
   const bool one = KS * nkb <= 32;               // (8 waves of 4 blocks or 16 of 2 hold x)
   const size_t sums = (size_t)KS * CT * RT * 1024, lds = one ? std::max(2 * sums, (size_t)KS * 4096) : sums + 8 * 4096;
   if (M > (glu ? 16 : 32) || (nkb != 2 && nkb != 4) || ((RT == 2 || glu) && !one) || lds > 65536) return false;
+  return one ? (KS > 1 || per < 3) && !(KS * nkb == 32 && tiles < 160 && (glu || nkb == 2)) : per == 1 && (tiles >= 160 || K <= 6144);
+}
+
+// One launch of w4row_k, or false where it does not serve (w4mm_k then does).
+bool launch_w4row(const void* X, int ldx, const uint8_t* codes, const float* sc2, int gs, const void* res, void* out, int M,
+                  int N, int K, int nkb, bool glu, hipStream_t st) {
+  if (!w4row_serves(M, N, K, nkb, glu)) return false;
+  const int KS = K / (128 * nkb), RT = M <= 16 ? 1 : 2, CT = glu ? 2 : 1, tiles = N / 16;
+  const bool one = KS * nkb <= 32;
+  const size_t sums = (size_t)KS * CT * RT * 1024, lds = one ? std::max(2 * sums, (size_t)KS * 4096) : sums + 8 * 4096;
   const int per = (tiles + 255) / 256, grid = one ? (tiles + per - 1) / per : tiles;   // tiles of a workgroup: even shares
 #define L(RT_, NKB_, CT_, GLU_, ONE_, NT_)                                                                       \
   w4row_k<RT_, NKB_, CT_, GLU_, ONE_, NT_><<<grid, ONE_ ? 64 * KS : 512, lds, st>>>(                             \

@@ -81,6 +81,28 @@ def test_w4mm_one_launch_keeps_the_sums(native_ext, M, N, K, gs):
     assert (h is not None) == (K in (4096, 1024, 2560))
 
 
+@pytest.mark.parametrize("M,N,K,glu,one", [
+    (12, 28672, 512, False, False), (12, 8192, 512, False, True), (3, 1024, 4096, False, False), (12, 1024, 4096, False, True),
+    (3, 4096, 4096, True, False), (12, 2048, 4096, True, False), (12, 24576, 4096, True, True), (12, 27648, 5120, False, False),
+    (3, 5120, 13824, False, False), (16, 1024, 12288, False, False), (16, 1024, 6144, False, True), (12, 4096, 12288, False, True),
+    (24, 24576, 4096, False, True), (24, 4096, 12288, False, False)])
+def test_w4mm_one_launch_only_where_it_is_not_slower(native_ext, M, N, K, glu, one):
+    """Shapes on both sides of the rule that chooses between one launch and the slices' partial sums."""
+    assert native_ext.w4mm_one(M, N, K, glu) == one
+
+
+@pytest.mark.parametrize("M", [3, 12, 16, 17, 24, 32])
+@pytest.mark.parametrize("nkb", [2, 4])
+@pytest.mark.parametrize("N,K,gs", [(4096, 1024, 128), (640, 2560, 128), (4096, 4096, 256), (2560, 5120, 128)])
+def test_w4mm_one_launch_has_the_bits_of_the_slices(native_ext, M, nkb, N, K, gs):
+    torch.manual_seed(M + nkb)
+    w = quantize_rtn(torch.randn(N, K, device=DEV), gs, False)
+    x, res = torch.randn(M, K, device=DEV).to(torch.bfloat16), torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    for r in (None, res):
+        a, b = (native_ext.w4mm(x, w.codes, w.w4mm_table(), N, gs, r, nkb, one) for one in (True, False))
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("N,K,gs,sym", [(256, 512, 128, False), (384, 1024, 64, True)])
 def test_int4_dequant_kernel_matches_fp32(native_ext, N, K, gs, sym):
     """The HBM-speed int4 -> bf16 expansion (the W4A16 prefill form) against the fp32 dequantisation."""
