@@ -410,15 +410,24 @@ __global__ __launch_bounds__(256) void k_gla_scan(const T* __restrict__ q, int l
 int seq_selective_max_states() { return 256; }
 int seq_gla_max_dk() { return 256; }
 
-// Tokens of a segment of the scan cut over time, or 0 where sequences run whole.  Whole, the longest sequence takes 0.226 us a
-// token as long as the chip is not full; cut, a step takes 8.5 us per 1000 tokens and 1000 channels and about 25 us.  Segments
-// of 32 tokens where those of 64 would leave the chip idle, else 64: their states pass through memory four times.
-int seq_selective_segment(int T_, int B, int C) {
-  if (B == 0 || 0.226f * T_ / B < 8.5e-6f * T_ * C + 25.f) return 0;
+// Tokens of a segment of the scan cut over time, or 0 where sequences run whole.  Whole, a sequence takes `whole` us a token as
+// long as the chip is not full, and more after that; cut, a step takes about 25 us and `cut` us per token and channel (every exponential
+// twice).  The lengths are not known here: their mean stands for the longest one, so that ragged steps run whole more often than they need.
+// us, whole -> cut, tokens x channels: 16 states 2048 x 4096 455 -> 89, 4 x 1024 x 8192 234 -> 228; 32 states 2048 x 8192 394 -> 224,
+// 16 x 400 x 1024 85 -> 113 (whole); 64 states 2048 x 4096 379 -> 210, 2048 x 8192 381 -> 398 (whole); 128 states 2048 x 4096 568 -> 396, 4 x
+// 1024 x 4096 463 -> 757 (whole); 256 states 2048 x 1024 1098 -> 253, 16 x 400 x 1024 364 -> 730 (whole).
+// Segments of 32 tokens where those of 64 would leave the chip idle, else 64: their states pass through memory four times.
+int seq_selective_segment(int T_, int B, int C, int N) {
+  const struct { int states; float whole, cut; } form[] = {       // (the tilings of seq_selective_scan)
+      {16, 0.226f, 8.5e-6f}, {32, 0.192f, 12e-6f}, {64, 0.185f, 23e-6f}, {128, 0.277f, 46e-6f}, {256, 0.54f, 125e-6f}};
+  int f = 0;
+  while (f < 4 && N > form[f].states) ++f;
+  if (B == 0 || form[f].whole * T_ / B < form[f].cut * T_ * C + 25.f) return 0;
+  if ((size_t)C * N > (size_t)256 * 65535) return 0;              // (the walk's grid)
   return (long)T_ * C < (1L << 22) ? 32 : 64;
 }
 size_t seq_selective_floats(int T_, int B, int C, int N) {
-  const int seg = seq_selective_segment(T_, B, C);
+  const int seg = seq_selective_segment(T_, B, C, N);
   return seg == 0 ? 0 : ((size_t)T_ / seg + B) * C * (N + 1);
 }
 
@@ -426,7 +435,7 @@ void seq_selective_scan(int code, const void* x, int ldx, const float* dtp, cons
                         const void* c, int ldc, const float* a_log, const float* dskip, const void* z, int ldz, float* S,
                         void* out, int ldo, float scale, int C, int N, float* ws, SeqDesc d, hipStream_t st) {
   if (d.B == 0) return;
-  const int seg = ws != nullptr ? seq_selective_segment(d.Ttot, d.B, C) : 1;
+  const int seg = ws != nullptr ? seq_selective_segment(d.Ttot, d.B, C, N) : 1;
   const size_t slots = (size_t)d.Ttot / seg + d.B;
   float* wdt = ws != nullptr ? ws + slots * C * N : nullptr;
 #define SEL_LAUNCH_(NS_, R_, MODE_, X_)                                                                                     \

@@ -74,6 +74,7 @@ void seq_residual_dyt(int, int, const float*, const void*, int, float, float*, i
 void seq_softcap(float*, size_t, float, hipStream_t);
 void seq_selective_scan(int, const void*, int, const float*, const float*, const void*, int, const void*, int, const float*,
                         const float*, const void*, int, float*, void*, int, float, int, int, float*, SeqDesc, hipStream_t);
+int seq_selective_segment(int, int, int, int);
 size_t seq_selective_floats(int, int, int, int);
 void seq_gla_scan(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float,
                   float*, float*, int, int, int, SeqDesc, hipStream_t);
@@ -1300,6 +1301,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sigmoid_gate", &sigmoid_gate);
   m.def("residual_dyt", &residual_dyt);
   m.def("softcap_", &softcap_);
+  m.def("selective_segment", [](int64_t T, int64_t B, int64_t C, int64_t N) {        // 0: sequences run whole
+    return seq_selective_segment((int)T, (int)B, (int)C, (int)N);
+  });
   m.def("selective_scan", &selective_scan);
   m.def("gated_linear_scan", &gated_linear_scan);
   m.def("delta_rule_gates", &delta_rule_gates);

@@ -293,3 +293,35 @@ def test_selective_cut_over_time(lens, starts, C, N, dt):
     _close((s1,), (s0,), ("state",))
     tol = TOL if dt == torch.float32 else 2.0 ** -8
     assert torch.isfinite(y1).all() and (y1.cpu() - y0).norm() <= tol * y0.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,B,C,N,cut", [
+    (2048, 1, 4096, 16, True), (4096, 4, 4096, 16, True), (6400, 16, 4096, 16, False), (2048, 1, 8192, 32, True),
+    (6400, 16, 1024, 32, False), (2048, 1, 4096, 64, True), (2048, 1, 8192, 64, False), (2048, 1, 4096, 128, True),
+    (4096, 4, 4096, 128, False), (2048, 1, 1024, 256, True), (6400, 16, 1024, 256, False), (4096, 8, 1024, 256, False),
+    (256, 1, 8192, 128, False), (256, 1, 4096, 256, False), (300, 1, 65536, 256, False)])
+def test_selective_is_cut_only_where_it_is_not_slower(T, B, C, N, cut):
+    """Timed shapes on both sides of the rule: the work of a token grows with its states, what a cut saves does not."""
+    from llm_in_practise_amd.ops._native import native_seq
+    assert (native_seq().selective_segment(T, B, C, N) > 0) == cut
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [17, 32, 64, 100, 256])
+def test_selective_cut_with_many_states(N):
+    lens, C = [700, 1100], 256
+    g = torch.Generator().manual_seed(N)
+    T = sum(lens)
+    x, z, bc = (torch.randn(T, n, generator=g) for n in (C, C, 2 * N))
+    dtp, dtb, skip = torch.randn(T, C, generator=g), torch.randn(C, generator=g) - 2, torch.randn(C, generator=g)
+    a_log = torch.randn(C, N, generator=g)
+    res = []
+    for dev in ("cpu", "cuda"):
+        st, sb = _batch({"S": ((C, N), "f32")}, lens, [0, 3], dev)
+        st["S"].fill_(0.25)
+        p = [t.to(dev) for t in (x, dtp, dtb, bc[:, :N], bc[:, N:], a_log, skip, z)]
+        res.append((R.selective_scan(*p, st["S"], sb), st["S"]))
+    from llm_in_practise_amd.ops._native import native_seq
+    assert native_seq().selective_segment(T, len(lens), C, N) > 0
+    _close(res[1], res[0], ("y", "state"))
