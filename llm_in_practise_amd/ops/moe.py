@@ -199,6 +199,18 @@ def route_tokens(h: torch.Tensor, router: torch.Tensor, correction: torch.Tensor
 PAD_ROWS = 128      # sorted path: an expert's products run over a multiple of this many rows (0: exactly its rows)
 
 
+def expert_tiles_win(pairs: int, E: int, F: int, W: int) -> bool:
+    """Do the tiles of csrc/kernels/seq/seq_moe_gemm.hip beat a vendor product pair per expert?  They need no sort, no host
+    round trip and no launches per expert (150 µs and 50 per expert), but run at 0.6 – 0.8 PFLOP/s where the vendor's large
+    products reach 1.0 – 1.3, and every 128 rows read the expert's weights again: at most 8 experts at a time, one per die, whose gate
+    and up weights the 256 MB cache behind the dies holds or not.  Rows per expert × F × W where the vendor's form wins, µs tiles → vendor: 8
+    experts of 4096 × 4096 (537 MB) 512 rows 843 → 913, 1024 1501 → 1198; 8 of 14336 × 4096 128 rows 956 → 1287, 1024 4766 → 3354; 4 of
+    4096 × 4096 (268 MB) 1024 rows 620 → 696, 2048 1113 → 977; 16 of 4096 × 2048 2048 rows 2254 → 2523, 4096 4270 → 3851; 1 of 4096 × 4096
+    (67 MB) 2048 rows 324 → 351, 8192 1038 → 855; 8 of 2048 × 2048 8192 rows 2170 → 2184."""
+    held = min(E, 8) * F * W * 4
+    return pairs // max(E, 1) * F * W < (14e9 if held >= 400e6 else 27e9 if held >= 200e6 else 50e9)
+
+
 def moe_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, idx: torch.Tensor,
                     weights: torch.Tensor, limit: float, shared: torch.Tensor | None = None,
                     few_tokens: bool = False, act: str = "clipped", shared_gate: torch.Tensor | None = None,
@@ -209,7 +221,8 @@ def moe_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tens
     ``w_down`` ``[E, W, F]``; ids ``>= E`` are identity experts (their output is ``h``); ``shared`` ``[T, W]`` is
     added.  ``few_tokens`` (decode steps, captured graphs): every (token, expert) pair streams its expert's rows in
     two kernels with no sort and no host round trip.  Otherwise the pairs are ordered by expert and every expert's
-    products run over tiles of its run (bf16, ``F`` and ``W`` multiples of 64: csrc/kernels/seq/seq_moe_gemm.hip; else one
+    products run over tiles of its run (bf16, ``F`` and ``W`` multiples of 64, and not too many rows of large experts
+    (:func:`expert_tiles_win`) or a stream that is being captured: csrc/kernels/seq/seq_moe_gemm.hip; else one
     vendor matrix product pair per expert, with one host read of the run lengths and long runs rounded up to a
     multiple of ``PAD_ROWS`` rows), and a kernel combines.  ``weight_input`` (``act="silu"``): a pair's weight multiplies
     the expert's input instead of its output, ``sum_e expert_e(w_e h)``; it is applied in float to the gate and up
@@ -229,7 +242,7 @@ def moe_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tens
     if use_seq(h) and few_tokens:
         return native_seq().moe_pairs(h.contiguous(), w_gate_up, w_down, idx, weights, shared, limit, mode, shared_gate,
                                       weight_input)
-    if use_seq(h):
+    if use_seq(h) and (expert_tiles_win(T * top, E, F_, W) or torch.cuda.is_current_stream_capturing()):
         out = native_seq().moe_tiles(h.contiguous(), w_gate_up, w_down, idx, weights, shared, limit, mode, shared_gate,
                                      weight_input)
         if out is not None:

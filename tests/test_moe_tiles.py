@@ -5,9 +5,18 @@ import torch
 
 from llm_in_practise_amd.ops import moe as M
 
-pytestmark = pytest.mark.gpu
+
+@pytest.mark.parametrize("E,F,W,rows,tiles", [
+    (8, 4096, 4096, 512, True), (8, 4096, 4096, 1024, False), (8, 14336, 4096, 128, True), (8, 14336, 4096, 512, False),
+    (4, 4096, 4096, 1024, True), (4, 4096, 4096, 2048, False), (16, 4096, 2048, 2048, True), (16, 4096, 2048, 4096, False),
+    (1, 4096, 4096, 2048, True), (1, 4096, 4096, 8192, False), (8, 2048, 2048, 8192, True), (8, 384, 2048, 30000, True),
+    (64, 2048, 4096, 2048, True), (8, 8192, 2048, 512, True), (8, 8192, 2048, 2048, False)])
+def test_tiles_only_where_they_are_not_slower(E, F, W, rows, tiles):
+    """Timed shapes on both sides of the choice between tiles and a vendor product pair per expert."""
+    assert M.expert_tiles_win(rows * E, E, F, W) == tiles
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,top,E,F,W,kind", [
     (40, 2, 8, 64, 64, "even"), (129, 2, 5, 192, 192, "even"), (300, 4, 8, 128, 320, "identity"), (257, 1, 1, 64, 128, "even"),
     (700, 3, 9, 448, 256, "skewed"), (33, 2, 16, 384, 64, "skewed"), (2100, 2, 3, 64, 64, "even")])
@@ -32,6 +41,23 @@ def test_expert_tiles(T, top, E, F, W, kind, act, weight_input, gate):
     assert torch.isfinite(got).all() and (got.cpu() - want).norm() <= 2.0 ** -8 * want.norm()
 
 
+@pytest.mark.gpu
+def test_many_rows_of_large_experts():
+    """A call past the tiles' range: the vendor's products, the same sums."""
+    g = torch.Generator().manual_seed(0)
+    T, top, E, F, W = 2100, 1, 1, 8192, 8192
+    assert not M.expert_tiles_win(T * top, E, F, W)
+    h, w = torch.randn(T, W, generator=g).bfloat16().cuda(), torch.rand(T, top, generator=g).cuda()
+    gu = (torch.randn(E, 2, F, W, device="cuda") * W ** -0.5).bfloat16()
+    d = (torch.randn(E, W, F, device="cuda") * F ** -0.5).bfloat16()
+    got = M.moe_glu_experts(h, gu, d, torch.zeros(T, top, dtype=torch.int32, device="cuda"), w, 7.0, None, False, act="silu")
+    z = h.float() @ gu[0].float().reshape(2 * F, W).t()
+    want = (torch.nn.functional.silu(z[:, :F]) * z[:, F:]) @ d[0].float().t() * w
+    # gate, up, the activation and an expert's output are rounded to bf16 once each: relative errors of at most 2^-9
+    assert (got - want).norm() <= 2.0 ** -7 * want.norm()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [256, 259, 1000])
 @pytest.mark.parametrize("n,W,top,groups,keep,kw", [
     (8, 2048, 2, 1, 1, dict(normalize=True)), (10, 1024, 4, 2, 1, dict(scale=2.0)), (16, 72, 3, 4, 2, dict(score="sigmoid", group_rank="top2")),
