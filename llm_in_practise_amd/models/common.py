@@ -202,8 +202,9 @@ class PackedPrefill:
         tb = torch.cat([torch.full((n,), b, dtype=torch.long) for b, n in enumerate(lens)])
         tp = torch.cat([torch.arange(n, dtype=torch.long) for n in lens])
         sl = torch.tensor(slots, dtype=torch.long)
-        if any(s < 0 or s * cache.max_len + n > cache.batch * cache.max_len for s, n in zip(slots, lens)):
-            raise IndexError(f"slots {slots} of {lens} tokens pass the cache's {cache.batch} rows of {cache.max_len}")
+        # (the rows are written without a look at their places: a prompt stays inside its own slot)
+        if any(not 0 <= s < cache.batch or n > cache.max_len for s, n in zip(slots, lens)) or len(set(slots)) != len(slots):
+            raise IndexError(f"slots {slots} of {lens} tokens: distinct rows of the cache's {cache.batch} of {cache.max_len}")
         self.positions = tp.to(device)[None]
         self._pad = tb * self.S + tp
         self.cache_idx = (sl[tb] * cache.max_len + tp).to(device)

@@ -373,3 +373,13 @@ def test_remote_kv_tier_shares_prefix_chunks_across_replicas():
         rb.close()
     finally:
         srv.should_exit = True
+
+
+@pytest.mark.parametrize("slots,lens", [([0], [5]), ([1, 2], [3, 5]), ([-1], [2]), ([3], [1]), ([1, 1], [2, 3])])
+def test_packed_prefill_keeps_prompts_inside_their_slots(slots, lens):
+    """A prompt longer than a slot would overwrite the next slot's rows, whichever slot it is; a slot takes one prompt."""
+    from llm_in_practise_amd.models.common import KVCache
+    cache = KVCache(1, 3, 4, 1, 8, torch.float32, "cpu")
+    with pytest.raises(IndexError):
+        cache.packed(slots, lens)
+    cache.packed([0, 2, 1], [4, 1, 4])
