@@ -205,16 +205,11 @@ class PackedPrefill:
         # (the rows are written without a look at their places: a prompt stays inside its own slot)
         if any(not 0 <= s < cache.batch or n > cache.max_len for s, n in zip(slots, lens)) or len(set(slots)) != len(slots):
             raise IndexError(f"slots {slots} of {lens} tokens: distinct rows of the cache's {cache.batch} of {cache.max_len}")
-        self.positions = tp.to(device)[None]
-        self._pad = tb * self.S + tp
-        self.cache_idx = (sl[tb] * cache.max_len + tp).to(device)
+        idx = torch.stack([tp, sl[tb] * cache.max_len + tp, tb * self.S + tp]).to(device)
+        self.positions, self.cache_idx, self.pad_idx = idx[:1], idx[1], idx[2]
         self.off = torch.tensor([0, *itertools.accumulate(lens)], dtype=torch.int32, device=device)
         self.kv_lens = torch.tensor(lens, dtype=torch.int32, device=device)
         self.last = (torch.cumsum(torch.tensor(lens), 0) - 1).to(device)
-
-    @functools.cached_property
-    def pad_idx(self) -> torch.Tensor:
-        return self._pad.to(self.cache_idx.device)
 
     def attend(self, layer: int, q, k, v, hq: int, hkv: int, d: int, attention_fn):
         write_cache_rows(self.cache.k[layer], self.cache.v[layer], self.cache_idx, k, v)

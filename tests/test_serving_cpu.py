@@ -383,3 +383,12 @@ def test_packed_prefill_keeps_prompts_inside_their_slots(slots, lens):
     with pytest.raises(IndexError):
         cache.packed(slots, lens)
     cache.packed([0, 2, 1], [4, 1, 4])
+
+
+def test_packed_prefill_makes_its_indices_once():
+    """Attention of a packed prefill copies nothing from the host (it may be captured): every index stands before the first layer."""
+    from llm_in_practise_amd.models.common import KVCache
+    pp = KVCache(1, 3, 8, 1, 8, torch.float32, "cpu").packed([2, 0], [3, 5])
+    assert isinstance(vars(pp)["pad_idx"], torch.Tensor)
+    assert pp.pad_idx.tolist() == [0, 1, 2, 5, 6, 7, 8, 9] and pp.cache_idx.tolist() == [16, 17, 18, 0, 1, 2, 3, 4]
+    assert pp.positions.tolist() == [[0, 1, 2, 0, 1, 2, 3, 4]]
