@@ -56,7 +56,8 @@ struct DecayArgs {
 template <typename T, int NS, bool DELTA>
 __global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk,
                                                     const T* __restrict__ v, int ldv, int dv, DecayArgs a,
-                                                    float* __restrict__ ws, unsigned* __restrict__ seen, int H, int G, SeqDesc d) {
+                                                    float* __restrict__ ws, unsigned* __restrict__ seen, int H, int G, Pieces pc,
+                                                    SeqDesc d) {
   constexpr int DK = 64 * NS;
   __shared__ __attribute__((aligned(16))) float sg[BT * DK];
   __shared__ __attribute__((aligned(16))) float sk[BT * DK];
@@ -64,17 +65,10 @@ __global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int
   __shared__ float sA[BT * BT];
   __shared__ float sb[BT];
   __shared__ int sbad[BT];
-  int lo = 0, hi = d.B - 1;
   const int slot = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x;
-  while (lo < hi) {                              // sequence s owns the slots from seq_off[s] / 16 + s on
-    const int mid = (lo + hi + 1) >> 1;
-    if (d.seq_off[mid] / BT + mid <= slot)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  const int o0 = d.seq_off[lo], t0 = o0 + (slot - (o0 / BT + lo)) * BT, n = min(BT, d.seq_off[lo + 1] - t0);
-  if (t0 < o0 || n <= 0 || (d.live && !d.live[lo])) return;
+  Piece blk;
+  if (!find_piece<BT>(d, pc, slot, blk)) return;
+  const int t0 = blk.t0, n = blk.n;
   const int j = tid >> 4, x = tid & 15, kh = hd / (H / G);
   const bool on = j < n;
   const size_t t = t0 + (on ? j : 0);
@@ -194,22 +188,23 @@ __global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int
 template <typename T, int NS, bool DELTA>
 __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float* __restrict__ ws, const unsigned* __restrict__ seen,
                                                                     const T* __restrict__ v, int ldv, float* __restrict__ S,
-                                                                    float* __restrict__ out, int H, int dv, SeqDesc d) {
+                                                                    float* __restrict__ out, int H, int dv, Pieces pc, SeqDesc d) {
   constexpr int DK = 64 * NS, CELL = cell_floats(DK), RING = NS == 1 ? 4 : 3;
   __shared__ __attribute__((aligned(16))) f32x4 red[2][4][2][64];
   const int s = blockIdx.x / H, hd = blockIdx.x % H, tid = threadIdx.x;
   if (d.live && !d.live[s]) return;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, col = blockIdx.y * 16 + (lane & 15);
   const bool colok = col < dv;
-  const int t0 = d.seq_off[s], t1 = d.seq_off[s + 1], steps = (t1 - t0 + BT - 1) / BT;
+  int slot;
+  const int t0 = d.seq_off[s] + pc.first * BT, t1 = d.seq_off[s + 1], steps = own_pieces<BT>(d, pc, s, slot);
   if (steps <= 0) return;
-  const float* cell = ws + ((size_t)(t0 / BT + s) * H + hd) * CELL;
+  const float* cell = ws + ((size_t)slot * H + hd) * CELL;
   const size_t step = (size_t)H * CELL;
   const T* vp = v + (size_t)t0 * ldv + (size_t)hd * dv;
   const unsigned vcol = colok ? col : 0, m = 3 * BT * DK + DK + (lane & 15) * BT + 4 * g;
   float* Sp = S + (((size_t)d.slots[s] * H + hd) * dv + (colok ? col : 0)) * DK + 16 * NS * w + 4 * g;
   f32x4 St[NS];
-  const bool old = d.pos0[s] > 0 && colok;
+  const bool old = (pc.first > 0 || d.pos0[s] > 0) && colok;
 #pragma unroll
   for (int c = 0; c < NS; ++c) St[c] = old ? row4(Sp + 16 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
   struct In {
@@ -316,7 +311,7 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
 #pragma unroll
   for (int x = 0; x < RING - 1; ++x) load(min(x, steps - 1), in[x]);
   u32x4 any = {0u, 0u, 0u, 0u};
-  for (int i = lane; i < steps; i += 64) any |= reinterpret_cast<const u32x4*>(seen)[((size_t)(t0 / BT + s) + i) * H + hd];
+  for (int i = lane; i < steps; i += 64) any |= reinterpret_cast<const u32x4*>(seen)[((size_t)slot + i) * H + hd];
   if (__any((any[0] | any[1]) | (any[2] | any[3]))) {
 #pragma unroll 1
     for (int i = 0; i < steps; ++i) {
@@ -346,29 +341,36 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
     for (int c = 0; c < NS; ++c) *reinterpret_cast<f32x4*>(Sp + 16 * c) = St[c];
 }
 
-size_t slots_of(int T_, int B) { return (size_t)T_ / BT + B; }
+// floats of a slot; 0.23 us a token at least in the token-by-token form
+size_t slot_floats(int H, int dk) { return (size_t)H * (cell_floats(dk) + 4); }
+PiecePlan block_plan(int T_, int B, int H, int dk, size_t most) {
+  return plan_pieces(T_, B, BT, slot_floats(H, dk), most, 0.23f);
+}
 
 template <typename T, int NS, bool DELTA>
 void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const DecayArgs& a, float* S, float* out,
-            float* ws, int H, int G, int dv, const SeqDesc& d, hipStream_t st) {
-  const size_t slots = slots_of(d.Ttot, d.B);
-  unsigned* seen = reinterpret_cast<unsigned*>(ws + slots * H * cell_floats(64 * NS));
-  hipLaunchKernelGGL((k_block_prep<T, NS, DELTA>), dim3((unsigned)slots, H), dim3(256), 0, st, (const T*)q, ldq, (const T*)k, ldk,
-                     (const T*)v, ldv, dv, a, ws, seen, H, G, d);
-  hipLaunchKernelGGL((k_block_scan<T, NS, DELTA>), dim3(d.B * H, (dv + 15) / 16), dim3(256), 0, st, ws, seen, (const T*)v, ldv, S,
-                     out, H, dv, d);
+            float* ws, size_t most, int H, int G, int dv, const SeqDesc& d, hipStream_t st) {
+  const PiecePlan plan = block_plan(d.Ttot, d.B, H, 64 * NS, most);
+  unsigned* seen = reinterpret_cast<unsigned*>(ws + plan.slots * H * cell_floats(64 * NS));
+  for (int w = 0; w < plan.windows; ++w) {
+    const Pieces pc = {BT, w * plan.count, plan.count};
+    hipLaunchKernelGGL((k_block_prep<T, NS, DELTA>), dim3((unsigned)plan.slots, H), dim3(256), 0, st, (const T*)q, ldq, (const T*)k,
+                       ldk, (const T*)v, ldv, dv, a, ws, seen, H, G, pc, d);
+    hipLaunchKernelGGL((k_block_scan<T, NS, DELTA>), dim3(d.B * H, (dv + 15) / 16), dim3(256), 0, st, ws, seen, (const T*)v, ldv,
+                       S, out, H, dv, pc, d);
+  }
   LIPA_CHECK_LAUNCH();
 }
 
 template <bool DELTA>
 void dispatch(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const DecayArgs& a, float* S,
-              float* out, float* ws, int H, int G, int dk, int dv, const SeqDesc& d, hipStream_t st) {
+              float* out, float* ws, size_t most, int H, int G, int dk, int dv, const SeqDesc& d, hipStream_t st) {
   SEQ_DISPATCH_T(code, {
     switch (dk / 64) {
-      case 1: launch<T, 1, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dv, d, st); break;
-      case 2: launch<T, 2, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dv, d, st); break;
-      case 3: launch<T, 3, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dv, d, st); break;
-      default: launch<T, 4, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dv, d, st); break;
+      case 1: launch<T, 1, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, d, st); break;
+      case 2: launch<T, 2, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, d, st); break;
+      case 3: launch<T, 3, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, d, st); break;
+      default: launch<T, 4, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, d, st); break;
     }
   });
 }
@@ -376,9 +378,10 @@ void dispatch(int code, const void* q, int ldq, const void* k, int ldk, const vo
 }  // namespace
 
 // Floats of workspace of the blocked form, or 0 where the token-by-token scan is the one to run: key sizes that are no multiple
-// of 64 or above 256, rows that vector loads of four channels cannot take, and steps of few tokens a sequence.
+// of 64 or above 256, rows that vector loads of four channels cannot take, and steps of few tokens a sequence.  At most `most`: longer
+// steps run in windows.
 size_t seq_block_floats(int code, bool delta, const void* q, int ldq, const void* k, int ldk, const void* g, const void* bias,
-                        const void* S, int T_, int B, int H, int dk, int dv) {
+                        const void* S, int T_, int B, int H, int dk, int dv, size_t most) {
   const int bytes = code == 0 ? 8 : 16;
   const auto fits = [](const void* p, int ld, int b) { return ld % 4 == 0 && ((uintptr_t)p & (b - 1)) == 0; };
   if (dk % 64 != 0 || dk > 256 || !fits(q, ldq, bytes) || !fits(k, ldk, bytes) || !fits(g, 4, 16) || !fits(bias, 4, 16) ||
@@ -392,19 +395,19 @@ size_t seq_block_floats(int code, bool delta, const void* q, int ldq, const void
   const long blocks = (long)B * H * ((dv + 15) / 16);
   const long least = delta ? (blocks <= 1024 ? 32 : 64) : blocks <= 512 ? 40 : blocks <= 1536 ? 64 : 1L << 40;
   if (T_ < least * B) return 0;
-  return slots_of(T_, B) * H * (cell_floats(dk) + 4);
+  return block_plan(T_, B, H, dk, most).slots * slot_floats(H, dk);
 }
 
 void seq_block_delta(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g,
-                     const float* bpre, float* S, float* out, float* ws, int H, int G, int dk, int dv, SeqDesc d,
-                     hipStream_t st) {
+                     const float* bpre, float* S, float* out, float* ws, size_t most, int H, int G, int dk, int dv,
+                     SeqDesc d, hipStream_t st) {
   const DecayArgs a = {g, nullptr, bpre, 1.f, 1.f};
-  dispatch<true>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, H, G, dk, dv, d, st);
+  dispatch<true>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dk, dv, d, st);
 }
 
 void seq_block_gla(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* z,
-                   const float* zb, float inv_tau, float qscale, float* S, float* out, float* ws, int H, int dk, int dv,
-                   SeqDesc d, hipStream_t st) {
+                   const float* zb, float inv_tau, float qscale, float* S, float* out, float* ws, size_t most, int H, int dk,
+                   int dv, SeqDesc d, hipStream_t st) {
   const DecayArgs a = {z, zb, nullptr, inv_tau, qscale};
-  dispatch<false>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, H, H, dk, dv, d, st);
+  dispatch<false>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, H, dk, dv, d, st);
 }

@@ -27,29 +27,6 @@ constexpr int KP = 64 + 8;              // row of 64 staged tokens, padded: 16-b
 constexpr int VP = CK + 4;              // row of a chunk's tokens, padded: 8-byte reads of 32 rows hit all banks
 constexpr double LOG2E = 1.4426950408889634074;
 
-struct Chunk {
-  int s, t0, n, idx;                    // sequence, first token, tokens, number within the sequence
-};
-
-// Chunk slots: sequence s owns slots seq_off[s] / CK + s, .., one per chunk (consecutive sequences never overlap).  False:
-// the slot holds no chunk.
-__device__ __forceinline__ bool find_chunk(const SeqDesc& d, int slot, Chunk& c) {
-  int lo = 0, hi = d.B - 1;
-  while (lo < hi) {                     // the last sequence whose first slot is not past this one
-    const int mid = (lo + hi + 1) >> 1;
-    if (d.seq_off[mid] / CK + mid <= slot)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  const int o0 = d.seq_off[lo], o1 = d.seq_off[lo + 1];
-  c.s = lo;
-  c.idx = slot - (o0 / CK + lo);
-  c.t0 = o0 + c.idx * CK;
-  c.n = min(CK, o1 - c.t0);
-  return c.idx >= 0 && c.n > 0 && !(d.live && !d.live[lo]);
-}
-
 // x = hi + mid + lo in bf16 to float accuracy (an infinity stays one)
 __device__ __forceinline__ void split3(float x, bf16& h, bf16& m, bf16& l) {
   h = (bf16)x;
@@ -87,7 +64,7 @@ struct Gate {                           // of a wave's lane: tokens 2 * lane and
 };
 
 template <bool MLSTM>
-__device__ __forceinline__ Gate gates(const GateArgs& g, const Chunk& c, int hd, int lane) {
+__device__ __forceinline__ Gate gates(const GateArgs& g, const Piece& c, int hd, int lane) {
   Gate r;
   double l[2], ig[2] = {0.0, 0.0};
   float w[2] = {0.f, 0.f};
@@ -164,15 +141,15 @@ __device__ __forceinline__ int c_row(int i, int half) { return (i & 3) + 8 * (i 
 template <int NK, bool MLSTM>
 __global__ __launch_bounds__(256, 3) void k_chunk_state(const bf16* __restrict__ k, int ldk, const bf16* __restrict__ v,
                                                      int ldv, GateArgs ga, float* __restrict__ U, float* __restrict__ NU,
-                                                     double* __restrict__ meta, int H, int G, int dv, SeqDesc d) {
+                                                     double* __restrict__ meta, int H, int G, int dv, Pieces pc, SeqDesc d) {
   constexpr int DK = 32 * NK;
   __shared__ __attribute__((aligned(16))) bf16 sk[DK * KP];              // [dk][token]
   __shared__ __attribute__((aligned(16))) bf16 sv[3 * 64 * KP];          // [part][dv][token]
   __shared__ float sw[CK];
   __shared__ float sn[256];
-  Chunk c;
+  Piece c;
   const int slot = blockIdx.x, hd = blockIdx.y, cb = blockIdx.z * 64, tid = threadIdx.x;
-  if (!find_chunk(d, slot, c)) return;
+  if (!find_piece<CK>(d, pc, slot, c)) return;
   const int w = tid >> 6, lane = tid & 63, l32 = lane & 31, half = lane >> 5, kh = hd / (H / G);
   const size_t cell = (size_t)slot * H + hd;
   const bf16* kp = k + (size_t)c.t0 * ldk + kh * DK;
@@ -299,17 +276,19 @@ __global__ __launch_bounds__(256, 3) void k_chunk_state(const bf16* __restrict__
 template <bool MLSTM>
 __global__ __launch_bounds__(256) void k_chunk_walk(float* __restrict__ U, float* __restrict__ NU, double* __restrict__ meta,
                                                     float* __restrict__ S, float* __restrict__ N,
-                                                    const float* __restrict__ M, int H, int dk, int dv, int nb, SeqDesc d) {
+                                                    const float* __restrict__ M, int H, int dk, int dv, int nb, Pieces pc,
+                                                    SeqDesc d) {
   const int s = blockIdx.x / H, hd = blockIdx.x % H, tid = threadIdx.x;
   if (d.live && !d.live[s]) return;
   const bool norm = MLSTM && (int)blockIdx.y == nb;        // the last block walks the normaliser
-  const int t0 = d.seq_off[s], len = d.seq_off[s + 1] - t0, n = (len + CK - 1) / CK, first = t0 / CK + s;
+  int first;
+  const int n = own_pieces<CK>(d, pc, s, first);
   const int size = norm ? dk : dv * dk, e = (norm ? 0 : (int)blockIdx.y * 1024) + 4 * tid;
   const size_t hbase = (size_t)d.slots[s] * H + hd, step = (size_t)H * size;
   float* st = (norm ? N : S) + hbase * size + e;
   float* u = (norm ? NU : U) + ((size_t)first * H + hd) * size + e;
   double* mt = meta + 3 * ((size_t)first * H + hd);
-  const bool on = e < size, old = d.pos0[s] > 0;
+  const bool on = e < size, old = pc.first > 0 || d.pos0[s] > 0;
   f32x4 x = {0.f, 0.f, 0.f, 0.f};
   if (on && old) x = *reinterpret_cast<const f32x4*>(st);
   double m = MLSTM && old ? (double)M[hbase] * LOG2E : 0.0;
@@ -364,16 +343,16 @@ __global__ __launch_bounds__(256, 2) void k_chunk_out(const bf16* __restrict__ q
                                                       const float* __restrict__ U, const float* __restrict__ NU,
                                                       const double* __restrict__ meta, float* __restrict__ M,
                                                       float* __restrict__ out, float* __restrict__ den,
-                                                      float* __restrict__ efl, int H, int G, int dv, SeqDesc d) {
+                                                      float* __restrict__ efl, int H, int G, int dv, Pieces pc, SeqDesc d) {
   constexpr int DK = 32 * NK, SP = DK + 8;
   __shared__ __attribute__((aligned(16))) bf16 ss[3 * 32 * SP];          // state: [part][dv][dk]
   __shared__ __attribute__((aligned(16))) bf16 sv[32 * VP];              // values: [dv][token]
   __shared__ __attribute__((aligned(16))) float sah[CK], sal[CK], sc[CK], sbh[CK], sbl[CK], sx[CK];
   __shared__ float sN[DK];
   __shared__ int sbad[2][32];                              // per column the first token whose value is no number
-  Chunk c;
+  Piece c;
   const int slot = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x;
-  if (!find_chunk(d, slot, c)) return;
+  if (!find_piece<CK>(d, pc, slot, c)) return;
   const int w = tid >> 6, lane = tid & 63, l32 = lane & 31, half = lane >> 5, kh = hd / (H / G);
   const size_t cell = (size_t)slot * H + hd;
   const bool old = c.idx > 0 || d.pos0[c.s] > 0;           // is there a state in front of the chunk
@@ -392,7 +371,8 @@ __global__ __launch_bounds__(256, 2) void k_chunk_out(const bf16* __restrict__ q
       x1 = mp - m1;
       if (2 * lane < c.n) efl[(size_t)(c.t0 + 2 * lane) * H + hd] = exp2f((float)(-(g.F0 + m0)));
       if (2 * lane + 1 < c.n) efl[(size_t)(c.t0 + 2 * lane + 1) * H + hd] = exp2f((float)(-(g.F1 + m1)));
-      if (lane == 63 && c.t0 + c.n == d.seq_off[c.s + 1])      // behind the last chunk (tokens past its end change nothing)
+      // behind the last chunk, here or at all (tokens past its end change nothing)
+      if (lane == 63 && (c.t0 + c.n == d.seq_off[c.s + 1] || (pc.count > 0 && c.idx == pc.first + pc.count - 1)))
         M[(size_t)d.slots[c.s] * H + hd] = (float)((g.F1 + m1) * 0.69314718055994530942);
     }
     const float ah0 = (float)g.a0, ah1 = (float)g.a1, bh0 = (float)b0, bh1 = (float)b1;
@@ -568,32 +548,41 @@ __global__ __launch_bounds__(256, 2) void k_chunk_out(const bf16* __restrict__ q
   }
 }
 
-size_t slots_of(int T_, int B) { return (size_t)T_ / CK + B; }
+// floats of a slot; 0.4 us a token in the token-by-token form
+size_t chunk_floats(int H, int dk, int dv) { return (size_t)H * (6 + (size_t)dk * (dv + 1)); }
+PiecePlan chunk_plan(int T_, int B, int H, int dk, int dv, size_t most) {
+  return plan_pieces(T_, B, CK, chunk_floats(H, dk, dv), most, 0.4f);
+}
 
 template <int NK, bool MLSTM>
 void chunk_launch(const bf16* q, int ldq, const bf16* k, int ldk, const bf16* v, int ldv, const GateArgs& ga, float* S, float* N,
-                  float* M, float* out, float* den, float* efl, float* ws, int H, int G, int dv, SeqDesc d, hipStream_t st) {
-  const size_t ns = slots_of(d.Ttot, d.B), cells = ns * H;
+                  float* M, float* out, float* den, float* efl, float* ws, size_t most, int H, int G, int dv, SeqDesc d,
+                  hipStream_t st) {
+  const PiecePlan plan = chunk_plan(d.Ttot, d.B, H, 32 * NK, dv, most);
+  const size_t ns = plan.slots, cells = ns * H;
   double* meta = reinterpret_cast<double*>(ws);
   float* U = ws + 6 * cells + (6 * cells & 3);
   float* NU = U + cells * dv * 32 * NK;
   const int nb = (dv * 32 * NK + 1023) / 1024;
-  hipLaunchKernelGGL((k_chunk_state<NK, MLSTM>), dim3((unsigned)ns, H, (dv + 63) / 64), dim3(256), 0, st, k, ldk, v, ldv, ga, U,
-                     NU, meta, H, G, dv, d);
-  hipLaunchKernelGGL((k_chunk_walk<MLSTM>), dim3(d.B * H, nb + (MLSTM ? 1 : 0)), dim3(256), 0, st, U, NU, meta, S, N, M, H,
-                     32 * NK, dv, nb, d);
-  hipLaunchKernelGGL((k_chunk_out<NK, MLSTM>), dim3((unsigned)ns, H), dim3(256), 0, st, q, ldq, k, ldk, v, ldv, ga, U, NU, meta,
-                     M, out, den, efl, H, G, dv, d);
+  for (int w = 0; w < plan.windows; ++w) {
+    const Pieces pc = {CK, w * plan.count, plan.count};
+    hipLaunchKernelGGL((k_chunk_state<NK, MLSTM>), dim3((unsigned)ns, H, (dv + 63) / 64), dim3(256), 0, st, k, ldk, v, ldv, ga, U,
+                       NU, meta, H, G, dv, pc, d);
+    hipLaunchKernelGGL((k_chunk_walk<MLSTM>), dim3(d.B * H, nb + (MLSTM ? 1 : 0)), dim3(256), 0, st, U, NU, meta, S, N, M, H,
+                       32 * NK, dv, nb, pc, d);
+    hipLaunchKernelGGL((k_chunk_out<NK, MLSTM>), dim3((unsigned)ns, H), dim3(256), 0, st, q, ldq, k, ldk, v, ldv, ga, U, NU, meta,
+                       M, out, den, efl, H, G, dv, pc, d);
+  }
   LIPA_CHECK_LAUNCH();
 }
 
 template <bool MLSTM>
 void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const GateArgs& ga, float* S, float* N,
-                    float* M, float* out, float* den, float* efl, float* ws, int H, int G, int dk, int dv, SeqDesc d,
-                    hipStream_t st) {
+                    float* M, float* out, float* den, float* efl, float* ws, size_t most, int H, int G, int dk, int dv,
+                    SeqDesc d, hipStream_t st) {
 #define CHUNK(NK_)                                                                                                          \
-  chunk_launch<NK_, MLSTM>((const bf16*)q, ldq, (const bf16*)k, ldk, (const bf16*)v, ldv, ga, S, N, M, out, den, efl, ws, H, G, \
-                           dv, d, st)
+  chunk_launch<NK_, MLSTM>((const bf16*)q, ldq, (const bf16*)k, ldk, (const bf16*)v, ldv, ga, S, N, M, out, den, efl, ws, \
+                           most, H, G, dv, d, st)
   switch (dk / 32) {
     case 1: CHUNK(1); break;
     case 2: CHUNK(2); break;
@@ -607,29 +596,30 @@ void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* 
 
 // Floats of workspace of the chunked form, or 0 where the token-by-token scan is the one to run: float activations, key sizes
 // that are no multiple of 32 or above 128, rows that 16-byte (q, k) or 8-byte (v) loads cannot take, and steps of few tokens a
-// sequence.
+// sequence.  At most `most`: longer steps run in windows.
 size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, int T_, int B, int H,
-                        int dk, int dv) {
+                        int dk, int dv, size_t most) {
   const auto fits = [](const void* p, int ld, int n) { return ld % n == 0 && ((uintptr_t)p & (2 * n - 1)) == 0; };
   if (code != 0 || dk % 32 != 0 || dk > 128 || dv % 4 != 0 || !fits(q, ldq, 8) || !fits(k, ldk, 8) || !fits(v, ldv, 4)) return 0;
   // three launches and a chunk of padding against 0.4 us a token (two heads a CU) in the token-by-token form: 64 tokens a
   // sequence are 21 / 32 / 96 us here and 30 / 36 / 148 us there (state space, 32 heads, 1 / 8 / 48 sequences), 48 are 21 / 32 / 94
   // and 24 / 29 / 118 us; mLSTM (8 heads of 128 x 192) at 64: 26 / 34 / 68 against 31 / 36 / 159 us
   if (B == 0 || T_ < 64 * B) return 0;
-  const size_t cells = slots_of(T_, B) * H;
-  return 6 * cells + 4 + cells * dk * (dv + 1);
+  const size_t slots = chunk_plan(T_, B, H, dk, dv, most).slots;
+  return slots == 0 ? 0 : slots * chunk_floats(H, dk, dv) + 4;
 }
 
 void seq_chunk_ssd(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const void* dt, int lddt,
-                   const float* dt_bias, const float* a_log, const float* dskip, float* S, float* out, float* ws, int H, int G,
-                   int dk, int dv, SeqDesc d, hipStream_t st) {
+                   const float* dt_bias, const float* a_log, const float* dskip, float* S, float* out, float* ws, size_t most,
+                   int H, int G, int dk, int dv, SeqDesc d, hipStream_t st) {
   const GateArgs ga = {(const bf16*)dt, lddt, dt_bias, a_log, dskip, nullptr, nullptr, nullptr, nullptr, 1.f, 1.f, H};
-  chunk_dispatch<false>(q, ldq, k, ldk, v, ldv, ga, S, nullptr, nullptr, out, nullptr, nullptr, ws, H, G, dk, dv, d, st);
+  chunk_dispatch<false>(q, ldq, k, ldk, v, ldv, ga, S, nullptr, nullptr, out, nullptr, nullptr, ws, most, H, G, dk, dv, d,
+                        st);
 }
 
 void seq_chunk_mlstm(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* ipre, const float* fpre,
                      const float* ib, const float* fb, float cap, float qscale, float* S, float* N, float* M, float* out,
-                     float* den, float* efl, float* ws, int H, int dk, int dv, SeqDesc d, hipStream_t st) {
+                     float* den, float* efl, float* ws, size_t most, int H, int dk, int dv, SeqDesc d, hipStream_t st) {
   const GateArgs ga = {nullptr, 0, nullptr, nullptr, nullptr, ipre, fpre, ib, fb, cap, qscale, H};
-  chunk_dispatch<true>(q, ldq, k, ldk, v, ldv, ga, S, N, M, out, den, efl, ws, H, H, dk, dv, d, st);
+  chunk_dispatch<true>(q, ldq, k, ldk, v, ldv, ga, S, N, M, out, den, efl, ws, most, H, H, dk, dv, d, st);
 }

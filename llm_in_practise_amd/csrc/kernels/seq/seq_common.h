@@ -20,6 +20,65 @@ struct SeqDesc {
   int B, Ttot;
 };
 
+// A step's sequences cut into pieces of LEN tokens (0: of `len`), each with a slot for what a kernel leaves of it.  count 0: every piece has
+// one, sequence s owns the slots from seq_off[s] / LEN + s on (consecutive sequences never overlap).  Else the pieces [first, first +
+// count) of every sequence, s owns the slots from s * count on: a step whose slots would take too much memory runs window after
+// window, and the state goes from one to the next through the sequence's own place.
+struct Pieces {
+  int len, first, count;
+};
+struct Piece {
+  int s, idx, t0, n;     // sequence, number within it, first token, tokens
+};
+// False: the slot holds no piece (or one of an idle sequence).
+template <int LEN>
+__device__ __forceinline__ bool find_piece(const SeqDesc& d, const Pieces& p, int slot, Piece& c) {
+  const int len = LEN > 0 ? LEN : p.len;
+  int lo = 0, hi = d.B - 1, at = 0;
+  if (p.count > 0) {
+    lo = slot / p.count;
+    at = lo * p.count - p.first;
+  } else {
+    while (lo < hi) {    // the last sequence whose first slot is not past this one
+      const int mid = (lo + hi + 1) >> 1;
+      if (d.seq_off[mid] / len + mid <= slot)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    at = d.seq_off[lo] / len + lo;
+  }
+  const int o0 = d.seq_off[lo], o1 = d.seq_off[lo + 1];
+  c.s = lo;
+  c.idx = slot - at;
+  c.t0 = o0 + c.idx * len;
+  c.n = min(len, o1 - c.t0);
+  return c.idx >= 0 && c.n > 0 && !(d.live && !d.live[lo]);
+}
+// a sequence's pieces here: how many, and the slot of the first
+template <int LEN>
+__device__ __forceinline__ int own_pieces(const SeqDesc& d, const Pieces& p, int s, int& slot) {
+  const int len = LEN > 0 ? LEN : p.len, o0 = d.seq_off[s], all = (d.seq_off[s + 1] - o0 + len - 1) / len;
+  slot = p.count > 0 ? s * p.count : o0 / len + s;
+  return p.count > 0 ? min(all - p.first, p.count) : all;
+}
+
+// Slots and windows for at most `most` floats at `per` a slot; no slots: the token-by-token form is to run, at token_us a token of the
+// mean length (a window costs 15 us at least, and one sequence may hold nearly all the tokens).
+struct PiecePlan {
+  size_t slots;
+  int count, windows;
+};
+inline PiecePlan plan_pieces(int T_, int B, int len, size_t per, size_t most, float token_us) {
+  const size_t all = (size_t)T_ / len + B;
+  if (all * per <= most) return {all, 0, 1};
+  const size_t count = most / (per * B);
+  if (count == 0) return {0, 0, 0};
+  const int windows = (int)((((size_t)T_ + len - 1) / len + count - 1) / count);
+  if (15.f * windows > token_us * T_ / B) return {0, 0, 0};
+  return {count * B, (int)count, windows};
+}
+
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + expf(-x)); }
 __device__ __forceinline__ float softplusf_(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 __device__ __forceinline__ float gelu_tanhf_(float v) {

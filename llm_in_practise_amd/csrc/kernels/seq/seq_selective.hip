@@ -92,20 +92,6 @@ __device__ __forceinline__ void store_state(float* p, int i0, int len, const flo
 constexpr int CH = 2;
 enum { WHOLE, LEAVES, FROM };       // a sequence; a segment from zero (state and step sizes); a segment from the state before it
 
-// segment slots: sequence s owns slots seq_off[s] / seg + s, .. (consecutive sequences never overlap)
-__device__ __forceinline__ int find_segment(const SeqDesc& d, int seg, int slot, int& first) {
-  int lo = 0, hi = d.B - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (d.seq_off[mid] / seg + mid <= slot)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  first = d.seq_off[lo] + (slot - (d.seq_off[lo] / seg + lo)) * seg;
-  return lo;
-}
-
 template <typename T, int NS, int R, int MODE>
 __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x, int ldx, const float* __restrict__ dtp,
                                                         const float* __restrict__ dtb, const T* __restrict__ bm, int ldb,
@@ -113,7 +99,7 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
                                                         const float* __restrict__ dskip, const T* __restrict__ z, int ldz,
                                                         float* __restrict__ S, T* __restrict__ out, int ldo, float scale,
                                                         int C, int N, float* __restrict__ ws, float* __restrict__ wdt,
-                                                        int seg, SeqDesc d) {
+                                                        Pieces pc, SeqDesc d) {
   constexpr int NC = 256 / R * CH, PER = CT * NC / 256, NP = NS * R, PB = (CT * NP + 255) / 256;
   __shared__ __attribute__((aligned(16))) float sdt[CT * NC];
   __shared__ __attribute__((aligned(16))) float sdx[CT * NC];     // dt x
@@ -123,12 +109,13 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
   const int tid = threadIdx.x;
   const int lane = tid & 63, grp = (tid >> 6) * (64 / R) + lane_group<R>(lane), row = lane >> 4;
   const int cb = blockIdx.y * NC, c0 = cb + grp * CH, n0 = lane_part<R>(lane) * NS;
-  int s = blockIdx.x, first = 0;
-  if (MODE != WHOLE) s = find_segment(d, seg, blockIdx.x, first);
+  Piece seg = {(int)blockIdx.x, 0, 0, 0};
+  if (MODE != WHOLE && !find_piece<0>(d, pc, blockIdx.x, seg)) return;
+  const int s = seg.s;
   if (d.live && !d.live[s]) return;
-  const int end = d.seq_off[s + 1], t0 = MODE == WHOLE ? d.seq_off[s] : first, t1 = MODE == WHOLE ? end : min(end, first + seg);
-  // (behind a sequence's last segment stands nothing that a leaving state would serve)
-  if (MODE != WHOLE && (t0 < d.seq_off[s] || t0 >= end || (MODE == LEAVES && t1 == end))) return;
+  const int end = d.seq_off[s + 1], t0 = MODE == WHOLE ? d.seq_off[s] : seg.t0, t1 = MODE == WHOLE ? end : t0 + seg.n;
+  const bool last = t1 == end || (pc.count > 0 && seg.idx == pc.first + pc.count - 1);     // of the sequence, or of it here
+  if (MODE == LEAVES && last) return;                 // (nothing that a leaving state would serve stands behind it)
   const int p0 = d.pos0[s], slot = d.slots[s];
   float Sr[CH][NS], A[CH][NS], sum[CH] = {0.f, 0.f};
 #pragma unroll
@@ -254,7 +241,7 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
       if (MODE == LEAVES) {
         store_state<NS>(ws + ((size_t)blockIdx.x * C + c0 + h) * N, n0, N, Sr[h]);
         if (n0 == 0) wdt[(size_t)blockIdx.x * C + c0 + h] = sum[h];
-      } else if (MODE == WHOLE || t1 == end) {
+      } else if (MODE == WHOLE || last) {
         store_state<NS>(S + ((size_t)slot * C + c0 + h) * N, n0, N, Sr[h]);
       }
     }
@@ -263,13 +250,15 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
 // The states in front of a sequence's segments, one (channel, state) per thread: they replace the states that the segments left.
 __global__ __launch_bounds__(256) void k_selective_walk(const float* __restrict__ a_log, const float* __restrict__ S,
                                                         float* __restrict__ ws, const float* __restrict__ wdt, int C, int N,
-                                                        int seg, SeqDesc d) {
+                                                        Pieces pc, SeqDesc d) {
   const int s = blockIdx.x;
   const size_t e = (size_t)blockIdx.y * 256 + threadIdx.x, size = (size_t)C * N;
   if ((d.live && !d.live[s]) || e >= size) return;
-  const int t0 = d.seq_off[s], n = (d.seq_off[s + 1] - t0 + seg - 1) / seg, first = t0 / seg + s;
+  int first;
+  const int n = own_pieces<0>(d, pc, s, first);
+  if (n <= 0) return;
   const float A = -expf(a_log[e]) * 1.4426950408889634f;
-  float x = d.pos0[s] > 0 ? S[(size_t)d.slots[s] * size + e] : 0.f;
+  float x = pc.first > 0 || d.pos0[s] > 0 ? S[(size_t)d.slots[s] * size + e] : 0.f;
   float* u = ws + (size_t)first * size + e;
   const float* dt = wdt + (size_t)first * C + e / N;
   constexpr int AHEAD = 16;                         // segments in flight (the last one left nothing)
@@ -417,40 +406,46 @@ int seq_gla_max_dk() { return 256; }
 // 16 x 400 x 1024 85 -> 113 (whole); 64 states 2048 x 4096 379 -> 210, 2048 x 8192 381 -> 398 (whole); 128 states 2048 x 4096 568 -> 396, 4 x
 // 1024 x 4096 463 -> 757 (whole); 256 states 2048 x 1024 1098 -> 253, 16 x 400 x 1024 364 -> 730 (whole).
 // Segments of 32 tokens where those of 64 would leave the chip idle, else 64: their states pass through memory four times.
-int seq_selective_segment(int T_, int B, int C, int N) {
+static int segment_of(int T_, int B, int C, int N, PiecePlan& plan, size_t most) {
   const struct { int states; float whole, cut; } form[] = {       // (the tilings of seq_selective_scan)
       {16, 0.226f, 8.5e-6f}, {32, 0.192f, 12e-6f}, {64, 0.185f, 23e-6f}, {128, 0.277f, 46e-6f}, {256, 0.54f, 125e-6f}};
   int f = 0;
   while (f < 4 && N > form[f].states) ++f;
   if (B == 0 || form[f].whole * T_ / B < form[f].cut * T_ * C + 25.f) return 0;
   if ((size_t)C * N > (size_t)256 * 65535) return 0;              // (the walk's grid)
-  return (long)T_ * C < (1L << 22) ? 32 : 64;
+  const int seg = (long)T_ * C < (1L << 22) ? 32 : 64;
+  plan = plan_pieces(T_, B, seg, (size_t)C * (N + 1), most, form[f].whole);
+  return plan.slots == 0 ? 0 : seg;
 }
-size_t seq_selective_floats(int T_, int B, int C, int N) {
-  const int seg = seq_selective_segment(T_, B, C, N);
-  return seg == 0 ? 0 : ((size_t)T_ / seg + B) * C * (N + 1);
+// Floats of its workspace, at most `most` (longer steps run in windows), or 0 where sequences run whole
+size_t seq_selective_floats(int T_, int B, int C, int N, size_t most) {
+  PiecePlan plan;
+  return segment_of(T_, B, C, N, plan, most) == 0 ? 0 : plan.slots * C * (N + 1);
 }
 
 void seq_selective_scan(int code, const void* x, int ldx, const float* dtp, const float* dtb, const void* b, int ldb,
                         const void* c, int ldc, const float* a_log, const float* dskip, const void* z, int ldz, float* S,
-                        void* out, int ldo, float scale, int C, int N, float* ws, SeqDesc d, hipStream_t st) {
+                        void* out, int ldo, float scale, int C, int N, float* ws, size_t most, SeqDesc d, hipStream_t st) {
   if (d.B == 0) return;
-  const int seg = ws != nullptr ? seq_selective_segment(d.Ttot, d.B, C, N) : 1;
-  const size_t slots = (size_t)d.Ttot / seg + d.B;
-  float* wdt = ws != nullptr ? ws + slots * C * N : nullptr;
+  PiecePlan plan = {0, 0, 1};
+  const int seg = ws != nullptr ? segment_of(d.Ttot, d.B, C, N, plan, most) : 1;
+  float* wdt = ws != nullptr ? ws + plan.slots * C * N : nullptr;
+  Pieces pc = {seg, 0, plan.count};
 #define SEL_LAUNCH_(NS_, R_, MODE_, X_)                                                                                     \
   hipLaunchKernelGGL((k_selective_scan<T, NS_, R_, MODE_>), dim3((unsigned)(X_), (C + 256 / R_ * CH - 1) / (256 / R_ * CH)), \
                      dim3(256), 0, st, (const T*)x, ldx, dtp, dtb, (const T*)b, ldb, (const T*)c, ldc, a_log, dskip,        \
-                     (const T*)z, ldz, S, (T*)out, ldo, scale, C, N, ws, wdt, seg, d)
+                     (const T*)z, ldz, S, (T*)out, ldo, scale, C, N, ws, wdt, pc, d)
 #define SEL_LAUNCH(NS_, R_)                                                                                              \
   do {                                                                                                                   \
     if (ws == nullptr) {                                                                                                 \
       SEL_LAUNCH_(NS_, R_, WHOLE, d.B);                                                                                  \
-    } else {                                                                                                             \
-      SEL_LAUNCH_(NS_, R_, LEAVES, slots);                                                                               \
+      break;                                                                                                             \
+    }                                                                                                                    \
+    for (int w = 0; w < plan.windows; ++w, pc.first += plan.count) {                                                     \
+      SEL_LAUNCH_(NS_, R_, LEAVES, plan.slots);                                                                          \
       hipLaunchKernelGGL(k_selective_walk, dim3(d.B, (unsigned)(((size_t)C * N + 255) / 256)), dim3(256), 0, st, a_log, S, ws, \
-                         wdt, C, N, seg, d);                                                                                  \
-      SEL_LAUNCH_(NS_, R_, FROM, slots);                                                                                 \
+                         wdt, C, N, pc, d);                                                                                   \
+      SEL_LAUNCH_(NS_, R_, FROM, plan.slots);                                                                            \
     }                                                                                                                    \
   } while (0)
   SEQ_DISPATCH_T(code, {

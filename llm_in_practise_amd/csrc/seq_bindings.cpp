@@ -73,9 +73,8 @@ void seq_residual_dyt(int, int, const float*, const void*, int, float, float*, i
                       SeqDesc, hipStream_t);
 void seq_softcap(float*, size_t, float, hipStream_t);
 void seq_selective_scan(int, const void*, int, const float*, const float*, const void*, int, const void*, int, const float*,
-                        const float*, const void*, int, float*, void*, int, float, int, int, float*, SeqDesc, hipStream_t);
-int seq_selective_segment(int, int, int, int);
-size_t seq_selective_floats(int, int, int, int);
+                        const float*, const void*, int, float*, void*, int, float, int, int, float*, size_t, SeqDesc, hipStream_t);
+size_t seq_selective_floats(int, int, int, int, size_t);
 void seq_gla_scan(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float,
                   float*, float*, int, int, int, SeqDesc, hipStream_t);
 int seq_dyt_max_taps();
@@ -98,18 +97,18 @@ void seq_delta_scan(int, const void*, int, const void*, int, const void*, int, c
 void seq_talk_attention(int, const void*, int, const void*, const void*, float*, float*, float*, const float*,
                         const void*, int, void*, int, int, int, int, int, int, float, const int*, const int*, int,
                         SeqDesc, hipStream_t);
-size_t seq_chunk_floats(int, const void*, int, const void*, int, const void*, int, int, int, int, int, int);
+size_t seq_chunk_floats(int, const void*, int, const void*, int, const void*, int, int, int, int, int, int, size_t);
 void seq_chunk_ssd(const void*, int, const void*, int, const void*, int, const void*, int, const float*, const float*,
-                   const float*, float*, float*, float*, int, int, int, int, SeqDesc, hipStream_t);
+                   const float*, float*, float*, float*, size_t, int, int, int, int, SeqDesc, hipStream_t);
 void seq_chunk_mlstm(const void*, int, const void*, int, const void*, int, const float*, const float*, const float*,
-                     const float*, float, float, float*, float*, float*, float*, float*, float*, float*, int, int, int, SeqDesc,
-                     hipStream_t);
+                     const float*, float, float, float*, float*, float*, float*, float*, float*, float*, size_t, int, int, int,
+                     SeqDesc, hipStream_t);
 size_t seq_block_floats(int, bool, const void*, int, const void*, int, const void*, const void*, const void*, int, int, int, int,
-                        int);
+                        int, size_t);
 void seq_block_delta(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float*, float*, float*,
-                     int, int, int, int, SeqDesc, hipStream_t);
+                     size_t, int, int, int, int, SeqDesc, hipStream_t);
 void seq_block_gla(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float, float*,
-                   float*, float*, int, int, int, SeqDesc, hipStream_t);
+                   float*, float*, size_t, int, int, int, SeqDesc, hipStream_t);
 int seq_scan_max_dk();
 int seq_conv_max_head();
 int seq_conv_max_taps();
@@ -325,9 +324,13 @@ static void check_state(const Tensor& S, int64_t H, int64_t dv, int64_t dk) {
 }
 
 // returns {numerators S^T q [T, H, dv], n.q [T, H], e^-m [T, H]}: the read-out kernel divides
+// The chunked and blocked scans and the selective scan cut over time keep at most this many floats beside their outputs (the
+// argument `most`): a longer step runs in windows of its sequences, or token by token.
+constexpr int64_t MOST_WS = 1ll << 28;
+
 std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor fpre, Tensor ib, Tensor fb, double cap,
                   double qscale, Tensor S, Tensor N, Tensor M, int64_t H, std::vector<Tensor> desc,
-                  optional<Tensor> live) {
+                  optional<Tensor> live, int64_t most) {
   const int code = code_of(q);
   const int64_t T = q.size(0);
   TORCH_CHECK(q.dim() == 2 && q.size(1) % H == 0 && v.dim() == 2 && v.size(1) % H == 0, "q/k/v: [T, H * d]");
@@ -350,12 +353,12 @@ std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor
   auto out = at::empty({T, H, dv}, S.options());
   auto den = at::empty({T, H}, S.options()), efl = at::empty({T, H}, S.options());
   if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), (int)T, d.B, (int)H,
-                                        (int)dk, (int)dv)) {
+                                        (int)dk, (int)dv, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_chunk_mlstm(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
                     fpre.data_ptr<float>(), ib.data_ptr<float>(), fb.data_ptr<float>(), (float)cap, (float)qscale,
                     S.data_ptr<float>(), N.data_ptr<float>(), M.data_ptr<float>(), out.data_ptr<float>(), den.data_ptr<float>(),
-                    efl.data_ptr<float>(), ws.data_ptr<float>(), (int)H, (int)dk, (int)dv, d, stream());
+                    efl.data_ptr<float>(), ws.data_ptr<float>(), (size_t)most, (int)H, (int)dk, (int)dv, d, stream());
     return {out, den, efl};
   }
   seq_mlstm_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
@@ -366,7 +369,7 @@ std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor
 }
 
 Tensor delta_scan(Tensor q, Tensor k, Tensor v, Tensor g, Tensor bpre, Tensor S, int64_t H, int64_t G,
-                  std::vector<Tensor> desc, optional<Tensor> live) {
+                  std::vector<Tensor> desc, optional<Tensor> live, int64_t most) {
   const int code = code_of(q);
   const int64_t T = q.size(0);
   TORCH_CHECK(G >= 1 && H % G == 0 && q.dim() == 2 && q.size(1) % G == 0 && v.dim() == 2 && v.size(1) % H == 0,
@@ -383,11 +386,11 @@ Tensor delta_scan(Tensor q, Tensor k, Tensor v, Tensor g, Tensor bpre, Tensor S,
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H, dv}, S.options());
   if (const size_t n = seq_block_floats(code, true, q.data_ptr(), ld(q), k.data_ptr(), ld(k), g.data_ptr(), nullptr,
-                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv)) {
+                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_block_delta(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), g.data_ptr<float>(),
-                    bpre.data_ptr<float>(), S.data_ptr<float>(), out.data_ptr<float>(), ws.data_ptr<float>(), (int)H, (int)G,
-                    (int)dk, (int)dv, d, stream());
+                    bpre.data_ptr<float>(), S.data_ptr<float>(), out.data_ptr<float>(), ws.data_ptr<float>(), (size_t)most, (int)H,
+                    (int)G, (int)dk, (int)dv, d, stream());
     return out;
   }
   seq_delta_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), g.data_ptr<float>(),
@@ -442,7 +445,7 @@ Tensor talk_attention(Tensor q, Tensor kc, Tensor vc, Tensor talk, Tensor gate, 
 
 // ---- selective state space (state-space duality form): q = C, k = B [T, G * N], v = x [T, H * P], dtraw [T, H]
 Tensor ssd_scan(Tensor q, Tensor k, Tensor v, Tensor dtraw, Tensor dt_bias, Tensor a_log, Tensor dskip, Tensor S,
-                int64_t H, int64_t G, std::vector<Tensor> desc, optional<Tensor> live) {
+                int64_t H, int64_t G, std::vector<Tensor> desc, optional<Tensor> live, int64_t most) {
   const int code = code_of(q);
   const int64_t T = q.size(0);
   TORCH_CHECK(G >= 1 && H % G == 0 && q.dim() == 2 && q.size(1) % G == 0 && v.dim() == 2 && v.size(1) % H == 0,
@@ -461,11 +464,11 @@ Tensor ssd_scan(Tensor q, Tensor k, Tensor v, Tensor dtraw, Tensor dt_bias, Tens
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H * dv}, S.options());
   if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), (int)T, d.B, (int)H,
-                                        (int)dk, (int)dv)) {
+                                        (int)dk, (int)dv, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_chunk_ssd(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), dtraw.data_ptr(), ld(dtraw),
                   dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), dskip.data_ptr<float>(), S.data_ptr<float>(),
-                  out.data_ptr<float>(), ws.data_ptr<float>(), (int)H, (int)G, (int)dk, (int)dv, d, stream());
+                  out.data_ptr<float>(), ws.data_ptr<float>(), (size_t)most, (int)H, (int)G, (int)dk, (int)dv, d, stream());
     return out;
   }
   seq_ssd_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), dtraw.data_ptr(), ld(dtraw),
@@ -1121,7 +1124,7 @@ Tensor softcap_(Tensor z, double cap) {
 
 // x, z [T, C], b, c [T, N] activation rows, dt_pre float [T, C] contiguous; S float [slots, C, N] in place
 Tensor selective_scan(Tensor x, Tensor dt_pre, Tensor dt_bias, Tensor b, Tensor c, Tensor a_log, Tensor d_skip, Tensor z,
-                      Tensor S, std::vector<Tensor> desc, optional<Tensor> live, optional<Tensor> out_, double scale) {
+                      Tensor S, std::vector<Tensor> desc, optional<Tensor> live, optional<Tensor> out_, double scale, int64_t most) {
   const int code = code_of(x);
   TORCH_CHECK(x.dim() == 2 && b.dim() == 2, "x: [T, C], b: [T, N]");
   const int64_t T = x.size(0), C = x.size(1), N = b.size(1);
@@ -1148,17 +1151,17 @@ Tensor selective_scan(Tensor x, Tensor dt_pre, Tensor dt_bias, Tensor b, Tensor 
   }
   if (T == 0) return out;
   Tensor ws;
-  if (const size_t n = seq_selective_floats((int)T, d.B, (int)C, (int)N)) ws = at::empty({(int64_t)n}, S.options());
+  if (const size_t n = seq_selective_floats((int)T, d.B, (int)C, (int)N, (size_t)most)) ws = at::empty({(int64_t)n}, S.options());
   seq_selective_scan(code, x.data_ptr(), ld(x), dt_pre.data_ptr<float>(), dt_bias.data_ptr<float>(), b.data_ptr(), ld(b),
                      c.data_ptr(), ld(c), a_log.data_ptr<float>(), d_skip.data_ptr<float>(), z.data_ptr(), ld(z),
                      S.data_ptr<float>(), out.data_ptr(), ld(out), (float)scale, (int)C, (int)N,
-                     ws.defined() ? ws.data_ptr<float>() : nullptr, d, stream());
+                     ws.defined() ? ws.data_ptr<float>() : nullptr, (size_t)most, d, stream());
   return out;
 }
 
 // q, k [T, H * dk], v [T, H * dv] activation rows, z float [T, H * dk] contiguous; S float [slots, H, dv, dk] in place
 Tensor gated_linear_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, double tau, double q_scale, Tensor S,
-                         int64_t H, std::vector<Tensor> desc, optional<Tensor> live) {
+                         int64_t H, std::vector<Tensor> desc, optional<Tensor> live, int64_t most) {
   const int code = code_of(q);
   TORCH_CHECK(H >= 1 && q.dim() == 2 && q.size(1) % H == 0 && v.dim() == 2 && v.size(1) % H == 0,
               "q/k: [T, H * dk], v: [T, H * dv]");
@@ -1175,11 +1178,11 @@ Tensor gated_linear_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, 
   auto out = at::empty({T, H, dv}, S.options());
   if (T == 0) return out;
   if (const size_t n = seq_block_floats(code, false, q.data_ptr(), ld(q), k.data_ptr(), ld(k), z.data_ptr(), z_bias.data_ptr(),
-                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv)) {
+                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_block_gla(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), z.data_ptr<float>(),
                   z_bias.data_ptr<float>(), (float)(1.0 / tau), (float)q_scale, S.data_ptr<float>(), out.data_ptr<float>(),
-                  ws.data_ptr<float>(), (int)H, (int)dk, (int)dv, d, stream());
+                  ws.data_ptr<float>(), (size_t)most, (int)H, (int)dk, (int)dv, d, stream());
     return out;
   }
   seq_gla_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), z.data_ptr<float>(),
@@ -1275,10 +1278,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("short_conv", &short_conv, py::arg("u"), py::arg("w"), py::arg("state"), py::arg("segs"), py::arg("seg_w"),
         py::arg("seg_scale"), py::arg("desc"), py::arg("live"), py::arg("eps"), py::arg("out_f32"),
         py::arg("bias") = py::none());
-  m.def("mlstm_scan", &mlstm_scan);
-  m.def("delta_scan", &delta_scan);
+  m.def("mlstm_scan", &mlstm_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("ipre"), py::arg("fpre"), py::arg("ib"),
+        py::arg("fb"), py::arg("cap"), py::arg("qscale"), py::arg("S"), py::arg("N"), py::arg("M"), py::arg("H"),
+        py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS);
+  m.def("delta_scan", &delta_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("g"), py::arg("bpre"), py::arg("S"),
+        py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS);
   m.def("talk_attention", &talk_attention);
-  m.def("ssd_scan", &ssd_scan);
+  m.def("ssd_scan", &ssd_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("dtraw"), py::arg("dt_bias"),
+        py::arg("a_log"), py::arg("dskip"), py::arg("S"), py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"),
+        py::arg("most") = MOST_WS);
   m.def("embed_pair", &embed_pair, py::arg("tok"), py::arg("table"), py::arg("pair"), py::arg("prev"), py::arg("scale"),
         py::arg("mul_prev"), py::arg("mul_cur"), py::arg("desc"), py::arg("live"), py::arg("out") = py::none());
   m.def("scaled_postnorm", &scaled_postnorm);
@@ -1301,11 +1309,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sigmoid_gate", &sigmoid_gate);
   m.def("residual_dyt", &residual_dyt);
   m.def("softcap_", &softcap_);
-  m.def("selective_segment", [](int64_t T, int64_t B, int64_t C, int64_t N) {        // 0: sequences run whole
-    return seq_selective_segment((int)T, (int)B, (int)C, (int)N);
-  });
-  m.def("selective_scan", &selective_scan);
-  m.def("gated_linear_scan", &gated_linear_scan);
+  m.def("selective_floats", [](int64_t T, int64_t B, int64_t C, int64_t N, int64_t most) {        // 0: sequences run whole
+    return (int64_t)seq_selective_floats((int)T, (int)B, (int)C, (int)N, (size_t)most);
+  }, py::arg("T"), py::arg("B"), py::arg("C"), py::arg("N"), py::arg("most") = MOST_WS);
+  m.def("selective_scan", &selective_scan, py::arg("x"), py::arg("dt_pre"), py::arg("dt_bias"), py::arg("b"), py::arg("c"),
+        py::arg("a_log"), py::arg("d_skip"), py::arg("z"), py::arg("S"), py::arg("desc"), py::arg("live"), py::arg("out"),
+        py::arg("scale"), py::arg("most") = MOST_WS);
+  m.def("gated_linear_scan", &gated_linear_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("z"), py::arg("z_bias"),
+        py::arg("tau"), py::arg("q_scale"), py::arg("S"), py::arg("H"), py::arg("desc"), py::arg("live"),
+        py::arg("most") = MOST_WS);
   m.def("delta_rule_gates", &delta_rule_gates);
   m.def("general_delta_scan", &general_delta_scan);
 }

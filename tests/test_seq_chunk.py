@@ -304,7 +304,7 @@ def test_selective_cut_over_time(lens, starts, C, N, dt):
 def test_selective_is_cut_only_where_it_is_not_slower(T, B, C, N, cut):
     """Timed shapes on both sides of the rule: the work of a token grows with its states, what a cut saves does not."""
     from llm_in_practise_amd.ops._native import native_seq
-    assert (native_seq().selective_segment(T, B, C, N) > 0) == cut
+    assert (native_seq().selective_floats(T, B, C, N) > 0) == cut
 
 
 @pytest.mark.gpu
@@ -323,5 +323,68 @@ def test_selective_cut_with_many_states(N):
         p = [t.to(dev) for t in (x, dtp, dtb, bc[:, :N], bc[:, N:], a_log, skip, z)]
         res.append((R.selective_scan(*p, st["S"], sb), st["S"]))
     from llm_in_practise_amd.ops._native import native_seq
-    assert native_seq().selective_segment(T, len(lens), C, N) > 0
+    assert native_seq().selective_floats(T, len(lens), C, N) > 0
     _close(res[1], res[0], ("y", "state"))
+
+
+def _scans(lens, starts, g):
+    """The five scans over one packed step: name -> (run() -> outputs and states, floats of workspace per slot, tokens of a slot)."""
+    T, B = sum(lens), len(lens)
+
+    def rand(*s, dt=torch.float32):
+        return torch.randn(*s, generator=g).to(dt).cuda()
+    H, dk, dv = 3, 64, 32
+    bf = torch.bfloat16
+    q, k, v = rand(T, H * dk, dt=bf), rand(T, H * dk, dt=bf), rand(T, H * dv, dt=bf)
+    dt, dtb, a_log, skip = rand(T, H, dt=bf), rand(H), rand(H), rand(H)
+    i, f = 4 * rand(T, H), 3 * rand(T, H)
+    decay, z, zb = torch.rand(T, H * dk, generator=g).cuda() ** 0.2, 3 * rand(T, H * dk), rand(H * dk)
+    kn = torch.nn.functional.normalize(k.float().view(T, H, dk), dim=-1).view(T, -1).to(bf)
+    C, N = 64, 16
+    sel = [rand(T, C), rand(T, C), rand(C) - 2, rand(T, N), rand(T, N), rand(C, N), rand(C), rand(T, C)]
+    mat = {"S": ((H, dv, dk), "f32")}
+
+    def go(spec, fn):
+        def run():
+            st, sb = _batch(spec, lens, starts, "cuda")
+            for s in st.values():
+                s.fill_(0.25)
+            out = fn(st, sb)
+            return [*(out if isinstance(out, (tuple, list)) else [out]), *st.values()]
+        return run
+    return {
+        "ssd": (go(mat, lambda st, sb: R.ssd_scan(q, k, v, dt, dtb, a_log, skip, st["S"], H, H, sb)), H * (6 + dk * (dv + 1)), 128),
+        "mlstm": (go({**mat, "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lambda st, sb: R.mlstm_scan(
+            q, k, v, i, f, dtb, dtb + 3, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb)), H * (6 + dk * (dv + 1)), 128),
+        "delta": (go(mat, lambda st, sb: R.gated_delta_scan(q, kn, v, decay, i, st["S"], H, H, sb)), H * (49 * dk + 516), 16),
+        "gla": (go(mat, lambda st, sb: R.gated_linear_scan(q, k, v, z, zb, 16.0, dk ** -0.5, st["S"], H, sb)),
+                H * (49 * dk + 516), 16),
+        "selective": (go({"S": ((C, N), "f32")}, lambda st, sb: R.selective_scan(*sel, st["S"], sb)), C * (N + 1), 32),
+    }
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["ssd", "mlstm", "delta", "gla", "selective"])
+@pytest.mark.parametrize("lens,starts", [([2100], [0]), ([1500, 1, 900, 640], [0, 0, 3, 512])])
+@pytest.mark.parametrize("count", [0, 1, 5, 100])
+def test_scans_in_windows_of_a_bounded_workspace(monkeypatch, name, lens, starts, count):
+    """Room for `count` slots a sequence: the same outputs and states window after window (or token by token, with no room or too
+    many windows), and no more memory than allowed."""
+    import functools
+    from llm_in_practise_amd.ops import _native
+    run, per, _ = _scans(lens, starts, torch.Generator().manual_seed(len(lens)))[name]
+    want = run()
+    seq, most = _native.native_seq(), count * per * len(lens) + 8
+    asked = {"ssd": "ssd_scan", "mlstm": "mlstm_scan", "delta": "delta_scan", "gla": "gated_linear_scan", "selective": "selective_scan"}
+
+    class Bounded:
+        def __getattr__(self, a):
+            return functools.partial(getattr(seq, a), most=most) if a == asked[name] else getattr(seq, a)
+    monkeypatch.setattr(R, "native_seq", Bounded)
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    got = run()
+    held = 4 * sum(t.numel() for t in got) + 4 * 4 * sum(lens)      # outputs, states, descriptors (rounded up to 512 bytes each)
+    assert torch.cuda.max_memory_allocated() - base <= held + 4 * most + 512 * 32
+    _close(got, want, [str(j) for j in range(len(got))])
