@@ -392,8 +392,21 @@ size_t seq_block_floats(int code, bool delta, const void* q, int ldq, const void
   // cheaper one.  us, tokens -> blocks, heads of 128 x 128 (delta) and 64 x 128: 64 delta heads (512 blocks) at 32 tokens 19 -> 16,
   // at 512 201 -> 83; 384 heads at 48 tokens 69 -> 73, at 64 88 -> 85, at 256 318 -> 290.  Linear attention: 64 heads at 32
   // tokens 11 -> 12, at 48 15 -> 12, at 512 119 -> 44; 128 heads at 48 16 -> 17, at 64 20 -> 19; 384 heads at 256 100 -> 120.
-  const long blocks = (long)B * H * ((dv + 15) / 16);
-  const long least = delta ? (blocks <= 1024 ? 32 : 64) : blocks <= 512 ? 40 : blocks <= 1536 ? 64 : 1L << 40;
+  // Many (sequence, head) pairs of few columns, or of keys of 64, leave the token form nothing to wait for, at any length: times its
+  // time, delta, 1024 pairs of 64 x 64 2.0, of 128 x 32 1.1, 4096 of 128 x 64 1.1, 256 of 64 x 256 1.2 (of 64 x 128 0.95 from 96 tokens on,
+  // of 128 x 32 1.2 at 64, 0.7 at 128); linear attention, 256 of 128 x 64 1.06, of 256 x 32 1.15 (of 64 x 32 1.07 at 64, 0.91 at 128).
+  const long pairs = (long)B * H, blocks = pairs * ((dv + 15) / 16), never = 1l << 40;
+  long least;
+  if (delta) {
+    least = pairs < 128 && blocks <= 1024 ? 32 : 64;
+    if (pairs >= 256 && dv <= 64) least = dv <= 32 ? 128 : 96;
+    if (dk == 64 && blocks > 1024) least = 96;
+    if ((dk == 64 && (pairs > 512 || blocks >= 4096)) || (dv <= 32 && pairs >= 1024) || (dv <= 64 && pairs >= 4096)) least = never;
+  } else if (pairs >= 256) {
+    least = blocks <= 512 && dk <= 192 ? 128 : never;
+  } else {
+    least = blocks > 1536 ? never : blocks > 512 || dk == 64 ? 64 : 40;
+  }
   if (T_ < least * B) return 0;
   return block_plan(T_, B, H, dk, most).slots * slot_floats(H, dk);
 }

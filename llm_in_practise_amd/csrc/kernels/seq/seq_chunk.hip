@@ -18,6 +18,8 @@
 // chunk's scores grow with its square.
 #include "seq_common.h"
 
+#include <algorithm>
+
 using namespace lipa;
 
 namespace {
@@ -601,10 +603,18 @@ size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk
                         int dk, int dv, size_t most) {
   const auto fits = [](const void* p, int ld, int n) { return ld % n == 0 && ((uintptr_t)p & (2 * n - 1)) == 0; };
   if (code != 0 || dk % 32 != 0 || dk > 128 || dv % 4 != 0 || !fits(q, ldq, 8) || !fits(k, ldk, 8) || !fits(v, ldv, 4)) return 0;
-  // three launches and a chunk of padding against 0.4 us a token (two heads a CU) in the token-by-token form: 64 tokens a
+  // Three launches and a chunk of padding against 0.4 us a token (two heads a CU) in the token-by-token form: 64 tokens a
   // sequence are 21 / 32 / 96 us here and 30 / 36 / 148 us there (state space, 32 heads, 1 / 8 / 48 sequences), 48 are 21 / 32 / 94
-  // and 24 / 29 / 118 us; mLSTM (8 heads of 128 x 192) at 64: 26 / 34 / 68 against 31 / 36 / 159 us
-  if (B == 0 || T_ < 64 * B) return 0;
+  // and 24 / 29 / 118 us; mLSTM (8 heads of 128 x 192) at 64: 26 / 34 / 68 against 31 / 36 / 159 us.  The outputs walk the columns 32 at a
+  // time, one after another: 512 of them 43 against 26 us at 64 tokens, even at 128 to 160.  Where (sequence, head) pairs fill the chip,
+  // the padding counts, and with small keys the token form is the cheaper one for longer: 1024 pairs of 64 x 64 take 1.3 times its time at
+  // 64 to 128 tokens, 0.94 at 192; 1024 of 32 x 128 1.2 at 192, 1.08 at 256, 0.92 at 512; 1024 of 128 x 64 are ahead from 64 on.
+  const long pairs = (long)B * H;
+  long least = std::max(64, std::min(dv * 5 / 12, 192));
+  if (pairs >= 256 && dk <= 64 && dv >= 128) least = std::max(least, 96l);
+  if (pairs >= 1024 && (dk <= 64 || dv <= 32)) least = 192;
+  if (pairs * dv >= 1l << 17 && dk <= 32) least = 256;
+  if (B == 0 || T_ < least * B) return 0;
   const size_t slots = chunk_plan(T_, B, H, dk, dv, most).slots;
   return slots == 0 ? 0 : slots * chunk_floats(H, dk, dv) + 4;
 }

@@ -1309,6 +1309,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sigmoid_gate", &sigmoid_gate);
   m.def("residual_dyt", &residual_dyt);
   m.def("softcap_", &softcap_);
+  // workspace of a step through the chunked ("ssd", "mlstm") or blocked ("delta", "gla") form, bf16 rows that its loads take; 0: token by token
+  m.def("scan_floats", [](const std::string& op, int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most) {
+    if (op == "ssd" || op == "mlstm")
+      return (int64_t)seq_chunk_floats(0, nullptr, 8, nullptr, 8, nullptr, 8, (int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most);
+    TORCH_CHECK(op == "delta" || op == "gla", "scan_floats: ssd, mlstm, delta or gla");
+    return (int64_t)seq_block_floats(0, op == "delta", nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H,
+                                     (int)dk, (int)dv, (size_t)most);
+  }, py::arg("op"), py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS);
   m.def("selective_floats", [](int64_t T, int64_t B, int64_t C, int64_t N, int64_t most) {        // 0: sequences run whole
     return (int64_t)seq_selective_floats((int)T, (int)B, (int)C, (int)N, (size_t)most);
   }, py::arg("T"), py::arg("B"), py::arg("C"), py::arg("N"), py::arg("most") = MOST_WS);

@@ -327,6 +327,23 @@ def test_selective_cut_with_many_states(N):
     _close(res[1], res[0], ("y", "state"))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("op,L,B,H,dk,dv,blocked", [
+    ("ssd", 64, 1, 64, 128, 64, True), ("ssd", 63, 1, 64, 128, 64, False), ("ssd", 128, 64, 16, 64, 64, False),
+    ("ssd", 192, 64, 16, 64, 64, True), ("ssd", 64, 64, 16, 128, 64, True), ("ssd", 64, 1, 8, 64, 512, False),
+    ("ssd", 192, 1, 8, 64, 512, True), ("ssd", 192, 64, 16, 32, 128, False), ("mlstm", 64, 16, 8, 64, 96, True),
+    ("mlstm", 72, 8, 8, 128, 192, False), ("mlstm", 80, 8, 8, 128, 192, True), ("mlstm", 80, 64, 4, 64, 128, False),
+    ("delta", 32, 1, 8, 128, 128, True), ("delta", 32, 16, 16, 64, 64, False), ("delta", 1024, 64, 16, 64, 64, False),
+    ("delta", 1024, 64, 16, 64, 128, False), ("delta", 96, 16, 16, 64, 128, True), ("delta", 512, 64, 16, 128, 32, False),
+    ("delta", 128, 16, 16, 128, 32, True), ("delta", 64, 64, 16, 128, 128, True), ("gla", 40, 1, 8, 128, 128, True),
+    ("gla", 48, 1, 8, 64, 128, False), ("gla", 64, 4, 16, 64, 128, True), ("gla", 1024, 16, 16, 256, 64, False),
+    ("gla", 128, 16, 16, 64, 32, True), ("gla", 256, 24, 16, 64, 128, False)])
+def test_chunks_and_blocks_only_where_they_are_not_slower(op, L, B, H, dk, dv, blocked):
+    """Timed shapes on both sides of the choice between chunks or blocks and the token-by-token forms."""
+    from llm_in_practise_amd.ops._native import native_seq
+    assert (native_seq().scan_floats(op, L * B, B, H, dk, dv) > 0) == blocked
+
+
 def _scans(lens, starts, g):
     """The five scans over one packed step: name -> (run() -> outputs and states, floats of workspace per slot, tokens of a slot)."""
     T, B = sum(lens), len(lens)
