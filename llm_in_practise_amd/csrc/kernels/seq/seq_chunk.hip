@@ -597,12 +597,14 @@ void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* 
 }  // namespace
 
 // Floats of workspace of the chunked form, or 0 where the token-by-token scan is the one to run: float activations, key sizes
-// that are no multiple of 32 or above 128, rows that 16-byte (q, k) or 8-byte (v) loads cannot take, and steps of few tokens a
-// sequence.  At most `most`: longer steps run in windows.
-size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, int T_, int B, int H,
-                        int dk, int dv, size_t most) {
+// that are no multiple of 32 or above 128, rows that 16-byte (q, k, the states S and N) or 8-byte (v) loads cannot take, and steps of
+// few tokens a sequence.  At most `most`: longer steps run in windows.
+size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const void* S,
+                        const void* N, int T_, int B, int H, int dk, int dv, size_t most) {
   const auto fits = [](const void* p, int ld, int n) { return ld % n == 0 && ((uintptr_t)p & (2 * n - 1)) == 0; };
-  if (code != 0 || dk % 32 != 0 || dk > 128 || dv % 4 != 0 || !fits(q, ldq, 8) || !fits(k, ldk, 8) || !fits(v, ldv, 4)) return 0;
+  if (code != 0 || dk % 32 != 0 || dk > 128 || dv % 4 != 0 || !fits(q, ldq, 8) || !fits(k, ldk, 8) || !fits(v, ldv, 4) ||
+      !fits(S, 8, 8) || !fits(N, 8, 8))
+    return 0;
   // Three launches and a chunk of padding against 0.4 us a token (two heads a CU) in the token-by-token form: 64 tokens a
   // sequence are 21 / 32 / 96 us here and 30 / 36 / 148 us there (state space, 32 heads, 1 / 8 / 48 sequences), 48 are 21 / 32 / 94
   // and 24 / 29 / 118 us; mLSTM (8 heads of 128 x 192) at 64: 26 / 34 / 68 against 31 / 36 / 159 us.  The outputs walk the columns 32 at a

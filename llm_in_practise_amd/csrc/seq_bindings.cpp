@@ -97,7 +97,8 @@ void seq_delta_scan(int, const void*, int, const void*, int, const void*, int, c
 void seq_talk_attention(int, const void*, int, const void*, const void*, float*, float*, float*, const float*,
                         const void*, int, void*, int, int, int, int, int, int, float, const int*, const int*, int,
                         SeqDesc, hipStream_t);
-size_t seq_chunk_floats(int, const void*, int, const void*, int, const void*, int, int, int, int, int, int, size_t);
+size_t seq_chunk_floats(int, const void*, int, const void*, int, const void*, int, const void*, const void*, int, int, int, int, int,
+                        size_t);
 void seq_chunk_ssd(const void*, int, const void*, int, const void*, int, const void*, int, const float*, const float*,
                    const float*, float*, float*, float*, size_t, int, int, int, int, SeqDesc, hipStream_t);
 void seq_chunk_mlstm(const void*, int, const void*, int, const void*, int, const float*, const float*, const float*,
@@ -352,8 +353,8 @@ std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H, dv}, S.options());
   auto den = at::empty({T, H}, S.options()), efl = at::empty({T, H}, S.options());
-  if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), (int)T, d.B, (int)H,
-                                        (int)dk, (int)dv, (size_t)most)) {
+  if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), S.data_ptr(),
+                                        N.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_chunk_mlstm(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
                     fpre.data_ptr<float>(), ib.data_ptr<float>(), fb.data_ptr<float>(), (float)cap, (float)qscale,
@@ -463,8 +464,8 @@ Tensor ssd_scan(Tensor q, Tensor k, Tensor v, Tensor dtraw, Tensor dt_bias, Tens
   check_state(S, H, dv, dk);
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H * dv}, S.options());
-  if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), (int)T, d.B, (int)H,
-                                        (int)dk, (int)dv, (size_t)most)) {
+  if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), S.data_ptr(), nullptr,
+                                        (int)T, d.B, (int)H, (int)dk, (int)dv, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_chunk_ssd(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), dtraw.data_ptr(), ld(dtraw),
                   dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), dskip.data_ptr<float>(), S.data_ptr<float>(),
@@ -1312,7 +1313,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   // workspace of a step through the chunked ("ssd", "mlstm") or blocked ("delta", "gla") form, bf16 rows that its loads take; 0: token by token
   m.def("scan_floats", [](const std::string& op, int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most) {
     if (op == "ssd" || op == "mlstm")
-      return (int64_t)seq_chunk_floats(0, nullptr, 8, nullptr, 8, nullptr, 8, (int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most);
+      return (int64_t)seq_chunk_floats(0, nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most);
     TORCH_CHECK(op == "delta" || op == "gla", "scan_floats: ssd, mlstm, delta or gla");
     return (int64_t)seq_block_floats(0, op == "delta", nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H,
                                      (int)dk, (int)dv, (size_t)most);

@@ -405,3 +405,46 @@ def test_scans_in_windows_of_a_bounded_workspace(monkeypatch, name, lens, starts
     held = 4 * sum(t.numel() for t in got) + 4 * 4 * sum(lens)      # outputs, states, descriptors (rounded up to 512 bytes each)
     assert torch.cuda.max_memory_allocated() - base <= held + 4 * most + 512 * 32
     _close(got, want, [str(j) for j in range(len(got))])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["ssd", "mlstm", "delta", "gla"])
+@pytest.mark.parametrize("which", ["q", "k", "v", "S", "row"])
+def test_rows_that_wide_loads_cannot_take(op, which):
+    """One operand a single element off, or rows of odd length: the same outputs and states as for aligned copies."""
+    lens, H, dk, dv, bf = [200, 90], 2, 64, 32, torch.bfloat16
+    g = torch.Generator().manual_seed(len(op))
+    T = sum(lens)
+    base = {n: torch.randn(T, H * w, generator=g).to(bf).cuda() for n, w in (("q", dk), ("k", dk), ("v", dv))}
+    if op == "delta":
+        base["k"] = torch.nn.functional.normalize(base["k"].float().view(T, H, dk), dim=-1).view(T, -1).to(bf)
+    i, f = torch.randn(T, H, generator=g).cuda(), torch.randn(T, H, generator=g).cuda()
+    decay, z, zb = torch.rand(T, H * dk, generator=g).cuda() ** 0.2, torch.randn(T, H * dk, generator=g).cuda(), torch.zeros(H * dk).cuda()
+    b = torch.randn(H, generator=g).cuda()
+
+    def off(t, by):                                     # the same values, `by` elements behind an aligned address
+        return torch.cat([t.new_zeros(by), t.reshape(-1)])[by:].view(t.shape)
+
+    def run(odd):
+        x = dict(base)
+        if odd and which == "row":
+            x = {n: torch.cat([t, t.new_zeros(T, 1)], 1)[:, :-1] for n, t in x.items()}
+        elif odd and which in x:
+            x[which] = off(x[which], 1)
+        spec = {"S": ((H, dv, dk), "f32")} | ({"N": ((H, dk), "f32"), "M": ((H,), "f32")} if op == "mlstm" else {})
+        st, sb = _batch(spec, lens, [0, 3], "cuda")
+        for s in st.values():
+            s.fill_(0.5)
+        if odd and which == "S":
+            st["S"] = off(st["S"], 1)
+        if op == "ssd":
+            o = R.ssd_scan(x["q"], x["k"], x["v"], i.to(bf), b, b, b, st["S"], H, H, sb)
+        elif op == "mlstm":
+            o = R.mlstm_scan(x["q"], x["k"], x["v"], i, f, b, b + 3, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb)
+        elif op == "delta":
+            o = R.gated_delta_scan(x["q"], x["k"], x["v"], decay, i, st["S"], H, H, sb)
+        else:
+            o = R.gated_linear_scan(x["q"], x["k"], x["v"], z, zb, 16.0, dk ** -0.5, st["S"], H, sb)
+        return [*(o if isinstance(o, (tuple, list)) else [o]), *st.values()]
+    got, want = run(True), run(False)
+    _close(got, want, [str(j) for j in range(len(got))])
