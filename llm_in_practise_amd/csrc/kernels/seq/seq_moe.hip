@@ -471,8 +471,10 @@ void seq_route_fused(int code, const void* h, int ldh, const float* router, cons
                      int always, hipStream_t st) {
   if (T_ == 0) return;
   const auto fits = [](const void* p, int b) { return ((uintptr_t)p & (b - 1)) == 0; };
-  // (below 256 tokens a block of 16 waves per token fills the chip better: 8 us at any number up to 200)
-  if (T_ >= 256 && n <= 16 && top + always <= 16 && W % 4 == 0 && ldh % 4 == 0 && fits(h, code == 0 ? 8 : 16) && fits(router, 16)) {
+  // (Below 256 tokens a block of 16 waves per token fills the chip better: 8 us at any number up to 200.  Rows above 8 KB are a long
+  // way for four waves, which only pays with many tokens: 1000 of width 8192, 12 outputs, 32 against 24 us in bf16, 512 in float 28 against
+  // 20; from 2000 on ahead.)
+  if (T_ >= 256 && (W * (code == 0 ? 2 : 4) <= 8192 || T_ >= 2000) && n <= 16 && top + always <= 16 && W % 4 == 0 && ldh % 4 == 0 && fits(h, code == 0 ? 8 : 16) && fits(router, 16)) {
 #define ROUTE_ROWS(NG_)                                                                                                      \
   hipLaunchKernelGGL((k_route_rows<T, NG_>), dim3((T_ + 3) / 4), dim3(256), 0, st, (const T*)h, ldh, router, corr, idx, w, T_, n,    \
                      W, top, groups, keep, scale, kind, extra, xout, always)

@@ -76,3 +76,16 @@ def test_routing_of_prompts(T, n, W, top, groups, keep, kw, dt):
     assert (got[1].cpu() - want[1])[same].abs().max() <= 1e-5 * max(1.0, kw.get("scale", 1.0))
     if kw.get("extra"):
         torch.testing.assert_close(got[2].cpu(), want[2], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,W,dt", [(1999, 4160, torch.bfloat16), (2000, 4160, torch.bfloat16), (300, 4096, torch.bfloat16),
+                                    (300, 2048, torch.float32), (300, 2052, torch.float32), (2001, 2052, torch.float32)])
+def test_routing_of_wide_rows(T, W, dt):
+    """On both sides of the width and the number of tokens from which four tokens share a block."""
+    g = torch.Generator().manual_seed(T + W)
+    h, router = torch.randn(T, W, generator=g).to(dt), torch.randn(12, W, generator=g) * W ** -0.5
+    got = M.route_tokens(h.cuda(), router.cuda(), torch.zeros(12).cuda(), 3, 1, 1, normalize=True)
+    want = M.route_tokens(h, router, torch.zeros(12), 3, 1, 1, normalize=True)
+    same = (got[0].cpu() == want[0]).all(1)             # (a choice can only differ where two scores are that close)
+    assert same.float().mean() >= 0.995 and (got[1].cpu() - want[1])[same].abs().max() <= 1e-5
