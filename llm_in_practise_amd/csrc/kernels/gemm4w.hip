@@ -149,9 +149,10 @@ G4wCfg gemm4w_cfg(int M, int N, int K, bool bt, int bn_req, int sp_req, int bm_r
   if (sp_req > 0) best.splits = std::min(sp_req, 8);
   if (w4) return best;
   // The tile again for those splits (they fix the order of a product's sums, the tile does not), at what the tiles take over
-  // several rounds: the 128-high ones 0.62 of the 256-high, the 128-wide ones 0.97 µs a K-tile, and 6 µs a round to fill and empty it.  Of 216
-  // shapes of 256 .. 8192 rows none gets slower by more than 2 %; 4700 rows of 24576 × 4096 894 → 775 µs, 2451 of
-  // 4096 × 12288 (4 splits) 291 → 272, 700 of it (8) 112 → 100.
+  // several rounds: the 128-high ones 0.62 of the 256-high, the 128-wide ones 0.97 µs a K-tile, and 6 µs a round to fill and empty it.  (The
+  // numbers above are those of one round; they stay for the splits alone, whose choice would move a product's bits.)  Of 288 shapes of
+  // 256 .. 8192 rows, W either way (profiles/gemm4w_tiles.txt), none gets slower by more than 4 %, where two runs of one side differ by
+  // up to 9; 4700 rows of 24576 × 4096 849 → 755 µs, 2451 of 4096 × 12288 (4 splits) 298 → 278, 700 of it (8) 113 → 104.
   best_t = 1e30;
   const int s = best.splits;
   for (int bm : {256, 128}) {

@@ -11,9 +11,9 @@
 // (v_mfma_f32_16x16x4_f32), whose result layout is also its operand layout: the state, u and the outputs never move
 // between lanes.
 //
-// Measured, token by token -> blocks: three sequences of 1500, 700 and 97 tokens, 8 delta heads of 128 x 128: 576 -> 110 us (25
-// for the first kernel, 88 for the walk); eight sequences of 512 tokens, 16 linear-attention heads of 64 x 128: 119 -> 69 us.
-// Error against 64 bits as before (2e-7).  Ten inputs a lane two or three blocks ahead gave 2.0 -> 0.94 us a block of the longest
+// Measured, token by token -> blocks: three sequences of 1500, 700 and 97 tokens, 8 delta heads of 128 x 128: 576 -> 112 us (26
+// for the first kernel, 86 for the walk); eight sequences of 512 tokens, 16 linear-attention heads of 64 x 128: 119 -> 71 us.
+// Error against 64 bits as before (2.1e-7).  Ten inputs a lane two or three blocks ahead gave 2.0 -> 0.94 us a block of the longest
 // sequence.
 #include "seq_common.h"
 

@@ -11,9 +11,9 @@
 // numbers, which hold its 24 bits: three products with float sums, at five times the rate of the float matrix units.  Log
 // decays are summed in 64 bits and kept as two floats, so that the difference of two large sums is exact.
 //
-// Measured, token by token -> chunks: state space, one prompt of 4093 tokens, 64 heads of 128 x 64: 2344 -> 144 us (state 45,
-// walk 24, outputs 78); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 92 us (38, 18, 38).  Error against
-// 64 bits 1.5e-7 -> 1.0e-7 and 4.8e-7 -> 2.0e-7: fewer roundings stand between a token and the outputs far behind it.
+// Measured, token by token -> chunks: state space, one prompt of 4093 tokens, 64 heads of 128 x 64: 2350 -> 151 us (state 46,
+// walk 25, outputs 80); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 94 us (36, 17, 41; under the profiler 39, 18,
+// 41).  Error against 64 bits 1.6e-7 -> 0.8e-7 and 4.4e-7 -> 1.9e-7: fewer roundings stand between a token and the outputs far behind it.
 // Chunks of 128 tokens: the states of a step pass through memory once per chunk (69 MB of the first case, three times), and a
 // chunk's scores grow with its square.
 #include "seq_common.h"

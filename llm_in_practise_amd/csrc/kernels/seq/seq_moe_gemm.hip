@@ -3,8 +3,8 @@
 // gathers its rows of the input as it loads them and ends in the gated activation, so neither the gathered input nor the gate
 // and up products ever stand in memory.
 //
-// 8000 tokens of width 2048, 8 experts of 384, top 2 (75 GFLOP): 634 -> 176 us with routing and the weighted sum: order 13, first
-// products 69 (730 TFLOP/s), second 38, sum 27, routing 18.  100 tokens: 533 -> 48 us.  The sort, the host's read of the run lengths
+// 8000 tokens of width 2048, 8 experts of 384, top 2 (75 GFLOP): 638 -> 175 us with routing and the weighted sum: order 13, first
+// products 71 (710 TFLOP/s), second 39 (650), sum 27, routing 18.  100 tokens: 533 -> 48 us.  The sort, the host's read of the run lengths
 // and a vendor product pair, an activation and their launch gaps per expert took 500 us at any number of tokens.
 #include "seq_common.h"
 

@@ -87,7 +87,7 @@ __device__ __forceinline__ void store_state(float* p, int i0, int len, const flo
 // chip is cut over time (k_selective_walk and the two cut modes): every segment of 32 or 64 tokens first runs from a zero state for
 // the state it leaves and the sum of its step sizes (its decay is e^{A sum dt}), a walk over a sequence's segments turns those
 // into the states in front of the segments, and every segment then runs from its own.  Two prompts of 2048 and 1337 tokens, 4096
-// channels of 16 states: 464 -> 125 us (49 for what segments leave, 15, 72: bound by one
+// channels of 16 states: 464 -> 127 us (50 for what segments leave, 16, 73: bound by one
 // quarter-rate exponential per channel, state and token).
 constexpr int CH = 2;
 enum { WHOLE, LEAVES, FROM };       // a sequence; a segment from zero (state and step sizes); a segment from the state before it
