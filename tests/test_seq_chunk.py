@@ -111,6 +111,41 @@ def test_mlstm_chunks_keep_decays_of_a_wide_cap():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B,H,dk,dv,L", [(1, 8, 128, 192, 1), (30, 8, 128, 192, 1), (96, 8, 64, 96, 1), (200, 4, 128, 64, 1),
+                                         (64, 8, 128, 192, 17), (3, 2, 16, 300, 1)])
+def test_mlstm_blocks_of_columns_read_the_old_maximum(B, H, dk, dv, L):
+    """More blocks of columns than run at once: those that start after others have ended decay by the maximum from before the step,
+    which every step raises here."""
+    g = torch.Generator().manual_seed(B)
+    T = B * L
+    q, k, v = (torch.randn(T, H * n, generator=g).bfloat16() for n in (dk, dk, dv))
+    i, f = 6.0 + torch.randn(T, H, generator=g), torch.randn(T, H, generator=g)
+    st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, [L] * B, [5] * B, "cuda",
+                    [int(b != 2) for b in range(B)])
+    for t in st.values():
+        t.fill_(0.25)
+    bias = torch.zeros(H, device="cuda")
+    got = R.mlstm_scan(q.cuda(), k.cuda(), v.cuda(), i.cuda(), f.cuda(), bias, bias + 3, 15.0, dk ** -0.5, st["S"], st["N"], st["M"],
+                       H, sb)
+    q, k, v, i, f = (x.double().view(B, L, H, -1) for x in (q, k, v, i, f))
+    ig, fg = 15.0 * torch.tanh(i / 15.0), torch.nn.functional.logsigmoid(15.0 * torch.tanh((f + 3) / 15.0))
+    S, N, M = (torch.full(s, 0.25, dtype=torch.float64) for s in ((B, H, dv, dk), (B, H, dk), (B, H, 1)))
+    want = [torch.empty(B, L, H, dv).double(), torch.empty(B, L, H).double(), torch.empty(B, L, H).double()]
+    for t in range(L):
+        m = torch.maximum(fg[:, t] + M, ig[:, t])
+        a, c, M = torch.exp(fg[:, t] + M - m), torch.exp(ig[:, t] - m), m
+        S = a[..., None] * S + (c * v[:, t])[..., None] * k[:, t, :, None]
+        N = a * N + c * k[:, t]
+        want[0][:, t], want[1][:, t] = (S * q[:, t, :, None]).sum(-1) * dk ** -0.5, (N * q[:, t]).sum(-1) * dk ** -0.5
+        want[2][:, t] = torch.exp(-m[..., 0])
+    on = torch.arange(B) != 2                           # (an idle row's outputs are nobody's, and its state stays)
+    _close([x.view(B, L, *x.shape[1:])[on.cuda()] for x in got], [x[on] for x in want], ("o", "den", "floor"))
+    for x, y in zip(st.values(), (S, N, M[..., 0])):    # (slots are the sequences in reverse)
+        assert B < 3 or (x.flip(0)[2] == 0.25).all()
+        _close([x.flip(0)[on.cuda()]], [y[on]], ["state"])
+
+
+@pytest.mark.gpu
 def test_idle_sequences_keep_their_state():
     lens, H, dk, dv = [130, 200, 70], 2, 64, 32
     g = torch.Generator().manual_seed(0)
