@@ -364,9 +364,86 @@ __global__ __launch_bounds__(256) void k_mlstm_scan(const T* __restrict__ q, int
   if (cb == 0 && tid == 0) top[blockIdx.x] = m;
 }
 
+// A step of one token a sequence (decode): a block owns a whole (sequence, head), P columns a group of R lanes, so that the maximum is
+// read and written in one place and one launch.  The sums are those of k_mlstm_scan.  us in a captured graph, 8 heads, against
+// k_mlstm_scan alone (k_mlstm_top adds 1.4 there and 3.8 from Python): 64 x 96 at 1 / 31 / 256 rows 4.7 / 6.4 / 30 (4.9 / 7.2 / 32),
+// 128 x 192 7.7 / 14.3 / 107 (5.4 / 18.8 / 108): one CU moves the 200 KB of a head, which takes it 2 us, and few rows wait for that.
+template <typename T, int R, int P>
+__global__ __launch_bounds__(1024) void k_mlstm_step(const T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk,
+                                                     const T* __restrict__ v, int ldv, const float* __restrict__ ipre,
+                                                     const float* __restrict__ fpre, const float* __restrict__ ib,
+                                                     const float* __restrict__ fb, float cap, float qscale,
+                                                     float* __restrict__ S, float* __restrict__ N, float* __restrict__ M,
+                                                     float* __restrict__ out, float* __restrict__ den,
+                                                     float* __restrict__ efl, int H, int dk, int dv, SeqDesc d) {
+  const int s = blockIdx.x / H, hd = blockIdx.x % H, tid = threadIdx.x;
+  if (d.live && !d.live[s]) return;
+  const int r0 = tid % R * KR, nc = blockDim.x / R, t0 = d.seq_off[s], t1 = d.seq_off[s + 1];
+  const bool old = d.pos0[s] > 0;
+  const size_t hbase = (size_t)d.slots[s] * H + hd;
+  __shared__ __attribute__((aligned(16))) float sk[KR * R];
+  __shared__ __attribute__((aligned(16))) float sq[KR * R];
+  __shared__ float sg[2];
+  float Sr[P][KR];
+  float* Sp[P];
+  int col[P];
+#pragma unroll
+  for (int c = 0; c < P; ++c) {
+    col[c] = tid / R + c * nc;
+    Sp[c] = col[c] == dv ? N + hbase * dk : S + (hbase * dv + min(col[c], dv - 1)) * dk;
+    load_rows(Sp[c], r0, dk, old && col[c] <= dv, Sr[c]);
+  }
+  float m = tid == 0 && old ? M[hbase] : 0.f;        // (thread 0 alone reads and writes it)
+  for (int t = t0; t < t1; ++t) {
+    const size_t th = (size_t)t * H + hd;
+    float x[P];
+#pragma unroll
+    for (int c = 0; c < P; ++c) x[c] = col[c] < dv ? (float)v[(size_t)t * ldv + hd * dv + col[c]] : 1.f;
+    for (int r = tid; r < KR * R; r += blockDim.x) {
+      sk[r] = r < dk ? (float)k[(size_t)t * ldk + hd * dk + r] : 0.f;
+      sq[r] = r < dk ? (float)q[(size_t)t * ldq + hd * dk + r] * qscale : 0.f;
+    }
+    if (tid == 0) {
+      float ig = cap * tanhf((ipre[th] + ib[hd]) / cap);
+      const float fg = logsigmoidf_(cap * tanhf((fpre[th] + fb[hd]) / cap));
+      asm("" : "+v"(ig));                            // (rounded here, as in k_mlstm_scan: not fused with the differences below)
+      const float mt = fg + fmaxf(m, ig - fg);
+      sg[0] = expf(fg + m - mt);
+      sg[1] = expf(ig - mt);
+      efl[th] = expf(-mt);
+      m = mt;
+    }
+    __syncthreads();
+    const float a = sg[0], b = sg[1];
+#pragma unroll
+    for (int c = 0; c < P; ++c) {
+      const float bv = b * x[c];
+      float num[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i4 = 0; i4 < KR / 4; ++i4) {
+        const f32x4 kk = *reinterpret_cast<const f32x4*>(sk + r0 + 4 * i4), qq = *reinterpret_cast<const f32x4*>(sq + r0 + 4 * i4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = 4 * i4 + j;
+          Sr[c][i] = a * Sr[c][i] + kk[j] * bv;
+          num[j] += Sr[c][i] * qq[j];
+        }
+      }
+      const float nm = group_sum<R>((num[0] + num[1]) + (num[2] + num[3]));
+      if (r0 == 0 && col[c] < dv) out[th * dv + col[c]] = nm;
+      if (r0 == 0 && col[c] == dv) den[th] = nm;
+    }
+    if (t + 1 < t1) __syncthreads();
+  }
+#pragma unroll
+  for (int c = 0; c < P; ++c)
+    if (col[c] <= dv) store_rows(Sp[c], r0, dk, Sr[c]);
+  if (tid == 0) M[hbase] = m;
+}
+
 // The running maximum that k_mlstm_scan leaves in top [B * H], into its slot.  A launch of its own: every block of columns reads the old
 // maximum, and one that starts after another has ended must still find it (in one launch the late blocks of 30 rows of 8 heads
-// decayed by the new one, and outputs were 0.08 off; 21.2 -> 23.1 us).
+// decayed by the new one, and outputs were 0.08 off).
 __global__ __launch_bounds__(256) void k_mlstm_top(const float* __restrict__ top, float* __restrict__ M, int H, SeqDesc d) {
   const int i = blockIdx.x * 256 + threadIdx.x, s = i / H;
   if (s >= d.B || (d.live && !d.live[s])) return;
@@ -689,6 +766,24 @@ void seq_short_conv(int code, int out_f32, const void* u, int ldu, const float* 
                          taps, d);
   });
   LIPA_CHECK_LAUNCH();
+}
+
+// Steps of one token a sequence; false: not one of those, or more columns than two for each group of R lanes of 1024 threads.
+bool seq_mlstm_step(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* ipre,
+                    const float* fpre, const float* ib, const float* fb, float cap, float qscale, float* S, float* N,
+                    float* M, float* out, float* den, float* efl, int H, int dk, int dv, SeqDesc d, hipStream_t st) {
+  const int Rr = rows_split(dk);
+  if (d.B == 0 || d.Ttot != d.B || (dv + 1) * Rr > 2048) return false;
+  const int P = (dv + 1) * Rr <= 1024 ? 1 : 2, threads = ((dv + P) / P * Rr + 63) / 64 * 64;
+#define MLSTM_STEP(P_)                                                                                                            \
+  hipLaunchKernelGGL((k_mlstm_step<T, R, P_>), dim3(d.B * H), dim3(threads), 0, st, (const T*)q, ldq, (const T*)k, ldk, (const T*)v, \
+                     ldv, ipre, fpre, ib, fb, cap, qscale, S, N, M, out, den, efl, H, dk, dv, d)
+  SEQ_DISPATCH_T(code, SEQ_DISPATCH_R(Rr, {
+    if (P == 1) MLSTM_STEP(1); else MLSTM_STEP(2);
+  }));
+#undef MLSTM_STEP
+  LIPA_CHECK_LAUNCH();
+  return true;
 }
 
 void seq_mlstm_scan(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* ipre,

@@ -89,6 +89,9 @@ int seq_hyper_max_streams();
 bool seq_attn_mfma_ok(int, int, int, int);
 void seq_ff_act(int, const void*, void*, int, int, int, float, const float*, hipStream_t);
 int seq_route_max_outputs();
+bool seq_mlstm_step(int, const void*, int, const void*, int, const void*, int, const float*, const float*, const float*,
+                    const float*, float, float, float*, float*, float*, float*, float*, float*, int, int, int, SeqDesc,
+                    hipStream_t);
 void seq_mlstm_scan(int, const void*, int, const void*, int, const void*, int, const float*, const float*, const float*,
                     const float*, float, float, float*, float*, float*, float*, float*, float*, float*, int, int, int, SeqDesc,
                     hipStream_t);
@@ -362,6 +365,11 @@ std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor
                     efl.data_ptr<float>(), ws.data_ptr<float>(), (size_t)most, (int)H, (int)dk, (int)dv, d, stream());
     return {out, den, efl};
   }
+  if (seq_mlstm_step(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
+                     fpre.data_ptr<float>(), ib.data_ptr<float>(), fb.data_ptr<float>(), (float)cap, (float)qscale,
+                     S.data_ptr<float>(), N.data_ptr<float>(), M.data_ptr<float>(), out.data_ptr<float>(),
+                     den.data_ptr<float>(), efl.data_ptr<float>(), (int)H, (int)dk, (int)dv, d, stream()))
+    return {out, den, efl};
   auto top = at::empty({(int64_t)d.B * H}, S.options());
   seq_mlstm_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
                  fpre.data_ptr<float>(), ib.data_ptr<float>(), fb.data_ptr<float>(), (float)cap, (float)qscale,

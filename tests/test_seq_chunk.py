@@ -112,10 +112,11 @@ def test_mlstm_chunks_keep_decays_of_a_wide_cap():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,dk,dv,L", [(1, 8, 128, 192, 1), (30, 8, 128, 192, 1), (96, 8, 64, 96, 1), (200, 4, 128, 64, 1),
-                                         (64, 8, 128, 192, 17), (3, 2, 16, 300, 1)])
+                                         (64, 8, 128, 192, 17), (3, 2, 16, 300, 1), (5, 3, 100, 40, 1), (33, 4, 256, 64, 1),
+                                         (40, 8, 128, 256, 1), (7, 1, 30, 511, 1)])
 def test_mlstm_blocks_of_columns_read_the_old_maximum(B, H, dk, dv, L):
     """More blocks of columns than run at once: those that start after others have ended decay by the maximum from before the step,
-    which every step raises here."""
+    which every step raises here (one block for all columns of a decode step where 1024 threads hold them)."""
     g = torch.Generator().manual_seed(B)
     T = B * L
     q, k, v = (torch.randn(T, H * n, generator=g).bfloat16() for n in (dk, dk, dv))
