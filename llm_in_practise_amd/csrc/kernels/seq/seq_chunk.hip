@@ -2,39 +2,44 @@
 // mLSTM - chunk by chunk instead of token by token.  With F_t the log decay summed from the chunk's first token,
 //   o_t = e^{F_t} S_prev^T q_t + sum_{j <= t} e^{F_t - F_j} c_j (q_t . k_j) v_j,
 //   S_end = e^{F_C} S_prev + sum_j e^{F_C - F_j} c_j k_j v_j^T,
-// which is matrix products over a chunk of CK tokens.  Three kernels: (1) every chunk's own contribution to the state, all
-// chunks at once; (2) the states in front of the chunks, an element-wise walk over a sequence's chunks that leaves them where
-// the contributions stood; (3) the outputs, all chunks at once.
+// which is matrix products over a chunk of CK tokens.  Three kernels: (1) every run of one, two or four chunks' own contribution to the
+// state, all runs at once, and what stands in front of the run's later chunks; (2) the states in front of the runs, an element-wise
+// walk over a sequence's runs that leaves them where the contributions stood; (3) the outputs, all chunks at once.
 //
 // What is float in the token-by-token scans stays float here.  q, k and v are bf16, so q.k runs on the bf16 matrix units
 // exactly (float sums).  A float factor of a product (decayed scores, weighted values, the state) is the sum of three bf16
 // numbers, which hold its 24 bits: three products with float sums, at five times the rate of the float matrix units.  Log
 // decays are summed in 64 bits and kept as two floats, so that the difference of two large sums is exact.
 //
-// Measured, token by token -> chunks: state space, one prompt of 4093 tokens, 64 heads of 128 x 64: 2350 -> 151 us (state 46,
-// walk 25, outputs 80); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 94 us (36, 17, 41; under the profiler 39, 18,
-// 41).  Error against 64 bits 1.6e-7 -> 0.8e-7 and 4.4e-7 -> 1.9e-7: fewer roundings stand between a token and the outputs far behind it.
-// Chunks of 128 tokens: the states of a step pass through memory once per chunk (69 MB of the first case, three times), and a
-// chunk's scores grow with its square.
+// Measured, token by token -> chunks: state space, one prompt of 4093 tokens, 64 heads of 128 x 64: 2350 -> 95 us (state 32, walk 9,
+// outputs 52); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 82 us (25, 11, 45).  Error against 64 bits
+// 1.6e-7 -> 0.9e-7 and 4.4e-7 -> 1.9e-7: fewer roundings stand between a token and the outputs far behind it.
+// The first case reads and writes 335 MB, 235 of them states and outputs, of which a copy moves 5 TB/s.  With every chunk's contribution
+// walked by itself (69 MB of states out, in, out and in), operands of the outputs loaded from memory rows as they are needed, an
+// exponential for each score and splits by rounding it took 150 us (46, 25, 80).
 #include "seq_common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 using namespace lipa;
 
 namespace {
 
 constexpr int CK = 128;                 // tokens of a chunk (4 waves x 32 queries)
-constexpr int KP = 64 + 8;              // row of 64 staged tokens, padded: 16-byte reads of 16 rows hit all banks
-constexpr int VP = CK + 4;              // row of a chunk's tokens, padded: 8-byte reads of 32 rows hit all banks
 constexpr double LOG2E = 1.4426950408889634074;
 
-// x = hi + mid + lo in bf16 to float accuracy (an infinity stays one)
-__device__ __forceinline__ void split3(float x, bf16& h, bf16& m, bf16& l) {
-  h = (bf16)x;
-  const float r = fabsf(x) < 3.38e38f ? x - (float)h : 0.f;
-  m = (bf16)r;
-  l = (bf16)(r - (float)m);
+// Two floats as sums of three bf16 numbers each, h + m + l, which hold their 24 bits exactly (an infinity stays one: what it leaves is
+// no number, and is bounded).  By cutting, since packing the upper halves of two words is one instruction.
+struct Split {
+  unsigned h, m, l;
+};
+__device__ __forceinline__ Split split3(float x0, float x1) {
+  const auto upper = [](float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); };
+  const auto pack = [](float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u); };
+  const float r0 = __builtin_amdgcn_fmed3f(x0 - upper(x0), -0x1p120f, 0x1p120f),
+              r1 = __builtin_amdgcn_fmed3f(x1 - upper(x1), -0x1p120f, 0x1p120f);
+  return {pack(x0, x1), pack(r0, r1), pack(r0 - upper(r0), r1 - upper(r1))};
 }
 
 __device__ __forceinline__ double shfl_up_d(double v, int o) {
@@ -44,8 +49,27 @@ __device__ __forceinline__ double shfl_up_d(double v, int o) {
 }
 __device__ __forceinline__ double last_lane_d(double v) {
   const long long b = __double_as_longlong(v);
-  const int lo = __shfl((int)b, 63, 64), hi = __shfl((int)(b >> 32), 63, 64);
+  const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// v of a lane further down (CTRL: by 1, 2, 4, 8 within a row of 16, or a row's last lane to the rows behind it), `none` where there is none
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double from_below(double v, double none) {
+  const long long b = __double_as_longlong(v), z = __double_as_longlong(none);
+  const int lo = __builtin_amdgcn_update_dpp((int)z, (int)b, CTRL, ROWS, 0xF, false),
+            hi = __builtin_amdgcn_update_dpp((int)(z >> 32), (int)(b >> 32), CTRL, ROWS, 0xF, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// op over a lane and those in front of it: a scan without a trip through LDS per step (6.5 -> 3.5 thousand cycles for a chunk's gates)
+template <typename Op>
+__device__ __forceinline__ double scan_lanes(double v, double none, Op op) {
+  v = op(v, from_below<0x111, 0xF>(v, none));      // row_shr 1, 2, 4, 8
+  v = op(v, from_below<0x112, 0xF>(v, none));
+  v = op(v, from_below<0x114, 0xF>(v, none));
+  v = op(v, from_below<0x118, 0xF>(v, none));
+  v = op(v, from_below<0x142, 0xA>(v, none));      // row_bcast 15 into rows 1 and 3, row_bcast 31 into rows 2 and 3
+  v = op(v, from_below<0x143, 0xC>(v, none));
+  return v;
 }
 
 struct GateArgs {
@@ -65,8 +89,23 @@ struct Gate {                           // of a wave's lane: tokens 2 * lane and
   float c0, c1;                         // factor of the input that is not in the logarithm (state space: dt)
 };
 
+struct GateIn {                         // a lane's two tokens as they stand in memory
+  float i[2], f[2];
+};
 template <bool MLSTM>
-__device__ __forceinline__ Gate gates(const GateArgs& g, const Piece& c, int hd, int lane) {
+__device__ __forceinline__ GateIn gate_in(const GateArgs& g, const Piece& c, int hd, int lane) {
+  GateIn r;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const size_t t = c.t0 + min(2 * lane + e, c.n - 1);
+    r.i[e] = MLSTM ? g.ipre[t * g.H + hd] : (float)g.dt[t * g.lddt + hd];
+    r.f[e] = MLSTM ? g.fpre[t * g.H + hd] : 0.f;
+  }
+  return r;
+}
+
+template <bool MLSTM>
+__device__ __forceinline__ Gate gates(const GateArgs& g, const GateIn& in, const Piece& c, int hd, int lane) {
   Gate r;
   double l[2], ig[2] = {0.0, 0.0};
   float w[2] = {0.f, 0.f};
@@ -74,15 +113,14 @@ __device__ __forceinline__ Gate gates(const GateArgs& g, const Piece& c, int hd,
   for (int e = 0; e < 2; ++e) {
     const int j = 2 * lane + e;
     const bool on = j < c.n;
-    const size_t t = c.t0 + (on ? j : 0);
     if (MLSTM) {
-      const float i = g.cap * tanhf((g.ipre[t * g.H + hd] + g.ib[hd]) / g.cap);
-      const float f = logsigmoidf_(g.cap * tanhf((g.fpre[t * g.H + hd] + g.fb[hd]) / g.cap));
+      const float i = g.cap * tanhf((in.i[e] + g.ib[hd]) / g.cap);
+      const float f = logsigmoidf_(g.cap * tanhf((in.f[e] + g.fb[hd]) / g.cap));
       ig[e] = on ? (double)i * LOG2E : -(double)INFINITY;
       l[e] = on ? (double)f * LOG2E : 0.0;
       w[e] = on ? 1.f : 0.f;
     } else {
-      const float dt = softplusf_((float)g.dt[t * g.lddt + hd] + g.dt_bias[hd]);
+      const float dt = softplusf_(in.i[e] + g.dt_bias[hd]);
       l[e] = on ? (double)(-expf(g.a_log[hd]) * dt) * LOG2E : 0.0;
       w[e] = on ? dt : 0.f;
     }
@@ -92,12 +130,7 @@ __device__ __forceinline__ Gate gates(const GateArgs& g, const Piece& c, int hd,
   if (!MLSTM)
 #pragma unroll
     for (int e = 0; e < 2; ++e) l[e] = l[e] < -512.0 ? -512.0 : l[e];
-  double sum = l[0] + l[1];
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const double t = shfl_up_d(sum, o);
-    if (lane >= o) sum += t;
-  }
+  const double sum = scan_lanes(l[0] + l[1], 0.0, [](double a, double b) { return a + b; });
   r.F1 = sum;
   const double before = shfl_up_d(sum, 1);
   r.F0 = l[1] == l[1] ? sum - l[1] : lane ? before + l[0] : l[0];      // (a NaN decay starts at its own token)
@@ -111,185 +144,263 @@ __device__ __forceinline__ Gate gates(const GateArgs& g, const Piece& c, int hd,
 
 // the running maximum of a over a chunk's tokens, up to and including this lane's two
 __device__ __forceinline__ void running_max(const Gate& g, int lane, double& m0, double& m1) {
-  double top = fmax(g.a0, g.a1);
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const double t = shfl_up_d(top, o);
-    if (lane >= o) top = fmax(top, t);
-  }
+  const double top = scan_lanes(fmax(g.a0, g.a1), -(double)INFINITY, [](double a, double b) { return fmax(a, b); });
   m1 = top;
   const double before = shfl_up_d(top, 1);
   m0 = lane ? fmax(before, g.a0) : g.a0;
 }
 
-// Four tokens x four columns of a row-major bf16 matrix, transposed: out[e] holds column e's four tokens (0 past the end).
-__device__ __forceinline__ void load_4x4(const bf16* __restrict__ p, size_t ld, int tokens, bool on, bf16x4 (&out)[4]) {
-  bf16x4 r[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    r[t] = bf16x4{(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
-    if (on && t < tokens) r[t] = *reinterpret_cast<const bf16x4*>(p + t * ld);
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) out[e] = bf16x4{r[0][e], r[1][e], r[2][e], r[3][e]};
-}
-
 __device__ __forceinline__ int c_row(int i, int half) { return (i & 3) + 8 * (i >> 2) + 4 * half; }   // 32x32 tile: row of register i
 
-// (1) U[slot, head, dv, dk] = sum_j w_j v_j k_j^T over a chunk, w_j = e^{F_C - F_j} c_j (mLSTM: against the chunk's largest),
-// for 64 value columns.  Bound by latency: a wave of a SIMD's three waits in turn for the gates, k and v, and the LDS, so the loads
-// stand before the gates and the second half's before the first half's products (56 -> 45 us for 4093 tokens of 64 heads, with
-// the registers held to three workgroups a CU; 40 -> 38 for the mLSTM's).
+// What the kernels leave for each other, per run of `sc` chunks of a sequence (a piece) and head, and per chunk of it.
+struct Ws {
+  double* sup;       // [slot, H, 3]: log decay of the run, log of the unit that E is counted in, log of the unit in front of the run
+  double* loc;       // [chunk, H, 2]: log decay from the run's start to the chunk, log of the unit that U is counted in
+  float* tab;        // [chunk, H, 3 or 6, CK]: the tokens' gates, a float and what it leaves: a; (input factor | F, running maximum of a)
+  float *E, *NE;     // [slot, H, dv, dk], [slot, H, dk]: the run's contribution to the state, later the state in front of the run
+  float *U, *NU;     // [slot, sc - 1, H, ..]: what the run's chunks in front of the second, third .. contribute
+  int sc;
+};
+
+// The 8-byte transposed read: of 16 lanes, lane l gets column l of the four rows that lanes 0, 4, 8, 12 point into.
+__device__ __forceinline__ bf16x4 read_tr(const bf16* p) {
+  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
+}
+// Where the 16-byte piece x8 of row r stands in an unpadded row of COLS bf16.  Transposed reads take four rows by two blocks of 16
+// columns at a time, operand reads 16 rows of one piece: both then meet every bank once.
+template <int COLS>
+__device__ __forceinline__ int tr_piece(int r, int x8) {
+  return COLS % 128 == 0 ? x8 ^ ((r & 3) << 2) : COLS % 128 == 64 ? x8 ^ ((r & 2) << 1) : x8;
+}
+template <int COLS>
+__device__ __forceinline__ int op_piece(int r, int x8) {
+  return x8 ^ (COLS % 128 == 0 ? r & 15 : COLS % 128 == 64 ? (r >> 1) & 7 : (r >> 2) & 3);
+}
+
+// (1) A run's contribution to the state, E[slot, head, dv, dk] = sum_j w_j v_j k_j^T with w_j = e^{F_end - F_j} c_j (mLSTM: against the
+// largest), for 64 value columns, and on the way what stands in front of its second, third .. chunk.  A wave works out the gates of
+// one chunk, all at once; then 64 tokens at a time go through LDS as they stand in memory, and the products, which sum over tokens,
+// read them transposed.  The next 64 tokens' loads are on their way under the products.
 template <int NK, bool MLSTM>
 __global__ __launch_bounds__(256, 3) void k_chunk_state(const bf16* __restrict__ k, int ldk, const bf16* __restrict__ v,
-                                                     int ldv, GateArgs ga, float* __restrict__ U, float* __restrict__ NU,
-                                                     double* __restrict__ meta, int H, int G, int dv, Pieces pc, SeqDesc d) {
-  constexpr int DK = 32 * NK;
-  __shared__ __attribute__((aligned(16))) bf16 sk[DK * KP];              // [dk][token]
-  __shared__ __attribute__((aligned(16))) bf16 sv[3 * 64 * KP];          // [part][dv][token]
-  __shared__ float sw[CK];
-  __shared__ float sn[256];
+                                                        int ldv, GateArgs ga, Ws ws, int H, int G, int dv, Pieces pc, SeqDesc d) {
+  constexpr int DK = 32 * NK, TILES = (NK + 1) / 2, TAB = MLSTM ? 6 : 3;
+  __shared__ __attribute__((aligned(16))) bf16 sk[64 * DK];              // [token][dk]
+  __shared__ __attribute__((aligned(16))) bf16 sv[3 * 64 * 64];          // [part][token][dv]
+  __shared__ float sw[4 * CK], sscale[4];
+  __shared__ double sF[4], sTop[4];
   Piece c;
   const int slot = blockIdx.x, hd = blockIdx.y, cb = blockIdx.z * 64, tid = threadIdx.x;
-  if (!find_piece<CK>(d, pc, slot, c)) return;
-  const int w = tid >> 6, lane = tid & 63, l32 = lane & 31, half = lane >> 5, kh = hd / (H / G);
+  if (!find_piece<0>(d, pc, slot, c)) return;
+  c.t0 = __builtin_amdgcn_readfirstlane(c.t0);
+  c.n = __builtin_amdgcn_readfirstlane(c.n);
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, g = lane >> 4, kh = hd / (H / G);
+  const int l32 = lane & 31, half = lane >> 5, chunks = (c.n + CK - 1) / CK;
   const size_t cell = (size_t)slot * H + hd;
   const bf16* kp = k + (size_t)c.t0 * ldk + kh * DK;
   const bf16* vp = v + (size_t)c.t0 * ldv + (size_t)hd * dv + cb;
-  constexpr int KL = (DK / 4 * 16 + 255) / 256;
-  bf16x4 rk[KL][4], rv[4];
-  const int c4 = tid & 15, vt = tid >> 4;
-  auto load = [&](int j0) {                    // (the second half over the products of the first)
+  Piece own = {c.s, 0, c.t0 + min(w, chunks - 1) * CK, 0, 0};
+  own.n = min(CK, c.t0 + c.n - own.t0);
+  const GateIn gi = gate_in<MLSTM>(ga, own, hd, lane);
+  bf16x8 rk[NK];
+  bf16x4 rv[2][2];
+  auto load = [&](int j0) {
 #pragma unroll
-    for (int i = 0; i < KL; ++i) {
-      const int e = tid + 256 * i, d4 = e % (DK / 4), t4 = j0 + 4 * (e / (DK / 4));
-      load_4x4(kp + (size_t)t4 * ldk + 4 * d4, ldk, c.n - t4, e < DK / 4 * 16, rk[i]);
+    for (int i = 0; i < NK; ++i) {
+      const int e = tid + 256 * i, r = min(j0 + e / (DK / 8), c.n - 1), x8 = e % (DK / 8);
+      rk[i] = *reinterpret_cast<const bf16x8*>(kp + (unsigned)(r * ldk + 8 * x8));
     }
-    load_4x4(vp + (size_t)(j0 + 4 * vt) * ldv + 4 * c4, ldv, c.n - j0 - 4 * vt, cb + 4 * c4 < dv, rv);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {             // (columns past the last give columns past the last)
+        const int e = tid + 256 * i, r = min(j0 + (e >> 3), c.n - 1), col = min(8 * (e & 7) + 4 * h, dv - cb - 4);
+        rv[i][h] = *reinterpret_cast<const bf16x4*>(vp + (unsigned)(r * ldv + col));
+      }
   };
   load(0);
-  if (w == 0) {
-    const Gate g = gates<MLSTM>(ga, c, hd, lane);
-    double top = 0.0, add = g.Fc;
-    if (MLSTM) {
-      double m0, m1;
-      running_max(g, lane, m0, m1);
-      top = last_lane_d(m1);
-      add = -top;
+  if (w < chunks) {
+    const Gate gt = gates<MLSTM>(ga, gi, own, hd, lane);
+    double m0 = 0.0, m1 = 0.0;
+    if (MLSTM) running_max(gt, lane, m0, m1);
+    if (lane == 0) sF[w] = gt.Fc;
+    if (lane == 63) sTop[w] = m1;
+    __syncthreads();
+    double F = 0.0, m = -(double)INFINITY;           // log decay and unit in front of the wave's chunk
+    for (int i = 0; i < w; ++i) {
+      F += sF[i];
+      m = fmax(m + sF[i], sF[i] + sTop[i]);
     }
-    sw[2 * lane] = 2 * lane < c.n ? exp2f((float)(g.a0 + add)) * g.c0 : 0.f;
-    sw[2 * lane + 1] = 2 * lane + 1 < c.n ? exp2f((float)(g.a1 + add)) * g.c1 : 0.f;
-    if (lane == 0 && cb == 0) {
-      meta[3 * cell] = g.Fc;
-      meta[3 * cell + 1] = g.Fc + top;         // log of the unit that U is counted in
+    const double mn = fmax(m + gt.Fc, gt.Fc + m1);   // (of lane 63)
+    const double unit = MLSTM ? last_lane_d(mn) : 0.0;
+    const int j = 2 * lane;
+    sw[CK * w + j] = j < own.n ? exp2f((float)(gt.a0 + (gt.Fc - unit))) * gt.c0 : 0.f;
+    sw[CK * w + j + 1] = j + 1 < own.n ? exp2f((float)(gt.a1 + (gt.Fc - unit))) * gt.c1 : 0.f;
+    if (lane == 0) sscale[w] = MLSTM ? exp2f((float)(m + gt.Fc - unit)) : exp2f((float)gt.Fc);
+    if (cb == 0) {
+      const size_t cc = ((size_t)slot * ws.sc + w) * H + hd;
+      if (lane == 0) {
+        ws.loc[2 * cc] = F;
+        ws.loc[2 * cc + 1] = m;
+        if (w == chunks - 1) {
+          ws.sup[3 * cell] = F + gt.Fc;
+          ws.sup[3 * cell + 1] = unit;
+        }
+      }
+      float* tab = ws.tab + cc * TAB * CK + j;
+      const auto two = [&](int i, double x0, double x1) {       // a double as a float and what that leaves
+        const float h0 = (float)x0, h1 = (float)x1;
+        *reinterpret_cast<float2*>(tab + i * CK) = float2{h0, h1};
+        *reinterpret_cast<float2*>(tab + (i + 1) * CK) =
+            float2{j < own.n ? (float)(x0 - (double)h0) : 0.f, j + 1 < own.n ? (float)(x1 - (double)h1) : 0.f};
+      };
+      two(0, gt.a0, gt.a1);
+      if (MLSTM) {
+        two(2, gt.F0, gt.F1);
+        two(4, m0, m1);
+      } else {
+        *reinterpret_cast<float2*>(tab + 2 * CK) = float2{gt.c0, gt.c1};
+      }
     }
+  } else {
+    __syncthreads();
   }
-  f32x16 acc[(NK + 1) / 2];
+  f32x16 acc[TILES];
 #pragma unroll
-  for (int t = 0; t < (NK + 1) / 2; ++t)
+  for (int t = 0; t < TILES; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
-  float nsum = 0.f;
-  for (int j0 = 0; j0 < c.n; j0 += 64) {
-    __syncthreads();                           // the last turn's reads are done; the weights stand
+  // the normaliser (the column whose value is always 1): two key channels per thread, a part of the tokens
+  constexpr int PARTS = NK == 3 ? 4 : 16 / NK, TOK = 64 / PARTS;
+  const int nc = tid % (DK / 2), part = tid / (DK / 2);
+  const bool norm = MLSTM && cb == 0;
+  float n0 = 0.f, n1 = 0.f;
+  // (what has no place goes past the end of its window and is dropped)
+  const int left = max(min(dv - cb - (w & 1) * 32, 32), 0);
+  auto store = [&](float* to) {
+    const auto win = __builtin_amdgcn_make_buffer_rsrc(to + (size_t)(cb + (w & 1) * 32) * DK, 0, left * DK * 4, 0x00020000);
 #pragma unroll
-    for (int i = 0; i < KL; ++i) {
-      const int e = tid + 256 * i, d4 = e % (DK / 4), t4 = e / (DK / 4);
-      if (e < DK / 4 * 16)
-#pragma unroll
-        for (int x = 0; x < 4; ++x) *reinterpret_cast<bf16x4*>(sk + (4 * d4 + x) * KP + 4 * t4) = rk[i][x];
-    }
-    const f32x4 wt = *reinterpret_cast<const f32x4*>(sw + j0 + 4 * vt);
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      bf16x4 h, m, l;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        bf16 a, b, e;
-        split3(wt[t] * (float)rv[x][t], a, b, e);
-        h[t] = a;
-        m[t] = b;
-        l[t] = e;
-      }
-      bf16* row = sv + (4 * c4 + x) * KP + 4 * vt;
-      *reinterpret_cast<bf16x4*>(row) = h;
-      *reinterpret_cast<bf16x4*>(row + 64 * KP) = m;
-      *reinterpret_cast<bf16x4*>(row + 2 * 64 * KP) = l;
-    }
-    if (j0 + 64 < c.n) load(j0 + 64);
-    __syncthreads();
-    const int vrow = (w & 1) * 32 + l32;
-    if (cb + (w & 1) * 32 < dv) {
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const bf16* ap = sv + vrow * KP + 16 * ks + 8 * half;
-        const bf16x8 ah = *reinterpret_cast<const bf16x8*>(ap), am = *reinterpret_cast<const bf16x8*>(ap + 64 * KP),
-                     al = *reinterpret_cast<const bf16x8*>(ap + 2 * 64 * KP);
-#pragma unroll
-        for (int t = 0; t < (NK + 1) / 2; ++t) {
-          const int kt = (w >> 1) + 2 * t;
-          if (kt < NK) {
-            const bf16x8 b = *reinterpret_cast<const bf16x8*>(sk + (kt * 32 + l32) * KP + 16 * ks + 8 * half);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, b, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, b, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, b, acc[t], 0, 0, 0);
-          }
-        }
-      }
-    }
-    if (MLSTM && cb == 0) {                    // the normaliser: the column whose value is always 1
-      constexpr int PARTS = 256 / DK;
-      const int r = tid % DK, part = tid / DK;
-      if (part < PARTS)
-        for (int j = part * 8; j < 64; j += 8 * PARTS) {
-          const bf16x8 kk = *reinterpret_cast<const bf16x8*>(sk + r * KP + j);
-#pragma unroll
-          for (int x = 0; x < 8; ++x) nsum += sw[j0 + j + x] * (float)kk[x];
-        }
-    }
-  }
-  if (cb + (w & 1) * 32 < dv) {
-#pragma unroll
-    for (int t = 0; t < (NK + 1) / 2; ++t) {
+    for (int t = 0; t < TILES; ++t) {
       const int kt = (w >> 1) + 2 * t;
-      if (kt < NK)
+      const unsigned at = kt < NK ? (4 * half * DK + kt * 32 + l32) * 4 : 0x80000000u;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int col = cb + (w & 1) * 32 + c_row(i, half);
-          if (col < dv) U[(cell * dv + col) * DK + kt * 32 + l32] = acc[t][i];
-        }
+      for (int i = 0; i < 16; ++i)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[t][i]), win, at + c_row(i, 0) * DK * 4, 0, 0);
     }
-  }
-  if (MLSTM && cb == 0) {
-    constexpr int PARTS = 256 / DK;
-    sn[tid] = nsum;
+  };
+  auto store_norm = [&](float* to) {
+    float* sn = reinterpret_cast<float*>(sv);         // (the last products' reads are past a barrier)
+    if (part < PARTS) *reinterpret_cast<float2*>(sn + part * DK + 2 * nc) = float2{n0, n1};
     __syncthreads();
     if (tid < DK) {
       float t = sn[tid];
 #pragma unroll
-      for (int p = 1; p < PARTS; ++p) t += sn[tid + p * DK];
-      NU[cell * DK + tid] = t;
+      for (int q = 1; q < PARTS; ++q) t += sn[tid + q * DK];
+      to[tid] = t;
     }
+  };
+  for (int j0 = 0; j0 < c.n; j0 += 64) {
+    __syncthreads();                           // the last turn's reads are done; the weights stand
+    const int ci = j0 / CK;
+    if (norm && j0 % CK == 0 && ci > 0) {
+      store_norm(ws.NU + (((size_t)slot * (ws.sc - 1) + ci - 1) * H + hd) * DK);
+      __syncthreads();
+      n0 *= sscale[ci];
+      n1 *= sscale[ci];
+    }
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const int e = tid + 256 * i, r = e / (DK / 8), x8 = e % (DK / 8);
+      *reinterpret_cast<bf16x8*>(sk + r * DK + 8 * tr_piece<DK>(r, x8)) = j0 + r < c.n ? rk[i] : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int e = tid + 256 * i, r = e >> 3, x8 = e & 7;
+      const float wt = sw[j0 + r];
+      const bool on = j0 + r < c.n;            // (tokens past the end repeat the last: an infinite one times 0 would be no number)
+      u32x4 o[3];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const bf16x4 y = rv[i][x >> 1];
+        const float y0 = wt * (float)y[2 * (x & 1)], y1 = wt * (float)y[2 * (x & 1) + 1];
+        const Split z = split3(on ? y0 : 0.f, on ? y1 : 0.f);
+        o[0][x] = z.h;
+        o[1][x] = z.m;
+        o[2][x] = z.l;
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(sv + (q * 64 + r) * 64 + 8 * tr_piece<64>(r, x8)) = o[q];
+    }
+    if (j0 % CK == 0 && ci > 0) {              // (in front of the loads: a wait for those then waits for nothing younger)
+      store(ws.U + (((size_t)slot * (ws.sc - 1) + ci - 1) * H + hd) * dv * DK);
+      const float f = sscale[ci];
+#pragma unroll
+      for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[t][i] *= f;
+    }
+    load(j0 + 64);                             // (past the end: its last token again)
+    __syncthreads();
+    // operand rows are columns here: lanes 16 g .. read the tokens of half g / 2 in columns 16 (g % 2) .., four tokens a read
+    const int row = 8 * (g >> 1) + (li >> 2);
+    const auto operand = [&](const bf16* base, auto cols, int r, int tile) {
+      constexpr int COLS = decltype(cols)::value;
+      const int x8 = 4 * tile + 2 * (g & 1) + ((li >> 1) & 1);
+      const bf16x4 lo = read_tr(base + r * COLS + 8 * tr_piece<COLS>(r, x8) + 4 * (li & 1)),
+                   hi = read_tr(base + (r + 4) * COLS + 8 * tr_piece<COLS>(r + 4, x8) + 4 * (li & 1));
+      return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    if (cb + (w & 1) * 32 < dv) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        bf16x8 a[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) a[q] = operand(sv + q * 64 * 64, std::integral_constant<int, 64>{}, 16 * ks + row, w & 1);
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+          const int kt = (w >> 1) + 2 * t;
+          if (kt < NK) {
+            const bf16x8 b = operand(sk, std::integral_constant<int, DK>{}, 16 * ks + row, kt);
+#pragma unroll
+            for (int q = 2; q >= 0; --q) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[q], b, acc[t], 0, 0, 0);
+          }
+        }
+      }
+    }
+    if (norm && part < PARTS) {
+#pragma unroll
+      for (int i = 0; i < TOK; ++i) {
+        const int r = part * TOK + i;
+        const bf16x2 kk = *reinterpret_cast<const bf16x2*>(sk + r * DK + 8 * tr_piece<DK>(r, nc >> 2) + 2 * (nc & 3));
+        n0 += sw[j0 + r] * (float)kk[0];
+        n1 += sw[j0 + r] * (float)kk[1];
+      }
+    }
+  }
+  store(ws.E + cell * dv * DK);
+  if (norm) {
+    __syncthreads();
+    store_norm(ws.NE + cell * DK);
   }
 }
 
-// (2) A sequence's chunks in order, four state elements per thread: the state in front of a chunk replaces the chunk's
+// (2) A sequence's runs in order, four state elements per thread: the state in front of a run replaces the run's
 // contribution, the state behind the last one goes to its slot.  Bound by memory: every contribution is read and written once.
 template <bool MLSTM>
-__global__ __launch_bounds__(256) void k_chunk_walk(float* __restrict__ U, float* __restrict__ NU, double* __restrict__ meta,
-                                                    float* __restrict__ S, float* __restrict__ N,
+__global__ __launch_bounds__(256) void k_chunk_walk(Ws ws, float* __restrict__ S, float* __restrict__ N,
                                                     const float* __restrict__ M, int H, int dk, int dv, int nb, Pieces pc,
                                                     SeqDesc d) {
   const int s = blockIdx.x / H, hd = blockIdx.x % H, tid = threadIdx.x;
   if (d.live && !d.live[s]) return;
   const bool norm = MLSTM && (int)blockIdx.y == nb;        // the last block walks the normaliser
   int first;
-  const int n = own_pieces<CK>(d, pc, s, first);
+  const int n = own_pieces<0>(d, pc, s, first);
   const int size = norm ? dk : dv * dk, e = (norm ? 0 : (int)blockIdx.y * 1024) + 4 * tid;
   const size_t hbase = (size_t)d.slots[s] * H + hd, step = (size_t)H * size;
   float* st = (norm ? N : S) + hbase * size + e;
-  float* u = (norm ? NU : U) + ((size_t)first * H + hd) * size + e;
-  double* mt = meta + 3 * ((size_t)first * H + hd);
+  float* u = (norm ? ws.NE : ws.E) + ((size_t)first * H + hd) * size + e;
+  double* mt = ws.sup + 3 * ((size_t)first * H + hd);
   const bool on = e < size, old = pc.first > 0 || d.pos0[s] > 0;
   f32x4 x = {0.f, 0.f, 0.f, 0.f};
   if (on && old) x = *reinterpret_cast<const f32x4*>(st);
@@ -335,245 +446,352 @@ __global__ __launch_bounds__(256) void k_chunk_walk(float* __restrict__ U, float
   if (on && n > 0) *reinterpret_cast<f32x4*>(st) = x;
 }
 
-// (3) Outputs of a chunk and head: a wave owns 32 queries, keeps their decayed scores against the chunk's keys as three bf16
-// parts in registers, and walks the value columns 32 at a time: scores . values, and queries . state with the state split into
-// LDS once for the block.  Scores are computed transposed (a lane owns one query), which is the operand layout of the second
-// product; its keys then come in the order of the score registers.
+// (3) Outputs of a chunk and head in 64 value columns: a wave owns 32 queries.  First queries . state, the state in front of the chunk
+// put together from the run's and the chunk's part and split into LDS once for the block; then its scores against the chunk's keys, 32
+// keys at a time, as three bf16 parts . values.  Scores are computed transposed (a lane owns one query), which is the operand layout
+// of the second product; its keys then come in the order of the score registers.
+// With R the decay at the wave's first query, e^{F_i - F_j} = e^{F_i - R} e^{R - F_j} for a key in front of that query: neither factor
+// is above 1, the second is one number per key, and the first scales sums (of the state's part too).  Only the 32 x 32 scores on the
+// diagonal take an exponential each.
 template <int NK, bool MLSTM>
-__global__ __launch_bounds__(256, 2) void k_chunk_out(const bf16* __restrict__ q, int ldq, const bf16* __restrict__ k, int ldk,
-                                                      const bf16* __restrict__ v, int ldv, GateArgs ga,
-                                                      const float* __restrict__ U, const float* __restrict__ NU,
-                                                      const double* __restrict__ meta, float* __restrict__ M,
-                                                      float* __restrict__ out, float* __restrict__ den,
+__global__ __launch_bounds__(256, 3) void k_chunk_out(const bf16* __restrict__ q, int ldq, const bf16* __restrict__ k, int ldk,
+                                                      const bf16* __restrict__ v, int ldv, GateArgs ga, Ws ws,
+                                                      float* __restrict__ M, float* __restrict__ out, float* __restrict__ den,
                                                       float* __restrict__ efl, int H, int G, int dv, Pieces pc, SeqDesc d) {
-  constexpr int DK = 32 * NK, SP = DK + 8;
-  __shared__ __attribute__((aligned(16))) bf16 ss[3 * 32 * SP];          // state: [part][dv][dk]
-  __shared__ __attribute__((aligned(16))) bf16 sv[32 * VP];              // values: [dv][token]
-  __shared__ __attribute__((aligned(16))) float sah[CK], sal[CK], sc[CK], sbh[CK], sbl[CK], sx[CK];
-  __shared__ float sN[DK];
-  __shared__ int sbad[2][32];                              // per column the first token whose value is no number
+  constexpr int DK = 32 * NK, TAB = MLSTM ? 6 : 3;
+  constexpr int HW = NK % 2 ? 32 : 64, NL = HW / 16;                     // key channels of a piece of the state, its loads a thread
+  constexpr int KV = CK * DK + CK * 64, ST = 3 * 64 * HW;
+  __shared__ __attribute__((aligned(16))) bf16 buf[KV > ST ? KV : ST];   // queries [token][dk]; state [part][dv][HW]; keys [token][dk], values
+  bf16* const sv = buf + CK * DK;                                        // [token][dv]
+  __shared__ __attribute__((aligned(16))) float sah[CK], sal[CK], sbh[CK], sbl[CK], sx[CK], swk[192];
+  __shared__ int sbad[64];                                 // per column the first token whose value is no number
+  static_assert(DK <= CK, "sx holds a normaliser");
   Piece c;
-  const int slot = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x;
-  if (!find_piece<CK>(d, pc, slot, c)) return;
-  const int w = tid >> 6, lane = tid & 63, l32 = lane & 31, half = lane >> 5, kh = hd / (H / G);
-  const size_t cell = (size_t)slot * H + hd;
-  const bool old = c.idx > 0 || d.pos0[c.s] > 0;           // is there a state in front of the chunk
-  if (w == 0) {
-    const Gate g = gates<MLSTM>(ga, c, hd, lane);
-    double b0 = g.F0, b1 = g.F1, x0 = g.F0, x1 = g.F1;
-    if (MLSTM) {
-      const double mp = meta[3 * cell + 2];
-      double m0, m1;
-      running_max(g, lane, m0, m1);
-      m0 = fmax(m0, mp);
-      m1 = fmax(m1, mp);
-      b0 = -m0;
-      b1 = -m1;
-      x0 = mp - m0;
-      x1 = mp - m1;
-      if (2 * lane < c.n) efl[(size_t)(c.t0 + 2 * lane) * H + hd] = exp2f((float)(-(g.F0 + m0)));
-      if (2 * lane + 1 < c.n) efl[(size_t)(c.t0 + 2 * lane + 1) * H + hd] = exp2f((float)(-(g.F1 + m1)));
-      // behind the last chunk, here or at all (tokens past its end change nothing)
-      if (lane == 63 && (c.t0 + c.n == d.seq_off[c.s + 1] || (pc.count > 0 && c.idx == pc.first + pc.count - 1)))
-        M[(size_t)d.slots[c.s] * H + hd] = (float)((g.F1 + m1) * 0.69314718055994530942);
-    }
-    const float ah0 = (float)g.a0, ah1 = (float)g.a1, bh0 = (float)b0, bh1 = (float)b1;
-    const int j = 2 * lane;
-    sah[j] = ah0;
-    sah[j + 1] = ah1;
-    sal[j] = j < c.n ? (float)(g.a0 - (double)ah0) : 0.f;
-    sal[j + 1] = j + 1 < c.n ? (float)(g.a1 - (double)ah1) : 0.f;
-    sc[j] = g.c0;
-    sc[j + 1] = g.c1;
-    sbh[j] = bh0;
-    sbh[j + 1] = bh1;
-    sbl[j] = (float)(b0 - (double)bh0);
-    sbl[j + 1] = (float)(b1 - (double)bh1);
-    sx[j] = exp2f((float)x0);
-    sx[j + 1] = exp2f((float)x1);
-  }
-  if (tid < 64) sbad[tid >> 5][tid & 31] = CK;
-  if (MLSTM && tid >= 256 - DK) sN[tid - (256 - DK)] = old ? NU[cell * DK + tid - (256 - DK)] : 0.f;
-  const bool work = 32 * w < c.n;
-  const int qi = 32 * w + l32;                              // this lane's query
-  bf16x8 qf[2 * NK], pf[4][2][3];
-  if (work) {
-    const bf16* qp = q + (size_t)(c.t0 + min(qi, c.n - 1)) * ldq + kh * DK + 8 * half;
+  const int slot = blockIdx.x / ws.sc, ci = blockIdx.x % ws.sc, hd = blockIdx.y, cb = blockIdx.z * 64, tid = threadIdx.x;
+  if (!find_piece<0>(d, pc, slot, c)) return;
+  const int t0 = __builtin_amdgcn_readfirstlane(c.t0 + ci * CK), n = __builtin_amdgcn_readfirstlane(min(CK, c.n - ci * CK));
+  if (n <= 0) return;
+  // Wave 3 has four times the scores of wave 0, and a block's waves go to the SIMDs in order: neighbours on a CU take turns.
+  const unsigned id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  const int w = __builtin_amdgcn_readfirstlane(((tid >> 6) + (id >> 8)) & 3), lane = tid & 63, l32 = lane & 31, half = lane >> 5, kh = hd / (H / G);
+  const size_t cell = (size_t)slot * H + hd, cc = (size_t)blockIdx.x * H + hd, cu = ((size_t)slot * (ws.sc - 1) + ci - 1) * H + hd;
+  const bool run = c.idx > 0 || c.pos0 > 0, old = run || ci > 0;    // is there a state in front of the run; of the chunk
+  float tv[TAB];
+  const float* tab = ws.tab + cc * TAB * CK + (tid & (CK - 1));
 #pragma unroll
-    for (int s = 0; s < 2 * NK; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + 16 * s);
+  for (int i = 0; i < TAB; ++i) tv[i] = tab[i * CK];
+  const double floc = ws.loc[2 * cc], mloc = ws.loc[2 * cc + 1], msup = MLSTM ? ws.sup[3 * cell + 2] + floc : floc;
+  // Rows of 16-byte pieces side by side: an operand's own load would touch 32 rows of memory.  All loads first.
+  constexpr int PER = 2 * NK;
+  const bf16 *qp = q + (size_t)t0 * ldq + kh * DK, *kp = k + (size_t)t0 * ldk + kh * DK, *vp = v + (size_t)t0 * ldv + (size_t)hd * dv + cb;
+  bf16x8 rq[PER], rk[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = lane + 64 * i, r = min(32 * w + e / (DK / 8), n - 1), x8 = e % (DK / 8);
+    rq[i] = *reinterpret_cast<const bf16x8*>(qp + (unsigned)(r * ldq + 8 * x8));
+  }
+  f32x4 re[NL], ru[NL];
+  const float *ep = ws.E + (cell * dv + cb) * DK, *up = ws.U + (cu * dv + cb) * DK;
+  auto load = [&](int h) {                                 // HW key channels of the state's two parts
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int e = tid + 256 * i, r = min(e / (HW / 4), dv - cb - 1), x4 = e % (HW / 4);
+      const unsigned at = r * DK + h * HW + 4 * x4;
+      re[i] = *reinterpret_cast<const f32x4*>(ep + at);     // (zeros in front of a fresh sequence's first run)
+      if (ci > 0) ru[i] = *reinterpret_cast<const f32x4*>(up + at);
+    }
+  };
+  if (old) load(0);
+  bf16x4 rv[4][2];
+  const int v8 = tid & 7, vr = tid >> 3;                   // a thread's columns and first token of 32 at a time
+  auto load_kv = [&] {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = tid + 256 * i, r = min(e / (DK / 8), n - 1), x8 = e % (DK / 8);
+      rk[i] = *reinterpret_cast<const bf16x8*>(kp + (unsigned)(r * ldk + 8 * x8));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+        rv[i][x] = *reinterpret_cast<const bf16x4*>(vp + (unsigned)(min(32 * i + vr, n - 1) * ldv + min(8 * v8 + 4 * x, dv - cb - 4)));
+  };
+  // the state in front of the chunk is fu U + fe E
+  const double mp = fmax(mloc, msup);
+  const float fe = !MLSTM ? exp2f((float)msup) : msup == mp ? 1.f : exp2f((float)(msup - mp));
+  const float fu = !MLSTM || mloc == mp ? 1.f : exp2f((float)(mloc - mp));
+  if (tid < CK) {
+    sah[tid] = tv[0];
+    sal[tid] = tv[1];
+    if (MLSTM) {
+      const double F = (double)tv[TAB - 4] + (double)tv[TAB - 3], m = fmax((double)tv[TAB - 2] + (double)tv[TAB - 1], mp);
+      const float h = (float)-m;
+      sbh[tid] = h;
+      sbl[tid] = (float)(-m - (double)h);
+      if (cb == 0 && tid < n) {
+        efl[(size_t)(t0 + tid) * H + hd] = exp2f((float)(-(F + m)));
+        // behind the last chunk, here or at all
+        if (tid == n - 1 && (t0 + n == d.seq_off[c.s + 1] || (pc.count > 0 && c.idx == pc.first + pc.count - 1 && t0 + n == c.t0 + c.n)))
+          M[(size_t)d.slots[c.s] * H + hd] = (float)((F + m) * 0.69314718055994530942);
+      }
+    } else {
+      sbh[tid] = -tv[0];
+      sbl[tid] = -tv[1];
+      sx[tid] = tv[2];
+    }
+  } else if (MLSTM && tid - CK < DK) {
+    const int r = tid - CK;
+    sx[r] = (run ? fe * ws.NE[cell * DK + r] : 0.f) + (ci > 0 ? fu * ws.NU[cu * DK + r] : 0.f);
+  }
+  if (tid < 64) sbad[tid] = CK;
+  const bool work = 32 * w < n;
+  const int qi = 32 * w + l32;                              // this lane's query
+  bf16x8 qf[2 * NK];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {                           // (each wave its own 32 rows)
+    const int e = lane + 64 * i, r = e / (DK / 8), x8 = e % (DK / 8);
+    *reinterpret_cast<bf16x8*>(buf + (32 * w + r) * DK + 8 * op_piece<DK>(r, x8)) = rq[i];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int s = 0; s < 2 * NK; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(buf + qi * DK + 8 * op_piece<DK>(l32, 2 * s + half));
+  __syncthreads();
+  const float rh = sbh[32 * w], rl = sbl[32 * w];
+  f32x16 acc[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
+  const bool two = cb + 32 < dv;
+  const float est = MLSTM ? exp2f((float)(mp + (double)rh + (double)rl)) : exp2f(rh + rl);   // factor of the state at the wave's first query
+  if (old) {
+#pragma unroll
+    for (int h = 0; h < DK / HW; ++h) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) {
+        const int e = tid + 256 * i, r = e / (HW / 4), x4 = e % (HW / 4);
+        f32x4 x;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) x[t] = ci > 0 ? fe * re[i][t] + fu * ru[i][t] : fe * re[i][t];
+        const Split a = split3(x[0], x[1]), b = split3(x[2], x[3]);
+        bf16* row = buf + r * HW + 8 * op_piece<HW>(r, x4 >> 1) + 4 * (x4 & 1);
+        *reinterpret_cast<u32x2*>(row) = u32x2{a.h, b.h};
+        *reinterpret_cast<u32x2*>(row + 64 * HW) = u32x2{a.m, b.m};
+        *reinterpret_cast<u32x2*>(row + 2 * 64 * HW) = u32x2{a.l, b.l};
+      }
+      if (h + 1 < DK / HW)
+        load(h + 1);
+      else
+        load_kv();
+      __syncthreads();
+      if (work)
+#pragma unroll
+        for (int s = 0; s < HW / 16; ++s)
+#pragma unroll
+          for (int p = 2; p >= 0; --p) {
+            const bf16* bp = buf + (p * 64 + l32) * HW + 8 * op_piece<HW>(l32, 2 * s + half);
+            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[h * (HW / 16) + s], *reinterpret_cast<const bf16x8*>(bp), acc[0], 0, 0, 0);
+            if (two)
+              acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[h * (HW / 16) + s], *reinterpret_cast<const bf16x8*>(bp + 32 * HW), acc[1], 0, 0, 0);
+          }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[t][i] *= est;
+  } else {
+    load_kv();
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = tid + 256 * i, r = e / (DK / 8), x8 = e % (DK / 8);
+    *reinterpret_cast<bf16x8*>(buf + r * DK + 8 * op_piece<DK>(r, x8)) = rk[i];
+  }
+  // A masked score is a 0 that multiplies a later token's value: an infinite or NaN value would reach the queries in front of
+  // it.  It counts as 0 in the products, and its column is NaN from its token on.
+  unsigned m2 = 0u;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const u32x2 u = __builtin_bit_cast(u32x2, rv[i][x]);
+      m2 |= ((u[0] & 0x7f807f80u) + 0x00800080u) | ((u[1] & 0x7f807f80u) + 0x00800080u);      // bit 15 of a half: its exponent is all ones
+    }
+  if (m2 & 0x80008000u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int x = 0; x < 8; ++x)
+        if (!isfinite((float)rv[i][x >> 2][x & 3])) {
+          rv[i][x >> 2][x & 3] = (bf16)0.f;
+          atomicMin(sbad + 8 * v8 + x, 32 * i + vr);
+        }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 32 * i + vr;
+    *reinterpret_cast<bf16x8*>(sv + r * 64 + 8 * tr_piece<64>(r, v8)) =
+        bf16x8{rv[i][0][0], rv[i][0][1], rv[i][0][2], rv[i][0][3], rv[i][1][0], rv[i][1][1], rv[i][1][2], rv[i][1][3]};
   }
   __syncthreads();
-  if (work) {
-    const float bh = sbh[qi], bl = sbl[qi];
-    float rsum = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-      if (kt <= w) {
-        const bf16* kp = k + (size_t)(c.t0 + min(32 * kt + l32, c.n - 1)) * ldk + kh * DK + 8 * half;
-        bf16x8 kf[2 * NK];
-#pragma unroll
-        for (int s = 0; s < 2 * NK; ++s) kf[s] = *reinterpret_cast<const bf16x8*>(kp + 16 * s);
-        f32x16 p;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) p[i] = 0.f;
-#pragma unroll
-        for (int s = 0; s < 2 * NK; ++s) p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qf[s], p, 0, 0, 0);
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int j0 = 32 * kt + 8 * g4 + 4 * half;
-          const f32x4 ah = *reinterpret_cast<const f32x4*>(sah + j0), al = *reinterpret_cast<const f32x4*>(sal + j0),
-                      cw = *reinterpret_cast<const f32x4*>(sc + j0);
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            float y = p[4 * g4 + x] * __builtin_amdgcn_exp2f((bh + ah[x]) + (bl + al[x]));
-            if (!MLSTM) y *= cw[x];
-            y = j0 + x <= qi ? y : 0.f;
-            if (MLSTM) rsum += y;
-            bf16 a, b, e;
-            split3(y, a, b, e);
-            const int i = 4 * g4 + x;
-            pf[kt][i >> 3][0][i & 7] = a;
-            pf[kt][i >> 3][1][i & 7] = b;
-            pf[kt][i >> 3][2][i & 7] = e;
-          }
-        }
-      }
-    if (MLSTM) {
-      float dot = 0.f;
-#pragma unroll
-      for (int s = 0; s < 2 * NK; ++s)
-#pragma unroll
-        for (int x = 0; x < 8; ++x) dot += (float)qf[s][x] * sN[16 * s + 8 * half + x];
-      float t = rsum + sx[qi] * dot;
-      t += __shfl_xor(t, 32, 64);
-      if (half == 0 && qi < c.n) den[(size_t)(c.t0 + qi) * H + hd] = t * ga.qscale;
-    }
+  if (!work) return;
+  const float bh = sbh[qi], bl = sbl[qi];
+  float* const wk = swk + 16 * w * (w - 1);                  // 0, 32, 64, 96 numbers
+  float rsum = 0.f, roff = 0.f;
+  for (int j = lane; j < 32 * w; j += 64) {
+    const float e = __builtin_amdgcn_exp2f((rh + sah[j]) + (rl + sal[j]));
+    wk[j] = MLSTM ? e : e * sx[j];
   }
-  const float skip = MLSTM ? 0.f : ga.dskip[hd];
-  const bf16* vp = v + (size_t)c.t0 * ldv + (size_t)hd * dv;
-  const float* up = U + cell * dv * DK;
-  for (int cb = 0; cb < dv; cb += 32) {
-    bf16x4 rv[4];
-    const int c4 = tid & 7, vt = tid >> 3;
-    load_4x4(vp + (size_t)(4 * vt) * ldv + cb + 4 * c4, ldv, c.n - 4 * vt, cb + 4 * c4 < dv, rv);
-    f32x4 ru[NK];
-    if (old) {
+  const float eq = __builtin_amdgcn_exp2f((bh - rh) + (bl - rl));         // of this lane's query against the first
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  if (half == 0) sbh[qi] = eq;                              // (no other wave reads its queries' decays)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  unsigned pw[2][3][4];
+  const auto scores = [&](int kt) {
+    f32x16 p;
 #pragma unroll
-      for (int i = 0; i < NK; ++i) {
-        const int e = tid + 256 * i, r = e / (DK / 4), x4 = e % (DK / 4);
-        ru[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (cb + r < dv) ru[i] = *reinterpret_cast<const f32x4*>(up + (size_t)(cb + r) * DK + 4 * x4);
-      }
-    }
-    if (cb) __syncthreads();                                // the last columns' reads are done
-    // A masked score is a 0 that multiplies a later token's value: an infinite or NaN value would reach the queries in front of
-    // it.  It counts as 0 in the products, and its column is NaN from its token on.
-    int* const bad = sbad[(cb >> 5) & 1];
-    unsigned m[2] = {0u, 0u};
+    for (int i = 0; i < 16; ++i) p[i] = 0.f;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const u32x2 u = __builtin_bit_cast(u32x2, rv[x]);
-      m[0] |= (u[0] & 0x7f807f80u) + 0x00800080u;           // bit 15 of a half: its exponent is all ones
-      m[1] |= (u[1] & 0x7f807f80u) + 0x00800080u;
-    }
-    if ((m[0] | m[1]) & 0x80008000u)
+    for (int s = 0; s < 2 * NK; ++s)
+      p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          *reinterpret_cast<const bf16x8*>(buf + (32 * kt + l32) * DK + 8 * op_piece<DK>(l32, 2 * s + half)), qf[s], p, 0, 0, 0);
+    return p;
+  };
+  const auto keep = [&](int g4, const f32x4& y) {           // the scores of registers 4 g4 ..
+    const Split a = split3(y[0], y[1]), b = split3(y[2], y[3]);
+    const int i = 2 * (g4 & 1);
+    pw[g4 >> 1][0][i] = a.h;
+    pw[g4 >> 1][1][i] = a.m;
+    pw[g4 >> 1][2][i] = a.l;
+    pw[g4 >> 1][0][i + 1] = b.h;
+    pw[g4 >> 1][1][i + 1] = b.m;
+    pw[g4 >> 1][2][i + 1] = b.l;
+  };
+  const int li = lane & 15, g2 = (lane >> 4) & 1;
+  const auto values = [&](int kt) {                         // the operand's tokens are in the order of the score registers
 #pragma unroll
-      for (int x = 0; x < 4; ++x)
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-          if (!isfinite((float)rv[x][t])) {
-            rv[x][t] = (bf16)0.f;
-            atomicMin(bad + 4 * c4 + x, 4 * vt + t);
-          }
-#pragma unroll
-    for (int x = 0; x < 4; ++x) *reinterpret_cast<bf16x4*>(sv + (4 * c4 + x) * VP + 4 * vt) = rv[x];
-    if (old) {
-#pragma unroll
-      for (int i = 0; i < NK; ++i) {
-        const int e = tid + 256 * i, r = e / (DK / 4), x4 = e % (DK / 4);
-        bf16x4 h, m, l;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          bf16 a, b, g;
-          split3(ru[i][t], a, b, g);
-          h[t] = a;
-          m[t] = b;
-          l[t] = g;
-        }
-        bf16* row = ss + r * SP + 4 * x4;
-        *reinterpret_cast<bf16x4*>(row) = h;
-        *reinterpret_cast<bf16x4*>(row + 32 * SP) = m;
-        *reinterpret_cast<bf16x4*>(row + 2 * 32 * SP) = l;
-      }
-    }
-    __syncthreads();
-    if (!work) continue;
-    f32x16 acc;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-    if (old) {
-#pragma unroll
-      for (int s = 0; s < 2 * NK; ++s) {
-        const bf16* bp = ss + l32 * SP + 16 * s + 8 * half;
-#pragma unroll
-        for (int part = 2; part >= 0; --part)
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[s], *reinterpret_cast<const bf16x8*>(bp + part * 32 * SP), acc, 0, 0, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] *= sx[32 * w + c_row(i, half)];
-    }
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-      if (kt <= w) {
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-          const bf16* bp = sv + l32 * VP + 32 * kt + 16 * ks + 4 * half;
-          const bf16x4 b0 = *reinterpret_cast<const bf16x4*>(bp), b1 = *reinterpret_cast<const bf16x4*>(bp + 8);
+      for (int t = 0; t < 2; ++t)
+        if (t == 0 || two) {
+          const int r = 32 * kt + 16 * ks + 4 * half + (li >> 2), x8 = 4 * t + 2 * g2 + ((li >> 1) & 1);
+          const bf16x4 b0 = read_tr(sv + r * 64 + 8 * tr_piece<64>(r, x8) + 4 * (li & 1)),
+                       b1 = read_tr(sv + (r + 8) * 64 + 8 * tr_piece<64>(r + 8, x8) + 4 * (li & 1));
           const bf16x8 b = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
 #pragma unroll
-          for (int part = 2; part >= 0; --part) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf[kt][ks][part], b, acc, 0, 0, 0);
+          for (int part = 2; part >= 0; --part)
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                __builtin_bit_cast(bf16x8, u32x4{pw[ks][part][0], pw[ks][part][1], pw[ks][part][2], pw[ks][part][3]}), b, acc[t], 0, 0, 0);
         }
-      }
-    if (tid < 32) sbad[(~cb >> 5) & 1][tid] = CK;           // (for the next columns; this one's last readers are past a barrier)
-    const int col = cb + l32;
-    const int first = bad[l32];
-    if (col < dv) {
+  };
+  for (int kt = 0; kt < w; ++kt) {
+    const f32x16 p = scores(kt);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = 32 * w + c_row(i, half);
-        if (r < c.n) {
-          const float y = MLSTM ? acc[i] * ga.qscale : acc[i] + skip * (float)sv[l32 * VP + r];
-          out[((size_t)(c.t0 + r) * H + hd) * dv + col] = r >= first ? NAN : y;
-        }
+    for (int g4 = 0; g4 < 4; ++g4) {
+      f32x4 y = *reinterpret_cast<const f32x4*>(wk + 32 * kt + 8 * g4 + 4 * half);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        y[x] *= p[4 * g4 + x];
+        if (MLSTM) roff += y[x];
       }
+      keep(g4, y);
+    }
+    values(kt);
+  }
+  {
+    const f32x16 p = scores(w);
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const int j0 = 8 * g4 + 4 * half;
+      const f32x4 ah = *reinterpret_cast<const f32x4*>(sah + 32 * w + j0), al = *reinterpret_cast<const f32x4*>(sal + 32 * w + j0),
+                  cw = *reinterpret_cast<const f32x4*>(sx + 32 * w + j0), e = *reinterpret_cast<const f32x4*>(sbh + 32 * w + j0);
+      f32x4 y;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        y[x] = p[4 * g4 + x] * __builtin_amdgcn_exp2f((bh + ah[x]) + (bl + al[x]));
+        if (!MLSTM) y[x] *= cw[x];
+        y[x] = j0 + x <= l32 ? y[x] : 0.f;
+        if (MLSTM) rsum += y[x];
+        acc[0][4 * g4 + x] *= e[x];                         // rows 8 g4 + 4 half + x, against their wave's first
+        acc[1][4 * g4 + x] *= e[x];
+      }
+      keep(g4, y);
+    }
+    values(w);
+  }
+  if (MLSTM && cb == 0) {
+    float dot = 0.f;
+#pragma unroll
+    for (int s = 0; s < 2 * NK; ++s)
+#pragma unroll
+      for (int x = 0; x < 8; ++x) dot += (float)qf[s][x] * sx[16 * s + 8 * half + x];
+    float t = rsum + eq * (roff + est * dot);
+    t += __shfl_xor(t, 32, 64);
+    if (half == 0 && qi < n) den[(size_t)(t0 + qi) * H + hd] = t * ga.qscale;
+  }
+  const float skip = MLSTM ? 0.f : ga.dskip[hd];
+  // (a store that has no place goes past the end of its window and is dropped)
+  const auto win = __builtin_amdgcn_make_buffer_rsrc(out + ((size_t)t0 * H + hd) * dv, 0, ((n - 1) * H + 1) * dv * 4, 0x00020000);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int col = 32 * t + l32, first = sbad[col];
+    if (__any(first < CK))
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[t][i] = 32 * w + c_row(i, half) >= first ? NAN : acc[t][i];
+    const unsigned at = cb + col < dv ? ((unsigned)((32 * w + 4 * half) * H) * dv + cb + col) * 4 : 0x80000000u;
+    const bf16* own = sv + (32 * w + 4 * half) * 64 + (col & 7);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float y = acc[t][i];
+      if (MLSTM)
+        y *= ga.qscale;
+      else
+        y += skip * (float)own[c_row(i, 0) * 64 + 8 * tr_piece<64>(c_row(i, 0), col >> 3)];
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), win, at + (unsigned)(c_row(i, 0) * H) * dv * 4, 0, 0);
     }
   }
 }
 
-// floats of a slot; 0.4 us a token in the token-by-token form
-size_t chunk_floats(int H, int dk, int dv) { return (size_t)H * (6 + (size_t)dk * (dv + 1)); }
-PiecePlan chunk_plan(int T_, int B, int H, int dk, int dv, size_t most) {
-  return plan_pieces(T_, B, CK, chunk_floats(H, dk, dv), most, 0.4f);
+// Chunks of a run.  Longer runs pass less of the state through memory, but are fewer and take their chunks one after another, so there
+// have to be enough of them.  us at 1 / 2 / 4 chunks (state space, 64 heads of 128 x 64; mLSTM, 8 heads of 128 x 192): one prompt of 4093
+// tokens 110 / 101 / 95, twelve of 700 243 / 234 / 243, one of 1000 42 / 42 / 47; one of 9000 134 / 112 / 103, eight of 333 to 1024 89 / 82 /
+// 87, one of 3000 54 / 52 / 55, one of 700 31 / 34 / 44.
+int run_chunks(int T_, int B, int H, int dv) {
+  const long blocks = (long)((T_ + CK - 1) / CK) * H * ((dv + 63) / 64), mean = T_ / B;
+  return blocks >= 1536 && mean >= 8 * CK ? 4 : blocks >= 512 && mean >= 3 * CK ? 2 : 1;
+}
+// floats of a run's slot; 0.4 us a token in the token-by-token form
+size_t run_floats(int sc, int H, int dk, int dv) { return (size_t)H * (6 + sc * (4 + 6 * CK + (size_t)dk * (dv + 1))); }
+PiecePlan run_plan(int T_, int B, int H, int dk, int dv, int sc, size_t most) {
+  return plan_pieces(T_, B, CK * sc, run_floats(sc, H, dk, dv), most, 0.4f);
 }
 
 template <int NK, bool MLSTM>
 void chunk_launch(const bf16* q, int ldq, const bf16* k, int ldk, const bf16* v, int ldv, const GateArgs& ga, float* S, float* N,
                   float* M, float* out, float* den, float* efl, float* ws, size_t most, int H, int G, int dv, SeqDesc d,
                   hipStream_t st) {
-  const PiecePlan plan = chunk_plan(d.Ttot, d.B, H, 32 * NK, dv, most);
-  const size_t ns = plan.slots, cells = ns * H;
-  double* meta = reinterpret_cast<double*>(ws);
-  float* U = ws + 6 * cells + (6 * cells & 3);
-  float* NU = U + cells * dv * 32 * NK;
-  const int nb = (dv * 32 * NK + 1023) / 1024;
+  const int sc = run_chunks(d.Ttot, d.B, H, dv), dk = 32 * NK;
+  const PiecePlan plan = run_plan(d.Ttot, d.B, H, dk, dv, sc, most);
+  const size_t cells = plan.slots * H, state = (size_t)dv * dk;
+  Ws w_;
+  w_.sc = sc;
+  w_.sup = reinterpret_cast<double*>(ws);
+  w_.loc = w_.sup + 3 * cells;
+  w_.tab = reinterpret_cast<float*>(w_.loc + 2 * cells * sc);
+  w_.tab += (4 - ((w_.tab - ws) & 3)) & 3;
+  w_.E = w_.tab + cells * sc * (MLSTM ? 6 : 3) * CK;
+  w_.U = w_.E + cells * state;
+  w_.NE = w_.U + cells * (sc - 1) * state;
+  w_.NU = w_.NE + cells * dk;
+  const int nb = (int)((state + 1023) / 1024), cols = (dv + 63) / 64;
   for (int w = 0; w < plan.windows; ++w) {
-    const Pieces pc = {CK, w * plan.count, plan.count};
-    hipLaunchKernelGGL((k_chunk_state<NK, MLSTM>), dim3((unsigned)ns, H, (dv + 63) / 64), dim3(256), 0, st, k, ldk, v, ldv, ga, U,
-                       NU, meta, H, G, dv, pc, d);
-    hipLaunchKernelGGL((k_chunk_walk<MLSTM>), dim3(d.B * H, nb + (MLSTM ? 1 : 0)), dim3(256), 0, st, U, NU, meta, S, N, M, H,
-                       32 * NK, dv, nb, pc, d);
-    hipLaunchKernelGGL((k_chunk_out<NK, MLSTM>), dim3((unsigned)ns, H), dim3(256), 0, st, q, ldq, k, ldk, v, ldv, ga, U, NU, meta,
-                       M, out, den, efl, H, G, dv, pc, d);
+    const Pieces pc = {CK * sc, w * plan.count, plan.count};
+    hipLaunchKernelGGL((k_chunk_state<NK, MLSTM>), dim3((unsigned)plan.slots, H, cols), dim3(256), 0, st, k, ldk, v, ldv, ga, w_, H, G,
+                       dv, pc, d);
+    hipLaunchKernelGGL((k_chunk_walk<MLSTM>), dim3(d.B * H, nb + (MLSTM ? 1 : 0)), dim3(256), 0, st, w_, S, N, M, H, dk, dv, nb, pc,
+                       d);
+    hipLaunchKernelGGL((k_chunk_out<NK, MLSTM>), dim3((unsigned)(plan.slots * sc), H, cols), dim3(256), 0, st, q, ldq, k, ldk, v, ldv,
+                       ga, w_, M, out, den, efl, H, G, dv, pc, d);
   }
   LIPA_CHECK_LAUNCH();
 }
@@ -602,7 +820,8 @@ void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* 
 size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const void* S,
                         const void* N, int T_, int B, int H, int dk, int dv, size_t most) {
   const auto fits = [](const void* p, int ld, int n) { return ld % n == 0 && ((uintptr_t)p & (2 * n - 1)) == 0; };
-  if (code != 0 || dk % 32 != 0 || dk > 128 || dv % 4 != 0 || !fits(q, ldq, 8) || !fits(k, ldk, 8) || !fits(v, ldv, 4) ||
+  if (code != 0 || dk % 32 != 0 || dk > 128 || dv % 4 != 0 || (long)H * dv >= 1l << 22 || std::max({ldq, ldk, ldv}) >= 1 << 22 ||
+      !fits(q, ldq, 8) || !fits(k, ldk, 8) || !fits(v, ldv, 4) ||
       !fits(S, 8, 8) || !fits(N, 8, 8))
     return 0;
   // Three launches and a chunk of padding against 0.4 us a token (two heads a CU) in the token-by-token form: 64 tokens a
@@ -617,8 +836,9 @@ size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk
   if (pairs >= 1024 && (dk <= 64 || dv <= 32)) least = 192;
   if (pairs * dv >= 1l << 17 && dk <= 32) least = 256;
   if (B == 0 || T_ < least * B) return 0;
-  const size_t slots = chunk_plan(T_, B, H, dk, dv, most).slots;
-  return slots == 0 ? 0 : slots * chunk_floats(H, dk, dv) + 4;
+  const int sc = run_chunks(T_, B, H, dv);
+  const size_t slots = run_plan(T_, B, H, dk, dv, sc, most).slots;
+  return slots == 0 ? 0 : slots * run_floats(sc, H, dk, dv) + 4;
 }
 
 void seq_chunk_ssd(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const void* dt, int lddt,

@@ -484,3 +484,43 @@ def test_rows_that_wide_loads_cannot_take(op, which):
         return [*(o if isinstance(o, (tuple, list)) else [o]), *st.values()]
     got, want = run(True), run(False)
     _close(got, want, [str(j) for j in range(len(got))])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["ssd", "mlstm"])
+@pytest.mark.parametrize("lens,H,dk,dv", [([2049, 2175], 48, 128, 64), ([385, 700, 513], 40, 64, 36), ([640, 129, 511], 32, 32, 100),
+                                          ([4100], 24, 96, 68), ([1280, 256], 16, 128, 192)])
+@pytest.mark.parametrize("bad", [None, 5, 300])
+def test_runs_of_chunks(op, lens, H, dk, dv, bad):
+    """Runs of two and four chunks, whole and cut off in each of them, against the token-by-token kernel; with an infinite value in the
+    first and in a later chunk: it reaches its own column of the outputs behind it and nothing else."""
+    from llm_in_practise_amd.ops._native import native_seq
+    ext = native_seq()
+    g = torch.Generator().manual_seed(dk + dv)
+    T, B = sum(lens), len(lens)
+    assert -(-T // 128) * H * -(-dv // 64) >= 512 and T // B >= 384
+
+    def rand(*s, dt=torch.float32):
+        return torch.randn(*s, generator=g).to(dt).cuda()
+    q, k, v = (rand(T, H * n, dt=torch.bfloat16) for n in (dk, dk, dv))
+    if bad is not None:
+        v[bad, dv + 1] = float("inf")                   # head 1, column 1 of the first sequence
+    i, f, a, b, skip = rand(T, H), rand(T, H), rand(H), rand(H), rand(H)
+    S0, N0 = rand(B, H, dv, dk), rand(B, H, dk)
+    res = []
+    for most in (1 << 28, 0):
+        st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lens, [7 * (j % 2) for j in range(B)], "cuda")
+        st["S"].copy_(S0)
+        st["N"].copy_(N0)
+        st["M"].fill_(0.5)
+        if op == "ssd":
+            out = [ext.ssd_scan(q, k, v, i.bfloat16(), a - 3, b, skip, st["S"], H, H, sb.desc, None, most=most).view(T, H, dv)]
+        else:
+            out = ext.mlstm_scan(q, k, v, i, f, a, b + 3, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb.desc, None, most=most)
+        res.append([*out, st["S"], st["N"], st["M"]])
+    assert ext.scan_floats(op, T, B, H, dk, dv) > 0
+    for x, y in zip(*res):
+        x, y = x.double(), y.double()
+        assert torch.equal(torch.isfinite(x), torch.isfinite(y))
+        x, y = (torch.nan_to_num(t, 0.0, 0.0, 0.0) for t in (x, y))
+        assert (x - y).norm() <= TOL * y.norm(), ((x - y).norm() / y.norm()).item()
