@@ -6,6 +6,9 @@
 // several rows: the reads, not the arithmetic, bound a scan whose lanes own one column each.
 #include "seq_common.h"
 
+#include <cfloat>
+#include <utility>
+
 using namespace lipa;
 
 namespace {
@@ -247,6 +250,168 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
     }
 }
 
+// ------------------------------------------------------------------------------- selective scan, one state per lane
+// Prompts whose sequences do not fill the chip: a lane owns ONE state, a row of 16 lanes a channel, so that two sequences of 4096 channels
+// of 16 states are two waves on every SIMD where the tiles of k_selective_scan are half a wave, and nothing has to be cut over time, which
+// takes every exponential twice.  64 tokens are staged at once: a thread fetches four tokens of one channel (and of one column of B and C) in
+// rows of 16, finishes their dt and dt x and leaves them transposed in LDS.  In the scan lane t of a row holds dt and dt x of token t of 16 and
+// hands them to the row with the multiplication that reads them (row_newbcast); a lane's 16 read-outs are summed over the row in
+// halves (15 adds for 16 sums), which leaves lane t with token t, in the place of its dt.
+// Bound by issue: a half-rate exponential and four instructions a token and state, three for the sums, three for the staging.  Two
+// prompts of 2048 and 1337 tokens, 4096 channels of 16: 129 -> 87 us (35 ns a token with one wave on a SIMD, 19 a wave with many).  With x, z
+// and dt fetched where they are needed (16 rows a load) the address units were busy for 80% of 123 us.
+constexpr int RT = 64, RLD = RT + 4, DLD = RT + 20;      // tokens staged at once; rows of B and C, of dt and dt x in LDS (for the banks)
+
+template <int L>
+__device__ __forceinline__ float row_lane(float v) {       // lane L of every row, in all lanes of the row
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + L, 0xF, 0xF, true));
+}
+// lanes where `hi` keep b and give a away, the others keep a and give b; the partner is the lane that CTRL names
+template <int CTRL>
+__device__ __forceinline__ float half_sum(float a, float b, bool hi) {
+  return (hi ? b : a) + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(hi ? a : b), CTRL, 0xF, 0xF, true));
+}
+// the bits of a T through a bounds-checked window
+template <typename T>
+struct Raw {
+  using type = unsigned short;
+  template <typename W>
+  static __device__ __forceinline__ type load(W w, unsigned o) { return __builtin_amdgcn_raw_buffer_load_b16(w, o, 0, 0); }
+  static __device__ __forceinline__ float value(type v) { return __uint_as_float((unsigned)v << 16); }
+  template <typename W>
+  static __device__ __forceinline__ void store(W w, unsigned o, float v) {
+    __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, (T)v), w, o, 0, 0);
+  }
+};
+template <>
+struct Raw<float> {
+  using type = unsigned;
+  template <typename W>
+  static __device__ __forceinline__ type load(W w, unsigned o) { return __builtin_amdgcn_raw_buffer_load_b32(w, o, 0, 0); }
+  static __device__ __forceinline__ float value(type v) { return __uint_as_float(v); }
+  template <typename W>
+  static __device__ __forceinline__ void store(W w, unsigned o, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), w, o, 0, 0);
+  }
+};
+__device__ __forceinline__ auto window(const void* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+
+// the decays and inputs of 16 tokens, for one state
+template <int... I>
+__device__ __forceinline__ void row_tokens(std::integer_sequence<int, I...>, float dt, float dx, float A, const float* b,
+                                           float (&e)[16], float (&in)[16]) {
+  ((e[I] = __builtin_amdgcn_exp2f(row_lane<I>(dt) * A), in[I] = row_lane<I>(dx) * b[I]), ...);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_selective_row(const T* __restrict__ x, int ldx, const float* __restrict__ dtp,
+                                                       const float* __restrict__ dtb, const T* __restrict__ bm, int ldb,
+                                                       const T* __restrict__ cm, int ldc, const float* __restrict__ a_log,
+                                                       const float* __restrict__ dskip, const T* __restrict__ z, int ldz,
+                                                       float* __restrict__ S, T* __restrict__ out, int ldo, float scale, int C,
+                                                       int N, SeqDesc d) {
+  __shared__ __attribute__((aligned(16))) float sB[16 * RLD];
+  __shared__ __attribute__((aligned(16))) float sC[16 * RLD];
+  __shared__ float sdt[16 * DLD];                                 // [channel][token]: dt, then the read-out that takes its place
+  __shared__ float sdx[16 * DLD];                                 // dt x
+  const int s = blockIdx.y, tid = threadIdx.x, lane = tid & 15, row = tid >> 4;
+  if (d.live && !d.live[s]) return;
+  // consecutive channels on the same die: a line of x, z or dt is read by up to four blocks
+  const int groups = gridDim.x, cg = groups % 8 == 0 ? (blockIdx.x & 7) * (groups >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const int t0 = d.seq_off[s], t1 = d.seq_off[s + 1];
+  // in the scan a thread is a state of channel `row`, everywhere else channel `lane` of token `row` of 16
+  const int c = cg * 16 + row, fc = cg * 16 + lane, ch = min(c, C - 1), fch = min(fc, C - 1);
+  const bool own = c < C && lane < N;
+  float* Sp = S + ((size_t)d.slots[s] * C + ch) * N + lane;
+  float st = own && d.pos0[s] > 0 ? *Sp : 0.f;
+  float A = -expf(own ? a_log[(size_t)ch * N + lane] : 0.f) * 1.4426950408889634f;      // decays as powers of two
+  A = A < -FLT_MAX ? -FLT_MAX : A;                                // (past a sequence's end it meets steps of 0)
+  const float bias = dtb[fch], skip = dskip[fch];
+  // Windows of 64 tokens move along the rows, so that a thread's places in them never change; what is past a sequence's end, or no
+  // state, reads as 0 and is not written.
+  constexpr unsigned E = sizeof(T), NOWHERE = ~0u - 64;
+  unsigned ox[4], oz[4], od[4], ob[4], oc[4], oo[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const unsigned t = 16 * i + row;
+    ox[i] = (t * ldx + fch) * E;
+    oz[i] = (t * ldz + fch) * E;
+    od[i] = (t * C + fch) * 4;
+    oo[i] = fc < C ? (t * ldo + fc) * E : NOWHERE;
+    ob[i] = lane < N ? (t * ldb + lane) * E : NOWHERE;
+    oc[i] = lane < N ? (t * ldc + lane) * E : NOWHERE;
+  }
+  typename Raw<T>::type fx[4], fz[4], fb[4], fcc[4];
+  float fd[4];
+  auto fetch = [&](int tb) {
+    const unsigned n = min(RT, t1 - tb);
+    const auto wx = window(x + (size_t)tb * ldx, n * ldx * E), wz = window(z + (size_t)tb * ldz, n * ldz * E),
+               wd = window(dtp + (size_t)tb * C, n * C * 4), wb = window(bm + (size_t)tb * ldb, n * ldb * E),
+               wc = window(cm + (size_t)tb * ldc, n * ldc * E);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      fd[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wd, od[i], 0, 0));
+      fx[i] = Raw<T>::load(wx, ox[i]);
+      fz[i] = Raw<T>::load(wz, oz[i]);
+      fb[i] = Raw<T>::load(wb, ob[i]);
+      fcc[i] = Raw<T>::load(wc, oc[i]);
+    }
+  };
+  if (t0 < t1) fetch(t0);
+  for (int tb = t0; tb < t1; tb += RT) {
+    const int n = min(RT, t1 - tb);
+    float gx[4], gz[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = 16 * i + row;
+      // (past the end tokens that change nothing; a selection would be a branch)
+      const float dt = __uint_as_float(__float_as_uint(softplus_fast(fd[i] + bias)) & (t < n ? ~0u : 0u));
+      gx[i] = Raw<T>::value(fx[i]);
+      gz[i] = Raw<T>::value(fz[i]);
+      sdt[lane * DLD + t] = dt;
+      sdx[lane * DLD + t] = dt * gx[i];
+      sB[lane * RLD + t] = Raw<T>::value(fb[i]);
+      sC[lane * RLD + t] = Raw<T>::value(fcc[i]);
+    }
+    __syncthreads();
+    if (tb + RT < t1) fetch(tb + RT);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (16 * u >= n) break;
+      float p[16], e[16], in[16], b[16];
+      const float *pb = sB + lane * RLD + 16 * u, *pc = sC + lane * RLD + 16 * u;
+      float& place = sdt[row * DLD + 16 * u + lane];
+      const float dt = place, dx = sdx[row * DLD + 16 * u + lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        *reinterpret_cast<f32x4*>(b + 4 * i) = *reinterpret_cast<const f32x4*>(pb + 4 * i);
+        *reinterpret_cast<f32x4*>(p + 4 * i) = *reinterpret_cast<const f32x4*>(pc + 4 * i);
+      }
+      row_tokens(std::make_integer_sequence<int, 16>{}, dt, dx, A, b, e, in);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        st = __builtin_fmaf(e[i], st, in[i]);
+        p[i] *= st;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) p[i] = half_sum<0x128>(p[i], p[i + 8], lane & 8);          // row_ror 8: lane ^ 8
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] = half_sum<0x141>(p[i], p[i + 4], lane & 4);          // row_half_mirror: lane ^ 7
+#pragma unroll
+      for (int i = 0; i < 2; ++i) p[i] = half_sum<0x4E>(p[i], p[i + 2], lane & 2);           // quad_perm [2, 3, 0, 1]
+      place = half_sum<0xB1>(p[0], p[1], lane & 1);                                          // quad_perm [1, 0, 3, 2]
+    }
+    __syncthreads();
+    const auto wo = window(out + (size_t)tb * ldo, (unsigned)n * ldo * E);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      Raw<T>::store(wo, oo[i], (sdt[lane * DLD + 16 * i + row] + skip * gx[i]) * silu_fast(gz[i]) * scale);
+  }
+  if (own) *Sp = st;
+}
+
 // The states in front of a sequence's segments, one (channel, state) per thread: they replace the states that the segments left.
 __global__ __launch_bounds__(256) void k_selective_walk(const float* __restrict__ a_log, const float* __restrict__ S,
                                                         float* __restrict__ ws, const float* __restrict__ wdt, int C, int N,
@@ -399,6 +564,17 @@ __global__ __launch_bounds__(256) void k_gla_scan(const T* __restrict__ q, int l
 int seq_selective_max_states() { return 256; }
 int seq_gla_max_dk() { return 256; }
 
+// Whether a step runs with a state per lane.  Its longest sequence takes 0.034 us a token; the mean length stands for the longest one, half
+// as much again where there are several.  Beyond 12 waves on a SIMD (49152 channels of sequences) both forms are bound by issue, and
+// eight states per lane need fewer instructions; below 32 tokens staging 64 is most of the work.  us, the other form -> a state per lane, 16
+// states, sequences x tokens x channels: 1 x 256 x 4096 30 -> 12, 1 x 1024 x 4096 61 -> 38, 1 x 4096 x 4096 155 -> 141, 1 x 9000 x 4096 320 ->
+// 334, 1 x 4096 x 2048 102 -> 143 (cut), 1 x 1024 x 1024 37 -> 37 (cut), 2048 + 1337 x 4096 129 -> 87, 4 x 512 x 4096 91 -> 49, 12 x 32 x 4096 14
+// -> 13, 16 x 16 x 4096 9.5 -> 15 (whole), 16 x 512 x 4096 164 -> 161, 16 x 512 x 8192 290 -> 314 (whole), 64 x 64 x 2048 42 -> 45 (whole).
+bool seq_selective_rows(int T_, int B, int C, int N) {
+  if (N <= 8 || N > 16 || T_ < 32l * B || (long)B * C > 49152) return false;
+  return 0.034f * (B > 1 ? 1.5f : 1.f) * T_ / B < 8.5e-6f * T_ * C + 25.f;
+}
+
 // Tokens of a segment of the scan cut over time, or 0 where sequences run whole.  Whole, a sequence takes `whole` us a token as
 // long as the chip is not full, and more after that; cut, a step takes about 25 us and `cut` us per token and channel (every exponential
 // twice).  The lengths are not known here: their mean stands for the longest one, so that ragged steps run whole more often than they need.
@@ -449,7 +625,10 @@ void seq_selective_scan(int code, const void* x, int ldx, const float* dtp, cons
     }                                                                                                                    \
   } while (0)
   SEQ_DISPATCH_T(code, {
-    if (N <= 16)
+    if (seq_selective_rows(d.Ttot, d.B, C, N))
+      hipLaunchKernelGGL((k_selective_row<T>), dim3((C + 15) / 16, d.B), dim3(256), 0, st, (const T*)x, ldx, dtp, dtb, (const T*)b, ldb,
+                         (const T*)c, ldc, a_log, dskip, (const T*)z, ldz, S, (T*)out, ldo, scale, C, N, d);
+    else if (N <= 16)
       SEL_LAUNCH(4, 4);
     else if (N <= 32)
       SEL_LAUNCH(4, 8);

@@ -332,6 +332,70 @@ def test_selective_cut_over_time(lens, starts, C, N, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lens,starts", [([64], [0]), ([63, 65, 16, 1, 129], [0, 3, 0, 0, 7]), ([17, 48, 80], [5, 0, 0]), ([400], [9])])
+@pytest.mark.parametrize("C,N,dt", [(16, 16, torch.bfloat16), (129, 16, torch.float32), (130, 9, torch.bfloat16), (40, 13, torch.float32)])
+def test_selective_with_a_state_per_lane(lens, starts, C, N, dt):
+    """Edges of the 16 and 64 tokens and 16 channels of a block, padded states, column slices, an idle sequence, decays of 0 and 1."""
+    from llm_in_practise_amd.ops._native import native_seq
+    g = torch.Generator().manual_seed(C + N)
+    T, live = sum(lens), [int(b != 2) for b in range(len(lens))]
+    assert native_seq().selective_rows(T, len(lens), C, N) or T < 32 * len(lens)
+    P, bc = torch.randn(T, 2 * C + 1, generator=g).to(dt), torch.randn(T, 2 * N + 3, generator=g).to(dt)
+    dtp, dtb, skip = torch.randn(T, C, generator=g), torch.randn(C, generator=g) - 2, torch.randn(C, generator=g)
+    a_log = torch.randn(C, N, generator=g)
+    a_log[:, 0], a_log[0] = -30.0, 100.0                # (the second: an infinite rate, a channel that forgets everything)
+    S0 = torch.randn(len(lens), C, N, generator=g)
+    res = []
+    for dev in ("cpu", "cuda"):
+        st, sb = _batch({"S": ((C, N), "f32")}, lens, starts, dev, live)
+        st["S"].copy_(S0)
+        p, q, out = P.to(dev), bc.to(dev), torch.zeros(T, C + 3, dtype=dt, device=dev)
+        R.selective_scan(p[:, :C], *[t.to(dev) for t in (dtp, dtb)], q[:, 1:N + 1], q[:, N + 2:2 * N + 2], a_log.to(dev), skip.to(dev),
+                         p[:, C + 1:], st["S"], sb, out[:, 1:C + 1], 0.5)
+        tok = torch.cat([torch.full((n,), bool(on)) for n, on in zip(lens, live)])
+        res.append((out[tok.to(dev)].float().cpu(), st["S"].cpu()))
+    (y1, s1), (y0, s0) = res[1], res[0]
+    _close((s1,), (s0,), ("state",))
+    if len(lens) > 2:
+        assert torch.equal(s1[len(lens) - 3], S0[len(lens) - 3])        # (slots run backwards)
+    tol = TOL if dt == torch.float32 else 2.0 ** -8      # (bf16 outputs: both sides round, to at most one unit of 2^-8 apart)
+    assert torch.isfinite(y1).all() and (y1 - y0).norm() <= tol * y0.norm()
+    assert (y1[:, 0] == 0).all() and (y1[:, C + 1:] == 0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,value", [("x", float("inf")), ("b", float("nan")), ("b", float("inf")), ("c", float("nan")), ("dt", float("nan"))])
+@pytest.mark.parametrize("t", [40, 102, 203])
+def test_selective_token_that_is_no_number(name, value, t):
+    """At the last token of a sequence too (102, 203): what stands behind it in a block of 64 changes nothing."""
+    lens, C, N = [103, 101], 40, 16
+    g = torch.Generator().manual_seed(t)
+    T = sum(lens)
+    inputs = {n: torch.randn(T, w, generator=g).cuda() for n, w in (("x", C), ("dt", C), ("b", N), ("c", N), ("z", C))}
+    dtb, a_log, skip = (torch.randn(*s, generator=g).cuda() for s in ((C,), (C, N), (C,)))
+
+    def run(x):
+        st, sb = _batch({"S": ((C, N), "f32")}, lens, [0, 5], "cuda")
+        st["S"].fill_(0.5)
+        y = R.selective_scan(x["x"], x["dt"], dtb, x["b"], x["c"], a_log, skip, x["z"], st["S"], sb)
+        run.state = st["S"]
+        return (y,)
+    _planted(run, inputs, name, t, 1, value, lens)
+    if name == "b" and value == float("inf"):
+        assert (run.state[0 if t >= 103 else 1, :, 1].abs() == value).all()      # an infinite state is not NaN
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,B,C,N,rows", [
+    (256, 1, 4096, 16, True), (4096, 1, 4096, 16, True), (4096, 1, 2048, 16, False), (3385, 2, 4096, 16, True), (3500, 2, 2048, 16, False),
+    (2048, 4, 4096, 16, True), (384, 12, 4096, 16, True), (256, 16, 4096, 16, False), (8192, 16, 8192, 16, False), (1000, 2, 4096, 8, False),
+    (1000, 2, 4096, 17, False), (1, 1, 4096, 16, False)])
+def test_selective_takes_a_state_per_lane_where_that_is_faster(T, B, C, N, rows):
+    from llm_in_practise_amd.ops._native import native_seq
+    assert native_seq().selective_rows(T, B, C, N) == rows
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,B,C,N,cut", [
     (2048, 1, 4096, 16, True), (4096, 4, 4096, 16, True), (6400, 16, 4096, 16, False), (2048, 1, 8192, 32, True),
     (6400, 16, 1024, 32, False), (2048, 1, 4096, 64, True), (2048, 1, 8192, 64, False), (2048, 1, 4096, 128, True),
