@@ -7,33 +7,90 @@
 //    18 of a 6144 × 4096 product.)
 //  * up to 16 rows K is cut into the S pieces of skinny_splits, whose sums are added in order: the order, and so every bit of a
 //    product, does not depend on how the pieces are shared out.  The gated form and more rows take units of 64 or 128 in turns.
-//  * W fragments are the MFMA A operands, loaded straight from HBM (16 B per lane, whole 128-byte lines per row); one batch
-//    of steps per wave is in flight while another is multiplied.  x (tiny, L2-resident) supplies the B operands.
-//  * no load sits behind a branch: a partial batch loads its last step again and does not multiply it.
+//  * x and W come by LDS-DMA, 8 rows × 128 B an instruction, into a ring of RING 64-deep units that belongs to one wave: no barrier in
+//    the loop, a wave waits for its own loads.  As MFMA fragments straight from memory, where neighbouring lanes stand in
+//    different rows, a CU takes 37 KB/µs of them at most, wherever they are; in whole 64-byte pieces 110.
+//  * chunk c (16 B) of row r of an 8-row image stands in slot c ^ r: the fragments' ds_read_b128 are free of conflicts.
+//
+// µs with fragments from memory → through LDS, W cold, bit for bit the same, at 1 / 12 / 16 rows: 4096 × 4096 9.0 / 10.4 / 11.0 → 9.1 / 9.4 /
+// 9.6, 6144 × 4096 14.4 / 16.2 / 17.1 → 13.8 / 14.5 / 15.1, 1024 × 2048 4.6 / 5.7 / 6.0 → 3.9 / 4.1 / 4.2, 2 × 12288 × 4096 gated 40.7 / 45.6 /
+// 48.7 → 37.6 / 37.0 / 37.3 (5.4 TB/s), 2 × 9728 × 2560 gated 26.0 / 28.7 / 30.1 → 22.9 / 22.7 / 23.1.
 #include "common.h"
 
 using namespace lipa;
 
 namespace {
 
-// CUT: S pieces of kc, each with its own sum (red: S tiles); else units of UNIT in turns, a sum per wave (red: NW tiles).
-// B: 32-deep steps per batch; FULL: every piece is whole batches.
-template <int CT, int MT, int NW, int B, bool GLU, bool CUT, bool FULL, int UNIT>
+typedef __attribute__((address_space(3))) void* lds_ptr;
+typedef __amdgpu_buffer_rsrc_t rsrc;
+
+__device__ __forceinline__ rsrc window(const void* base) {
+  const uint64_t p = reinterpret_cast<uint64_t>(base);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)p), hi = __builtin_amdgcn_readfirstlane((uint32_t)(p >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), 0, 0xFFFFFFFFu, 0x00020000);
+}
+// 64 lanes x 16 bytes from memory into LDS [dst, dst + 1 KB), lane after lane; M0 is put back
+__device__ __forceinline__ void to_lds(const rsrc& rs, uint32_t dst, uint32_t voff, uint32_t soff) {
+  uint32_t keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %2, %3, %4 offen lds\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "s"(dst), "v"(voff), "s"(rs), "s"(soff)
+      : "memory");
+}
+// until all but the last `left` units (at most R), of D loads each, have landed
+template <int D, int R>
+__device__ __forceinline__ void wait_units(int left) {
+  if constexpr (R == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else {
+    if (left >= R)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R * D) : "memory");
+    else
+      wait_units<D, R - 1>(left);
+  }
+}
+
+// How K is cut into parts, each a chain of products whose sums are added in order: S pieces, or a part per wave of units of 64 or 128 in turns
+enum { PIECES, TURNS64, TURNS128 };
+
+template <int CT, int MT, int NW, int RING, bool GLU, int CUT, int PARTS>
 __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W,
                                                          const bf16* __restrict__ res, bf16* __restrict__ out, int M, int N,
                                                          int K, int S) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  f32x4(*red)[CT * MT][64] = reinterpret_cast<f32x4(*)[CT * MT][64]>(smem);
+  constexpr int CO = GLU ? CT / 2 : CT, UB = (CT + MT) * 2048, D = 2 * (CT + MT), RINGS = NW * RING * UB, SUMS = PARTS * CT * MT * 1024;
+  constexpr bool BESIDE = CUT == PIECES;        // (sums are left while the rings run; else they take the rings' place)
+  static_assert((RING - 1) * D < 64, "the counter of outstanding loads");
+  __shared__ __attribute__((aligned(1024))) char smem[BESIDE ? RINGS + SUMS : RINGS > SUMS ? RINGS : SUMS];
+  f32x4(*red)[CT * MT][64] = reinterpret_cast<f32x4(*)[CT * MT][64]>(smem + (BESIDE ? RINGS : 0));
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * (GLU ? CT / 2 : CT);
-  const bf16 *wr[CT], *xr[MT];
+  const int n0 = blockIdx.x * 16 * CO;
+  const rsrc wr = window(W + (size_t)n0 * K), ur = window(W + (size_t)(GLU ? N + n0 : n0) * K), xr = window(X);
+  uint32_t wo[2 * CO], xo[2 * MT];
+  const int r8 = lane >> 3, ch = ((lane & 7) ^ r8) * 16;
 #pragma unroll
-  for (int t = 0; t < CT; ++t) {
-    const int n = GLU ? (t < CT / 2 ? 0 : N) + min(n0 + 16 * (t % (CT / 2 > 0 ? CT / 2 : 1)) + li, N - 1) : min(n0 + 16 * t + li, N - 1);
-    wr[t] = W + (size_t)n * K + 8 * g;
-  }
+  for (int j = 0; j < 2 * CO; ++j) wo[j] = (uint32_t)min(8 * j + r8, N - 1 - n0) * (uint32_t)K * 2 + ch;
 #pragma unroll
-  for (int m = 0; m < MT; ++m) xr[m] = X + (size_t)min(16 * m + li, M - 1) * ldx + 8 * g;
+  for (int j = 0; j < 2 * MT; ++j) xo[j] = (uint32_t)min(8 * j + r8, M - 1) * (uint32_t)ldx * 2 + ch;
+  const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)smem) + w * RING * UB;
+  // 64-deep units of a part in a row (per), of this wave (cnt), and the next one to load: part or turn lp, place lb in it.  A piece may
+  // end in half a unit: the one that ends there is loaded, and its second half multiplied.
+  const int len = CUT == PIECES ? K / S : CUT == TURNS64 ? 64 : 128, per = (len + 63) / 64, turns = CUT == PIECES ? S : K / len;
+  const int odd = CUT == PIECES ? len & 32 : 0;
+  const int cnt = (turns - w + NW - 1) / NW * per;
+  int lp = w, lb = 0;
+  auto fill = [&](int slot) {
+    const uint32_t dst = base + slot * UB, k = (lp * len + 64 * lb - (lb == per - 1 ? odd : 0)) * 2;
+#pragma unroll
+    for (int j = 0; j < 2 * CT; ++j) to_lds(GLU && j >= 2 * CO ? ur : wr, dst + j * 1024, wo[j % (2 * CO)], k);
+#pragma unroll
+    for (int j = 0; j < 2 * MT; ++j) to_lds(xr, dst + (2 * CT + j) * 1024, xo[j], k);
+    if (++lb == per) lb = 0, lp += NW;
+  };
   f32x4 acc[CT][MT];
   auto clear = [&] {
 #pragma unroll
@@ -41,77 +98,59 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict_
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
-  auto leave = [&](int slot) {
+  auto leave = [&](int part) {
 #pragma unroll
     for (int t = 0; t < CT; ++t)
 #pragma unroll
-      for (int m = 0; m < MT; ++m) red[slot][t * MT + m][lane] = acc[t][m];
+      for (int m = 0; m < MT; ++m) red[part][t * MT + m][lane] = acc[t][m];
   };
-  struct Batch {
-    bf16x8 a[B][CT], b[B][MT];
-  };
-  // steps of one piece (of the whole wave, if not CUT), batches of one piece, batches of this wave
-  const int kc = CUT ? K / S : K, steps = CUT ? kc / 32 : UNIT / 32 * ((K / UNIT - w + NW - 1) / NW), per = (steps + B - 1) / B;
-  const int nb = CUT ? (S - w + NW - 1) / NW * per : per;
-  int lp = w, lb = 0;                            // the next batch to load: its piece, its place in it
-  auto load = [&](Batch& s) {
+  clear();
+  for (int i = 0; i < min(RING, cnt); ++i) fill(i);
+  int rp = w, rb = 0;
+  for (int i = 0, slot = 0; i < cnt; ++i) {
+    wait_units<D, RING - 1>(cnt - 1 - i);
+    const char* p = smem + (w * RING + slot) * UB;
+    bf16x8 a[2][CT], b[2][MT];
 #pragma unroll
-    for (int u = 0; u < B; ++u) {
-      const int e = FULL ? lb * B + u : min(lb * B + u, steps - 1);
-      const int k = CUT ? lp * kc + 32 * e : UNIT * (w + NW * (e / (UNIT / 32))) + 32 * (e % (UNIT / 32));
+    for (int h = 0; h < 2; ++h) {
+      const int c = li * 128 + ((4 * h + g) ^ (li & 7)) * 16;
 #pragma unroll
-      for (int t = 0; t < CT; ++t) s.a[u][t] = *reinterpret_cast<const bf16x8*>(wr[t] + k);
+      for (int t = 0; t < CT; ++t) a[h][t] = *reinterpret_cast<const bf16x8*>(p + t * 2048 + c);
 #pragma unroll
-      for (int m = 0; m < MT; ++m) s.b[u][m] = *reinterpret_cast<const bf16x8*>(xr[m] + k);
+      for (int m = 0; m < MT; ++m) b[h][m] = *reinterpret_cast<const bf16x8*>(p + (CT + m) * 2048 + c);
     }
-    if (++lb == per) lb = 0, lp += NW;
-  };
-  int rp = w, rb = 0;                            // the next batch to multiply
-  auto run = [&](const Batch& s) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // the unit is in registers: its place is free
+    if (i + RING < cnt) fill(slot);
 #pragma unroll
-    for (int u = 0; u < B; ++u) {
-      if (!FULL && rb * B + u >= steps) break;
+    for (int h = 0; h < 2; ++h) {
+      if (CUT == PIECES && h == 0 && odd && rb == per - 1) continue;
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int t = 0; t < CT; ++t)
-          acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.a[u][t], s.b[u][m], acc[t][m], 0, 0, 0);
+        for (int t = 0; t < CT; ++t) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][t], b[h][m], acc[t][m], 0, 0, 0);
     }
-    if (++rb == per && CUT) {
+    if (CUT == PIECES && ++rb == per) {
       leave(rp);
       clear();
       rb = 0, rp += NW;
     }
-  };
-  clear();
-  if (nb > 0) {
-    Batch p, q;
-    load(p);
-    int i = 0;
-    for (; i + 2 < nb; i += 2) {
-      load(q);
-      run(p);
-      load(p);
-      run(q);
-    }
-    if (i + 1 < nb) {
-      load(q);
-      run(p);
-      run(q);
-    } else {
-      run(p);
-    }
+    slot = slot + 1 == RING ? 0 : slot + 1;
   }
-  if (!CUT) leave(w);
-  const int parts = CUT ? S : NW;
+  if (!BESIDE) {
+    __syncthreads();
+    leave(w);
+  }
+  const int parts = CUT == PIECES ? S : NW;
   __syncthreads();
   // lane holds C[n = n0 + 16 t + 4 g + i][m = 16 mt + li]
-  for (int c = w; c < (GLU ? CT / 2 : CT) * MT; c += NW) {
+  for (int c = w; c < CO * MT; c += NW) {
     const int t = c / MT, m = 16 * (c % MT) + li, n = n0 + 16 * t + 4 * g;
     f32x4 v = red[0][c][lane], up = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
     for (int s = 1; s < parts; ++s) v += red[s][c][lane];
     if (GLU) {
-      for (int s = 0; s < parts; ++s) up += red[s][c + CT / 2 * MT][lane];
+#pragma unroll 4
+      for (int s = 0; s < parts; ++s) up += red[s][c + CO * MT][lane];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {          // (rounded like the products they would have been)
         const float gt = (float)(bf16)v[e], ut = (float)(bf16)up[e];
@@ -138,47 +177,32 @@ static int skinny_splits(int N, int K) {
   return s;
 }
 
-// Column tiles and waves per workgroup, us at 1 / 8 / 16 rows: two tiles of 8 waves take 13.2 / 13.9 / 15.1 for 6144 x 4096 (one tile
-// of 4 waves 13.7 / 15.5 / 17.5) and 9.7 / 10.8 / 12.3 for 6144 x 2560 (10.7 / 12.3 / 14.4), but 4096 rows of W fill half the CUs with
-// them: 11.9 / 13.2 / 14.9 for K = 4096 against 9.0 / 9.7 / 10.9.  Batches of 5 steps where the pieces divide by them (2560: whole
-// batches 9.7, partial ones 11.8).
-// The gated form pairs 16 gate with 16 up rows.  4 waves of 64-deep units against 2 of 128-deep ones: with few workgroups the
-// waves count, 2 x 3072 x 1024 5.3 / 5.7 / 6.0 against 6.1 / 6.3 / 6.4, 2 x 2048 x 4096 12.4 / 13.7 / 14.9 against 15.7 / 16.5 / 17.2; with
-// many, the longer units: 2 x 8192 x 3072 20.7 / 22.5 / 24.9 against 19.8 / 20.5 / 22.4, 2 x 6912 x 2304 16.2 / 18.7 / 20.7 against 14.6 / 15.3
-// / 16.6.  Where K is a multiple of 2048 the four waves are ahead at one row all the same (2 x 12288 x 4096 39.1 / 40.8 / 45.7 against
-// 40.2 / 39.4 / 42.1, 2 x 8192 x 2048 16.5 / 17.6 / 17.9 against 17.1 / 17.3 / 16.5) and stay, since one row is where latency counts.
+// One tile of W a workgroup (GLU: 16 gate and 16 up rows).  Eight waves where one workgroup a CU holds all of W's tiles, else four, so
+// that two fit into a CU's LDS (6144 × 4096, 12 rows: 12.3 µs against 13.5 with two tiles of 8 waves); the gated form takes three of them.
 void launch_gemm_skinny(const void* X, int ldx, const void* W, const void* res, void* out, int M, int N, int K, bool glu,
                         hipStream_t st) {
-  const int pieces = skinny_splits(N, K), kc = K / pieces;        // (one tile of 1 KB of LDS each: up to 32)
-#define L(CT_, MT_, NW_, B_, GLU_, CUT_, FULL_, UNIT_)                                                                          \
-  gemm_skinny_k<CT_, MT_, NW_, B_, GLU_, CUT_, FULL_, UNIT_>                                                                       \
-      <<<(N + 16 * (GLU_ ? CT_ / 2 : CT_) - 1) / (16 * (GLU_ ? CT_ / 2 : CT_)), 64 * NW_, (CUT_ ? pieces : NW_) * CT_ * MT_ * 1024, \
-         st>>>((const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, pieces)
-#define PIECES(CT_, NW_, B_)                                                                         \
-  do {                                                                                               \
-    if (kc % (32 * B_) == 0) L(CT_, 1, NW_, B_, false, true, true, 64);                              \
-    else if (kc % 160 == 0) L(CT_, 1, NW_, 5, false, true, true, 64);                                \
-    else L(CT_, 1, NW_, 4, false, true, false, 64);                                                  \
-  } while (0)
-#define TURNS(CT_, NW_, B_, GLU_, UNIT_)                                                             \
-  do {                                                                                               \
-    if (M <= 16 && K % (UNIT_ * NW_) == 0 && K % (32 * B_ * NW_) == 0) L(CT_, 1, NW_, B_, GLU_, false, true, UNIT_); \
-    else if (M <= 16) L(CT_, 1, NW_, 4, GLU_, false, false, UNIT_);                                  \
-    else if (M <= 32) L(CT_, 2, NW_, 4, GLU_, false, false, UNIT_);                                  \
-    else L(CT_, 4, NW_, 4, GLU_, false, false, UNIT_);                                               \
-  } while (0)
-  if (glu) {
-    if (N > 4096 && K % 2048 && K % 128 == 0) TURNS(2, 2, 4, true, 128);
-    else TURNS(2, 4, 4, true, 64);
-  } else if (pieces <= 32 && M <= 16) {
-    if (N >= 6144) PIECES(2, 8, 4);
-    else PIECES(1, 4, 8);
+  const int pieces = skinny_splits(N, K);
+#define L(CT_, MT_, NW_, RING_, GLU_, CUT_, PARTS_)                                                                        \
+  gemm_skinny_k<CT_, MT_, NW_, RING_, GLU_, CUT_, PARTS_><<<(N + 15) / 16, 64 * NW_, 0, st>>>(                             \
+      (const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, pieces)
+  if (M > 32) {
+    if (glu) L(2, 4, 4, 3, true, TURNS64, 4);
+    else L(1, 4, 4, 3, false, TURNS64, 4);
+  } else if (M > 16) {
+    if (glu) L(2, 2, 4, 3, true, TURNS64, 4);
+    else L(1, 2, 4, 4, false, TURNS64, 4);
+  } else if (glu) {
+    if (N > 4096 && K % 2048 && K % 128 == 0) L(2, 1, 2, 4, true, TURNS128, 2);
+    else L(2, 1, 4, 2, true, TURNS64, 4);
+  } else if (pieces > 32) {
+    L(1, 1, 4, 4, false, TURNS64, 4);
+  } else if (pieces > 16) {
+    L(1, 1, 8, 3, false, PIECES, 32);
+  } else if (pieces >= 8 && N <= 4096) {
+    L(1, 1, 8, 4, false, PIECES, 16);
   } else {
-    if (N >= 6144) TURNS(2, 8, 4, false, 64);
-    else TURNS(1, 4, 8, false, 64);
+    L(1, 1, 4, 4, false, PIECES, 16);
   }
-#undef TURNS
-#undef PIECES
 #undef L
   LIPA_CHECK_LAUNCH();
 }

@@ -122,10 +122,9 @@ class _SkinnySwiGLUFn(torch.autograd.Function):
 def skinny_swiglu(x: torch.Tensor, gu_base) -> torch.Tensor | None:
     """``silu(x·W_gateᵀ)·(x·W_upᵀ)`` of up to 16 decode rows in one launch (csrc/kernels/skinny.hip), or None where that kernel
     does not serve: a bf16 [gate | up] weight, no gradient.  The products are rounded to bf16 before the activation, as the
-    separate kernels round them.  4096 → 2 × 12288, product and activation: 45 → 39 µs at 1 row, 46 → 46 at 16; above that a
-    library product pulls ahead (24 rows 44 + 5 against 52), and so it does for wider or deeper weights: 5120 → 2 × 17408 75 against
-    81 µs at 1 row and 77 against 98 at 16, 2560 → 2 × 27648 53 against 55 and 54 against 67, 5120 → 2 × 5120 25 against 28 and 26
-    against 36.  Up to 2 × 14336 and 4096 no width is slower (14336 × 4096 62 → 49 and 63 → 58, 3072 × 1024 10.1 → 5.3 and 10.4 → 6.0)."""
+    separate kernels round them.  Library and activation → here, µs at 1 / 16 rows: 4096 → 2 × 12288 48 / 49 → 38 / 37, 2560 → 2 × 9728
+    48 / 48 → 23 / 23, 1024 → 2 × 3072 10.1 / 10.1 → 5.1 / 5.2, 4096 → 2 × 14336 67 / 69 → 45 / 46.  Wider and deeper weights, and more rows,
+    stay with the library's product."""
     x2 = x.reshape(-1, x.shape[-1])
     if (torch.is_grad_enabled() and x.requires_grad) or not (
             x.is_cuda and x.dtype == torch.bfloat16 and isinstance(gu_base, torch.Tensor) and gu_base.dtype == torch.bfloat16

@@ -194,6 +194,19 @@ def test_gemm_skinny_pieces(native_ext, M, N, K):
         assert ((native_ext.gemm_skinny_swiglu(x, w).double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("N,K", [(512, 8192), (48, 576), (2048, 1984), (6160, 4096), (96, 64)])
+def test_gemm_skinny_rows_do_not_depend_on_their_number(native_ext, N, K):
+    """Pieces of 4 units to 32, of half a unit more, of one wave alone: a row's bits are those it has beside 15 others."""
+    torch.manual_seed(N)
+    xb, w = torch.randn(16, K + 8, device=DEV).to(torch.bfloat16), (torch.randn(N, K, device=DEV) * 0.02).to(torch.bfloat16)
+    x, res = xb[:, :K], torch.randn(16, N, device=DEV).to(torch.bfloat16)
+    y, h = native_ext.gemm_skinny(x, w, res), native_ext.gemm_skinny_swiglu(x, w)
+    assert (y.double() - (x.double() @ w.double().t() + res.double())).norm() <= 2.0 ** -8 * y.double().norm()
+    for m in (1, 9):
+        assert torch.equal(native_ext.gemm_skinny(x[:m], w, res[:m]), y[:m])
+        assert torch.equal(native_ext.gemm_skinny_swiglu(x[:m], w), h[:m])
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 40])
 @pytest.mark.parametrize("N,K", [(32, 64), (1056, 192), (6144, 1088), (64, 1984), (96, 20480)])
 def test_gemm_skinny_infinite_weights(native_ext, M, N, K):
