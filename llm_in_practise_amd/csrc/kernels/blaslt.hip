@@ -151,6 +151,7 @@ bool make_plan(Plan& p, bool ta, bool tb, long m, long n, long k, long lda, long
 
 // D = op(A)·op(B) (+ C when C != nullptr; beta = 1), column-major, bf16 in/out, fp32 accumulate.
 // tune: time the heuristic's top candidates on the first calls of the shape and keep the fastest.
+// ws nullptr: the heuristic's first choice, where that needs no workspace (else false).
 // Returns false when hipBLASLt has no plan for the problem (the caller falls back).
 bool lt_gemm(bool ta, bool tb, long m, long n, long k, const void* A, long lda, const void* B, long ldb,
              const void* C, void* D, long ldc, int batch, long sa, long sb, long sc, void* ws, size_t ws_bytes,
@@ -168,6 +169,7 @@ bool lt_gemm(bool ta, bool tb, long m, long n, long k, const void* A, long lda, 
     }
     p = &it->second;
   }
+  if (ws == nullptr && p->cand[0].workspaceSize > 0) return false;
   const float alpha = 1.f, beta = C ? 1.f : 0.f;
   if (p->chosen < 0 && !p->pending.empty()) {
     std::lock_guard<std::mutex> lk(g_mu);
@@ -177,7 +179,7 @@ bool lt_gemm(bool ta, bool tb, long m, long n, long k, const void* A, long lda, 
       fprintf(stderr, "[lt] m=%ld n=%ld k=%ld b=%d C=%d: candidate %d of %zu (%.1f us; first %.1f us)\n", m, n, k,
               batch, C != nullptr, p->chosen, p->cand.size(), 1e3f * p->best[p->chosen], 1e3f * p->best[0]);
   }
-  int idx = p->chosen;
+  int idx = ws == nullptr ? 0 : p->chosen;
   Plan::Pending timing{-1, nullptr, nullptr};
   if (idx < 0 && (!tune || (getenv("LIPA_DETERMINISTIC") && atoi(getenv("LIPA_DETERMINISTIC"))))) {
     // reproducible runs, or a shape called once per step: the heuristic's first choice, no rotation
@@ -198,7 +200,7 @@ bool lt_gemm(bool ta, bool tb, long m, long n, long k, const void* A, long lda, 
   }
   const hipblasStatus_t s =
       hipblasLtMatmul(g_handle, p->desc, &alpha, A, p->a, B, p->b, &beta, C ? C : D, p->c, D, p->d,
-                      &p->cand[idx].algo, ws, ws_bytes, st);
+                      &p->cand[idx].algo, ws, ws == nullptr ? 0 : ws_bytes, st);
   if (s != HIPBLAS_STATUS_SUCCESS) {
     fprintf(stderr, "hipBLASLt matmul failed (%d) m=%ld n=%ld k=%ld\n", (int)s, m, n, k);
     return false;

@@ -172,9 +172,9 @@ def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
     N = base.shape[0]
     if (x.is_cuda and M <= 16 and N <= 8192 and K <= 8192 and N % 16 == 0 and K % 64 == 0 and x.stride(0) % 8 == 0
             and x.stride(1) == 1 and base.is_contiguous()):
-        # decode-sized q|k|v / o projections: the weight-streaming MFMA kernel (csrc/kernels/skinny.hip) takes 9-11 µs for
-        # 4096 × 4096 and 1-16 rows, residual included, where hipBLASLt takes 15.5 (13.2-15.1 against 14.2 for 6144 rows of W).
-        # A long K re-reads x in every workgroup: 4096 × 12288 is even at 1-8 rows and 25.6 against 21.6 µs at 16
+        # decode-sized q|k|v / o projections: the weight-streaming MFMA kernel (csrc/kernels/skinny.hip) takes 9.1-9.6 µs for
+        # 4096 × 4096 and 1-16 rows, residual included, where hipBLASLt takes 17.4 (13.8-15.1 against 14.0-14.4 for 6144 rows of W,
+        # 27 against 29-31 for 8192 × 8192).  A longer K stays with the library, whose sums' order its users have
         _count("decode")
         y = native().gemm_skinny(x, base, residual)
         return y if ext_a is None else y.addmm_(ext_a, ext_b.t())
@@ -185,7 +185,12 @@ def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
     # shapes gemm4w does not take (CPU, M < 256, K % 64): torch — residual = addmm's beta term, the LoRA
     # K-slice one rank-Σr update
     _count("library")
-    y = torch.addmm(residual, x, base.t()) if residual is not None else x @ base.t()
+    if residual is None:
+        y = x @ base.t()
+    elif x.is_cuda and M <= 64:             # (decode rows: the same product without a launch that copies the residual)
+        y = native().lt_addmm(residual, x, base)
+    else:
+        y = torch.addmm(residual, x, base.t())
     if ext_a is not None:
         y.addmm_(ext_a, ext_b.t())
     return y

@@ -194,7 +194,7 @@ def test_gemm_skinny_pieces(native_ext, M, N, K):
         assert ((native_ext.gemm_skinny_swiglu(x, w).double() - want).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("N,K", [(512, 8192), (48, 576), (2048, 1984), (6160, 4096), (96, 64)])
+@pytest.mark.parametrize("N,K", [(512, 8192), (64, 576), (2048, 1984), (6176, 4096), (96, 64)])
 def test_gemm_skinny_rows_do_not_depend_on_their_number(native_ext, N, K):
     """Pieces of 4 units to 32, of half a unit more, of one wave alone: a row's bits are those it has beside 15 others."""
     torch.manual_seed(N)
@@ -220,6 +220,29 @@ def test_gemm_skinny_infinite_weights(native_ext, M, N, K):
     assert torch.equal(y.isinf(), want.isinf()) and not y.isnan().any()
     h = native_ext.gemm_skinny_swiglu(x, w).float()
     assert torch.equal(h.isinf(), want[:, :N // 2].isinf() | want[:, N // 2:].isinf()) and not h.isnan().any()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 12288), (33, 4096, 4096), (64, 2560, 9728), (17, 40, 72), (5, 24, 8)])
+def test_product_with_residual_has_addmms_bits(native_ext, M, N, K):
+    """Without the copy of the residual; forms that are not taken so (strides, broadcasts, an address off) reach torch.addmm, and
+    replays of a captured call see new inputs."""
+    torch.manual_seed(M)
+    w, x, r = torch.randn(N, K, device=DEV).bfloat16(), torch.randn(M, K, device=DEV).bfloat16(), torch.randn(M, N, device=DEV).bfloat16()
+    off = torch.cat([r.new_zeros(1), r.reshape(-1)])[1:].view(M, N)
+    for res in (r, off, r[:1].expand(M, N), r.t().contiguous().t(), r[0]):
+        before = res.clone()
+        assert torch.equal(native_ext.lt_addmm(res, x, w), torch.addmm(res, x, w.t())) and torch.equal(res, before)
+    xt = x.t().contiguous().t()
+    assert torch.equal(native_ext.lt_addmm(r, xt, w), torch.addmm(r, xt, w.t()))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = native_ext.lt_addmm(r, x, w)
+    for seed in range(3):
+        torch.manual_seed(seed)
+        x.copy_(torch.randn(M, K, device=DEV))
+        r.copy_(torch.randn(M, N, device=DEV))
+        g.replay()
+        assert torch.equal(y, torch.addmm(r, x, w.t()))
 
 
 @pytest.mark.parametrize("F,K,own", [(14336, 128, True), (14352, 128, False), (17408, 5120, False), (32, 4096, True), (32, 4160, False)])
