@@ -14,8 +14,8 @@
 // Measured, token by token -> blocks: three sequences of 1500, 700 and 97 tokens, 8 delta heads of 128 x 128: 576 -> 112 us (26
 // for the first kernel, 86 for the walk); eight sequences of 512 tokens, 16 linear-attention heads of 64 x 128: 119 -> 71 us.
 // Error against 64 bits as before (2.1e-7).  Ten inputs a lane two or three blocks ahead gave 2.0 -> 0.94 us a block of the longest
-// sequence.
-#include "seq_common.h"
+// sequence.  Long delta prompts that fill the chip at most once run in blocks of 32 tokens (seq_delta.hip).
+#include "seq_block.h"
 
 #include <type_traits>
 
@@ -23,25 +23,9 @@ using namespace lipa;
 
 namespace {
 
-constexpr int BT = 16;      // tokens of a block
-
 // what the first kernel leaves per (block, head): [k G | q G | k G_16 / G] in operand order, G_16, T, B; and behind these, per
 // (block, head) and of each of its four waves, whether a value of its tokens is infinite or NaN
 __host__ __device__ constexpr int cell_floats(int dk) { return 3 * BT * dk + dk + 2 * BT * BT; }
-
-__device__ __forceinline__ float row16_sum(float v) {       // over the 16 lanes of a row, in all of them
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));    // quad_perm [1, 0, 3, 2]
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));    // quad_perm [2, 3, 0, 1]
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true));   // row_half_mirror
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xF, 0xF, true));   // row_mirror
-  return v;
-}
-
-__device__ __forceinline__ f32x4 row4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
-__device__ __forceinline__ f32x4 row4(const bf16* p) {
-  const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
-  return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
-}
 
 struct DecayArgs {
   const float* g;           // [T, H * dk]: decays (delta rule) or their pre-activations (linear attention)
@@ -377,6 +361,10 @@ void dispatch(int code, const void* q, int ldq, const void* k, int ldk, const vo
 
 }  // namespace
 
+size_t seq_delta_floats(int, int, int, int, int, size_t);
+void seq_delta(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float*, float*, float*, size_t,
+               int, int, int, int, SeqDesc, hipStream_t);
+
 // Floats of workspace of the blocked form, or 0 where the token-by-token scan is the one to run: key sizes that are no multiple
 // of 64 or above 256, rows that vector loads of four channels cannot take, and steps of few tokens a sequence.  At most `most`: longer
 // steps run in windows.
@@ -408,12 +396,17 @@ size_t seq_block_floats(int code, bool delta, const void* q, int ldq, const void
     least = blocks > 1536 ? never : blocks > 512 || dk == 64 ? 64 : 40;
   }
   if (T_ < least * B) return 0;
+  if (const size_t n = delta ? seq_delta_floats(T_, B, H, dk, dv, most) : 0) return n;
   return block_plan(T_, B, H, dk, most).slots * slot_floats(H, dk);
 }
 
 void seq_block_delta(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g,
                      const float* bpre, float* S, float* out, float* ws, size_t most, int H, int G, int dk, int dv,
                      SeqDesc d, hipStream_t st) {
+  if (seq_delta_floats(d.Ttot, d.B, H, dk, dv, most) > 0) {
+    seq_delta(code, q, ldq, k, ldk, v, ldv, g, bpre, S, out, ws, most, H, G, dk, dv, d, st);
+    return;
+  }
   const DecayArgs a = {g, nullptr, bpre, 1.f, 1.f};
   dispatch<true>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dk, dv, d, st);
 }

@@ -1,0 +1,487 @@
+// Prompts through the gated delta rule in blocks of 32 tokens, two tiles of 16.  With G_t the product of the decays from the block's first
+// token up to t (per key channel) and S the state in front of the block,
+//   u_t = beta_t (v_t - (k_t G_t)^T S - sum_{j<t} A_tj u_j),   A_tj = sum_d k_td k_jd G_td / G_jd
+//   o_t = (q_t G_t)^T S + sum_{j<=t} B_tj u_j,                 B_tj = sum_d q_td k_jd G_td / G_jd
+//   S  <- G_32 S + sum_j (k_j G_32 / G_j) u_j^T.
+// A first kernel forms, for all blocks at once, everything that does not read the state: the scaled rows, B, and - with T = (I + beta A)^-1
+// beta - the rows W = T (k G) and U = T v, so that u = U - W S and one product with the state stands between two states.  Every tile
+// of 16 is solved by itself; the second one's rows then take what the first one's u adds, A_21 = (k G)_2 (k G_16 / G)_1^T.  The
+// ratios G_t / G_j are running products of the decays themselves, never quotients, so a decay of 0 (or any other value) is what
+// it is in the token-by-token scan.  The second kernel walks a sequence's blocks with the state in registers; all products are float on
+// the float matrix units (v_mfma_f32_16x16x4_f32), whose result layout is also its operand layout.
+//
+// Measured, blocks of 16 -> of 32 tokens: three sequences of 1500, 700 and 97 tokens, 8 heads of 128 x 128: 112 -> 96 us (32 for the first
+// kernel, 64 for the walk, which is bound by the longest sequence's chain: 1.3 us a block of 32, 0.7 of them products of a wave on the
+// float matrix unit; 0.94 us a block of 16).  Error against 64 bits of outputs, blocks of 16 -> 32: 3.2 -> 2.8e-7 where decays are next
+// to 1, 1.6 -> 1.7 at 0.95, 1.25 -> 1.4 at 0.8, 1.1 -> 1.2 at 0.4.
+#include "seq_block.h"
+
+#include <type_traits>
+
+using namespace lipa;
+
+namespace {
+
+constexpr int LEN = 2 * BT;
+
+// what the first kernel leaves per (block, head): W | q G | k G_32 / G in operand order (two tiles each), G_32, B of the tiles 1-1, 2-1 and 2-2,
+// U in result order (two tiles of every 16 columns); and behind these, per (block, head) and wave, whether it met a value that is
+// infinite or NaN
+__host__ __device__ constexpr int cell_floats(int dk, int dv) { return 3 * LEN * dk + dk + 3 * BT * BT + LEN * ((dv + 15) & ~15); }
+constexpr int SEEN = 8;
+
+__device__ __forceinline__ f32x4 mfma4(const f32x4& a, const f32x4& b, f32x4 c) {      // c + a b over 16 k, lane group g holding 4g .. 4g+3
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+  return c;
+}
+
+// 512 threads, half of them a tile: token j = tid / 16 of it, and the four channels 4 x .. of every 64 (x = tid % 16).  A thread carries
+// its token's key times the decays of the tokens behind it; at token s the 16 threads of a row sum k_s and q_s against it, and lane
+// s keeps the sums.
+template <typename T, int NS>
+__global__ __launch_bounds__(512, 6) void k_delta_prep(const T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk,
+                                                    const T* __restrict__ v, int ldv, int dv, const float* __restrict__ decay,
+                                                    const float* __restrict__ beta, float* __restrict__ ws,
+                                                    unsigned* __restrict__ seen, int H, int G, Pieces pc, SeqDesc d) {
+  constexpr int DK = 64 * NS, ROWS = BT * DK;
+  __shared__ __attribute__((aligned(16))) float sg[2 * ROWS];        // decays, then k G_16 / G of the first tile
+  __shared__ __attribute__((aligned(16))) float sk[2 * ROWS];        // keys, then k G
+  __shared__ __attribute__((aligned(16))) float sq[2 * ROWS];        // queries, then q G of the second tile
+  __shared__ __attribute__((aligned(16))) float sG[2][DK];           // G_16 of the tiles
+  __shared__ __attribute__((aligned(16))) float sT[2][BT * BT];
+  __shared__ __attribute__((aligned(16))) float sA[2][BT * BT];      // A; then A_21 in place of the first
+  __shared__ float sb[LEN];
+  __shared__ int sbad[LEN];
+  const int slot = blockIdx.y, hd = blockIdx.x, tid = threadIdx.x;
+  Piece blk;
+  if (!find_piece<LEN>(d, pc, slot, blk)) return;
+  const int t0 = blk.t0, n = blk.n;
+  const int half = tid >> 8, j = (tid >> 4) & 15, x = tid & 15, tok = BT * half + j, kh = hd / (H / G);
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, g4 = lane >> 4, vtiles = (dv + 15) / 16;
+  const bool on = tok < n;
+  const size_t t = t0 + (on ? tok : 0);
+  // the wave's first tile of values is on its way from here on
+  T vraw[2][4];
+  auto load_values = [&](int vt) {
+    const int c = hd * dv + min(16 * vt + li, dv - 1);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vraw[h][e] = v[(size_t)(t0 + min(BT * h + 4 * g4 + e, n - 1)) * ldv + c];
+  };
+  if (w < vtiles) load_values(w);
+  f32x4 kj[NS], qj[NS], W[NS], Gm[NS];
+#pragma unroll
+  for (int c = 0; c < NS; ++c) {
+    const int D = 64 * c + 4 * x;
+    f32x4 g = row4(decay + (t * H + hd) * DK + D);
+    kj[c] = row4(k + t * ldk + kh * DK + D);
+    qj[c] = row4(q + t * ldq + kh * DK + D);
+    if (!on) {                                               // past the end: tokens that change nothing
+      kj[c] = qj[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      g = f32x4{1.f, 1.f, 1.f, 1.f};
+    }
+    *reinterpret_cast<f32x4*>(sg + tok * DK + D) = g;
+    *reinterpret_cast<f32x4*>(sk + tok * DK + D) = kj[c];
+    *reinterpret_cast<f32x4*>(sq + tok * DK + D) = qj[c];
+    W[c] = kj[c];
+    Gm[c] = f32x4{1.f, 1.f, 1.f, 1.f};
+  }
+  if (tid < LEN) sb[tid] = tid < n ? sigmoidf_(beta[(size_t)(t0 + tid) * H + hd]) : 0.f;
+  __syncthreads();
+  float ra = 0.f, rb = 0.f;                                  // A and B of (token x, token j)
+#pragma unroll 2
+  for (int s = 0; s < BT; ++s) {
+    float pa = 0.f, pb = 0.f;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      const int D = half * ROWS + s * DK + 64 * c + 4 * x;
+      const f32x4 g = row4(sg + D);
+      if (s <= j)
+        Gm[c] *= g;
+      else
+        W[c] *= g;
+      const f32x4 qs = row4(sq + D), ks = row4(sk + D);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        pb += qs[e] * W[c][e];
+        pa += ks[e] * W[c][e];
+      }
+    }
+    pb = row16_sum(pb);
+    pa = row16_sum(pa);
+    if (x == s) {
+      rb = pb;
+      ra = pa;
+    }
+  }
+  // From the first token on whose key, decays or beta are no numbers everything is NaN.  In front of it T and B are 0 there, and
+  // 0 x NaN is NaN: such rows of k G and T are 0, and NaN stands in B's rows, which reach the outputs of these tokens, and in the key
+  // that is written to the state - and to the second tile, all of which is behind.
+  float z = 0.f;
+#pragma unroll
+  for (int c = 0; c < NS; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) z += 0.f * (kj[c][e] * Gm[c][e]);
+  const bool bad = !(row16_sum(z) == 0.f && isfinite(sb[tok]));
+  if (x == 0) sbad[tok] = bad ? j : BT;
+  sA[half][x * BT + j] = ra;
+  __syncthreads();                                           // keys, queries and decays are read
+  int first = sbad[BT * half + x];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, 16));
+  float* cell = ws + ((size_t)slot * H + hd) * cell_floats(DK, dv);
+  float *ck = cell, *cq = ck + 2 * ROWS, *cp = cq + 2 * ROWS, *cg = cp + 2 * ROWS, *cB = cg + DK, *cU = cB + 3 * BT * BT;
+  cB[2 * half * BT * BT + x * BT + j] = x >= first ? NAN : x >= j ? rb : 0.f;
+#pragma unroll
+  for (int c = 0; c < NS; ++c) {
+    const int D = 64 * c + 4 * x;
+    *reinterpret_cast<f32x4*>(sk + tok * DK + D) = bad ? f32x4{0.f, 0.f, 0.f, 0.f} : kj[c] * Gm[c];
+    if (half == 1) *reinterpret_cast<f32x4*>(sq + j * DK + D) = qj[c] * Gm[c];
+    if (half == 0) *reinterpret_cast<f32x4*>(sg + j * DK + D) = bad ? f32x4{NAN, NAN, NAN, NAN} : W[c];
+    if (j == BT - 1) *reinterpret_cast<f32x4*>(&sG[half][D]) = Gm[c];
+  }
+  if ((tid & 255) < BT) {                                    // column x of (I + beta A)^-1 beta, row after row
+    float r[BT];
+#pragma unroll
+    for (int s = 0; s < BT; ++s) {
+      float acc = s == x ? 1.f : 0.f;
+#pragma unroll
+      for (int i = 0; i < s; ++i) acc -= sA[half][s * BT + i] * r[i];
+      r[s] = s >= first ? 0.f : sb[BT * half + s] * acc;
+      sT[half][s * BT + x] = r[s];
+    }
+  }
+  __syncthreads();
+  // the scaled rows that leave as they are
+#pragma unroll
+  for (int c = 0; c < NS; ++c) {
+    // operand order of the 16x16x4 products: [tile of 16 channels][4 channels][token][channel of the 4] for the rows, and
+    // [tile][4 tokens][channel][token of the 4] for the keys that are written to the state
+    const int D = 64 * c + 4 * x, tile = 4 * c + (x >> 2), base = half * ROWS + (tile * 64 + (x & 3) * 16 + j) * 4;
+    const f32x4 G1 = row4(&sG[0][D]), G2 = row4(&sG[1][D]);
+    *reinterpret_cast<f32x4*>(cq + base) = half == 0 ? qj[c] * Gm[c] : qj[c] * Gm[c] * G1;
+    const f32x4 P = half == 0 ? W[c] * G2 : W[c];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) cp[half * ROWS + (tile * 64 + (j >> 2) * 16 + 4 * (x & 3) + e) * 4 + (j & 3)] = bad ? NAN : P[e];
+    if (tid < 16) *reinterpret_cast<f32x4*>(cg + D) = G1 * G2;
+  }
+  if (w < 2) {                                               // A_21 and B_21: rows of the second tile against the keys of the first
+    const float* rows = (w == 0 ? sk + ROWS : sq) + li * DK + 4 * g4;
+    f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+#pragma unroll
+    for (int c = 0; c < 4 * NS; c += 2) {
+      a0 = mfma4(row4(rows + 16 * c), row4(sg + li * DK + 16 * c + 4 * g4), a0);
+      a1 = mfma4(row4(rows + 16 * c + 16), row4(sg + li * DK + 16 * c + 16 + 4 * g4), a1);
+    }
+    a0 += a1;
+    float* to = w == 0 ? sA[0] : cB + BT * BT;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) to[(4 * g4 + e) * BT + li] = a0[e];
+  }
+  __syncthreads();
+  // W and U, a wave a tile of 16 columns at a time: y1 = T_1 x1, y2 = T_2 (x2 - A_21 y1)
+  const f32x4 T1 = row4(&sT[0][li * BT + 4 * g4]), T2 = row4(&sT[1][li * BT + 4 * g4]), X = -row4(&sA[0][li * BT + 4 * g4]);
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  for (int kt = w; kt < 4 * NS; kt += 8) {
+    f32x4 x1, x2;
+    const float G1 = sG[0][16 * kt + li];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x1[e] = sk[(4 * g4 + e) * DK + 16 * kt + li];
+      x2[e] = sk[ROWS + (4 * g4 + e) * DK + 16 * kt + li] * G1;
+    }
+    const f32x4 y1 = mfma4(T1, x1, zero), y2 = mfma4(T2, mfma4(X, y1, x2), zero);
+    float* to = ck + (kt * 64 + (li >> 2) * 16 + 4 * g4) * 4 + (li & 3);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      to[4 * e] = y1[e];
+      to[ROWS + 4 * e] = y2[e];
+    }
+  }
+  bool odd = false;
+  for (int vt = w; vt < vtiles; vt += 8) {
+    if (vt != w) load_values(vt);
+    f32x4 x1, x2;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = 16 * vt + li < dv;
+      x1[e] = in && 4 * g4 + e < n ? (float)vraw[0][e] : 0.f;
+      x2[e] = in && BT + 4 * g4 + e < n ? (float)vraw[1][e] : 0.f;
+      odd |= !isfinite(x1[e]) || !isfinite(x2[e]);           // (the walk makes up for what counts as 0 here)
+      x1[e] = isfinite(x1[e]) ? x1[e] : 0.f;
+      x2[e] = isfinite(x2[e]) ? x2[e] : 0.f;
+    }
+    const f32x4 y1 = mfma4(T1, x1, zero), y2 = mfma4(T2, mfma4(X, y1, x2), zero);
+    *reinterpret_cast<f32x4*>(cU + (vt * 64 + lane) * 4) = y1;
+    *reinterpret_cast<f32x4*>(cU + ((vtiles + vt) * 64 + lane) * 4) = y2;
+  }
+  odd = __any(odd);
+  if (lane == 0) seen[((size_t)slot * H + hd) * SEEN + w] = odd;
+}
+
+// A block owns 16 value columns of one (sequence, head) and walks its blocks of tokens, a window between two barriers for each.  Four waves
+// hold a quarter of the state's rows each, in registers in operand layout: they finish u from the shares of the key products, update
+// their rows, leave these in LDS and form their shares of the next block's key products.  Four more, one on every SIMD beside them, take
+// the state of the window before from LDS for the query products and finish the outputs of the block before that.  One wave alone
+// on a SIMD leaves the float matrix unit idle in every barrier and round trip (3000 cycles a block for 1630 of products).
+template <typename T, int NS>
+__global__ __launch_bounds__(512, 2) void k_delta_walk(const float* __restrict__ ws, const unsigned* __restrict__ seen,
+                                                       const T* __restrict__ v, int ldv, float* __restrict__ S,
+                                                       float* __restrict__ out, int H, int dv, Pieces pc, SeqDesc d) {
+  constexpr int DK = 64 * NS, ROWS = BT * DK;
+  __shared__ __attribute__((aligned(16))) f32x4 rk[2][4][2][64];     // shares of the key products, of the query products
+  __shared__ __attribute__((aligned(16))) f32x4 rq[2][4][2][64];
+  __shared__ __attribute__((aligned(16))) f32x4 su[2][2][64];        // u
+  __shared__ __attribute__((aligned(16))) f32x4 ss[2][4][NS][64];    // the state
+  const int s = blockIdx.x / H, hd = blockIdx.x % H, tid = threadIdx.x;
+  if (d.live && !d.live[s]) return;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), w = wv & 3, lane = tid & 63, g = lane >> 4, col = blockIdx.y * 16 + (lane & 15);
+  const bool colok = col < dv;
+  int slot;
+  const int t0 = d.seq_off[s] + pc.first * LEN, t1 = d.seq_off[s + 1], steps = own_pieces<LEN>(d, pc, s, slot), vtiles = (dv + 15) / 16;
+  if (steps <= 0) return;
+  const int CELL = cell_floats(DK, dv);
+  const float* cell = ws + ((size_t)slot * H + hd) * CELL;
+  const size_t step = (size_t)H * CELL;
+  const T* vp = v + (size_t)t0 * ldv + (size_t)hd * dv;
+  const unsigned vcol = colok ? col : 0, rows = (NS * w * 64 + lane) * 4;
+  // A value that is infinite or NaN: it counts as 0 in the products, its column of the state is NaN, and its column of the
+  // outputs from its token on.  (A sequence without such values runs the loops that do not look at them.)
+  auto number = [&](int i, int h, int e) {
+    const int tt = i * LEN + BT * h + 4 * g + e;
+    return t0 + tt >= t1 || isfinite((float)vp[(size_t)min(tt, t1 - t0 - 1) * ldv + vcol]);
+  };
+  u32x4 any = {0u, 0u, 0u, 0u};
+  for (int i = lane; i < 2 * steps; i += 64) any |= reinterpret_cast<const u32x4*>(seen)[(((size_t)slot + i / 2) * H + hd) * 2 + (i & 1)];
+  const bool some = __any((any[0] | any[1]) | (any[2] | any[3]));
+  const int half = w & 1;                                   // the tile whose outputs a wave finishes, every other block
+  if (wv < 4) {
+    __builtin_amdgcn_s_setprio(3);                          // (the other wave's products fill the gaps)
+    float* Sp = S + (((size_t)d.slots[s] * H + hd) * dv + (colok ? col : 0)) * DK + 16 * NS * w + 4 * g;
+    const bool old = (pc.first > 0 || d.pos0[s] > 0) && colok;
+    f32x4 St[NS];
+    struct In {
+      f32x4 k[2][NS], p[2][NS], g[NS], u[2];
+    } in[2];
+    auto load_k = [&](int i, In& x) {
+      const float* c0 = cell + (size_t)i * step;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < NS; ++c) x.k[h][c] = row4(c0 + h * ROWS + rows + c * 256);
+    };
+    auto load = [&](int i, In& x) {
+      const float* c0 = cell + (size_t)i * step;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) x.u[h] = row4(c0 + 6 * ROWS + DK + 3 * BT * BT + ((h * vtiles + blockIdx.y) * 64 + lane) * 4);
+#pragma unroll
+      for (int c = 0; c < NS; ++c) x.g[c] = row4(c0 + 6 * ROWS + 16 * (NS * w + c) + (unsigned)(4 * g));
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < NS; ++c) x.p[h][c] = row4(c0 + (4 + h) * ROWS + rows + c * 256);
+    };
+    auto keys = [&](int i, const In& x) {                   // shares of block i's key products, with the state in front of it
+      f32x4 xk[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int c = 0; c < NS; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) xk[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[h][c][e], St[c][e], xk[h], 0, 0, 0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) rk[i & 1][w][h][lane] = xk[h];
+    };
+    // block i between its barrier and the next: u, the state behind it, the next block's key products.  An operand's place takes the one
+    // two blocks later as soon as it is read
+    auto window = [&](int i, In& x, In& next, auto odd) {
+      f32x4 r[4][2], u[2];
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) r[a][h] = rk[i & 1][a][h][lane];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) u[h] = x.u[h] - ((r[0][h] + r[1][h]) + (r[2][h] + r[3][h]));
+      su[i & 1][half][lane] = half ? u[1] : u[0];           // (two waves write the same)
+      if constexpr (odd)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) u[h][e] = number(i, h, e) ? u[h][e] : NAN;
+      f32x4 add[NS] = {};                                   // (added up by itself: fewer sums rounded at the state's size)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int c = 0; c < NS; ++c) add[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[h][c][e], u[h][e], add[c], 0, 0, 0);
+#pragma unroll
+      for (int c = 0; c < NS; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) St[c][e] = fmaf(St[c][e], x.g[c][e], add[c][e]);
+      load(min(i + 2, steps - 1), x);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < NS; ++c) ss[(i + 1) & 1][w][c][lane] = St[c];
+      keys(i + 1, next);                                    // (past the last block: nobody reads them)
+      load_k(min(i + 3, steps - 1), next);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    load_k(0, in[0]);
+    load(0, in[0]);
+    load_k(min(1, steps - 1), in[1]);
+    load(min(1, steps - 1), in[1]);
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      St[c] = old ? row4(Sp + 16 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
+      ss[0][w][c][lane] = St[c];
+    }
+    keys(0, in[0]);
+    load_k(min(2, steps - 1), in[0]);
+    auto walk = [&](auto odd) {
+      int i = 0;
+      for (; i + 2 <= steps; i += 2) {
+        __syncthreads();
+        window(i, in[0], in[1], odd);
+        __syncthreads();
+        window(i + 1, in[1], in[0], odd);
+      }
+      if (i < steps) {
+        __syncthreads();
+        window(i, in[0], in[1], odd);
+      }
+      __syncthreads();                                      // (the outputs of the last block)
+    };
+    if (some)
+      walk(std::true_type{});
+    else
+      walk(std::false_type{});
+    if (colok)
+#pragma unroll
+      for (int c = 0; c < NS; ++c) *reinterpret_cast<f32x4*>(Sp + 16 * c) = St[c];
+    return;
+  }
+  struct In {
+    f32x4 q[2][NS], b[2];
+  } in[2];
+  auto load = [&](int i, In& x) {
+    const float* c0 = cell + (size_t)i * step;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int c = 0; c < NS; ++c) x.q[h][c] = row4(c0 + (2 + h) * ROWS + rows + c * 256);
+      x.b[h] = row4(c0 + 6 * ROWS + DK + (half ? 1 + h : 0) * BT * BT + (lane & 15) * BT + 4 * g);
+    }
+  };
+  f32x4 bo[2];                                              // B of the block before
+  int oo[4];                                                // (a store that has no place goes past the end of its window and is dropped)
+#pragma unroll
+  for (int e = 0; e < 4; ++e) oo[e] = colok ? (((BT * half + 4 * g + e) * H + hd) * dv + col) * 4 : -4;
+  auto outputs = [&](int i, auto odd) {
+    const auto& r = rq[i & 1];
+    const f32x4 u0 = su[i & 1][0][lane], u1 = su[i & 1][1][lane];
+    f32x4 o = (r[0][half][lane] + r[1][half][lane]) + (r[2][half][lane] + r[3][half][lane]);
+    o = mfma4(bo[0], u0, o);
+    if (half) o = mfma4(bo[1], u1, o);
+    if constexpr (odd) {
+      int first = LEN;
+#pragma unroll
+      for (int h = 1; h >= 0; --h)
+#pragma unroll
+        for (int e = 3; e >= 0; --e) first = number(i, h, e) ? first : BT * h + 4 * g + e;
+      first = min(first, __shfl_xor(first, 16, 64));
+      first = min(first, __shfl_xor(first, 32, 64));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = BT * half + 4 * g + e >= first ? NAN : o[e];
+    }
+    const int b0 = t0 + i * LEN;
+    const auto win = __builtin_amdgcn_make_buffer_rsrc(out + (size_t)b0 * H * dv, 0, min(LEN, t1 - b0) * H * dv * 4, 0x00020000);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[e]), win, oo[e], 0, 0);
+  };
+  auto window = [&](int i, In& x, auto odd) {
+    f32x4 xq[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, St[NS];
+#pragma unroll
+    for (int c = 0; c < NS; ++c) St[c] = ss[i & 1][w][c][lane];
+#pragma unroll
+    for (int c = 0; c < NS; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) xq[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[h][c][e], St[c][e], xq[h], 0, 0, 0);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) rq[i & 1][w][h][lane] = xq[h];
+    if (i > 0 && w >> 1 == (i & 1)) outputs(i - 1, odd);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) bo[h] = x.b[h];
+    load(min(i + 2, steps - 1), x);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  load(0, in[0]);
+  load(min(1, steps - 1), in[1]);
+  auto walk = [&](auto odd) {
+    int i = 0;
+    for (; i + 2 <= steps; i += 2) {
+      __syncthreads();
+      window(i, in[0], odd);
+      __syncthreads();
+      window(i + 1, in[1], odd);
+    }
+    if (i < steps) {
+      __syncthreads();
+      window(i, in[0], odd);
+    }
+    __syncthreads();
+    if (w >> 1 == (steps & 1)) outputs(steps - 1, odd);
+  };
+  if (some)
+    walk(std::true_type{});
+  else
+    walk(std::false_type{});
+}
+
+// floats of a slot; 0.23 us a token at least in the token-by-token form
+size_t slot_floats(int H, int dk, int dv) { return (size_t)H * (cell_floats(dk, dv) + SEEN); }
+PiecePlan delta_plan(int T_, int B, int H, int dk, int dv, size_t most) {
+  return plan_pieces(T_, B, LEN, slot_floats(H, dk, dv), most, 0.23f);
+}
+
+template <typename T, int NS>
+void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g, const float* beta, float* S,
+            float* out, float* ws, size_t most, int H, int G, int dv, const SeqDesc& d, hipStream_t st) {
+  const PiecePlan plan = delta_plan(d.Ttot, d.B, H, 64 * NS, dv, most);
+  unsigned* seen = reinterpret_cast<unsigned*>(ws + plan.slots * H * cell_floats(64 * NS, dv));
+  for (int w = 0; w < plan.windows; ++w) {
+    const Pieces pc = {LEN, w * plan.count, plan.count};
+    hipLaunchKernelGGL((k_delta_prep<T, NS>), dim3(H, (unsigned)plan.slots), dim3(512), 0, st, (const T*)q, ldq, (const T*)k, ldk,
+                       (const T*)v, ldv, dv, g, beta, ws, seen, H, G, pc, d);
+    hipLaunchKernelGGL((k_delta_walk<T, NS>), dim3(d.B * H, (dv + 15) / 16), dim3(512), 0, st, ws, seen, (const T*)v, ldv, S, out, H,
+                       dv, pc, d);
+  }
+  LIPA_CHECK_LAUNCH();
+}
+
+}  // namespace
+
+// Floats of workspace for at most `most` (longer steps run in windows), or 0 where blocks of 16 (seq_block.hip) are not slower or there is
+// no room.  Two tiles between two barriers pay where one block of threads a CU walks a long sequence; the first kernel is the longer
+// one, and blocks of 16 fit a CU twice.  us, 16 -> 32 tokens, heads of 128 x 128: 8 heads x 1000 tokens 75 -> 61, x 4000 262 -> 208, x 200 24.5
+// -> 25.4, 1500 + 700 + 97 112 -> 96, 4 x 2000 (256 blocks of threads) 181 -> 160, 12 x 700 (768) 172 -> 183; 4 heads x 9000 540 -> 425, 12 x 700
+// (384) 104 -> 113; keys of 64, 8 x 64 columns, 1000 + 500 59 -> 44; of 192 97 -> 95, of 256 146 -> 151.
+size_t seq_delta_floats(int T_, int B, int H, int dk, int dv, size_t most) {
+  if (dk > 128 || T_ < 300l * B || (long)B * H * ((dv + 15) / 16) > 256) return 0;
+  return delta_plan(T_, B, H, dk, dv, most).slots * slot_floats(H, dk, dv);
+}
+
+void seq_delta(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g, const float* bpre, float* S,
+               float* out, float* ws, size_t most, int H, int G, int dk, int dv, SeqDesc d, hipStream_t st) {
+  SEQ_DISPATCH_T(code, {
+    if (dk == 64)
+      launch<T, 1>(q, ldq, k, ldk, v, ldv, g, bpre, S, out, ws, most, H, G, dv, d, st);
+    else
+      launch<T, 2>(q, ldq, k, ldk, v, ldv, g, bpre, S, out, ws, most, H, G, dv, d, st);
+  });
+}

@@ -288,6 +288,54 @@ def test_delta_token_that_is_no_number(name, value, t, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lens,starts", [([320], [0]), ([351, 1, 640, 209], [0, 3, 0, 9]), ([305, 336], [7, 0]), ([592, 49], [0, 0])])
+@pytest.mark.parametrize("H,G,dk,dv,dt", [(3, 1, 64, 36, torch.float32), (2, 2, 128, 20, torch.bfloat16), (4, 2, 128, 64, torch.float32),
+                                          (1, 1, 64, 4, torch.bfloat16)])
+def test_delta_blocks_of_two_tiles(lens, starts, H, G, dk, dv, dt):
+    """Long sequences: a last block of one token, one tile, a tile and a token, all 32; a sequence that does not run."""
+    g = torch.Generator().manual_seed(dk + dv + len(lens))
+    T, live = sum(lens), [int(b != 3) for b in range(len(lens))]
+    P = torch.randn(T, 2 * G * dk + H * dv, generator=g)
+    for j in (0, 1):
+        x = P[:, j * G * dk:(j + 1) * G * dk].view(T, G, dk)
+        x.copy_(torch.nn.functional.normalize(x, dim=-1))
+    P, decay, beta = P.to(dt), torch.rand(T, H * dk, generator=g) ** 0.2, 2 * torch.randn(T, H, generator=g)
+    decay[::7, ::3] = 0.0                               # channels that forget everything
+    S0 = torch.randn(len(lens), H, dv, dk, generator=g)
+    tok = torch.cat([torch.full((n,), bool(on)) for n, on in zip(lens, live)])
+    res = []
+    for dev in ("cpu", "cuda"):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, starts, dev, live)
+        st["S"].copy_(S0)
+        p = P.to(dev)
+        o = R.gated_delta_scan(p[:, :G * dk], p[:, G * dk:2 * G * dk], p[:, 2 * G * dk:], decay.to(dev), beta.to(dev), st["S"], H,
+                               G, sb)
+        res.append((o.cpu()[tok], st["S"]))
+    _close(res[1], res[0], ("o", "state"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,value", [("v", float("inf")), ("v", float("nan")), ("k", float("-inf")), ("q", float("nan")),
+                                        ("g", float("nan")), ("g", float("inf")), ("b", float("nan"))])
+@pytest.mark.parametrize("t", [310, 325, 326, 341, 342, 650, 669])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_delta_token_that_is_no_number_in_two_tiles(name, value, t, dt):
+    """On both sides of a tile (326) and of a block (310, 342), in a block of one tile (650) and at the end."""
+    lens, H, dk, dv = [310, 360], 2, 128, 20
+    g = torch.Generator().manual_seed(t)
+    T = sum(lens)
+    inputs = {n: torch.nn.functional.normalize(torch.randn(T, dk, generator=g), dim=-1).to(dt).cuda() for n in "qk"}
+    inputs |= {"v": torch.randn(T, H * dv, generator=g).to(dt).cuda(), "g": (torch.rand(T, H * dk, generator=g) ** 0.2).cuda(),
+               "b": torch.randn(T, H, generator=g).cuda()}
+
+    def run(x):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, [3, 0], "cuda")
+        st["S"].fill_(0.5)
+        return (R.gated_delta_scan(x["q"], x["k"], x["v"], x["g"], x["b"], st["S"], H, 1, sb),)
+    _planted(run, inputs, name, t, 1, value, lens)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("name,value", [("v", float("-inf")), ("v", float("nan")), ("k", float("inf")), ("q", float("nan")),
                                         ("z", float("nan"))])
 @pytest.mark.parametrize("t", [53, 68, 95, 96, 110])
