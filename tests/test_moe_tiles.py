@@ -42,6 +42,55 @@ def test_expert_tiles(T, top, E, F, W, kind, act, weight_input, gate):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,E,F,W", [(4000, 8, 256, 128), (4100, 8, 192, 256), (3900, 6, 320, 64), (2200, 4, 640, 192), (1900, 24, 1216, 192)])
+def test_expert_tiles_of_many_rows(T, E, F, W):
+    """More tiles than CUs: tiles of 128 columns of the activation, the last one half empty at 1216, and of 64 where that pads too much."""
+    g = torch.Generator().manual_seed(T)
+    top = 3
+    h = torch.randn(T, W, generator=g).bfloat16()
+    gu, d = (torch.randn(E, 2, F, W, generator=g) * W ** -0.5).bfloat16(), (torch.randn(E, W, F, generator=g) * F ** -0.5).bfloat16()
+    idx = torch.rand(T, E, generator=g).argsort(1)[:, :top].int().contiguous()
+    w = torch.rand(T, top, generator=g)
+    assert (T * top // 128 + E) * -(-F // 64) > 256 and M.expert_tiles_win(T * top, E, F, W)
+    got = M.moe_glu_experts(*(t.cuda() for t in (h, gu, d, idx, w)), 7.0, None, False, act="silu")
+    want = M.moe_glu_experts(h.float(), gu.float(), d.float(), idx, w, 7.0, None, False, act="silu")
+    assert (got.cpu() - want).norm() <= 2.0 ** -8 * want.norm()         # (rounded to bf16 twice, 2^-9 each)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,T", [(64, 300), (65, 300), (130, 77)])
+def test_tiles_of_many_experts(E, T):
+    """A tile's expert is found 64 experts at a time; most experts of the last call have no pair."""
+    g = torch.Generator().manual_seed(E)
+    F, W, top = 64, 128, 2
+    h = torch.randn(T, W, generator=g).bfloat16()
+    gu, d = (torch.randn(E, 2, F, W, generator=g) * W ** -0.5).bfloat16(), (torch.randn(E, W, F, generator=g) * F ** -0.5).bfloat16()
+    idx = torch.rand(T, E, generator=g).argsort(1)[:, :top].int().contiguous()
+    idx[:, 0] = E - 1
+    w = torch.rand(T, top, generator=g)
+    got = M.moe_glu_experts(*(t.cuda() for t in (h, gu, d, idx, w)), 7.0, None, False, act="silu")
+    want = M.moe_glu_experts(h.float(), gu.float(), d.float(), idx, w, 7.0, None, False, act="silu")
+    assert (got.cpu() - want).norm() <= 2.0 ** -8 * want.norm()         # (rounded to bf16 twice, 2^-9 each)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu", "clipped"])
+def test_tiles_activation_of_extreme_values(act):
+    """Gates from -3e38 to 3e38, one a token, each beside an up product of 1; infinite and NaN ones reach no other token."""
+    gates = [-3e38, -1e4, -200.0, -90.0, -80.0, -20.0, -1.0, -1e-3, 0.0, 1e-3, 1.0, 20.0, 90.0, 1e4, 3e38, float("inf"), -float("inf"), float("nan")]
+    E, F, W = 1, 64, 64
+    h = torch.zeros(len(gates), W)
+    h[:, 0], h[:, 1] = torch.tensor(gates), 1.0
+    gu, d = torch.zeros(E, 2, F, W), torch.eye(W)[None].contiguous()
+    gu[0, 0, :, 0], gu[0, 1, :, 1] = 1.0, 1.0
+    h, gu, d = (t.bfloat16() for t in (h, gu, d))
+    idx, w = torch.zeros(len(gates), 1, dtype=torch.int32), torch.ones(len(gates), 1)
+    got = M.moe_glu_experts(*(t.cuda() for t in (h, gu, d, idx, w)), 7.0, None, False, act=act).cpu()[:15]
+    want = M.moe_glu_experts(h.float(), gu.float(), d.float(), idx, w, 7.0, None, False, act=act)[:15]
+    torch.testing.assert_close(got, want, rtol=2.0 ** -8, atol=1e-35)   # (one rounding to bf16; a product below 2^-126 may be 0)
+
+
+@pytest.mark.gpu
 def test_many_rows_of_large_experts():
     """A call past the tiles' range: the vendor's products, the same sums."""
     g = torch.Generator().manual_seed(0)
