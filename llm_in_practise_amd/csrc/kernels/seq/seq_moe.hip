@@ -12,30 +12,54 @@ using namespace lipa;
 
 constexpr int RPL = 4;   // router outputs per lane: experts + identity experts <= 64 * RPL
 
+// the value of lane ^ M inside rows of 16, by a move between lanes where one does it: a trip through LDS takes ten times as long,
+// and routing is one chain of them
+template <int M>
+__device__ __forceinline__ int lane_xor(int v) {
+  if constexpr (M == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);          // quad_perm [1, 0, 3, 2]
+  else if constexpr (M == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);     // quad_perm [2, 3, 0, 1]
+  else if constexpr (M == 4)                                                               // row_shl:4, row_shr:4 in lanes 4-7, 12-15
+    return __builtin_amdgcn_update_dpp(__builtin_amdgcn_mov_dpp(v, 0x104, 0xF, 0xF, true), v, 0x114, 0xF, 0xA, false);
+  else if constexpr (M == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);    // row_ror:8
+  else return __shfl_xor(v, M, 64);
+}
+template <int M>
+__device__ __forceinline__ float lane_xor(float v) {
+  return __int_as_float(lane_xor<M>(__float_as_int(v)));
+}
 // (value, index) maximum over GW lanes; ties go to the lower index
 template <int GW>
 __device__ __forceinline__ void group_argmax(float& v, int& i) {
-#pragma unroll
-  for (int o = GW / 2; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o, GW);
-    const int oi = __shfl_xor(i, o, GW);
-    if (ov > v || (ov == v && oi < i)) {
-      v = ov;
-      i = oi;
-    }
+  const float ov = lane_xor<GW / 2>(v);
+  const int oi = lane_xor<GW / 2>(i);
+  if (ov > v || (ov == v && oi < i)) {
+    v = ov;
+    i = oi;
   }
+  if constexpr (GW > 2) group_argmax<GW / 2>(v, i);
 }
 template <int GW>
 __device__ __forceinline__ float group_max(float v) {
-#pragma unroll
-  for (int o = GW / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, GW));
+  v = fmaxf(v, lane_xor<GW / 2>(v));
+  if constexpr (GW > 2) v = group_max<GW / 2>(v);
   return v;
 }
 template <int GW>
 __device__ __forceinline__ float group_add(float v) {
-#pragma unroll
-  for (int o = GW / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, GW);
+  v += lane_xor<GW / 2>(v);
+  if constexpr (GW > 2) v = group_add<GW / 2>(v);
   return v;
+}
+// v[i] and v[i + HALF] of lanes `HALF` apart: a lane keeps the sum of the one that its bit names
+template <int HALF>
+__device__ __forceinline__ void fold(float (&v)[64], int lane) {
+  const bool up = lane & HALF;
+#pragma unroll
+  for (int i = 0; i < HALF; ++i) {
+    const float keep = up ? v[i + HALF] : v[i], send = up ? v[i] : v[i + HALF];
+    v[i] = keep + lane_xor<HALF>(send);
+  }
+  if constexpr (HALF > 1) fold<HALF / 2>(v, lane);
 }
 
 // GW lanes route one token from its n router logits, RP a lane (z[i]: output lane + GW i).  s = softmax(z) over all n outputs;
@@ -259,7 +283,8 @@ __global__ __launch_bounds__(64 * NW) void k_route_fused(const T* __restrict__ h
 // The same for prompts and up to 16 outputs: a block takes four tokens, a wave a quarter of their columns, so that a router row
 // read from the cache serves four tokens; the 4 x 16 sums over a wave's lanes leave (token, output) in lane 16 token + output, and
 // after the four waves' sums meet in LDS each 16 lanes of the first route their token.  8000 tokens of width 2048, 8 outputs: 41
-// -> 18 us (a block per token read the whole router from L2, 0.6 GB in all, and routed with 64 lanes).
+// -> 17 us (a block per token read the whole router from L2, 0.6 GB in all, and routed with 64 lanes); moves between lanes through LDS instead
+// of between registers 19.  Bound by issue, 8 waves a SIMD of 800 instructions; 6 blocks a CU spill and take 20 us, 8 32.
 template <typename T, int NG>
 __global__ __launch_bounds__(256) void k_route_rows(const T* __restrict__ h, int ldh, const float* __restrict__ router,
                                                     const float* __restrict__ corr, int* __restrict__ idx,
@@ -286,15 +311,7 @@ __global__ __launch_bounds__(256) void k_route_rows(const T* __restrict__ h, int
   for (int i = 0; i < 32; ++i) v[i] = swap32_add(v[i], v[i + 32]);
 #pragma unroll
   for (int i = 0; i < 16; ++i) v[i] = swap16_add(v[i], v[i + 16]);
-#pragma unroll
-  for (int half = 8; half > 0; half >>= 1) {
-    const bool up = lane & half;
-#pragma unroll
-    for (int i = 0; i < half; ++i) {
-      const float keep_ = up ? v[i + half] : v[i], send = up ? v[i] : v[i + half];
-      v[i] = keep_ + __shfl_xor(send, half, 64);
-    }
-  }
+  fold<8>(v, lane);
   part[w][lane] = v[0];
   __syncthreads();
   const int t = t0 + (lane >> 4), o = lane & 15;
