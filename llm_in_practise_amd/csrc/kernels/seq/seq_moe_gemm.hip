@@ -3,8 +3,8 @@
 // gathers its rows of the input as it loads them and ends in the gated activation, so neither the gathered input nor the gate
 // and up products ever stand in memory.
 //
-// 8000 tokens of width 2048, 8 experts of 384, top 2 (75 GFLOP): 638 -> 165 us with routing and the weighted sum: order 14, first
-// products 61 (820 TFLOP/s), second 42 (600), sum 27, routing 18.  100 tokens: 533 -> 41 us.  The sort, the host's read of the run lengths
+// 8000 tokens of width 2048, 8 experts of 384, top 2 (75 GFLOP): 638 -> 155 us with routing and the weighted sum: order 5.5, first
+// products 61 (820 TFLOP/s), second 42 (600), sum 27, routing 17.  100 tokens: 533 -> 40 us.  The sort, the host's read of the run lengths
 // and a vendor product pair, an activation and their launch gaps per expert took 500 us at any number of tokens.
 #include "seq_common.h"
 
@@ -21,51 +21,82 @@ typedef __amdgpu_buffer_rsrc_t rsrc;
 
 constexpr int PT = 1024;                        // threads of the ordering kernel
 
-// One block per expert e: its place in the order is the number of pairs of lower experts; its pairs keep their order.
-// perm: pair at a place; pos: place of a pair (0 for pairs of no expert); offs [E + 1].
-__global__ __launch_bounds__(PT) void k_moe_order(const int* __restrict__ idx, int P, int E, int* __restrict__ offs,
+// Blocks (e, part): expert e's place in the order is the number of pairs of lower experts, that of a part of its pairs behind the
+// ones in front of it; pairs keep their order.  perm: pair at a place; pos: place of a pair (0 for pairs of no expert); offs [E + 1].
+// Every block counts over all pairs, four neighbouring ones a load and four loads on their way, then places its part: parts of 4096
+// pairs, one turn of the block, as long as there are 256 blocks or fewer.  Bound by latency: one block an expert that read turn after
+// turn, twice, took 14 us for 16000 pairs of 8 experts; this 5.5 (24000 pairs 7, 200 4).
+typedef int int4u __attribute__((ext_vector_type(4), aligned(4)));
+constexpr int TURN = 4 * PT;
+__global__ __launch_bounds__(PT) void k_moe_order(const int* __restrict__ idx, int P, int E, int turns, int* __restrict__ offs,
                                                   int* __restrict__ perm, long* __restrict__ pos) {
-  __shared__ int wsum[PT / 64], wlow[PT / 64];
-  const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  int low = 0, eq = 0;
-  for (int p = 4 * tid; p < P; p += 4 * PT)
+  __shared__ int wsum[PT / 64], wlow[PT / 64], wall[PT / 64];
+  const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, first = blockIdx.y * turns, all = (P + TURN - 1) / TURN;
+  auto load = [&](int turn) {
+    const int p = turn * TURN + 4 * tid;
+    int4u v = {-1, -1, -1, -1};
+    if (p + 4 <= P) {
+      v = *reinterpret_cast<const int4u*>(idx + p);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        if (p + i < P) v[i] = idx[p + i];
+    }
+    return v;
+  };
+  const int4u mine = load(first);
+  int low = 0, before = 0, eq = 0;                     // (eq: of the block that writes the last place)
+  auto count = [&](const int4u& v, bool ahead) {
+    int n = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int v = p + i < P ? idx[p + i] : -1;
-      low += v >= 0 && v < e;
-      eq += v == e;
+      low += (unsigned)v[i] < (unsigned)e;
+      n += v[i] == e;
     }
+    eq += n;
+    before += ahead ? n : 0;
+  };
+  for (int t = 0; t < all - 1; t += 4) {               // all turns but the block's own first one
+    int4u v[4];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    low += __shfl_xor(low, o, 64);
-    eq += __shfl_xor(eq, o, 64);
+    for (int j = 0; j < 4; ++j) v[j] = load(t + j + (t + j >= first));     // (turns past the last one load nothing)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) count(v[j], t + j < first);
   }
-  if (lane == 0) {
-    wlow[w] = low;
-    wsum[w] = eq;
-  }
+  count(mine, false);
+  auto total = [&](int v, int* part) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (lane == 0) part[w] = v;
+  };
+  const bool last = e == E - 1 && blockIdx.y == 0;
+  total(low, wlow);
+  if (first > 0) total(before, wsum);
+  if (last) total(eq, wall);
   __syncthreads();
-  int at = 0, all = 0;
+  int at = 0, ahead0 = 0, count0 = 0;
 #pragma unroll
   for (int i = 0; i < PT / 64; ++i) {
     at += wlow[i];
-    all += wsum[i];
+    ahead0 += first > 0 ? wsum[i] : 0;
+    count0 += last ? wall[i] : 0;
   }
-  if (tid == 0) {
+  if (tid == 0 && blockIdx.y == 0) {
     offs[e] = at;
-    if (e == E - 1) offs[E] = at + all;
+    if (last) offs[E] = at + count0;
   }
-  for (int p0 = 0; p0 < P; p0 += 4 * PT) {            // four neighbouring pairs a thread
-    const int p = p0 + 4 * tid;
-    int v[4], ahead = 0, count = 0;
+  at += ahead0;
+  for (int t = first; t < min(first + turns, all); ++t) {
+    const int4u v = t == first ? mine : load(t);
+    const int p = t * TURN + 4 * tid;
+    int ahead = 0, count = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      v[i] = p + i < P ? idx[p + i] : -1;
       const unsigned long long m = __ballot(v[i] == e);
       ahead += __popcll(m & ((1ull << lane) - 1));
       count += __popcll(m);
     }
-    __syncthreads();                                  // the last turn's counts are read
+    __syncthreads();                                  // the last counts are read
     if (lane == 0) wsum[w] = count;
     __syncthreads();
     int turn = 0;
@@ -324,7 +355,8 @@ void seq_moe_tiles(const void* h, const void* wgu, const void* wd, const int* id
   if (P == 0) return;
   const Rows r = {offs, perm, E, P, top};
   const int mt = P / BM + E;
-  hipLaunchKernelGGL(k_moe_order, dim3(E), dim3(PT), 0, st, idx, P, E, offs, perm, pos);
+  const int all = (P + TURN - 1) / TURN, parts = min(all, max(1, 256 / E)), turns = (all + parts - 1) / parts;
+  hipLaunchKernelGGL(k_moe_order, dim3(E, (all + turns - 1) / turns), dim3(PT), 0, st, idx, P, E, turns, offs, perm, pos);
   // Where every CU gets one tile of 128 x 128 at most, three stages; where there are more, tiles twice as wide unless they would pad
   // the columns by more than a twentieth, and two blocks a CU otherwise.  us, 2 x 128 two stages / 2 x 128 three / 4 x 256 three, with the
   // second products, routing and sum: 8 experts, width 2048, F 384, tokens 100 51 / 42 / 47, 1500 (186 blocks) 61 / 52 / 57, 3000 (324)

@@ -58,6 +58,26 @@ def test_expert_tiles_of_many_rows(T, E, F, W):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("E", [1, 7, 130, 300])
+@pytest.mark.parametrize("pairs", [1, 4095, 4096, 4097, 12291, 36867])
+def test_order_of_pairs(E, pairs):
+    """Around the turns of 4096 pairs, several to a block where experts are many; identity experts between the others; ids that start at
+    an address of 4 bytes more than a multiple of 16."""
+    g = torch.Generator().manual_seed(E + pairs)
+    F, W = 64, 64
+    h = torch.randn(pairs, W, generator=g).bfloat16()
+    gu, d = (torch.randn(E, 2, F, W, generator=g) * W ** -0.5).bfloat16(), (torch.randn(E, W, F, generator=g) * F ** -0.5).bfloat16()
+    idx, w = torch.randint(0, E + 2, (pairs, 1), generator=g).int(), torch.rand(pairs, 1, generator=g)
+    far = torch.cat([idx.new_zeros(1, 1), idx]).cuda()[1:]
+    got = M.moe_glu_experts(h.cuda(), gu.cuda(), d.cuda(), far, w.cuda(), 7.0, None, False, act="silu")
+    want = M.moe_glu_experts(h.float(), gu.float(), d.float(), idx, w, 7.0, None, False, act="silu")
+    assert M.expert_tiles_win(pairs, E, F, W)
+    # every token's row by itself: rounded to bf16 twice, 2^-9 each
+    assert ((got.cpu() - want).norm(dim=1) <= 2.0 ** -7 * want.norm(dim=1) + 1e-6).all()
+    assert (got.cpu() - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("E,T", [(64, 300), (65, 300), (130, 77)])
 def test_tiles_of_many_experts(E, T):
     """A tile's expert is found 64 experts at a time; most experts of the last call have no pair."""
