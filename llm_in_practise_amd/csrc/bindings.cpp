@@ -41,7 +41,8 @@ bool lt_gemm(bool, bool, long, long, long, const void*, long, const void*, long,
              long, long, void*, size_t, hipStream_t, bool);
 void lt_reset();
 void launch_sum_slices(const void*, void*, int, size_t, size_t, hipStream_t);
-void launch_gemm_skinny(const void*, int, const void*, const void*, void*, int, int, int, bool, hipStream_t);
+bool skinny_norms(int, int, bool);
+void launch_gemm_skinny(const void*, int, const void*, const void*, void*, int, int, int, bool, const void*, float, hipStream_t);
 bool w4mm_supported(int, int, int, int);
 bool w4g_supported(int, int, int, int);
 int w4g_splits(int, int, int);
@@ -542,7 +543,18 @@ static void check_skinny(const Tensor& x, const Tensor& w) {
               "gemm_skinny: 16-B aligned operands");
 }
 
-Tensor gemm_skinny(Tensor x, Tensor w, optional<Tensor> residual) {
+// the weight of an RMSNorm in front of the product
+static const void* check_norm(const optional<Tensor>& norm, int64_t M, int64_t K, bool glu) {
+  if (!norm.has_value() || !norm->defined()) return nullptr;
+  CHECK_BF16((*norm));
+  CHECK_CONTIG((*norm));
+  TORCH_CHECK(norm->is_cuda() && norm->dim() == 1 && norm->size(0) == K && reinterpret_cast<uintptr_t>(norm->data_ptr()) % 16 == 0 &&
+                  skinny_norms((int)M, (int)K, glu),
+              "gemm_skinny: norm weight [K], 16-B aligned, rows that fit beside W's units");
+  return norm->data_ptr();
+}
+
+Tensor gemm_skinny(Tensor x, Tensor w, optional<Tensor> residual, optional<Tensor> norm, double eps) {
   check_skinny(x, w);
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   const void* rp = nullptr;
@@ -553,17 +565,17 @@ Tensor gemm_skinny(Tensor x, Tensor w, optional<Tensor> residual) {
     rp = residual->data_ptr();
   }
   Tensor out = at::empty({M, N}, x.options());
-  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), rp, out.data_ptr(), M, N, K, false, stream());
+  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), rp, out.data_ptr(), M, N, K, false, check_norm(norm, M, K, false), (float)eps, stream());
   return out;
 }
 
 // h [M, F] = silu(x Wgᵀ) (x Wuᵀ), w [2F, K] = [gate | up] rows
-Tensor gemm_skinny_swiglu(Tensor x, Tensor w) {
+Tensor gemm_skinny_swiglu(Tensor x, Tensor w, optional<Tensor> norm, double eps) {
   check_skinny(x, w);
   const int64_t M = x.size(0), K = x.size(1), F = w.size(0) / 2;
   TORCH_CHECK(w.size(0) % 32 == 0, "gemm_skinny_swiglu: W [2F, K], F % 16 == 0");
   Tensor out = at::empty({M, F}, x.options());
-  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), nullptr, out.data_ptr(), M, F, K, true, stream());
+  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), nullptr, out.data_ptr(), M, F, K, true, check_norm(norm, M, K, true), (float)eps, stream());
   return out;
 }
 
@@ -1797,8 +1809,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("nf4_quantize", &nf4_quantize);
   m.def("nf4_dequant", &nf4_dequant);
   m.def("nf4_dequant_fast", &nf4_dequant_fast);
-  m.def("gemm_skinny", &gemm_skinny);
-  m.def("gemm_skinny_swiglu", &gemm_skinny_swiglu);
+  m.def("skinny_norms", &skinny_norms);
+  m.def("gemm_skinny", &gemm_skinny, py::arg("x"), py::arg("w"), py::arg("residual"), py::arg("norm") = py::none(), py::arg("eps") = 0.0);
+  m.def("gemm_skinny_swiglu", &gemm_skinny_swiglu, py::arg("x"), py::arg("w"), py::arg("norm") = py::none(), py::arg("eps") = 0.0);
   m.def("lt_linear", &lt_linear);
   m.def("lt_addmm", &lt_addmm);
   m.def("lt_dx", &lt_dx);

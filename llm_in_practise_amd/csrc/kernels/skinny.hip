@@ -55,17 +55,28 @@ __device__ __forceinline__ void wait_units(int left) {
   }
 }
 
+// An RMSNorm in front of the product: the norm's weight (null: none).  A row is summed by wpr waves, 8 elements a lane and turn, as the norm's
+// own kernel does (norm.hip), so that the normed rows, rounded to bf16 as it rounds them, are the same bit for bit.
+struct Norm {
+  const bf16* w;
+  float eps;
+  int wpr;
+};
+
 // How K is cut into parts, each a chain of products whose sums are added in order: S pieces, or a part per wave of units of 64 or 128 in turns
 enum { PIECES, TURNS64, TURNS128 };
 
-template <int CT, int MT, int NW, int RING, bool GLU, int CUT, int PARTS>
+// NORM: the rows of x come first, are normed in LDS behind the static part (M rows of 2 K + 64 bytes, then the norm's weight) while W's first
+// units are on their way, and stay there; the rings hold W alone.
+template <int CT, int MT, int NW, int RING, bool GLU, int CUT, int PARTS, bool NORM>
 __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W,
                                                          const bf16* __restrict__ res, bf16* __restrict__ out, int M, int N,
-                                                         int K, int S) {
-  constexpr int CO = GLU ? CT / 2 : CT, UB = (CT + MT) * 2048, D = 2 * (CT + MT), RINGS = NW * RING * UB, SUMS = PARTS * CT * MT * 1024;
+                                                         int K, int S, Norm nrm) {
+  constexpr int CO = GLU ? CT / 2 : CT, UB = (CT + (NORM ? 0 : MT)) * 2048, D = UB / 1024, RINGS = NW * RING * UB, SUMS = PARTS * CT * MT * 1024;
   constexpr bool BESIDE = CUT == PIECES;        // (sums are left while the rings run; else they take the rings' place)
-  static_assert((RING - 1) * D < 64, "the counter of outstanding loads");
+  static_assert((NORM ? RING : RING - 1) * D < 64 && (!NORM || MT == 1), "the counter of outstanding loads");
   __shared__ __attribute__((aligned(1024))) char smem[BESIDE ? RINGS + SUMS : RINGS > SUMS ? RINGS : SUMS];
+  extern __shared__ __attribute__((aligned(16))) char rows[];
   f32x4(*red)[CT * MT][64] = reinterpret_cast<f32x4(*)[CT * MT][64]>(smem + (BESIDE ? RINGS : 0));
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * 16 * CO;
@@ -87,8 +98,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict_
     const uint32_t dst = base + slot * UB, k = (lp * len + 64 * lb - (lb == per - 1 ? odd : 0)) * 2;
 #pragma unroll
     for (int j = 0; j < 2 * CT; ++j) to_lds(GLU && j >= 2 * CO ? ur : wr, dst + j * 1024, wo[j % (2 * CO)], k);
+    if (!NORM)
 #pragma unroll
-    for (int j = 0; j < 2 * MT; ++j) to_lds(xr, dst + (2 * CT + j) * 1024, xo[j], k);
+      for (int j = 0; j < 2 * MT; ++j) to_lds(xr, dst + (2 * CT + j) * 1024, xo[j], k);
     if (++lb == per) lb = 0, lp += NW;
   };
   f32x4 acc[CT][MT];
@@ -105,7 +117,56 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict_
       for (int m = 0; m < MT; ++m) red[part][t * MT + m][lane] = acc[t][m];
   };
   clear();
+  // a wave brings the 1 KB pieces that it will read itself: row m's and the weight's, pieces p, p + wpr, ..
+  const int stride = 2 * K + 64, pieces = NORM ? K / (512 * nrm.wpr) : 0, p0 = NORM ? w % nrm.wpr : 0;
+  const int step = NORM ? NW / nrm.wpr : 1;
+  if (NORM) {
+    const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)rows);
+    const rsrc gr = window(nrm.w);
+    for (int c = 0; c < pieces; ++c) {
+      const uint32_t o = (c * nrm.wpr + p0) * 1024;
+      to_lds(gr, at + M * stride + o, lane * 16, o);
+      for (int m = w / nrm.wpr; m < M; m += step) to_lds(xr, at + m * stride + o, (uint32_t)m * (uint32_t)ldx * 2 + lane * 16, o);
+    }
+  }
   for (int i = 0; i < min(RING, cnt); ++i) fill(i);
+  if (NORM) {
+    __shared__ float part[4][2];
+    wait_units<D, RING>(min(RING, cnt));
+    for (int m = w / nrm.wpr; m < M; m += step) {
+      float ss = 0.f;
+#pragma unroll 4
+      for (int c = 0; c < pieces; ++c) {
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(rows + m * stride + (c * nrm.wpr + p0) * 1024 + lane * 16);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += (float)v[i] * (float)v[i];
+      }
+      ss = wave_sum(ss);
+      if (lane == 0) part[m][p0] = ss;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                 // (not a fence: it would wait for W's units too)
+    asm volatile("" ::: "memory");
+    for (int m = w / nrm.wpr; m < M; m += step) {
+      float tot = 0.f;
+      for (int i = 0; i < nrm.wpr; ++i) tot += part[m][i];
+      const float r = rsqrtf(tot / K + nrm.eps);
+#pragma unroll 4
+      for (int c = 0; c < pieces; ++c) {
+        const int o = (c * nrm.wpr + p0) * 1024 + lane * 16;
+        bf16x8* at = reinterpret_cast<bf16x8*>(rows + m * stride + o);
+        const bf16x8 v = *at, wv = *reinterpret_cast<const bf16x8*>(rows + M * stride + o);
+        bf16x8 y;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = (bf16)((float)v[i] * r * (float)wv[i]);
+        *at = y;
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
+  int cp = w, cb = 0;                             // (NORM: the part and the place in it of the unit that is multiplied)
   int rp = w, rb = 0;
   for (int i = 0, slot = 0; i < cnt; ++i) {
     wait_units<D, RING - 1>(cnt - 1 - i);
@@ -116,9 +177,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict_
       const int c = li * 128 + ((4 * h + g) ^ (li & 7)) * 16;
 #pragma unroll
       for (int t = 0; t < CT; ++t) a[h][t] = *reinterpret_cast<const bf16x8*>(p + t * 2048 + c);
+      if (NORM) {
+        const int k = cp * len + 64 * cb - (cb == per - 1 ? odd : 0);
+        b[h][0] = *reinterpret_cast<const bf16x8*>(rows + min(li, M - 1) * stride + 2 * k + 64 * h + 16 * g);
+      } else {
 #pragma unroll
-      for (int m = 0; m < MT; ++m) b[h][m] = *reinterpret_cast<const bf16x8*>(p + (CT + m) * 2048 + c);
+        for (int m = 0; m < MT; ++m) b[h][m] = *reinterpret_cast<const bf16x8*>(p + (CT + m) * 2048 + c);
+      }
     }
+    if (NORM && ++cb == per) cb = 0, cp += NW;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // the unit is in registers: its place is free
     if (i + RING < cnt) fill(slot);
 #pragma unroll
@@ -177,31 +244,55 @@ static int skinny_splits(int N, int K) {
   return s;
 }
 
+// Rows that gemm_skinny norms itself, the norm's weight and the rows beside the rings in LDS: as many as leave the workgroups a CU holds where
+// they were, and where a workgroup norms them in the time that W takes to come.  µs, norm and product → here, 1 / 2 / 3 / 4 rows: 6144 × 4096
+// 15.4 → 12.5 / 12.7 / 19.3 / 19.6, 2 × 12288 × 4096 gated 39.8 → 37.3 / 40.0 / 39.4 / 38.3, 2 × 9728 × 2560 gated 25.8 → 22.0 / 21.1 / 22.7 / 26.0,
+// 6144 × 2560 12.9 → 9.6 to 4 rows; 4096 × 1024 5.8 → 4.6 / 4.8 / 5.5 / 5.5, at 5 rows 6.2, at 8 7.0.
+static size_t norm_bytes(int M, int K) { return (size_t)M * (2 * K + 64) + 2 * K; }
+bool skinny_norms(int M, int K, bool glu) { return M <= 4 && K <= 4096 && K % 512 == 0 && norm_bytes(M, K) <= (glu ? 21 : 30) * 1024; }
+
 // One tile of W a workgroup (GLU: 16 gate and 16 up rows).  Eight waves where one workgroup a CU holds all of W's tiles, else four, so
 // that two fit into a CU's LDS (6144 × 4096, 12 rows: 12.3 µs against 13.5 with two tiles of 8 waves); the gated form takes three of them.
-void launch_gemm_skinny(const void* X, int ldx, const void* W, const void* res, void* out, int M, int N, int K, bool glu,
+template <bool NORM>
+static void launch_rows(const void* X, int ldx, const void* W, const void* res, void* out, int M, int N, int K, bool glu, const Norm& nrm,
                         hipStream_t st) {
   const int pieces = skinny_splits(N, K);
-#define L(CT_, MT_, NW_, RING_, GLU_, CUT_, PARTS_)                                                                        \
-  gemm_skinny_k<CT_, MT_, NW_, RING_, GLU_, CUT_, PARTS_><<<(N + 15) / 16, 64 * NW_, 0, st>>>(                             \
-      (const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, pieces)
-  if (M > 32) {
-    if (glu) L(2, 4, 4, 3, true, TURNS64, 4);
-    else L(1, 4, 4, 3, false, TURNS64, 4);
-  } else if (M > 16) {
-    if (glu) L(2, 2, 4, 3, true, TURNS64, 4);
-    else L(1, 2, 4, 4, false, TURNS64, 4);
-  } else if (glu) {
-    if (N > 4096 && K % 2048 && K % 128 == 0) L(2, 1, 2, 4, true, TURNS128, 2);
-    else L(2, 1, 4, 2, true, TURNS64, 4);
+  const size_t extra = NORM ? norm_bytes(M, K) : 0;
+#define L(CT_, NW_, RING_, GLU_, CUT_, PARTS_)                                                                             \
+  gemm_skinny_k<CT_, 1, NW_, RING_, GLU_, CUT_, PARTS_, NORM><<<(N + 15) / 16, 64 * NW_, extra, st>>>(                     \
+      (const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, pieces, nrm)
+  if (glu) {
+    if (N > 4096 && K % 2048 && K % 128 == 0) L(2, 2, 4, true, TURNS128, 2);
+    else L(2, 4, 2, true, TURNS64, 4);
   } else if (pieces > 32) {
-    L(1, 1, 4, 4, false, TURNS64, 4);
+    L(1, 4, 4, false, TURNS64, 4);
   } else if (pieces > 16) {
-    L(1, 1, 8, 3, false, PIECES, 32);
+    L(1, 8, 3, false, PIECES, 32);
   } else if (pieces >= 8 && N <= 4096) {
-    L(1, 1, 8, 4, false, PIECES, 16);
+    L(1, 8, 4, false, PIECES, 16);
   } else {
-    L(1, 1, 4, 4, false, PIECES, 16);
+    L(1, 4, 4, false, PIECES, 16);
+  }
+#undef L
+}
+
+// norm: the weight of an RMSNorm in front of the product, or null (else skinny_norms(M, K, glu))
+void launch_gemm_skinny(const void* X, int ldx, const void* W, const void* res, void* out, int M, int N, int K, bool glu,
+                        const void* norm, float eps, hipStream_t st) {
+  const Norm nrm = {(const bf16*)norm, eps, K == 1024 || K == 2048 || K == 4096 ? 2 : 1};
+#define L(CT_, MT_, RING_, GLU_)                                                                                          \
+  gemm_skinny_k<CT_, MT_, 4, RING_, GLU_, TURNS64, 4, false><<<(N + 15) / 16, 256, 0, st>>>(                              \
+      (const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, 1, nrm)
+  if (M > 32) {
+    if (glu) L(2, 4, 3, true);
+    else L(1, 4, 3, false);
+  } else if (M > 16) {
+    if (glu) L(2, 2, 3, true);
+    else L(1, 2, 4, false);
+  } else if (norm != nullptr) {
+    launch_rows<true>(X, ldx, W, res, out, M, N, K, glu, nrm, st);
+  } else {
+    launch_rows<false>(X, ldx, W, res, out, M, N, K, glu, nrm, st);
   }
 #undef L
   LIPA_CHECK_LAUNCH();

@@ -26,6 +26,7 @@ import torch.nn as nn
 
 from ..ops import reference as ref
 from ..ops.activation import swiglu_fused
+from ..ops.gemm import normed_rows
 from ..ops.mlp import fusable as mlp_fusable, skinny_swiglu, swiglu_mlp
 from ..ops.attention import flash_attention, flash_attention_prefix
 from ..ops.decode import decode_attention_append
@@ -143,6 +144,11 @@ def qwen3_config(name: str, **overrides) -> Qwen3Config:
     return Qwen3Config(**kw)
 
 
+def _adapted(mods) -> bool:
+    """Whether any of these projections carries an adapter beside its weight."""
+    return any((isinstance(m, LoraLayer) and not m.merged) or getattr(_leaf_linear(m), "_mlora", None) is not None for m in mods)
+
+
 class Qwen3Attention(nn.Module):
     def __init__(self, cfg: Qwen3Config, layer_idx: int):
         super().__init__()
@@ -166,10 +172,18 @@ class Qwen3Attention(nn.Module):
         mods = [self.q_proj, self.k_proj, self.v_proj]
         self._qkv = FusedProjection(mods) if can_fuse(mods) else None
 
+    def normed_few_rows(self, x, norm):
+        """q | k | v of a decode step's rows in front of their norm, or None (adapters, other weights, more rows)."""
+        f = self._qkv
+        if x.shape[0] > 4 or f is None or self.tp_group is not None or f.bias is not None or _adapted(f.mods):
+            return None
+        return normed_rows(x, norm.weight, norm.eps, f.base)
+
     def forward(self, x, cos, sin, B, S, residual=None, cache: KVCache | None = None, start: int = 0,
-                kv_lens=None):
+                kv_lens=None, qkv=None):
         tr = self.training
-        qkv = project([self.q_proj, self.k_proj, self.v_proj], x, None, tr, self._qkv)
+        if qkv is None:
+            qkv = project([self.q_proj, self.k_proj, self.v_proj], x, None, tr, self._qkv)
         if self.q_norm is not None:
             q, k, v = qk_norm_rope(qkv, self.q_norm.weight, self.k_norm.weight, cos, sin,
                                    self.hq, self.hkv, self.d, self.cfg.rms_norm_eps)
@@ -238,19 +252,25 @@ class Qwen3MLP(nn.Module):
 
     def _few_rows(self, x):
         """The activated gate|up product of a decode step in one launch, or None (adapters, other weights, more rows)."""
-        if self._gu is None or self._gu.bias is not None or any(
-                (isinstance(m, LoraLayer) and not m.merged) or getattr(_leaf_linear(m), "_mlora", None) is not None
-                for m in (self.gate_proj, self.up_proj)):
+        if self._gu is None or self._gu.bias is not None or _adapted((self.gate_proj, self.up_proj)):
             return None
         base = self._gu.base
         return int4_swiglu(x, base) if isinstance(base, Int4Weight) else skinny_swiglu(x, base)
 
-    def forward(self, x, residual=None):
+    def normed_few_rows(self, x, norm):
+        """The same of rows in front of their norm, or None."""
+        if x.shape[0] > 4 or self._gu is None or self.tp_group is not None or self._gu.bias is not None or \
+                _adapted((self.gate_proj, self.up_proj)) or self._fused_bases(x) is not None:
+            return None
+        return skinny_swiglu(x, self._gu.base, norm.weight, norm.eps)
+
+    def forward(self, x, residual=None, h=None):
         tr = self.training
-        bases = self._fused_bases(x)
+        bases = self._fused_bases(x) if h is None else None
         if bases is not None:
             return swiglu_mlp(x, bases[0], bases[1], residual)
-        h = self._few_rows(x)
+        if h is None:
+            h = self._few_rows(x)
         if h is None:
             h = swiglu_fused(project([self.gate_proj, self.up_proj], x, None, tr, self._gu))
         if self.tp_group is None:
@@ -268,8 +288,12 @@ class Qwen3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
 
     def forward(self, x, cos, sin, B, S, cache=None, start=0, kv_lens=None):
-        xn, skip = rms_norm_residual(x, self.input_layernorm.weight, self.input_layernorm.eps)
-        h = self.self_attn(xn, cos, sin, B, S, residual=skip, cache=cache, start=start, kv_lens=kv_lens)
+        qkv = self.self_attn.normed_few_rows(x, self.input_layernorm)
+        xn, skip = (x, x) if qkv is not None else rms_norm_residual(x, self.input_layernorm.weight, self.input_layernorm.eps)
+        h = self.self_attn(xn, cos, sin, B, S, residual=skip, cache=cache, start=start, kv_lens=kv_lens, qkv=qkv)
+        act = self.mlp.normed_few_rows(h, self.post_attention_layernorm)
+        if act is not None:
+            return self.mlp(h, residual=h, h=act)
         hn, skip = rms_norm_residual(h, self.post_attention_layernorm.weight, self.post_attention_layernorm.eps)
         return self.mlp(hn, residual=skip)
 

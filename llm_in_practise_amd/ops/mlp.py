@@ -26,7 +26,7 @@ import torch
 from ..quant.nf4 import NF4Weight
 from ._native import force_reference, native, fn_apply
 from .checkpoint import _sac_recording, sac_put, sac_take, saves_discarded, tail_skippable
-from .gemm import _MIN_M, _count, _nf4_expand, _nf4_w4
+from .gemm import _MIN_M, _count, _nf4_expand, _nf4_w4, norms_rows
 
 
 def _operand(base, reused: bool):
@@ -115,16 +115,17 @@ def swiglu_mlp(x: torch.Tensor, gu_base, down_base, residual: torch.Tensor | Non
 class _SkinnySwiGLUFn(torch.autograd.Function):
     """(No backward: skinny_swiglu leaves what needs a gradient to the differentiable ops.)"""
     @staticmethod
-    def forward(ctx, x, w):
-        return native().gemm_skinny_swiglu(x, w)
+    def forward(ctx, x, w, norm=None, eps=0.0):
+        return native().gemm_skinny_swiglu(x, w, norm, eps)
 
 
-def skinny_swiglu(x: torch.Tensor, gu_base) -> torch.Tensor | None:
+def skinny_swiglu(x: torch.Tensor, gu_base, norm=None, eps: float = 0.0) -> torch.Tensor | None:
     """``silu(x·W_gateᵀ)·(x·W_upᵀ)`` of up to 16 decode rows in one launch (csrc/kernels/skinny.hip), or None where that kernel
     does not serve: a bf16 [gate | up] weight, no gradient.  The products are rounded to bf16 before the activation, as the
     separate kernels round them.  Library and activation → here, µs at 1 / 16 rows: 4096 → 2 × 12288 48 / 49 → 38 / 37, 2560 → 2 × 9728
     48 / 48 → 23 / 23, 1024 → 2 × 3072 10.1 / 10.1 → 5.1 / 5.2, 4096 → 2 × 14336 67 / 69 → 45 / 46.  Wider and deeper weights, and more rows,
-    stay with the library's product."""
+    stay with the library's product.  With ``norm`` the rows stand in front of the RMSNorm of that weight, which the launch forms bit for
+    bit as its own kernel does (:func:`~.gemm.norms_rows`; else None): 39.7 → 37.3 µs, 25.8 → 22 and 6.8 → 5.4 at 1 row, norm included."""
     x2 = x.reshape(-1, x.shape[-1])
     if (torch.is_grad_enabled() and x.requires_grad) or not (
             x.is_cuda and x.dtype == torch.bfloat16 and isinstance(gu_base, torch.Tensor) and gu_base.dtype == torch.bfloat16
@@ -133,5 +134,7 @@ def skinny_swiglu(x: torch.Tensor, gu_base) -> torch.Tensor | None:
             and x2.stride(0) % 8 == 0 and x2.shape[1] % 64 == 0 and gu_base.shape[0] % 32 == 0
             and x2.data_ptr() % 16 == 0 and gu_base.data_ptr() % 16 == 0 and not force_reference()):
         return None
+    if norm is not None and not norms_rows(x2, norm, gu_base, True):
+        return None
     _count("decode")
-    return fn_apply(_SkinnySwiGLUFn, x2, gu_base).view(*x.shape[:-1], gu_base.shape[0] // 2)
+    return fn_apply(_SkinnySwiGLUFn, x2, gu_base, norm, eps).view(*x.shape[:-1], gu_base.shape[0] // 2)

@@ -207,6 +207,73 @@ def test_gemm_skinny_rows_do_not_depend_on_their_number(native_ext, N, K):
         assert torch.equal(native_ext.gemm_skinny_swiglu(x[:m], w), h[:m])
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,K", [(16, 512), (6144, 1024), (128, 4096), (4096, 4096), (8192, 1536), (4608, 3584), (9728, 2560), (2560, 2048)])
+def test_product_of_rows_in_front_of_their_norm(native_ext, M, N, K):
+    """One wave or two a row, W's tiles to 4 and 8 waves in all their cuts: the bits of the norm's own kernel and the product; a row that
+    holds an infinity or NaN is NaN and changes no other; rows a stride apart; nothing that does not fit; replays of a captured call."""
+    from llm_in_practise_amd.ops.norm import rms_norm
+    torch.manual_seed(N + M)
+    xb, nw = (3 * torch.randn(M, K + 8, device=DEV)).bfloat16(), torch.randn(K, device=DEV).bfloat16()
+    w, x = (torch.randn(2 * N, K, device=DEV) * K ** -0.5).bfloat16(), xb[:, :K]
+    forms = [(lambda x: native_ext.gemm_skinny(x, w[:N], None, nw, 1e-6), lambda x: native_ext.gemm_skinny(x, w[:N], None), False),
+             (lambda x: native_ext.gemm_skinny_swiglu(x, w, nw, 1e-6), lambda x: native_ext.gemm_skinny_swiglu(x, w), True)]
+    for one, product, glu in forms:
+        if not native_ext.skinny_norms(M, K, glu):
+            with pytest.raises(RuntimeError):
+                one(x)
+            continue
+        assert torch.equal(one(x), product(rms_norm(x.contiguous(), nw, 1e-6)))
+        for bad in (float("inf"), float("nan")):
+            y = x.clone()
+            y[M - 1, K - 1] = bad
+            got = one(y)
+            assert got[M - 1].isnan().all() and torch.equal(got[:M - 1], one(x)[:M - 1])
+        y = x.clone()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = one(y)
+        for seed in range(3):
+            y.copy_(torch.randn(M, K, device=DEV))
+            g.replay()
+            assert torch.equal(out, product(rms_norm(y, nw, 1e-6)))
+    assert not native_ext.skinny_norms(5, K, False) and not native_ext.skinny_norms(1, K + 64, False)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 4, 5])
+def test_decode_layers_norm_their_rows_in_the_products(native_ext, monkeypatch, rows):
+    """The same logits as with the norm's own kernel, fused products and separate ones, adapters, a gradient."""
+    from llm_in_practise_amd.models import qwen3
+    m = qwen3.Qwen3ForCausalLM.from_config(qwen3.qwen3_config("qwen3-small"), dtype=torch.bfloat16, device=DEV, seed=0).eval()
+    m.requires_grad_(False)
+    ids = torch.randint(0, 4096, (1, rows), device=DEV)
+    calls = []
+    real = qwen3.normed_rows
+
+    def counted(*a):
+        y = real(*a)
+        calls.append(y is not None)
+        return y
+    monkeypatch.setattr(qwen3, "normed_rows", counted)
+    for fused in (False, True):
+        if fused:
+            for layer in m.model.layers:
+                layer.self_attn.fuse()
+                layer.mlp.fuse()
+        calls.clear()
+        with torch.no_grad():
+            got = m(ids).logits
+        assert any(calls) == (fused and rows <= 4)
+        with monkeypatch.context() as c, torch.no_grad():
+            c.setattr(qwen3.Qwen3Attention, "normed_few_rows", lambda *a: None)
+            c.setattr(qwen3.Qwen3MLP, "normed_few_rows", lambda *a: None)
+            assert torch.equal(m(ids).logits, got)
+    x = torch.randn(rows, m.config.hidden_size, device=DEV).bfloat16().requires_grad_()
+    layer = m.model.layers[0]
+    assert layer.self_attn.normed_few_rows(x, layer.input_layernorm) is None        # (the norm's gradient)
+    assert layer.mlp.normed_few_rows(x, layer.post_attention_layernorm) is None
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 40])
 @pytest.mark.parametrize("N,K", [(32, 64), (1056, 192), (6144, 1088), (64, 1984), (96, 20480)])
 def test_gemm_skinny_infinite_weights(native_ext, M, N, K):
