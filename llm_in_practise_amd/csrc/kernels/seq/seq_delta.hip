@@ -10,8 +10,8 @@
 // it is in the token-by-token scan.  The second kernel walks a sequence's blocks with the state in registers; all products are float on
 // the float matrix units (v_mfma_f32_16x16x4_f32), whose result layout is also its operand layout.
 //
-// Measured, blocks of 16 -> of 32 tokens: three sequences of 1500, 700 and 97 tokens, 8 heads of 128 x 128: 112 -> 96 us (32 for the first
-// kernel, 64 for the walk, which is bound by the longest sequence's chain: 1.3 us a block of 32, 0.7 of them products of a wave on the
+// Measured, blocks of 16 -> of 32 tokens: three sequences of 1500, 700 and 97 tokens, 8 heads of 128 x 128: 112 -> 90 us (26 for the first
+// kernel - 32 with two blocks a CU and rows that left four bytes a lane - and 64 for the walk, which is bound by the longest sequence's chain: 1.3 us a block of 32, 0.7 of them products of a wave on the
 // float matrix unit; 0.94 us a block of 16).  Error against 64 bits of outputs, blocks of 16 -> 32: 3.2 -> 2.8e-7 where decays are next
 // to 1, 1.6 -> 1.7 at 0.95, 1.25 -> 1.4 at 0.8, 1.1 -> 1.2 at 0.4.
 #include "seq_block.h"
@@ -36,6 +36,14 @@ __device__ __forceinline__ f32x4 mfma4(const f32x4& a, const f32x4& b, f32x4 c) 
   return c;
 }
 
+// element e of lane row r <-> element r of lane row e
+__device__ __forceinline__ f32x4 turn_rows(const f32x4& v) {
+  auto u = [](float f) { return __float_as_uint(f); };
+  const auto a = __builtin_amdgcn_permlane32_swap(u(v[0]), u(v[2]), false, false), b = __builtin_amdgcn_permlane32_swap(u(v[1]), u(v[3]), false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false), d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return f32x4{__uint_as_float(c[0]), __uint_as_float(c[1]), __uint_as_float(d[0]), __uint_as_float(d[1])};
+}
+
 // 512 threads, half of them a tile: token j = tid / 16 of it, and the four channels 4 x .. of every 64 (x = tid % 16).  A thread carries
 // its token's key times the decays of the tokens behind it; at token s the 16 threads of a row sum k_s and q_s against it, and lane
 // s keeps the sums.
@@ -47,12 +55,13 @@ __global__ __launch_bounds__(512, 6) void k_delta_prep(const T* __restrict__ q, 
   constexpr int DK = 64 * NS, ROWS = BT * DK;
   __shared__ __attribute__((aligned(16))) float sg[2 * ROWS];        // decays, then k G_16 / G of the first tile
   __shared__ __attribute__((aligned(16))) float sk[2 * ROWS];        // keys, then k G
-  __shared__ __attribute__((aligned(16))) float sq[2 * ROWS];        // queries, then q G of the second tile
-  __shared__ __attribute__((aligned(16))) float sG[2][DK];           // G_16 of the tiles
+  __shared__ __attribute__((aligned(16))) float sq[2 * ROWS];        // queries, then q G of the second tile and G_16 of both
   __shared__ __attribute__((aligned(16))) float sT[2][BT * BT];
   __shared__ __attribute__((aligned(16))) float sA[2][BT * BT];      // A; then A_21 in place of the first
   __shared__ float sb[LEN];
   __shared__ int sbad[LEN];
+  // G_16 of the tiles, where the second tile's queries stood: with a place of its own a CU holds two of these blocks, not three
+  float(*sG)[DK] = reinterpret_cast<float(*)[DK]>(sq + ROWS);
   const int slot = blockIdx.y, hd = blockIdx.x, tid = threadIdx.x;
   Piece blk;
   if (!find_piece<LEN>(d, pc, slot, blk)) return;
@@ -162,9 +171,9 @@ __global__ __launch_bounds__(512, 6) void k_delta_prep(const T* __restrict__ q, 
     const int D = 64 * c + 4 * x, tile = 4 * c + (x >> 2), base = half * ROWS + (tile * 64 + (x & 3) * 16 + j) * 4;
     const f32x4 G1 = row4(&sG[0][D]), G2 = row4(&sG[1][D]);
     *reinterpret_cast<f32x4*>(cq + base) = half == 0 ? qj[c] * Gm[c] : qj[c] * Gm[c] * G1;
-    const f32x4 P = half == 0 ? W[c] * G2 : W[c];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) cp[half * ROWS + (tile * 64 + (j >> 2) * 16 + 4 * (x & 3) + e) * 4 + (j & 3)] = bad ? NAN : P[e];
+    const f32x4 P = half == 0 ? W[c] * G2 : W[c], own = bad ? f32x4{NAN, NAN, NAN, NAN} : P;
+    // a row of lanes holds a token: turned, row r has channel 4 x + r of the wave's four tokens
+    *reinterpret_cast<f32x4*>(cp + half * ROWS + (tile * 64 + (j >> 2) * 16 + 4 * (x & 3) + (j & 3)) * 4) = turn_rows(own);
     if (tid < 16) *reinterpret_cast<f32x4*>(cg + D) = G1 * G2;
   }
   if (w < 2) {                                               // A_21 and B_21: rows of the second tile against the keys of the first
@@ -192,13 +201,10 @@ __global__ __launch_bounds__(512, 6) void k_delta_prep(const T* __restrict__ q, 
       x1[e] = sk[(4 * g4 + e) * DK + 16 * kt + li];
       x2[e] = sk[ROWS + (4 * g4 + e) * DK + 16 * kt + li] * G1;
     }
-    const f32x4 y1 = mfma4(T1, x1, zero), y2 = mfma4(T2, mfma4(X, y1, x2), zero);
-    float* to = ck + (kt * 64 + (li >> 2) * 16 + 4 * g4) * 4 + (li & 3);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      to[4 * e] = y1[e];
-      to[ROWS + 4 * e] = y2[e];
-    }
+    // (with the factors the other way round a lane holds four channels of a token, as the rows stand in memory)
+    float* to = ck + (kt * 64 + g4 * 16 + li) * 4;
+    *reinterpret_cast<f32x4*>(to) = mfma4(x1, T1, zero);
+    *reinterpret_cast<f32x4*>(to + ROWS) = mfma4(mfma4(X, mfma4(T1, x1, zero), x2), T2, zero);
   }
   bool odd = false;
   for (int vt = w; vt < vtiles; vt += 8) {
@@ -468,8 +474,8 @@ void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int l
 
 // Floats of workspace for at most `most` (longer steps run in windows), or 0 where blocks of 16 (seq_block.hip) are not slower or there is
 // no room.  Two tiles between two barriers pay where one block of threads a CU walks a long sequence; the first kernel is the longer
-// one, and blocks of 16 fit a CU twice.  us, 16 -> 32 tokens, heads of 128 x 128: 8 heads x 1000 tokens 75 -> 61, x 4000 262 -> 208, x 200 24.5
-// -> 25.4, 1500 + 700 + 97 112 -> 96, 4 x 2000 (256 blocks of threads) 181 -> 160, 12 x 700 (768) 172 -> 183; 4 heads x 9000 540 -> 425, 12 x 700
+// one, and blocks of 16 fit a CU twice.  us, 16 -> 32 tokens, heads of 128 x 128: 8 heads x 1000 tokens 75 -> 58, x 4000 262 -> 197, x 200 24.5
+// -> 25, 1500 + 700 + 97 112 -> 90, 4 x 2000 (256 blocks of threads) 181 -> 160, 12 x 700 (768) 172 -> 183; 4 heads x 9000 540 -> 425, 12 x 700
 // (384) 104 -> 113; keys of 64, 8 x 64 columns, 1000 + 500 59 -> 44; of 192 97 -> 95, of 256 146 -> 151.
 size_t seq_delta_floats(int T_, int B, int H, int dk, int dv, size_t most) {
   if (dk > 128 || T_ < 300l * B || (long)B * H * ((dv + 15) / 16) > 256) return 0;
