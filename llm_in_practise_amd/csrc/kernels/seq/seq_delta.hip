@@ -473,12 +473,15 @@ void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int l
 }  // namespace
 
 // Floats of workspace for at most `most` (longer steps run in windows), or 0 where blocks of 16 (seq_block.hip) are not slower or there is
-// no room.  Two tiles between two barriers pay where one block of threads a CU walks a long sequence; the first kernel is the longer
-// one, and blocks of 16 fit a CU twice.  us, 16 -> 32 tokens, heads of 128 x 128: 8 heads x 1000 tokens 75 -> 58, x 4000 262 -> 197, x 200 24.5
-// -> 25, 1500 + 700 + 97 112 -> 90, 4 x 2000 (256 blocks of threads) 181 -> 160, 12 x 700 (768) 172 -> 183; 4 heads x 9000 540 -> 425, 12 x 700
-// (384) 104 -> 113; keys of 64, 8 x 64 columns, 1000 + 500 59 -> 44; of 192 97 -> 95, of 256 146 -> 151.
+// no room.  Two tiles between two barriers pay where one block of threads a CU walks a long sequence, and, with few columns, where the first
+// kernel, whose blocks take all columns at once, is most of the work; with many columns blocks of 16 fit a CU twice.  us, 16 -> 32 tokens,
+// heads of 128 x 128: 8 heads x 1000 tokens 75 -> 60, x 4000 262 -> 200, x 200 24.3 -> 24.1, 5 x 300 52 -> 52, 1500 + 700 + 97 112 -> 90, 4 x 2000
+// (256 blocks of threads) 181 -> 147, 12 x 100 40 -> 44, 12 x 700 (768) 170 -> 164; 4 heads x 9000 540 -> 414, x 64 15.7 -> 17.5; 64 heads
+// 2 x 1000 (1024) 336 -> 358, 4 x 256 203 -> 208.  Of 128 x 64: 32 heads 8 x 512 (1024) 285 -> 236, 16 heads 20 x 400 (1280) 288 -> 240; of
+// 128 x 32, 8 x 512 103 -> 78; of 64 x 64, 4 x 600 (512) 86 -> 80, 40 x 320 (1280) 123 -> 122; of 64 x 128, 16 heads 16 x 512 (2048) 230 -> 238,
+// 64 heads 4 x 300 136 -> 159.  Keys of 192 97 -> 95, of 256 146 -> 151.
 size_t seq_delta_floats(int T_, int B, int H, int dk, int dv, size_t most) {
-  if (dk > 128 || T_ < 300l * B || (long)B * H * ((dv + 15) / 16) > 256) return 0;
+  if (dk > 128 || T_ < 300l * B || (dv > 64 && (long)B * H * ((dv + 15) / 16) > 256)) return 0;
   return delta_plan(T_, B, H, dk, dv, most).slots * slot_floats(H, dk, dv);
 }
 

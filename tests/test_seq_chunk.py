@@ -315,6 +315,19 @@ def test_delta_blocks_of_two_tiles(lens, starts, H, G, dk, dv, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("L,B,H,dk,dv,long", [
+    (1000, 1, 8, 128, 128, True), (200, 1, 8, 128, 128, False), (300, 5, 6, 128, 128, True), (299, 5, 6, 128, 128, False),
+    (2000, 4, 8, 128, 128, True), (2000, 5, 8, 128, 128, False), (400, 20, 16, 128, 64, True), (400, 20, 16, 128, 68, False),
+    (512, 8, 16, 128, 32, True), (600, 4, 32, 64, 64, True), (512, 16, 16, 64, 128, False), (1000, 2, 4, 192, 128, False),
+    (1000, 2, 4, 256, 64, False)])
+def test_delta_blocks_are_long_only_where_they_are_not_slower(L, B, H, dk, dv, long):
+    """Timed shapes on both sides of the choice between blocks of 16 and of 32 tokens: what a slot holds says which it is."""
+    from llm_in_practise_amd.ops._native import native_seq
+    floats = native_seq().scan_floats("delta", L * B, B, H, dk, dv)
+    assert floats > 0 and (floats % (H * (49 * dk + 516)) != 0) == long
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("name,value", [("v", float("inf")), ("v", float("nan")), ("k", float("-inf")), ("q", float("nan")),
                                         ("g", float("nan")), ("g", float("inf")), ("b", float("nan"))])
 @pytest.mark.parametrize("t", [310, 325, 326, 341, 342, 650, 669])
