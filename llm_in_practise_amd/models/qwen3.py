@@ -175,7 +175,7 @@ class Qwen3Attention(nn.Module):
     def normed_few_rows(self, x, norm):
         """q | k | v of a decode step's rows in front of their norm, or None (adapters, other weights, more rows)."""
         f = self._qkv
-        if x.shape[0] > 4 or f is None or self.tp_group is not None or f.bias is not None or _adapted(f.mods):
+        if f is None or self.tp_group is not None or f.bias is not None or _adapted(f.mods):
             return None
         return normed_rows(x, norm.weight, norm.eps, f.base)
 
@@ -259,7 +259,7 @@ class Qwen3MLP(nn.Module):
 
     def normed_few_rows(self, x, norm):
         """The same of rows in front of their norm, or None."""
-        if x.shape[0] > 4 or self._gu is None or self.tp_group is not None or self._gu.bias is not None or \
+        if self._gu is None or self.tp_group is not None or self._gu.bias is not None or \
                 _adapted((self.gate_proj, self.up_proj)) or self._fused_bases(x) is not None:
             return None
         return skinny_swiglu(x, self._gu.base, norm.weight, norm.eps)
@@ -288,10 +288,11 @@ class Qwen3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
 
     def forward(self, x, cos, sin, B, S, cache=None, start=0, kv_lens=None):
-        qkv = self.self_attn.normed_few_rows(x, self.input_layernorm)
+        few = B * S <= 4                # rows that their products norm themselves
+        qkv = self.self_attn.normed_few_rows(x, self.input_layernorm) if few else None
         xn, skip = (x, x) if qkv is not None else rms_norm_residual(x, self.input_layernorm.weight, self.input_layernorm.eps)
         h = self.self_attn(xn, cos, sin, B, S, residual=skip, cache=cache, start=start, kv_lens=kv_lens, qkv=qkv)
-        act = self.mlp.normed_few_rows(h, self.post_attention_layernorm)
+        act = self.mlp.normed_few_rows(h, self.post_attention_layernorm) if few else None
         if act is not None:
             return self.mlp(h, residual=h, h=act)
         hn, skip = rms_norm_residual(h, self.post_attention_layernorm.weight, self.post_attention_layernorm.eps)
