@@ -20,7 +20,7 @@ import os
 import torch
 
 from ..quant.nf4 import NF4Weight, dequantize_nf4
-from ._native import fn_apply, force_reference, native
+from ._native import _functorch_active, fn_apply, force_reference, native
 
 _MIN_M = 256     # training / prefill-sized GEMMs: gemm4w and the fused LoRA paths
 
@@ -153,8 +153,8 @@ def head_logits(h: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 def norms_rows(x: torch.Tensor, weight, base, glu: bool) -> bool:
     """Whether the decode products (csrc/kernels/skinny.hip) take these rows in front of their RMSNorm: few bf16 rows of 512 .. 4096
-    that fit into LDS, no gradient, a norm's weight of their type and a bf16 weight that the product takes."""
-    return (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and 1 <= x.shape[0] <= 4 and x.is_contiguous() and x.data_ptr() % 16 == 0
+    that fit into LDS, no gradient and no transform, a norm's weight of their type and a bf16 weight that the product takes."""
+    return (not _functorch_active() and x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and 1 <= x.shape[0] <= 4 and x.is_contiguous() and x.data_ptr() % 16 == 0
             and isinstance(weight, torch.Tensor) and weight.is_cuda and weight.dtype == torch.bfloat16 and weight.is_contiguous()
             and weight.shape == x.shape[1:] and weight.data_ptr() % 16 == 0
             and isinstance(base, torch.Tensor) and base.is_cuda and base.dtype == torch.bfloat16 and base.is_contiguous()

@@ -268,6 +268,14 @@ def test_decode_layers_norm_their_rows_in_the_products(native_ext, monkeypatch, 
             c.setattr(qwen3.Qwen3Attention, "normed_few_rows", lambda *a: None)
             c.setattr(qwen3.Qwen3MLP, "normed_few_rows", lambda *a: None)
             assert torch.equal(m(ids).logits, got)
+    seen = []
+    for sub in (m.model.layers[1].self_attn, m.model.layers[1].mlp):    # a hook sees normed rows, whatever their number
+        handle = sub.register_forward_pre_hook(lambda mod, args: seen.append(args[0]))
+        with torch.no_grad():
+            assert torch.equal(m(ids).logits, got)
+        handle.remove()
+        rms = seen[-1].float().pow(2).mean(-1).sqrt()
+        assert (rms - 1).abs().max() < 0.1             # (the norms' weights are ones)
     x = torch.randn(rows, m.config.hidden_size, device=DEV).bfloat16().requires_grad_()
     layer = m.model.layers[0]
     assert layer.self_attn.normed_few_rows(x, layer.input_layernorm) is None        # (the norm's gradient)
