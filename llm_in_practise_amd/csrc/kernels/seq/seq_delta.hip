@@ -12,8 +12,10 @@
 //
 // Measured, blocks of 16 -> of 32 tokens: three sequences of 1500, 700 and 97 tokens, 8 heads of 128 x 128: 112 -> 90 us (26 for the first
 // kernel - 32 with two blocks a CU and rows that left four bytes a lane - and 64 for the walk, which is bound by the longest sequence's chain: 1.3 us a block of 32, 0.7 of them products of a wave on the
-// float matrix unit; 0.94 us a block of 16).  Error against 64 bits of outputs, blocks of 16 -> 32: 3.2 -> 2.8e-7 where decays are next
-// to 1, 1.6 -> 1.7 at 0.95, 1.25 -> 1.4 at 0.8, 1.1 -> 1.2 at 0.4.
+// float matrix unit; 0.94 us a block of 16).  Error against 64 bits of outputs, blocks of 16 -> 32: 3.2 -> 2.6e-7 where decays are next
+// to 1, 1.6 -> 1.55 at 0.95, 1.25 -> 1.28 at 0.8, 1.08 -> 1.10 at 0.4: the state and a tile's sums are added up by themselves and
+// rounded once at the size of what they are added to.
+
 #include "seq_block.h"
 
 #include <type_traits>
@@ -190,7 +192,8 @@ __global__ __launch_bounds__(512, 6) void k_delta_prep(const T* __restrict__ q, 
     for (int e = 0; e < 4; ++e) to[(4 * g4 + e) * BT + li] = a0[e];
   }
   __syncthreads();
-  // W and U, a wave a tile of 16 columns at a time: y1 = T_1 x1, y2 = T_2 (x2 - A_21 y1)
+  // W and U, a wave a tile of 16 columns at a time: y1 = T_1 x1, y2 = T_2 (x2 - A_21 y1), with sums of 16 by themselves: begun at x2 each
+  // would be rounded at its size
   const f32x4 T1 = row4(&sT[0][li * BT + 4 * g4]), T2 = row4(&sT[1][li * BT + 4 * g4]), X = -row4(&sA[0][li * BT + 4 * g4]);
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   for (int kt = w; kt < 4 * NS; kt += 8) {
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(512, 6) void k_delta_prep(const T* __restrict__ q, 
     // (with the factors the other way round a lane holds four channels of a token, as the rows stand in memory)
     float* to = ck + (kt * 64 + g4 * 16 + li) * 4;
     *reinterpret_cast<f32x4*>(to) = mfma4(x1, T1, zero);
-    *reinterpret_cast<f32x4*>(to + ROWS) = mfma4(mfma4(X, mfma4(T1, x1, zero), x2), T2, zero);
+    *reinterpret_cast<f32x4*>(to + ROWS) = mfma4(x2 + mfma4(X, mfma4(T1, x1, zero), zero), T2, zero);
   }
   bool odd = false;
   for (int vt = w; vt < vtiles; vt += 8) {
@@ -219,7 +222,7 @@ __global__ __launch_bounds__(512, 6) void k_delta_prep(const T* __restrict__ q, 
       x1[e] = isfinite(x1[e]) ? x1[e] : 0.f;
       x2[e] = isfinite(x2[e]) ? x2[e] : 0.f;
     }
-    const f32x4 y1 = mfma4(T1, x1, zero), y2 = mfma4(T2, mfma4(X, y1, x2), zero);
+    const f32x4 y1 = mfma4(T1, x1, zero), y2 = mfma4(T2, x2 + mfma4(X, y1, zero), zero);
     *reinterpret_cast<f32x4*>(cU + (vt * 64 + lane) * 4) = y1;
     *reinterpret_cast<f32x4*>(cU + ((vtiles + vt) * 64 + lane) * 4) = y2;
   }
@@ -389,9 +392,9 @@ __global__ __launch_bounds__(512, 2) void k_delta_walk(const float* __restrict__
   auto outputs = [&](int i, auto odd) {
     const auto& r = rq[i & 1];
     const f32x4 u0 = su[i & 1][0][lane], u1 = su[i & 1][1][lane];
-    f32x4 o = (r[0][half][lane] + r[1][half][lane]) + (r[2][half][lane] + r[3][half][lane]);
-    o = mfma4(bo[0], u0, o);
+    f32x4 o = mfma4(bo[0], u0, f32x4{0.f, 0.f, 0.f, 0.f});
     if (half) o = mfma4(bo[1], u1, o);
+    o += (r[0][half][lane] + r[1][half][lane]) + (r[2][half][lane] + r[3][half][lane]);
     if constexpr (odd) {
       int first = LEN;
 #pragma unroll
