@@ -6,6 +6,7 @@
 // several rows: the reads, not the arithmetic, bound a scan whose lanes own one column each.
 #include "seq_common.h"
 
+#include <algorithm>
 #include <cfloat>
 #include <utility>
 
@@ -570,7 +571,10 @@ int seq_gla_max_dk() { return 256; }
 // states, sequences x tokens x channels: 1 x 256 x 4096 30 -> 12, 1 x 1024 x 4096 61 -> 38, 1 x 4096 x 4096 155 -> 141, 1 x 9000 x 4096 320 ->
 // 334, 1 x 4096 x 2048 102 -> 143 (cut), 1 x 1024 x 1024 37 -> 37 (cut), 2048 + 1337 x 4096 129 -> 87, 4 x 512 x 4096 91 -> 49, 12 x 32 x 4096 14
 // -> 13, 16 x 16 x 4096 9.5 -> 15 (whole), 16 x 512 x 4096 164 -> 161, 16 x 512 x 8192 290 -> 314 (whole), 64 x 64 x 2048 42 -> 45 (whole).
-bool seq_selective_rows(int T_, int B, int C, int N) {
+// Its windows take rows that are no shorter than their columns (where rows repeat or overlap, what stands past a sequence's end is inside the
+// window) and 32-bit offsets into 64 of them; other strides take the other form.
+bool seq_selective_rows(int T_, int B, int C, int N, int ldx, int ldz, int ldb, int ldc, int ldo) {
+  if (std::min({ldx, ldz, ldo}) < C || std::min(ldb, ldc) < N || std::max({ldx, ldz, ldb, ldc, ldo}) >= 1 << 24) return false;
   if (N <= 8 || N > 16 || T_ < 32l * B || (long)B * C > 49152) return false;
   return 0.034f * (B > 1 ? 1.5f : 1.f) * T_ / B < 8.5e-6f * T_ * C + 25.f;
 }
@@ -625,7 +629,7 @@ void seq_selective_scan(int code, const void* x, int ldx, const float* dtp, cons
     }                                                                                                                    \
   } while (0)
   SEQ_DISPATCH_T(code, {
-    if (seq_selective_rows(d.Ttot, d.B, C, N))
+    if (seq_selective_rows(d.Ttot, d.B, C, N, ldx, ldz, ldb, ldc, ldo))
       hipLaunchKernelGGL((k_selective_row<T>), dim3((C + 15) / 16, d.B), dim3(256), 0, st, (const T*)x, ldx, dtp, dtb, (const T*)b, ldb,
                          (const T*)c, ldc, a_log, dskip, (const T*)z, ldz, S, (T*)out, ldo, scale, C, N, d);
     else if (N <= 16)

@@ -75,7 +75,7 @@ void seq_softcap(float*, size_t, float, hipStream_t);
 void seq_selective_scan(int, const void*, int, const float*, const float*, const void*, int, const void*, int, const float*,
                         const float*, const void*, int, float*, void*, int, float, int, int, float*, size_t, SeqDesc, hipStream_t);
 size_t seq_selective_floats(int, int, int, int, size_t);
-bool seq_selective_rows(int, int, int, int);
+bool seq_selective_rows(int, int, int, int, int, int, int, int, int);
 void seq_gla_scan(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float,
                   float*, float*, int, int, int, SeqDesc, hipStream_t);
 int seq_dyt_max_taps();
@@ -1162,7 +1162,7 @@ Tensor selective_scan(Tensor x, Tensor dt_pre, Tensor dt_bias, Tensor b, Tensor 
   }
   if (T == 0) return out;
   Tensor ws;
-  if (!seq_selective_rows((int)T, d.B, (int)C, (int)N))
+  if (!seq_selective_rows((int)T, d.B, (int)C, (int)N, ld(x), ld(z), ld(b), ld(c), ld(out)))
     if (const size_t n = seq_selective_floats((int)T, d.B, (int)C, (int)N, (size_t)most)) ws = at::empty({(int64_t)n}, S.options());
   seq_selective_scan(code, x.data_ptr(), ld(x), dt_pre.data_ptr<float>(), dt_bias.data_ptr<float>(), b.data_ptr(), ld(b),
                      c.data_ptr(), ld(c), a_log.data_ptr<float>(), d_skip.data_ptr<float>(), z.data_ptr(), ld(z),
@@ -1332,8 +1332,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("selective_floats", [](int64_t T, int64_t B, int64_t C, int64_t N, int64_t most) {        // 0: sequences run whole
     return (int64_t)seq_selective_floats((int)T, (int)B, (int)C, (int)N, (size_t)most);
   }, py::arg("T"), py::arg("B"), py::arg("C"), py::arg("N"), py::arg("most") = MOST_WS);
-  m.def("selective_rows", [](int64_t T, int64_t B, int64_t C, int64_t N) {       // whether a step runs with a state per lane
-    return seq_selective_rows((int)T, (int)B, (int)C, (int)N);
+  m.def("selective_rows", [](int64_t T, int64_t B, int64_t C, int64_t N) {       // whether a step of rows side by side runs with a state per lane
+    return seq_selective_rows((int)T, (int)B, (int)C, (int)N, (int)C, (int)C, (int)N, (int)N, (int)C);
   });
   m.def("selective_scan", &selective_scan, py::arg("x"), py::arg("dt_pre"), py::arg("dt_bias"), py::arg("b"), py::arg("c"),
         py::arg("a_log"), py::arg("d_skip"), py::arg("z"), py::arg("S"), py::arg("desc"), py::arg("live"), py::arg("out"),

@@ -425,6 +425,37 @@ def test_selective_with_a_state_per_lane(lens, starts, C, N, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("which", ["x", "z", "b", "c"])
+@pytest.mark.parametrize("form", ["one", "overlapping", "far"])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_selective_rows_of_any_stride(which, form, dt):
+    """One row for all tokens, rows that share elements, rows too far apart for 32-bit offsets into 64 of them."""
+    from llm_in_practise_amd.ops._native import native_seq
+    lens, C, N = [70, 33], 40, 16
+    g = torch.Generator().manual_seed(len(which + form))
+    T, w = sum(lens), C if which in "xz" else N
+    p = {k: torch.randn(T, n, generator=g).to(dt) for k, n in (("x", C), ("z", C), ("b", N), ("c", N))}
+    flat, ld = torch.randn(T + w, generator=g).to(dt), {"one": 0, "overlapping": 1}.get(form, (1 << 32) // (64 * p["x"].element_size()) + 8)
+    dtp, dtb, skip, a_log = (torch.randn(*s, generator=g) for s in ((T, C), (C,), (C,), (C, N)))
+    assert native_seq().selective_rows(T, 2, C, N)
+    res = []
+    for dev in ("cpu", "cuda"):
+        st, sb = _batch({"S": ((C, N), "f32")}, lens, [0, 3], dev)
+        st["S"].fill_(0.5)
+        q = {k: t.to(dev) for k, t in p.items()}
+        if form != "far":
+            q[which] = flat.to(dev).as_strided((T, w), (ld, 1))
+        elif dev == "cuda":
+            q[which] = torch.empty((T - 1) * ld + w, dtype=dt, device=dev).as_strided((T, w), (ld, 1)).copy_(p[which])
+        y = R.selective_scan(q["x"], dtp.to(dev), dtb.to(dev), q["b"], q["c"], a_log.to(dev), skip.to(dev), q["z"], st["S"], sb)
+        res.append((y.float().cpu(), st["S"].cpu()))
+    (y1, s1), (y0, s0) = res[1], res[0]
+    _close((s1,), (s0,), ("state",))
+    tol = TOL if dt == torch.float32 else 2.0 ** -8      # (bf16 outputs: both sides round, to at most one unit of 2^-8 apart)
+    assert torch.isfinite(y1).all() and (y1 - y0).norm() <= tol * y0.norm()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("name,value", [("x", float("inf")), ("b", float("nan")), ("b", float("inf")), ("c", float("nan")), ("dt", float("nan"))])
 @pytest.mark.parametrize("t", [40, 102, 203])
 def test_selective_token_that_is_no_number(name, value, t):
