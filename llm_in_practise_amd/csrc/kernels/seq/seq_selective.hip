@@ -565,18 +565,25 @@ __global__ __launch_bounds__(256) void k_gla_scan(const T* __restrict__ q, int l
 int seq_selective_max_states() { return 256; }
 int seq_gla_max_dk() { return 256; }
 
-// Whether a step runs with a state per lane.  Its longest sequence takes 0.034 us a token; the mean length stands for the longest one, half
-// as much again where there are several.  Beyond 12 waves on a SIMD (49152 channels of sequences) both forms are bound by issue, and
-// eight states per lane need fewer instructions; below 32 tokens staging 64 is most of the work.  us, the other form -> a state per lane, 16
-// states, sequences x tokens x channels: 1 x 256 x 4096 30 -> 12, 1 x 1024 x 4096 61 -> 38, 1 x 4096 x 4096 155 -> 141, 1 x 9000 x 4096 320 ->
-// 334, 1 x 4096 x 2048 102 -> 143 (cut), 1 x 1024 x 1024 37 -> 37 (cut), 2048 + 1337 x 4096 129 -> 87, 4 x 512 x 4096 91 -> 49, 12 x 32 x 4096 14
-// -> 13, 16 x 16 x 4096 9.5 -> 15 (whole), 16 x 512 x 4096 164 -> 161, 16 x 512 x 8192 290 -> 314 (whole), 64 x 64 x 2048 42 -> 45 (whole).
+// Whether a step runs with a state per lane.  Its longest sequence takes 0.034 us a token where a CU has one block of 16 channels, 0.048 where
+// it has two; the mean length stands for the longest one, half as much again where there are several, most of whose blocks then end
+// early.  From three blocks a CU on it is ahead at any length, up to 12 waves on a SIMD (49152 channels of sequences), where both forms are
+// bound by issue and eight states per lane need fewer instructions; below 32 tokens staging 64 is most of the work.  The form cut over
+// time takes 27 us, 7 ps per token and channel, and 4 ns per token of a sequence's walk.
+// us, the other form -> a state per lane, 16 states, sequences x tokens x channels: 1 x 256 x 4096 30 -> 12, 1 x 1024 x 1024 37 -> 36, 1 x 1024 x
+// 4096 61 -> 37, 1 x 4096 x 2048 106 -> 134 (cut), 1 x 4096 x 4096 159 -> 134, 1 x 9000 x 4096 325 -> 294, 1 x 1024 x 5120 64 -> 52, 1 x 4096 x
+// 5120 181 -> 196 (cut), 1 x 9000 x 4112 353 -> 431 (cut), 1 x 9000 x 6144 475 -> 455, 1 x 9000 x 8192 590 -> 446, 2048 + 1337 x 4096 129 -> 84,
+// 2 x 3000 x 2560 147 -> 145 and ragged, 5000 + 1000, 161 -> 186 (cut), 4 x 512 x 4096 94 -> 46, 12 x 32 x 4096 14 -> 13, 16 x 16 x 4096 9.5 -> 15
+// (whole), 24 x 700 x 4096 301 -> 332 (whole), 24 x 700 x 2048 219 -> 178.  A sequence that is longer than the guess is the slower for it:
+// 10000 + 2000 x 3072 330 -> 389.
 // Its windows take rows that are no shorter than their columns (where rows repeat or overlap, what stands past a sequence's end is inside the
 // window) and 32-bit offsets into 64 of them; other strides take the other form.
 bool seq_selective_rows(int T_, int B, int C, int N, int ldx, int ldz, int ldb, int ldc, int ldo) {
   if (std::min({ldx, ldz, ldo}) < C || std::min(ldb, ldc) < N || std::max({ldx, ldz, ldb, ldc, ldo}) >= 1 << 24) return false;
   if (N <= 8 || N > 16 || T_ < 32l * B || (long)B * C > 49152) return false;
-  return 0.034f * (B > 1 ? 1.5f : 1.f) * T_ / B < 8.5e-6f * T_ * C + 25.f;
+  const long blocks = (long)B * ((C + 15) / 16);
+  const float len = (B > 1 ? 1.5f : 1.f) * T_ / B;
+  return blocks > 512 || (blocks > 256 && B == 1 ? 0.048f : 0.034f) * len < 27.f + 7e-6f * T_ * C + 0.004f * len;
 }
 
 // Tokens of a segment of the scan cut over time, or 0 where sequences run whole.  Whole, a sequence takes `whole` us a token as
