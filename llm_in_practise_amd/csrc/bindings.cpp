@@ -475,14 +475,17 @@ Tensor lt_linear(Tensor x, Tensor w, optional<Tensor> residual, bool tune) {
   return out;
 }
 
-// y = x·wᵀ + residual of a few rows, bit for bit at::addmm (the same first choice of the heuristic, asked with the same workspace), but
-// without the launch that copies the residual into y first (4.7 µs of the 26 of a 4096 x 12288 product): hipBLASLt takes C and D apart.  No
-// workspace is handed over, so that calls of several streams share nothing; what at::addmm takes beyond this form goes to it.
+// y = x·wᵀ + residual of a few rows without the launch that at::addmm copies the residual into y with first (4.7 µs of the 26 of a 4096 x
+// 12288 product): hipBLASLt takes C and D apart.  The heuristic's first choice, asked with the workspace that at::addmm asks with by default:
+// its bits as long as torch's choice of library, workspace and tuning are the defaults.  No workspace is handed over, so that calls of several
+// streams share nothing.  What at::addmm takes beyond this form, tensors of other devices than the current one among it, goes to it.
 Tensor lt_addmm(Tensor residual, Tensor x, Tensor w) {
   const auto plain = [](const Tensor& t) {
     return t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == 2 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
-  if (plain(residual) && plain(x) && plain(w) && w.is_contiguous() && residual.is_contiguous() && x.is_contiguous() &&
+  int dev = -1;
+  if (plain(residual) && plain(x) && plain(w) && hipGetDevice(&dev) == hipSuccess && x.get_device() == dev && w.get_device() == dev &&
+      residual.get_device() == dev && w.is_contiguous() && residual.is_contiguous() && x.is_contiguous() &&
       x.size(1) == w.size(1) && residual.size(0) == x.size(0) && residual.size(1) == w.size(0) && x.numel() > 0 && w.numel() > 0) {
     const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
     Tensor out = at::empty({M, N}, x.options());

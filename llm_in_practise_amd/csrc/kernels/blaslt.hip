@@ -33,7 +33,8 @@ namespace {
     }                                                                                        \
   } while (0)
 
-using Key = std::tuple<int, int, long, long, long, long, long, long, long, int, long, long, int>;
+// device, transposes, m, n, k, lda, ldb, ldc, batch, strides, whether there is a C
+using Key = std::tuple<int, int, int, long, long, long, long, long, long, int, long, long, int>;
 
 struct Plan {
   hipblasLtMatmulDesc_t desc = nullptr;
@@ -88,7 +89,7 @@ void poll_timings(Plan& p, int reps) {
   p.chosen = bi;
 }
 
-hipblasLtHandle_t g_handle = nullptr;
+std::map<int, hipblasLtHandle_t> g_handles;      // one per device
 std::map<Key, Plan> g_plans;
 std::mutex g_mu;
 
@@ -107,7 +108,7 @@ int tune_reps() {
   return n;
 }
 
-bool make_plan(Plan& p, bool ta, bool tb, long m, long n, long k, long lda, long ldb, long ldc, int batch,
+bool make_plan(hipblasLtHandle_t handle, Plan& p, bool ta, bool tb, long m, long n, long k, long lda, long ldb, long ldc, int batch,
                long sa, long sb, long sc, size_t ws) {
   const hipDataType dt = HIP_R_16BF;
   LT_OK(hipblasLtMatmulDescCreate(&p.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F));
@@ -135,7 +136,7 @@ bool make_plan(Plan& p, bool ta, bool tb, long m, long n, long k, long lda, long
   std::vector<hipblasLtMatmulHeuristicResult_t> res(16);
   int got = 0;
   const hipblasStatus_t hs =
-      hipblasLtMatmulAlgoGetHeuristic(g_handle, p.desc, p.a, p.b, p.c, p.d, pref, 16, res.data(), &got);
+      hipblasLtMatmulAlgoGetHeuristic(handle, p.desc, p.a, p.b, p.c, p.d, pref, 16, res.data(), &got);
   hipblasLtMatmulPreferenceDestroy(pref);
   if (hs != HIPBLAS_STATUS_SUCCESS || got == 0) return false;
   for (int i = 0; i < got && (int)p.cand.size() < n_candidates(); ++i)
@@ -152,19 +153,24 @@ bool make_plan(Plan& p, bool ta, bool tb, long m, long n, long k, long lda, long
 // D = op(A)·op(B) (+ C when C != nullptr; beta = 1), column-major, bf16 in/out, fp32 accumulate.
 // tune: time the heuristic's top candidates on the first calls of the shape and keep the fastest.
 // ws nullptr: the heuristic's first choice, where that needs no workspace (else false).
-// Returns false when hipBLASLt has no plan for the problem (the caller falls back).
+// Operands on the current device.  Returns false when hipBLASLt has no plan for the problem (the caller falls back).
 bool lt_gemm(bool ta, bool tb, long m, long n, long k, const void* A, long lda, const void* B, long ldb,
              const void* C, void* D, long ldc, int batch, long sa, long sb, long sc, void* ws, size_t ws_bytes,
              hipStream_t st, bool tune) {
   Plan* p;
+  hipblasLtHandle_t handle;
+  int dev;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (!g_handle && hipblasLtCreate(&g_handle) != HIPBLAS_STATUS_SUCCESS) return false;
-    const Key key{ta, tb, m, n, k, lda, ldb, ldc, 0, batch, sa, sb, C != nullptr};
+    hipblasLtHandle_t& own = g_handles[dev];
+    if (!own && hipblasLtCreate(&own) != HIPBLAS_STATUS_SUCCESS) return false;
+    handle = own;
+    const Key key{dev, ta, tb, m, n, k, lda, ldb, ldc, batch, sa, sb, C != nullptr};
     auto it = g_plans.find(key);
     if (it == g_plans.end()) {
       Plan np;
-      if (!make_plan(np, ta, tb, m, n, k, lda, ldb, ldc, batch, sa, sb, sc, ws_bytes)) return false;
+      if (!make_plan(handle, np, ta, tb, m, n, k, lda, ldb, ldc, batch, sa, sb, sc, ws_bytes)) return false;
       it = g_plans.emplace(key, np).first;
     }
     p = &it->second;
@@ -199,7 +205,7 @@ bool lt_gemm(bool ta, bool tb, long m, long n, long k, const void* A, long lda, 
     }
   }
   const hipblasStatus_t s =
-      hipblasLtMatmul(g_handle, p->desc, &alpha, A, p->a, B, p->b, &beta, C ? C : D, p->c, D, p->d,
+      hipblasLtMatmul(handle, p->desc, &alpha, A, p->a, B, p->b, &beta, C ? C : D, p->c, D, p->d,
                       &p->cand[idx].algo, ws, ws == nullptr ? 0 : ws_bytes, st);
   if (s != HIPBLAS_STATUS_SUCCESS) {
     fprintf(stderr, "hipBLASLt matmul failed (%d) m=%ld n=%ld k=%ld\n", (int)s, m, n, k);

@@ -320,6 +320,13 @@ def test_product_with_residual_has_addmms_bits(native_ext, M, N, K):
         assert torch.equal(y, torch.addmm(r, x, w.t()))
 
 
+def test_product_with_residual_refuses_another_devices_tensors(native_ext):
+    x, w, r = torch.zeros(1, 64, device=DEV).bfloat16(), torch.zeros(32, 64, device=DEV).bfloat16(), torch.zeros(1, 32, device=DEV).bfloat16()
+    for args in ((r.cpu(), x, w), (r, x.cpu(), w), (r, x, w.cpu())):
+        with pytest.raises(RuntimeError):
+            native_ext.lt_addmm(*args)
+
+
 @pytest.mark.parametrize("F,K,own", [(14336, 128, True), (14352, 128, False), (17408, 5120, False), (32, 4096, True), (32, 4160, False)])
 def test_gated_product_of_wide_weights_stays_with_the_library(native_ext, F, K, own):
     """One launch for gate, up and activation only up to the widths where it is not the slower form."""
