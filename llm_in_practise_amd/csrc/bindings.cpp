@@ -40,6 +40,7 @@ void launch_int4_dequant(const uint8_t*, const float*, const float*, void*, size
 bool lt_gemm(bool, bool, long, long, long, const void*, long, const void*, long, const void*, void*, long, int, long,
              long, long, void*, size_t, hipStream_t, bool);
 void lt_reset();
+int lt_plans();
 void launch_sum_slices(const void*, void*, int, size_t, size_t, hipStream_t);
 bool skinny_norms(int, int, bool);
 void launch_gemm_skinny(const void*, int, const void*, const void*, void*, int, int, int, bool, const void*, float, hipStream_t);
@@ -1819,6 +1820,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("lt_addmm", &lt_addmm);
   m.def("lt_dx", &lt_dx);
   m.def("lt_reset", &lt_reset);
+  m.def("lt_plans", &lt_plans);
   m.def("w4mm", &w4mm, py::arg("x"), py::arg("codes"), py::arg("sc2"), py::arg("N"), py::arg("gs"),
         py::arg("residual") = py::none(), py::arg("nkb") = 0, py::arg("one") = true);
   m.def("w4mm_ok", &w4mm_ok);

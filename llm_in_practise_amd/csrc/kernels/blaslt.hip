@@ -33,8 +33,8 @@ namespace {
     }                                                                                        \
   } while (0)
 
-// device, transposes, m, n, k, lda, ldb, ldc, batch, strides, whether there is a C
-using Key = std::tuple<int, int, int, long, long, long, long, long, long, int, long, long, int>;
+// device, transposes, m, n, k, lda, ldb, ldc, workspace asked with, batch, strides, whether there is a C
+using Key = std::tuple<int, int, int, long, long, long, long, long, long, size_t, int, long, long, int>;
 
 struct Plan {
   hipblasLtMatmulDesc_t desc = nullptr;
@@ -166,7 +166,7 @@ bool lt_gemm(bool ta, bool tb, long m, long n, long k, const void* A, long lda, 
     hipblasLtHandle_t& own = g_handles[dev];
     if (!own && hipblasLtCreate(&own) != HIPBLAS_STATUS_SUCCESS) return false;
     handle = own;
-    const Key key{dev, ta, tb, m, n, k, lda, ldb, ldc, batch, sa, sb, C != nullptr};
+    const Key key{dev, ta, tb, m, n, k, lda, ldb, ldc, ws_bytes, batch, sa, sb, C != nullptr};
     auto it = g_plans.find(key);
     if (it == g_plans.end()) {
       Plan np;
@@ -217,6 +217,12 @@ bool lt_gemm(bool ta, bool tb, long m, long n, long k, const void* A, long lda, 
     p->pending.push_back(timing);
   }
   return true;
+}
+
+// shapes planned so far (tests)
+int lt_plans() {
+  std::lock_guard<std::mutex> lk(g_mu);
+  return (int)g_plans.size();
 }
 
 // reset the per-shape choices (tests / A-B runs)

@@ -1,5 +1,8 @@
 """Decode-attention and sampler kernels vs the PyTorch references (fp32)."""
 import math
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -318,6 +321,26 @@ def test_product_with_residual_has_addmms_bits(native_ext, M, N, K):
         r.copy_(torch.randn(M, N, device=DEV))
         g.replay()
         assert torch.equal(y, torch.addmm(r, x, w.t()))
+
+
+def test_products_of_another_workspace_have_plans_of_their_own():
+    """lt_linear with a workspace of 1 MiB beside lt_addmm, which asks with more: neither takes the other's candidates."""
+    code = """if True:
+        import torch
+        from llm_in_practise_amd.ops._native import native
+        ext, plans = native(), 0
+        for M, N, K in ((1, 4096, 12288), (17, 4096, 4096), (64, 2560, 9728)):
+            x, w, r = (torch.randn(*s, device="cuda").bfloat16() for s in ((M, K), (N, K), (M, N)))
+            want = x.double() @ w.double().t() + r.double()
+            for y in (ext.lt_addmm(r, x, w), *(ext.lt_linear(x, w, r, True) for _ in range(6)), ext.lt_addmm(r, x, w)):
+                assert (y.double() - want).norm() <= 2.0 ** -8 * want.norm()         # (one rounding to bf16, float sums)
+            plans += 2
+            assert ext.lt_plans() == plans
+    """
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    res = subprocess.run([sys.executable, "-c", code], env={**os.environ, "LIPA_LT_WS_MB": "1"}, cwd=root, capture_output=True, text=True,
+                         timeout=110)
+    assert res.returncode == 0, res.stderr[-2000:]
 
 
 def test_product_with_residual_refuses_another_devices_tensors(native_ext):
