@@ -547,6 +547,14 @@ static void check_skinny(const Tensor& x, const Tensor& w) {
               "gemm_skinny: 16-B aligned operands");
 }
 
+// The kernel's offsets into x and into 16 rows of W are 32 bits of bytes: rows further apart come as a copy; false where a row is too long.
+static bool skinny_offsets(Tensor& x) {
+  const int64_t M = x.size(0), K = x.size(1);
+  if (K >= 1 << 25) return false;
+  if (((M - 1) * x.stride(0) + K) * 2 >= 1LL << 32) x = x.contiguous();
+  return true;
+}
+
 // the weight of an RMSNorm in front of the product
 static const void* check_norm(const optional<Tensor>& norm, int64_t M, int64_t K, bool glu) {
   if (!norm.has_value() || !norm->defined()) return nullptr;
@@ -568,8 +576,10 @@ Tensor gemm_skinny(Tensor x, Tensor w, optional<Tensor> residual, optional<Tenso
     TORCH_CHECK(residual->size(0) == M && residual->size(1) == N, "gemm_skinny: residual shape");
     rp = residual->data_ptr();
   }
+  const void* np = check_norm(norm, M, K, false);
+  if (!skinny_offsets(x)) return rp ? at::addmm(*residual, x, w.t()) : at::mm(x, w.t());
   Tensor out = at::empty({M, N}, x.options());
-  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), rp, out.data_ptr(), M, N, K, false, check_norm(norm, M, K, false), (float)eps, stream());
+  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), rp, out.data_ptr(), M, N, K, false, np, (float)eps, stream());
   return out;
 }
 
@@ -578,8 +588,10 @@ Tensor gemm_skinny_swiglu(Tensor x, Tensor w, optional<Tensor> norm, double eps)
   check_skinny(x, w);
   const int64_t M = x.size(0), K = x.size(1), F = w.size(0) / 2;
   TORCH_CHECK(w.size(0) % 32 == 0, "gemm_skinny_swiglu: W [2F, K], F % 16 == 0");
+  const void* np = check_norm(norm, M, K, true);
+  if (!skinny_offsets(x)) return swiglu_fwd(at::mm(x, w.t()));
   Tensor out = at::empty({M, F}, x.options());
-  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), nullptr, out.data_ptr(), M, F, K, true, check_norm(norm, M, K, true), (float)eps, stream());
+  launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), nullptr, out.data_ptr(), M, F, K, true, np, (float)eps, stream());
   return out;
 }
 

@@ -210,6 +210,20 @@ def test_gemm_skinny_rows_do_not_depend_on_their_number(native_ext, N, K):
         assert torch.equal(native_ext.gemm_skinny_swiglu(x[:m], w), h[:m])
 
 
+@pytest.mark.parametrize("M,ld", [(9, 1 << 28), (16, 143165800), (4, 1 << 30), (40, 55063688)])
+def test_gemm_skinny_rows_far_apart(native_ext, M, ld):
+    """Rows that a 32-bit offset in bytes does not reach: the bits of rows side by side, with a norm and without."""
+    torch.manual_seed(M)
+    N, K = 64, 512
+    near, w = torch.randn(M, K, device=DEV).bfloat16(), (torch.randn(2 * N, K, device=DEV) * K ** -0.5).bfloat16()
+    nw = torch.randn(K, device=DEV).bfloat16()
+    x = torch.empty((M - 1) * ld + K, dtype=torch.bfloat16, device=DEV).as_strided((M, K), (ld, 1)).copy_(near)
+    norms = [(None, 0.0)] + [(nw, 1e-6)] * (M <= 4)
+    for norm, eps in norms:
+        assert torch.equal(native_ext.gemm_skinny(x, w[:N], None, norm, eps), native_ext.gemm_skinny(near, w[:N], None, norm, eps))
+        assert torch.equal(native_ext.gemm_skinny_swiglu(x, w, norm, eps), native_ext.gemm_skinny_swiglu(near, w, norm, eps))
+
+
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 @pytest.mark.parametrize("N,K", [(16, 512), (6144, 1024), (128, 4096), (4096, 4096), (8192, 1536), (4608, 3584), (9728, 2560), (2560, 2048)])
 def test_product_of_rows_in_front_of_their_norm(native_ext, M, N, K):
