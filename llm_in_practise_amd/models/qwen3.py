@@ -150,8 +150,10 @@ def _adapted(mods) -> bool:
     return any((isinstance(m, LoraLayer) and not m.merged) or getattr(_leaf_linear(m), "_mlora", None) is not None for m in mods)
 
 
-def _hooked(m: nn.Module) -> bool:
-    return bool(m._forward_pre_hooks or m._forward_hooks or _hooks._global_forward_pre_hooks or _hooks._global_forward_hooks)
+def _own(m: nn.Module, cls: type) -> bool:
+    """Whether a call of ``m`` is ``cls.forward`` and nothing else: no module in its place, no forward of its own, no hook."""
+    return type(m) is cls and "forward" not in m.__dict__ and not (
+        m._forward_pre_hooks or m._forward_hooks or _hooks._global_forward_pre_hooks or _hooks._global_forward_hooks)
 
 
 class Qwen3Attention(nn.Module):
@@ -293,11 +295,12 @@ class Qwen3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
 
     def forward(self, x, cos, sin, B, S, cache=None, start=0, kv_lens=None):
-        few = B * S <= 4                # rows that their products norm themselves (a hook is to see them normed)
-        qkv = self.self_attn.normed_few_rows(x, self.input_layernorm) if few and not _hooked(self.self_attn) else None
+        few = B * S <= 4                # rows that their products norm themselves (what stands in a sublayer's place is to see them normed)
+        qkv = self.self_attn.normed_few_rows(x, self.input_layernorm) if few and _own(self.self_attn, Qwen3Attention) else None
         xn, skip = (x, x) if qkv is not None else rms_norm_residual(x, self.input_layernorm.weight, self.input_layernorm.eps)
-        h = self.self_attn(xn, cos, sin, B, S, residual=skip, cache=cache, start=start, kv_lens=kv_lens, qkv=qkv)
-        act = self.mlp.normed_few_rows(h, self.post_attention_layernorm) if few and not _hooked(self.mlp) else None
+        given = {} if qkv is None else {"qkv": qkv}
+        h = self.self_attn(xn, cos, sin, B, S, residual=skip, cache=cache, start=start, kv_lens=kv_lens, **given)
+        act = self.mlp.normed_few_rows(h, self.post_attention_layernorm) if few and _own(self.mlp, Qwen3MLP) else None
         if act is not None:
             return self.mlp(h, residual=h, h=act)
         hn, skip = rms_norm_residual(h, self.post_attention_layernorm.weight, self.post_attention_layernorm.eps)

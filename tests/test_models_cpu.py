@@ -266,3 +266,49 @@ def test_gradient_checkpointing_kwargs_select_the_form(monkeypatch):
     m = Qwen3ForCausalLM.from_config(qwen3_config("qwen3-tiny"), dtype=torch.float32, seed=3)
     with pytest.raises(ValueError):
         m.gradient_checkpointing_enable({"preserve_rng": True})
+
+
+@pytest.mark.parametrize("form", ["wrapped", "subclass", "patched"])
+@pytest.mark.parametrize("tokens", [1, 4, 9])
+def test_decoder_layer_calls_what_stands_in_its_sublayers_places(form, tokens):
+    """Modules around the sublayers, subclasses and patched forwards with the arguments of the call: they see normed rows, whatever
+    their number."""
+    from llm_in_practise_amd.models import qwen3
+    m = qwen3.Qwen3ForCausalLM.from_config(qwen3.qwen3_config("qwen3-small", num_hidden_layers=2), dtype=torch.float32, device="cpu", seed=0).eval()
+    ids, seen = torch.arange(tokens)[None], []
+    with torch.no_grad():
+        want = m(ids).logits
+
+    def attn(of):
+        def forward(x, cos, sin, B, S, residual=None, cache=None, start=0, kv_lens=None):
+            seen.append(x)
+            return of(x, cos, sin, B, S, residual=residual, cache=cache, start=start, kv_lens=kv_lens)
+        return forward
+
+    def mlp(of):
+        def forward(x, residual=None):
+            seen.append(x)
+            return of(x, residual=residual)
+        return forward
+    layer = m.model.layers[1]
+    for name, wrap in (("self_attn", attn), ("mlp", mlp)):
+        sub = getattr(layer, name)
+        if form == "wrapped":
+            class Around(torch.nn.Module):
+                def __init__(self, of, wrap):
+                    super().__init__()
+                    self.of, self.call = of, wrap(of)
+
+                def forward(self, *a, **kw):
+                    return self.call(*a, **kw)
+            setattr(layer, name, Around(sub, wrap))
+        elif form == "subclass":
+            sub.__class__ = type("Own", (type(sub),), {"forward": lambda self, *a, _w=wrap, _c=type(sub), **kw: _w(
+                lambda *b, **kb: _c.forward(self, *b, **kb))(*a, **kw)})
+        else:
+            sub.forward = wrap(sub.forward)
+    with torch.no_grad():
+        assert torch.equal(m(ids).logits, want)
+    assert len(seen) == 2
+    for x in seen:                                         # (the norms' weights are ones)
+        torch.testing.assert_close(x.pow(2).mean(-1), torch.ones(tokens), rtol=0, atol=1e-3)
