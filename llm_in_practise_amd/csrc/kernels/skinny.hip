@@ -261,13 +261,16 @@ static void launch_rows(const void* X, int ldx, const void* W, const void* res, 
 #define L(CT_, NW_, RING_, GLU_, CUT_, PARTS_)                                                                             \
   gemm_skinny_k<CT_, 1, NW_, RING_, GLU_, CUT_, PARTS_, NORM><<<(N + 15) / 16, 64 * NW_, extra, st>>>(                     \
       (const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, pieces, nrm)
+  if constexpr (!NORM) {                        // (rows that are normed here have 4096 elements at most: 16 pieces of 256)
+    if (!glu && pieces > 16) {
+      if (pieces > 32) L(1, 4, 4, false, TURNS64, 4);
+      else L(1, 8, 3, false, PIECES, 32);
+      return;
+    }
+  }
   if (glu) {
     if (N > 4096 && K % 2048 && K % 128 == 0) L(2, 2, 4, true, TURNS128, 2);
     else L(2, 4, 2, true, TURNS64, 4);
-  } else if (pieces > 32) {
-    L(1, 4, 4, false, TURNS64, 4);
-  } else if (pieces > 16) {
-    L(1, 8, 3, false, PIECES, 32);
   } else if (pieces >= 8 && N <= 4096) {
     L(1, 8, 4, false, PIECES, 16);
   } else {
