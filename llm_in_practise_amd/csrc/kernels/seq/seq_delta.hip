@@ -482,9 +482,11 @@ void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int l
 // 2 x 1000 (1024) 336 -> 358, 4 x 256 203 -> 208.  Of 128 x 64: 32 heads 8 x 512 (1024) 285 -> 236, 16 heads 20 x 400 (1280) 288 -> 240; of
 // 128 x 32, 8 x 512 103 -> 78; of 64 x 64, 4 x 600 (512) 86 -> 80, 40 x 320 (1280) 123 -> 122; of 64 x 128, 16 heads 16 x 512 (2048) 230 -> 238,
 // 64 heads 4 x 300 136 -> 159.  Keys of 192 97 -> 95, of 256 146 -> 151.
+// The first kernel's grid has 65535 slots at most.
 size_t seq_delta_floats(int T_, int B, int H, int dk, int dv, size_t most) {
   if (dk > 128 || T_ < 300l * B || (dv > 64 && (long)B * H * ((dv + 15) / 16) > 256)) return 0;
-  return delta_plan(T_, B, H, dk, dv, most).slots * slot_floats(H, dk, dv);
+  const size_t slots = delta_plan(T_, B, H, dk, dv, most).slots;
+  return slots > 65535 ? 0 : slots * slot_floats(H, dk, dv);
 }
 
 void seq_delta(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g, const float* bpre, float* S,

@@ -75,6 +75,7 @@ void seq_softcap(float*, size_t, float, hipStream_t);
 void seq_selective_scan(int, const void*, int, const float*, const float*, const void*, int, const void*, int, const float*,
                         const float*, const void*, int, float*, void*, int, float, int, int, float*, size_t, SeqDesc, hipStream_t);
 size_t seq_selective_floats(int, int, int, int, size_t);
+size_t seq_delta_floats(int, int, int, int, int, size_t);
 bool seq_selective_rows(int, int, int, int, int, int, int, int, int);
 void seq_gla_scan(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float,
                   float*, float*, int, int, int, SeqDesc, hipStream_t);
@@ -1329,6 +1330,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return (int64_t)seq_block_floats(0, op == "delta", nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H,
                                      (int)dk, (int)dv, (size_t)most);
   }, py::arg("op"), py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS);
+  m.def("delta_block", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most) {      // tokens of a block, 0: token by token
+    if (seq_block_floats(0, true, nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most) == 0) return 0;
+    return seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most) > 0 ? 32 : 16;
+  }, py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS);
   m.def("selective_floats", [](int64_t T, int64_t B, int64_t C, int64_t N, int64_t most) {        // 0: sequences run whole
     return (int64_t)seq_selective_floats((int)T, (int)B, (int)C, (int)N, (size_t)most);
   }, py::arg("T"), py::arg("B"), py::arg("C"), py::arg("N"), py::arg("most") = MOST_WS);

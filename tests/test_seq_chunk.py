@@ -321,10 +321,16 @@ def test_delta_blocks_of_two_tiles(lens, starts, H, G, dk, dv, dt):
     (512, 8, 16, 128, 32, True), (600, 4, 32, 64, 64, True), (512, 16, 16, 64, 128, False), (1000, 2, 4, 192, 128, False),
     (1000, 2, 4, 256, 64, False)])
 def test_delta_blocks_are_long_only_where_they_are_not_slower(L, B, H, dk, dv, long):
-    """Timed shapes on both sides of the choice between blocks of 16 and of 32 tokens: what a slot holds says which it is."""
+    """Timed shapes on both sides of the choice between blocks of 16 and of 32 tokens."""
     from llm_in_practise_amd.ops._native import native_seq
-    floats = native_seq().scan_floats("delta", L * B, B, H, dk, dv)
-    assert floats > 0 and (floats % (H * (49 * dk + 516)) != 0) == long
+    assert native_seq().delta_block(L * B, B, H, dk, dv) == (32 if long else 16)
+
+
+@pytest.mark.gpu
+def test_delta_long_blocks_stay_inside_their_grid():
+    from llm_in_practise_amd.ops._native import native_seq
+    ext, room = native_seq(), 1 << 40
+    assert [ext.delta_block(32 * n, 1, 1, 64, 16, room) for n in (65534, 65535)] == [32, 16]       # (a slot more than whole blocks)
 
 
 @pytest.mark.gpu
