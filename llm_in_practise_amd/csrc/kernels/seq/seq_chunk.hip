@@ -763,7 +763,7 @@ int run_chunks(int T_, int B, int H, int dv) {
 // floats of a run's slot; 0.4 us a token in the token-by-token form
 size_t run_floats(int sc, int H, int dk, int dv) { return (size_t)H * (6 + sc * (4 + 6 * CK + (size_t)dk * (dv + 1))); }
 PiecePlan run_plan(int T_, int B, int H, int dk, int dv, int sc, size_t most) {
-  return plan_pieces(T_, B, CK * sc, run_floats(sc, H, dk, dv), most, 0.4f);
+  return plan_pieces(T_, B, CK * sc, run_floats(sc, H, dk, dv), most < 4 ? 0 : most - 4, 0.4f);      // (4 for the tables' alignment)
 }
 
 template <int NK, bool MLSTM>

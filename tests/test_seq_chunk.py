@@ -656,8 +656,8 @@ def test_rows_that_wide_loads_cannot_take(op, which):
                                           ([4100], 24, 96, 68), ([1280, 256], 16, 128, 192)])
 @pytest.mark.parametrize("bad", [None, 5, 300])
 def test_runs_of_chunks(op, lens, H, dk, dv, bad):
-    """Runs of two and four chunks, whole and cut off in each of them, against the token-by-token kernel; with an infinite value in the
-    first and in a later chunk: it reaches its own column of the outputs behind it and nothing else."""
+    """Runs of two and four chunks, whole and cut off in each of them, against the token-by-token kernel, in one window and in several; with
+    an infinite value in the first and in a later chunk: it reaches its own column of the outputs behind it and nothing else."""
     from llm_in_practise_amd.ops._native import native_seq
     ext = native_seq()
     g = torch.Generator().manual_seed(dk + dv)
@@ -671,8 +671,10 @@ def test_runs_of_chunks(op, lens, H, dk, dv, bad):
         v[bad, dv + 1] = float("inf")                   # head 1, column 1 of the first sequence
     i, f, a, b, skip = rand(T, H), rand(T, H), rand(H), rand(H), rand(H)
     S0, N0 = rand(B, H, dv, dk), rand(B, H, dk)
+    room = ext.scan_floats(op, T, B, H, dk, dv)
+    assert 0 < ext.scan_floats(op, T, B, H, dk, dv, room // 2) <= room // 2        # (several windows)
     res = []
-    for most in (1 << 28, 0):
+    for most in (room, room // 2, 0):
         st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lens, [7 * (j % 2) for j in range(B)], "cuda")
         st["S"].copy_(S0)
         st["N"].copy_(N0)
@@ -682,9 +684,9 @@ def test_runs_of_chunks(op, lens, H, dk, dv, bad):
         else:
             out = ext.mlstm_scan(q, k, v, i, f, a, b + 3, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb.desc, None, most=most)
         res.append([*out, st["S"], st["N"], st["M"]])
-    assert ext.scan_floats(op, T, B, H, dk, dv) > 0
-    for x, y in zip(*res):
-        x, y = x.double(), y.double()
-        assert torch.equal(torch.isfinite(x), torch.isfinite(y))
-        x, y = (torch.nan_to_num(t, 0.0, 0.0, 0.0) for t in (x, y))
-        assert (x - y).norm() <= TOL * y.norm(), ((x - y).norm() / y.norm()).item()
+    for got in res[:2]:
+        for x, y in zip(got, res[2]):
+            x, y = x.double(), y.double()
+            assert torch.equal(torch.isfinite(x), torch.isfinite(y))
+            x, y = (torch.nan_to_num(t, 0.0, 0.0, 0.0) for t in (x, y))
+            assert (x - y).norm() <= TOL * y.norm(), ((x - y).norm() / y.norm()).item()
