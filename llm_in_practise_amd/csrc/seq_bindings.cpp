@@ -1334,7 +1334,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     if (seq_block_floats(0, true, nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most) == 0) return 0;
     return seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most) > 0 ? 32 : 16;
   }, py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS);
-  m.def("selective_floats", [](int64_t T, int64_t B, int64_t C, int64_t N, int64_t most) {        // 0: sequences run whole
+  m.def("selective_floats", [](int64_t T, int64_t B, int64_t C, int64_t N, int64_t most) {        // 0: rows side by side are not cut over time
+    if (seq_selective_rows((int)T, (int)B, (int)C, (int)N, (int)C, (int)C, (int)N, (int)N, (int)C)) return (int64_t)0;
     return (int64_t)seq_selective_floats((int)T, (int)B, (int)C, (int)N, (size_t)most);
   }, py::arg("T"), py::arg("B"), py::arg("C"), py::arg("N"), py::arg("most") = MOST_WS);
   m.def("selective_rows", [](int64_t T, int64_t B, int64_t C, int64_t N) {       // whether a step of rows side by side runs with a state per lane

@@ -58,10 +58,10 @@ def test_expert_tiles_of_many_rows(T, E, F, W):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("E", [1, 7, 130, 300])
+@pytest.mark.parametrize("E", [1, 7, 100, 130, 300])
 @pytest.mark.parametrize("pairs", [1, 4095, 4096, 4097, 12291, 36867])
 def test_order_of_pairs(E, pairs):
-    """Around the turns of 4096 pairs, several to a block where experts are many; identity experts between the others; ids that start at
+    """Around the turns of 4096 pairs, several to a block where experts are many (100 of them: two parts of five turns); identity experts between the others; ids that start at
     an address of 4 bytes more than a multiple of 16."""
     g = torch.Generator().manual_seed(E + pairs)
     F, W = 64, 64

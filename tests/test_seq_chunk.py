@@ -373,12 +373,16 @@ def test_gla_token_that_is_no_number(name, value, t):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("lens,starts,C,N,dt", [([160], [0], 40, 16, torch.bfloat16), ([129, 256, 1, 320], [0, 7, 0, 0], 33, 5, torch.float32),
-                                                ([127, 130], [0, 3], 130, 40, torch.bfloat16), ([200], [0], 64, 200, torch.float32),
-                                                ([1089], [0], 4096, 16, torch.bfloat16), ([60, 64], [0, 0], 64, 16, torch.float32)])
-def test_selective_cut_over_time(lens, starts, C, N, dt):
+@pytest.mark.parametrize("lens,starts,C,N,dt,cut", [
+    ([2100], [0], 40, 16, torch.bfloat16, True), ([129, 256, 1, 320], [0, 7, 0, 0], 33, 5, torch.float32, True),
+    ([127, 130], [0, 3], 130, 40, torch.bfloat16, False), ([200], [0], 64, 200, torch.float32, True),
+    ([2305], [0], 2048, 16, torch.bfloat16, True), ([1409, 1, 1500], [5, 0, 0], 64, 16, torch.float32, True),
+    ([20, 31], [0, 0], 64, 16, torch.float32, False)])
+def test_selective_cut_over_time(lens, starts, C, N, dt, cut):
+    from llm_in_practise_amd.ops._native import native_seq
     g = torch.Generator().manual_seed(C + N)
     T = sum(lens)
+    assert not native_seq().selective_rows(T, len(lens), C, N) and (native_seq().selective_floats(T, len(lens), C, N) > 0) == cut
     x, z, bc = (torch.randn(T, n, generator=g).to(dt) for n in (C, C, 2 * N))
     dtp, dtb, skip = torch.randn(T, C, generator=g), torch.randn(C, generator=g) - 2, torch.randn(C, generator=g)
     a_log = torch.randn(C, N, generator=g)
@@ -497,7 +501,7 @@ def test_selective_takes_a_state_per_lane_where_that_is_faster(T, B, C, N, rows)
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,B,C,N,cut", [
-    (2048, 1, 4096, 16, True), (4096, 4, 4096, 16, True), (6400, 16, 4096, 16, False), (2048, 1, 8192, 32, True),
+    (4096, 1, 2048, 16, True), (9000, 1, 4112, 16, True), (2048, 1, 4096, 16, False), (6400, 16, 4096, 16, False), (2048, 1, 8192, 32, True),
     (6400, 16, 1024, 32, False), (2048, 1, 4096, 64, True), (2048, 1, 8192, 64, False), (2048, 1, 4096, 128, True),
     (4096, 4, 4096, 128, False), (2048, 1, 1024, 256, True), (6400, 16, 1024, 256, False), (4096, 8, 1024, 256, False),
     (256, 1, 8192, 128, False), (256, 1, 4096, 256, False), (300, 1, 65536, 256, False)])
@@ -690,3 +694,49 @@ def test_runs_of_chunks(op, lens, H, dk, dv, bad):
             assert torch.equal(torch.isfinite(x), torch.isfinite(y))
             x, y = (torch.nan_to_num(t, 0.0, 0.0, 0.0) for t in (x, y))
             assert (x - y).norm() <= TOL * y.norm(), ((x - y).norm() / y.norm()).item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["ssd", "mlstm", "delta", "delta-16", "gla", "selective"])
+@pytest.mark.parametrize("B", [64, 65, 129, 200])
+def test_pieces_of_more_sequences_than_a_wave_has_lanes(op, B):
+    """Ragged sequences, some of one token, some idle: every block finds the sequence of its piece; against the token-by-token kernels."""
+    from llm_in_practise_amd.ops._native import native_seq
+    ext = native_seq()
+    g = torch.Generator().manual_seed(B)
+    lens = [1 if b % 9 == 4 else 250 + 37 * b % 411 for b in range(B)]
+    T, H, dk, dv, live = sum(lens), 1, 192 if op == "delta-16" else 64, 32, [int(b % 7 != 3) for b in range(B)]
+
+    def rand(*s, dt=torch.float32):
+        return torch.randn(*s, generator=g).to(dt).cuda()
+    q, k, v = (rand(T, H * n, dt=torch.bfloat16) for n in (dk, dk, dv))
+    k = torch.nn.functional.normalize(k.float().view(T, H, dk), dim=-1).view(T, -1).bfloat16()
+    i, f, a, b, z, zb = rand(T, H), rand(T, H), rand(H), rand(H), rand(T, H * dk), rand(H * dk)
+    C, N = 16, 32
+    sel = [rand(T, C), rand(T, C), rand(C) - 2, rand(T, N), rand(T, N), rand(C, N), rand(C), rand(T, C)]
+    if op == "selective":
+        assert ext.selective_floats(T, B, C, N) > 0
+    elif op.startswith("delta"):
+        assert ext.delta_block(T, B, H, dk, dv) == (16 if op == "delta-16" else 32)
+    else:
+        assert ext.scan_floats(op, T, B, H, dk, dv) > 0
+    tok = torch.repeat_interleave(torch.tensor(live, dtype=torch.bool), torch.tensor(lens)).cuda()
+    res = []
+    for most in (1 << 28, 0):
+        spec = {"S": ((C, N) if op == "selective" else (H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}
+        st, sb = _batch(spec, lens, [3 * (j % 2) for j in range(B)], "cuda", live)
+        for s in st.values():
+            s.fill_(0.25)
+        on = sb.live
+        if op == "ssd":
+            out = [ext.ssd_scan(q, k, v, i.bfloat16(), a - 3, b, a, st["S"], H, H, sb.desc, on, most=most)]
+        elif op == "mlstm":
+            out = ext.mlstm_scan(q, k, v, i, f, a, b + 3, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb.desc, on, most=most)
+        elif op == "gla":
+            out = [ext.gated_linear_scan(q, k, v, z, zb, 16.0, dk ** -0.5, st["S"], H, sb.desc, on, most=most)]
+        elif op == "selective":
+            out = [ext.selective_scan(*sel, st["S"], sb.desc, on, None, 1.0, most=most)]
+        else:
+            out = [ext.delta_scan(q, k, v, torch.sigmoid(z + 3), i, st["S"], H, H, sb.desc, on, most=most)]
+        res.append([*(t[tok] for t in out), *st.values()])
+    _close(res[0], res[1], [str(j) for j in range(len(res[0]))])
