@@ -11,10 +11,11 @@
 // (v_mfma_f32_16x16x4_f32), whose result layout is also its operand layout: the state, u and the outputs never move
 // between lanes.
 //
-// Measured, token by token -> blocks: three sequences of 1500, 700 and 97 tokens, 8 delta heads of 128 x 128: 576 -> 112 us (26
-// for the first kernel, 86 for the walk); eight sequences of 512 tokens, 16 linear-attention heads of 64 x 128: 119 -> 71 us.
+// Measured, token by token -> blocks: 12 sequences of 700 tokens, 8 delta heads of 128 x 128: 431 -> 163 us, of 200 tokens 124 -> 60; eight
+// sequences of 512 tokens, 16 linear-attention heads of 64 x 128: 119 -> 71 us.
 // Error against 64 bits as before (2.1e-7).  Ten inputs a lane two or three blocks ahead gave 2.0 -> 0.94 us a block of the longest
-// sequence.  Long delta prompts that fill the chip at most once run in blocks of 32 tokens (seq_delta.hip).
+// sequence.  Long delta prompts that fill the chip at most once, or whose heads have 64 columns at most, run in blocks of 32 tokens
+// (seq_delta.hip).
 #include "seq_block.h"
 
 #include <type_traits>

@@ -90,9 +90,9 @@ __device__ __forceinline__ void store_state(float* p, int i0, int len, const flo
 // One prompt keeps C / NC blocks busy for as long as it has tokens (0.23 us each), so a step whose sequences do not fill the
 // chip is cut over time (k_selective_walk and the two cut modes): every segment of 32 or 64 tokens first runs from a zero state for
 // the state it leaves and the sum of its step sizes (its decay is e^{A sum dt}), a walk over a sequence's segments turns those
-// into the states in front of the segments, and every segment then runs from its own.  Two prompts of 2048 and 1337 tokens, 4096
-// channels of 16 states: 464 -> 127 us (50 for what segments leave, 16, 73: bound by one
-// quarter-rate exponential per channel, state and token).
+// into the states in front of the segments, and every segment then runs from its own.  One prompt of 4096 tokens, 2048
+// channels of 16 states: 886 -> 103 us (37 for what segments leave, 27, 48 under a profiler: bound by one half-rate exponential per
+// channel, state and token in either pass).  Steps that a state per lane serves better (k_selective_row) go there.
 constexpr int CH = 2;
 enum { WHOLE, LEAVES, FROM };       // a sequence; a segment from zero (state and step sizes); a segment from the state before it
 
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256) void k_selective_scan(const T* __restrict__ x,
 // hands them to the row with the multiplication that reads them (row_newbcast); a lane's 16 read-outs are summed over the row in
 // halves (15 adds for 16 sums), which leaves lane t with token t, in the place of its dt.
 // Bound by issue: a half-rate exponential and four instructions a token and state, three for the sums, three for the staging.  Two
-// prompts of 2048 and 1337 tokens, 4096 channels of 16: 129 -> 87 us (35 ns a token with one wave on a SIMD, 19 a wave with many).  With x, z
+// prompts of 2048 and 1337 tokens, 4096 channels of 16: 129 -> 84 us (33 ns a token with one wave on a SIMD, 19 a wave with many).  With x, z
 // and dt fetched where they are needed (16 rows a load) the address units were busy for 80% of 123 us.
 constexpr int RT = 64, RLD = RT + 4, DLD = RT + 20;      // tokens staged at once; rows of B and C, of dt and dt x in LDS (for the banks)
 
@@ -589,7 +589,8 @@ bool seq_selective_rows(int T_, int B, int C, int N, int ldx, int ldz, int ldb, 
 // Tokens of a segment of the scan cut over time, or 0 where sequences run whole.  Whole, a sequence takes `whole` us a token as
 // long as the chip is not full, and more after that; cut, a step takes about 25 us and `cut` us per token and channel (every exponential
 // twice).  The lengths are not known here: their mean stands for the longest one, so that ragged steps run whole more often than they need.
-// us, whole -> cut, tokens x channels: 16 states 2048 x 4096 455 -> 89, 4 x 1024 x 8192 234 -> 228; 32 states 2048 x 8192 394 -> 224,
+// us, whole -> cut, tokens x channels: 16 states 4096 x 2048 886 -> 103, 9000 x 4112 1953 -> 353; 8 states 2048 x 4096 444 -> 88, 4 x 1024 x
+// 8192 225 -> 227; 32 states 2048 x 8192 394 -> 224,
 // 16 x 400 x 1024 85 -> 113 (whole); 64 states 2048 x 4096 379 -> 210, 2048 x 8192 381 -> 398 (whole); 128 states 2048 x 4096 568 -> 396, 4 x
 // 1024 x 4096 463 -> 757 (whole); 256 states 2048 x 1024 1098 -> 253, 16 x 400 x 1024 364 -> 730 (whole).
 // Segments of 32 tokens where those of 64 would leave the chip idle, else 64: their states pass through memory four times.

@@ -203,7 +203,8 @@ def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
             and x.stride(1) == 1 and base.is_contiguous()):
         # decode-sized q|k|v / o projections: the weight-streaming MFMA kernel (csrc/kernels/skinny.hip) takes 9.1-9.6 µs for
         # 4096 × 4096 and 1-16 rows, residual included, where hipBLASLt takes 17.4 (13.8-15.1 against 14.0-14.4 for 6144 rows of W,
-        # 27 against 29-31 for 8192 × 8192).  A longer K stays with the library, whose sums' order its users have
+        # 27 against 29-31 for 8192 × 8192).  A longer K and more rows stay with the library: this kernel's order of sums there
+        # has not been compared with the library's against 64 bits
         _count("decode")
         y = native().gemm_skinny(x, base, residual)
         return y if ext_a is None else y.addmm_(ext_a, ext_b.t())
