@@ -565,25 +565,26 @@ __global__ __launch_bounds__(256) void k_gla_scan(const T* __restrict__ q, int l
 int seq_selective_max_states() { return 256; }
 int seq_gla_max_dk() { return 256; }
 
-// Whether a step runs with a state per lane.  Its longest sequence takes 0.034 us a token where a CU has one block of 16 channels, 0.048 where
-// it has two; the mean length stands for the longest one, half as much again where there are several, most of whose blocks then end
-// early.  From three blocks a CU on it is ahead at any length, up to 12 waves on a SIMD (49152 channels of sequences), where both forms are
-// bound by issue and eight states per lane need fewer instructions; below 32 tokens staging 64 is most of the work.  The form cut over
-// time takes 27 us, 7 ps per token and channel, and 4 ns per token of a sequence's walk.
-// us, the other form -> a state per lane, 16 states, sequences x tokens x channels: 1 x 256 x 4096 30 -> 12, 1 x 1024 x 1024 37 -> 36, 1 x 1024 x
-// 4096 61 -> 37, 1 x 4096 x 2048 106 -> 134 (cut), 1 x 4096 x 4096 159 -> 134, 1 x 9000 x 4096 325 -> 294, 1 x 1024 x 5120 64 -> 52, 1 x 4096 x
-// 5120 181 -> 196 (cut), 1 x 9000 x 4112 353 -> 431 (cut), 1 x 9000 x 6144 475 -> 455, 1 x 9000 x 8192 590 -> 446, 2048 + 1337 x 4096 129 -> 84,
-// 2 x 3000 x 2560 147 -> 145 and ragged, 5000 + 1000, 161 -> 186 (cut), 4 x 512 x 4096 94 -> 46, 12 x 32 x 4096 14 -> 13, 16 x 16 x 4096 9.5 -> 15
-// (whole), 24 x 700 x 4096 301 -> 332 (whole), 24 x 700 x 2048 219 -> 178.  A sequence that is longer than the guess is the slower for it:
-// 10000 + 2000 x 3072 330 -> 389.
+// Whether a step runs with a state per lane.  Its longest sequence takes 0.034 us a token, 0.048 where it is the only one and some CUs have
+// two of its blocks of 16 channels; the mean length stands for the longest one, half as much again where there are several, most of whose
+// blocks then end early.  Beyond 12 waves on a SIMD (49152 channels of sequences) both forms are bound by issue, and eight states per lane
+// need fewer instructions; below 32 tokens staging 64 is most of the work.  The form cut over time takes 25 us and 8.5 ps per token and
+// channel.  Beside two blocks a CU the two are close: what a state per lane takes more a token, fitted to 94 timed shapes, is 29.6 ns less 4.6
+// ps per channel, and what it saves 22 us; the choice is within 1% of the faster one at all of them.
+// us, the other form -> a state per lane, 16 states, sequences x tokens x channels: 1 x 256 x 4096 30 -> 12, 1 x 1024 x 1024 37 -> 36 (cut), 1 x
+// 1024 x 4096 61 -> 37, 1 x 4096 x 2048 106 -> 134 (cut), 1 x 4096 x 4096 159 -> 134, 1 x 9000 x 4096 325 -> 294, 1 x 9000 x 3072 268 -> 307 (cut),
+// 1 x 1024 x 5120 64 -> 52, 1 x 4096 x 5120 181 -> 196 (cut), 1 x 9000 x 4112 353 -> 431 (cut), 1 x 9000 x 6144 475 -> 455, 1 x 9000 x 8192 590 ->
+// 446, 2048 + 1337 x 4096 129 -> 84, 4 x 512 x 4096 94 -> 46, 12 x 32 x 4096 14 -> 13, 16 x 16 x 4096 9.5 -> 15 (whole), 24 x 700 x 4096 301 ->
+// 332 (whole), 24 x 700 x 2048 219 -> 178.  A sequence that is longer than the guess is the slower for it: 3000 + 3000 x 2560 147 -> 145, but
+// 5000 + 1000 161 -> 186.
 // Its windows take rows that are no shorter than their columns (where rows repeat or overlap, what stands past a sequence's end is inside the
 // window) and 32-bit offsets into 64 of them; other strides take the other form.
 bool seq_selective_rows(int T_, int B, int C, int N, int ldx, int ldz, int ldb, int ldc, int ldo) {
   if (std::min({ldx, ldz, ldo}) < C || std::min(ldb, ldc) < N || std::max({ldx, ldz, ldb, ldc, ldo}) >= 1 << 24) return false;
   if (N <= 8 || N > 16 || T_ < 32l * B || (long)B * C > 49152) return false;
-  const long blocks = (long)B * ((C + 15) / 16);
-  const float len = (B > 1 ? 1.5f : 1.f) * T_ / B;
-  return blocks > 512 || (blocks > 256 && B == 1 ? 0.048f : 0.034f) * len < 27.f + 7e-6f * T_ * C + 0.004f * len;
+  const int blocks = (C + 15) / 16;
+  if (B == 1 && blocks > 256 && blocks <= 512) return T_ * (0.0296f - 4.6e-6f * C) < 22.f;
+  return 0.034f * (B > 1 ? 1.5f : 1.f) * T_ / B < 8.5e-6f * T_ * C + 25.f;
 }
 
 // Tokens of a segment of the scan cut over time, or 0 where sequences run whole.  Whole, a sequence takes `whole` us a token as

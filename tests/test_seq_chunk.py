@@ -493,7 +493,7 @@ def test_selective_token_that_is_no_number(name, value, t):
     (2048, 4, 4096, 16, True), (384, 12, 4096, 16, True), (256, 16, 4096, 16, False), (8192, 16, 8192, 16, False), (1000, 2, 4096, 8, False),
     (1000, 2, 4096, 17, False), (1, 1, 4096, 16, False), (9000, 1, 4096, 16, True), (20000, 1, 4096, 16, True), (9000, 1, 4112, 16, False),
     (1024, 1, 5120, 16, True), (4096, 1, 5120, 16, False), (20000, 1, 5632, 16, False), (9000, 1, 8192, 16, True), (9000, 1, 3072, 16, False),
-    (6000, 2, 2560, 16, False), (20000, 1, 8208, 16, True), (1024, 1, 1024, 16, True)])
+    (20000, 1, 8208, 16, True), (1024, 1, 1024, 16, False), (2048, 1, 2560, 16, False), (2048, 1, 4112, 16, True), (3072, 1, 4608, 16, False)])
 def test_selective_takes_a_state_per_lane_where_that_is_faster(T, B, C, N, rows):
     from llm_in_practise_amd.ops._native import native_seq
     assert native_seq().selective_rows(T, B, C, N) == rows
