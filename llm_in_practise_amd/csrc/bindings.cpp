@@ -969,9 +969,8 @@ Tensor gemm4w_loradx(Tensor dy, Tensor w, optional<Tensor> wscale, int64_t n_w4,
     ld.r[i] = (int)a.size(0);
     ld.ds[i] = (float)(1.0 / (1.0 - ps[i]));
   }
-  // the kernel's prologue always loads the keep bits (a branch without dropout passes an all-ones plane)
-  TORCH_CHECK(masks && masks->defined(), "gemm4w_loradx: keep bits required");
-  {
+  // without masks everything is kept; of several branches one without dropout passes an all-ones plane
+  if (masks && masks->defined()) {
     TORCH_CHECK(masks->scalar_type() == at::kByte && masks->is_contiguous() && masks->numel() >= nbr * M * (N / 8) &&
                     masks->numel() % (M * (N / 8)) == 0, "gemm4w_loradx: keep bits uint8 [P >= nbr, M, N/8]");
     for (int i = 0; i < nbr; ++i) ld.keep[i] = masks->data_ptr<uint8_t>() + (size_t)i * M * (N / 8);

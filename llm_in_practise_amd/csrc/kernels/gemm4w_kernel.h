@@ -705,10 +705,11 @@ __global__ __launch_bounds__(NT, 1) void gemm4w_k(const bf16* __restrict__ A, in
           if (b >= ldx.nbr) break;
           const float* gp = ldx.g[b] + (size_t)m * ldx.ldg + (kq < ldx.r[b] ? kq : 0);
           // keep bits: 16 B = the lane's row over [n0 + wc·BN/2, + 128) (BN/2 ≤ 128 columns)
-          const unsigned char* kp = ldx.keep[b] + (size_t)m * (N >> 3) + min(kb0, (N >> 3) - 16);
           lga[b][i] = *reinterpret_cast<const u32x4*>(gp);
           lgb[b][i] = *reinterpret_cast<const u32x4*>(gp + 4);
-          lkeep[b][i] = *reinterpret_cast<const u32x4*>(kp);
+          lkeep[b][i] = u32x4{~0u, ~0u, ~0u, ~0u};     // (no dropout: everything is kept)
+          if (ldx.keep[b] != nullptr)
+            lkeep[b][i] = *reinterpret_cast<const u32x4*>(ldx.keep[b] + (size_t)m * (N >> 3) + min(kb0, (N >> 3) - 16));
         }
       }
       __builtin_amdgcn_s_waitcnt(WAIT_VM0);

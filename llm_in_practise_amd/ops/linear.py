@@ -16,7 +16,7 @@ projection of the stack runs through.
   - general — anything else (rank > 16, odd widths, > 4 adapters): torch matmuls as an extra K-slice of the base
     GEMM.
   At training sizes the adapters' B term rides inside the forward GEMM as extra MFMA K-steps (``gemm4w_lora``)
-  and the masked input-gradient term inside the dX GEMM's prologue (``gemm4w_loradx``); at decode / small M the
+  and the (masked) input-gradient term inside the dX GEMM's prologue (``gemm4w_loradx``); at decode / small M the
   B term is added into the adapters' column blocks (``lora_apply``).
 
 Reference parity: PEFT ``LoraConfig(r, lora_alpha, lora_dropout, target_modules)``
@@ -156,6 +156,34 @@ def _fast_lora_ok(x, branches) -> bool:
     K = x.shape[1]
     return (K % 128 == 0 and len(branches) <= 4
             and all(br.a.shape[0] <= 16 and (br.c1 - br.c0) % 128 == 0 for br in branches))
+
+
+def _lora_dx(dy, wb, g_list, a_list):
+    """``dY·W + Σ_i g_i·A_i`` (adapters without dropout) in one launch, or None where that is not served: 1-2 adapters
+    of rank 8, 16, 24 or 32 with float ``g``, training-sized M, a base that gemm4w's transposed form takes.  The other form makes the
+    sum an extra K-slice of the product: casts, two concatenations, padding, a transpose and a GEMM, ten launches
+    (160 µs of host time a projection).  That GEMM may split K, which this one cannot, and is ahead by it only where K is deep and
+    the rows are few enough for eight splits: 256 rows of 10240 × 4096 65 -> 77 µs (not taken), of 6144 × 4096 52 -> 50, 402 rows of
+    10240 × 4096 81 -> 79, of 2048 × 1024 39 -> 23, 2048 rows of 6144 × 4096 122 -> 96.  The sum is rounded once: error against 64 bits
+    2.35e-3 -> 1.66e-3."""
+    r = a_list[0].shape[0]
+    if not (1 <= len(g_list) <= 2 and dy.shape[0] >= _MIN_M and wb.shape[1] % 128 == 0 and r % 8 == 0 and r <= 32):
+        return None
+    for g, a in zip(g_list, a_list):
+        if not (g.dtype == torch.float32 and g.shape[1] == a.shape[0] == r and g.stride() == g_list[0].stride() and g.stride(1) == 1
+                and g.stride(0) % 4 == 0 and g.data_ptr() % 16 == 0 and a.dtype == torch.bfloat16 and a.is_contiguous()
+                and a.data_ptr() % 16 == 0):
+            return None
+    w4 = isinstance(wb, NF4Weight)
+    if not (_w4_ok(dy, wb, True) if w4 else _g4w_ok(dy, wb, True)):
+        return None
+    if dy.shape[1] > 8192 and native().gemm4w_plan_info(dy.shape[0], wb.shape[1], dy.shape[1], True, w4)[0] > 4:
+        return None
+    _count("gemm4w-nf4" if w4 else "gemm4w")
+    if w4:
+        codes, sc = wb.g4w_pack()
+        return native().gemm4w_loradx(dy, codes, sc, wb.shape[1], g_list, a_list, None, [0.0] * len(g_list))
+    return native().gemm4w_loradx(dy, wb, None, 0, g_list, a_list, None, [0.0] * len(g_list))
 
 
 class _FusedLinearFn(torch.autograd.Function):
@@ -431,8 +459,10 @@ class _FusedLinearFn(torch.autograd.Function):
                 done_dA = True
             else:
                 assert done_quad is None, "lora_acc_quad ran but the keep-bit dX path did not"
-                ext_a, ext_b = fold_ext()
-                dx = _base_gemm_t(dy, wb, ext_a, ext_b)
+                dx = _lora_dx(dy, wb, g_list, [bf16_view(a, dy.dtype) for a in ab[0::2]]) if nb and len(fold) == nb else None
+                if dx is None:
+                    ext_a, ext_b = fold_ext()
+                    dx = _base_gemm_t(dy, wb, ext_a, ext_b)
                 done_dA = False
         else:
             done_dA = False
@@ -497,10 +527,12 @@ def _multi_backward(ctx, dy, x, weight, xa_list, base, branches, dense, dest):
     if ctx.needs_input_grad[0]:
         wb = ctx.wdq if ctx.wdq is not None else (base if not dense else weight)
         a_list = [bf16_view(ab[2 * i], dy.dtype) for i in range(nb)]
-        if masks is None:    # no dropout: the adapters' g·A as an extra K-slice of the dX GEMM
-            ea = _pad_cols(torch.cat([g.to(dy.dtype) for g in g_list], 1))
-            eb = torch.cat(a_list, 0)
-            dx = _base_gemm_t(dy, wb, ea, F.pad(eb, (0, 0, 0, ea.shape[1] - eb.shape[0])).t().contiguous())
+        if masks is None:    # no dropout: the adapters' g·A in the dX GEMM, or as an extra K-slice of it
+            dx = _lora_dx(dy, wb, g_list, a_list)
+            if dx is None:
+                ea = _pad_cols(torch.cat([g.to(dy.dtype) for g in g_list], 1))
+                eb = torch.cat(a_list, 0)
+                dx = _base_gemm_t(dy, wb, ea, F.pad(eb, (0, 0, 0, ea.shape[1] - eb.shape[0])).t().contiguous())
         else:
             fused = nb <= 2 and wb.shape[1] % 128 == 0 and all(g.shape[1] == g_list[0].shape[1] for g in g_list)
             if fused and isinstance(wb, torch.Tensor) and _g4w_ok(dy, wb, True):

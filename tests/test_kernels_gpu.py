@@ -866,6 +866,34 @@ def test_gemm4w_loradx_epilogue(native_ext, M, Nk, K, r, w4):
         assert rel_err(dx, ref2) < 1e-2
 
 
+@pytest.mark.parametrize("nb", [1, 2])
+@pytest.mark.parametrize("M,N,K,r,w4", [(256, 128, 64, 8, False), (257, 128, 512, 8, True), (402, 1024, 2048, 8, False),
+                                        (300, 640, 1024, 16, False), (511, 768, 192, 32, False), (385, 384, 8256, 24, False),
+                                        (256, 256, 8256, 8, False), (300, 192, 512, 8, False), (300, 256, 512, 4, False)])
+def test_lora_dx_without_dropout(native_ext, M, N, K, r, w4, nb):
+    """dX = dY·W + Σ_i g_i·A_i in one launch (no keep bits), rows, columns and depths at the tiles' edges, against 64 bits; where it
+    is not served (columns no multiple of 128, rank no multiple of 8, a deep K that the other form splits) it says so."""
+    from llm_in_practise_amd.ops.linear import _lora_dx
+    torch.manual_seed(M + r)
+    dy = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (0.05 * torch.randn(K, N, device=DEV)).to(torch.bfloat16)
+    gs = list(torch.randn(nb, M, r, device=DEV))
+    As = [torch.randn(r, N, device=DEV).to(torch.bfloat16) for _ in range(nb)]
+    if w4:
+        w = quantize_nf4(w, 64, True)
+        wd = dequantize_nf4(w, torch.bfloat16)
+    else:
+        wd = w
+    dx = _lora_dx(dy, w, gs, As)
+    if N % 128 or r % 8 or (K > 8192 and native_ext.gemm4w_plan_info(M, N, K, True, w4)[0] > 4):
+        assert dx is None
+        return
+    want = dy.double() @ wd.double() + sum(g.to(torch.bfloat16).double() @ a.double() for g, a in zip(gs, As))
+    # one rounding to bf16 (half of the last of 8 bits: 2^-8 of the value at most) beside float sums
+    assert rel_err(dx, want) < 2 ** -8 + 1e-5
+    assert (dx.double() - want).abs().max() <= (2 ** -8 + 1e-5) * want.abs().max()
+
+
 @pytest.mark.parametrize("M,N,K,g,sym,splits", [(64, 6144, 4096, 128, False, 0), (256, 4096, 4096, 128, True, 1),
                                               (300, 1024, 512, 64, False, 2), (2048, 4096, 12288, 128, False, 0)])
 def test_gemm4w_int4_affine(native_ext, M, N, K, g, sym, splits):
