@@ -5,6 +5,7 @@
 #include <ATen/hip/HIPContext.h>
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <map>
 #include <vector>
 
@@ -27,6 +28,10 @@ void launch_swiglu_bwd(const void*, const void*, void*, int, int, hipStream_t);
 void launch_gelu_fwd(int, const void*, void*, size_t, hipStream_t);
 void launch_gelu_bwd(int, const void*, const void*, void*, size_t, hipStream_t);
 void launch_ce_fwd_bwd(int, void*, const int64_t*, float*, int, int, int, const float*, float, int, hipStream_t);
+void launch_shift_labels(const int64_t*, int64_t*, size_t, int, int64_t, hipStream_t);
+void launch_ce_scale(const int64_t*, float*, int, int, int64_t, hipStream_t);
+void launch_ce_loss(const float*, const float*, float*, int, int, bool, hipStream_t);
+void launch_scale_bf16(const void*, const float*, void*, size_t, hipStream_t);
 void launch_grad_norm(int, const void*, size_t, float*, float*, float, int, hipStream_t);
 void launch_adamw(int, float*, const void*, float*, float*, void*, size_t, float, float, float, float, float, float,
                   float, const float*, const float*, hipStream_t);
@@ -370,6 +375,46 @@ Tensor ce_fwd_bwd(Tensor logits, Tensor labels, int64_t ignore_index, Tensor sca
   launch_ce_fwd_bwd(dtype_code(logits), logits.data_ptr(), labels.contiguous().data_ptr<int64_t>(),
                     loss.data_ptr<float>(), M, V, ignore_index, sc.data_ptr<float>(), 1.f, rows_per_scale, stream());
   return loss;
+}
+
+// labels [.., S] -> the label of the next position, the last one ignored
+Tensor shift_labels(Tensor labels, int64_t ignore_index) {
+  CHECK_CONTIG(labels);
+  TORCH_CHECK(labels.is_cuda() && labels.scalar_type() == at::kLong && labels.dim() >= 1 && labels.size(-1) <= INT_MAX, "labels int64 [.., S]");
+  c10::DeviceGuard guard(labels.device());
+  auto out = at::empty_like(labels);
+  launch_shift_labels(labels.data_ptr<int64_t>(), out.data_ptr<int64_t>(), labels.numel(), (int)labels.size(-1), ignore_index, stream());
+  return out;
+}
+
+// per row group: 1 / (groups · labels that count, at least 1)
+Tensor ce_scale(Tensor labels, int64_t groups, int64_t ignore_index) {
+  CHECK_CONTIG(labels);
+  TORCH_CHECK(labels.is_cuda() && labels.scalar_type() == at::kLong && groups >= 1 && labels.numel() > 0 &&
+                  labels.numel() % groups == 0 && labels.numel() <= INT_MAX, "labels int64, some and as many for each group");
+  auto inv = at::empty({groups}, labels.options().dtype(at::kFloat));
+  launch_ce_scale(labels.data_ptr<int64_t>(), inv.data_ptr<float>(), (int)groups, (int)(labels.numel() / groups), ignore_index, stream());
+  return inv;
+}
+
+// loss (0-dim float, in place) = (add ? loss : 0) + sum over groups of inv[g] · (sum of the group's row losses)
+void ce_loss(Tensor row_loss, Tensor inv, Tensor loss, bool add) {
+  CHECK_CONTIG(row_loss);
+  CHECK_CONTIG(inv);
+  TORCH_CHECK(row_loss.scalar_type() == at::kFloat && inv.scalar_type() == at::kFloat && loss.scalar_type() == at::kFloat &&
+                  loss.numel() == 1 && inv.numel() >= 1 && row_loss.numel() % inv.numel() == 0, "row losses, scales, loss: float");
+  const int M = (int)row_loss.numel();
+  launch_ce_loss(row_loss.data_ptr<float>(), inv.data_ptr<float>(), loss.data_ptr<float>(), M, std::max(1, M / (int)inv.numel()), add, stream());
+}
+
+// x · bf16(s), s one float on the device
+Tensor scale_bf16(Tensor x, Tensor s) {
+  CHECK_BF16(x);
+  CHECK_CONTIG(x);
+  TORCH_CHECK(s.is_cuda() && s.scalar_type() == at::kFloat && s.numel() == 1 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "bf16 rows, one float");
+  auto y = at::empty_like(x);
+  launch_scale_bf16(x.data_ptr(), s.data_ptr<float>(), y.data_ptr(), x.numel(), stream());
+  return y;
 }
 
 // ------------------------------------------------------------------ optimizers
@@ -1793,6 +1838,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("swiglu_bwd", &swiglu_bwd);
   m.def("gelu_fwd", &gelu_fwd);
   m.def("gelu_bwd", &gelu_bwd);
+  m.def("shift_labels", &shift_labels);
+  m.def("ce_scale", &ce_scale);
+  m.def("ce_loss", &ce_loss);
+  m.def("scale_bf16", &scale_bf16);
   m.def("ce_fwd_bwd", &ce_fwd_bwd);
   m.def("dropout_fwd", &dropout_fwd);
   m.def("embedding_fwd", &embedding_fwd, py::arg("weight"), py::arg("ids"), py::arg("oob") = py::none());

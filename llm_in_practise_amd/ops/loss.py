@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 from . import reference as ref
-from ._native import native, use_native, fn_apply
+from ._native import _functorch_active, fn_apply, native, use_native
 from .gemm import _count, _g4w_ok
 
 
@@ -29,14 +29,13 @@ class _FusedLinearCEFn(torch.autograd.Function):
         loss is the mean of their per-micro-batch mean losses (row scale 1/(G·n_valid_g)), so
         the LM head runs as ONE larger GEMM instead of G smaller ones."""
         T = h.shape[0]
-        valid = (labels != ignore_index).view(groups, -1).sum(1).clamp_min(1).float()
-        inv = 1.0 / (valid * groups)                                # [G] per-row-group loss scale
+        inv = native().ce_scale(labels, groups, ignore_index)       # [G] per-row-group loss scale
         rows_g = T // groups
         if chunk % rows_g and groups > 1:
             chunk = rows_g * max(1, chunk // rows_g)               # chunks hold whole micro-batches
         dh = torch.empty_like(h)
         dw = torch.zeros(weight.shape, dtype=torch.float32, device=h.device) if need_wgrad else None
-        loss = torch.zeros((), dtype=torch.float32, device=h.device)
+        loss = torch.empty((), dtype=torch.float32, device=h.device)
         for s in range(0, T, chunk):
             hc = h[s:s + chunk]
             g4w = _g4w_ok(hc, weight, False)
@@ -44,7 +43,7 @@ class _FusedLinearCEFn(torch.autograd.Function):
             logits = native().gemm4w(hc, weight, None, 0, False) if g4w else hc @ weight.t()
             g0, g1 = s // rows_g, (s + hc.shape[0]) // rows_g
             row_loss = native().ce_fwd_bwd(logits, labels[s:s + chunk], ignore_index, inv[g0:g1])
-            loss += (row_loss.view(g1 - g0, -1).sum(1) * inv[g0:g1]).sum()
+            native().ce_loss(row_loss, inv[g0:g1], loss, s > 0)
             dx_g4w = g4w and _g4w_ok(logits, weight, True)
             _count("gemm4w" if dx_g4w else "library")
             if dx_g4w:
@@ -63,7 +62,10 @@ class _FusedLinearCEFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gloss):
         dh, dw = ctx.saved_tensors
-        return ((dh * gloss.to(dh.dtype)), (None if dw is None else (dw * gloss).to(torch.bfloat16)),
+        # (a gradient of this gradient needs the product as torch's op)
+        own = (dh.dtype == torch.bfloat16 and gloss.dtype == torch.float32 and gloss.is_cuda and dh.is_contiguous() and dh.data_ptr() % 16 == 0
+               and not torch.is_grad_enabled() and not _functorch_active())
+        return ((native().scale_bf16(dh, gloss) if own else dh * gloss.to(dh.dtype)), (None if dw is None else (dw * gloss).to(torch.bfloat16)),
                 None, None, None, None, None)
 
 
@@ -86,6 +88,9 @@ def fused_linear_cross_entropy(h: torch.Tensor, weight: torch.Tensor, labels: to
 
 def shift_labels(labels: torch.Tensor, ignore_index: int = -100) -> torch.Tensor:
     """HF causal-LM convention: position t predicts token t+1; last position ignored."""
+    if (labels.is_cuda and labels.dtype == torch.int64 and labels.dim() and labels.is_contiguous() and use_native(labels)
+            and not _functorch_active()):
+        return native().shift_labels(labels, ignore_index)
     out = torch.full_like(labels, ignore_index)
     out[..., :-1] = labels[..., 1:]
     return out

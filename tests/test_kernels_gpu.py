@@ -173,6 +173,39 @@ def test_cross_entropy(native_ext, V):
     assert rel_err(lg, lf.grad) < 2e-2
 
 
+@pytest.mark.parametrize("B,S,groups", [(1, 1, 1), (1, 2, 1), (2, 201, 1), (4, 64, 4), (3, 257, 3), (6, 1023, 2)])
+def test_loss_launches(native_ext, B, S, groups):
+    """Labels moved by one, the groups' scales, the loss of rows in two pieces and the scaled gradient: torch's values, bit for bit but for
+    the loss (a sum in 64 bits, rounded once or twice)."""
+    from llm_in_practise_amd.ops.loss import shift_labels
+    torch.manual_seed(S)
+    labels = torch.randint(0, 50, (B, S), device=DEV)
+    labels[torch.rand(B, S, device=DEV) < 0.3] = -100
+    if groups > 1:
+        labels[:B // groups] = -100                     # a group without a label that counts
+    want = torch.full_like(labels, -100)
+    want[..., :-1] = labels[..., 1:]
+    assert torch.equal(shift_labels(labels), want)
+    assert torch.equal(shift_labels(labels.t()), torch.cat([labels.t()[:, 1:], torch.full_like(labels.t()[:, :1], -100)], 1))
+    flat = want.reshape(-1)
+    inv = native_ext.ce_scale(flat, groups, -100)
+    valid = (flat != -100).view(groups, -1).sum(1).clamp_min(1).float()
+    assert torch.equal(inv, 1.0 / (valid * groups))
+    rows = torch.rand(B * S, device=DEV) * 12
+    loss = torch.full((), float("nan"), device=DEV)
+    n = B * S // groups
+    native_ext.ce_loss(rows[:n], inv[:1], loss, False)
+    if groups > 1:
+        native_ext.ce_loss(rows[n:], inv[1:], loss, True)
+    exact = (rows.double().view(groups, -1).sum(1) * inv.double()).sum()
+    assert abs(loss.double() - exact) <= 2 ** -23 * exact
+    x, f = torch.randn(B * S + 3, device=DEV).bfloat16(), torch.tensor(0.37, device=DEV)
+    assert torch.equal(native_ext.scale_bf16(x, f), x * f.to(torch.bfloat16))
+    with pytest.raises(RuntimeError):
+        native_ext.ce_scale(flat[:0], 1, -100)
+
+
+
 @pytest.mark.parametrize("groups", [1, 2])
 def test_fused_linear_ce_groups(native_ext, groups):
     """LM head + CE in one pass over G fused micro-batches = mean of the per-micro-batch mean
