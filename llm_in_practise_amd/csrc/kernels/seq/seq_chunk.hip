@@ -29,19 +29,6 @@ namespace {
 constexpr int CK = 128;                 // tokens of a chunk (4 waves x 32 queries)
 constexpr double LOG2E = 1.4426950408889634074;
 
-// Two floats as sums of three bf16 numbers each, h + m + l, which hold their 24 bits exactly (an infinity stays one: what it leaves is
-// no number, and is bounded).  By cutting, since packing the upper halves of two words is one instruction.
-struct Split {
-  unsigned h, m, l;
-};
-__device__ __forceinline__ Split split3(float x0, float x1) {
-  const auto upper = [](float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); };
-  const auto pack = [](float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u); };
-  const float r0 = __builtin_amdgcn_fmed3f(x0 - upper(x0), -0x1p120f, 0x1p120f),
-              r1 = __builtin_amdgcn_fmed3f(x1 - upper(x1), -0x1p120f, 0x1p120f);
-  return {pack(x0, x1), pack(r0, r1), pack(r0 - upper(r0), r1 - upper(r1))};
-}
-
 __device__ __forceinline__ double shfl_up_d(double v, int o) {
   const long long b = __double_as_longlong(v);
   const int lo = __shfl_up((int)b, o, 64), hi = __shfl_up((int)(b >> 32), o, 64);

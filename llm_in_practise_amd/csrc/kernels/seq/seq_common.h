@@ -109,6 +109,19 @@ __device__ __forceinline__ float log1p_exp_neg(float a) {
   return 2.f * s * (p * q + 1.f);
 }
 
+// Two floats as sums of three bf16 numbers each, h + m + l, which hold their 24 bits exactly (an infinity stays one: what it leaves is
+// no number, and is bounded).  By cutting, since packing the upper halves of two words is one instruction.
+struct Split {
+  unsigned h, m, l;
+};
+__device__ __forceinline__ Split split3(float x0, float x1) {
+  const auto upper = [](float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); };
+  const auto pack = [](float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u); };
+  const float r0 = __builtin_amdgcn_fmed3f(x0 - upper(x0), -0x1p120f, 0x1p120f),
+              r1 = __builtin_amdgcn_fmed3f(x1 - upper(x1), -0x1p120f, 0x1p120f);
+  return {pack(x0, x1), pack(r0, r1), pack(r0 - upper(r0), r1 - upper(r1))};
+}
+
 // sums of two values over exchanged lanes
 __device__ __forceinline__ float swap32_add(float a, float b) {       // lanes 0-31: sum of a, lanes 32-63: sum of b
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);

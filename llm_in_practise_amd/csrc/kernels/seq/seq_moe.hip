@@ -282,9 +282,10 @@ __global__ __launch_bounds__(64 * NW) void k_route_fused(const T* __restrict__ h
 
 // The same for prompts and up to 16 outputs: a block takes four tokens, a wave a quarter of their columns, so that a router row
 // read from the cache serves four tokens; the 4 x 16 sums over a wave's lanes leave (token, output) in lane 16 token + output, and
-// after the four waves' sums meet in LDS each 16 lanes of the first route their token.  8000 tokens of width 2048, 8 outputs: 41
-// -> 17 us (a block per token read the whole router from L2, 0.6 GB in all, and routed with 64 lanes); moves between lanes through LDS instead
-// of between registers 19.  Bound by issue, 8 waves a SIMD of 800 instructions; 6 blocks a CU spill and take 20 us, 8 32.
+// after the four waves' sums meet in LDS each 16 lanes of the first route their token.  8000 float tokens or rows that the tiles below
+// do not take, width 2048, 8 outputs: 41 -> 17 us (a block per token read the whole router from L2, 0.6 GB in all, and routed with 64
+// lanes); moves between lanes through LDS instead of between registers 19.  Bound by issue, 8 waves a SIMD of 800 instructions; 6 blocks
+// a CU spill and take 20 us, 8 32.
 template <typename T, int NG>
 __global__ __launch_bounds__(256) void k_route_rows(const T* __restrict__ h, int ldh, const float* __restrict__ router,
                                                     const float* __restrict__ corr, int* __restrict__ idx,
@@ -318,6 +319,92 @@ __global__ __launch_bounds__(256) void k_route_rows(const T* __restrict__ h, int
   if (w != 0 || t >= T_) return;
   const float z[1] = {(part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane])};
   if (o >= n - extra && o < n) xout[(size_t)t * extra + o - (n - extra)] = z[0];
+  route_lanes<16, 1>(z, corr, idx + (size_t)t * (top + always), wout + (size_t)t * (top + always), o, n - extra, top, groups, keep,
+                     scale, kind, always);
+}
+
+// The same of bf16 rows on the matrix units: a block takes 16 tokens, a wave every fourth 64 of their columns.  A router weight is the sum of
+// three bf16 numbers (split3: its 24 bits), so a product of 32 columns is three of v_mfma_f32_16x16x32_bf16 with float sums.  Rows come
+// in pieces of 128 bytes and turn into operands through 8 KB of LDS a wave (pieces of row r turned by r / 2: no bank conflicts);
+// operands straight from memory, 64 lines a load, took 12.5 us.  The waves' sums meet in LDS and each 16 lanes route a token.
+template <int U, int NG>                      // a wave's pieces of 64 columns on their way at once; router rows / 4
+__global__ __launch_bounds__(256, 2) void k_route_tiles(const bf16* __restrict__ h, int ldh, const float* __restrict__ router,
+                                                        const float* __restrict__ corr, int* __restrict__ idx,
+                                                        float* __restrict__ wout, int T_, int n, int W, int top, int groups, int keep,
+                                                        float scale, int kind, int extra, float* __restrict__ xout, int always) {
+  __shared__ __attribute__((aligned(16))) bf16 buf[4][4][16 * 64];            // [wave][tokens, the weights' three parts][row][column]
+  __shared__ float part[4][16][16];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, q = lane >> 4, t0 = blockIdx.x * 16;
+  const int r8 = lane >> 3, c8 = lane & 7, r4 = lane >> 4, c4 = lane & 15;    // in memory: rows of 8 or 16 lanes
+  const bf16* x[2];
+  const float* r[NG];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) x[i] = h + (size_t)min(t0 + 8 * i + r8, T_ - 1) * ldh + 8 * c8;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) r[g] = router + (size_t)min(4 * g + r4, n - 1) * W + 4 * c4;
+  const auto piece = [](int row, int p) { return 64 * row + 8 * (p ^ ((row >> 1) & 7)); };
+  f32x4 hi[4], lo[2];                         // (sums of few terms each: fewer roundings at the sum's size)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) hi[i] = lo[i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int c0 = 64 * w; c0 < W; c0 += 256 * U) {
+    bf16x8 a[U][2];
+    f32x4 b[2][NG];
+    const auto weights = [&](int u) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g) b[u & 1][g] = *reinterpret_cast<const f32x4*>(r[g] + min(c0 + 256 * u, W - 64));
+    };
+    weights(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) a[u][i] = *reinterpret_cast<const bf16x8*>(x[i] + min(c0 + 256 * u, W - 64));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u + 1 < U) weights(u + 1);
+      const bool on = c0 + 256 * u < W;       // (past the row: its last columns again, which count as 0)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        u32x4 v = __builtin_bit_cast(u32x4, a[u][i]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = on ? v[e] : 0u;
+        *reinterpret_cast<u32x4*>(buf[w][0] + piece(8 * i + r8, c8)) = v;
+      }
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const f32x4 y = b[u & 1][g];
+        const Split s0 = split3(y[0], y[1]), s1 = split3(y[2], y[3]);
+        bf16* to = buf[w][1] + piece(4 * g + r4, c4 >> 1) + 4 * (c4 & 1);
+        *reinterpret_cast<u32x2*>(to) = u32x2{s0.h, s1.h};
+        *reinterpret_cast<u32x2*>(to + 1024) = u32x2{s0.m, s1.m};
+        *reinterpret_cast<u32x2*>(to + 2048) = u32x2{s0.l, s1.l};
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const auto at = [&](int k) { return *reinterpret_cast<const bf16x8*>(buf[w][k] + piece(li, 4 * i + q)); };
+        const bf16x8 t = at(0);
+        f32x4& big = hi[2 * (u & 1) + i];
+        big = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t, at(1), big, 0, 0, 0);
+        lo[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t, at(3), lo[i], 0, 0, 0);
+        lo[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t, at(2), lo[i], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) part[w][4 * q + i][li] = ((hi[0][i] + hi[1][i]) + (hi[2][i] + hi[3][i])) + (lo[0][i] + lo[1][i]);
+  __syncthreads();
+  const int tt = 4 * w + q, t = t0 + tt, o = li;
+  if (t >= T_) return;
+  float z[1] = {(part[0][tt][o] + part[1][tt][o]) + (part[2][tt][o] + part[3][tt][o])};
+  if (o >= n - extra && o < n) {
+    if (!isfinite(z[0])) {               // (an infinity meets weights' parts that are 0: what it is without parts)
+      z[0] = 0.f;
+      for (int c = 0; c < W; ++c) z[0] += router[(size_t)o * W + c] * (float)h[(size_t)t * ldh + c];
+    }
+    xout[(size_t)t * extra + o - (n - extra)] = z[0];
+  }
   route_lanes<16, 1>(z, corr, idx + (size_t)t * (top + always), wout + (size_t)t * (top + always), o, n - extra, top, groups, keep,
                      scale, kind, always);
 }
@@ -488,6 +575,25 @@ void seq_route_fused(int code, const void* h, int ldh, const float* router, cons
                      int always, hipStream_t st) {
   if (T_ == 0) return;
   const auto fits = [](const void* p, int b) { return ((uintptr_t)p & (b - 1)) == 0; };
+  // us, a block's four tokens (rows above 8 KB and few tokens: a block per token) -> tiles of 16: 256 / 2000 / 8000 tokens of width 2048, 8
+  // outputs 6.8 -> 6.4, 7.3 -> 6.7, 15.5 -> 9.7 (15.2 -> 9.1), 16 outputs 9.5 -> 8.3, 10.5 -> 8.7, 29.7 -> 12.2; 1000 of 8192 17.5 -> 14.8.
+  // Short rows and few outputs give a wave too little to do to make up for the way through LDS: 1000 tokens of width 1024, 8 outputs 4.7 -> 5.2 (not
+  // taken), 8000 8.6 -> 6.5; 4 outputs of 4096 7.7 -> 8.1 (not taken), 8000 17.5 -> 17.0.  Error of the weights against 64 bits as before (0.7e-7).
+  if (T_ >= 256 && ((long)T_ * n >= 40000 || (W > 1024 && n > 4)) && code == 0 && n <= 16 && top + always <= 16 && W % 64 == 0 && ldh % 8 == 0 &&
+      fits(h, 16) && fits(router, 16)) {
+#define ROUTE_TILES(NG_)                                                                                                          \
+  hipLaunchKernelGGL((W <= 1024 ? k_route_tiles<4, NG_> : k_route_tiles<8, NG_>), dim3((T_ + 15) / 16), dim3(256), 0, st, (const bf16*)h, \
+                   ldh, router, corr, idx, w, T_, n, W, top, groups, keep, scale, kind, extra, xout, always)
+    switch ((n + 3) / 4) {
+      case 1: ROUTE_TILES(1); break;
+      case 2: ROUTE_TILES(2); break;
+      case 3: ROUTE_TILES(3); break;
+      default: ROUTE_TILES(4); break;
+    }
+#undef ROUTE_TILES
+    LIPA_CHECK_LAUNCH();
+    return;
+  }
   // (Below 256 tokens a block of 16 waves per token fills the chip better: 8 us at any number up to 200.  Rows above 8 KB are a long
   // way for four waves, which only pays with many tokens: 1000 of width 8192, 12 outputs, 32 against 24 us in bf16, 512 in float 28 against
   // 20; from 2000 on ahead.)

@@ -353,6 +353,45 @@ def test_router_bias(device, n, top, score):
         route_tokens(d(h), d(r), d(b), top, bias=d(b))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,W,n,extra,ld", [(256, 1088, 5, 0, 1088), (257, 1216, 9, 1, 1224), (271, 2048, 16, 0, 2048), (300, 2240, 12, 2, 2248),
+                                            (8000, 64, 8, 1, 64), (10001, 128, 4, 0, 136), (2503, 960, 16, 3, 960), (512, 4160, 8, 0, 4160),
+                                            (300, 2048, 8, 1, 2052), (300, 2056, 8, 0, 2056)])
+def test_router_tiles(T, W, n, extra, ld):
+    """Routing of prompts on the matrix units (the last two: rows that its loads do not take): ids and weights of 64 bits, rows that
+    are a slice of wider ones, and a token with infinities or NaN keeps to itself."""
+    from llm_in_practise_amd.ops.moe import route_tokens
+    g = torch.Generator(device="cuda").manual_seed(T)
+    wide = torch.randn(T, ld, generator=g, device="cuda").bfloat16()
+    h, r = wide[:, :W], torch.randn(n, W, generator=g, device="cuda") * W ** -0.5
+    m, top = n - extra, min(3, n - extra)
+    b = torch.randn(m, generator=g, device="cuda") * 0.2
+
+    def run():
+        return (*route_tokens(h, r, None, top, normalize=True, bias=b, extra=extra, always=1), torch.empty(T, 0, device="cuda"))[:3]
+    idx, w, ex = run()
+    z = h.double() @ r.double().t()
+    p = torch.softmax(z[:, :m] + b.double(), -1).topk(top, -1)
+    # a sum of W float products is off by 2^-24 of its terms' size a few times over: nearer ties may fall either way
+    gap = torch.sort(z[:, :m] + b.double(), -1, descending=True).values
+    sure = ((gap[:, :-1] - gap[:, 1:])[:, :top].amin(-1) > 1e-5) if m > top else torch.ones(T, dtype=torch.bool, device="cuda")
+    assert sure.float().mean() > 0.99
+    assert torch.equal(idx[sure][:, :top].long(), p.indices[sure] if m > top else idx[sure][:, :top].long())
+    got = torch.zeros(T, m, dtype=F64, device="cuda").scatter_(1, idx[:, :top].long(), w[:, :top].double())
+    want = torch.zeros(T, m, dtype=F64, device="cuda").scatter_(1, p.indices, p.values / (p.values.sum(-1, keepdim=True) + 1e-20))
+    assert (got - want)[sure].abs().max() < 4e-6 and bool((idx[:, top] == m).all()) and bool((w[:, top] == 1).all())
+    if extra:
+        assert (ex.double() - z[:, m:]).abs().max() < 4e-6 * z.abs().max()
+    h[5], h[T - 1, 7] = float("nan"), float("inf")
+    idx2, w2, ex2 = run()
+    rest = torch.ones(T, dtype=torch.bool, device="cuda")
+    rest[[5, T - 1]] = False
+    assert torch.equal(idx2[rest], idx[rest]) and torch.equal(w2[rest], w[rest]) and torch.equal(ex2[rest], ex[rest])
+    assert int(idx2.min()) >= 0 and int(idx2[:, :top].max()) < m
+    if extra:
+        assert bool(ex2[5].isnan().all()) and bool((ex2[T - 1] == r[m:, 7].sign() * float("inf")).all())
+
+
 @pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("W", [1, 36, 37, 600, 4100])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
