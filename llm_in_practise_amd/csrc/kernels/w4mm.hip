@@ -198,39 +198,118 @@ __global__ __launch_bounds__(256) void w4mm_reduce_k(const float* __restrict__ p
 // w4mm's slices and sums with all of K in one workgroup: it owns 16·CT columns at a time, its waves take the 128·NKB-deep slices, and
 // the slices' tiles meet in LDS, added in order — the bits of w4mm and its reduce without the second launch, and with the
 // residual or SwiGLU (GLU: CT/2 gate and CT/2 up tiles of W [2N, K], products rounded to bf16 first) in the end.
-//  * ONE: as many waves as slices.  A wave keeps its slice of x in MFMA order, with its sums, in registers and walks column tiles,
-//    the codes of the next tile in flight while it multiplies this one: x is read once per workgroup, not per 16 columns.
-//  * else (long K): 8 waves take the slices of one tile in turns, the next slice's codes and x in flight.
-// x comes in whole rows of 256 B and turns through 4 KB of LDS per wave (as fragments straight from memory, 64 lines a load, the 16
-// rows of 4096 x 12288 took 20 µs, not 16).  Rows past M repeat row M - 1 and are not stored.  4.0 TB/s of codes at 24576 x 4096;
-// smaller products are the chain of launch, x, its turn and the sums: 8.3 µs for 4096 x 4096, 1.6 for each further tile.
-template <int RT, int NKB, int CT, bool GLU, bool ONE, int NT>
-__global__ __launch_bounds__(NT) void w4row_k(const bf16* __restrict__ X, int ldx, const uint8_t* __restrict__ codes,
-                                              const float2* __restrict__ sc, int gs, const bf16* __restrict__ residual,
-                                              bf16* __restrict__ out, int M, int N, int K) {
-  constexpr int CO = GLU ? CT / 2 : CT;
-  extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+//  * as many waves as slices (long K: w4long_k).  A wave keeps its slice of x in MFMA order, with its sums, in registers and walks column tiles:
+//    x is read once per workgroup, not per 16 columns.
+//  * codes and their scales come by LDS-DMA, a unit (16 columns × the slice) a slot of a ring that belongs to one wave: whole pieces of 256
+//    B of a row, no register, and no wait but the wave's own.  As operands straight from memory (16 rows × 64 B and 16 times
+//    a scale an instruction, half of them scales) a wave stood 3 µs in front of its first products until the loads were taken, and as long
+//    again at each tile.  µs, 12 rows, W cold: 24576 × 4096 ended in SwiGLU 20.4 → 16.4 (3.5 TB/s), 6144 × 4096 10.2 → 8.2, 4096 × 4096 8.3 →
+//    6.5 (1.7 of them the launch), 2 × 9728 × 2560 in SwiGLU 13.2 → 12.1, 2 × 3072 × 1024 5.8 → 5.4; 24 rows of 24576 × 4096 24.2 → 19.4.
+//  * x comes in whole rows of 256 B and turns through LDS, in the place of units that are not on their way yet (as fragments straight from
+//    memory, 64 lines a load, the 16 rows of 4096 x 12288 took 20 µs, not 16).  Rows past M repeat row M - 1 and are not stored.
+typedef __attribute__((address_space(3))) void* lds_ptr;
+typedef __amdgpu_buffer_rsrc_t rsrc;
+
+__device__ __forceinline__ rsrc window(const void* base, uint32_t bytes) {
+  const uint64_t p = reinterpret_cast<uint64_t>(base);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)p), hi = __builtin_amdgcn_readfirstlane((uint32_t)(p >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+// 64 lanes x 16 (4) bytes from memory into LDS [dst, ..), lane after lane; M0 is put back
+__device__ __forceinline__ void to_lds16(const rsrc& rs, uint32_t dst, uint32_t voff, uint32_t soff) {
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(dst), "v"(voff), "s"(rs), "s"(soff) : "memory");
+}
+__device__ __forceinline__ void to_lds4(const rsrc& rs, uint32_t dst, uint32_t voff, uint32_t soff) {
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dword %2, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(dst), "v"(voff), "s"(rs), "s"(soff) : "memory");
+}
+// until at most n of a wave's loads are on their way, n rounded down to a multiple of S, or to R · S
+template <int S, int R>
+__device__ __forceinline__ void wait_loads(int n) {
+  if constexpr (R == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else {
+    if (n >= R * S)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R * S) : "memory");
+    else
+      wait_loads<S, R - 1>(n);
+  }
+}
+// Σ of a row over its four lanes (li + 16 q), the rows 4 q .. 4 q + 3 of them in every lane of q
+template <int I>
+__device__ __forceinline__ float row_sum_of(float v) {
+  const int x = __float_as_int(v);
+  int r = __builtin_amdgcn_update_dpp(0, x, 0x150 + I, 0x1, 0xF, false);         // row_newbcast, each into its own row of lanes
+  r = __builtin_amdgcn_update_dpp(r, x, 0x154 + I, 0x2, 0xF, false);
+  r = __builtin_amdgcn_update_dpp(r, x, 0x158 + I, 0x4, 0xF, false);
+  return __int_as_float(__builtin_amdgcn_update_dpp(r, x, 0x15C + I, 0x8, 0xF, false));
+}
+__device__ __forceinline__ f32x4 rows_sums(float v) {
+  const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(s16[0]) + __uint_as_float(s16[1]);
+  const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
+  return f32x4{row_sum_of<0>(v), row_sum_of<1>(v), row_sum_of<2>(v), row_sum_of<3>(v)};
+}
+// codes: chunk c (16 B) of row r of a slice stands in this slot of the row, so that 16 rows of a column of chunks meet every bank once
+template <int NKB>
+__device__ __forceinline__ int turned(int c, int r) { return NKB == 4 ? c ^ (r & 15) : c ^ ((r >> 1) & 7); }
+// a barrier that leaves loads on their way (a fence would wait for them)
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+constexpr int W4_SLICES = 32;                  // of w4long_k, 1 KB of sums each
+
+template <int RT, int NKB, int CT, bool GLU, bool RES>
+__global__ __launch_bounds__(NKB == 2 ? 1024 : 512) void w4row_k(const bf16* __restrict__ X, int ldx, const uint8_t* __restrict__ codes,
+                                                                        const float2* __restrict__ sc, int gs, const bf16* __restrict__ residual,
+                                                                        bf16* __restrict__ out, int M, int N, int K) {
+  constexpr int WAVES = NKB == 2 ? 16 : 8, CO = GLU ? CT / 2 : CT, TILE = CT * RT * 256;       // TILE: floats of one slice's sums
+  constexpr int UB = NKB * (1024 + 128), LOADS = NKB + NKB / 2;              // a unit: bytes of codes and of scales, the loads that bring it
+  constexpr int LDS = 160 * 1024, SUMS = WAVES * TILE * 4;
+  constexpr int RING = WAVES * 4 * UB + SUMS <= LDS ? 4 : 3;
+  constexpr int TURN = NKB / 2;                                             // 128-deep blocks of x that turn at once
+  constexpr int OWN = RING * UB;                                             // a wave's share of LDS
+  constexpr int FIRST = (RING * UB - TURN * 4096) / UB;                      // units on their way while x turns
+  constexpr bool TWICE = WAVES * OWN + 2 * SUMS <= LDS;               // two places for the sums
+  static_assert(FIRST >= 1 && RING * LOADS < 64, "ring");
+  __shared__ __attribute__((aligned(1024))) char smem[WAVES * OWN + (TWICE ? 2 : 1) * SUMS];
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, q = lane >> 4;
-  const int nw = blockDim.x >> 6, KS = K / (128 * NKB), G = K / gs, nt = N / (16 * CO);
-  char* xw = lds_raw + w * 4096;                                     // (ONE: the sums take its place afterwards)
-  char* sums = lds_raw + (ONE ? 0 : nw * 4096);
-  struct Codes {
-    u32x4 c[NKB][CT];
-    float2 s[NKB][CT];
+  // (blockDim and gridDim where they are used are loads, which are waited for with all that is on its way)
+  const int KS = K / (128 * NKB), G = K / gs, nt = N / (16 * CO), per = gs / 128;
+  const int nw = __builtin_amdgcn_readfirstlane(KS), blocks = __builtin_amdgcn_readfirstlane(gridDim.x);
+  char* own = smem + w * OWN;
+  char* xw = own + FIRST * UB;
+  char* sums = smem + WAVES * OWN;
+  const uint32_t ring = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)smem) + w * OWN;
+  const uint32_t row_bytes = (uint32_t)K / 2, rows_w = (uint32_t)(GLU ? 2 * N : N);
+  const rsrc rc = window(codes, rows_w * row_bytes), rs = window(sc, rows_w * (uint32_t)G * 8u);
+  constexpr int CH = 4 * NKB;                    // chunks of a row
+  uint32_t vc[NKB];
+#pragma unroll
+  for (int i = 0; i < NKB; ++i) {
+    const int r = i * (64 / CH) + lane / CH;
+    vc[i] = r * row_bytes + 16 * turned<NKB>(lane % CH, r);
+  }
+  // scales: (scale, c) of block b of row r at dword (r · NKB + b) · 2
+  const int sr = lane / (2 * NKB), sb = lane % (2 * NKB) >> 1;
+  auto fill = [&](int slot, int tile, int ct, int slice) {
+    const uint32_t dst = ring + slot * UB, n0 = (GLU && ct >= CO ? N : 0) + tile * 16 * CO + 16 * (ct % CO);
+#pragma unroll
+    for (int i = 0; i < NKB; ++i) to_lds16(rc, dst + i * 1024, vc[i], n0 * row_bytes + slice * 64 * NKB);
+#pragma unroll
+    for (int i = 0; i < NKB / 2; ++i)
+      to_lds4(rs, dst + NKB * 1024 + i * 256,
+              ((uint32_t)(sr + i * (32 / NKB)) * G + (uint32_t)(slice * NKB + sb) / (uint32_t)per) * 8u + 4u * (lane & 1), n0 * (uint32_t)G * 8u);
   };
   struct Rows {
     u32x4 x[NKB][RT][4];
-  };
-  auto load_codes = [&](Codes& s, int tile, int slice) {
-#pragma unroll
-    for (int b = 0; b < NKB; ++b)
-#pragma unroll
-      for (int t = 0; t < CT; ++t) {
-        const size_t n = (size_t)((GLU && t >= CO ? N : 0) + tile * 16 * CO + 16 * (t % CO) + li);
-        const int kb = slice * NKB + b;
-        s.c[b][t] = *reinterpret_cast<const u32x4*>(codes + n * (K / 2) + 16 * q + kb * 64);
-        s.s[b][t] = sc[n * G + kb * 128 / gs];
-      }
   };
   auto load_rows = [&](Rows& s, int slice) {
 #pragma unroll
@@ -246,129 +325,252 @@ __global__ __launch_bounds__(NT) void w4row_k(const bf16* __restrict__ X, int ld
   f32x4 ax[NKB][RT];                             // Σx of rows 4q .. 4q+3
   auto turn = [&](const Rows& s) {
 #pragma unroll
-    for (int b = 0; b < NKB; ++b)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
+      for (int b0 = 0; b0 < NKB; b0 += TURN) {
         asm volatile("" ::: "memory");           // (a wave's LDS accesses are in order)
 #pragma unroll
-        for (int p = 0; p < 4; ++p)
-          *reinterpret_cast<u32x4*>(xw + (4 * p + q) * 256 + 16 * (li ^ (4 * p + q))) = s.x[b][rt][p];
+        for (int b = 0; b < TURN; ++b)
+#pragma unroll
+          for (int p = 0; p < 4; ++p)
+            *reinterpret_cast<u32x4*>(xw + 4096 * b + (4 * p + q) * 256 + 16 * (li ^ (4 * p + q))) = s.x[b0 + b][rt][p];
         asm volatile("" ::: "memory");
-        float t[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const u32x4 d = *reinterpret_cast<const u32x4*>(xw + li * 256 + 16 * ((4 * q + j) ^ li));
-          const bf16x8 v = __builtin_bit_cast(bf16x8, d);
-          t[j] = 0.f;
+        for (int b = 0; b < TURN; ++b) {
+          float t[4];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) t[j] += (float)v[e];
-          xa[b][rt][j] = __builtin_bit_cast(bf16x8, x_perm(d));
+          for (int j = 0; j < 4; ++j) {
+            const u32x4 d = *reinterpret_cast<const u32x4*>(xw + 4096 * b + li * 256 + 16 * ((4 * q + j) ^ li));
+            const bf16x8 v = __builtin_bit_cast(bf16x8, d);
+            t[j] = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) t[j] += (float)v[e];
+            xa[b0 + b][rt][j] = __builtin_bit_cast(bf16x8, x_perm(d));
+          }
+          ax[b0 + b][rt] = rows_sums((t[0] + t[1]) + (t[2] + t[3]));         // (the pairs of w4mm_k's staging: same bits)
         }
-        float sum = (t[0] + t[1]) + (t[2] + t[3]);                   // (the pairs of w4mm_k's staging: same bits)
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ax[b][rt][i] = __shfl(sum, 4 * q + i, 64);
       }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");               // (units take the place of what has been read)
   };
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](const Codes& s, char* to) {
-    f32x4 acc[CT][RT];
+  // the unit in a slot times the slice of x in registers; next() may fill the slot again
+  auto multiply = [&](int slot, f32x4 (&acc)[RT], auto next) {
+    const char* p = own + slot * UB;
+    u32x4 c[NKB];
+    f32x4 s[NKB / 2];
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+    for (int b = 0; b < NKB; ++b) c[b] = *reinterpret_cast<const u32x4*>(p + li * (64 * NKB) + 16 * turned<NKB>(4 * b + q, li));
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = zero;
+    for (int b = 0; b < NKB / 2; ++b) s[b] = *reinterpret_cast<const f32x4*>(p + NKB * 1024 + (li * NKB + 2 * b) * 8);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    next();
 #pragma unroll
-    for (int b = 0; b < NKB; ++b)
+    for (int rt = 0; rt < RT; ++rt) acc[rt] = zero;
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        bf16x8 bq[4];
+    for (int b = 0; b < NKB; ++b) {
+      bf16x8 bq[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bq[j] = i4_bf16(s.c[b][ct][j]);
-        const float sv = s.s[b][ct].x, cc = s.s[b][ct].y;
+      for (int j = 0; j < 4; ++j) bq[j] = i4_bf16(c[b][j]);
+      const float sv = s[b >> 1][2 * (b & 1)], cc = s[b >> 1][2 * (b & 1) + 1];
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-          f32x4 g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[b][rt][0], bq[0], zero, 0, 0, 0);
+      for (int rt = 0; rt < RT; ++rt) {
+        f32x4 g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[b][rt][0], bq[0], zero, 0, 0, 0);
 #pragma unroll
-          for (int j = 1; j < 4; ++j) g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[b][rt][j], bq[j], g, 0, 0, 0);
+        for (int j = 1; j < 4; ++j) g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[b][rt][j], bq[j], g, 0, 0, 0);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[ct][rt][i] = fmaf(sv, g[i], fmaf(cc, ax[b][rt][i], acc[ct][rt][i]));
-        }
+        for (int i = 0; i < 4; ++i) acc[rt][i] = fmaf(sv, g[i], fmaf(cc, ax[b][rt][i], acc[rt][i]));
       }
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) *reinterpret_cast<f32x4*>(to + ((ct * RT + rt) * 64 + lane) * 16) = acc[ct][rt];
+    }
   };
-  constexpr int TILE = CT * RT * 256;            // floats of one slice's sums
-  auto finish = [&](const char* from, int tile) {                    // element e: y[m = 16·rt + 4q + i][its column]
+  auto row_of = [&](int e) { return 16 * ((e >> 8) % RT) + 4 * ((e >> 6) & 3) + (e & 3); };       // element e: y[m = 16·rt + 4q + i][its column]
+  auto col_of = [&](int e, int tile) { return tile * 16 * CO + 16 * ((e >> 8) / RT) + ((e >> 2) & 15); };
+  // a thread's first residual, on its way under the products
+  const int e0 = min(tid, CO * RT * 256 - 1);
+  auto first_residual = [&](int tile) -> unsigned {
+    return RES ? __builtin_bit_cast(unsigned short, residual[(size_t)min(row_of(e0), M - 1) * N + col_of(e0, tile)]) : 0u;
+  };
+  auto finish = [&](const char* from, int tile, unsigned res) {
     const float* rf = reinterpret_cast<const float*>(from);
-    for (int e = tid; e < CO * RT * 256; e += blockDim.x) {
-      const int i = e & 3, l = (e >> 2) & 63, c = e >> 8, m = 16 * (c % RT) + 4 * (l >> 4) + i;
-      const int n = tile * 16 * CO + 16 * (c / RT) + (l & 15);
+    for (int e = tid; e < CO * RT * 256; e += 64 * nw) {
       float v = 0.f, up = 0.f;
 #pragma unroll 8
       for (int s = 0; s < KS; ++s) {
         v += rf[s * TILE + e];
         if (GLU) up += rf[s * TILE + CO * RT * 256 + e];
       }
-      if (m >= M) continue;
+      if (row_of(e) >= M) continue;
+      const size_t at = (size_t)row_of(e) * N + col_of(e, tile);
       if (GLU) {
         const float gt = (float)(bf16)v, ut = (float)(bf16)up;
         v = gt / (1.f + __expf(-gt)) * ut;
-      } else if (residual) {
-        v += (float)residual[(size_t)m * N + n];
+      } else if (RES) {
+        v += e == tid ? __uint_as_float(res << 16) : (float)residual[at];
       }
-      out[(size_t)m * N + n] = (bf16)v;
+      out[at] = (bf16)v;
     }
   };
-  if constexpr (ONE) {
-    Codes p, r;
-    {
-      Rows x;
-      load_rows(x, w);
-      load_codes(p, blockIdx.x, w);
-      turn(x);
-    }
-    __syncthreads();
-    int buf = 0;
-    auto step = [&](const Codes& now, Codes& next, int tile) {
-      load_codes(next, min(tile + (int)gridDim.x, nt - 1), w);
-      char* to = sums + buf * KS * TILE * 4;
-      multiply(now, to + w * TILE * 4);
-      __syncthreads();                           // (the other buffer is read before the next of these)
-      finish(to, tile);
-      buf ^= 1;
-    };
-    for (int tile = blockIdx.x; tile < nt; tile += 2 * gridDim.x) {
-      step(p, r, tile);
-      if (tile + (int)gridDim.x < nt) step(r, p, tile + gridDim.x);
-    }
-  } else {
-    const int tile = blockIdx.x;
-    Codes p, r;
-    Rows xp, xr;
-    int s = w;
-    if (s < KS) {
-      load_rows(xp, s);
-      load_codes(p, tile, s);
-    }
-    auto step = [&](const Codes& now, const Rows& xn, Codes& next, Rows& xt) {
-      const int n = min(s + nw, KS - 1);
-      load_rows(xt, n);
-      load_codes(next, tile, n);
-      turn(xn);
-      multiply(now, sums + s * TILE * 4);
-      s += nw;
-    };
-    while (s < KS) {
-      step(p, xp, r, xr);
-      if (s >= KS) break;
-      step(r, xr, p, xp);
-    }
-    __syncthreads();
-    finish(sums, tile);
+  auto leave = [&](char* to, int ct, const f32x4 (&acc)[RT]) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) *reinterpret_cast<f32x4*>(to + ((ct * RT + rt) * 64 + lane) * 16) = acc[rt];
+  };
+  const int b0 = blockIdx.x, cnt = (nt - b0 + blocks - 1) / blocks * CT;         // units of this wave
+  int fu = 0, ft = b0, fs = 0;                                                   // the next one to come, its tile and slot
+  auto fill_next = [&] {
+    if (fu >= cnt) return;
+    fill(fs, ft, CT == 1 ? 0 : fu % CT, w);
+    if (CT == 1 || fu % CT == CT - 1) ft += blocks;
+    ++fu;
+    fs = fs + 1 == RING ? 0 : fs + 1;
+  };
+  {
+    Rows x;
+    load_rows(x, w);
+    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));                        // vmcnt(0): what the compiler counts has come
+#pragma unroll
+    for (int i = 0; i < FIRST; ++i) fill_next();
+    turn(x);
   }
+#pragma unroll
+  for (int i = FIRST; i < RING; ++i) fill_next();
+  int u = 0, slot = 0, buf = 0;
+  for (int tile = b0; tile < nt; tile += blocks) {
+    const unsigned res = first_residual(tile);
+    char* to = sums + buf * SUMS;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct, ++u) {
+      f32x4 acc[RT];
+      wait_loads<LOADS, RING - 1>((cnt - 1 - u) * LOADS);
+      multiply(slot, acc, fill_next);
+      slot = slot + 1 == RING ? 0 : slot + 1;
+      leave(to + w * TILE * 4, ct, acc);
+    }
+    lds_barrier();
+    finish(to, tile, res);
+    if (TWICE)
+      buf ^= 1;                                // (the other place is read before the next of these barriers)
+    else if (tile + blocks < nt)
+      lds_barrier();
+  }
+}
+
+// The same sums for long K and up to 16 rows: 12 waves take the slices of one tile in turns.  x comes by LDS-DMA too, 128-deep blocks in a
+// ring of two (XI: loads of four rows each, as many as M needs); a slice's codes and scales wait in LDS until the wave takes them all into
+// registers and the next slice's follow.  4096 x 12288, 12 rows: 16.5 -> 13.1 µs, x through registers, a slice of it on its way, against
+// this.  Bound by what a workgroup does with x beside its one tile (24 slices of its sums, 80 of 160 vector instructions a block) and by the
+// address unit; 8 waves took 14.8, blocks of codes and scales brought one by one 14.1.
+template <int NKB, int XI>
+__global__ __launch_bounds__(XI == 4 ? 640 : 768) void w4long_k(const bf16* __restrict__ X, int ldx, const uint8_t* __restrict__ codes,
+                                                const float2* __restrict__ sc, int gs, const bf16* __restrict__ residual,
+                                                bf16* __restrict__ out, int M, int N, int K) {
+  constexpr int WAVES = XI == 4 ? 10 : 12, RING = 2, XB = 1024 * XI, OWN = RING * XB + NKB * (1024 + 128), CH = 4 * NKB;
+  __shared__ __attribute__((aligned(1024))) char smem[WAVES * OWN + W4_SLICES * 1024];
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, q = lane >> 4, tile = blockIdx.x;
+  const int KS = K / (128 * NKB), G = K / gs, per = gs / 128;
+  const int m = 4 * ((tid >> 6) & 3) + (tid & 3), n = tile * 16 + ((tid >> 2) & 15);            // y[m][n] is this thread's to finish
+  float* sums = reinterpret_cast<float*>(smem + WAVES * OWN);
+  float res = 0.f;
+  if (residual != nullptr) res = (float)residual[(size_t)min(m, M - 1) * N + n];
+  const char* own = smem + w * OWN;
+  const uint32_t xs = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)smem) + w * OWN, cs = xs + RING * XB;
+  const uint32_t row_bytes = (uint32_t)K / 2, n0 = (uint32_t)tile * 16;
+  const rsrc rx = window(X, ((uint32_t)(M - 1) * (uint32_t)ldx + (uint32_t)K) * 2u), rc = window(codes, (uint32_t)N * row_bytes),
+             rs = window(sc, (uint32_t)N * (uint32_t)G * 8u);
+  uint32_t vx[XI], vc[NKB];
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int r = 4 * i + q;
+    vx[i] = (uint32_t)min(r, M - 1) * (uint32_t)ldx * 2u + 16 * (li ^ r);
+  }
+#pragma unroll
+  for (int i = 0; i < NKB; ++i) {
+    const int r = i * (64 / CH) + lane / CH;
+    vc[i] = r * row_bytes + 16 * turned<NKB>(lane % CH, r);
+  }
+  auto fill_x = [&](int place, int block) {
+#pragma unroll
+    for (int i = 0; i < XI; ++i) to_lds16(rx, xs + place * XB + i * 1024, vx[i], block * 256);
+  };
+  // a slice's scales, NKB a row: by 16 (8 ..) bytes where its groups are neighbours
+  const bool wide = NKB == 4 && per == 1 && G % 2 == 0 && ((uintptr_t)sc & 15) == 0;
+  const uint32_t vs = wide ? (uint32_t)((lane >> 1) & 15) * G * 8u + 16 * (lane & 1) : 4u * (lane & 1);
+  const int sr = lane / (2 * NKB), sb = lane % (2 * NKB) >> 1;
+  constexpr int SCALES = NKB / 2;                // loads of them (wide: the second one is left out, and one counted too many)
+  auto fill_codes = [&](int slice) {
+#pragma unroll
+    for (int i = 0; i < NKB; ++i) to_lds16(rc, cs + i * 1024, vc[i], n0 * row_bytes + slice * 64 * NKB);
+    if (wide) {
+      const uint32_t dst = __builtin_amdgcn_readfirstlane(cs + NKB * 1024);        // (an address kept in a vector register has no place in M0)
+      if (lane < 32) to_lds16(rs, dst, vs, (n0 * G + slice * NKB) * 8u);
+    } else {
+#pragma unroll
+      for (int i = 0; i < SCALES; ++i)
+        to_lds4(rs, cs + NKB * 1024 + i * 256, ((uint32_t)(sr + i * (32 / NKB)) * G + (uint32_t)(slice * NKB + sb) / (uint32_t)per) * 8u + vs,
+                n0 * (uint32_t)G * 8u);
+    }
+  };
+  constexpr int C = NKB + 1;                     // (the fewest loads that bring a slice's codes)
+  if (w < KS) {
+    fill_codes(w);
+    fill_x(0, w * NKB);
+    fill_x(1, w * NKB + 1);
+  }
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  for (int slice = w; slice < KS; slice += WAVES) {
+    const int next = slice + WAVES;
+    const bool more = next < KS;
+    if (slice == w || NKB == RING) wait_loads<RING * XI, 1>(RING * XI);         // (later ones are older than x that has been waited for)
+    u32x4 c[NKB];
+    f32x4 s[NKB / 2];
+#pragma unroll
+    for (int b = 0; b < NKB; ++b) c[b] = *reinterpret_cast<const u32x4*>(own + RING * XB + li * (64 * NKB) + 16 * turned<NKB>(4 * b + q, li));
+#pragma unroll
+    for (int b = 0; b < NKB / 2; ++b) s[b] = *reinterpret_cast<const f32x4*>(own + RING * XB + NKB * 1024 + (li * NKB + 2 * b) * 8);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (more) fill_codes(next);
+    f32x4 acc = zero;
+#pragma unroll
+    for (int b = 0; b < NKB; ++b) {
+      // younger: the next block of x, and the next slice's codes where they went out behind this one
+      if (more) {
+        if (b < RING) wait_loads<XI + C, 1>(XI + C); else wait_loads<XI, 1>(XI);
+      } else if (b < NKB - 1) {
+        wait_loads<XI, 1>(XI);
+      } else {
+        wait_loads<1, 0>(0);
+      }
+      const char* p = own + b % RING * XB;
+      u32x4 d[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[j] = *reinterpret_cast<const u32x4*>(p + min(li, 4 * XI - 1) * 256 + 16 * ((4 * q + j) ^ min(li, 4 * XI - 1)));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (b + RING < NKB)
+        fill_x(b % RING, slice * NKB + b + RING);
+      else if (more)
+        fill_x(b % RING, next * NKB + b + RING - NKB);
+      float t[4];
+      f32x4 g = zero;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bf16x8 v = __builtin_bit_cast(bf16x8, d[j]);
+        t[j] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[j] += (float)v[e];
+        g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x_perm(d[j])), i4_bf16(c[b][j]), g, 0, 0, 0);
+      }
+      const f32x4 ax = rows_sums((t[0] + t[1]) + (t[2] + t[3]));
+      const float sv = s[b >> 1][2 * (b & 1)], cc = s[b >> 1][2 * (b & 1) + 1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = fmaf(sv, g[i], fmaf(cc, ax[i], acc[i]));
+    }
+    *reinterpret_cast<f32x4*>(sums + slice * 256 + lane * 4) = acc;
+  }
+  __syncthreads();
+  if (tid >= 256 || m >= M) return;
+  float v = 0.f;
+#pragma unroll 8
+  for (int s = 0; s < KS; ++s) v += sums[s * 256 + tid];
+  if (residual != nullptr) v += res;
+  out[(size_t)m * N + n] = (bf16)v;
 }
 
 // ============================================================================ w4g: 32 < M <= 64
@@ -548,49 +750,54 @@ int w4mm_nkb(int M, int N, int K) {
   return kb % 2 == 0 ? 2 : 1;
 }
 
-// Does w4row_k serve (N: columns of the result)?  Against w4mm_k and its reduce, us in a captured graph at 12 / 24 rows:
-// 6144 x 4096 9.9 / 12.9 (13.4 / 17.1), 4096 x 4096 8.3 / 11.1 (10.1 / 13.3), 24576 x 4096 19.0 / 24.1 (26.9 / 37.0; ended in SwiGLU
-// 19.9 at 12 rows, but 31.5 at 24, where 32 rows of x and two tiles of sums leave the registers).  Where w4mm_k is the better one, us of
-// w4row_k against it:
-//  * one workgroup holds all of x: a single slice is a single wave, too few for the codes of 3 tiles or more (28672 x 512, 12 rows, 11.2
-//    against 6.6); 32 blocks over few tiles are a chain of 16 waves' sums (1024 x 4096, 3 rows, 7.8 against 7.0; ended in SwiGLU
-//    11.1 against 8.9 at 3 rows, 11.3 against 10.8 at 12).
-//  * slices in turns: from the second tile on x is read and turned again (5120 x 5120 11.1 against 10.9 at 3 rows, 27648 x 5120 41.0
-//    against 29.7, 5120 x 13824 25.3 against 20.0; 4096 x 12288 13.8 against 15.2); few tiles of a long K leave the chip idle (1024 x
-//    12288, 16 rows, 13.2 against 10.6; 1024 x 6144 8.4 against 9.7).
+// Does one launch serve (N: columns of the result)?  Against w4mm_k and its reduce, us in a captured graph at 12 / 24 rows:
+// 6144 x 4096 8.4 / 11.6 (13.4 / 17.4), 4096 x 4096 6.7 / 9.5 (11.2 / 14.0), 24576 x 4096 16.0 / 19.8 (27.4 / 37.4; ended in SwiGLU
+// 16.8 at 12 rows, but 31.5 at 24, where 32 rows of x and two tiles of sums left the registers).  Where w4mm_k is the better one, us of
+// one launch against it:
+//  * one workgroup holds all of x: a single slice is a single wave, too few for the codes of 3 tiles or more (28672 x 512, 12 rows, 11.6
+//    against 6.9).  32 blocks over few tiles, a chain of 16 waves' sums, are ahead by now (1024 x 4096, 3 rows, 5.3 against 7.2; ended in
+//    SwiGLU 6.1, 7.0 at 12) and still left to it.
+//  * slices in turns: from the second tile on x is read again (27648 x 5120, 12 rows, 44.5 against 36.4, 5120 x 13824 25.3 against 22.5,
+//    5120 x 5120 13.1 against 13.7; one tile each, 4096 x 12288 13.1, 16 rows 14.7 against 18.8, 2560 x 9728 10.4 against 14.0); few tiles of
+//    a long K leave the chip idle (1024 x 12288, 16 rows, 12.6 against 11.5; 2048 x 12288, 12 rows, 11.8 against 14.3, 1024 x 8192 8.0
+//    against 10.1).
 bool w4row_serves(int M, int N, int K, int nkb, bool glu) {
-  const int KS = K / (128 * nkb), RT = M <= 16 ? 1 : 2, CT = glu ? 2 : 1, tiles = N / 16, per = (tiles + 255) / 256;
+  const int KS = K / (128 * nkb), RT = M <= 16 ? 1 : 2, tiles = N / 16, per = (tiles + 255) / 256;
   const bool one = KS * nkb <= 32;               // (8 waves of 4 blocks or 16 of 2 hold x)
-  const size_t sums = (size_t)KS * CT * RT * 1024, lds = one ? std::max(2 * sums, (size_t)KS * 4096) : sums + 8 * 4096;
-  if (M > (glu ? 16 : 32) || (nkb != 2 && nkb != 4) || ((RT == 2 || glu) && !one) || lds > 65536) return false;
-  return one ? (KS > 1 || per < 3) && !(KS * nkb == 32 && tiles < 160 && (glu || nkb == 2)) : per == 1 && (tiles >= 160 || K <= 6144);
+  if (M > (glu ? 16 : 32) || (nkb != 2 && nkb != 4) || ((RT == 2 || glu) && !one) || (!one && KS > W4_SLICES)) return false;
+  return one ? (KS > 1 || per < 3) && !(KS * nkb == 32 && tiles < 160 && (glu || nkb == 2)) : per == 1 && (tiles >= 128 || K <= 8192);
 }
 
 // One launch of w4row_k, or false where it does not serve (w4mm_k then does).
 bool launch_w4row(const void* X, int ldx, const uint8_t* codes, const float* sc2, int gs, const void* res, void* out, int M,
                   int N, int K, int nkb, bool glu, hipStream_t st) {
   if (!w4row_serves(M, N, K, nkb, glu)) return false;
-  const int KS = K / (128 * nkb), RT = M <= 16 ? 1 : 2, CT = glu ? 2 : 1, tiles = N / 16;
+  if (K > 128 * nkb * (nkb == 4 ? 8 : 16) && ((uint64_t)(M - 1) * ldx + K) * 2 > 0xFFFFFFFFull) return false;       // (w4long_k's offsets into x)
+  const int KS = K / (128 * nkb), RT = M <= 16 ? 1 : 2, tiles = N / 16;
   const bool one = KS * nkb <= 32;
-  const size_t sums = (size_t)KS * CT * RT * 1024, lds = one ? std::max(2 * sums, (size_t)KS * 4096) : sums + 8 * 4096;
   const int per = (tiles + 255) / 256, grid = one ? (tiles + per - 1) / per : tiles;   // tiles of a workgroup: even shares
-#define L(RT_, NKB_, CT_, GLU_, ONE_, NT_)                                                                       \
-  w4row_k<RT_, NKB_, CT_, GLU_, ONE_, NT_><<<grid, ONE_ ? 64 * KS : 512, lds, st>>>(                             \
-      (const bf16*)X, ldx, codes, (const float2*)sc2, gs, (const bf16*)res, (bf16*)out, M, N, K)
+#define L(RT_, NKB_, CT_, GLU_)                                                                                      \
+  do {                                                                                                             \
+    const auto k = res && !GLU_ ? w4row_k<RT_, NKB_, CT_, GLU_, !GLU_> : w4row_k<RT_, NKB_, CT_, GLU_, false>;      \
+    k<<<grid, 64 * KS, 0, st>>>((const bf16*)X, ldx, codes, (const float2*)sc2, gs, (const bf16*)res, (bf16*)out, M, N, K); \
+  } while (0)
+#define LONG(NKB_, XI_)                                                                                             \
+  w4long_k<NKB_, XI_><<<grid, XI_ == 4 ? 640 : 768, 0, st>>>((const bf16*)X, ldx, codes, (const float2*)sc2, gs, (const bf16*)res, (bf16*)out, M, N, K)
   if (one && glu) {
-    if (nkb == 4) L(1, 4, 2, true, true, 512);
-    else L(1, 2, 2, true, true, 1024);
+    if (nkb == 4) L(1, 4, 2, true);
+    else L(1, 2, 2, true);
   } else if (one && RT == 1) {
-    if (nkb == 4) L(1, 4, 1, false, true, 512);
-    else L(1, 2, 1, false, true, 1024);
+    if (nkb == 4) L(1, 4, 1, false);
+    else L(1, 2, 1, false);
   } else if (one) {
-    if (nkb == 4) L(2, 4, 1, false, true, 512);
-    else L(2, 2, 1, false, true, 1024);
+    if (nkb == 4) L(2, 4, 1, false);
+    else L(2, 2, 1, false);
   } else if (nkb == 4) {
-    L(1, 4, 1, false, false, 512);
+    if (M <= 8) LONG(4, 2); else if (M <= 12) LONG(4, 3); else LONG(4, 4);
   } else {
-    L(1, 2, 1, false, false, 512);
+    if (M <= 8) LONG(2, 2); else if (M <= 12) LONG(2, 3); else LONG(2, 4);
   }
+#undef LONG
 #undef L
   LIPA_CHECK_LAUNCH();
   return true;

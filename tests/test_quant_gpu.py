@@ -103,6 +103,22 @@ def test_w4mm_one_launch_has_the_bits_of_the_slices(native_ext, M, nkb, N, K, gs
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("M", [1, 4, 5, 9, 13, 16, 17])
+@pytest.mark.parametrize("nkb,N,K,gs", [(4, 4224, 4096, 128), (4, 640, 4608, 512), (4, 128, 5632, 256), (4, 2048, 12288, 128), (4, 128, 6656, 128),
+                                        (2, 12416, 768, 384), (2, 256, 5376, 128), (2, 2560, 8192, 256), (4, 128, 512, 512), (4, 16512, 1536, 128)])
+def test_w4mm_one_launch_rings(native_ext, nkb, N, K, gs, M):
+    """More units than a ring holds and fewer, ragged shares of slices and tiles, groups of several blocks, an odd number of them, a
+    table that 16-byte loads cannot take, rows of x that are a slice of wider ones or all the same one: the bits of the slices' kernel."""
+    torch.manual_seed(M + K)
+    w = quantize_rtn(torch.randn(N, K, device=DEV), gs, False)
+    table = w.w4mm_table()
+    shifted = torch.empty(table.numel() + 2, device=DEV)[2:].view(table.shape).copy_(table)
+    wide, res = torch.randn(M, K + 24, device=DEV).to(torch.bfloat16), torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    for x, t, r in ((wide[:, 8:K + 8], table, None), (wide[:, 16:K + 16].contiguous(), shifted, res), (wide[:1, 8:K + 8].expand(M, K), table, res)):
+        a, b = (native_ext.w4mm(x, w.codes, t, N, gs, r, nkb, one) for one in (True, False))
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("N,K,gs,sym", [(256, 512, 128, False), (384, 1024, 64, True)])
 def test_int4_dequant_kernel_matches_fp32(native_ext, N, K, gs, sym):
     """The HBM-speed int4 -> bf16 expansion (the W4A16 prefill form) against the fp32 dequantisation."""
