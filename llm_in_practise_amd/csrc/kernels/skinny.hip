@@ -15,45 +15,17 @@
 // µs with fragments from memory → through LDS, W cold, bit for bit the same, at 1 / 12 / 16 rows: 4096 × 4096 9.0 / 10.4 / 11.0 → 9.1 / 9.4 /
 // 9.6, 6144 × 4096 14.4 / 16.2 / 17.1 → 13.8 / 14.5 / 15.1, 1024 × 2048 4.6 / 5.7 / 6.0 → 3.9 / 4.1 / 4.2, 2 × 12288 × 4096 gated 40.7 / 45.6 /
 // 48.7 → 37.6 / 37.0 / 37.3 (5.4 TB/s), 2 × 9728 × 2560 gated 26.0 / 28.7 / 30.1 → 22.9 / 22.7 / 23.1.
-#include "common.h"
+//
+// W's lines, which one wave reads once, come by loads that leave nothing in the caches on their way.  1 / 16 rows, W cold: 4096 × 4096
+// 9.3 / 10.1 → 8.3 / 9.3, 6144 × 4096 13.4 / 14.9 → 12.6 / 14.3, 8192 × 8192 26.5 / 27.6 → 23.9 / 26.1, 4096 × 12288 20.9 / 24.2 → 18.8 / 22.9, 1024 ×
+// 1024 3.5 / 3.8 → 3.2 / 3.5, 2 × 12288 × 4096 gated 35.5 → 32.4 (6.2 TB/s), 2 × 9728 × 2560 gated 22.5 / 23.4 → 20.6 / 22.0.  Where a piece ends in the
+// middle of a line the line is read twice and has to stay: 2560 × 9728 15.8 / 20.6 with, 16.1 / 21.6 without.  (Weights that a caller multiplies with
+// again and again and that fit into L2 or the last cache lose: 6144 × 2560 alone 6.5 → 8.2, 4096 × 4096 7.8 → 7.4.  A model's layers do not fit.)
+#include "lds_dma.h"
 
 using namespace lipa;
 
 namespace {
-
-typedef __attribute__((address_space(3))) void* lds_ptr;
-typedef __amdgpu_buffer_rsrc_t rsrc;
-
-__device__ __forceinline__ rsrc window(const void* base) {
-  const uint64_t p = reinterpret_cast<uint64_t>(base);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)p), hi = __builtin_amdgcn_readfirstlane((uint32_t)(p >> 32));
-  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), 0, 0xFFFFFFFFu, 0x00020000);
-}
-// 64 lanes x 16 bytes from memory into LDS [dst, dst + 1 KB), lane after lane; M0 is put back
-__device__ __forceinline__ void to_lds(const rsrc& rs, uint32_t dst, uint32_t voff, uint32_t soff) {
-  uint32_t keep;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "buffer_load_dwordx4 %2, %3, %4 offen lds\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(keep)
-      : "s"(dst), "v"(voff), "s"(rs), "s"(soff)
-      : "memory");
-}
-// until all but the last `left` units (at most R), of D loads each, have landed
-template <int D, int R>
-__device__ __forceinline__ void wait_units(int left) {
-  if constexpr (R == 0) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  } else {
-    if (left >= R)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R * D) : "memory");
-    else
-      wait_units<D, R - 1>(left);
-  }
-}
 
 // An RMSNorm in front of the product: the norm's weight (null: none).  A row is summed by wpr waves, 8 elements a lane and turn, as the norm's
 // own kernel does (norm.hip), so that the normed rows, rounded to bf16 as it rounds them, are the same bit for bit.
@@ -96,8 +68,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_k(const bf16* __restrict_
   int lp = w, lb = 0;
   auto fill = [&](int slot) {
     const uint32_t dst = base + slot * UB, k = (lp * len + 64 * lb - (lb == per - 1 ? odd : 0)) * 2;
+    if (CUT == PIECES && odd) {                          // (a line of W that two units share is found in L2 the second time)
 #pragma unroll
-    for (int j = 0; j < 2 * CT; ++j) to_lds(GLU && j >= 2 * CO ? ur : wr, dst + j * 1024, wo[j % (2 * CO)], k);
+      for (int j = 0; j < 2 * CT; ++j) to_lds(GLU && j >= 2 * CO ? ur : wr, dst + j * 1024, wo[j % (2 * CO)], k);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2 * CT; ++j) to_lds_once(GLU && j >= 2 * CO ? ur : wr, dst + j * 1024, wo[j % (2 * CO)], k);
+    }
     if (!NORM)
 #pragma unroll
       for (int j = 0; j < 2 * MT; ++j) to_lds(xr, dst + (2 * CT + j) * 1024, xo[j], k);

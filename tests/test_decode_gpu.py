@@ -197,6 +197,22 @@ def test_gemm_skinny_pieces(native_ext, M, N, K):
         assert ((native_ext.gemm_skinny_swiglu(x, w).double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("M", [1, 16, 33])
+@pytest.mark.parametrize("N,K", [(48, 64), (80, 576), (2560, 1216), (96, 4096)])
+def test_gemm_skinny_weight_off_lines(native_ext, M, N, K):
+    """A weight that starts 16 bytes into a line of memory, its pieces in whole units and ending in half of one: every bit as from
+    the weight at a line's start, and nothing of its neighbours."""
+    torch.manual_seed(N + M)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV) * 0.02).to(torch.bfloat16)
+    far = torch.full((N * K + 16,), float("nan"), dtype=torch.bfloat16, device=DEV)
+    off = far[8:8 + N * K].view(N, K).copy_(w)
+    assert w.data_ptr() % 128 == 0 and off.data_ptr() % 128 == 16
+    assert torch.equal(native_ext.gemm_skinny(x, off, None), native_ext.gemm_skinny(x, w, None))
+    if N % 32 == 0:
+        assert torch.equal(native_ext.gemm_skinny_swiglu(x, off), native_ext.gemm_skinny_swiglu(x, w))
+
+
 @pytest.mark.parametrize("N,K", [(512, 8192), (64, 576), (2048, 1984), (6176, 4096), (96, 64)])
 def test_gemm_skinny_rows_do_not_depend_on_their_number(native_ext, N, K):
     """Pieces of 4 units to 32, of half a unit more, of one wave alone: a row's bits are those it has beside 15 others."""
