@@ -190,6 +190,9 @@ __global__ __launch_bounds__(D) void decode_attn_merge_k(const float* __restrict
 //  * the new token's K/V rows are read from the projection output (not the cache), and the
 //    split holding the last key writes them into the cache at pos — no separate scatter
 //    kernel, no read-after-write hazard (no workgroup reads cache[pos] in this launch);
+//  * V's lines, and K's of 64 elements a head, are read once and leave nothing in the caches.  µs before → now, 32 query on 8 heads of 128: 64 x
+//    1024 keys 59.7 → 57.2 (4.75 TB/s), 16 x 4096 59.9 → 57.2, 1 x 1024 10.0; 14 on 2 heads of 64: 64 x 512 11.4 → 10.6, 1 x 4096 9.2 → 8.4.
+//    K of 128 a head, whose lines take two loads, the same way: 64 x 1024 59.9, 1 x 4096 13.3 → 12.5.
 //  * lengths come from pos (int64, len = pos + 1) — no host-side lens tensor.
 __device__ __forceinline__ bf16x4 dec_tr_read(const bf16* p) {
   typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
@@ -260,14 +263,17 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
       const int key = min(t + 16 * kt + li, k1 - 1);
       const bf16* kp = key == len - 1 ? knb : kcb + (size_t)key * rs;
 #pragma unroll
-      for (int s = 0; s < NS; ++s) kr[kt][s] = *reinterpret_cast<const bf16x8*>(kp + 32 * s + 8 * g);
+      for (int s = 0; s < NS; ++s) {
+        const bf16x8* at = reinterpret_cast<const bf16x8*>(kp + 32 * s + 8 * g);
+        kr[kt][s] = D == 64 ? __builtin_nontemporal_load(at) : *at;
+      }
     }
 #pragma unroll
     for (int p = 0; p < VL; ++p) {
       const int ci = p * 64 + lane, row = ci / CH, ch = ci % CH;
       const int key = min(t + row, k1 - 1);
       const bf16* vp = key == len - 1 ? vnb : vcb + (size_t)key * rs;
-      vr[p] = *reinterpret_cast<const bf16x8*>(vp + 8 * ch);
+      vr[p] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(vp + 8 * ch));
     }
     f32x4 sc[2];
 #pragma unroll
