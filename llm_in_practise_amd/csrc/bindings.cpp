@@ -48,6 +48,7 @@ void lt_reset();
 int lt_plans();
 void launch_sum_slices(const void*, void*, int, size_t, size_t, hipStream_t);
 bool skinny_norms(int, int, bool);
+void launch_rows_swiglu(const void*, int, const void*, void*, int, int, int, hipStream_t);
 void launch_gemm_skinny(const void*, int, const void*, const void*, void*, int, int, int, bool, const void*, float, hipStream_t);
 bool w4mm_supported(int, int, int, int);
 bool w4g_supported(int, int, int, int);
@@ -637,6 +638,17 @@ Tensor gemm_skinny_swiglu(Tensor x, Tensor w, optional<Tensor> norm, double eps)
   if (!skinny_offsets(x)) return swiglu_fwd(at::mm(x, w.t()));
   Tensor out = at::empty({M, F}, x.options());
   launch_gemm_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), nullptr, out.data_ptr(), M, F, K, true, np, (float)eps, stream());
+  return out;
+}
+
+// h [M, F] = silu(x Wgᵀ) (x Wuᵀ) of 17 to 64 rows, every sum one chain over K (csrc/kernels/rows.hip): w [2F, K]
+Tensor rows_swiglu(Tensor x, Tensor w) {
+  check_skinny(x, w);
+  const int64_t M = x.size(0), K = x.size(1), F = w.size(0) / 2;
+  TORCH_CHECK(M > 16 && K % 128 == 0 && K < 1 << 24 && w.size(0) % 32 == 0, "rows_swiglu: 17 to 64 rows, W [2F, K], F%16, K%128");
+  skinny_offsets(x);
+  Tensor out = at::empty({M, F}, x.options());
+  launch_rows_swiglu(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), M, F, K, stream());
   return out;
 }
 
@@ -1875,6 +1887,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("nf4_dequant_fast", &nf4_dequant_fast);
   m.def("skinny_norms", &skinny_norms);
   m.def("gemm_skinny", &gemm_skinny, py::arg("x"), py::arg("w"), py::arg("residual"), py::arg("norm") = py::none(), py::arg("eps") = 0.0);
+  m.def("rows_swiglu", &rows_swiglu);
   m.def("gemm_skinny_swiglu", &gemm_skinny_swiglu, py::arg("x"), py::arg("w"), py::arg("norm") = py::none(), py::arg("eps") = 0.0);
   m.def("lt_linear", &lt_linear);
   m.def("lt_addmm", &lt_addmm);

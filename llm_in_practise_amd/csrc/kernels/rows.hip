@@ -1,0 +1,132 @@
+// The gated product of 17 to 64 decode rows, h[M, F] = silu(x·Wgᵀ)·(x·Wuᵀ) of W [2 F, K] (gate above up), every sum one chain of MFMA over K in
+// order: the bits of the library's product of such widths and of the activation behind it.  What bounds it is W from memory and, beside it, x,
+// which every workgroup reads whole: a workgroup takes as many columns as leave one workgroup for each CU, four tiles of 16 at most.
+//
+//  * a workgroup of 8 waves walks K in stages of 128: its rows of W and x come by LDS-DMA, 4 rows × 256 B an instruction (chunk c of row r
+//    in slot c ^ r % 16: the fragments' reads are free of conflicts), into a ring of all LDS.  The waves share out a stage's loads and meet in one
+//    barrier per stage, at which the stage read before it is free for the next loads.  (Stages of 64: 47.4 µs where these take 45.8.)
+//  * W's lines leave nothing in the caches on their way (45.8 → 39.9 µs).
+//  * wave w multiplies row tile w % 4 with the gate columns, or, from wave 4 on, with the up columns; they meet in LDS at the end.
+//
+// µs at 17 / 32 / 48 / 64 rows, W cold, the library's product and the activation → here: 2 × 12288 × 4096 48.0 / 47.7 / 48.2 / 49.0 → 39.6 / 38.9 /
+// 39.1 / 39.9 (5.1 TB/s), 2 × 14336 × 4096 56 / 56 / 62 / 55 → 46 / 46 / 46 / 47, 2 × 9728 × 2560 27.4 / 29.0 / 29.5 / 30.0 → 20.7 / 21.9 / 21.7 / 23.1,
+// 2 × 3072 × 1024 14 → 6.4 / 6.4 / 7.2 / 7.0.  Without the gated end it takes as long as the library's 6144 × 4096 (17.4 and 17.8 µs at 64 rows).
+#include "lds_dma.h"
+
+using namespace lipa;
+
+namespace {
+
+constexpr int ring_of(int stage) { return 163840 / stage < 8 ? 163840 / stage : 8; }
+
+// MT: row tiles, CO: column tiles of the result
+template <int MT, int CO>
+__global__ __launch_bounds__(512) void rows_swiglu_k(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W, bf16* __restrict__ out,
+                                                     int M, int N, int K) {
+  constexpr int CT = 2 * CO, PIECES = 4 * (CT + MT), D = (PIECES + 7) / 8, SB = PIECES * 1024, RING = ring_of(SB);
+  static_assert(RING >= 3 && (RING - 2) * D < 64 && MT * CO * 1024 <= RING * SB, "ring");
+  __shared__ __attribute__((aligned(1024))) char smem[RING * SB];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16 * CO, r4 = lane >> 4;
+  const rsrc wr = window(W + (size_t)n0 * K), ur = window(W + (size_t)(N + n0) * K), xr = window(X);
+  const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)smem);
+  // pieces of a stage: 4 rows each, W's column tiles first (gate, up), then x; wave w brings pieces w, w + 8, ..
+  const bool full = w + 8 * (D - 1) < PIECES;
+  uint32_t vo[D];
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    const int p = min(w + 8 * j, PIECES - 1), ch = (li ^ (4 * (p & 3) + r4)) * 16;
+    vo[j] = p < 4 * CT ? (uint32_t)min(4 * (p >= 4 * CO ? p - 4 * CO : p) + r4, N - 1 - n0) * (uint32_t)K * 2 + ch
+                       : (uint32_t)min(4 * (p - 4 * CT) + r4, M - 1) * (uint32_t)ldx * 2 + ch;
+  }
+  auto fill = [&](int slot, int stage) {
+    const uint32_t dst = base + slot * SB + w * 1024, k = stage * 256;
+#pragma unroll
+    for (int j = 0; j < D; ++j)
+      if (j < D - 1 || full) {
+        const int p = w + 8 * j;
+        if (p >= 4 * CT) to_lds(xr, dst + j * 8192, vo[j], k);
+        else if (p >= 4 * CO) to_lds_once(ur, dst + j * 8192, vo[j], k);
+        else to_lds_once(wr, dst + j * 8192, vo[j], k);
+      }
+  };
+  const int stages = K / 128, mt = w & 3, c0 = w < 4 ? 0 : CO;
+  const bool work = mt < MT;
+  f32x4 acc[CO];
+#pragma unroll
+  for (int t = 0; t < CO; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < RING - 1; ++s)
+    if (s < stages) fill(s, s);
+  for (int s = 0, slot = 0; s < stages; ++s) {
+    const int left = min(stages - 1 - s, RING - 2);
+    if (full) wait_units<D, RING - 2>(left); else wait_units<D - 1, RING - 2>(left);
+    __builtin_amdgcn_s_barrier();                          // the stage is here, and the one before it is read
+    asm volatile("" ::: "memory");
+    if (s + RING - 1 < stages) fill(slot == 0 ? RING - 1 : slot - 1, s + RING - 1);
+    if (work) {
+      const char* p = smem + slot * SB;
+#pragma unroll
+      for (int h2 = 0; h2 < 2; ++h2) {
+        bf16x8 a[2][CO], b[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int c = li * 256 + ((8 * h2 + 4 * h + g) ^ li) * 16;
+          b[h] = *reinterpret_cast<const bf16x8*>(p + (CT + mt) * 4096 + c);
+#pragma unroll
+          for (int t = 0; t < CO; ++t)
+            a[h][t] = *reinterpret_cast<const bf16x8*>(p + (c0 + t) * 4096 + c);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int t = 0; t < CO; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][t], b[h], acc[t], 0, 0, 0);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    slot = slot + 1 == RING ? 0 : slot + 1;
+  }
+  const int m = 16 * mt + li;
+  f32x4(*up)[CO][64] = reinterpret_cast<f32x4(*)[CO][64]>(smem);
+  __syncthreads();
+  if (work && w >= 4)
+#pragma unroll
+    for (int t = 0; t < CO; ++t) up[mt][t][lane] = acc[t];
+  __syncthreads();
+  if (!work || w >= 4 || m >= M) return;
+#pragma unroll
+  for (int t = 0; t < CO; ++t) {
+    const int n = n0 + 16 * t + 4 * g;
+    if (n >= N) continue;
+    const f32x4 u = up[mt][t][lane];
+    bf16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {                        // (rounded like the products they would have been)
+      const float gt = (float)(bf16)acc[t][e], ut = (float)(bf16)u[e];
+      o[e] = (bf16)(gt / (1.f + __expf(-gt)) * ut);
+    }
+    *reinterpret_cast<bf16x4*>(out + (size_t)m * N + n) = o;
+  }
+}
+
+}  // namespace
+
+// F: columns of the result, a multiple of 16 (W has 2 F rows); K a multiple of 128; 17 <= M <= 64
+void launch_rows_swiglu(const void* X, int ldx, const void* W, void* out, int M, int F, int K, hipStream_t st) {
+  const int tiles = F / 16, t = tiles <= 256 ? 1 : tiles <= 512 ? 2 : tiles <= 768 ? 3 : 4;
+#define L(MT_, CO_) rows_swiglu_k<MT_, CO_><<<(tiles + t - 1) / t, 512, 0, st>>>((const bf16*)X, ldx, (const bf16*)W, (bf16*)out, M, F, K)
+#define LT(MT_)               \
+  do {                        \
+    if (t == 1) L(MT_, 1);    \
+    else if (t == 2) L(MT_, 2); \
+    else if (t == 3) L(MT_, 3); \
+    else L(MT_, 4);           \
+  } while (0)
+  if (M > 48) LT(4);
+  else if (M > 32) LT(3);
+  else LT(2);
+#undef LT
+#undef L
+  LIPA_CHECK_LAUNCH();
+}

@@ -116,24 +116,28 @@ class _SkinnySwiGLUFn(torch.autograd.Function):
     """(No backward: skinny_swiglu leaves what needs a gradient to the differentiable ops.)"""
     @staticmethod
     def forward(ctx, x, w, norm=None, eps=0.0):
-        return native().gemm_skinny_swiglu(x, w, norm, eps)
+        return native().gemm_skinny_swiglu(x, w, norm, eps) if x.shape[0] <= 16 else native().rows_swiglu(x, w)
 
 
 def skinny_swiglu(x: torch.Tensor, gu_base, norm=None, eps: float = 0.0) -> torch.Tensor | None:
-    """``silu(x·W_gateᵀ)·(x·W_upᵀ)`` of up to 16 decode rows in one launch (csrc/kernels/skinny.hip), or None where that kernel
-    does not serve: a bf16 [gate | up] weight, no gradient.  The products are rounded to bf16 before the activation, as the
-    separate kernels round them.  Library and activation → here, µs at 1 / 16 rows: 4096 → 2 × 12288 48 / 49 → 38 / 37, 2560 → 2 × 9728
-    48 / 48 → 23 / 23, 1024 → 2 × 3072 10.1 / 10.1 → 5.1 / 5.2, 4096 → 2 × 14336 67 / 69 → 45 / 46.  Wider and deeper weights, and more rows,
-    stay with the library's product.  With ``norm`` the rows stand in front of the RMSNorm of that weight, which the launch forms bit for
-    bit as its own kernel does (:func:`~.gemm.norms_rows`; else None): 39.7 → 37.3 µs, 25.8 → 22 and 6.8 → 5.4 at 1 row, norm included."""
+    """``silu(x·W_gateᵀ)·(x·W_upᵀ)`` of up to 64 decode rows in one launch (csrc/kernels/skinny.hip up to 16, rows.hip beyond them), or None
+    where they do not serve: a bf16 [gate | up] weight, no gradient.  The products are rounded to bf16 before the activation, as the
+    separate kernels round them.  Library and activation → here, µs at 1 / 16 / 17 / 64 rows: 4096 → 2 × 12288 48 / 49 / 48 / 49 → 32 / 33 / 40 / 40,
+    2560 → 2 × 9728 48 / 48 / 27 / 30 → 21 / 22 / 21 / 23, 1024 → 2 × 3072 10 / 10 / 14 / 14 → 4.6 / 4.9 / 6.4 / 7.0, 4096 → 2 × 14336 67 / 69 / 56 / 55 →
+    40 / 41 / 46 / 47.  (skinny.hip takes 37 / 48 at 17 / 64 rows of 2 × 12288, in an order of sums that is not the library's there.)  Wider and
+    deeper weights, and more rows, stay with the library's product.  With ``norm`` the rows stand in front of the RMSNorm of that weight, which
+    the launch forms bit for bit as its own kernel does (:func:`~.gemm.norms_rows`; else None): 39.7 → 37.3 µs, 25.8 → 22 and 6.8 → 5.4 at 1 row
+    before the weight's loads passed the caches by, norm included."""
     x2 = x.reshape(-1, x.shape[-1])
     if (torch.is_grad_enabled() and x.requires_grad) or not (
             x.is_cuda and x.dtype == torch.bfloat16 and isinstance(gu_base, torch.Tensor) and gu_base.dtype == torch.bfloat16
-            and not gu_base.requires_grad and gu_base.is_contiguous() and 1 <= x2.shape[0] <= 16 and x2.stride(1) == 1
+            and not gu_base.requires_grad and gu_base.is_contiguous() and 1 <= x2.shape[0] <= 64 and x2.stride(1) == 1
             and x2.shape[1] <= 4096 and gu_base.shape[0] <= 2 * 14336
-            and x2.stride(0) % 8 == 0 and x2.shape[1] % 64 == 0 and gu_base.shape[0] % 32 == 0
+            and x2.stride(0) % 8 == 0 and x2.shape[1] % (64 if x2.shape[0] <= 16 else 128) == 0 and gu_base.shape[0] % 32 == 0
             and x2.data_ptr() % 16 == 0 and gu_base.data_ptr() % 16 == 0 and not force_reference()):
         return None
+    if x2.shape[0] > 16 and gu_base.shape[0] < 6144 and x2.shape[1] > 1024:
+        return None         # (a stage costs what it costs for a tile: 2 × 1024 × 4096, 48 rows, 15.7 µs against 14.3; 2 × 256 × 512 4.3 and 8.7)
     if norm is not None and not norms_rows(x2, norm, gu_base, True):
         return None
     _count("decode")

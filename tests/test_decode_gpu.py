@@ -197,6 +197,33 @@ def test_gemm_skinny_pieces(native_ext, M, N, K):
         assert ((native_ext.gemm_skinny_swiglu(x, w).double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 49, 64])
+@pytest.mark.parametrize("F,K", [(16, 128), (80, 640), (4112, 384), (8208, 256), (12320, 256), (14336, 128)])
+def test_rows_swiglu(native_ext, M, F, K):
+    """The gated product of more rows, one to four column tiles a workgroup with and without a remainder, fewer stages than the ring holds
+    and more: against 64 bits (each sum of K products in float within (K + 1) half-ulps of the absolute sum, rounded to bf16, then the
+    activation, rounded again; |d silu| <= 1.1), for rows of x side by side and far apart, and a saturated gate."""
+    torch.manual_seed(F + M)
+    far = torch.randn(M, K + 24, device=DEV).to(torch.bfloat16)
+    far[M - 1] = 100.0 * far[M - 1].sign()
+    w = (torch.randn(2 * F, K, device=DEV) * 0.02).to(torch.bfloat16)
+    w[3] = -1.0 * far[M - 1, :K].sign()                        # gate -100 K: its silu is 0
+    x = far[:, :K].contiguous()
+    exact = x.double() @ w.double().t()
+    slack = 2 * (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    g, u = exact[:, :F], exact[:, F:]
+    eg, eu = 2.0 ** -8 * g.abs() + slack[:, :F], 2.0 ** -8 * u.abs() + slack[:, F:]
+    want = g * torch.sigmoid(g) * u
+    bound = 1.1 * eg * (u.abs() + eu) + (g * torch.sigmoid(g)).abs() * eu + 2.0 ** -7 * want.abs() + 1e-6
+    got = native_ext.rows_swiglu(x, w)
+    assert ((got.double() - want).abs() <= bound).all() and got[M - 1, 3] == 0
+    assert torch.equal(native_ext.rows_swiglu(far[:, :K], w), got)
+    big = x.clone()
+    big[:, 5] = float("inf")                                   # infinities and what becomes of them, as from the separate kernels
+    h = native_ext.swiglu_fwd(big @ w.t())
+    assert torch.equal(torch.isnan(native_ext.rows_swiglu(big, w)), torch.isnan(h))
+
+
 @pytest.mark.parametrize("M", [1, 16, 33])
 @pytest.mark.parametrize("N,K", [(48, 64), (80, 576), (2560, 1216), (96, 4096)])
 def test_gemm_skinny_weight_off_lines(native_ext, M, N, K):
