@@ -180,6 +180,25 @@ def normed_rows(x: torch.Tensor, weight, eps: float, base) -> torch.Tensor | Non
     return fn_apply(_NormedRowsFn, x, weight, eps, base)
 
 
+def _rows_ok(x, base, residual) -> bool:
+    """Whether the decode products (csrc/kernels/skinny.hip) take more than 16 rows, or a K beyond 8192, of a narrow bf16 weight: where they
+    are the faster ones, and where their order of sums is the library's or the weight is short (a chain over all of K would round worse).
+    Library → here in µs, W cold, residual included: 4096 × 12288 at 1 / 16 / 32 rows 21.4 / 21.5 / 26.1 → 18.0 / 20.3 / 26.0 (48: 31.0 and 32.9),
+    2560 × 9728 18.1 / 16.0 / 20.1 → 12.1 / 15.0 / 19.3, 2048 × 16384 at 16 / 24 23.0 / 23.8 → 22.0 / 26.2, 4096 × 4096 at 17 / 32 13.7 / 13.0 → 9.3 / 9.9,
+    2560 × 4096 12.5 / 12.4 → 7.8 / 9.0; at 17 / 64, 4096 × 1024 11.4 / 11.7 → 3.9 / 5.3, 1024 × 3072 11.6 / 11.9 → 6.1 / 9.8, 4096 × 3072 12.3 / 16.1 →
+    6.8 / 10.8.  5120 × 4096 at 17 / 32: 15.4 / 14.7 and 14.2 / 16.4."""
+    M, K = x.shape
+    N = base.shape[0]
+    if not (x.is_cuda and M <= 64 and N <= 4096 and N % 16 == 0 and K % 64 == 0 and x.dtype == base.dtype == torch.bfloat16
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and base.is_contiguous() and x.data_ptr() % 16 == 0 and base.data_ptr() % 16 == 0
+            and (residual is None or (residual.dtype == torch.bfloat16 and residual.shape == (M, N) and residual.is_contiguous()
+                                      and residual.data_ptr() % 16 == 0))):
+        return False
+    if K > 8192:
+        return K % 128 == 0 and K < 1 << 24 and M <= (32 if N > 2048 else 16)
+    return 16 < M <= (64 if K < 4096 else 32)
+
+
 def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
     if isinstance(base, NF4Weight):
         if x.shape[0] <= 8 and base.kernel_ok():   # decode: weight-streaming GEMV, no MFMA tile
@@ -200,11 +219,10 @@ def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
     M, K = x.shape
     N = base.shape[0]
     if (x.is_cuda and M <= 16 and N <= 8192 and K <= 8192 and N % 16 == 0 and K % 64 == 0 and x.stride(0) % 8 == 0
-            and x.stride(1) == 1 and base.is_contiguous()):
-        # decode-sized q|k|v / o projections: the weight-streaming MFMA kernel (csrc/kernels/skinny.hip) takes 9.1-9.6 µs for
-        # 4096 × 4096 and 1-16 rows, residual included, where hipBLASLt takes 17.4 (13.8-15.1 against 14.0-14.4 for 6144 rows of W,
-        # 27 against 29-31 for 8192 × 8192).  A longer K and more rows stay with the library: this kernel's order of sums there
-        # has not been compared with the library's against 64 bits
+            and x.stride(1) == 1 and base.is_contiguous()) or _rows_ok(x, base, residual):
+        # decode-sized q|k|v / o projections: the weight-streaming MFMA kernel (csrc/kernels/skinny.hip) takes 8.3-9.3 µs for
+        # 4096 × 4096 and 1-16 rows, residual included, where hipBLASLt takes 15.3 (12.6-14.2 against 15 for 6144 rows of W,
+        # 24 against 29-31 for 8192 × 8192)
         _count("decode")
         y = native().gemm_skinny(x, base, residual)
         return y if ext_a is None else y.addmm_(ext_a, ext_b.t())

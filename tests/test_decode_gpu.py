@@ -197,6 +197,34 @@ def test_gemm_skinny_pieces(native_ext, M, N, K):
         assert ((native_ext.gemm_skinny_swiglu(x, w).double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(16, 8320), (2064, 8704), (4096, 12288)])
+def test_gemm_skinny_deep(native_ext, M, N, K):
+    """Weights deeper than 8192: four parts of 128-deep units in turns, whole rounds and not, against 64 bits (as the cuts of K above), rows
+    of x far apart, and the rule that sends a product there."""
+    from llm_in_practise_amd.ops import gemm
+    torch.manual_seed(N + M)
+    far, w = torch.randn(M, K + 40, device=DEV).to(torch.bfloat16), (torch.randn(N, K, device=DEV) * 0.02).to(torch.bfloat16)
+    x, res = far[:, :K].contiguous(), torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    exact = x.double() @ w.double().t()
+    slack = 2 * (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    for r in (None, res):
+        want = exact if r is None else exact + r.double()
+        got = native_ext.gemm_skinny(far[:, :K], w, r)
+        assert ((got.double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all()
+        assert gemm._rows_ok(x, w, r) == (M <= 16 or N > 2048)
+        if gemm._rows_ok(x, w, r):
+            assert torch.equal(gemm._base_gemm(x, w, residual=r), got)
+    # what the kernel does not take stays with the library: a residual whose rows stand apart, or off 16 bytes, and an x off 16 bytes
+    wide, off = torch.randn(M, N + 8, device=DEV).to(torch.bfloat16)[:, :N], torch.randn(M * N + 4, device=DEV).to(torch.bfloat16)[4:].view(M, N)
+    xo = torch.zeros(M * K + 4, dtype=torch.bfloat16, device=DEV)[4:].view(M, K).copy_(x)
+    for a, r in ((x, wide), (x, off), (xo, None)):
+        if r is None or not r.is_contiguous() or r.data_ptr() % 16:
+            assert not gemm._rows_ok(a, w, r) or (M == 1 and r is wide)
+        want = exact if r is None else exact + r.double()
+        assert ((gemm._base_gemm(a, w, residual=r).double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all()
+
+
 @pytest.mark.parametrize("M", [17, 32, 33, 49, 64])
 @pytest.mark.parametrize("F,K", [(16, 128), (80, 640), (4112, 384), (8208, 256), (12320, 256), (14336, 128)])
 def test_rows_swiglu(native_ext, M, F, K):
