@@ -49,6 +49,7 @@ int lt_plans();
 void launch_sum_slices(const void*, void*, int, size_t, size_t, hipStream_t);
 bool skinny_norms(int, int, bool);
 void launch_rows_swiglu(const void*, int, const void*, void*, int, int, int, hipStream_t);
+void launch_rows_parts(const void*, int, const void*, const void*, void*, float*, int, int, int, int, hipStream_t);
 void launch_gemm_skinny(const void*, int, const void*, const void*, void*, int, int, int, bool, const void*, float, hipStream_t);
 bool w4mm_supported(int, int, int, int);
 bool w4g_supported(int, int, int, int);
@@ -649,6 +650,25 @@ Tensor rows_swiglu(Tensor x, Tensor w) {
   skinny_offsets(x);
   Tensor out = at::empty({M, F}, x.options());
   launch_rows_swiglu(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), M, F, K, stream());
+  return out;
+}
+
+// y = x wᵀ (+ residual) of 17 to 64 rows, K summed in four parts that take units (64 or 128 deep) of it in turns (csrc/kernels/rows.hip): w [N, K]
+Tensor rows_parts(Tensor x, Tensor w, optional<Tensor> residual, int64_t unit) {
+  check_skinny(x, w);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M > 16 && K % 512 == 0 && K < 1 << 24 && N < 1 << 24 && (unit == 64 || unit == 128), "rows_parts: 17 to 64 rows, W [N%16, K%512]");
+  const void* rp = nullptr;
+  if (residual.has_value() && residual->defined()) {
+    CHECK_BF16((*residual));
+    CHECK_CONTIG((*residual));
+    TORCH_CHECK(residual->is_cuda() && residual->dim() == 2 && residual->size(0) == M && residual->size(1) == N &&
+                    reinterpret_cast<uintptr_t>(residual->data_ptr()) % 8 == 0, "rows_parts: residual [M, N]");
+    rp = residual->data_ptr();
+  }
+  skinny_offsets(x);
+  Tensor out = at::empty({M, N}, x.options()), part = at::empty({4, M, N}, x.options().dtype(at::kFloat));
+  launch_rows_parts(x.data_ptr(), x.stride(0), w.data_ptr(), rp, out.data_ptr(), part.data_ptr<float>(), M, N, K, (int)unit, stream());
   return out;
 }
 
@@ -1888,6 +1908,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_norms", &skinny_norms);
   m.def("gemm_skinny", &gemm_skinny, py::arg("x"), py::arg("w"), py::arg("residual"), py::arg("norm") = py::none(), py::arg("eps") = 0.0);
   m.def("rows_swiglu", &rows_swiglu);
+  m.def("rows_parts", &rows_parts);
   m.def("gemm_skinny_swiglu", &gemm_skinny_swiglu, py::arg("x"), py::arg("w"), py::arg("norm") = py::none(), py::arg("eps") = 0.0);
   m.def("lt_linear", &lt_linear);
   m.def("lt_addmm", &lt_addmm);

@@ -11,6 +11,12 @@
 // µs at 17 / 32 / 48 / 64 rows, W cold, the library's product and the activation → here: 2 × 12288 × 4096 48.0 / 47.7 / 48.2 / 49.0 → 39.6 / 38.9 /
 // 39.1 / 39.9 (5.1 TB/s), 2 × 14336 × 4096 56 / 56 / 62 / 55 → 46 / 46 / 46 / 47, 2 × 9728 × 2560 27.4 / 29.0 / 29.5 / 30.0 → 20.7 / 21.9 / 21.7 / 23.1,
 // 2 × 3072 × 1024 14 → 6.4 / 6.4 / 7.2 / 7.0.  Without the gated end it takes as long as the library's 6144 × 4096 (17.4 and 17.8 µs at 64 rows).
+//
+// The narrow product y[M, N] = x·Wᵀ (+ residual) of a deep weight has too few columns for that: 256 workgroups of 16 columns each read all of x,
+// at 64 rows four times what they read of W.  There K is summed in four parts that take its units in turns, one workgroup a part and up to 64
+// columns, and a second launch adds the parts in order: the library's order at 17 to 32 rows (units of 128 beyond K = 8192, else 64) and at 64 (units
+// of 64).  µs at 17 / 32 / 64 rows, W cold, the library → here (both launches): 4096 × 12288 23.7 / 28.2 / 36.6 → 22.2 / 23.5 / 28.0, 2560 × 9728
+// 20.0 / 20.0 / 28.0 → 16.1 / 16.5 / 19.2, 1024 × 12288 16.5 / 21.8 / 18.1 → 13.0 / 13.5 / 17.3; at 64 rows 4096 × 4096 14.9 → 12.8, 2560 × 4096 14.2 → 11.3.
 #include "lds_dma.h"
 
 using namespace lipa;
@@ -19,42 +25,46 @@ namespace {
 
 constexpr int ring_of(int stage) { return 163840 / stage < 8 ? 163840 / stage : 8; }
 
-// MT: row tiles, CO: column tiles of the result
-template <int MT, int CO>
-__global__ __launch_bounds__(512) void rows_swiglu_k(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W, bf16* __restrict__ out,
-                                                     int M, int N, int K) {
-  constexpr int CT = 2 * CO, PIECES = 4 * (CT + MT), D = (PIECES + 7) / 8, SB = PIECES * 1024, RING = ring_of(SB);
-  static_assert(RING >= 3 && (RING - 2) * D < 64 && MT * CO * 1024 <= RING * SB, "ring");
+// MT: row tiles, CT: tiles of W's rows (GLU: half of them gate's, half up's), UNIT: 0 for the gated product, else how deep the units are that the
+// four parts of K take in turns: workgroup 4 b + p sums part p of columns block b, and leaves it in part[p]
+template <int MT, int CT, int UNIT>
+__global__ __launch_bounds__(512) void rows_k(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W, bf16* __restrict__ out,
+                                              float* __restrict__ part, int M, int N, int K) {
+  constexpr bool GLU = UNIT == 0;
+  constexpr int CO = GLU ? CT / 2 : CT, PIECES = 4 * (CT + MT), D = (PIECES + 7) / 8, SB = PIECES * 1024, RING = ring_of(SB);
+  constexpr int HALF = (CT + 1) / 2;                       // tiles of the first four waves
+  static_assert(RING >= 3 && (RING - 2) * D < 64 && (!GLU || MT * CO * 1024 <= RING * SB), "ring");
   __shared__ __attribute__((aligned(1024))) char smem[RING * SB];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * CO, r4 = lane >> 4;
-  const rsrc wr = window(W + (size_t)n0 * K), ur = window(W + (size_t)(N + n0) * K), xr = window(X);
+  const int n0 = (GLU ? blockIdx.x : blockIdx.x / 4) * 16 * CO, pt = GLU ? 0 : blockIdx.x % 4, r4 = lane >> 4;
+  const rsrc wr = window(W + (size_t)n0 * K), ur = window(W + (size_t)(GLU ? N + n0 : n0) * K), xr = window(X);
   const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)smem);
   // pieces of a stage: 4 rows each, W's column tiles first (gate, up), then x; wave w brings pieces w, w + 8, ..
   const bool full = w + 8 * (D - 1) < PIECES;
   uint32_t vo[D];
 #pragma unroll
   for (int j = 0; j < D; ++j) {
-    const int p = min(w + 8 * j, PIECES - 1), ch = (li ^ (4 * (p & 3) + r4)) * 16;
-    vo[j] = p < 4 * CT ? (uint32_t)min(4 * (p >= 4 * CO ? p - 4 * CO : p) + r4, N - 1 - n0) * (uint32_t)K * 2 + ch
+    const int p = min(w + 8 * j, PIECES - 1), c = li ^ (4 * (p & 3) + r4), ch = 16 * c + (UNIT == 64 && c >= 8 ? 384 : 0);
+    vo[j] = p < 4 * CT ? (uint32_t)min(4 * (GLU && p >= 4 * CO ? p - 4 * CO : p) + r4, N - 1 - n0) * (uint32_t)K * 2 + ch
                        : (uint32_t)min(4 * (p - 4 * CT) + r4, M - 1) * (uint32_t)ldx * 2 + ch;
   }
   auto fill = [&](int slot, int stage) {
-    const uint32_t dst = base + slot * SB + w * 1024, k = stage * 256;
+    const uint32_t dst = base + slot * SB + w * 1024;
+    const uint32_t k = GLU ? stage * 256 : UNIT == 64 ? (8 * stage + pt) * 128 : (4 * stage + pt) * 256;
 #pragma unroll
     for (int j = 0; j < D; ++j)
       if (j < D - 1 || full) {
         const int p = w + 8 * j;
         if (p >= 4 * CT) to_lds(xr, dst + j * 8192, vo[j], k);
-        else if (p >= 4 * CO) to_lds_once(ur, dst + j * 8192, vo[j], k);
+        else if (GLU && p >= 4 * CO) to_lds_once(ur, dst + j * 8192, vo[j], k);
         else to_lds_once(wr, dst + j * 8192, vo[j], k);
       }
   };
-  const int stages = K / 128, mt = w & 3, c0 = w < 4 ? 0 : CO;
+  const int stages = (GLU ? K : K / 4) / 128, mt = w & 3, c0 = w < 4 ? 0 : HALF;
   const bool work = mt < MT;
-  f32x4 acc[CO];
+  f32x4 acc[HALF];
 #pragma unroll
-  for (int t = 0; t < CO; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < HALF; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < RING - 1; ++s)
     if (s < stages) fill(s, s);
@@ -68,26 +78,36 @@ __global__ __launch_bounds__(512) void rows_swiglu_k(const bf16* __restrict__ X,
       const char* p = smem + slot * SB;
 #pragma unroll
       for (int h2 = 0; h2 < 2; ++h2) {
-        bf16x8 a[2][CO], b[2];
+        bf16x8 a[2][HALF], b[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int c = li * 256 + ((8 * h2 + 4 * h + g) ^ li) * 16;
           b[h] = *reinterpret_cast<const bf16x8*>(p + (CT + mt) * 4096 + c);
 #pragma unroll
-          for (int t = 0; t < CO; ++t)
-            a[h][t] = *reinterpret_cast<const bf16x8*>(p + (c0 + t) * 4096 + c);
+          for (int t = 0; t < HALF; ++t)
+            if (c0 + t < CT) a[h][t] = *reinterpret_cast<const bf16x8*>(p + (c0 + t) * 4096 + c);
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int t = 0; t < CO; ++t)
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][t], b[h], acc[t], 0, 0, 0);
+          for (int t = 0; t < HALF; ++t)
+            if (c0 + t < CT) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][t], b[h], acc[t], 0, 0, 0);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     slot = slot + 1 == RING ? 0 : slot + 1;
   }
   const int m = 16 * mt + li;
+  if constexpr (!GLU) {
+    if (!work || m >= M) return;
+    part += (size_t)pt * M * N + (size_t)m * N;
+#pragma unroll
+    for (int t = 0; t < HALF; ++t) {
+      const int n = n0 + 16 * (c0 + t) + 4 * g;
+      if (c0 + t < CT && n < N) *reinterpret_cast<f32x4*>(part + n) = acc[t];
+    }
+    return;
+  }
   f32x4(*up)[CO][64] = reinterpret_cast<f32x4(*)[CO][64]>(smem);
   __syncthreads();
   if (work && w >= 4)
@@ -110,12 +130,28 @@ __global__ __launch_bounds__(512) void rows_swiglu_k(const bf16* __restrict__ X,
   }
 }
 
+// y = part[0] + part[1] + part[2] + part[3] (+ res), four elements a thread
+__global__ __launch_bounds__(256) void parts_sum_k(const float* __restrict__ part, const bf16* __restrict__ res, bf16* __restrict__ y, int n4) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  const f32x4* p = reinterpret_cast<const f32x4*>(part) + i;
+  f32x4 v = p[0];
+#pragma unroll
+  for (int s = 1; s < 4; ++s) v += p[(size_t)s * n4];
+  if (res != nullptr) {
+    const bf16x4 r = reinterpret_cast<const bf16x4*>(res)[i];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += (float)r[e];
+  }
+  reinterpret_cast<bf16x4*>(y)[i] = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+}
+
 }  // namespace
 
 // F: columns of the result, a multiple of 16 (W has 2 F rows); K a multiple of 128; 17 <= M <= 64
 void launch_rows_swiglu(const void* X, int ldx, const void* W, void* out, int M, int F, int K, hipStream_t st) {
   const int tiles = F / 16, t = tiles <= 256 ? 1 : tiles <= 512 ? 2 : tiles <= 768 ? 3 : 4;
-#define L(MT_, CO_) rows_swiglu_k<MT_, CO_><<<(tiles + t - 1) / t, 512, 0, st>>>((const bf16*)X, ldx, (const bf16*)W, (bf16*)out, M, F, K)
+#define L(MT_, CO_) rows_k<MT_, 2 * CO_, 0><<<(tiles + t - 1) / t, 512, 0, st>>>((const bf16*)X, ldx, (const bf16*)W, (bf16*)out, nullptr, M, F, K)
 #define LT(MT_)               \
   do {                        \
     if (t == 1) L(MT_, 1);    \
@@ -128,5 +164,32 @@ void launch_rows_swiglu(const void* X, int ldx, const void* W, void* out, int M,
   else LT(2);
 #undef LT
 #undef L
+  LIPA_CHECK_LAUNCH();
+}
+
+// y [M, N] = x wᵀ (+ res): K in four parts of units in turns, a multiple of 512; N a multiple of 16; 17 <= M <= 64; part: 4 M N floats
+void launch_rows_parts(const void* X, int ldx, const void* W, const void* res, void* y, float* part, int M, int N, int K, int unit, hipStream_t st) {
+  const int tiles = N / 16, t = tiles <= 64 ? 1 : tiles <= 128 ? 2 : tiles <= 192 ? 3 : 4;
+#define L(MT_, CT_, UNIT_) rows_k<MT_, CT_, UNIT_><<<(tiles + t - 1) / t * 4, 512, 0, st>>>((const bf16*)X, ldx, (const bf16*)W, nullptr, part, M, N, K)
+#define LT(MT_, UNIT_)                 \
+  do {                                 \
+    if (t == 1) L(MT_, 1, UNIT_);      \
+    else if (t == 2) L(MT_, 2, UNIT_); \
+    else if (t == 3) L(MT_, 3, UNIT_); \
+    else L(MT_, 4, UNIT_);             \
+  } while (0)
+#define LM(UNIT_)                     \
+  do {                                \
+    if (M > 32) LT(4, UNIT_);         \
+    else LT(2, UNIT_);                \
+  } while (0)
+  if (unit == 64) LM(64);
+  else LM(128);
+#undef LM
+#undef LT
+#undef L
+  LIPA_CHECK_LAUNCH();
+  const int n4 = M * N / 4;
+  parts_sum_k<<<(n4 + 255) / 256, 256, 0, st>>>(part, (const bf16*)res, (bf16*)y, n4);
   LIPA_CHECK_LAUNCH();
 }

@@ -239,6 +239,12 @@ static void launch_rows(const void* X, int ldx, const void* W, const void* res, 
   gemm_skinny_k<CT_, 1, NW_, RING_, GLU_, CUT_, PARTS_, NORM><<<(N + 15) / 16, 64 * NW_, extra, st>>>(                     \
       (const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, pieces, nrm)
   if constexpr (!NORM) {                        // (rows that are normed here have 4096 elements at most: 16 pieces of 256)
+    // Deep weights: the four parts of 128-deep units that the library's product sums there, a wave each with a long ring (one workgroup a CU, with
+    // all of its LDS).  In pieces 4096 × 12288 took 18.0 / 21.2 µs at 1 / 16 rows, and takes 18.0 / 20.3; 2560 × 9728 16.0 / 20.2, and 12.1 / 15.0.
+    if (!glu && K > 8192 && K % 128 == 0) {
+      L(1, 4, 8, false, TURNS128, 4);
+      return;
+    }
     if (!glu && pieces > 16) {
       if (pieces > 32) L(1, 4, 4, false, TURNS64, 4);
       else L(1, 8, 3, false, PIECES, 32);
@@ -260,16 +266,10 @@ static void launch_rows(const void* X, int ldx, const void* W, const void* res, 
 void launch_gemm_skinny(const void* X, int ldx, const void* W, const void* res, void* out, int M, int N, int K, bool glu,
                         const void* norm, float eps, hipStream_t st) {
   const Norm nrm = {(const bf16*)norm, eps, K == 1024 || K == 2048 || K == 4096 ? 2 : 1};
-#define LC(CT_, MT_, RING_, GLU_, CUT_)                                                                                   \
-  gemm_skinny_k<CT_, MT_, 4, RING_, GLU_, CUT_, 4, false><<<(N + 15) / 16, 256, 0, st>>>(                                 \
+#define L(CT_, MT_, RING_, GLU_)                                                                                          \
+  gemm_skinny_k<CT_, MT_, 4, RING_, GLU_, TURNS64, 4, false><<<(N + 15) / 16, 256, 0, st>>>(                              \
       (const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, 1, nrm)
-#define L(CT_, MT_, RING_, GLU_) LC(CT_, MT_, RING_, GLU_, TURNS64)
-  // Deep weights: the four parts of 128-deep units that the library's product sums there, a wave each with a long ring (one workgroup a CU, with
-  // all of its LDS).  In pieces, or units of 64, 4096 × 12288 took 18.0 / 21.2 µs at 1 / 16 rows, and takes 18.0 / 20.3; 2560 × 9728 16.0 / 20.2, 12.1 / 15.0.
-  if (!glu && M <= 32 && K > 8192 && K % 128 == 0) {
-    if (M > 16) LC(1, 2, 6, false, TURNS128);
-    else LC(1, 1, 8, false, TURNS128);
-  } else if (M > 32) {
+  if (M > 32) {
     if (glu) L(2, 4, 3, true);
     else L(1, 4, 3, false);
   } else if (M > 16) {
@@ -281,6 +281,5 @@ void launch_gemm_skinny(const void* X, int ldx, const void* W, const void* res, 
     launch_rows<false>(X, ldx, W, res, out, M, N, K, glu, nrm, st);
   }
 #undef L
-#undef LC
   LIPA_CHECK_LAUNCH();
 }

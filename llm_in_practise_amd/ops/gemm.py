@@ -180,23 +180,27 @@ def normed_rows(x: torch.Tensor, weight, eps: float, base) -> torch.Tensor | Non
     return fn_apply(_NormedRowsFn, x, weight, eps, base)
 
 
-def _rows_ok(x, base, residual) -> bool:
-    """Whether the decode products (csrc/kernels/skinny.hip) take more than 16 rows, or a K beyond 8192, of a narrow bf16 weight: where they
-    are the faster ones, and where their order of sums is the library's or the weight is short (a chain over all of K would round worse).
-    Library → here in µs, W cold, residual included: 4096 × 12288 at 1 / 16 / 32 rows 21.4 / 21.5 / 26.1 → 18.0 / 20.3 / 26.0 (48: 31.0 and 32.9),
-    2560 × 9728 18.1 / 16.0 / 20.1 → 12.1 / 15.0 / 19.3, 2048 × 16384 at 16 / 24 23.0 / 23.8 → 22.0 / 26.2, 4096 × 4096 at 17 / 32 13.7 / 13.0 → 9.3 / 9.9,
-    2560 × 4096 12.5 / 12.4 → 7.8 / 9.0; at 17 / 64, 4096 × 1024 11.4 / 11.7 → 3.9 / 5.3, 1024 × 3072 11.6 / 11.9 → 6.1 / 9.8, 4096 × 3072 12.3 / 16.1 →
-    6.8 / 10.8.  5120 × 4096 at 17 / 32: 15.4 / 14.7 and 14.2 / 16.4."""
+def _narrow_rows(x, base, residual):
+    """How the product of up to 64 rows and a narrow bf16 weight runs: 1 in the decode products (csrc/kernels/skinny.hip), 64 or 128 in four
+    parts of units of that depth (csrc/kernels/rows.hip), 0 by what stands below.  Each where it is the fastest, and where its order of sums is
+    the library's (up to 32 rows, and 64) or the weight is short (K < 4096; a chain over all of K would round worse).
+    Library / decode products / parts in µs, W cold, residual included, at 17 / 32 / 64 rows: 4096 × 12288 23.7 / 28.2 / 36.6, 21.2 / 25.9 /
+    35.3 and 22.2 / 23.5 / 28.0, 2560 × 9728 20.0 / 20.0 / 28.0, 18.0 / 19.2 / 26.7 and 16.1 / 16.5 / 19.2, 1024 × 12288 16.5 / 21.8 / 18.1, 17.9 / 22.3 /
+    32.2 and 13.0 / 13.5 / 17.3, 4096 × 4096 13.6 / 12.9 / 14.9, 9.4 / 9.8 / 13.1 and 11.1 / 11.5 / 12.8, 2560 × 4096 12.5 / 12.3 / 14.2, 8.1 / 9.2 / 12.3 and 10.2 /
+    11.0 / 11.3, 1024 × 3072 11.6 / 9.9 / 11.9, 6.0 / 7.3 / 9.9 and 6.7 / 7.2 / 8.4, 4096 × 2048 11.8 / 11.7 / 12.0, 5.9 / 6.3 / 8.1 and 8.0 / 8.5 / 10.5.  At 1 / 16 rows
+    4096 × 12288 21.4 / 21.5 and 18.0 / 20.3, 2560 × 9728 18.1 / 16.0 and 12.1 / 15.0.  (5120 × 4096 at 17 / 32: 15.4 / 14.7 and 14.2 / 16.4.)"""
     M, K = x.shape
     N = base.shape[0]
-    if not (x.is_cuda and M <= 64 and N <= 4096 and N % 16 == 0 and K % 64 == 0 and x.dtype == base.dtype == torch.bfloat16
+    if not (x.is_cuda and M <= 64 and N <= 4096 and N % 16 == 0 and K % 64 == 0 and K < 1 << 24 and x.dtype == base.dtype == torch.bfloat16
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and base.is_contiguous() and x.data_ptr() % 16 == 0 and base.data_ptr() % 16 == 0
             and (residual is None or (residual.dtype == torch.bfloat16 and residual.shape == (M, N) and residual.is_contiguous()
                                       and residual.data_ptr() % 16 == 0))):
-        return False
-    if K > 8192:
-        return K % 128 == 0 and K < 1 << 24 and M <= (32 if N > 2048 else 16)
-    return 16 < M <= (64 if K < 4096 else 32)
+        return 0
+    if M <= 16:
+        return int(K > 8192 and K % 128 == 0)
+    if K < 4096 or (M <= 32 and K <= 8192):
+        return 1
+    return 0 if K % 512 or 32 < M < 64 else 128 if M <= 32 else 64
 
 
 def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
@@ -218,13 +222,14 @@ def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
         return _base_gemm(x, w, ext_a, ext_b, residual)
     M, K = x.shape
     N = base.shape[0]
+    narrow = _narrow_rows(x, base, residual)
     if (x.is_cuda and M <= 16 and N <= 8192 and K <= 8192 and N % 16 == 0 and K % 64 == 0 and x.stride(0) % 8 == 0
-            and x.stride(1) == 1 and base.is_contiguous()) or _rows_ok(x, base, residual):
+            and x.stride(1) == 1 and base.is_contiguous()) or narrow:
         # decode-sized q|k|v / o projections: the weight-streaming MFMA kernel (csrc/kernels/skinny.hip) takes 8.3-9.3 µs for
         # 4096 × 4096 and 1-16 rows, residual included, where hipBLASLt takes 15.3 (12.6-14.2 against 15 for 6144 rows of W,
         # 24 against 29-31 for 8192 × 8192)
         _count("decode")
-        y = native().gemm_skinny(x, base, residual)
+        y = native().rows_parts(x, base, residual, narrow) if narrow > 1 else native().gemm_skinny(x, base, residual)
         return y if ext_a is None else y.addmm_(ext_a, ext_b.t())
     if _g4w_ok(x, base, False):
         _count("gemm4w")

@@ -197,32 +197,36 @@ def test_gemm_skinny_pieces(native_ext, M, N, K):
         assert ((native_ext.gemm_skinny_swiglu(x, w).double() - want).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("M", [1, 16, 17, 32])
-@pytest.mark.parametrize("N,K", [(16, 8320), (2064, 8704), (4096, 12288)])
-def test_gemm_skinny_deep(native_ext, M, N, K):
-    """Weights deeper than 8192: four parts of 128-deep units in turns, whole rounds and not, against 64 bits (as the cuts of K above), rows
-    of x far apart, and the rule that sends a product there."""
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(16, 8320), (1040, 8704), (2064, 4608), (3088, 512), (4096, 12288), (2560, 1024)])
+def test_narrow_rows(native_ext, M, N, K):
+    """The products of few rows and a narrow weight, in four parts of units in turns (whole rounds and not; one to four column tiles a
+    workgroup, with and without a remainder; fewer stages than the ring holds and more) and by the rule that picks them, against 64 bits
+    (sums of K products in float lie within (K + 1) half-ulps of the absolute sum, then one rounding to bf16), rows of x far apart too.  What
+    they do not take stays with the library: a residual whose rows stand apart, or off 16 bytes, and an x off 16 bytes."""
     from llm_in_practise_amd.ops import gemm
     torch.manual_seed(N + M)
     far, w = torch.randn(M, K + 40, device=DEV).to(torch.bfloat16), (torch.randn(N, K, device=DEV) * 0.02).to(torch.bfloat16)
     x, res = far[:, :K].contiguous(), torch.randn(M, N, device=DEV).to(torch.bfloat16)
     exact = x.double() @ w.double().t()
     slack = 2 * (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    forms = [] if M <= 16 or K % 512 else [lambda a, r, u=u: native_ext.rows_parts(a, w, r, u) for u in (64, 128)]
+    if M <= 16:
+        forms.append(lambda a, r: native_ext.gemm_skinny(a, w, r))
+    forms.append(lambda a, r: gemm._base_gemm(a, w, residual=r))
     for r in (None, res):
         want = exact if r is None else exact + r.double()
-        got = native_ext.gemm_skinny(far[:, :K], w, r)
-        assert ((got.double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all()
-        assert gemm._rows_ok(x, w, r) == (M <= 16 or N > 2048)
-        if gemm._rows_ok(x, w, r):
-            assert torch.equal(gemm._base_gemm(x, w, residual=r), got)
-    # what the kernel does not take stays with the library: a residual whose rows stand apart, or off 16 bytes, and an x off 16 bytes
+        for form in forms:
+            got = form(x, r)
+            assert ((got.double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all()
+            assert torch.equal(form(far[:, :K], r), got)
     wide, off = torch.randn(M, N + 8, device=DEV).to(torch.bfloat16)[:, :N], torch.randn(M * N + 4, device=DEV).to(torch.bfloat16)[4:].view(M, N)
     xo = torch.zeros(M * K + 4, dtype=torch.bfloat16, device=DEV)[4:].view(M, K).copy_(x)
     for a, r in ((x, wide), (x, off), (xo, None)):
-        if r is None or not r.is_contiguous() or r.data_ptr() % 16:
-            assert not gemm._rows_ok(a, w, r) or (M == 1 and r is wide)
-        want = exact if r is None else exact + r.double()
-        assert ((gemm._base_gemm(a, w, residual=r).double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all()
+        if M > 16:
+            assert gemm._narrow_rows(a, w, r) == 0
+            want = exact if r is None else exact + r.double()
+            assert ((gemm._base_gemm(a, w, residual=r).double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all()
 
 
 @pytest.mark.parametrize("M", [17, 32, 33, 49, 64])
