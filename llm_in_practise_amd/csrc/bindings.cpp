@@ -67,6 +67,7 @@ void launch_nf4_dequant(const uint8_t*, const float*, const uint8_t*, const floa
 bool gemm4w_supported(int, int, int, int, int, bool, bool);
 int gemm4w_plan(int, int, int, bool, int, int, int*, int, int*, bool);
 int gemm4w_tiles(int, int, int, int);
+int gemm4w_rows(int, int, int, bool, int, int*, int*, int*, int*);
 void launch_mlora_apply(const void*, int, const void*, const void*, const int64_t*, const void*, int, void*, int, int, int,
                         int, int, int, hipStream_t);
 void launch_gemm4w_swiglu(const void*, int, const void*, const float*, void*, void*, int, int, int, int, int,
@@ -868,6 +869,13 @@ std::vector<int64_t> gemm4w_plan_info(int64_t M, int64_t N, int64_t K, bool bt, 
   return {sp, bn, bm};
 }
 
+// the rows of its first launch (M: it is the only one)
+int64_t gemm4w_row_cut(int64_t M, int64_t N, int64_t K, bool bt) {
+  int bn = 0, bm = 0, bn2 = 0, bm2 = 0;
+  const int sp = gemm4w_plan((int)M, (int)N, (int)K, bt, 0, 0, &bn, 0, &bm, false);
+  return gemm4w_rows((int)M, (int)N, (int)K, bt, sp, &bn, &bm, &bn2, &bm2);
+}
+
 // y = x·wᵀ (+ residual) through the one-wave-per-SIMD AGPR-accumulator MFMA GEMM (gemm4w.hip);
 // x [M, K] (row stride any multiple of 8), w [N, K] contiguous rows.  bt: y = x·w with w [K, N]
 // (the dX = dY·W of a frozen [N_w, K_w] weight, no transpose copy).  splits <= 0: auto split-K;
@@ -903,8 +911,15 @@ Tensor gemm4w(Tensor x, Tensor w, optional<Tensor> residual, int64_t splits, boo
                     wzero->numel() == wscale->numel(), "gemm4w: wzero fp32 [K/64, N] with wscale, forward only");
     zp = wzero->data_ptr<float>();
   }
-  launch_gemm4w(x.data_ptr(), x.stride(0), b.ptr, b.ld, res, y.data_ptr(), sp > 1 ? ws.data_ptr<float>() : nullptr,
-                b.scale, zp, M, N, K, sp, bt, bn_used, bm_used, stream());
+  int bn2 = 0, bm2 = 0;
+  const int64_t rows = w4 || bn || bm ? M : gemm4w_rows(M, N, K, bt, sp, &bn_used, &bm_used, &bn2, &bm2);
+  float* slabs = sp > 1 ? ws.data_ptr<float>() : nullptr;
+  launch_gemm4w(x.data_ptr(), x.stride(0), b.ptr, b.ld, res, y.data_ptr(), slabs, b.scale, zp, rows, N, K, sp, bt, bn_used, bm_used, stream());
+  if (rows < M) {
+    const int64_t at = rows * N;
+    launch_gemm4w(x.data_ptr<at::BFloat16>() + rows * x.stride(0), x.stride(0), b.ptr, b.ld, res ? (const at::BFloat16*)res + at : nullptr,
+                  y.data_ptr<at::BFloat16>() + at, slabs, b.scale, zp, M - rows, N, K, sp, bt, bn2, bm2, stream());
+  }
   return y;
 }
 
@@ -927,8 +942,13 @@ std::vector<Tensor> gemm4w_swiglu(Tensor x, Tensor w, optional<Tensor> wscale, i
   Tensor gu, h;
   if (want_gu) gu = at::empty({M, 2 * F}, x.options());
   if (want_h) h = at::empty({M, F}, x.options());
-  launch_gemm4w_swiglu(x.data_ptr(), x.stride(0), b.ptr, b.scale, want_gu ? gu.data_ptr() : nullptr,
-                       want_h ? h.data_ptr() : nullptr, M, F, K, bn, bm, stream());
+  int bn2 = 0, bm2 = 0;
+  const int64_t rows = w4 ? M : gemm4w_rows(M, 2 * F, K, false, 1, &bn, &bm, &bn2, &bm2);
+  at::BFloat16 *gp = want_gu ? gu.data_ptr<at::BFloat16>() : nullptr, *hp = want_h ? h.data_ptr<at::BFloat16>() : nullptr;
+  launch_gemm4w_swiglu(x.data_ptr(), x.stride(0), b.ptr, b.scale, gp, hp, rows, F, K, bn, bm, stream());
+  if (rows < M)
+    launch_gemm4w_swiglu(x.data_ptr<at::BFloat16>() + rows * x.stride(0), x.stride(0), b.ptr, b.scale, gp ? gp + rows * 2 * F : nullptr,
+                         hp ? hp + rows * F : nullptr, M - rows, F, K, bn2, bm2, stream());
   return {gu, h};
 }
 
@@ -946,8 +966,12 @@ Tensor gemm4w_dswiglu(Tensor dy, Tensor w, Tensor gu, optional<Tensor> wscale) {
   int bn = 0, bm = 0;
   gemm4w_plan(M, F, Nw, true, 0, 1, &bn, 0, &bm, w4);
   auto dgu = at::empty({M, 2 * F}, dy.options());
-  launch_gemm4w_dswiglu(dy.data_ptr(), dy.stride(0), b.ptr, b.scale, gu.data_ptr(), dgu.data_ptr(), M, F, Nw, bn, bm,
-                        stream());
+  int bn2 = 0, bm2 = 0;
+  const int64_t rows = w4 ? M : gemm4w_rows(M, F, Nw, true, 1, &bn, &bm, &bn2, &bm2);
+  launch_gemm4w_dswiglu(dy.data_ptr(), dy.stride(0), b.ptr, b.scale, gu.data_ptr(), dgu.data_ptr(), rows, F, Nw, bn, bm, stream());
+  if (rows < M)
+    launch_gemm4w_dswiglu(dy.data_ptr<at::BFloat16>() + rows * dy.stride(0), dy.stride(0), b.ptr, b.scale, gu.data_ptr<at::BFloat16>() + rows * 2 * F,
+                          dgu.data_ptr<at::BFloat16>() + rows * 2 * F, M - rows, F, Nw, bn2, bm2, stream());
   return dgu;
 }
 
@@ -1926,6 +1950,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("w4g_splits", &w4g_splits);
   m.def("set_dequant_variant", &set_dequant_variant);
   m.def("gemm4w_ok", &gemm4w_ok);
+  m.def("gemm4w_row_cut", &gemm4w_row_cut);
   m.def("gemm4w_plan_info", &gemm4w_plan_info);
   m.def("g4w_pack", &g4w_pack);
   m.def("gemm4w_lora", &gemm4w_lora);

@@ -117,6 +117,12 @@ bool gemm4w_supported(int M, int N, int K, int lda, int ldb, bool bt, bool w4) {
 struct G4wCfg {
   int bm, bn, splits;
 };
+// µs of M rows in such tiles, at what they take over several rounds of 256 workgroups, 6 µs a round to fill and empty it
+double tiles_us(int M, int N, int nk, bool bt, int s, int bm, int bn) {
+  double kt_us = bn == 256 ? (bt ? 1.52 : 1.5) : bn == 192 ? (bt ? 1.24 : 1.22) : 0.97;
+  if (bm == 128) kt_us *= 0.62;
+  return (double)(((int64_t)tiles_of(M, N, bm, bn) * s + 255) / 256) * ((nk + s - 1) / s * kt_us + 6.0);
+}
 G4wCfg gemm4w_cfg(int M, int N, int K, bool bt, int bn_req, int sp_req, int bm_req, bool w4) {
   // W4 (NF4 codes expanded in-kernel): the measured cost of a K-tile relative to bf16 per tile height
   // (profiles/r4/gemm4w_nf4_ab.txt)
@@ -160,9 +166,7 @@ G4wCfg gemm4w_cfg(int M, int N, int K, bool bt, int bn_req, int sp_req, int bm_r
     for (int bn : {256, 192, 128}) {
       if (bn == 192 && bt && bm != 256) continue;
       if (bn_req > 0 ? bn != bn_req : bn_req < 0 && bn == 192) continue;
-      double kt_us = bn == 256 ? (bt ? 1.52 : 1.5) : bn == 192 ? (bt ? 1.24 : 1.22) : 0.97;
-      if (bm == 128) kt_us *= 0.62;
-      const double t = (double)((tiles_of(M, N, bm, bn) * s + 255) / 256) * ((nk + s - 1) / s * kt_us + 6.0);
+      const double t = tiles_us(M, N, nk, bt, s, bm, bn);
       if (t < best_t - 1e-9) {
         best_t = t;
         best.bm = bm;
@@ -183,6 +187,40 @@ int gemm4w_plan(int M, int N, int K, bool bt, int bn, int splits, int* bn_out, i
 }
 
 int gemm4w_tiles(int M, int N, int bm, int bn) { return tiles_of(M, N, bm, bn); }
+
+// A last round of few tiles costs what a full one does.  Rows of the first of two launches, which fills whole rounds of 256 workgroups with
+// the tile (bm, bn); the rest go to a second one with the tile (bm2, bn2).  M: one launch with the tile that came in.  (K is cut
+// the same way in both: every bit is that of one launch.)  µs, one launch → two, of 195 products of 256 .. 2608 rows the 19 that it cuts: 2451 rows of
+// 4096 × 12288 272 → 254, 1500 of it 169 → 151, 2100 of 24576 × 4096 with SwiGLU 383 → 335, 2608 460 → 417, 2048 of 19456 × 2560 191 → 168; W as stored,
+// 520 of 4096 × 24576 166 → 139, 2100 499 → 469; the least gain 1500 of 4096 × 6144, 105.3 → 100.3.
+int gemm4w_rows(int M, int N, int K, bool bt, int s, int* bn, int* bm, int* bn2, int* bm2) {
+  const int nk = K / BK;
+  if ((int64_t)tiles_of(M, N, *bm, *bn) * s <= 256) return M;
+  const double whole = tiles_us(M, N, nk, bt, s, *bm, *bn);
+  double best_t = 0.95 * whole - 4.0;                       // (a launch, and what the estimate is worth)
+  int rows = M, n1 = *bn, m1 = *bm;
+  auto each = [&](auto f) {
+    for (int h : {256, 128})
+      for (int w : {256, 192, 128})
+        if (!(w == 192 && bt && h != 256)) f(h, w);
+  };
+  each([&](int h, int w) {
+    const int64_t line = (int64_t)((N + w - 1) / w) * s;    // workgroups of a row of tiles
+    const int64_t rounds = (int64_t)((M + h - 1) / h) * line / 256;
+    for (int64_t r = rounds; r >= 1 && r > rounds - 3; --r) {
+      const int first = (int)(r * 256 / line) * h;
+      if (first <= 0 || first >= M) continue;
+      const double t1 = tiles_us(first, N, nk, bt, s, h, w);
+      each([&](int h2, int w2) {
+        const double t = t1 + tiles_us(M - first, N, nk, bt, s, h2, w2);
+        if (t < best_t - 1e-9) best_t = t, rows = first, m1 = h, n1 = w, *bm2 = h2, *bn2 = w2;
+      });
+    }
+  });
+  *bm = m1;
+  *bn = n1;
+  return rows;
+}
 
 // ws: splits·M·N fp32 slabs (splits > 1).  Callers pass the (bm, bn, splits) that gemm4w_plan
 // returned.  bscale != nullptr: B is g4w-packed NF4 codes, bscale the transposed fp32 block absmax.

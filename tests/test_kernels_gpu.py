@@ -707,6 +707,33 @@ def test_gemm4w_matches_fp32(native_ext, M, N, K, splits, bt, resid, bn, bm):
     assert rel_err(y, want) < 1e-2
 
 
+@pytest.mark.parametrize("M,N,K,bt", [(700, 4096, 12288, False), (520, 4096, 24576, True), (4400, 8192, 512, False), (4400, 8192, 512, True)])
+def test_gemm4w_row_cut(native_ext, M, N, K, bt):
+    """Rows in two launches (a last round of few tiles is cut off, and takes smaller ones), with K in parts and whole: every bit is that of
+    one launch, for the product, a residual, rows of x far apart, and the ends in SwiGLU and its gradient."""
+    rows = native_ext.gemm4w_row_cut(M, N, K, bt)
+    assert 0 < rows < M
+    torch.manual_seed(M)
+    far = torch.randn(M, K + 16, device=DEV).to(torch.bfloat16)
+    x, w = far[:, :K], (torch.randn(*((K, N) if bt else (N, K)), device=DEV) * 0.02).to(torch.bfloat16)
+    res = torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    splits, bn, bm = native_ext.gemm4w_plan_info(M, N, K, bt, False)
+    for r in (None, res):
+        assert torch.equal(native_ext.gemm4w(x, w, r, 0, bt), native_ext.gemm4w(x, w, r, splits, bt, bn, bm))
+    if splits > 1:
+        return
+    half = M // 2 // 8 * 8                                    # (too few rows to cut, or cut elsewhere: the bits are the same)
+    if bt:
+        gu = torch.randn(M, 2 * N, device=DEV).to(torch.bfloat16)
+        whole = native_ext.gemm4w_dswiglu(x, w, gu)
+        assert torch.equal(whole, torch.cat([native_ext.gemm4w_dswiglu(x[a:b], w, gu[a:b]) for a, b in ((0, half), (half, M))]))
+    else:
+        gu, h = native_ext.gemm4w_swiglu(x, w)
+        parts = [native_ext.gemm4w_swiglu(x[a:b], w) for a, b in ((0, half), (half, M))]
+        assert torch.equal(gu, torch.cat([p[0] for p in parts])) and torch.equal(h, torch.cat([p[1] for p in parts]))
+        assert torch.equal(native_ext.gemm4w_swiglu(x, w, want_gu=False)[1], h) and torch.equal(native_ext.gemm4w_swiglu(x, w, want_h=False)[0], gu)
+
+
 def test_gemm4w_asymmetric_operands(native_ext):
     """integer-valued, asymmetric operands (exact in fp32): a transposed fragment map or a swapped
     C-write shows as a large error (cdna_hip_programming.md §3)"""
