@@ -40,6 +40,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_fwd_k(const bf16* __restrict
                                                           bf16* __restrict__ k, float* __restrict__ rq,
                                                           float* __restrict__ rk, int T, int hq, int hkv, float eps) {
   constexpr int P = D / 8, H = D / 2;
+  // (all arguments at once: the choices between q and k below would each wait for theirs)
+  asm volatile("" ::"s"(qkv), "s"(qw), "s"(kw), "s"(cosb), "s"(sinb), "s"(q), "s"(k), "s"(rq), "s"(rk));
   const int gid = blockIdx.x * 256 + threadIdx.x;
   const int row = gid / P, j = gid % P;
   const int nq = T * hq, nrows = nq + T * hkv;
@@ -49,26 +51,28 @@ __global__ __launch_bounds__(256) void qk_norm_rope_fwd_k(const bf16* __restrict
   const int h = isq ? row % hq : (row - nq) % hkv;
   const int ld = (hq + 2 * hkv) * D;
   const bf16* src = qkv + (size_t)t * ld + (isq ? h * D : (hq + h) * D);
-  float a[4], b[4];
+  // every load goes out before the sum is formed, a missing weight's in the row itself: behind branches they were three round trips to memory
+  // (12 / 2451 rows of 32 + 8 heads of 128: 2.30 / 11.6 → 2.07 / 10.6 µs)
+  const bf16* w = isq ? qw : kw;
+  const bool has = w != nullptr;
+  if (!has) w = src;
+  float a[4], b[4], wa[4], wb[4], c[4], s[4];
   ld4(src + 4 * j, a);
   ld4(src + H + 4 * j, b);
+  ld4(w + 4 * j, wa);
+  ld4(w + H + 4 * j, wb);
+  ld4f(cosb + (size_t)t * H + 4 * j, c);
+  ld4f(sinb + (size_t)t * H + 4 * j, s);
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) ss += a[i] * a[i] + b[i] * b[i];
   ss = group_sum<P>(ss);
   const float r = rsqrtf(ss / D + eps);
-  const bf16* w = isq ? qw : kw;
-  float wa[4], wb[4];
-  if (w) {
-    ld4(w + 4 * j, wa);
-    ld4(w + H + 4 * j, wb);
-  } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wa[i] = wb[i] = 1.f;
+  for (int i = 0; i < 4; ++i) {
+    wa[i] = has ? wa[i] : 1.f;
+    wb[i] = has ? wb[i] : 1.f;
   }
-  float c[4], s[4];
-  ld4f(cosb + (size_t)t * H + 4 * j, c);
-  ld4f(sinb + (size_t)t * H + 4 * j, s);
   float oa[4], ob[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -81,10 +85,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_fwd_k(const bf16* __restrict
   bf16* dst = isq ? q + (size_t)t * hq * D + h * D : k + (size_t)t * hkv * D + h * D;
   st4(dst + 4 * j, oa);
   st4(dst + H + 4 * j, ob);
-  if (j == 0) {
-    if (isq) rq[row] = r;
-    else rk[row - nq] = r;
-  }
+  if (j == 0) *(isq ? rq + row : rk + (row - nq)) = r;
 }
 
 template <int D>

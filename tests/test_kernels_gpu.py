@@ -707,6 +707,36 @@ def test_gemm4w_matches_fp32(native_ext, M, N, K, splits, bt, resid, bn, bm):
     assert rel_err(y, want) < 1e-2
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N", [8, 504, 520, 1024, 1544, 2560, 3080, 3584, 4096, 4616, 5120, 8184, 8192])
+def test_rmsnorm_widths(native_ext, N, dtype):
+    """Rows of one piece of 512 to sixteen, whole and in part, with a weight and without one, the last rows of the tensor at its end: against
+    64 bits (N squares in float lie within (N + 1) half-ulps of their sum, the root halves that, three more roundings, then the type's)."""
+    for M in (1, 5):
+        torch.manual_seed(N + M)
+        x, w = torch.randn(M, N, device=DEV).to(dtype), torch.randn(N, device=DEV).to(dtype)
+        for wt in (w, None):
+            y, rstd = native_ext.rmsnorm_fwd(x, wt, 1e-6)
+            r = torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-6)
+            want = x.double() * r * (1.0 if wt is None else wt.double())
+            rel = (N / 2 + 8) * 2.0 ** -24
+            assert ((rstd.double() - r[:, 0]).abs() <= rel * r[:, 0]).all()
+            assert ((y.double() - want).abs() <= (rel + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)) * want.abs()).all()
+
+
+@pytest.mark.parametrize("T,hq,hkv,d", [(1, 1, 1, 32), (3, 5, 2, 64), (17, 4, 1, 128), (2, 3, 3, 256)])
+def test_qk_norm_rope_without_weights(native_ext, T, hq, hkv, d):
+    """A head norm without its weight is one of ones, and one of q alone leaves k's as it is."""
+    torch.manual_seed(T)
+    qkv = torch.randn(T, (hq + 2 * hkv) * d, device=DEV).to(torch.bfloat16)
+    w, ones = torch.randn(d, device=DEV).to(torch.bfloat16), torch.ones(d, device=DEV, dtype=torch.bfloat16)
+    c, s = torch.randn(T, d // 2, device=DEV), torch.randn(T, d // 2, device=DEV)
+    for a, b in ((None, None), (w, None), (None, w)):
+        got = native_ext.qk_norm_rope_fwd(qkv, a, b, c, s, hq, hkv, d, 1e-6)
+        want = native_ext.qk_norm_rope_fwd(qkv, ones if a is None else a, ones if b is None else b, c, s, hq, hkv, d, 1e-6)
+        assert all(torch.equal(g, v) for g, v in zip(got, want))
+
+
 @pytest.mark.parametrize("M,N,K,bt", [(700, 4096, 12288, False), (520, 4096, 24576, True), (4400, 8192, 512, False), (4400, 8192, 512, True)])
 def test_gemm4w_row_cut(native_ext, M, N, K, bt):
     """Rows in two launches (a last round of few tiles is cut off, and takes smaller ones), with K in parts and whole: every bit is that of
