@@ -158,3 +158,28 @@ def test_routing_of_wide_rows(T, W, dt):
     want = M.route_tokens(h, router, torch.zeros(12), 3, 1, 1, normalize=True)
     same = (got[0].cpu() == want[0]).all(1)             # (a choice can only differ where two scores are that close)
     assert same.float().mean() >= 0.995 and (got[1].cpu() - want[1])[same].abs().max() <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("top", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("T,W", [(1, 4), (7, 1028), (65, 2048)])
+def test_combine_rows_together(T, W, top, dtype):
+    """Rows of a token's choices loaded together: choices of no expert (-1) and of the token itself (>= E), a NaN in whatever is read and not
+    chosen, a shared expert with and without its gate; against 64 bits (top + 1 products and sums in float)."""
+    from llm_in_practise_amd.ops._native import native_seq
+    torch.manual_seed(T + top)
+    E, dev = 4, "cuda"
+    ys, h = torch.randn(T * top, W, device=dev).to(dtype), torch.randn(T, W, device=dev).to(dtype)
+    shared, gate, w = torch.randn(T, W, device=dev).to(dtype), torch.randn(T, device=dev), torch.randn(T, top, device=dev)
+    idx = torch.randint(-1, E + 2, (T, top), device=dev, dtype=torch.int32)
+    pos = torch.randperm(T * top, device=dev).view(T, top)
+    h[(idx < E).all(1)] = float("nan")
+    ys[pos[(idx < 0) | (idx >= E)]] = float("nan")
+    rows = torch.where((idx >= E)[..., None], h[:, None].double(), ys[pos].double())
+    terms = torch.where((idx >= 0)[..., None], rows * w[..., None].double(), 0.0)
+    for sh, g in ((None, None), (shared, None), (shared, gate)):
+        base = torch.zeros(T, W, device=dev, dtype=torch.float64) if sh is None else sh.double() * (1.0 if g is None else torch.sigmoid(g.double())[:, None])
+        got = native_seq().moe_combine_sorted(ys, pos, idx, w, h, sh, E, g).double()
+        bound = (top + 8) * 2.0 ** -23 * (base.abs() + terms.abs().sum(1))
+        assert ((got - base - terms.sum(1)).abs() <= bound).all()
