@@ -11,8 +11,8 @@
 // numbers, which hold its 24 bits: three products with float sums, at five times the rate of the float matrix units.  Log
 // decays are summed in 64 bits and kept as two floats, so that the difference of two large sums is exact.
 //
-// Measured, token by token -> chunks: state space, one prompt of 4093 tokens, 64 heads of 128 x 64: 2350 -> 95 us (state 32, walk 9,
-// outputs 52); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 82 us (25, 11, 45).  Error against 64 bits
+// Measured, token by token -> chunks: state space, one prompt of 4093 tokens, 64 heads of 128 x 64: 2350 -> 92 us (state 32, walk 9,
+// outputs 50); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 80 us (25, 11, 43).  Error against 64 bits
 // 1.6e-7 -> 0.9e-7 and 4.4e-7 -> 1.9e-7: fewer roundings stand between a token and the outputs far behind it.
 // The first case reads and writes 335 MB, 235 of them states and outputs, of which a copy moves 5 TB/s.  With every chunk's contribution
 // walked by itself (69 MB of states out, in, out and in), operands of the outputs loaded from memory rows as they are needed, an
@@ -717,7 +717,9 @@ __global__ __launch_bounds__(256, 3) void k_chunk_out(const bf16* __restrict__ q
     if (half == 0 && qi < n) den[(size_t)(t0 + qi) * H + hd] = t * ga.qscale;
   }
   const float skip = MLSTM ? 0.f : ga.dskip[hd];
-  // (a store that has no place goes past the end of its window and is dropped)
+  // (a store that has no place goes past the end of its window and is dropped.  The outputs leave nothing in the caches, which hold the states that
+  // other blocks are about to read: state space, 4093 tokens 93.4 -> 91.8 us, 8 prompts of 333 to 1024 169.7 -> 159; mLSTM, the same 82.1 -> 80.1.  The
+  // states, just written, as loads that leave nothing: 99.5 and 165.)
   const auto win = __builtin_amdgcn_make_buffer_rsrc(out + ((size_t)t0 * H + hd) * dv, 0, ((n - 1) * H + 1) * dv * 4, 0x00020000);
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
@@ -734,7 +736,7 @@ __global__ __launch_bounds__(256, 3) void k_chunk_out(const bf16* __restrict__ q
         y *= ga.qscale;
       else
         y += skip * (float)own[c_row(i, 0) * 64 + 8 * tr_piece<64>(c_row(i, 0), col >> 3)];
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), win, at + (unsigned)(c_row(i, 0) * H) * dv * 4, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), win, at + (unsigned)(c_row(i, 0) * H) * dv * 4, 0, 2);
     }
   }
 }
