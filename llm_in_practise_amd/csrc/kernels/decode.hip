@@ -193,6 +193,9 @@ __global__ __launch_bounds__(D) void decode_attn_merge_k(const float* __restrict
 //  * V's lines, and K's of 64 elements a head, are read once and leave nothing in the caches.  µs before → now, 32 query on 8 heads of 128: 64 x
 //    1024 keys 59.7 → 57.2 (4.75 TB/s), 16 x 4096 59.9 → 57.2, 1 x 1024 10.0; 14 on 2 heads of 64: 64 x 512 11.4 → 10.6, 1 x 4096 9.2 → 8.4.
 //    K of 128 a head, whose lines take two loads, the same way: 64 x 1024 59.9, 1 x 4096 13.3 → 12.5.
+//  * what stands in front of the first keys is one round trip after the length: the queries in one go (behind a branch four trips), every argument
+//    with the first; the new row is copied by the wave that has the fewest tiles.  Both launches, 1 x 1024 keys 9.9 → 9.5 µs, 12 x 700 15.2 →
+//    14.7, 64 x 1024 57.2 → 56.3.  (Loads of the next tile in front of this one's softmax: 166 registers, 57.3; four waves a SIMD spill, 73.)
 //  * lengths come from pos (int64, len = pos + 1) — no host-side lens tensor.
 __device__ __forceinline__ bf16x4 dec_tr_read(const bf16* p) {
   typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
@@ -223,6 +226,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
   __shared__ float sm[4][16], sl[4][16];
   static_assert(4 * 16 * D * 4 <= 4 * VT * 2, "merge buffer aliases the V tiles");
 
+  asm volatile("" ::"s"(q), "s"(knew), "s"(vnew), "s"(kc), "s"(vc), "s"(ldq), "s"(ldkn), "s"(ldvn));   // (all at once, not behind the length)
   const int split = blockIdx.x, kh = blockIdx.y, b = blockIdx.z;
   const int G = hq / hkv;
   const int len = (int)pos[b] + 1;
@@ -236,7 +240,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
   bf16* vcb = vc + (size_t)b * Smax * rs + kh * D;
   const bf16* knb = knew + (size_t)b * ldkn + kh * D;
   const bf16* vnb = vnew + (size_t)b * ldvn + kh * D;
-  if (k1 == len && w == 0 && lane < 2 * CH) {      // append the new token's K/V rows
+  if (k1 == len && w == 3 && lane < 2 * CH) {      // append the new token's K/V rows (the wave that has the fewest tiles)
     const int c = lane % CH;
     if (lane < CH)
       *reinterpret_cast<bf16x8*>(kcb + (size_t)(len - 1) * rs + 8 * c) = *reinterpret_cast<const bf16x8*>(knb + 8 * c);
@@ -247,8 +251,8 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
   bf16x8 qf[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    if (li < G) qf[s] = *reinterpret_cast<const bf16x8*>(q + (size_t)b * ldq + (kh * G + li) * D + 32 * s + 8 * g);
-    else qf[s] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    // (columns without a head repeat the last one's and are not read; behind a branch each load waited for the one before it)
+    qf[s] = *reinterpret_cast<const bf16x8*>(q + (size_t)b * ldq + (kh * G + min(li, G - 1)) * D + 32 * s + 8 * g);
   }
   f32x4 acc[ND];
 #pragma unroll
