@@ -129,6 +129,21 @@ def test_decode_attention_append_split_plans(native_ext, B, max_len):
     assert (o.float() - r).abs().max().item() < 2e-2
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("max_len", [33, 500, 900, 4097, 9000])
+def test_decode_attention_append_merge(native_ext, max_len, d):
+    """The merge of fewer splits than it takes in one go, as many, and more, of which few, all or all but one have keys."""
+    torch.manual_seed(max_len)
+    P = torch.tensor([0, max_len // 3, max_len - 1, 32], device=DEV)
+    B, hq, hkv = len(P), 3, 1
+    kc, vc = (torch.randn(B, max_len, hkv * d, device=DEV).to(torch.bfloat16) for _ in range(2))
+    q, k, v = (torch.randn(B, n * d, device=DEV).to(torch.bfloat16) for n in (hq, hkv, hkv))
+    o = native_ext.decode_attention_append(q, k, v, kc, vc, P, hq, hkv, d, max_len, 1 / math.sqrt(d))
+    r = decode_attention_reference(q.float(), kc.float(), vc.float(), (P + 1).int(), hq, hkv, d)
+    # weights and values in bf16: 2^-8 of the largest value for each, and the output's own rounding
+    assert (o.float() - r).abs().max().item() < 3 * 2.0 ** -8 * vc.float().abs().max().item()
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 33, 64])
 @pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 12288), (272, 192)])
 def test_gemm_skinny_matches_fp32(native_ext, M, N, K):
