@@ -222,7 +222,7 @@ def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
         return _base_gemm(x, w, ext_a, ext_b, residual)
     M, K = x.shape
     N = base.shape[0]
-    narrow = _narrow_rows(x, base, residual)
+    narrow = _narrow_rows(x, base, residual) if M <= 64 else 0
     if (x.is_cuda and M <= 16 and N <= 8192 and K <= 8192 and N % 16 == 0 and K % 64 == 0 and x.stride(0) % 8 == 0
             and x.stride(1) == 1 and base.is_contiguous()) or narrow:
         # decode-sized q|k|v / o projections: the weight-streaming MFMA kernel (csrc/kernels/skinny.hip) takes 8.3-9.3 µs for
