@@ -284,7 +284,7 @@ def int4_linear(x: torch.Tensor, w: Int4Weight, bias: torch.Tensor | None = None
 
 def int4_swiglu(x: torch.Tensor, w: Int4Weight) -> torch.Tensor | None:
     """``silu(gate)·up`` of the [gate | up] product of 3 .. 16 decode rows in one launch, or None where w4mm.hip does not serve
-    it so.  Bit for bit int4_linear and the activation (24576 × 4096, 12 rows: 26.9 + 5 → 19.9 µs)."""
+    it so.  Bit for bit int4_linear and the activation (24576 × 4096, 12 rows: 26.9 + 5 → 16.4 µs)."""
     from ..ops._native import native, use_native
     x2 = x.reshape(-1, x.shape[-1])
     n, k = w.shape
