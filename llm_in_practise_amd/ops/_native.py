@@ -105,6 +105,26 @@ def fn_apply(fn, *args):
     return super(_Function, fn).apply(*args)
 
 
+_compiling = torch.compiler.is_compiling
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_jit_trace = torch._C._get_tracing_state
+_batched = torch._C._functorch.is_legacy_batchedtensor      # (the rows of ``torch.autograd.grad(.., is_grads_batched=True)``)
+_forward_ad = torch.autograd.forward_ad
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def eager(*tensors: torch.Tensor | None) -> bool:
+    """True when a kernel may read these tensors now: nothing transforms or records the call, and each is a plain tensor or parameter with
+    memory of its own, not one that stands for others (fake, batched, wrapped).  An op that torch's own operations can do instead asks this
+    before it hands pointers to a kernel: a tensor without memory passes for one at address 0."""
+    if _compiling() or _functorch_active() or _dispatch_modes() or _jit_trace() is not None or _forward_ad._current_level >= 0:
+        return False
+    for t in tensors:
+        if t is not None and (type(t) not in _PLAIN or _batched(t)):
+            return False
+    return True
+
+
 def use_native(*tensors: torch.Tensor | None) -> bool:
     """True when the op must run on the HIP kernels."""
     for t in tensors:

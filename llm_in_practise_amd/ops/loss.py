@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 from . import reference as ref
-from ._native import _functorch_active, fn_apply, native, use_native
+from ._native import _functorch_active, eager, fn_apply, native, use_native
 from .gemm import _count, _g4w_ok
 
 
@@ -88,8 +88,7 @@ def fused_linear_cross_entropy(h: torch.Tensor, weight: torch.Tensor, labels: to
 
 def shift_labels(labels: torch.Tensor, ignore_index: int = -100) -> torch.Tensor:
     """HF causal-LM convention: position t predicts token t+1; last position ignored."""
-    if (labels.is_cuda and labels.dtype == torch.int64 and labels.dim() and labels.is_contiguous() and use_native(labels)
-            and not _functorch_active()):
+    if eager(labels) and labels.is_cuda and labels.dtype == torch.int64 and labels.dim() and labels.is_contiguous() and use_native(labels):
         return native().shift_labels(labels, ignore_index)
     out = torch.full_like(labels, ignore_index)
     out[..., :-1] = labels[..., 1:]
