@@ -407,7 +407,8 @@ class ServingEngine:
         # models whose sequences hold more than K/V rows (recurrent state, convolution inputs) bring their own slot
         # pool (models/common.py SeqStateCache); it answers the same view calls as KVCache
         self.stateful = hasattr(self.lm, "make_cache")
-        self._head = getattr(self.lm, "compute_logits", None) or (lambda h: head_logits(h, self.lm.lm_head.weight))
+        lm = self.lm                             # (a closure over self would keep a dropped engine, and its graphs, until a collection)
+        self._head = getattr(lm, "compute_logits", None) or (lambda h: head_logits(h, lm.lm_head.weight))
         if self.stateful and (prefix_cache_blocks > 0 or lora_modules or tp_group is not None):
             raise ValueError("prefix caching, LoRA modules and tensor parallelism need a plain K/V model: a recurrent "
                              "state cannot be rebuilt from cached K/V chunks")

@@ -15,6 +15,9 @@ kept on the device (no host sync), and the split-K decode-attention grid sized b
 """
 from __future__ import annotations
 
+import contextlib
+import gc
+
 import torch
 
 from ..models.common import KVCache
@@ -28,6 +31,20 @@ def _buckets(max_batch: int) -> list[int]:
         b *= 2
     out.append(max_batch)
     return out
+
+
+@contextlib.contextmanager
+def capture(graph, pool):
+    """``torch.cuda.graph`` with Python's automatic collection off.  The end of a ``CUDAGraph`` waits for the device, which a capture does not
+    allow: one that a collection finds in a dropped reference cycle ends the process, by an exception out of its destructor."""
+    was = gc.isenabled()
+    gc.disable()
+    try:
+        with torch.cuda.graph(graph, pool=pool):
+            yield
+    finally:
+        if was:
+            gc.enable()
 
 
 class DecodeGraphs:
@@ -64,7 +81,7 @@ class DecodeGraphs:
         torch.cuda.current_stream().wait_stream(s)
         for n in reversed(self.buckets):    # largest first: smaller graphs reuse its pool
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, pool=self.pool):
+            with capture(g, self.pool):
                 self.logits[n] = self._forward(n)
             if self.pool is None:
                 self.pool = g.pool()

@@ -392,3 +392,39 @@ def test_packed_prefill_makes_its_indices_once():
     assert isinstance(vars(pp)["pad_idx"], torch.Tensor)
     assert pp.pad_idx.tolist() == [0, 1, 2, 5, 6, 7, 8, 9] and pp.cache_idx.tolist() == [16, 17, 18, 0, 1, 2, 3, 4]
     assert pp.positions.tolist() == [[0, 1, 2, 0, 1, 2, 3, 4]]
+
+
+def test_dropped_engine_goes_without_a_collection():
+    """What an engine holds (captured graphs above all) ends with its last reference, not in a collection in the middle of something else."""
+    import gc
+    import weakref
+    lm = Qwen3ForCausalLM.from_config(qwen3_config("qwen3-tiny")).eval()
+    gc.collect()
+    gc.disable()
+    try:
+        eng = ServingEngine(lm, None, max_batch=2, max_model_len=64, use_graphs=False, start=False)
+        gone = weakref.ref(eng)
+        del eng
+        assert gone() is None
+    finally:
+        gc.enable()
+
+
+def test_capture_runs_without_automatic_collection(monkeypatch):
+    import contextlib
+    import gc
+    from llm_in_practise_amd.infer import graphs
+    monkeypatch.setattr(torch.cuda, "graph", lambda g, pool=None: contextlib.nullcontext())
+    with graphs.capture(None, None):
+        assert not gc.isenabled()
+    assert gc.isenabled()
+    with pytest.raises(ValueError), graphs.capture(None, None):
+        raise ValueError
+    assert gc.isenabled()
+    gc.disable()
+    try:
+        with graphs.capture(None, None):
+            pass
+        assert not gc.isenabled()
+    finally:
+        gc.enable()
