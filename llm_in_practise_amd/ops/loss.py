@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 from . import reference as ref
-from ._native import _functorch_active, eager, fn_apply, native, use_native
+from ._native import eager, fn_apply, native, use_native
 from .gemm import _count, _g4w_ok
 
 
@@ -62,9 +62,9 @@ class _FusedLinearCEFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gloss):
         dh, dw = ctx.saved_tensors
-        # (a gradient of this gradient needs the product as torch's op)
-        own = (dh.dtype == torch.bfloat16 and gloss.dtype == torch.float32 and gloss.is_cuda and dh.is_contiguous() and dh.data_ptr() % 16 == 0
-               and not torch.is_grad_enabled() and not _functorch_active())
+        # (a gradient of this gradient, and one of several rows at once, need the product as torch's op)
+        own = (not torch.is_grad_enabled() and eager(dh, gloss) and dh.dtype == torch.bfloat16 and gloss.dtype == torch.float32 and gloss.is_cuda
+               and dh.is_contiguous() and dh.data_ptr() % 16 == 0)
         return ((native().scale_bf16(dh, gloss) if own else dh * gloss.to(dh.dtype)), (None if dw is None else (dw * gloss).to(torch.bfloat16)),
                 None, None, None, None, None)
 

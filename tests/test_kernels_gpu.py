@@ -226,6 +226,22 @@ def test_fused_linear_ce_groups(native_ext, groups):
     assert rel_err(h.grad, hr.grad) < 2e-2 and rel_err(w.grad, wr.grad) < 2e-2
 
 
+def test_fused_linear_ce_batched_gradients(native_ext):
+    """Several gradients of the loss in one backward (``is_grads_batched``, ``jacobian(vectorize=True)``): each row the gradient times its own
+    factor, as the single backward gives it."""
+    from llm_in_practise_amd.ops.loss import fused_linear_cross_entropy
+    torch.manual_seed(0)
+    h = torch.randn(256, 128, device=DEV).to(torch.bfloat16).requires_grad_(True)
+    w = (0.05 * torch.randn(1000, 128, device=DEV)).to(torch.bfloat16)
+    lab = torch.randint(0, 1000, (256,), device=DEV)
+    loss = fused_linear_cross_entropy(h, w, lab)
+    one, = torch.autograd.grad(loss, h, retain_graph=True)
+    three = torch.tensor([1.0, 0.5, -2.0], device=DEV)
+    got, = torch.autograd.grad(loss, h, three, retain_graph=True, is_grads_batched=True)
+    assert torch.equal(got, three.to(torch.bfloat16)[:, None, None] * one)
+    assert torch.equal(torch.autograd.functional.jacobian(lambda t: fused_linear_cross_entropy(t, w, lab), h.detach(), vectorize=True), one)
+
+
 # ----------------------------------------------------------------------------- optimizer
 def test_adamw_matches_torch(native_ext):
     n = 100_003
