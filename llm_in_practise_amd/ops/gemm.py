@@ -20,7 +20,7 @@ import os
 import torch
 
 from ..quant.nf4 import NF4Weight, dequantize_nf4
-from ._native import _functorch_active, fn_apply, force_reference, native
+from ._native import _functorch_active, eager, fn_apply, force_reference, native
 
 _MIN_M = 256     # training / prefill-sized GEMMs: gemm4w and the fused LoRA paths
 
@@ -191,7 +191,7 @@ def _narrow_rows(x, base, residual):
     4096 × 12288 21.4 / 21.5 and 18.0 / 20.3, 2560 × 9728 18.1 / 16.0 and 12.1 / 15.0.  (5120 × 4096 at 17 / 32: 15.4 / 14.7 and 14.2 / 16.4.)"""
     M, K = x.shape
     N = base.shape[0]
-    if not (x.is_cuda and M <= 64 and N <= 4096 and not _functorch_active() and N % 16 == 0 and K % 64 == 0 and K < 1 << 24 and x.dtype == base.dtype == torch.bfloat16
+    if not (x.is_cuda and M <= 64 and N <= 4096 and N % 16 == 0 and K % 64 == 0 and K < 1 << 24 and eager(x, base, residual) and x.dtype == base.dtype == torch.bfloat16
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and base.is_contiguous() and x.data_ptr() % 16 == 0 and base.data_ptr() % 16 == 0
             and x.get_device() == base.get_device() == torch.cuda.current_device()
             and (residual is None or (residual.dtype == torch.bfloat16 and residual.shape == (M, N) and residual.is_contiguous()
@@ -223,9 +223,10 @@ def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
         return _base_gemm(x, w, ext_a, ext_b, residual)
     M, K = x.shape
     N = base.shape[0]
-    narrow = _narrow_rows(x, base, residual) if M <= 64 else 0
-    if (x.is_cuda and M <= 16 and N <= 8192 and K <= 8192 and N % 16 == 0 and K % 64 == 0 and x.stride(0) % 8 == 0
-            and x.stride(1) == 1 and base.is_contiguous()) or narrow:
+    few = (x.is_cuda and M <= 16 and N <= 8192 and K <= 8192 and N % 16 == 0 and K % 64 == 0 and x.stride(0) % 8 == 0
+           and x.stride(1) == 1 and base.is_contiguous())
+    narrow = _narrow_rows(x, base, residual) if M <= 64 and not few else 0
+    if few or narrow:
         # decode-sized q|k|v / o projections: the weight-streaming MFMA kernel (csrc/kernels/skinny.hip) takes 8.3-9.3 µs for
         # 4096 × 4096 and 1-16 rows, residual included, where hipBLASLt takes 15.3 (12.6-14.2 against 15 for 6144 rows of W,
         # 24 against 29-31 for 8192 × 8192)

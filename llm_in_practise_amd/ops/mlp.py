@@ -24,7 +24,7 @@ from __future__ import annotations
 import torch
 
 from ..quant.nf4 import NF4Weight
-from ._native import _functorch_active, force_reference, native, fn_apply
+from ._native import eager, force_reference, native, fn_apply
 from .checkpoint import _sac_recording, sac_put, sac_take, saves_discarded, tail_skippable
 from .gemm import _MIN_M, _count, _nf4_expand, _nf4_w4, norms_rows
 
@@ -134,9 +134,10 @@ def skinny_swiglu(x: torch.Tensor, gu_base, norm=None, eps: float = 0.0) -> torc
             and not gu_base.requires_grad and gu_base.is_contiguous() and 1 <= x2.shape[0] <= 64 and x2.stride(1) == 1
             and x2.shape[1] <= 4096 and gu_base.shape[0] <= 2 * 14336
             and x2.stride(0) % 8 == 0 and x2.shape[1] % (64 if x2.shape[0] <= 16 else 128) == 0 and gu_base.shape[0] % 32 == 0
+            and (x2.shape[0] <= 16 or eager(x2, gu_base))
             and x2.data_ptr() % 16 == 0 and gu_base.data_ptr() % 16 == 0 and not force_reference()):
         return None
-    if x2.shape[0] > 16 and (_functorch_active() or not x2.get_device() == gu_base.get_device() == torch.cuda.current_device()):
+    if x2.shape[0] > 16 and not x2.get_device() == gu_base.get_device() == torch.cuda.current_device():
         return None
     if x2.shape[0] > 16 and gu_base.shape[0] < 6144 and x2.shape[1] > 1024:
         return None         # (a stage costs what it costs for a tile: 2 × 1024 × 4096, 48 rows, 15.7 µs against 14.3; 2 × 256 × 512 4.3 and 8.7)
