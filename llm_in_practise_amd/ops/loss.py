@@ -41,9 +41,9 @@ class _FusedLinearCEFn(torch.autograd.Function):
             g4w = _g4w_ok(hc, weight, False)
             _count("gemm4w" if g4w else "library")
             logits = native().gemm4w(hc, weight, None, 0, False) if g4w else hc @ weight.t()
-            g0, g1 = s // rows_g, (s + hc.shape[0]) // rows_g
-            row_loss = native().ce_fwd_bwd(logits, labels[s:s + chunk], ignore_index, inv[g0:g1])
-            native().ce_loss(row_loss, inv[g0:g1], loss, s > 0)
+            scale = inv if groups == 1 else inv[s // rows_g:(s + hc.shape[0]) // rows_g]
+            row_loss = native().ce_fwd_bwd(logits, labels[s:s + chunk], ignore_index, scale)
+            native().ce_loss(row_loss, scale, loss, s > 0)
             dx_g4w = g4w and _g4w_ok(logits, weight, True)
             _count("gemm4w" if dx_g4w else "library")
             if dx_g4w:

@@ -242,6 +242,27 @@ def test_fused_linear_ce_batched_gradients(native_ext):
     assert torch.equal(torch.autograd.functional.jacobian(lambda t: fused_linear_cross_entropy(t, w, lab), h.detach(), vectorize=True), one)
 
 
+@pytest.mark.parametrize("T,groups,chunk", [(640, 1, 256), (640, 2, 256), (300, 1, 299), (900, 3, 700), (257, 1, 64)])
+def test_fused_linear_ce_chunks(native_ext, T, groups, chunk):
+    """More rows than a chunk, the last chunk not full, one row group that spans the chunks and several within them: loss, dh and dW in float64."""
+    from llm_in_practise_amd.ops.loss import fused_linear_cross_entropy
+    torch.manual_seed(T)
+    d, V = 128, 1000
+    h = torch.randn(T, d, device=DEV).to(torch.bfloat16).requires_grad_(True)
+    w = (0.05 * torch.randn(V, d, device=DEV)).to(torch.bfloat16).requires_grad_(True)
+    lab = torch.randint(0, V, (T,), device=DEV)
+    lab[: T // groups // 3] = -100
+    loss = fused_linear_cross_entropy(h, w, lab, chunk=chunk, groups=groups)
+    loss.backward()
+    hr, wr = h.detach().double().requires_grad_(True), w.detach().double().requires_grad_(True)
+    lg = (hr @ wr.t()).view(groups, -1, V)
+    ref = sum(F.cross_entropy(lg[g], lab.view(groups, -1)[g], ignore_index=-100) for g in range(groups)) / groups
+    ref.backward()
+    # logits in bf16: each off by 2^-9 of its size (4 at most here); the gradients are rounded to bf16 before their products and after
+    assert abs(loss.item() - ref.item()) < 4 * 2 ** -9 * ref.item()
+    assert rel_err(h.grad, hr.grad) < 2e-2 and rel_err(w.grad, wr.grad) < 2e-2
+
+
 # ----------------------------------------------------------------------------- optimizer
 def test_adamw_matches_torch(native_ext):
     n = 100_003
