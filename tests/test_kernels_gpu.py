@@ -1021,6 +1021,16 @@ def test_lora_dx_without_dropout(native_ext, M, N, K, r, w4, nb):
     assert (dx.double() - want).abs().max() <= (2 ** -8 + 1e-5) * want.abs().max()
 
 
+def test_gemm4w_loradx_refuses_dropout_without_masks(native_ext):
+    """No keep bits mean that everything is kept: a dropout rate beside them would scale by 1 / (1 - p) and mask nothing."""
+    dy, w = torch.randn(256, 128, device=DEV).to(torch.bfloat16), torch.randn(128, 128, device=DEV).to(torch.bfloat16)
+    gs, As = [torch.randn(256, 8, device=DEV) for _ in range(2)], [torch.randn(8, 128, device=DEV).to(torch.bfloat16) for _ in range(2)]
+    for ps in ([0.1, 0.1], [0.0, 0.1]):
+        with pytest.raises(RuntimeError, match="keep bits"):
+            native_ext.gemm4w_loradx(dy, w, None, 0, gs, As, None, ps)
+    native_ext.gemm4w_loradx(dy, w, None, 0, gs, As, None, [0.0, 0.0])
+
+
 @pytest.mark.parametrize("M,N,K,g,sym,splits", [(64, 6144, 4096, 128, False, 0), (256, 4096, 4096, 128, True, 1),
                                               (300, 1024, 512, 64, False, 2), (2048, 4096, 12288, 128, False, 0)])
 def test_gemm4w_int4_affine(native_ext, M, N, K, g, sym, splits):
