@@ -191,7 +191,7 @@ def _narrow_rows(x, base, residual):
     4096 × 12288 21.4 / 21.5 and 18.0 / 20.3, 2560 × 9728 18.1 / 16.0 and 12.1 / 15.0.  (5120 × 4096 at 17 / 32: 15.4 / 14.7 and 14.2 / 16.4.)"""
     M, K = x.shape
     N = base.shape[0]
-    if not (x.is_cuda and M <= 64 and N <= 4096 and N % 16 == 0 and K % 64 == 0 and K < 1 << 24 and eager(x, base, residual) and x.dtype == base.dtype == torch.bfloat16
+    if not (x.is_cuda and 1 <= M <= 64 and N <= 4096 and N % 16 == 0 and K % 64 == 0 and K < 1 << 24 and eager(x, base, residual) and x.dtype == base.dtype == torch.bfloat16
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and base.is_contiguous() and x.data_ptr() % 16 == 0 and base.data_ptr() % 16 == 0
             and x.get_device() == base.get_device() == torch.cuda.current_device()
             and (residual is None or (residual.dtype == torch.bfloat16 and residual.shape == (M, N) and residual.is_contiguous()

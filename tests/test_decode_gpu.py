@@ -244,6 +244,15 @@ def test_narrow_rows(native_ext, M, N, K):
             assert ((gemm._base_gemm(a, w, residual=r).double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all()
 
 
+@pytest.mark.parametrize("N,K", [(4096, 12288), (1024, 8320)])
+def test_no_rows_and_a_deep_narrow_weight(native_ext, N, K):
+    """A product of no rows is an empty one, as the library has it."""
+    from llm_in_practise_amd.ops import gemm
+    x, w = torch.empty(0, K, dtype=torch.bfloat16, device=DEV), torch.zeros(N, K, dtype=torch.bfloat16, device=DEV)
+    for r in (None, torch.empty(0, N, dtype=torch.bfloat16, device=DEV)):
+        assert gemm._base_gemm(x, w, residual=r).shape == (0, N)
+
+
 @pytest.mark.parametrize("M", [17, 32, 33, 49, 64])
 @pytest.mark.parametrize("F,K", [(16, 128), (80, 640), (4112, 384), (8208, 256), (12320, 256), (14336, 128)])
 def test_rows_swiglu(native_ext, M, F, K):
