@@ -1,5 +1,5 @@
 // The gated product of 17 to 64 decode rows, h[M, F] = silu(x·Wgᵀ)·(x·Wuᵀ) of W [2 F, K] (gate above up), every sum one chain of MFMA over K in
-// order: the bits of the library's product of such widths and of the activation behind it.  What bounds it is W from memory and, beside it, x,
+// order, rounded as the product and the activation behind it would be.  What bounds it is W from memory and, beside it, x,
 // which every workgroup reads whole: a workgroup takes as many columns as leave one workgroup for each CU, four tiles of 16 at most.
 //
 //  * a workgroup of 8 waves walks K in stages of 128: its rows of W and x come by LDS-DMA, 4 rows × 256 B an instruction (chunk c of row r
@@ -14,9 +14,12 @@
 //
 // The narrow product y[M, N] = x·Wᵀ (+ residual) of a deep weight has too few columns for that: 256 workgroups of 16 columns each read all of x,
 // at 64 rows four times what they read of W.  There K is summed in four parts that take its units in turns, one workgroup a part and up to 64
-// columns, and a second launch adds the parts in order: the library's order at 17 to 32 rows (units of 128 beyond K = 8192, else 64) and at 64 (units
-// of 64).  µs at 17 / 32 / 64 rows, W cold, the library → here (both launches): 4096 × 12288 23.7 / 28.2 / 36.6 → 22.2 / 23.5 / 28.0, 2560 × 9728
-// 20.0 / 20.0 / 28.0 → 16.1 / 16.5 / 19.2, 1024 × 12288 16.5 / 21.8 / 18.1 → 13.0 / 13.5 / 17.3; at 64 rows 4096 × 4096 14.9 → 12.8, 2560 × 4096 14.2 → 11.3.
+// columns, and a second launch adds the parts in order.  µs at 17 / 32 / 48 / 64 rows, W cold, the library → here (both launches, residual
+// included): 4096 × 12288 26.6 / 30.1 / 35.8 / 39.5 → 23.3 / 25.1 / 25.3 / 26.9, 2560 × 9728 22.4 / 23.6 / 23.7 / 30.9 → 15.8 / 16.9 / 19.0 / 19.5, 1024 × 12288
+// 18.8 / 24.1 / 19.6 / 20.5 → 13.0 / 13.4 / 15.1 / 16.5; at 48 and 64 rows 4096 × 4096 16.2 / 17.8 → 12.2 / 12.8, 2560 × 4096 14.6 / 16.6 → 10.6 / 11.3.
+// Units of 64 and of 128 take the same time within 5 %; a sum is a chain of K / 4 products with either, and off 64 bits by no more than the
+// library's.  For many shapes these are the library's own sums, bit for bit (units of 128 of deep weights up to 32 rows, of 64 at 64 rows), for
+// others not (1024 × 12288 at 64 rows, 4096 × 14336 at 64).
 #include "lds_dma.h"
 
 using namespace lipa;

@@ -182,13 +182,18 @@ def normed_rows(x: torch.Tensor, weight, eps: float, base) -> torch.Tensor | Non
 
 def _narrow_rows(x, base, residual):
     """How the product of up to 64 rows and a narrow bf16 weight runs: 1 in the decode products (csrc/kernels/skinny.hip), 64 or 128 in four
-    parts of units of that depth (csrc/kernels/rows.hip), 0 by what stands below.  Each where it is the fastest, and where its order of sums is
-    the library's (up to 32 rows, and 64) or the weight is short (K < 4096; a chain over all of K would round worse).
-    Library / decode products / parts in µs, W cold, residual included, at 17 / 32 / 64 rows: 4096 × 12288 23.7 / 28.2 / 36.6, 21.2 / 25.9 /
-    35.3 and 22.2 / 23.5 / 28.0, 2560 × 9728 20.0 / 20.0 / 28.0, 18.0 / 19.2 / 26.7 and 16.1 / 16.5 / 19.2, 1024 × 12288 16.5 / 21.8 / 18.1, 17.9 / 22.3 /
-    32.2 and 13.0 / 13.5 / 17.3, 4096 × 4096 13.6 / 12.9 / 14.9, 9.4 / 9.8 / 13.1 and 11.1 / 11.5 / 12.8, 2560 × 4096 12.5 / 12.3 / 14.2, 8.1 / 9.2 / 12.3 and 10.2 /
-    11.0 / 11.3, 1024 × 3072 11.6 / 9.9 / 11.9, 6.0 / 7.3 / 9.9 and 6.7 / 7.2 / 8.4, 4096 × 2048 11.8 / 11.7 / 12.0, 5.9 / 6.3 / 8.1 and 8.0 / 8.5 / 10.5.  At 1 / 16 rows
-    4096 × 12288 21.4 / 21.5 and 18.0 / 20.3, 2560 × 9728 18.1 / 16.0 and 12.1 / 15.0.  (5120 × 4096 at 17 / 32: 15.4 / 14.7 and 14.2 / 16.4.)"""
+    parts of units of that depth (csrc/kernels/rows.hip), 0 by what stands below.  Up to 32 rows and K = 8192, and below K = 4096, the decode
+    products are the fastest or next to it (a chain is K / 4 long there too); deeper weights and more rows take the parts, one launch more, where
+    x is read by a quarter of the workgroups.
+    Library / decode products / parts in µs, W cold, residual included, at 17 / 32 / 48 / 64 rows: 4096 × 12288 26.6 / 30.1 / 35.8 / 39.5, 22.0 / 29.4 /
+    35.2 / 37.0 and 23.3 / 25.1 / 25.3 / 26.9, 2560 × 9728 22.4 / 23.6 / 23.7 / 30.9, 15.7 / 19.2 / 25.0 / 27.1 and 15.8 / 16.9 / 19.0 / 19.5, 1024 × 12288
+    18.8 / 24.1 / 19.6 / 20.5, 17.5 / 21.9 / 29.5 / 31.8 and 13.0 / 13.4 / 15.1 / 16.5, 4096 × 4096 16.1 / 16.1 / 16.2 / 17.8, 8.9 / 9.9 / 12.4 / 13.1 and 11.1 /
+    11.6 / 12.2 / 12.8, 2560 × 4096 14.8 / 14.5 / 14.6 / 16.6, 7.8 / 9.1 / 11.5 / 12.3 and 10.3 / 10.7 / 10.6 / 11.3, 1024 × 3072 13.5 / 11.8 / 13.6 / 13.8, 6.0 /
+    7.3 / 9.1 / 9.7 and 6.7 / 7.1 / 7.8 / 8.1.  At 1 / 16 rows library and decode products 4096 × 12288 21.4 / 21.5 and 18.0 / 20.3, 2560 × 9728 18.1 / 16.0 and
+    12.1 / 15.0.  (5120 × 4096 at 17 / 32: 15.4 / 14.7 and 14.2 / 16.4.)
+    Error against 64 bits, residual included: 1.65e-3 to 1.67e-3 from all three; results that are not the exact one rounded, per 100 000, library
+    and here: 4096 × 12288 33 and 33 at 32 rows, 44 and 33 at 48, 39 and 39 at 64, 4096 × 4096 16 and 16, 26 and 18, 18 and 18, 2560 × 9728 33 and 33, 28 and
+    28, 34 and 34 (of 500 000 results or more)."""
     M, K = x.shape
     N = base.shape[0]
     if not (x.is_cuda and 1 <= M <= 64 and N <= 4096 and N % 16 == 0 and K % 64 == 0 and K < 1 << 24 and eager(x, base, residual) and x.dtype == base.dtype == torch.bfloat16
@@ -201,7 +206,7 @@ def _narrow_rows(x, base, residual):
         return int(K > 8192 and K % 128 == 0)
     if K < 4096 or (M <= 32 and K <= 8192):
         return 1
-    return 0 if K % 512 or 32 < M < 64 else 128 if M <= 32 else 64
+    return 0 if K % 512 else 128 if M <= 32 else 64
 
 
 def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):

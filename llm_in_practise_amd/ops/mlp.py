@@ -124,8 +124,8 @@ def skinny_swiglu(x: torch.Tensor, gu_base, norm=None, eps: float = 0.0) -> torc
     where they do not serve: a bf16 [gate | up] weight, no gradient.  The products are rounded to bf16 before the activation, as the
     separate kernels round them.  Library and activation → here, µs at 1 / 16 / 17 / 64 rows: 4096 → 2 × 12288 48 / 49 / 48 / 49 → 32 / 33 / 40 / 40,
     2560 → 2 × 9728 48 / 48 / 27 / 30 → 21 / 22 / 21 / 23, 1024 → 2 × 3072 10 / 10 / 14 / 14 → 4.6 / 4.9 / 6.4 / 7.0, 4096 → 2 × 14336 67 / 69 / 56 / 55 →
-    40 / 41 / 46 / 47.  (skinny.hip takes 37 / 48 at 17 / 64 rows of 2 × 12288, in an order of sums that is not the library's there.)  Wider and
-    deeper weights, and more rows, stay with the library's product.  With ``norm`` the rows stand in front of the RMSNorm of that weight, which
+    40 / 41 / 46 / 47.  (skinny.hip takes 37 / 48 at 17 / 64 rows of 2 × 12288, in units in turns: not the one chain over K that rows.hip has, and that
+    the library's products of the 4B and 8B models' widths were seen to have.)  Wider and deeper weights, and more rows, stay with the library's product.  With ``norm`` the rows stand in front of the RMSNorm of that weight, which
     the launch forms bit for bit as its own kernel does (:func:`~.gemm.norms_rows`; else None): 39.7 → 37.3 µs, 25.8 → 22 and 6.8 → 5.4 at 1 row
     before the weight's loads passed the caches by, norm included."""
     x2 = x.reshape(-1, x.shape[-1])

@@ -244,6 +244,29 @@ def test_narrow_rows(native_ext, M, N, K):
             assert ((gemm._base_gemm(a, w, residual=r).double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all()
 
 
+@pytest.mark.parametrize("N,K,form", [(4096, 12288, (128, 64)), (1024, 8704, (128, 64)), (4096, 4096, (1, 64)), (2048, 8192, (1, 64)), (1024, 3072, (1, 1)),
+                                      (1024, 8320, (0, 0))])
+def test_narrow_rows_rule_has_no_row_count_of_its_own(native_ext, N, K, form):
+    """One form from 17 to 32 rows and one from 33 to 64, whatever their number (a server's largest batch is any number)."""
+    from llm_in_practise_amd.ops import gemm
+    w, x = torch.zeros(N, K, dtype=torch.bfloat16, device=DEV), torch.zeros(64, K, dtype=torch.bfloat16, device=DEV)
+    assert [gemm._narrow_rows(x[:m], w, None) for m in range(17, 65)] == [form[0]] * 16 + [form[1]] * 32
+
+
+@pytest.mark.parametrize("M", [33, 40, 48, 63, 64])
+@pytest.mark.parametrize("N,K", [(4096, 4096), (2560, 9728), (1024, 4608)])
+def test_narrow_rows_round_as_well_as_the_library(native_ext, M, N, K):
+    """Results that are not the exact one rounded to bf16: no more than from the library's product, but for the chance of their number (three
+    standard deviations of a count)."""
+    from llm_in_practise_amd.ops import gemm
+    torch.manual_seed(N + M)
+    x, r = torch.randn(M, K, device=DEV).to(torch.bfloat16), torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV) * 0.02).to(torch.bfloat16)
+    right = (x.double() @ w.double().t() + r.double()).to(torch.bfloat16)
+    here, there = ((y != right).sum().item() for y in (gemm._base_gemm(x, w, residual=r), torch.addmm(r, x, w.t())))
+    assert gemm._narrow_rows(x, w, r) == 64 and here <= there + 3 * (here + there + 1) ** 0.5
+
+
 @pytest.mark.parametrize("N,K", [(4096, 12288), (1024, 8320)])
 def test_no_rows_and_a_deep_narrow_weight(native_ext, N, K):
     """A product of no rows is an empty one, as the library has it."""
