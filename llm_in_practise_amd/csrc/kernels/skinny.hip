@@ -239,15 +239,14 @@ static void launch_rows(const void* X, int ldx, const void* W, const void* res, 
   gemm_skinny_k<CT_, 1, NW_, RING_, GLU_, CUT_, PARTS_, NORM><<<(N + 15) / 16, 64 * NW_, extra, st>>>(                     \
       (const bf16*)X, ldx, (const bf16*)W, (const bf16*)res, (bf16*)out, M, N, K, pieces, nrm)
   if constexpr (!NORM) {                        // (rows that are normed here have 4096 elements at most: 16 pieces of 256)
-    // Deep weights: the four parts of 128-deep units that the library's product sums there, a wave each with a long ring (one workgroup a CU, with
+    // Deep weights: four parts of 128-deep units in turns, a wave each with a long ring (one workgroup a CU, with
     // all of its LDS).  In pieces 4096 × 12288 took 18.0 / 21.2 µs at 1 / 16 rows, and takes 18.0 / 20.3; 2560 × 9728 16.0 / 20.2, and 12.1 / 15.0.
     if (!glu && K > 8192 && K % 128 == 0) {
       L(1, 4, 8, false, TURNS128, 4);
       return;
     }
-    if (!glu && pieces > 16) {
-      if (pieces > 32) L(1, 4, 4, false, TURNS64, 4);
-      else L(1, 8, 3, false, PIECES, 32);
+    if (!glu && pieces > 16) {                  // (32, of K = 8192 alone: any K with more of them is deeper and a multiple of 128)
+      L(1, 8, 3, false, PIECES, 32);
       return;
     }
   }
