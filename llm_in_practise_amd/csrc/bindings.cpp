@@ -728,9 +728,9 @@ optional<Tensor> w4mm_swiglu(Tensor x, Tensor codes, Tensor sc2, int64_t N, int6
   return out;
 }
 
-// Does one launch serve w4mm (glu: w4mm_swiglu)?
-bool w4mm_one(int64_t M, int64_t N, int64_t K, bool glu) {
-  return w4row_serves((int)M, (int)(glu ? N / 2 : N), (int)K, w4mm_nkb((int)M, (int)N, (int)K), glu);
+// Does one launch serve w4mm (glu: w4mm_swiglu) with slices of nkb blocks (0: those that it takes by itself)?
+bool w4mm_one(int64_t M, int64_t N, int64_t K, bool glu, int64_t nkb) {
+  return w4row_serves((int)M, (int)(glu ? N / 2 : N), (int)K, nkb > 0 ? (int)nkb : w4mm_nkb((int)M, (int)N, (int)K), glu);
 }
 
 // The decode-batch tiling of the same W4A16 GEMM (w4mm.hip w4g_k): 1 <= M <= 64, same operands as w4mm.
@@ -1944,7 +1944,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("w4mm", &w4mm, py::arg("x"), py::arg("codes"), py::arg("sc2"), py::arg("N"), py::arg("gs"),
         py::arg("residual") = py::none(), py::arg("nkb") = 0, py::arg("one") = true);
   m.def("w4mm_ok", &w4mm_ok);
-  m.def("w4mm_one", &w4mm_one);
+  m.def("w4mm_one", &w4mm_one, py::arg("M"), py::arg("N"), py::arg("K"), py::arg("glu"), py::arg("nkb") = 0);
   m.def("w4mm_swiglu", &w4mm_swiglu);
   m.def("w4g", &w4g, py::arg("x"), py::arg("codes"), py::arg("sc2"), py::arg("N"), py::arg("gs"),
         py::arg("residual") = py::none(), py::arg("ks") = 0);

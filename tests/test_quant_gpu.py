@@ -95,6 +95,7 @@ def test_w4mm_one_launch_only_where_it_is_not_slower(native_ext, M, N, K, glu, o
 @pytest.mark.parametrize("nkb", [2, 4])
 @pytest.mark.parametrize("N,K,gs", [(4096, 1024, 128), (640, 2560, 128), (4096, 4096, 256), (2560, 5120, 128)])
 def test_w4mm_one_launch_has_the_bits_of_the_slices(native_ext, M, nkb, N, K, gs):
+    assert native_ext.w4mm_one(M, N, K, False, nkb) == (M <= 16 or K <= 4096)      # (else both are the slices' kernel)
     torch.manual_seed(M + nkb)
     w = quantize_rtn(torch.randn(N, K, device=DEV), gs, False)
     x, res = torch.randn(M, K, device=DEV).to(torch.bfloat16), torch.randn(M, N, device=DEV).to(torch.bfloat16)
@@ -109,6 +110,7 @@ def test_w4mm_one_launch_has_the_bits_of_the_slices(native_ext, M, nkb, N, K, gs
 def test_w4mm_one_launch_rings(native_ext, nkb, N, K, gs, M):
     """More units than a ring holds and fewer, ragged shares of slices and tiles, groups of several blocks, an odd number of them, a
     table that 16-byte loads cannot take, rows of x that are a slice of wider ones or all the same one: the bits of the slices' kernel."""
+    assert native_ext.w4mm_one(M, N, K, False, nkb) == (M <= 16 or K <= 4096)      # (17 rows of a long K: both are the slices' kernel)
     torch.manual_seed(M + K)
     w = quantize_rtn(torch.randn(N, K, device=DEV), gs, False)
     table = w.w4mm_table()
