@@ -88,7 +88,8 @@ def fused_linear_cross_entropy(h: torch.Tensor, weight: torch.Tensor, labels: to
 
 def shift_labels(labels: torch.Tensor, ignore_index: int = -100) -> torch.Tensor:
     """HF causal-LM convention: position t predicts token t+1; last position ignored."""
-    if eager(labels) and labels.is_cuda and labels.dtype == torch.int64 and labels.dim() and labels.is_contiguous() and use_native(labels):
+    if (eager(labels) and labels.is_cuda and labels.dtype == torch.int64 and labels.dim() and labels.is_contiguous() and labels.numel() < 1 << 31
+            and use_native(labels)):                               # (a grid of one thread a label ends at 2^32, the kernel's row at 2^31)
         return native().shift_labels(labels, ignore_index)
     out = torch.full_like(labels, ignore_index)
     out[..., :-1] = labels[..., 1:]

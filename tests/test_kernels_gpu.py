@@ -226,6 +226,20 @@ def test_fused_linear_ce_groups(native_ext, groups):
     assert rel_err(h.grad, hr.grad) < 2e-2 and rel_err(w.grad, wr.grad) < 2e-2
 
 
+def test_shift_labels_longer_than_a_launch(native_ext):
+    """Labels past what one launch counts, 17 GB of them, keep torch's operations."""
+    from llm_in_practise_amd.ops.loss import shift_labels
+    n = (1 << 31) + 5
+    if torch.cuda.mem_get_info()[0] < 6 * 8 * n:
+        pytest.skip("needs 100 GB of free GPU memory")
+    labels = torch.empty(n, dtype=torch.int64, device=DEV)
+    labels[:2], labels[-2:] = 7, 9
+    out = shift_labels(labels)
+    assert out[0] == 7 and out[-3:].tolist() == [9, 9, -100]
+    del labels, out
+    torch.cuda.empty_cache()
+
+
 def test_fused_linear_ce_batched_gradients(native_ext):
     """Several gradients of the loss in one backward (``is_grads_batched``, ``jacobian(vectorize=True)``): each row the gradient times its own
     factor, as the single backward gives it."""
