@@ -516,7 +516,8 @@ __global__ __launch_bounds__(256) void k_moe_combine(const T* __restrict__ ys, c
 
 // The same, four columns per thread (16-byte or 8-byte accesses); a token's ids, rows and weights are read once into LDS.  Its rows, N at a time (a
 // choice of no expert reads h's and leaves it), are loaded together, and the sums leave nothing in the caches: one by one behind branches, and kept,
-// 8000 tokens of 2048 with two choices took 28.0 µs, and take 22.9 (5.7 TB/s); four and a shared expert 44.5 → 39.1, 3000 with two 10.3 → 9.4.
+// 8000 tokens of 2048 with two choices took 28.0 µs, and take 22.9 (5.7 TB/s; 26 in a call, behind the experts'
+// products); four and a shared expert 44.5 → 39.1, 3000 with two 10.3 → 9.4.
 // (The rows as loads that leave nothing: 27.6, they have just been written.)
 constexpr int MAXTOP = 64;
 template <typename T, int N>
@@ -585,7 +586,7 @@ void seq_route_fused(int code, const void* h, int ldh, const float* router, cons
   if (T_ == 0) return;
   const auto fits = [](const void* p, int b) { return ((uintptr_t)p & (b - 1)) == 0; };
   // us, a block's four tokens (rows above 8 KB and few tokens: a block per token) -> tiles of 16: 256 / 2000 / 8000 tokens of width 2048, 8
-  // outputs 6.8 -> 6.4, 7.3 -> 6.7, 15.5 -> 9.7 (15.2 -> 9.1), 16 outputs 9.5 -> 8.3, 10.5 -> 8.7, 29.7 -> 12.2; 1000 of 8192 17.5 -> 14.8.
+  // outputs 6.8 -> 6.4, 7.3 -> 6.7, 15.5 -> 9.7 (15.2 -> 9.1; 13 with rows that come from memory), 16 outputs 9.5 -> 8.3, 10.5 -> 8.7, 29.7 -> 12.2; 1000 of 8192 17.5 -> 14.8.
   // Short rows and few outputs give a wave too little to do to make up for the way through LDS: 1000 tokens of width 1024, 8 outputs 4.7 -> 5.2 (not
   // taken), 8000 8.6 -> 6.5; 4 outputs of 4096 7.7 -> 8.1 (not taken), 8000 17.5 -> 17.0.  Error of the weights against 64 bits as before (0.7e-7).
   if (T_ >= 256 && ((long)T_ * n >= 40000 || (W > 1024 && n > 4)) && code == 0 && n <= 16 && top + always <= 16 && W % 64 == 0 && ldh % 8 == 0 &&

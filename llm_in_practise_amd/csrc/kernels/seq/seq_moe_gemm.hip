@@ -3,8 +3,8 @@
 // gathers its rows of the input as it loads them and ends in the gated activation, so neither the gathered input nor the gate
 // and up products ever stand in memory.
 //
-// 8000 tokens of width 2048, 8 experts of 384, top 2 (75 GFLOP): 638 -> 155 us with routing and the weighted sum: order 5.5, first
-// products 61 (820 TFLOP/s), second 42 (600), sum 27, routing 17.  100 tokens: 533 -> 40 us.  The sort, the host's read of the run lengths
+// 8000 tokens of width 2048, 8 experts of 384, top 2 (75 GFLOP): 638 -> 143 us with routing and the weighted sum: order 5, first
+// products 60 (840 TFLOP/s), second 40 (630), sum 26, routing 13 (171 where the inputs come from memory).  100 tokens: 533 -> 40 us.  The sort, the host's read of the run lengths
 // and a vendor product pair, an activation and their launch gaps per expert took 500 us at any number of tokens.
 #include "seq_common.h"
 

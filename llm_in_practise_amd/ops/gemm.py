@@ -183,8 +183,8 @@ def normed_rows(x: torch.Tensor, weight, eps: float, base) -> torch.Tensor | Non
 def _narrow_rows(x, base, residual):
     """How the product of up to 64 rows and a narrow bf16 weight runs: 1 in the decode products (csrc/kernels/skinny.hip), 64 or 128 in four
     parts of units of that depth (csrc/kernels/rows.hip), 0 by what stands below.  Up to 32 rows and K = 8192, and below K = 4096, the decode
-    products are the fastest or next to it (a chain is K / 4 long there too); deeper weights and more rows take the parts, one launch more, where
-    x is read by a quarter of the workgroups.
+    products are the fastest or within 10 % of it (1024 × 3072 from 40 rows on 10 to 20 %; it is left at one launch); deeper weights and more rows take
+    the parts, one launch more, where x is read by a quarter of the workgroups.
     Library / decode products / parts in µs, W cold, residual included, at 17 / 32 / 48 / 64 rows: 4096 × 12288 26.6 / 30.1 / 35.8 / 39.5, 22.0 / 29.4 /
     35.2 / 37.0 and 23.3 / 25.1 / 25.3 / 26.9, 2560 × 9728 22.4 / 23.6 / 23.7 / 30.9, 15.7 / 19.2 / 25.0 / 27.1 and 15.8 / 16.9 / 19.0 / 19.5, 1024 × 12288
     18.8 / 24.1 / 19.6 / 20.5, 17.5 / 21.9 / 29.5 / 31.8 and 13.0 / 13.4 / 15.1 / 16.5, 4096 × 4096 16.1 / 16.1 / 16.2 / 17.8, 8.9 / 9.9 / 12.4 / 13.1 and 11.1 /
