@@ -719,7 +719,7 @@ __global__ __launch_bounds__(256, 3) void k_chunk_out(const bf16* __restrict__ q
   const float skip = MLSTM ? 0.f : ga.dskip[hd];
   // (a store that has no place goes past the end of its window and is dropped.  The outputs leave nothing in the caches, which hold the states that
   // other blocks are about to read: state space, 4093 tokens 93.4 -> 91.8 us, 8 prompts of 333 to 1024 169.7 -> 159; mLSTM, the same 82.1 -> 80.1.
-  // (Calls on the same inputs, which then stay in the last cache; on inputs from memory 4093 tokens take 104 and the mLSTM 95, as before.)  The
+  // (Calls on the same inputs, which then stay in the last cache; on inputs from memory 4093 tokens take 109 to 117 and the mLSTM 98, as before.)  The
   // states, just written, as loads that leave nothing: 99.5 and 165.)
   const auto win = __builtin_amdgcn_make_buffer_rsrc(out + ((size_t)t0 * H + hd) * dv, 0, ((n - 1) * H + 1) * dv * 4, 0x00020000);
 #pragma unroll
