@@ -17,58 +17,20 @@
 // The first case reads and writes 335 MB, 235 of them states and outputs, of which a copy moves 5 TB/s.  With every chunk's contribution
 // walked by itself (69 MB of states out, in, out and in), operands of the outputs loaded from memory rows as they are needed, an
 // exponential for each score and splits by rounding it took 150 us (46, 25, 80).
-#include "seq_common.h"
+#include "seq_gates.h"
 
 #include <algorithm>
 #include <type_traits>
 
 using namespace lipa;
 
+size_t seq_walk_floats(int, int, int, int, int, int, size_t);
+void seq_walk(bool, const void*, int, const void*, int, const void*, int, const GateArgs&, float*, float*, float*, float*, float*, float*, float*, size_t,
+              int, int, int, int, int, const SeqDesc&, hipStream_t);
+
 namespace {
 
 constexpr int CK = 128;                 // tokens of a chunk (4 waves x 32 queries)
-constexpr double LOG2E = 1.4426950408889634074;
-
-__device__ __forceinline__ double shfl_up_d(double v, int o) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __shfl_up((int)b, o, 64), hi = __shfl_up((int)(b >> 32), o, 64);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double last_lane_d(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-// v of a lane further down (CTRL: by 1, 2, 4, 8 within a row of 16, or a row's last lane to the rows behind it), `none` where there is none
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double from_below(double v, double none) {
-  const long long b = __double_as_longlong(v), z = __double_as_longlong(none);
-  const int lo = __builtin_amdgcn_update_dpp((int)z, (int)b, CTRL, ROWS, 0xF, false),
-            hi = __builtin_amdgcn_update_dpp((int)(z >> 32), (int)(b >> 32), CTRL, ROWS, 0xF, false);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-// op over a lane and those in front of it: a scan without a trip through LDS per step (6.5 -> 3.5 thousand cycles for a chunk's gates)
-template <typename Op>
-__device__ __forceinline__ double scan_lanes(double v, double none, Op op) {
-  v = op(v, from_below<0x111, 0xF>(v, none));      // row_shr 1, 2, 4, 8
-  v = op(v, from_below<0x112, 0xF>(v, none));
-  v = op(v, from_below<0x114, 0xF>(v, none));
-  v = op(v, from_below<0x118, 0xF>(v, none));
-  v = op(v, from_below<0x142, 0xA>(v, none));      // row_bcast 15 into rows 1 and 3, row_bcast 31 into rows 2 and 3
-  v = op(v, from_below<0x143, 0xC>(v, none));
-  return v;
-}
-
-struct GateArgs {
-  // state space: dt (bf16, row stride lddt), per head bias and log rate
-  const bf16* dt;
-  int lddt;
-  const float *dt_bias, *a_log, *dskip;
-  // mLSTM: gate pre-activations [T, H], per head biases, cap
-  const float *ipre, *fpre, *ib, *fb;
-  float cap, qscale;
-  int H;
-};
 
 struct Gate {                           // of a wave's lane: tokens 2 * lane and 2 * lane + 1, in powers of two
   double F0, F1, Fc;                    // log decays from the chunk's start, and of the whole chunk
@@ -149,11 +111,6 @@ struct Ws {
   int sc;
 };
 
-// The 8-byte transposed read: of 16 lanes, lane l gets column l of the four rows that lanes 0, 4, 8, 12 point into.
-__device__ __forceinline__ bf16x4 read_tr(const bf16* p) {
-  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
-  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
-}
 // Where the 16-byte piece x8 of row r stands in an unpadded row of COLS bf16.  Transposed reads take four rows by two blocks of 16
 // columns at a time, operand reads 16 rows of one piece: both then meet every bank once.
 template <int COLS>
@@ -789,7 +746,9 @@ void chunk_launch(const bf16* q, int ldq, const bf16* k, int ldk, const bf16* v,
 template <bool MLSTM>
 void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const GateArgs& ga, float* S, float* N,
                     float* M, float* out, float* den, float* efl, float* ws, size_t most, int H, int G, int dk, int dv,
-                    SeqDesc d, hipStream_t st) {
+                    int longest, SeqDesc d, hipStream_t st) {
+  if (seq_walk_floats(d.Ttot, d.B, H, dk, dv, longest, most) > 0)
+    return seq_walk(MLSTM, q, ldq, k, ldk, v, ldv, ga, S, N, M, out, den, efl, ws, most, H, G, dk, dv, longest, d, st);
 #define CHUNK(NK_)                                                                                                          \
   chunk_launch<NK_, MLSTM>((const bf16*)q, ldq, (const bf16*)k, ldk, (const bf16*)v, ldv, ga, S, N, M, out, den, efl, ws, \
                            most, H, G, dv, d, st)
@@ -808,7 +767,7 @@ void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* 
 // that are no multiple of 32 or above 128, rows that 16-byte (q, k, the states S and N) or 8-byte (v) loads cannot take, and steps of
 // few tokens a sequence.  At most `most`: longer steps run in windows.
 size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const void* S,
-                        const void* N, int T_, int B, int H, int dk, int dv, size_t most) {
+                        const void* N, int T_, int B, int H, int dk, int dv, int longest, size_t most) {
   const auto fits = [](const void* p, int ld, int n) { return ld % n == 0 && ((uintptr_t)p & (2 * n - 1)) == 0; };
   if (code != 0 || dk % 32 != 0 || dk > 128 || dv % 4 != 0 || (long)H * dv >= 1l << 22 || std::max({ldq, ldk, ldv}) >= 1 << 22 ||
       !fits(q, ldq, 8) || !fits(k, ldk, 8) || !fits(v, ldv, 4) ||
@@ -826,6 +785,7 @@ size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk
   if (pairs >= 1024 && (dk <= 64 || dv <= 32)) least = 192;
   if (pairs * dv >= 1l << 17 && dk <= 32) least = 256;
   if (B == 0 || T_ < least * B) return 0;
+  if (const size_t n = seq_walk_floats(T_, B, H, dk, dv, longest, most)) return n;      // (the state never leaves its block)
   const int sc = run_chunks(T_, B, H, dv);
   const size_t slots = run_plan(T_, B, H, dk, dv, sc, most).slots;
   return slots == 0 ? 0 : slots * run_floats(sc, H, dk, dv) + 4;
@@ -833,15 +793,14 @@ size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk
 
 void seq_chunk_ssd(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const void* dt, int lddt,
                    const float* dt_bias, const float* a_log, const float* dskip, float* S, float* out, float* ws, size_t most,
-                   int H, int G, int dk, int dv, SeqDesc d, hipStream_t st) {
+                   int H, int G, int dk, int dv, int longest, SeqDesc d, hipStream_t st) {
   const GateArgs ga = {(const bf16*)dt, lddt, dt_bias, a_log, dskip, nullptr, nullptr, nullptr, nullptr, 1.f, 1.f, H};
-  chunk_dispatch<false>(q, ldq, k, ldk, v, ldv, ga, S, nullptr, nullptr, out, nullptr, nullptr, ws, most, H, G, dk, dv, d,
-                        st);
+  chunk_dispatch<false>(q, ldq, k, ldk, v, ldv, ga, S, nullptr, nullptr, out, nullptr, nullptr, ws, most, H, G, dk, dv, longest, d, st);
 }
 
 void seq_chunk_mlstm(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* ipre, const float* fpre,
                      const float* ib, const float* fb, float cap, float qscale, float* S, float* N, float* M, float* out,
-                     float* den, float* efl, float* ws, size_t most, int H, int dk, int dv, SeqDesc d, hipStream_t st) {
+                     float* den, float* efl, float* ws, size_t most, int H, int dk, int dv, int longest, SeqDesc d, hipStream_t st) {
   const GateArgs ga = {nullptr, 0, nullptr, nullptr, nullptr, ipre, fpre, ib, fb, cap, qscale, H};
-  chunk_dispatch<true>(q, ldq, k, ldk, v, ldv, ga, S, N, M, out, den, efl, ws, most, H, H, dk, dv, d, st);
+  chunk_dispatch<true>(q, ldq, k, ldk, v, ldv, ga, S, N, M, out, den, efl, ws, most, H, H, dk, dv, longest, d, st);
 }

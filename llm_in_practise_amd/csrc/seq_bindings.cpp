@@ -102,13 +102,14 @@ void seq_delta_scan(int, const void*, int, const void*, int, const void*, int, c
 void seq_talk_attention(int, const void*, int, const void*, const void*, float*, float*, float*, const float*,
                         const void*, int, void*, int, int, int, int, int, int, float, const int*, const int*, int,
                         SeqDesc, hipStream_t);
-size_t seq_chunk_floats(int, const void*, int, const void*, int, const void*, int, const void*, const void*, int, int, int, int, int,
+size_t seq_chunk_floats(int, const void*, int, const void*, int, const void*, int, const void*, const void*, int, int, int, int, int, int,
                         size_t);
+int seq_walk_tiles(int, int, int, int, int, int);
 void seq_chunk_ssd(const void*, int, const void*, int, const void*, int, const void*, int, const float*, const float*,
-                   const float*, float*, float*, float*, size_t, int, int, int, int, SeqDesc, hipStream_t);
+                   const float*, float*, float*, float*, size_t, int, int, int, int, int, SeqDesc, hipStream_t);
 void seq_chunk_mlstm(const void*, int, const void*, int, const void*, int, const float*, const float*, const float*,
                      const float*, float, float, float*, float*, float*, float*, float*, float*, float*, size_t, int, int, int,
-                     SeqDesc, hipStream_t);
+                     int, SeqDesc, hipStream_t);
 size_t seq_block_floats(int, bool, const void*, int, const void*, int, const void*, const void*, const void*, int, int, int, int,
                         int, size_t);
 void seq_block_delta(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float*, float*, float*,
@@ -336,7 +337,7 @@ constexpr int64_t MOST_WS = 1ll << 28;
 
 std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor fpre, Tensor ib, Tensor fb, double cap,
                   double qscale, Tensor S, Tensor N, Tensor M, int64_t H, std::vector<Tensor> desc,
-                  optional<Tensor> live, int64_t most) {
+                  optional<Tensor> live, int64_t most, int64_t longest) {
   const int code = code_of(q);
   const int64_t T = q.size(0);
   TORCH_CHECK(q.dim() == 2 && q.size(1) % H == 0 && v.dim() == 2 && v.size(1) % H == 0, "q/k/v: [T, H * d]");
@@ -359,12 +360,12 @@ std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor
   auto out = at::empty({T, H, dv}, S.options());
   auto den = at::empty({T, H}, S.options()), efl = at::empty({T, H}, S.options());
   if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), S.data_ptr(),
-                                        N.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (size_t)most)) {
+                                        N.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_chunk_mlstm(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
                     fpre.data_ptr<float>(), ib.data_ptr<float>(), fb.data_ptr<float>(), (float)cap, (float)qscale,
                     S.data_ptr<float>(), N.data_ptr<float>(), M.data_ptr<float>(), out.data_ptr<float>(), den.data_ptr<float>(),
-                    efl.data_ptr<float>(), ws.data_ptr<float>(), (size_t)most, (int)H, (int)dk, (int)dv, d, stream());
+                    efl.data_ptr<float>(), ws.data_ptr<float>(), (size_t)most, (int)H, (int)dk, (int)dv, (int)longest, d, stream());
     return {out, den, efl};
   }
   if (seq_mlstm_step(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
@@ -457,7 +458,7 @@ Tensor talk_attention(Tensor q, Tensor kc, Tensor vc, Tensor talk, Tensor gate, 
 
 // ---- selective state space (state-space duality form): q = C, k = B [T, G * N], v = x [T, H * P], dtraw [T, H]
 Tensor ssd_scan(Tensor q, Tensor k, Tensor v, Tensor dtraw, Tensor dt_bias, Tensor a_log, Tensor dskip, Tensor S,
-                int64_t H, int64_t G, std::vector<Tensor> desc, optional<Tensor> live, int64_t most) {
+                int64_t H, int64_t G, std::vector<Tensor> desc, optional<Tensor> live, int64_t most, int64_t longest) {
   const int code = code_of(q);
   const int64_t T = q.size(0);
   TORCH_CHECK(G >= 1 && H % G == 0 && q.dim() == 2 && q.size(1) % G == 0 && v.dim() == 2 && v.size(1) % H == 0,
@@ -476,11 +477,11 @@ Tensor ssd_scan(Tensor q, Tensor k, Tensor v, Tensor dtraw, Tensor dt_bias, Tens
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H * dv}, S.options());
   if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), S.data_ptr(), nullptr,
-                                        (int)T, d.B, (int)H, (int)dk, (int)dv, (size_t)most)) {
+                                        (int)T, d.B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_chunk_ssd(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), dtraw.data_ptr(), ld(dtraw),
                   dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), dskip.data_ptr<float>(), S.data_ptr<float>(),
-                  out.data_ptr<float>(), ws.data_ptr<float>(), (size_t)most, (int)H, (int)G, (int)dk, (int)dv, d, stream());
+                  out.data_ptr<float>(), ws.data_ptr<float>(), (size_t)most, (int)H, (int)G, (int)dk, (int)dv, (int)longest, d, stream());
     return out;
   }
   seq_ssd_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), dtraw.data_ptr(), ld(dtraw),
@@ -1293,13 +1294,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias") = py::none());
   m.def("mlstm_scan", &mlstm_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("ipre"), py::arg("fpre"), py::arg("ib"),
         py::arg("fb"), py::arg("cap"), py::arg("qscale"), py::arg("S"), py::arg("N"), py::arg("M"), py::arg("H"),
-        py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS);
+        py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS, py::arg("longest") = 0);
   m.def("delta_scan", &delta_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("g"), py::arg("bpre"), py::arg("S"),
         py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS);
   m.def("talk_attention", &talk_attention);
   m.def("ssd_scan", &ssd_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("dtraw"), py::arg("dt_bias"),
         py::arg("a_log"), py::arg("dskip"), py::arg("S"), py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"),
-        py::arg("most") = MOST_WS);
+        py::arg("most") = MOST_WS, py::arg("longest") = 0);
   m.def("embed_pair", &embed_pair, py::arg("tok"), py::arg("table"), py::arg("pair"), py::arg("prev"), py::arg("scale"),
         py::arg("mul_prev"), py::arg("mul_cur"), py::arg("desc"), py::arg("live"), py::arg("out") = py::none());
   m.def("scaled_postnorm", &scaled_postnorm);
@@ -1323,13 +1324,19 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("residual_dyt", &residual_dyt);
   m.def("softcap_", &softcap_);
   // workspace of a step through the chunked ("ssd", "mlstm") or blocked ("delta", "gla") form, bf16 rows that its loads take; 0: token by token
-  m.def("scan_floats", [](const std::string& op, int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most) {
+  m.def("scan_floats", [](const std::string& op, int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most, int64_t longest) {
     if (op == "ssd" || op == "mlstm")
-      return (int64_t)seq_chunk_floats(0, nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most);
+      return (int64_t)seq_chunk_floats(0, nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most);
     TORCH_CHECK(op == "delta" || op == "gla", "scan_floats: ssd, mlstm, delta or gla");
     return (int64_t)seq_block_floats(0, op == "delta", nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H,
                                      (int)dk, (int)dv, (size_t)most);
-  }, py::arg("op"), py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS);
+  }, py::arg("op"), py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS, py::arg("longest") = 0);
+  // columns of a block that walks the tokens with the state at hand ("ssd", "mlstm"), 0: chunks, or token by token
+  m.def("scan_walk", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t longest) {
+    if (seq_chunk_floats(0, nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)MOST_WS) == 0)
+      return 0;
+    return 16 * seq_walk_tiles((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest);
+  });
   m.def("delta_block", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most) {      // tokens of a block, 0: token by token
     if (seq_block_floats(0, true, nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most) == 0) return 0;
     return seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most) > 0 ? 32 : 16;

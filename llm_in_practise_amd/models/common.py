@@ -305,6 +305,7 @@ class SeqBatch:
         self.B, self.T = int(desc[1].numel()), T
         self.max_pos = cache.max_len if max_pos is None else max_pos      # bound on any key position this step
         self.decode = host is None
+        self.longest = 1 if host is None else max((b - a for a, b in zip(host[0], host[0][1:])), default=0)      # tokens of one sequence
         self.positions = desc[4][None]
         self.len, self.pos = 0, None                                      # KVCache duck-typing (unused)
         # a sequence that continues with more than one token: blocks of a kernel that split it over time must not

@@ -697,6 +697,62 @@ def test_runs_of_chunks(op, lens, H, dk, dv, bad):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("op", ["ssd", "mlstm"])
+@pytest.mark.parametrize("lens,H,dk,dv,cols", [([65, 193, 1, 128, 64], 4, 128, 36, 16), ([129, 255], 65, 128, 32, 32), ([384, 320], 33, 128, 100, 48),
+                                               ([191, 66, 200], 4, 64, 20, 16), ([130, 90], 90, 64, 24, 32), ([64, 257], 100, 64, 44, 48),
+                                               ([300, 128, 63], 80, 64, 52, 64)])
+@pytest.mark.parametrize("bad", [None, 40, 64])
+@pytest.mark.parametrize("whole", [True, False])
+def test_walk_with_the_state_at_hand(op, lens, H, dk, dv, cols, bad, whole):
+    """Pieces of 64 tokens cut off everywhere, every width of a block and columns that end inside it, against the token-by-token kernel: in one
+    window and in several, with an idle sequence, with an infinite value in a first and in a second piece."""
+    from llm_in_practise_amd.ops._native import native_seq
+    ext = native_seq()
+    g = torch.Generator().manual_seed(dk + dv)
+    T, B, longest = sum(lens), len(lens), max(lens)
+    assert ext.scan_walk(T, B, H, dk, dv, longest) == cols
+
+    def rand(*s, dt=torch.float32):
+        return torch.randn(*s, generator=g).to(dt).cuda()
+    q, k, v = (rand(T, H * n, dt=torch.bfloat16) for n in (dk, dk, dv))
+    if bad is not None:
+        v[bad, dv + 1] = float("inf")                   # head 1, column 1 of the first sequence
+    i, f, a, b, skip = 3 * rand(T, H), 3 * rand(T, H), rand(H), rand(H), rand(H)
+    S0, N0 = rand(B, H, dv, dk), rand(B, H, dk)
+    live = [int(j != 1) for j in range(B)]
+    tok = torch.repeat_interleave(torch.tensor(live, dtype=torch.bool), torch.tensor(lens)).cuda()
+    room = ext.scan_floats(op, T, B, H, dk, dv, longest=longest)
+    res = []
+    for most in (room if whole else B * H * 1040, 0):     # (two pieces a sequence at a time; too many windows: token by token)
+        st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lens, [7 * (j % 2) for j in range(B)], "cuda", live)
+        st["S"].copy_(S0)
+        st["N"].copy_(N0)
+        st["M"].fill_(0.5)
+        if op == "ssd":
+            out = [ext.ssd_scan(q, k, v, i.bfloat16(), a - 3, b, skip, st["S"], H, H, sb.desc, sb.live, most=most, longest=longest).view(T, H, dv)]
+        else:
+            out = ext.mlstm_scan(q, k, v, i, f, a, b + 3, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb.desc, sb.live, most=most,
+                                 longest=longest)
+        res.append([*(x[tok] for x in out), st["S"], st["N"], st["M"]])
+    for x, y in zip(*res):
+        x, y = x.double(), y.double()
+        assert torch.equal(torch.isfinite(x), torch.isfinite(y))
+        x, y = (torch.nan_to_num(t, 0.0, 0.0, 0.0) for t in (x, y))
+        assert (x - y).norm() <= TOL * y.norm(), ((x - y).norm() / y.norm()).item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,B,H,dk,dv,longest,cols", [
+    (4093, 1, 64, 128, 64, 4093, 0), (1000, 1, 64, 128, 64, 1000, 16), (2000, 4, 64, 128, 64, 512, 32), (7040, 8, 8, 128, 192, 1024, 48),
+    (512, 1, 8, 64, 96, 512, 16), (2048, 1, 8, 64, 96, 2048, 0), (4096, 8, 8, 64, 96, 512, 32), (9060, 12, 8, 64, 96, 9000 - 640, 0),
+    (9060, 12, 8, 64, 96, 0, 0), (512, 1, 8, 96, 96, 512, 0)])
+def test_walk_only_where_it_is_not_slower(T, B, H, dk, dv, longest, cols):
+    """Timed shapes on both sides of the choice between chunks and the walk; one long sequence among short ones, known or not, is not walked."""
+    from llm_in_practise_amd.ops._native import native_seq
+    assert native_seq().scan_walk(T, B, H, dk, dv, longest) == cols
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("op", ["ssd", "mlstm", "delta", "delta-16", "gla", "selective"])
 @pytest.mark.parametrize("B", [64, 65, 129, 200])
 def test_pieces_of_more_sequences_than_a_wave_has_lanes(op, B):
