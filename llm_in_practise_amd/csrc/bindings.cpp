@@ -50,6 +50,8 @@ void launch_sum_slices(const void*, void*, int, size_t, size_t, hipStream_t);
 bool skinny_norms(int, int, bool);
 void launch_rows_swiglu(const void*, int, const void*, void*, int, int, int, hipStream_t);
 void launch_rows_parts(const void*, int, const void*, const void*, void*, float*, int, int, int, int, hipStream_t);
+bool parts_norm_ok(int);
+void launch_parts_norm(const float*, int, const void*, const void*, void*, void*, int, int, float, hipStream_t);
 void launch_gemm_skinny(const void*, int, const void*, const void*, void*, int, int, int, bool, const void*, float, hipStream_t);
 bool w4mm_supported(int, int, int, int);
 bool w4g_supported(int, int, int, int);
@@ -673,6 +675,29 @@ Tensor rows_parts(Tensor x, Tensor w, optional<Tensor> residual, int64_t unit) {
   return out;
 }
 
+// The rows' parts, their sum with the residual and its RMSNorm: (y, norm(y)), two launches; none where the norm's form does not serve
+bool parts_norm_serves(int64_t N) { return parts_norm_ok((int)N); }
+
+static void check_parts_norm(const Tensor& x, const Tensor& residual, const Tensor& norm, int64_t N) {
+  CHECK_BF16(residual); CHECK_CONTIG(residual); CHECK_BF16(norm); CHECK_CONTIG(norm);
+  TORCH_CHECK(residual.is_cuda() && residual.dim() == 2 && residual.size(0) == x.size(0) && residual.size(1) == N && norm.is_cuda() &&
+                  norm.numel() == N && reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(norm.data_ptr()) % 16 == 0 && parts_norm_ok((int)N),
+              "product and norm: residual [M, N], weight [N], rows of N a multiple of 512 up to 8192");
+}
+
+std::vector<Tensor> rows_parts_norm(Tensor x, Tensor w, Tensor residual, int64_t unit, Tensor norm, double eps) {
+  check_skinny(x, w);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M > 16 && K % 512 == 0 && K < 1 << 24 && (unit == 64 || unit == 128), "rows_parts: 17 to 64 rows, W [N%16, K%512]");
+  check_parts_norm(x, residual, norm, N);
+  skinny_offsets(x);
+  Tensor y = at::empty({M, N}, x.options()), yn = at::empty({M, N}, x.options()), part = at::empty({4, M, N}, x.options().dtype(at::kFloat));
+  launch_rows_parts(x.data_ptr(), x.stride(0), w.data_ptr(), nullptr, nullptr, part.data_ptr<float>(), M, N, K, (int)unit, stream());
+  launch_parts_norm(part.data_ptr<float>(), 4, residual.data_ptr(), norm.data_ptr(), y.data_ptr(), yn.data_ptr(), M, N, (float)eps, stream());
+  return {y, yn};
+}
+
 // W4A16 MFMA GEMM (csrc/kernels/w4mm.hip): x [M<=64, K] bf16, codes u8 [N, K/2] (high nibble = even k),
 // sc2 fp32 [N, K/gs, 2] = (scale, bias − 128·scale)
 bool w4mm_ok(int64_t M, int64_t N, int64_t K, int64_t gs) { return w4mm_supported((int)M, (int)N, (int)K, (int)gs); }
@@ -761,6 +786,26 @@ Tensor w4g(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, optional<T
   launch_w4g(x.data_ptr(), (int)x.stride(0), codes.data_ptr<uint8_t>(), sc2.data_ptr<float>(), (int)gs, rp,
              out.data_ptr(), s > 1 ? part.data_ptr<float>() : nullptr, (int)M, (int)N, (int)K, s, stream());
   return out;
+}
+
+// A W4A16 product whose sums of K's slices go through memory, their sum with the residual and its RMSNorm: (y, norm(y)); none where one launch
+// holds all of K, or w4g takes it in one slice.  few: as w4mm runs it, else as w4g does.
+std::vector<Tensor> w4_parts_norm(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, bool few, Tensor residual, Tensor norm, double eps) {
+  check_w4mm(x, codes, sc2, N, gs);
+  const int64_t M = x.size(0), K = x.size(1);
+  const int nb = w4mm_nkb((int)M, (int)N, (int)K), s = few ? (int)(K / (128 * nb)) : w4g_splits((int)M, (int)N, (int)K);
+  if (s <= 1 || (few && w4row_serves((int)M, (int)N, (int)K, nb, false))) return {};
+  TORCH_CHECK(few || w4g_supported((int)M, (int)N, (int)K, (int)gs), "w4g: M<=64, N%128, K%128, gs%128");
+  check_parts_norm(x, residual, norm, N);
+  Tensor y = at::empty({M, N}, x.options()), yn = at::empty({M, N}, x.options()), part = at::empty({s, M, N}, x.options().dtype(at::kFloat));
+  if (few)
+    launch_w4mm(x.data_ptr(), (int)x.stride(0), codes.data_ptr<uint8_t>(), sc2.data_ptr<float>(), (int)gs, nullptr, nullptr, part.data_ptr<float>(),
+                (int)M, (int)N, (int)K, nb, stream());
+  else
+    launch_w4g(x.data_ptr(), (int)x.stride(0), codes.data_ptr<uint8_t>(), sc2.data_ptr<float>(), (int)gs, nullptr, nullptr, part.data_ptr<float>(),
+               (int)M, (int)N, (int)K, s, stream());
+  launch_parts_norm(part.data_ptr<float>(), s, residual.data_ptr(), norm.data_ptr(), y.data_ptr(), yn.data_ptr(), M, N, (float)eps, stream());
+  return {y, yn};
 }
 
 // codes [N, K/2] u8 (bnb layout), absmax fp32 [N*K/64] (decoded) → bf16 [N, K]
@@ -1935,6 +1980,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_skinny", &gemm_skinny, py::arg("x"), py::arg("w"), py::arg("residual"), py::arg("norm") = py::none(), py::arg("eps") = 0.0);
   m.def("rows_swiglu", &rows_swiglu);
   m.def("rows_parts", &rows_parts);
+  m.def("rows_parts_norm", &rows_parts_norm);
+  m.def("w4_parts_norm", &w4_parts_norm);
+  m.def("parts_norm_serves", &parts_norm_serves);
   m.def("gemm_skinny_swiglu", &gemm_skinny_swiglu, py::arg("x"), py::arg("w"), py::arg("norm") = py::none(), py::arg("eps") = 0.0);
   m.def("lt_linear", &lt_linear);
   m.def("lt_addmm", &lt_addmm);

@@ -730,7 +730,7 @@ void launch_w4g(const void* X, int ldx, const uint8_t* codes, const float* sc2, 
   w4g_k<4, 2, 2><<<grid, 256, 0, st>>>((const bf16*)X, ldx, codes, (const float2*)sc2, gs,
                                        ks > 1 ? nullptr : (const bf16*)res, (bf16*)out, ks > 1 ? part : nullptr, M, N,
                                        K, ncs, 1, nkb);
-  if (ks > 1) {
+  if (ks > 1 && out != nullptr) {                        // (without out the slices' sums are left where they are)
     const size_t MN = (size_t)M * N;
     w4mm_reduce_k<8><<<(MN / 2 + 255) / 256, 256, 0, st>>>(part, (const bf16*)res, (bf16*)out, ks, MN);
   }
@@ -818,7 +818,7 @@ void launch_w4mm(const void* X, int ldx, const uint8_t* codes, const float* sc2,
   if (RT == 1) LN(1); else if (RT == 2) LN(2); else LN(4);
 #undef LN
 #undef L
-  if (KS > 1) {
+  if (KS > 1 && out != nullptr) {                        // (without out the slices' sums are left where they are)
     const size_t MN = (size_t)M * N;
     w4mm_reduce_k<8><<<(MN / 2 + 255) / 256, 256, 0, st>>>(part, (const bf16*)res, (bf16*)out, KS, MN);
   }

@@ -27,7 +27,7 @@ from torch.nn.modules import module as _hooks
 
 from ..ops import reference as ref
 from ..ops.activation import swiglu_fused
-from ..ops.gemm import normed_rows
+from ..ops.gemm import normed_rows, rows_normed
 from ..ops.mlp import fusable as mlp_fusable, skinny_swiglu, swiglu_mlp
 from ..ops.attention import flash_attention, flash_attention_prefix
 from ..ops.decode import decode_attention_append
@@ -37,7 +37,7 @@ from ..ops.norm import RMSNorm, rms_norm, rms_norm_residual
 from ..ops.rope import apply_rope, qk_norm_rope
 from ..parallel.tensor_parallel import tp_all_reduce
 from ..peft.lora import LoraLayer, base_of
-from ..quant.int4 import Int4Linear, Int4Weight, int4_swiglu
+from ..quant.int4 import Int4Linear, Int4Weight, int4_normed, int4_swiglu
 from ..ops.embedding import Embedding
 from .common import CausalLMOutput, FusedProjection, KVCache, PackedPrefill, _leaf_linear, can_fuse, project
 
@@ -156,6 +156,17 @@ def _own(m: nn.Module, cls: type) -> bool:
         m._forward_pre_hooks or m._forward_hooks or _hooks._global_forward_pre_hooks or _hooks._global_forward_hooks)
 
 
+def _with_norm(m: nn.Module, x, residual, norm):
+    """``(y, norm(y))`` of ``y = m(x) + residual`` for decode rows, or None: an adapter or bias beside the weight, something else in the
+    projection's or the norm's place, rows whose product takes no launch that could form the norm."""
+    if residual is None or not _own(norm, RMSNorm) or not (_own(m, nn.Linear) or _own(m, Int4Linear)) or m.bias is not None or \
+            getattr(m, "_mlora", None) is not None:
+        return None
+    if type(m) is Int4Linear:
+        return int4_normed(x, m.int4, residual, norm.weight, norm.eps)
+    return None if m.weight.requires_grad else rows_normed(x, m.weight, residual, norm.weight, norm.eps)
+
+
 class Qwen3Attention(nn.Module):
     def __init__(self, cfg: Qwen3Config, layer_idx: int):
         super().__init__()
@@ -187,7 +198,8 @@ class Qwen3Attention(nn.Module):
         return normed_rows(x, norm.weight, norm.eps, f.base)
 
     def forward(self, x, cos, sin, B, S, residual=None, cache: KVCache | None = None, start: int = 0,
-                kv_lens=None, qkv=None):
+                kv_lens=None, qkv=None, then=None):
+        """``then``: the norm behind the block; the result is then ``(y, norm(y))``, or ``(y, None)`` where the caller is to form it."""
         tr = self.training
         if qkv is None:
             qkv = project([self.q_proj, self.k_proj, self.v_proj], x, None, tr, self._qkv)
@@ -219,9 +231,12 @@ class Qwen3Attention(nn.Module):
                 o = flash_attention_prefix(q, c, cache.v[self.layer_idx], B, S, start + S, self.hq, self.hkv,
                                            self.d, q_offs=start, kv_lens=kv_lens, kv_rows=c.shape[1])
         if self.tp_group is None:
+            if then is not None:
+                return _with_norm(self.o_proj, o, residual, then) or (project([self.o_proj], o, residual, tr), None)
             return project([self.o_proj], o, residual, tr)
         # row-parallel o_proj: partial sums + the residual on rank 0 only, then one all-reduce
-        return tp_all_reduce(project([self.o_proj], o, residual if self.tp_rank == 0 else None, tr), self.tp_group)
+        y = tp_all_reduce(project([self.o_proj], o, residual if self.tp_rank == 0 else None, tr), self.tp_group)
+        return y if then is None else (y, None)
 
 
 class Qwen3MLP(nn.Module):
@@ -271,19 +286,24 @@ class Qwen3MLP(nn.Module):
             return None
         return skinny_swiglu(x, self._gu.base, norm.weight, norm.eps)
 
-    def forward(self, x, residual=None, h=None):
+    def forward(self, x, residual=None, h=None, then=None):
+        """``then``: as for the attention block."""
         tr = self.training
         bases = self._fused_bases(x) if h is None else None
         if bases is not None:
-            return swiglu_mlp(x, bases[0], bases[1], residual)
+            y = swiglu_mlp(x, bases[0], bases[1], residual)
+            return y if then is None else (y, None)
         if h is None:
             h = self._few_rows(x)
         if h is None:
             h = swiglu_fused(project([self.gate_proj, self.up_proj], x, None, tr, self._gu))
         if self.tp_group is None:
+            if then is not None:
+                return _with_norm(self.down_proj, h, residual, then) or (project([self.down_proj], h, residual, tr), None)
             return project([self.down_proj], h, residual, tr)
         y = project([self.down_proj], h, residual if self.tp_rank == 0 else None, tr)
-        return tp_all_reduce(y, self.tp_group)
+        y = tp_all_reduce(y, self.tp_group)
+        return y if then is None else (y, None)
 
 
 class Qwen3DecoderLayer(nn.Module):
@@ -294,17 +314,31 @@ class Qwen3DecoderLayer(nn.Module):
         self.input_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
 
-    def forward(self, x, cos, sin, B, S, cache=None, start=0, kv_lens=None):
+    def forward(self, x, cos, sin, B, S, cache=None, start=0, kv_lens=None, xn=None, then=None):
+        """``xn``: the rows normed already.  ``then``: the norm behind the layer; the result is then ``(x, norm(x))``, or ``(x, None)``."""
         few = B * S <= 4                # rows that their products norm themselves (what stands in a sublayer's place is to see them normed)
+        some = then is not None and not few     # decode rows whose products may form the norm behind them
         qkv = self.self_attn.normed_few_rows(x, self.input_layernorm) if few and _own(self.self_attn, Qwen3Attention) else None
-        xn, skip = (x, x) if qkv is not None else rms_norm_residual(x, self.input_layernorm.weight, self.input_layernorm.eps)
+        if xn is not None:
+            skip = x
+        else:
+            xn, skip = (x, x) if qkv is not None else rms_norm_residual(x, self.input_layernorm.weight, self.input_layernorm.eps)
         given = {} if qkv is None else {"qkv": qkv}
-        h = self.self_attn(xn, cos, sin, B, S, residual=skip, cache=cache, start=start, kv_lens=kv_lens, **given)
+        if some and _own(self.self_attn, Qwen3Attention):
+            h, hn = self.self_attn(xn, cos, sin, B, S, residual=skip, cache=cache, start=start, kv_lens=kv_lens, then=self.post_attention_layernorm)
+        else:
+            h, hn = self.self_attn(xn, cos, sin, B, S, residual=skip, cache=cache, start=start, kv_lens=kv_lens, **given), None
         act = self.mlp.normed_few_rows(h, self.post_attention_layernorm) if few and _own(self.mlp, Qwen3MLP) else None
         if act is not None:
-            return self.mlp(h, residual=h, h=act)
-        hn, skip = rms_norm_residual(h, self.post_attention_layernorm.weight, self.post_attention_layernorm.eps)
-        return self.mlp(hn, residual=skip)
+            x = self.mlp(h, residual=h, h=act)
+            return x if then is None else (x, None)
+        skip = h
+        if hn is None:
+            hn, skip = rms_norm_residual(h, self.post_attention_layernorm.weight, self.post_attention_layernorm.eps)
+        if some and _own(self.mlp, Qwen3MLP):
+            return self.mlp(hn, residual=skip, then=then)
+        x = self.mlp(hn, residual=skip)
+        return x if then is None else (x, None)
 
 
 class Qwen3Model(nn.Module):
@@ -351,18 +385,25 @@ class Qwen3Model(nn.Module):
         x = self.embed_tokens(input_ids).reshape(B * S, -1)
         if self.pp is not None:
             x = self.pp.enter(x)        # stages > 0: the previous stage's hidden states
-        for layer in self.layers:
+        # a decode step's rows: a product that adds up parts forms the norm behind it as well, the next layer's or the last one
+        norms = [layer.input_layernorm if _own(layer, Qwen3DecoderLayer) else None for layer in self.layers[1:]] + [self.norm] \
+            if decoding and 4 < B <= 64 and self.pp is None and x.is_cuda else None
+        xn = None
+        for i, layer in enumerate(self.layers):
             if self.gradient_checkpointing and self.training and cache is None:
                 x = lora_checkpoint(layer, x, cos, sin, B, S, None, 0, kv_lens, **self.ckpt_kwargs)
+            elif norms is not None and norms[i] is not None and _own(layer, Qwen3DecoderLayer):
+                x, xn = layer(x, cos, sin, B, S, cache, start, kv_lens, xn=xn, then=norms[i])
             else:
-                x = layer(x, cos, sin, B, S, cache, start, kv_lens)
+                x = layer(x, cos, sin, B, S, cache, start, kv_lens) if xn is None else layer(x, cos, sin, B, S, cache, start, kv_lens, xn=xn)
+                xn = None
         if self.pp is not None:
             x = self.pp.exit(x)         # hand to the next stage; every stage gets the last one's output
         if decoding:
             cache.pos += 1
         elif cache is not None:
             cache.len = start + S
-        return rms_norm(x, self.norm.weight, self.norm.eps)
+        return rms_norm(x, self.norm.weight, self.norm.eps) if xn is None else xn
 
 
 class Qwen3ForCausalLM(nn.Module):

@@ -209,6 +209,37 @@ def _narrow_rows(x, base, residual):
     return 0 if K % 512 else 128 if M <= 32 else 64
 
 
+class _RowsNormedFn(torch.autograd.Function):
+    """(No backward: rows_normed leaves what needs a gradient to the differentiable ops.)"""
+    @staticmethod
+    def forward(ctx, x, base, residual, unit, weight, eps):
+        return tuple(native().rows_parts_norm(x, base, residual, unit, weight, eps))
+
+
+def norm_follows(x: torch.Tensor, residual, weight, N: int) -> bool:
+    """Whether the launch that adds up a decode product's parts may form the RMSNorm behind it as well (csrc/kernels/rows.hip): bf16 rows and a
+    norm's weight of their type, in memory of their own and without gradients, of a width the kernel takes."""
+    return (x.is_cuda and isinstance(residual, torch.Tensor) and isinstance(weight, torch.Tensor) and eager(x, residual, weight)
+            and x.dim() == 2 and x.dtype == residual.dtype == weight.dtype == torch.bfloat16 and weight.get_device() == residual.get_device() == x.get_device()
+            and residual.shape == (x.shape[0], N) and residual.is_contiguous() and residual.data_ptr() % 16 == 0
+            and weight.shape == (N,) and weight.is_contiguous() and weight.data_ptr() % 16 == 0 and not force_reference()
+            and not (torch.is_grad_enabled() and (x.requires_grad or residual.requires_grad or weight.requires_grad))
+            and native().parts_norm_serves(N))
+
+
+def rows_normed(x: torch.Tensor, base, residual, weight, eps: float):
+    """``(y, rms_norm(y))`` of ``y = x · baseᵀ + residual`` for 17 to 64 decode rows whose product adds up parts of K: every bit as from the
+    product and the norm behind it, a launch less; None where that is not served."""
+    if not (isinstance(base, torch.Tensor) and 16 < x.shape[0] <= 64 and not base.requires_grad
+            and norm_follows(x, residual, weight, base.shape[0])):
+        return None
+    unit = _narrow_rows(x, base, residual)
+    if unit <= 1:
+        return None
+    _count("decode")
+    return fn_apply(_RowsNormedFn, x, base, residual, unit, weight, eps)
+
+
 def _base_gemm(x, base, ext_a=None, ext_b=None, residual=None):
     if isinstance(base, NF4Weight):
         if x.shape[0] <= 8 and base.kernel_ok():   # decode: weight-streaming GEMV, no MFMA tile

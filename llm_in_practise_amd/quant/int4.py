@@ -282,6 +282,21 @@ def int4_linear(x: torch.Tensor, w: Int4Weight, bias: torch.Tensor | None = None
     return y.view(*shape[:-1], n)
 
 
+def int4_normed(x: torch.Tensor, w: Int4Weight, residual: torch.Tensor, weight, eps: float):
+    """``(y, rms_norm(y))`` of ``y = int4_linear(x) + residual`` for decode rows whose product adds up slices of K through memory: every bit as from
+    the product and the norm behind it, a launch less; None where that is not served."""
+    from ..ops._native import native
+    from ..ops.gemm import norm_follows
+    n, k = w.shape
+    M = x.shape[0]
+    if not (2 < M <= _W4G_MAX and x.dim() == 2 and x.stride(-1) == 1 and norm_follows(x, residual, weight, n)):
+        return None
+    few = M <= _W4MM_MAX and native().w4mm_ok(M, n, k, w.group_size)
+    if not few and not native().w4g_ok(M, n, k, w.group_size):
+        return None
+    return tuple(native().w4_parts_norm(x.contiguous(), w.codes, w.w4mm_table(), n, w.group_size, few, residual, weight, eps)) or None
+
+
 def int4_swiglu(x: torch.Tensor, w: Int4Weight) -> torch.Tensor | None:
     """``silu(gate)·up`` of the [gate | up] product of 3 .. 16 decode rows in one launch, or None where w4mm.hip does not serve
     it so.  Bit for bit int4_linear and the activation (24576 × 4096, 12 rows: 26.9 + 5 → 16.4 µs)."""

@@ -421,6 +421,88 @@ def test_decode_layers_norm_their_rows_in_the_products(native_ext, monkeypatch, 
     assert layer.mlp.normed_few_rows(x, layer.post_attention_layernorm) is None
 
 
+@pytest.mark.parametrize("M", [17, 33, 64])
+@pytest.mark.parametrize("N,K", [(512, 4096), (1024, 4608), (1536, 512), (2560, 9728), (3584, 4096), (4096, 12288)])
+def test_parts_and_the_norm_behind_them(native_ext, M, N, K):
+    """The launch that adds up a product's parts and norms the rows: the bits of the sum's launch and the norm's own kernel (one wave or two a
+    row), bf16 parts and slices of 4-bit weights (one to many, odd numbers of them); a row that holds an infinity changes no other; a replay."""
+    from llm_in_practise_amd.ops.norm import rms_norm
+    from llm_in_practise_amd.quant.int4 import int4_linear, int4_normed, quantize_rtn
+    torch.manual_seed(N + M)
+    x, res, nw = torch.randn(M, K, device=DEV).bfloat16(), torch.randn(M, N, device=DEV).bfloat16(), torch.randn(N, device=DEV).bfloat16()
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    forms = [(lambda x, u=u: native_ext.rows_parts_norm(x, w, res, u, nw, 1e-6), lambda x, u=u: native_ext.rows_parts(x, w, res, u)) for u in (64, 128)]
+    w4 = quantize_rtn(w, 128)
+    forms.append((lambda x: int4_normed(x, w4, res, nw, 1e-6), lambda x: int4_linear(x, w4, None, res)))
+    for form, product in forms:
+        got = form(x)
+        if got is None:                                 # (one launch holds all of K)
+            assert M <= 32
+            continue
+        want = product(x)
+        assert torch.equal(got[0], want) and torch.equal(got[1], rms_norm(want, nw, 1e-6))
+        y = x.clone()
+        y[M - 1, 5] = float("inf")
+        bad = form(y)
+        assert torch.equal(bad[1][:M - 1], got[1][:M - 1]) and not torch.isfinite(bad[1][M - 1].float()).all()
+        y = x.clone()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = form(y)
+        for _ in range(3):
+            y.copy_(torch.randn(M, K, device=DEV))
+            g.replay()
+            want = product(y)
+            assert torch.equal(out[0], want) and torch.equal(out[1], rms_norm(want, nw, 1e-6))
+    assert not native_ext.parts_norm_serves(N + 16) and not native_ext.parts_norm_serves(8704)
+
+
+@pytest.mark.parametrize("rows", [5, 17, 33, 64])
+@pytest.mark.parametrize("weights", ["bf16", "int4"])
+def test_decode_steps_norm_rows_where_parts_are_added_up(native_ext, monkeypatch, rows, weights):
+    """A decode step's logits are those of the norm's own kernel; a hooked or replaced sublayer, a hooked layer and trainable weights keep it."""
+    from llm_in_practise_amd.models import qwen3
+    from llm_in_practise_amd.models.common import KVCache
+    from llm_in_practise_amd.quant.gptq import replace_with_int4
+    from llm_in_practise_amd.quant.int4 import quantize_rtn
+    m = qwen3.Qwen3ForCausalLM.from_config(qwen3.qwen3_config("qwen3-small", num_attention_heads=32, intermediate_size=4608),
+                                           dtype=torch.bfloat16, device=DEV, seed=0).eval()
+    m.requires_grad_(False)
+    if weights == "int4":
+        replace_with_int4(m, {n: quantize_rtn(mod.weight.detach(), 128) for n, mod in m.named_modules()
+                              if isinstance(mod, torch.nn.Linear) and n.startswith("model.layers")})
+    m.fuse_projections()
+    ids = torch.randint(0, 4096, (rows, 1), device=DEV)
+    real, calls = qwen3._with_norm, []
+
+    def counted(*a):
+        y = real(*a)
+        calls.append(y is not None)
+        return y
+
+    def step():
+        calls.clear()
+        cache = KVCache(m.config.num_hidden_layers, rows, 64, m.config.num_key_value_heads, m.config.head_dim, torch.bfloat16, DEV)
+        cache.start_decode(torch.full((rows,), 7, dtype=torch.long, device=DEV))
+        with torch.no_grad():
+            return m.model(ids, cache=cache)
+    monkeypatch.setattr(qwen3, "_with_norm", counted)
+    got = step()
+    assert len(calls) == 8 and any(calls) == (weights == "int4" or rows > 32)
+    with monkeypatch.context() as c:
+        c.setattr(qwen3, "_with_norm", lambda *a: None)
+        assert torch.equal(step(), got)
+    for sub in (m.model.layers[1].self_attn, m.model.layers[1].mlp, m.model.layers[2]):
+        seen = []
+        handle = sub.register_forward_pre_hook(lambda mod, args: seen.append(args[0]))
+        assert torch.equal(step(), got) and len(seen) == 1 and len(calls) < 8
+        handle.remove()
+    if weights == "bf16":
+        m.model.layers[0].mlp.down_proj.weight.requires_grad_()
+        step()
+        assert not calls[1]
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 40])
 @pytest.mark.parametrize("N,K", [(32, 64), (1056, 192), (6144, 1088), (64, 1984), (96, 20480)])
 def test_gemm_skinny_infinite_weights(native_ext, M, N, K):
