@@ -362,15 +362,15 @@ void dispatch(int code, const void* q, int ldq, const void* k, int ldk, const vo
 
 }  // namespace
 
-size_t seq_delta_floats(int, int, int, int, int, size_t);
+size_t seq_delta_floats(int, int, int, int, int, int, size_t);
 void seq_delta(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float*, float*, float*, size_t,
-               int, int, int, int, SeqDesc, hipStream_t);
+               int, int, int, int, int, SeqDesc, hipStream_t);
 
 // Floats of workspace of the blocked form, or 0 where the token-by-token scan is the one to run: key sizes that are no multiple
 // of 64 or above 256, rows that vector loads of four channels cannot take, and steps of few tokens a sequence.  At most `most`: longer
 // steps run in windows.
 size_t seq_block_floats(int code, bool delta, const void* q, int ldq, const void* k, int ldk, const void* g, const void* bias,
-                        const void* S, int T_, int B, int H, int dk, int dv, size_t most) {
+                        const void* S, int T_, int B, int H, int dk, int dv, int longest, size_t most) {
   const int bytes = code == 0 ? 8 : 16;
   const auto fits = [](const void* p, int ld, int b) { return ld % 4 == 0 && ((uintptr_t)p & (b - 1)) == 0; };
   if (dk % 64 != 0 || dk > 256 || !fits(q, ldq, bytes) || !fits(k, ldk, bytes) || !fits(g, 4, 16) || !fits(bias, 4, 16) ||
@@ -397,15 +397,15 @@ size_t seq_block_floats(int code, bool delta, const void* q, int ldq, const void
     least = blocks > 1536 ? never : blocks > 512 || dk == 64 ? 64 : 40;
   }
   if (T_ < least * B) return 0;
-  if (const size_t n = delta ? seq_delta_floats(T_, B, H, dk, dv, most) : 0) return n;
+  if (const size_t n = delta ? seq_delta_floats(T_, B, H, dk, dv, longest, most) : 0) return n;
   return block_plan(T_, B, H, dk, most).slots * slot_floats(H, dk);
 }
 
 void seq_block_delta(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g,
                      const float* bpre, float* S, float* out, float* ws, size_t most, int H, int G, int dk, int dv,
-                     SeqDesc d, hipStream_t st) {
-  if (seq_delta_floats(d.Ttot, d.B, H, dk, dv, most) > 0) {
-    seq_delta(code, q, ldq, k, ldk, v, ldv, g, bpre, S, out, ws, most, H, G, dk, dv, d, st);
+                     int longest, SeqDesc d, hipStream_t st) {
+  if (seq_delta_floats(d.Ttot, d.B, H, dk, dv, longest, most) > 0) {
+    seq_delta(code, q, ldq, k, ldk, v, ldv, g, bpre, S, out, ws, most, H, G, dk, dv, longest, d, st);
     return;
   }
   const DecayArgs a = {g, nullptr, bpre, 1.f, 1.f};
@@ -414,7 +414,7 @@ void seq_block_delta(int code, const void* q, int ldq, const void* k, int ldk, c
 
 void seq_block_gla(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* z,
                    const float* zb, float inv_tau, float qscale, float* S, float* out, float* ws, size_t most, int H, int dk,
-                   int dv, SeqDesc d, hipStream_t st) {
+                   int dv, int longest, SeqDesc d, hipStream_t st) {
   const DecayArgs a = {z, zb, nullptr, inv_tau, qscale};
   dispatch<false>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, H, dk, dv, d, st);
 }

@@ -17,6 +17,7 @@
 // the state and a tile's sums are added up by themselves and rounded once at the size of what they are added to.
 #include "seq_block.h"
 
+#include <algorithm>
 #include <type_traits>
 
 using namespace lipa;
@@ -229,27 +230,98 @@ __global__ __launch_bounds__(512, 6) void k_delta_prep(const T* __restrict__ q, 
   if (lane == 0) seen[((size_t)slot * H + hd) * SEEN + w] = odd;
 }
 
+// What is known of the state between two parts of a sequence of `blocks` blocks each, per (part, head): where the part leaves a state that
+// it finds at 0 (the first part: at the one in front of it), 16 columns at a time in operand layout, and its product of transitions P,
+// by which any other state in front of it goes on, as the left operand of the 16x16x4 products.  (The first part needs no P: the state in
+// front of it stands there, since the last part may have written its own by the time the first one runs again.)
+struct Parts {
+  float* at;
+  int blocks;
+};
+// Part `id` of all that run, without a sequence's last one for `ends`; place: the sequence's first place.  (Counted, not bounded as the
+// pieces are: blocks of threads that find nothing to do leave others side by side on one CU, 84 us for 45.)
+struct Part {
+  int s, idx, place, t0, t1, end;
+};
+__device__ __forceinline__ bool find_part(const SeqDesc& d, int len, int id, bool ends, Part& p) {
+  int before = 0;                                            // parts in the lower half, places in the upper one
+  for (int b0 = 0; b0 < d.B; b0 += 64) {
+    const int lane = threadIdx.x & 63, b = min(b0 + lane, d.B - 1);
+    const int s0 = d.seq_off[b], s1 = d.seq_off[b + 1], on = d.live ? d.live[b] : 1;
+    const int n = on && b0 + lane < d.B ? (s1 - s0 + len - 1) / len : 0, own = n + (max(n - 1, 0) << 16);
+    int sum = own;
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) {
+      const int x = __shfl_up(sum, o, 64);
+      sum += lane >= o ? x : 0;
+    }
+    sum += before;
+    const unsigned long long m = __ballot((ends ? sum >> 16 : sum & 0xffff) > id);
+    if (m) {
+      const int at = __builtin_ctzll(m), first = __builtin_amdgcn_readlane(sum - own, at);
+      p.s = b0 + at;
+      p.idx = id - (ends ? first >> 16 : first & 0xffff);
+      p.place = first >> 16;
+      p.end = __builtin_amdgcn_readlane(s1, at);
+      p.t0 = __builtin_amdgcn_readlane(s0, at) + p.idx * len;
+      p.t1 = min(p.t0 + len, p.end);
+      return true;
+    }
+    before = __builtin_amdgcn_readlane(sum, 63);
+  }
+  return false;
+}
+__host__ __device__ constexpr int part_floats(int dk, int dv) { return dk * (((dv + 15) & ~15) + (dk > dv ? dk : (dv + 15) & ~15)); }
+
+enum { WHOLE, ENDS, PARTS };
+
 // A block owns 16 value columns of one (sequence, head) and walks its blocks of tokens, a window between two barriers for each.  Four waves
 // hold a quarter of the state's rows each, in registers in operand layout: they finish u from the shares of the key products, update
 // their rows, leave these in LDS and form their shares of the next block's key products.  Four more, one on every SIMD beside them, take
 // the state of the window before from LDS for the query products and finish the outputs of the block before that.  One wave alone
 // on a SIMD leaves the float matrix unit idle in every barrier and round trip (3000 cycles a block for 1630 of products).
-template <typename T, int NS>
-__global__ __launch_bounds__(512, 2) void k_delta_walk(const float* __restrict__ ws, const unsigned* __restrict__ seen,
+//
+// Few long sequences leave most CUs idle behind that chain.  They are cut into parts that run side by side, in two launches: ENDS walks every
+// part but a sequence's last without outputs (four waves), and beside its columns from a state of 0 - the recurrence is linear in the
+// state - 16 columns of the unit matrix at a time without values, which become P.  PARTS then walks each part from the state in front of it,
+// S <- P S + end over the parts before, and has the outputs.
+template <typename T, int NS, int FORM>
+__global__ __launch_bounds__(FORM == ENDS ? 256 : 512, FORM == WHOLE ? 2 : FORM == ENDS ? 3 : 4) void k_delta_walk(const float* __restrict__ ws, const unsigned* __restrict__ seen,
                                                        const T* __restrict__ v, int ldv, float* __restrict__ S,
-                                                       float* __restrict__ out, int H, int dv, Pieces pc, SeqDesc d) {
-  constexpr int DK = 64 * NS, ROWS = BT * DK;
+                                                       float* __restrict__ out, int H, int dv, Pieces pc, Parts pt, SeqDesc d) {
+  constexpr int DK = 64 * NS, ROWS = BT * DK, RING = FORM == WHOLE ? 2 : 1;
   __shared__ __attribute__((aligned(16))) f32x4 rk[2][4][2][64];     // shares of the key products, of the query products
-  __shared__ __attribute__((aligned(16))) f32x4 rq[2][4][2][64];
-  __shared__ __attribute__((aligned(16))) f32x4 su[2][2][64];        // u
-  __shared__ __attribute__((aligned(16))) f32x4 ss[2][4][NS][64];    // the state
-  const int s = blockIdx.x / H, hd = blockIdx.x % H, tid = threadIdx.x;
-  if (d.live && !d.live[s]) return;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), w = wv & 3, lane = tid & 63, g = lane >> 4, col = blockIdx.y * 16 + (lane & 15);
+  __shared__ __attribute__((aligned(16))) f32x4 rq[FORM == ENDS ? 1 : 2][4][2][64];
+  __shared__ __attribute__((aligned(16))) f32x4 su[FORM == ENDS ? 1 : 2][2][64];        // u
+  __shared__ __attribute__((aligned(16))) f32x4 ss[FORM == ENDS ? 1 : 2][4][NS][64];    // the state
+  const int tid = threadIdx.x, vtiles = (dv + 15) / 16;
+  int s, hd, slot, t0, t1, steps, part = 0, place = 0, tile = blockIdx.y;
+  bool last = true;
+  if constexpr (FORM == WHOLE) {
+    s = blockIdx.x / H, hd = blockIdx.x % H;
+    if (d.live && !d.live[s]) return;
+    t0 = d.seq_off[s] + pc.first * LEN, t1 = d.seq_off[s + 1], steps = own_pieces<LEN>(d, pc, s, slot);
+    if (steps <= 0) return;
+  } else {
+    // (a (part, head)'s columns, which read the same rows, are 8 apart: on one die)
+    const int tiles = vtiles + (FORM == ENDS ? 4 * NS : 0), x = blockIdx.x / (8 * tiles) * 8 + blockIdx.x % 8;
+    Part own;
+    if (!find_part(d, pt.blocks * LEN, x / H, FORM == ENDS, own)) return;
+    s = own.s, hd = x % H, part = own.idx, place = own.place, t0 = own.t0, t1 = own.t1, steps = (t1 - t0 + LEN - 1) / LEN;
+    tile = blockIdx.x / 8 % tiles;
+    slot = (t0 - part * pt.blocks * LEN) / LEN + s + part * pt.blocks;
+    last = t1 == own.end;
+    if (FORM == ENDS && part == 0 && tile >= vtiles) return;
+  }
+  const bool unit = FORM == ENDS && tile >= vtiles;         // columns of the unit matrix
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), w = wv & 3, lane = tid & 63, g = lane >> 4;
+  const int col = unit ? dv : tile * 16 + (lane & 15);
   const bool colok = col < dv;
-  int slot;
-  const int t0 = d.seq_off[s] + pc.first * LEN, t1 = d.seq_off[s + 1], steps = own_pieces<LEN>(d, pc, s, slot), vtiles = (dv + 15) / 16;
-  if (steps <= 0) return;
+  // the places of the sequence's parts, and what this block's waves have in each
+  const int PART = FORM == WHOLE ? 0 : part_floats(DK, dv), ENDF = FORM == WHOLE ? 0 : vtiles * 16 * DK;
+  float* first = FORM == WHOLE ? nullptr : pt.at + ((size_t)place * H + hd) * PART;
+  const size_t part_step = (size_t)H * PART;
+  const unsigned own = (unsigned)(((FORM == WHOLE ? 0 : tile) * 4 * NS + NS * w) * 64 + lane) * 4;
   const int CELL = cell_floats(DK, dv);
   const float* cell = ws + ((size_t)slot * H + hd) * CELL;
   const size_t step = (size_t)H * CELL;
@@ -258,21 +330,22 @@ __global__ __launch_bounds__(512, 2) void k_delta_walk(const float* __restrict__
   // A value that is infinite or NaN: it counts as 0 in the products, its column of the state is NaN, and its column of the
   // outputs from its token on.  (A sequence without such values runs the loops that do not look at them.)
   auto number = [&](int i, int h, int e) {
+    if (FORM == ENDS && unit) return true;
     const int tt = i * LEN + BT * h + 4 * g + e;
     return t0 + tt >= t1 || isfinite((float)vp[(size_t)min(tt, t1 - t0 - 1) * ldv + vcol]);
   };
   u32x4 any = {0u, 0u, 0u, 0u};
   for (int i = lane; i < 2 * steps; i += 64) any |= reinterpret_cast<const u32x4*>(seen)[(((size_t)slot + i / 2) * H + hd) * 2 + (i & 1)];
-  const bool some = __any((any[0] | any[1]) | (any[2] | any[3]));
+  const bool some = !unit && __any((any[0] | any[1]) | (any[2] | any[3]));
   const int half = w & 1;                                   // the tile whose outputs a wave finishes, every other block
-  if (wv < 4) {
+  if (FORM == ENDS || wv < 4) {
     __builtin_amdgcn_s_setprio(3);                          // (the other wave's products fill the gaps)
     float* Sp = S + (((size_t)d.slots[s] * H + hd) * dv + (colok ? col : 0)) * DK + 16 * NS * w + 4 * g;
     const bool old = (pc.first > 0 || d.pos0[s] > 0) && colok;
     f32x4 St[NS];
     struct In {
       f32x4 k[2][NS], p[2][NS], g[NS], u[2];
-    } in[2];
+    } in[RING];
     auto load_k = [&](int i, In& x) {
       const float* c0 = cell + (size_t)i * step;
 #pragma unroll
@@ -283,7 +356,8 @@ __global__ __launch_bounds__(512, 2) void k_delta_walk(const float* __restrict__
     auto load = [&](int i, In& x) {
       const float* c0 = cell + (size_t)i * step;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) x.u[h] = row4(c0 + 6 * ROWS + DK + 3 * BT * BT + ((h * vtiles + blockIdx.y) * 64 + lane) * 4);
+      for (int h = 0; h < 2; ++h)
+        x.u[h] = row4(c0 + 6 * ROWS + DK + 3 * BT * BT + ((h * vtiles + (unit ? 0 : tile)) * 64 + lane) * 4);
 #pragma unroll
       for (int c = 0; c < NS; ++c) x.g[c] = row4(c0 + 6 * ROWS + 16 * (NS * w + c) + (unsigned)(4 * g));
 #pragma unroll
@@ -310,10 +384,13 @@ __global__ __launch_bounds__(512, 2) void k_delta_walk(const float* __restrict__
       for (int a = 0; a < 4; ++a)
 #pragma unroll
         for (int h = 0; h < 2; ++h) r[a][h] = rk[i & 1][a][h][lane];
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (RING == 2) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int h = 0; h < 2; ++h) u[h] = x.u[h] - ((r[0][h] + r[1][h]) + (r[2][h] + r[3][h]));
-      su[i & 1][half][lane] = half ? u[1] : u[0];           // (two waves write the same)
+      for (int h = 0; h < 2; ++h) {
+        const f32x4 own = FORM == ENDS && unit ? f32x4{0.f, 0.f, 0.f, 0.f} : x.u[h];   // (looked at in its turn)
+        u[h] = own - ((r[0][h] + r[1][h]) + (r[2][h] + r[3][h]));
+      }
+      if constexpr (FORM != ENDS) su[i & 1][half][lane] = half ? u[1] : u[0];      // (two waves write the same)
       if constexpr (odd)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
@@ -330,36 +407,79 @@ __global__ __launch_bounds__(512, 2) void k_delta_walk(const float* __restrict__
       for (int c = 0; c < NS; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e) St[c][e] = fmaf(St[c][e], x.g[c][e], add[c][e]);
-      load(min(i + 2, steps - 1), x);
+      load(min(i + RING, steps - 1), x);
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (FORM != ENDS)
 #pragma unroll
-      for (int c = 0; c < NS; ++c) ss[(i + 1) & 1][w][c][lane] = St[c];
+        for (int c = 0; c < NS; ++c) ss[(i + 1) & 1][w][c][lane] = St[c];
       keys(i + 1, next);                                    // (past the last block: nobody reads them)
-      load_k(min(i + 3, steps - 1), next);
+      load_k(min(i + 1 + RING, steps - 1), next);
       __builtin_amdgcn_sched_barrier(0);
     };
-    load_k(0, in[0]);
-    load(0, in[0]);
-    load_k(min(1, steps - 1), in[1]);
-    load(min(1, steps - 1), in[1]);
-#pragma unroll
-    for (int c = 0; c < NS; ++c) {
-      St[c] = old ? row4(Sp + 16 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
-      ss[0][w][c][lane] = St[c];
+    if constexpr (RING == 2) {
+      load_k(0, in[0]);
+      load(0, in[0]);
+      load_k(min(1, steps - 1), in[RING - 1]);
+      load(min(1, steps - 1), in[RING - 1]);
     }
+    if constexpr (FORM == ENDS) {
+#pragma unroll
+      for (int c = 0; c < NS; ++c) {
+        St[c] = part == 0 && old ? row4(Sp + 16 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
+        if (part == 0) *reinterpret_cast<f32x4*>(first + ENDF + own + c * 256) = St[c];
+        if (unit)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) St[c][e] = 16 * (NS * w + c) + 4 * g + e == 16 * (tile - vtiles) + (lane & 15) ? 1.f : 0.f;
+      }
+    } else if (FORM == PARTS && !(part == 0 && last)) {
+#pragma unroll
+      for (int c = 0; c < NS; ++c) St[c] = row4(first + (part == 0 ? ENDF : 0) + own + c * 256);
+#pragma unroll 1
+      for (int j = 1; j < part; ++j) {
+        const float* f = first + j * part_step;
+        f32x4 P[NS][4 * NS];
+#pragma unroll
+        for (int c = 0; c < NS; ++c)
+#pragma unroll
+          for (int k = 0; k < 4 * NS; ++k) P[c][k] = row4(f + ENDF + (unsigned)(((NS * w + c) * 4 * NS + k) * 64 + lane) * 4);
+#pragma unroll
+        for (int c = 0; c < NS; ++c) ss[j & 1][w][c][lane] = St[c];
+        __syncthreads();
+        f32x4 sum[NS] = {};
+#pragma unroll
+        for (int k = 0; k < 4 * NS; ++k) {
+          const f32x4 x = ss[j & 1][k / NS][k % NS][lane];
+#pragma unroll
+          for (int c = 0; c < NS; ++c) sum[c] = mfma4(P[c][k], x, sum[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < NS; ++c) St[c] = row4(f + own + c * 256) + sum[c];
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < NS; ++c) St[c] = old ? row4(Sp + 16 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if constexpr (RING == 1) {
+      load_k(0, in[0]);
+      load(0, in[0]);
+    }
+    if constexpr (FORM == PARTS) __syncthreads();           // (the place of the first state is read)
+    if constexpr (FORM != ENDS)
+#pragma unroll
+      for (int c = 0; c < NS; ++c) ss[0][w][c][lane] = St[c];
     keys(0, in[0]);
-    load_k(min(2, steps - 1), in[0]);
+    load_k(min(RING, steps - 1), in[0]);
     auto walk = [&](auto odd) {
       int i = 0;
       for (; i + 2 <= steps; i += 2) {
         __syncthreads();
-        window(i, in[0], in[1], odd);
+        window(i, in[0], in[RING - 1], odd);
         __syncthreads();
-        window(i + 1, in[1], in[0], odd);
+        window(i + 1, in[RING - 1], in[0], odd);
       }
       if (i < steps) {
         __syncthreads();
-        window(i, in[0], in[1], odd);
+        window(i, in[0], in[RING - 1], odd);
       }
       __syncthreads();                                      // (the outputs of the last block)
     };
@@ -367,14 +487,31 @@ __global__ __launch_bounds__(512, 2) void k_delta_walk(const float* __restrict__
       walk(std::true_type{});
     else
       walk(std::false_type{});
-    if (colok)
+    if constexpr (FORM == ENDS) {
+      float* mine = first + part * part_step;
+#pragma unroll
+      for (int c = 0; c < NS; ++c) {
+        if (!unit) *reinterpret_cast<f32x4*>(mine + own + c * 256) = St[c];
+        // row 4 g + e, column (lane & 15) of its 16 x 16 as the left operand has them
+        float* P = mine + ENDF + (((NS * w + c) * 4 * NS + tile - vtiles) * 64 + ((lane & 15) >> 2) * 16 + 4 * g) * 4 + (lane & 3);
+        if (unit)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) P[4 * e] = St[c][e];
+      }
+      return;
+    }
+    if (colok && last)
 #pragma unroll
       for (int c = 0; c < NS; ++c) *reinterpret_cast<f32x4*>(Sp + 16 * c) = St[c];
     return;
   }
+  if constexpr (FORM == PARTS) {
+    for (int j = 1; j < part; ++j) __syncthreads();
+    __syncthreads();
+  }
   struct In {
     f32x4 q[2][NS], b[2];
-  } in[2];
+  } in[RING];
   auto load = [&](int i, In& x) {
     const float* c0 = cell + (size_t)i * step;
 #pragma unroll
@@ -425,18 +562,18 @@ __global__ __launch_bounds__(512, 2) void k_delta_walk(const float* __restrict__
     if (i > 0 && w >> 1 == (i & 1)) outputs(i - 1, odd);
 #pragma unroll
     for (int h = 0; h < 2; ++h) bo[h] = x.b[h];
-    load(min(i + 2, steps - 1), x);
+    load(min(i + RING, steps - 1), x);
     __builtin_amdgcn_sched_barrier(0);
   };
   load(0, in[0]);
-  load(min(1, steps - 1), in[1]);
+  if constexpr (RING == 2) load(min(1, steps - 1), in[RING - 1]);
   auto walk = [&](auto odd) {
     int i = 0;
     for (; i + 2 <= steps; i += 2) {
       __syncthreads();
       window(i, in[0], odd);
       __syncthreads();
-      window(i + 1, in[1], odd);
+      window(i + 1, in[RING - 1], odd);
     }
     if (i < steps) {
       __syncthreads();
@@ -457,17 +594,71 @@ PiecePlan delta_plan(int T_, int B, int H, int dk, int dv, size_t most) {
   return plan_pieces(T_, B, LEN, slot_floats(H, dk, dv), most, 0.23f);
 }
 
+// Blocks of a part, 0: sequences in one piece.  A window takes 1.36 us alone on its CU, whatever the others do, so the longest sequence bounds
+// a step that leaves CUs idle; in parts the windows of all of them count: 1.42 us a window of the outputs' walk where a CU has one block,
+// 1.15 where it has two or more at once, 0.95 and 0.82 a window of the ends' (which bring 35 KB each, 7 to 10 TB/s out of the caches), 2 us
+// for each part in front of the last one's state and 8 for the launch and what stands in front of the first windows (keys of 128; of 64
+// three quarters).  The other sequences are taken to be of one length.  us, in one piece -> in parts, 4 heads of 128 x 128: 1000 tokens 62 -> 47,
+// 4093 198 -> 87, 9000 422 -> 170, 3000 + 1700 155 -> 103, 5000 and three of 40 240 -> 114 (400 33 -> 35, 4 x 2000 122 -> 121, 1000 + 700 + 500
+// + 600 + 800 67 -> 73: in one piece); 8 heads: 700 47 -> 43, 1000 61 -> 54, 1500 + 700 + 97 94 -> 87, 4093 209 -> 140, 9000 445 -> 295, 3000 +
+// 1700 167 -> 142 (4 x 2000 149 -> 206: in one piece).
+int part_blocks(int T_, int B, int H, int dk, int dv, int longest) {
+  const int tiles = (dv + 15) / 16, units = dk / 16, top = (longest + LEN - 1) / LEN;
+  if (longest > T_ || top < 2 || (long)B * H * tiles > 256) return 0;
+  const int rest = B > 1 ? ((T_ - longest) / (B - 1) + LEN - 1) / LEN : 0;
+  const auto cus = [](float n) { return ceilf(n / 256.f); };
+  const float scale = dk == 64 ? 0.75f : 1.f;
+  float best = 0.92f * (1.36f * scale * top + 4.f);
+  int blocks = 0;
+  for (int parts = 2; parts <= 12; ++parts) {
+    const int L = (top + parts - 1) / parts;
+    if (L < 6) break;
+    const int n = (top + L - 1) / L, m = (rest + L - 1) / L;
+    const float walk = cus((float)(n + (B - 1) * m) * H * tiles);
+    const float ends = cus(H * ((float)tiles * (n - 1 + (B - 1) * std::max(m - 1, 0)) + (float)units * (n - 2 + (B - 1) * std::max(m - 2, 0))));
+    const float us = scale * (L * ((walk > 1.f ? 1.15f * walk : 1.42f) + (ends > 1.f ? 0.82f * ends : 0.95f)) + 2.f * (n - 2)) + 8.f;
+    if (us < best) best = us, blocks = L;
+  }
+  return blocks;
+}
+struct DeltaPlan {
+  PiecePlan p;
+  int blocks;            // of a part, 0: sequences in one piece
+  size_t floats;
+};
+DeltaPlan plan_of(int T_, int B, int H, int dk, int dv, int longest, size_t most) {
+  DeltaPlan r = {delta_plan(T_, B, H, dk, dv, most), 0, 0};
+  r.floats = r.p.slots * slot_floats(H, dk, dv);
+  if (r.p.count != 0) return r;
+  if (const int blocks = part_blocks(T_, B, H, dk, dv, longest)) {
+    const size_t more = (size_t)T_ / (blocks * LEN) * H * part_floats(dk, dv);
+    if (r.floats + more <= most) r.blocks = blocks, r.floats += more;
+  }
+  return r;
+}
+
 template <typename T, int NS>
 void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g, const float* beta, float* S,
-            float* out, float* ws, size_t most, int H, int G, int dv, const SeqDesc& d, hipStream_t st) {
-  const PiecePlan plan = delta_plan(d.Ttot, d.B, H, 64 * NS, dv, most);
-  unsigned* seen = reinterpret_cast<unsigned*>(ws + plan.slots * H * cell_floats(64 * NS, dv));
-  for (int w = 0; w < plan.windows; ++w) {
-    const Pieces pc = {LEN, w * plan.count, plan.count};
-    hipLaunchKernelGGL((k_delta_prep<T, NS>), dim3(H, (unsigned)plan.slots), dim3(512), 0, st, (const T*)q, ldq, (const T*)k, ldk,
+            float* out, float* ws, size_t most, int H, int G, int dv, int longest, const SeqDesc& d, hipStream_t st) {
+  constexpr int DK = 64 * NS;
+  const DeltaPlan plan = plan_of(d.Ttot, d.B, H, DK, dv, longest, most);
+  unsigned* seen = reinterpret_cast<unsigned*>(ws + plan.p.slots * H * cell_floats(DK, dv));
+  const Parts pt = {ws + plan.p.slots * slot_floats(H, DK, dv), plan.blocks};
+  const unsigned tiles = (dv + 15) / 16;
+  const unsigned all = plan.blocks > 0 ? d.Ttot / (plan.blocks * LEN) : 0, ends = (all * H + 7) / 8 * 8, parts = ((all + d.B) * H + 7) / 8 * 8;
+  for (int w = 0; w < plan.p.windows; ++w) {
+    const Pieces pc = {LEN, w * plan.p.count, plan.p.count};
+    hipLaunchKernelGGL((k_delta_prep<T, NS>), dim3(H, (unsigned)plan.p.slots), dim3(512), 0, st, (const T*)q, ldq, (const T*)k, ldk,
                        (const T*)v, ldv, dv, g, beta, ws, seen, H, G, pc, d);
-    hipLaunchKernelGGL((k_delta_walk<T, NS>), dim3(d.B * H, (dv + 15) / 16), dim3(512), 0, st, ws, seen, (const T*)v, ldv, S, out, H,
-                       dv, pc, d);
+    if (plan.blocks == 0) {
+      hipLaunchKernelGGL((k_delta_walk<T, NS, WHOLE>), dim3(d.B * H, tiles), dim3(512), 0, st, ws, seen, (const T*)v, ldv, S, out, H, dv,
+                         pc, pt, d);
+      continue;
+    }
+    hipLaunchKernelGGL((k_delta_walk<T, NS, ENDS>), dim3(ends * (tiles + 4 * NS)), dim3(256), 0, st, ws, seen, (const T*)v,
+                       ldv, S, out, H, dv, pc, pt, d);
+    hipLaunchKernelGGL((k_delta_walk<T, NS, PARTS>), dim3(parts * tiles), dim3(512), 0, st, ws, seen, (const T*)v, ldv, S,
+                       out, H, dv, pc, pt, d);
   }
   LIPA_CHECK_LAUNCH();
 }
@@ -483,18 +674,23 @@ void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int l
 // 128 x 32, 8 x 512 103 -> 78; of 64 x 64, 4 x 600 (512) 86 -> 80, 40 x 320 (1280) 123 -> 122; of 64 x 128, 16 heads 16 x 512 (2048) 230 -> 238,
 // 64 heads 4 x 300 136 -> 159.  Keys of 192 97 -> 95, of 256 146 -> 151.
 // The first kernel's grid has 65535 slots at most.
-size_t seq_delta_floats(int T_, int B, int H, int dk, int dv, size_t most) {
+size_t seq_delta_floats(int T_, int B, int H, int dk, int dv, int longest, size_t most) {
   if (dk > 128 || T_ < 300l * B || (dv > 64 && (long)B * H * ((dv + 15) / 16) > 256)) return 0;
-  const size_t slots = delta_plan(T_, B, H, dk, dv, most).slots;
-  return slots > 65535 ? 0 : slots * slot_floats(H, dk, dv);
+  const DeltaPlan plan = plan_of(T_, B, H, dk, dv, longest, most);
+  return plan.p.slots > 65535 ? 0 : plan.floats;
+}
+
+// blocks of 32 tokens in a part of a sequence, 0: in one piece
+int seq_delta_parts(int T_, int B, int H, int dk, int dv, int longest, size_t most) {
+  return plan_of(T_, B, H, dk, dv, longest, most).blocks;
 }
 
 void seq_delta(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g, const float* bpre, float* S,
-               float* out, float* ws, size_t most, int H, int G, int dk, int dv, SeqDesc d, hipStream_t st) {
+               float* out, float* ws, size_t most, int H, int G, int dk, int dv, int longest, SeqDesc d, hipStream_t st) {
   SEQ_DISPATCH_T(code, {
     if (dk == 64)
-      launch<T, 1>(q, ldq, k, ldk, v, ldv, g, bpre, S, out, ws, most, H, G, dv, d, st);
+      launch<T, 1>(q, ldq, k, ldk, v, ldv, g, bpre, S, out, ws, most, H, G, dv, longest, d, st);
     else
-      launch<T, 2>(q, ldq, k, ldk, v, ldv, g, bpre, S, out, ws, most, H, G, dv, d, st);
+      launch<T, 2>(q, ldq, k, ldk, v, ldv, g, bpre, S, out, ws, most, H, G, dv, longest, d, st);
   });
 }

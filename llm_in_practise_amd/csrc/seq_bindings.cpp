@@ -75,7 +75,8 @@ void seq_softcap(float*, size_t, float, hipStream_t);
 void seq_selective_scan(int, const void*, int, const float*, const float*, const void*, int, const void*, int, const float*,
                         const float*, const void*, int, float*, void*, int, float, int, int, float*, size_t, SeqDesc, hipStream_t);
 size_t seq_selective_floats(int, int, int, int, size_t);
-size_t seq_delta_floats(int, int, int, int, int, size_t);
+size_t seq_delta_floats(int, int, int, int, int, int, size_t);
+int seq_delta_parts(int, int, int, int, int, int, size_t);
 bool seq_selective_rows(int, int, int, int, int, int, int, int, int);
 void seq_gla_scan(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float,
                   float*, float*, int, int, int, SeqDesc, hipStream_t);
@@ -111,11 +112,11 @@ void seq_chunk_mlstm(const void*, int, const void*, int, const void*, int, const
                      const float*, float, float, float*, float*, float*, float*, float*, float*, float*, size_t, int, int, int,
                      int, SeqDesc, hipStream_t);
 size_t seq_block_floats(int, bool, const void*, int, const void*, int, const void*, const void*, const void*, int, int, int, int,
-                        int, size_t);
+                        int, int, size_t);
 void seq_block_delta(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float*, float*, float*,
-                     size_t, int, int, int, int, SeqDesc, hipStream_t);
+                     size_t, int, int, int, int, int, SeqDesc, hipStream_t);
 void seq_block_gla(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float, float*,
-                   float*, float*, size_t, int, int, int, SeqDesc, hipStream_t);
+                   float*, float*, size_t, int, int, int, int, SeqDesc, hipStream_t);
 int seq_scan_max_dk();
 int seq_conv_max_head();
 int seq_conv_max_taps();
@@ -382,7 +383,7 @@ std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor
 }
 
 Tensor delta_scan(Tensor q, Tensor k, Tensor v, Tensor g, Tensor bpre, Tensor S, int64_t H, int64_t G,
-                  std::vector<Tensor> desc, optional<Tensor> live, int64_t most) {
+                  std::vector<Tensor> desc, optional<Tensor> live, int64_t most, int64_t longest) {
   const int code = code_of(q);
   const int64_t T = q.size(0);
   TORCH_CHECK(G >= 1 && H % G == 0 && q.dim() == 2 && q.size(1) % G == 0 && v.dim() == 2 && v.size(1) % H == 0,
@@ -399,11 +400,11 @@ Tensor delta_scan(Tensor q, Tensor k, Tensor v, Tensor g, Tensor bpre, Tensor S,
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H, dv}, S.options());
   if (const size_t n = seq_block_floats(code, true, q.data_ptr(), ld(q), k.data_ptr(), ld(k), g.data_ptr(), nullptr,
-                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (size_t)most)) {
+                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_block_delta(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), g.data_ptr<float>(),
                     bpre.data_ptr<float>(), S.data_ptr<float>(), out.data_ptr<float>(), ws.data_ptr<float>(), (size_t)most, (int)H,
-                    (int)G, (int)dk, (int)dv, d, stream());
+                    (int)G, (int)dk, (int)dv, (int)longest, d, stream());
     return out;
   }
   seq_delta_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), g.data_ptr<float>(),
@@ -1175,7 +1176,7 @@ Tensor selective_scan(Tensor x, Tensor dt_pre, Tensor dt_bias, Tensor b, Tensor 
 
 // q, k [T, H * dk], v [T, H * dv] activation rows, z float [T, H * dk] contiguous; S float [slots, H, dv, dk] in place
 Tensor gated_linear_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, double tau, double q_scale, Tensor S,
-                         int64_t H, std::vector<Tensor> desc, optional<Tensor> live, int64_t most) {
+                         int64_t H, std::vector<Tensor> desc, optional<Tensor> live, int64_t most, int64_t longest) {
   const int code = code_of(q);
   TORCH_CHECK(H >= 1 && q.dim() == 2 && q.size(1) % H == 0 && v.dim() == 2 && v.size(1) % H == 0,
               "q/k: [T, H * dk], v: [T, H * dv]");
@@ -1192,11 +1193,11 @@ Tensor gated_linear_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, 
   auto out = at::empty({T, H, dv}, S.options());
   if (T == 0) return out;
   if (const size_t n = seq_block_floats(code, false, q.data_ptr(), ld(q), k.data_ptr(), ld(k), z.data_ptr(), z_bias.data_ptr(),
-                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (size_t)most)) {
+                                        S.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_block_gla(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), z.data_ptr<float>(),
                   z_bias.data_ptr<float>(), (float)(1.0 / tau), (float)q_scale, S.data_ptr<float>(), out.data_ptr<float>(),
-                  ws.data_ptr<float>(), (size_t)most, (int)H, (int)dk, (int)dv, d, stream());
+                  ws.data_ptr<float>(), (size_t)most, (int)H, (int)dk, (int)dv, (int)longest, d, stream());
     return out;
   }
   seq_gla_scan(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), z.data_ptr<float>(),
@@ -1296,7 +1297,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("fb"), py::arg("cap"), py::arg("qscale"), py::arg("S"), py::arg("N"), py::arg("M"), py::arg("H"),
         py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS, py::arg("longest") = 0);
   m.def("delta_scan", &delta_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("g"), py::arg("bpre"), py::arg("S"),
-        py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS);
+        py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS, py::arg("longest") = 0);
   m.def("talk_attention", &talk_attention);
   m.def("ssd_scan", &ssd_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("dtraw"), py::arg("dt_bias"),
         py::arg("a_log"), py::arg("dskip"), py::arg("S"), py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"),
@@ -1329,7 +1330,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       return (int64_t)seq_chunk_floats(0, nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most);
     TORCH_CHECK(op == "delta" || op == "gla", "scan_floats: ssd, mlstm, delta or gla");
     return (int64_t)seq_block_floats(0, op == "delta", nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H,
-                                     (int)dk, (int)dv, (size_t)most);
+                                     (int)dk, (int)dv, (int)longest, (size_t)most);
   }, py::arg("op"), py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS, py::arg("longest") = 0);
   // columns of a block that walks the tokens with the state at hand ("ssd", "mlstm"), 0: chunks, or token by token
   m.def("scan_walk", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t longest) {
@@ -1338,9 +1339,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return 16 * seq_walk_tiles((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest);
   });
   m.def("delta_block", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most) {      // tokens of a block, 0: token by token
-    if (seq_block_floats(0, true, nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most) == 0) return 0;
-    return seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, (size_t)most) > 0 ? 32 : 16;
+    if (seq_block_floats(0, true, nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, 0, (size_t)most) == 0) return 0;
+    return seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, 0, (size_t)most) > 0 ? 32 : 16;
   }, py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS);
+  // blocks of tokens in a part of a sequence, where parts run side by side ("delta": of 32); 0: sequences in one piece
+  m.def("scan_parts", [](const std::string& op, int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t longest, int64_t most) {
+    TORCH_CHECK(op == "delta", "scan_parts: delta");
+    if (seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most) == 0) return 0;
+    return seq_delta_parts((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most);
+  }, py::arg("op"), py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("longest"), py::arg("most") = MOST_WS);
   m.def("selective_floats", [](int64_t T, int64_t B, int64_t C, int64_t N, int64_t most) {        // 0: rows side by side are not cut over time
     if (seq_selective_rows((int)T, (int)B, (int)C, (int)N, (int)C, (int)C, (int)N, (int)N, (int)C)) return (int64_t)0;
     return (int64_t)seq_selective_floats((int)T, (int)B, (int)C, (int)N, (size_t)most);
@@ -1353,7 +1360,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("scale"), py::arg("most") = MOST_WS);
   m.def("gated_linear_scan", &gated_linear_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("z"), py::arg("z_bias"),
         py::arg("tau"), py::arg("q_scale"), py::arg("S"), py::arg("H"), py::arg("desc"), py::arg("live"),
-        py::arg("most") = MOST_WS);
+        py::arg("most") = MOST_WS, py::arg("longest") = 0);
   m.def("delta_rule_gates", &delta_rule_gates);
   m.def("general_delta_scan", &general_delta_scan);
 }

@@ -47,7 +47,7 @@ def gated_delta_scan(q, k, v, g, beta_pre, S, heads: int, kv_heads: int, sb):
     o = S^T q``.  Returns float ``[T, H, dv]``."""
     if use_seq(q):
         return native_seq().delta_scan(q, k, v, g.contiguous(), beta_pre.contiguous(), S, heads, kv_heads, sb.desc,
-                                       sb.live)
+                                       sb.live, longest=sb.longest)
     return ref.delta_scan(q, k, v, g, beta_pre, S, heads, kv_heads, sb)
 
 
@@ -103,5 +103,6 @@ def gated_linear_scan(q, k, v, z, z_bias, tau: float, q_scale: float, S, heads: 
     float ``[T, H*dk]``, ``z_bias`` float ``[H*dk]``; ``S`` float ``[slots, H, dv, dk]`` in place.  Decays and the state are
     float (the decay as ``exp(log sigmoid / tau)``).  Returns float ``[T, H, dv]``."""
     if use_seq(q):
-        return native_seq().gated_linear_scan(q, k, v, z, z_bias, tau, q_scale, S, heads, sb.desc, sb.live)
+        return native_seq().gated_linear_scan(q, k, v, z, z_bias, tau, q_scale, S, heads, sb.desc, sb.live,
+                                               longest=sb.longest)
     return ref.gated_linear_scan(q, k, v, z, z_bias, tau, q_scale, S, heads, sb)

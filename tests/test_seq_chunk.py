@@ -315,6 +315,55 @@ def test_delta_blocks_of_two_tiles(lens, starts, H, G, dk, dv, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lens,starts,live", [([1000], [0], [1]), ([1, 997, 30, 610], [0, 7, 5, 0], [1, 1, 1, 1]),
+                                              ([640, 800, 64, 33], [3, 0, 0, 0], [0, 1, 1, 1])])
+@pytest.mark.parametrize("H,G,dk,dv,dt", [(2, 1, 128, 20, torch.bfloat16), (3, 3, 64, 36, torch.float32), (1, 1, 128, 132, torch.float32)])
+def test_delta_sequences_in_parts(lens, starts, live, H, G, dk, dv, dt):
+    """Long sequences in parts that run side by side: a first state, a last part of one token or tile, sequences of one part
+    and one that does not run; and a value and a key that are no numbers reach what is behind them, part or not."""
+    from llm_in_practise_amd.ops._native import native_seq
+    T = sum(lens)
+    blocks = native_seq().scan_parts("delta", T, len(lens), H, dk, dv, max(lens))
+    assert 0 < 2 * 32 * blocks < max(lens) + 32 * blocks
+    g = torch.Generator().manual_seed(dk + dv + len(lens))
+    P = torch.randn(T, 2 * G * dk + H * dv, generator=g)
+    for j in (0, 1):
+        x = P[:, j * G * dk:(j + 1) * G * dk].view(T, G, dk)
+        x.copy_(torch.nn.functional.normalize(x, dim=-1))
+    P, decay, beta = P.to(dt), torch.rand(T, H * dk, generator=g) ** 0.02, 2 * torch.randn(T, H, generator=g)
+    decay[::97, ::3] = 0.0
+    S0 = torch.randn(len(lens), H, dv, dk, generator=g)
+    tok = torch.cat([torch.full((n,), bool(on)) for n, on in zip(lens, live)])
+
+    def run(dev, p):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, starts, dev, live)
+        st["S"].copy_(S0)
+        p = p.to(dev)
+        o = R.gated_delta_scan(p[:, :G * dk], p[:, G * dk:2 * G * dk], p[:, 2 * G * dk:], decay.to(dev), beta.to(dev), st["S"], H, G, sb)
+        return o.cpu()[tok], st["S"].cpu()
+    want, got = run("cpu", P), run("cuda", P)
+    _close(got, want, ("o", "state"))
+    for column in (2 * G * dk + 5, G * dk + 5):              # a value; a key
+        bad, first = P.clone(), sum(lens[:1]) if len(lens) > 1 else 0
+        bad[first + 32 * blocks - 3, column] = float("nan")  # near the end of a part
+        a, b = run("cpu", bad), run("cuda", bad)
+        for x, y in zip(a, b):
+            assert torch.equal(x.isnan(), y.isnan())
+        _close((b[0].nan_to_num(),), (a[0].nan_to_num(),), ("o",))
+
+
+@pytest.mark.gpu
+def test_delta_parts_find_room_beside_the_blocks():
+    from llm_in_practise_amd.ops._native import native_seq
+    ext, shape = native_seq(), (4093, 1, 4, 128, 128)
+    whole, parts = ext.scan_floats("delta", *shape), ext.scan_floats("delta", *shape, longest=4093)
+    assert whole < parts and ext.scan_parts("delta", *shape, longest=4093, most=parts) > 0
+    assert ext.scan_parts("delta", *shape, longest=4093, most=parts - 1) == 0
+    assert ext.scan_floats("delta", *shape, most=parts - 1, longest=4093) == whole
+    assert ext.scan_parts("delta", *shape, longest=0) == 0
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("L,B,H,dk,dv,long", [
     (1000, 1, 8, 128, 128, True), (200, 1, 8, 128, 128, False), (300, 5, 6, 128, 128, True), (299, 5, 6, 128, 128, False),
     (2000, 4, 8, 128, 128, True), (2000, 5, 8, 128, 128, False), (400, 20, 16, 128, 64, True), (400, 20, 16, 128, 68, False),
