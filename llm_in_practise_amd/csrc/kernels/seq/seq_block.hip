@@ -18,6 +18,7 @@
 // (seq_delta.hip).
 #include "seq_block.h"
 
+#include <algorithm>
 #include <type_traits>
 
 using namespace lipa;
@@ -170,28 +171,76 @@ __global__ __launch_bounds__(256) void k_block_prep(const T* __restrict__ q, int
 // and the waves take turns at summing them into outputs, one block of tokens later.  Bound by the chain of a block of tokens
 // (key products, LDS round trip, u, update); what it reads is on its way two or three blocks ahead, since it comes from memory
 // or another die's cache.
-template <typename T, int NS, bool DELTA>
+//
+// Few long sequences of linear attention leave most CUs idle behind that chain: they run in parts side by side, in two launches.  ENDS
+// walks every part but a sequence's last from a state of 0 (the first part: from the state in front of it), without queries, outputs or
+// barriers, and leaves the state behind it and the product of its decays; PARTS walks each part from S <- decays x S + end over the
+// parts before.  Per (part, head): 16 columns of the state at a time in operand layout, the state in front of the sequence (the last
+// part may have written its own by the time the first one runs again), the decays.
+struct Parts {
+  float* at;
+  int blocks;
+};
+__host__ __device__ constexpr int part_floats(int dk, int dv) { return 2 * dk * ((dv + 15) & ~15) + dk; }
+
+template <typename T, int NS, bool DELTA, int FORM>
 __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float* __restrict__ ws, const unsigned* __restrict__ seen,
                                                                     const T* __restrict__ v, int ldv, float* __restrict__ S,
-                                                                    float* __restrict__ out, int H, int dv, Pieces pc, SeqDesc d) {
+                                                                    float* __restrict__ out, int H, int dv, Pieces pc, Parts pt, SeqDesc d) {
   constexpr int DK = 64 * NS, CELL = cell_floats(DK), RING = NS == 1 ? 4 : 3;
-  __shared__ __attribute__((aligned(16))) f32x4 red[2][4][2][64];
-  const int s = blockIdx.x / H, hd = blockIdx.x % H, tid = threadIdx.x;
-  if (d.live && !d.live[s]) return;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, col = blockIdx.y * 16 + (lane & 15);
+  __shared__ __attribute__((aligned(16))) f32x4 red[FORM == ENDS ? 1 : 2][FORM == ENDS ? 1 : 4][2][64];
+  const int tid = threadIdx.x, vtiles = (dv + 15) / 16;
+  int s, hd, slot, t0, t1, steps, part = 0, place = 0, tile = blockIdx.y;
+  bool last = true;
+  if constexpr (FORM == WHOLE) {
+    s = blockIdx.x / H, hd = blockIdx.x % H;
+    if (d.live && !d.live[s]) return;
+    t0 = d.seq_off[s] + pc.first * BT, t1 = d.seq_off[s + 1], steps = own_pieces<BT>(d, pc, s, slot);
+    if (steps <= 0) return;
+  } else {
+    // (a (part, head)'s columns, which read the same rows, are 8 apart: on one die)
+    const int x = blockIdx.x / (8 * vtiles) * 8 + blockIdx.x % 8;
+    Part own;
+    if (!find_part(d, pt.blocks * BT, x / H, FORM == ENDS, own)) return;
+    s = own.s, hd = x % H, part = own.idx, place = own.place, t0 = own.t0, t1 = own.t1, steps = (t1 - t0 + BT - 1) / BT;
+    tile = blockIdx.x / 8 % vtiles;
+    slot = (t0 - part * pt.blocks * BT) / BT + s + part * pt.blocks;
+    last = t1 == own.end;
+  }
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, col = tile * 16 + (lane & 15);
   const bool colok = col < dv;
-  int slot;
-  const int t0 = d.seq_off[s] + pc.first * BT, t1 = d.seq_off[s + 1], steps = own_pieces<BT>(d, pc, s, slot);
-  if (steps <= 0) return;
   const float* cell = ws + ((size_t)slot * H + hd) * CELL;
   const size_t step = (size_t)H * CELL;
   const T* vp = v + (size_t)t0 * ldv + (size_t)hd * dv;
   const unsigned vcol = colok ? col : 0, m = 3 * BT * DK + DK + (lane & 15) * BT + 4 * g;
   float* Sp = S + (((size_t)d.slots[s] * H + hd) * dv + (colok ? col : 0)) * DK + 16 * NS * w + 4 * g;
-  f32x4 St[NS];
+  f32x4 St[NS], Gs[NS];                           // the state; ENDS: the decays so far
   const bool old = (pc.first > 0 || d.pos0[s] > 0) && colok;
+  const int ENDF = vtiles * 16 * DK;
+  const size_t part_step = (size_t)H * part_floats(DK, dv);
+  float* first = FORM == WHOLE ? nullptr : pt.at + ((size_t)place * H + hd) * part_floats(DK, dv);       // the sequence's first part's
+  const unsigned own = (unsigned)((tile * 4 * NS + NS * w) * 64 + lane) * 4, rows = 16 * NS * w + 4 * g;
 #pragma unroll
-  for (int c = 0; c < NS; ++c) St[c] = old ? row4(Sp + 16 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < NS; ++c) Gs[c] = f32x4{1.f, 1.f, 1.f, 1.f};
+  if (FORM == PARTS && !(part == 0 && last)) {
+#pragma unroll
+    for (int c = 0; c < NS; ++c) St[c] = row4(first + (part == 0 ? ENDF : 0) + own + c * 256);
+    for (int j = 1; j < part; ++j) {
+      const float* f = first + j * part_step;
+#pragma unroll
+      for (int c = 0; c < NS; ++c) {
+        const f32x4 D = row4(f + 2 * ENDF + 16 * c + rows), end = row4(f + own + c * 256);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) St[c][e] = fmaf(D[e], St[c][e], end[e]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < NS; ++c) St[c] = part == 0 && old ? row4(Sp + 16 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (FORM == ENDS && part == 0)
+#pragma unroll
+    for (int c = 0; c < NS; ++c) *reinterpret_cast<f32x4*>(first + ENDF + own + c * 256) = St[c];
   struct In {
     f32x4 k[NS], q[NS], p[NS], g[NS], tm, bm;
     T v[4];
@@ -202,12 +251,12 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
     for (int c = 0; c < NS; ++c) {
       const unsigned o = ((NS * w + c) * 64 + lane) * 4;
       if (DELTA) x.k[c] = row4(c0 + o);
-      x.q[c] = row4(c0 + BT * DK + o);
+      if (FORM != ENDS) x.q[c] = row4(c0 + BT * DK + o);
       x.p[c] = row4(c0 + 2 * BT * DK + o);
       x.g[c] = row4(c0 + 3 * BT * DK + 16 * (NS * w + c) + (unsigned)(4 * g));
     }
     if (DELTA) x.tm = row4(c0 + m);
-    x.bm = row4(c0 + m + BT * BT);
+    if (FORM != ENDS) x.bm = row4(c0 + m + BT * BT);
     // (values are not looked at before their turn: that would wait for every load issued before them)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -253,12 +302,14 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
       }
       r[w][0][lane] = x0 + x1;
     }
-    __syncthreads();
     f32x4 xq = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (FORM != ENDS) {
+      __syncthreads();
 #pragma unroll
-    for (int c = 0; c < NS; ++c)
+      for (int c = 0; c < NS; ++c)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) xq = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[c][e], St[c][e], xq, 0, 0, 0);
+        for (int e = 0; e < 4; ++e) xq = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[c][e], St[c][e], xq, 0, 0, 0);
+    }
     f32x4 u;
 #pragma unroll
     for (int e = 0; e < 4; ++e) u[e] = t0 + i * BT + 4 * g + e < t1 ? (float)x.v[e] : 0.f;
@@ -275,7 +326,7 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
 #pragma unroll
       for (int j = 0; j < 4; ++j) u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.tm[j], e[j], u, 0, 0, 0);
     }
-    r[w][1][lane] = xq;
+    if constexpr (FORM != ENDS) r[w][1][lane] = xq;
     f32x4 us = u;
     if constexpr (odd)
 #pragma unroll
@@ -283,9 +334,11 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
 #pragma unroll
     for (int c = 0; c < NS; ++c) {
       St[c] *= x.g[c];
+      if constexpr (FORM == ENDS) Gs[c] *= x.g[c];
 #pragma unroll
       for (int e = 0; e < 4; ++e) St[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[c][e], us[e], St[c], 0, 0, 0);
     }
+    if constexpr (FORM == ENDS) return;
     if (w == (i & 3) && i > 0) outputs(i - 1, odd);    // its query products were written in front of this barrier
     uo = u;
     bo = x.bm;
@@ -303,8 +356,10 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
       load(i, in[0]);
       run(i, in[0], std::true_type{});
     }
-    __syncthreads();                              // the last query products stand
-    if (w == (steps & 3)) outputs(steps - 1, std::true_type{});
+    if constexpr (FORM != ENDS) {
+      __syncthreads();                            // the last query products stand
+      if (w == (steps & 3)) outputs(steps - 1, std::true_type{});
+    }
   } else {
     constexpr std::false_type odd{};
     int i = 0;
@@ -318,44 +373,103 @@ __global__ __launch_bounds__(256, NS > 2 ? 1 : 2) void k_block_scan(const float*
 #pragma unroll
     for (int x = 0; x < RING - 1; ++x)
       if (i + x < steps) run(i + x, in[x], odd);
-    __syncthreads();
-    if (w == (steps & 3)) outputs(steps - 1, odd);
+    if constexpr (FORM != ENDS) {
+      __syncthreads();
+      if (w == (steps & 3)) outputs(steps - 1, odd);
+    }
   }
-  if (colok)
+  if constexpr (FORM == ENDS) {
+    float* mine = first + part * part_step;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      *reinterpret_cast<f32x4*>(mine + own + c * 256) = St[c];
+      if (tile == 0 && (lane & 15) == 0) *reinterpret_cast<f32x4*>(mine + 2 * ENDF + 16 * c + rows) = Gs[c];
+    }
+    return;
+  }
+  if (colok && last)
 #pragma unroll
     for (int c = 0; c < NS; ++c) *reinterpret_cast<f32x4*>(Sp + 16 * c) = St[c];
 }
 
 // floats of a slot; 0.23 us a token at least in the token-by-token form
 size_t slot_floats(int H, int dk) { return (size_t)H * (cell_floats(dk) + 4); }
-PiecePlan block_plan(int T_, int B, int H, int dk, size_t most) {
-  return plan_pieces(T_, B, BT, slot_floats(H, dk), most, 0.23f);
+
+// Blocks of a part of linear attention, 0: sequences in one piece.  A block of tokens takes 0.49 us where a CU has one or two blocks of threads,
+// whatever the others do; in parts the blocks of all of them count, twice: 0.28 us for each block of threads on a CU, at least as for 1.3,
+// 0.6 for a part in front of the last one's state and 6 for the launch and the first blocks (keys of 64).  The other sequences are taken
+// to be of one length.  us, in one piece -> in parts, 8 heads of 64 x 128: 1000 tokens 40 -> 26, 4093 137 -> 63, 9000 288 -> 118, 3000 + 1700
+// 107 -> 77, 5000 and three of 40 165 -> 76 (400 21 -> 20, 4 x 2000 86 -> 91, 10 x 700 74 -> 89: in one piece); 16 heads: 1000 45 -> 38, 4093
+// 147 -> 100, 9000 312 -> 203, 5000 and three of 40 224 -> 127 (400 22 -> 25, 3000 + 1700 118 -> 113: in one piece).
+int part_blocks(int T_, int B, int H, int dk, int dv, int longest) {
+  const int top = (longest + BT - 1) / BT, rest = B > 1 ? ((T_ - longest) / (B - 1) + BT - 1) / BT : 0;
+  if (longest > T_ || (long)B * H * ((dv + 15) / 16) > 1024) return 0;
+  const float full = H * ((dv + 15) / 16) / 256.f, scale = (dk + 64) / 128.f;
+  float best = 0.85f * 0.49f * scale * top;
+  int blocks = 0;
+  for (int parts = 2; parts <= 16; ++parts) {
+    const int L = (top + parts - 1) / parts;
+    if (L < 8) break;
+    const int n = (top + L - 1) / L, m = (rest + L - 1) / L;
+    const float walk = full * (n + (B - 1) * m), ends = full * (n - 1 + (B - 1) * std::max(m - 1, 0));
+    const float us = scale * (0.28f * L * (std::max(walk, 1.3f) + std::max(ends, 1.3f)) + 0.6f * (n - 2)) + 6.f;
+    if (us < best) best = us, blocks = L;
+  }
+  return blocks;
+}
+
+struct BlockPlan {
+  PiecePlan p;
+  int blocks;            // of a part, 0: sequences in one piece
+  size_t floats;
+};
+BlockPlan block_plan(bool delta, int T_, int B, int H, int dk, int dv, int longest, size_t most) {
+  BlockPlan r = {plan_pieces(T_, B, BT, slot_floats(H, dk), most, 0.23f), 0, 0};
+  r.floats = r.p.slots * slot_floats(H, dk);
+  if (delta || r.p.slots == 0 || r.p.count != 0) return r;
+  if (const int blocks = part_blocks(T_, B, H, dk, dv, longest)) {
+    const size_t more = (size_t)T_ / (blocks * BT) * H * part_floats(dk, dv);
+    if (r.floats + more <= most) r.blocks = blocks, r.floats += more;
+  }
+  return r;
 }
 
 template <typename T, int NS, bool DELTA>
 void launch(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const DecayArgs& a, float* S, float* out,
-            float* ws, size_t most, int H, int G, int dv, const SeqDesc& d, hipStream_t st) {
-  const PiecePlan plan = block_plan(d.Ttot, d.B, H, 64 * NS, most);
-  unsigned* seen = reinterpret_cast<unsigned*>(ws + plan.slots * H * cell_floats(64 * NS));
-  for (int w = 0; w < plan.windows; ++w) {
-    const Pieces pc = {BT, w * plan.count, plan.count};
-    hipLaunchKernelGGL((k_block_prep<T, NS, DELTA>), dim3((unsigned)plan.slots, H), dim3(256), 0, st, (const T*)q, ldq, (const T*)k,
+            float* ws, size_t most, int H, int G, int dv, int longest, const SeqDesc& d, hipStream_t st) {
+  constexpr int DK = 64 * NS;
+  const BlockPlan plan = block_plan(DELTA, d.Ttot, d.B, H, DK, dv, longest, most);
+  unsigned* seen = reinterpret_cast<unsigned*>(ws + plan.p.slots * H * cell_floats(DK));
+  const Parts pt = {ws + plan.p.slots * slot_floats(H, DK), plan.blocks};
+  const unsigned tiles = (dv + 15) / 16;
+  for (int w = 0; w < plan.p.windows; ++w) {
+    const Pieces pc = {BT, w * plan.p.count, plan.p.count};
+    hipLaunchKernelGGL((k_block_prep<T, NS, DELTA>), dim3((unsigned)plan.p.slots, H), dim3(256), 0, st, (const T*)q, ldq, (const T*)k,
                        ldk, (const T*)v, ldv, dv, a, ws, seen, H, G, pc, d);
-    hipLaunchKernelGGL((k_block_scan<T, NS, DELTA>), dim3(d.B * H, (dv + 15) / 16), dim3(256), 0, st, ws, seen, (const T*)v, ldv,
-                       S, out, H, dv, pc, d);
+    if constexpr (!DELTA)
+      if (plan.blocks > 0) {
+        const unsigned all = d.Ttot / (plan.blocks * BT), ends = (all * H + 7) / 8 * 8, parts = ((all + d.B) * H + 7) / 8 * 8;
+        hipLaunchKernelGGL((k_block_scan<T, NS, DELTA, ENDS>), dim3(ends * tiles), dim3(256), 0, st, ws, seen, (const T*)v, ldv, S, out, H,
+                           dv, pc, pt, d);
+        hipLaunchKernelGGL((k_block_scan<T, NS, DELTA, PARTS>), dim3(parts * tiles), dim3(256), 0, st, ws, seen, (const T*)v, ldv, S, out,
+                           H, dv, pc, pt, d);
+        continue;
+      }
+    hipLaunchKernelGGL((k_block_scan<T, NS, DELTA, WHOLE>), dim3(d.B * H, tiles), dim3(256), 0, st, ws, seen, (const T*)v, ldv, S, out, H,
+                       dv, pc, pt, d);
   }
   LIPA_CHECK_LAUNCH();
 }
 
 template <bool DELTA>
 void dispatch(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const DecayArgs& a, float* S,
-              float* out, float* ws, size_t most, int H, int G, int dk, int dv, const SeqDesc& d, hipStream_t st) {
+              float* out, float* ws, size_t most, int H, int G, int dk, int dv, int longest, const SeqDesc& d, hipStream_t st) {
   SEQ_DISPATCH_T(code, {
     switch (dk / 64) {
-      case 1: launch<T, 1, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, d, st); break;
-      case 2: launch<T, 2, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, d, st); break;
-      case 3: launch<T, 3, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, d, st); break;
-      default: launch<T, 4, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, d, st); break;
+      case 1: launch<T, 1, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, longest, d, st); break;
+      case 2: launch<T, 2, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, longest, d, st); break;
+      case 3: launch<T, 3, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, longest, d, st); break;
+      default: launch<T, 4, DELTA>(q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dv, longest, d, st); break;
     }
   });
 }
@@ -398,7 +512,12 @@ size_t seq_block_floats(int code, bool delta, const void* q, int ldq, const void
   }
   if (T_ < least * B) return 0;
   if (const size_t n = delta ? seq_delta_floats(T_, B, H, dk, dv, longest, most) : 0) return n;
-  return block_plan(T_, B, H, dk, most).slots * slot_floats(H, dk);
+  return block_plan(delta, T_, B, H, dk, dv, longest, most).floats;
+}
+
+// blocks of 16 tokens in a part of a sequence of linear attention, 0: in one piece
+int seq_gla_parts(int T_, int B, int H, int dk, int dv, int longest, size_t most) {
+  return block_plan(false, T_, B, H, dk, dv, longest, most).blocks;
 }
 
 void seq_block_delta(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* g,
@@ -409,12 +528,12 @@ void seq_block_delta(int code, const void* q, int ldq, const void* k, int ldk, c
     return;
   }
   const DecayArgs a = {g, nullptr, bpre, 1.f, 1.f};
-  dispatch<true>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dk, dv, d, st);
+  dispatch<true>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, G, dk, dv, longest, d, st);
 }
 
 void seq_block_gla(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const float* z,
                    const float* zb, float inv_tau, float qscale, float* S, float* out, float* ws, size_t most, int H, int dk,
                    int dv, int longest, SeqDesc d, hipStream_t st) {
   const DecayArgs a = {z, zb, nullptr, inv_tau, qscale};
-  dispatch<false>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, H, dk, dv, d, st);
+  dispatch<false>(code, q, ldq, k, ldk, v, ldv, a, S, out, ws, most, H, H, dk, dv, longest, d, st);
 }

@@ -238,42 +238,7 @@ struct Parts {
   float* at;
   int blocks;
 };
-// Part `id` of all that run, without a sequence's last one for `ends`; place: the sequence's first place.  (Counted, not bounded as the
-// pieces are: blocks of threads that find nothing to do leave others side by side on one CU, 84 us for 45.)
-struct Part {
-  int s, idx, place, t0, t1, end;
-};
-__device__ __forceinline__ bool find_part(const SeqDesc& d, int len, int id, bool ends, Part& p) {
-  int before = 0;                                            // parts in the lower half, places in the upper one
-  for (int b0 = 0; b0 < d.B; b0 += 64) {
-    const int lane = threadIdx.x & 63, b = min(b0 + lane, d.B - 1);
-    const int s0 = d.seq_off[b], s1 = d.seq_off[b + 1], on = d.live ? d.live[b] : 1;
-    const int n = on && b0 + lane < d.B ? (s1 - s0 + len - 1) / len : 0, own = n + (max(n - 1, 0) << 16);
-    int sum = own;
-#pragma unroll
-    for (int o = 1; o < 64; o *= 2) {
-      const int x = __shfl_up(sum, o, 64);
-      sum += lane >= o ? x : 0;
-    }
-    sum += before;
-    const unsigned long long m = __ballot((ends ? sum >> 16 : sum & 0xffff) > id);
-    if (m) {
-      const int at = __builtin_ctzll(m), first = __builtin_amdgcn_readlane(sum - own, at);
-      p.s = b0 + at;
-      p.idx = id - (ends ? first >> 16 : first & 0xffff);
-      p.place = first >> 16;
-      p.end = __builtin_amdgcn_readlane(s1, at);
-      p.t0 = __builtin_amdgcn_readlane(s0, at) + p.idx * len;
-      p.t1 = min(p.t0 + len, p.end);
-      return true;
-    }
-    before = __builtin_amdgcn_readlane(sum, 63);
-  }
-  return false;
-}
 __host__ __device__ constexpr int part_floats(int dk, int dv) { return dk * (((dv + 15) & ~15) + (dk > dv ? dk : (dv + 15) & ~15)); }
-
-enum { WHOLE, ENDS, PARTS };
 
 // A block owns 16 value columns of one (sequence, head) and walks its blocks of tokens, a window between two barriers for each.  Four waves
 // hold a quarter of the state's rows each, in registers in operand layout: they finish u from the shares of the key products, update

@@ -77,6 +77,7 @@ void seq_selective_scan(int, const void*, int, const float*, const float*, const
 size_t seq_selective_floats(int, int, int, int, size_t);
 size_t seq_delta_floats(int, int, int, int, int, int, size_t);
 int seq_delta_parts(int, int, int, int, int, int, size_t);
+int seq_gla_parts(int, int, int, int, int, int, size_t);
 bool seq_selective_rows(int, int, int, int, int, int, int, int, int);
 void seq_gla_scan(int, const void*, int, const void*, int, const void*, int, const float*, const float*, float, float,
                   float*, float*, int, int, int, SeqDesc, hipStream_t);
@@ -1342,9 +1343,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     if (seq_block_floats(0, true, nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, 0, (size_t)most) == 0) return 0;
     return seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, 0, (size_t)most) > 0 ? 32 : 16;
   }, py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS);
-  // blocks of tokens in a part of a sequence, where parts run side by side ("delta": of 32); 0: sequences in one piece
+  // blocks of tokens in a part of a sequence, where parts run side by side ("delta": of 32 tokens, "gla": of 16); 0: sequences in one piece
   m.def("scan_parts", [](const std::string& op, int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t longest, int64_t most) {
-    TORCH_CHECK(op == "delta", "scan_parts: delta");
+    TORCH_CHECK(op == "delta" || op == "gla", "scan_parts: delta or gla");
+    const bool delta = op == "delta";
+    if (seq_block_floats(0, delta, nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most) == 0)
+      return 0;
+    if (!delta) return seq_gla_parts((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most);
     if (seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most) == 0) return 0;
     return seq_delta_parts((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most);
   }, py::arg("op"), py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("longest"), py::arg("most") = MOST_WS);

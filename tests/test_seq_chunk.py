@@ -353,14 +353,45 @@ def test_delta_sequences_in_parts(lens, starts, live, H, G, dk, dv, dt):
 
 
 @pytest.mark.gpu
-def test_delta_parts_find_room_beside_the_blocks():
+@pytest.mark.parametrize("lens,starts,live", [([1025], [0], [1]), ([1, 997, 30, 610], [0, 7, 5, 0], [1, 1, 1, 1]),
+                                              ([640, 800, 64, 33], [3, 0, 0, 0], [0, 1, 1, 1])])
+@pytest.mark.parametrize("H,dk,dv,dt", [(2, 64, 20, torch.bfloat16), (3, 128, 36, torch.float32), (1, 256, 4, torch.bfloat16)])
+def test_gla_sequences_in_parts(lens, starts, live, H, dk, dv, dt):
     from llm_in_practise_amd.ops._native import native_seq
-    ext, shape = native_seq(), (4093, 1, 4, 128, 128)
-    whole, parts = ext.scan_floats("delta", *shape), ext.scan_floats("delta", *shape, longest=4093)
-    assert whole < parts and ext.scan_parts("delta", *shape, longest=4093, most=parts) > 0
-    assert ext.scan_parts("delta", *shape, longest=4093, most=parts - 1) == 0
-    assert ext.scan_floats("delta", *shape, most=parts - 1, longest=4093) == whole
-    assert ext.scan_parts("delta", *shape, longest=0) == 0
+    T = sum(lens)
+    blocks = native_seq().scan_parts("gla", T, len(lens), H, dk, dv, max(lens))
+    assert 0 < 2 * 16 * blocks < max(lens) + 16 * blocks
+    g = torch.Generator().manual_seed(dk + dv + len(lens))
+    P, z, zb = torch.randn(T, 2 * H * dk + H * dv, generator=g).to(dt), torch.randn(T, H * dk, generator=g), torch.randn(H * dk, generator=g)
+    z[::97, ::3] = -2000.0                               # channels that forget everything
+    S0 = torch.randn(len(lens), H, dv, dk, generator=g)
+    tok = torch.cat([torch.full((n,), bool(on)) for n, on in zip(lens, live)])
+
+    def run(dev, p):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, starts, dev, live)
+        st["S"].copy_(S0)
+        p = p.to(dev)
+        o = R.gated_linear_scan(p[:, :H * dk], p[:, H * dk:2 * H * dk], p[:, 2 * H * dk:], z.to(dev), zb.to(dev), 16.0, dk ** -0.5, st["S"], H, sb)
+        return o.cpu()[tok], st["S"].cpu()
+    _close(run("cuda", P), run("cpu", P), ("o", "state"))
+    bad, first = P.clone(), sum(lens[:1]) if len(lens) > 1 else 0
+    bad[first + 16 * blocks - 3, 2 * H * dk + 3] = float("nan")            # a value near the end of a part
+    a, b = run("cpu", bad), run("cuda", bad)
+    for x, y in zip(a, b):
+        assert torch.equal(x.isnan(), y.isnan())
+    _close((b[0].nan_to_num(),), (a[0].nan_to_num(),), ("o",))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op,dk", [("delta", 128), ("gla", 64)])
+def test_parts_find_room_beside_the_blocks(op, dk):
+    from llm_in_practise_amd.ops._native import native_seq
+    ext, shape = native_seq(), (4093, 1, 4, dk, 128)
+    whole, parts = ext.scan_floats(op, *shape), ext.scan_floats(op, *shape, longest=4093)
+    assert whole < parts and ext.scan_parts(op, *shape, longest=4093, most=parts) > 0
+    assert ext.scan_parts(op, *shape, longest=4093, most=parts - 1) == 0
+    assert ext.scan_floats(op, *shape, most=parts - 1, longest=4093) == whole
+    assert ext.scan_parts(op, *shape, longest=0) == 0
 
 
 @pytest.mark.gpu
