@@ -339,7 +339,7 @@ constexpr int64_t MOST_WS = 1ll << 28;
 
 std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor fpre, Tensor ib, Tensor fb, double cap,
                   double qscale, Tensor S, Tensor N, Tensor M, int64_t H, std::vector<Tensor> desc,
-                  optional<Tensor> live, int64_t most, int64_t longest) {
+                  optional<Tensor> live, int64_t longest, int64_t most) {
   const int code = code_of(q);
   const int64_t T = q.size(0);
   TORCH_CHECK(q.dim() == 2 && q.size(1) % H == 0 && v.dim() == 2 && v.size(1) % H == 0, "q/k/v: [T, H * d]");
@@ -384,7 +384,7 @@ std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor
 }
 
 Tensor delta_scan(Tensor q, Tensor k, Tensor v, Tensor g, Tensor bpre, Tensor S, int64_t H, int64_t G,
-                  std::vector<Tensor> desc, optional<Tensor> live, int64_t most, int64_t longest) {
+                  std::vector<Tensor> desc, optional<Tensor> live, int64_t longest, int64_t most) {
   const int code = code_of(q);
   const int64_t T = q.size(0);
   TORCH_CHECK(G >= 1 && H % G == 0 && q.dim() == 2 && q.size(1) % G == 0 && v.dim() == 2 && v.size(1) % H == 0,
@@ -460,7 +460,7 @@ Tensor talk_attention(Tensor q, Tensor kc, Tensor vc, Tensor talk, Tensor gate, 
 
 // ---- selective state space (state-space duality form): q = C, k = B [T, G * N], v = x [T, H * P], dtraw [T, H]
 Tensor ssd_scan(Tensor q, Tensor k, Tensor v, Tensor dtraw, Tensor dt_bias, Tensor a_log, Tensor dskip, Tensor S,
-                int64_t H, int64_t G, std::vector<Tensor> desc, optional<Tensor> live, int64_t most, int64_t longest) {
+                int64_t H, int64_t G, std::vector<Tensor> desc, optional<Tensor> live, int64_t longest, int64_t most) {
   const int code = code_of(q);
   const int64_t T = q.size(0);
   TORCH_CHECK(G >= 1 && H % G == 0 && q.dim() == 2 && q.size(1) % G == 0 && v.dim() == 2 && v.size(1) % H == 0,
@@ -1177,7 +1177,7 @@ Tensor selective_scan(Tensor x, Tensor dt_pre, Tensor dt_bias, Tensor b, Tensor 
 
 // q, k [T, H * dk], v [T, H * dv] activation rows, z float [T, H * dk] contiguous; S float [slots, H, dv, dk] in place
 Tensor gated_linear_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, double tau, double q_scale, Tensor S,
-                         int64_t H, std::vector<Tensor> desc, optional<Tensor> live, int64_t most, int64_t longest) {
+                         int64_t H, std::vector<Tensor> desc, optional<Tensor> live, int64_t longest, int64_t most) {
   const int code = code_of(q);
   TORCH_CHECK(H >= 1 && q.dim() == 2 && q.size(1) % H == 0 && v.dim() == 2 && v.size(1) % H == 0,
               "q/k: [T, H * dk], v: [T, H * dv]");
@@ -1296,13 +1296,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias") = py::none());
   m.def("mlstm_scan", &mlstm_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("ipre"), py::arg("fpre"), py::arg("ib"),
         py::arg("fb"), py::arg("cap"), py::arg("qscale"), py::arg("S"), py::arg("N"), py::arg("M"), py::arg("H"),
-        py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS, py::arg("longest") = 0);
+        py::arg("desc"), py::arg("live"), py::arg("longest") = 0, py::arg("most") = MOST_WS);
   m.def("delta_scan", &delta_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("g"), py::arg("bpre"), py::arg("S"),
-        py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"), py::arg("most") = MOST_WS, py::arg("longest") = 0);
+        py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"), py::arg("longest") = 0, py::arg("most") = MOST_WS);
   m.def("talk_attention", &talk_attention);
   m.def("ssd_scan", &ssd_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("dtraw"), py::arg("dt_bias"),
         py::arg("a_log"), py::arg("dskip"), py::arg("S"), py::arg("H"), py::arg("G"), py::arg("desc"), py::arg("live"),
-        py::arg("most") = MOST_WS, py::arg("longest") = 0);
+        py::arg("longest") = 0, py::arg("most") = MOST_WS);
   m.def("embed_pair", &embed_pair, py::arg("tok"), py::arg("table"), py::arg("pair"), py::arg("prev"), py::arg("scale"),
         py::arg("mul_prev"), py::arg("mul_cur"), py::arg("desc"), py::arg("live"), py::arg("out") = py::none());
   m.def("scaled_postnorm", &scaled_postnorm);
@@ -1365,7 +1365,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("scale"), py::arg("most") = MOST_WS);
   m.def("gated_linear_scan", &gated_linear_scan, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("z"), py::arg("z_bias"),
         py::arg("tau"), py::arg("q_scale"), py::arg("S"), py::arg("H"), py::arg("desc"), py::arg("live"),
-        py::arg("most") = MOST_WS, py::arg("longest") = 0);
+        py::arg("longest") = 0, py::arg("most") = MOST_WS);
   m.def("delta_rule_gates", &delta_rule_gates);
   m.def("general_delta_scan", &general_delta_scan);
 }

@@ -30,7 +30,7 @@ def mlstm_scan(q, k, v, i_pre, f_pre, i_bias, f_bias, cap: float, q_scale: float
     and ``None, None``)."""
     if use_seq(q):
         return tuple(native_seq().mlstm_scan(q, k, v, i_pre, f_pre, i_bias, f_bias, cap, q_scale, S, N, M, heads,
-                                             sb.desc, sb.live, longest=sb.longest))
+                                             sb.desc, sb.live, sb.longest))
     return ref.mlstm_scan(q, k, v, i_pre, f_pre, i_bias, f_bias, cap, q_scale, S, N, M, heads, sb), None, None
 
 
@@ -47,7 +47,7 @@ def gated_delta_scan(q, k, v, g, beta_pre, S, heads: int, kv_heads: int, sb):
     o = S^T q``.  Returns float ``[T, H, dv]``."""
     if use_seq(q):
         return native_seq().delta_scan(q, k, v, g.contiguous(), beta_pre.contiguous(), S, heads, kv_heads, sb.desc,
-                                       sb.live, longest=sb.longest)
+                                       sb.live, sb.longest)
     return ref.delta_scan(q, k, v, g, beta_pre, S, heads, kv_heads, sb)
 
 
@@ -57,7 +57,7 @@ def ssd_scan(c, b, x, dt_raw, dt_bias, a_log, d_skip, S, heads: int, groups: int
     in the activation dtype, ``dt_raw`` ``[T, H]`` (a column slice is fine); head ``h`` reads group ``h // (H/G)``;
     ``S`` float ``[slots, H, P, N]``.  Step sizes, decays and the state are float.  Returns float ``[T, H*P]``."""
     if use_seq(c):
-        return native_seq().ssd_scan(c, b, x, dt_raw, dt_bias, a_log, d_skip, S, heads, groups, sb.desc, sb.live, longest=sb.longest)
+        return native_seq().ssd_scan(c, b, x, dt_raw, dt_bias, a_log, d_skip, S, heads, groups, sb.desc, sb.live, sb.longest)
     return ref.ssd_scan(c, b, x, dt_raw, dt_bias, a_log, d_skip, S, heads, groups, sb)
 
 
@@ -104,5 +104,5 @@ def gated_linear_scan(q, k, v, z, z_bias, tau: float, q_scale: float, S, heads: 
     float (the decay as ``exp(log sigmoid / tau)``).  Returns float ``[T, H, dv]``."""
     if use_seq(q):
         return native_seq().gated_linear_scan(q, k, v, z, z_bias, tau, q_scale, S, heads, sb.desc, sb.live,
-                                               longest=sb.longest)
+                                               sb.longest)
     return ref.gated_linear_scan(q, k, v, z, z_bias, tau, q_scale, S, heads, sb)
