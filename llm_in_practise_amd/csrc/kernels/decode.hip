@@ -201,7 +201,57 @@ __device__ __forceinline__ bf16x4 dec_tr_read(const bf16* p) {
   typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
   return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p));
 }
-__device__ __forceinline__ int split_chunk32(int len, int nsplit) { return ((len + nsplit - 1) / nsplit + 31) & ~31; }
+// a / b, both positive, without a division's forty instructions
+__device__ __forceinline__ int quotient(int a, int b) {
+  int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
+  q -= q * b > a;
+  q += (q + 1) * b <= a;
+  return q;
+}
+__device__ __forceinline__ int split_chunk32(int len, int nsplit, int least) { return (max(quotient(len + nsplit - 1, nsplit), least) + 31) & ~31; }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int plus_dpp(int v) { return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false); }
+__device__ __forceinline__ int scan64(int v) {               // sum over the lanes up to this one
+  v = plus_dpp<0x111, 0xF>(v);                               // row_shr 1, 2, 4, 8
+  v = plus_dpp<0x112, 0xF>(v);
+  v = plus_dpp<0x114, 0xF>(v);
+  v = plus_dpp<0x118, 0xF>(v);
+  v = plus_dpp<0x142, 0xA>(v);                               // row_bcast 15 into the rows 1 and 3, 31 into 2 and 3
+  return plus_dpp<0x143, 0xC>(v);
+}
+// Item `id` of all (row, kv head, split of its keys) that hold keys: rows one after the other, of each the heads, of each the splits.  False past
+// the last one.  (Counted over the rows' lengths, 64 of them at a time; what a wave holds once is read into scalar registers, or every
+// address behind it is a lane's own: 15.6 -> 17.7 us for 12 rows.)
+struct SplitItem {
+  int b, kh, split, len, chunk;
+};
+__device__ __forceinline__ bool find_split(const int64_t* __restrict__ pos, int B, int hkv, int nsplit, int least, int id, SplitItem& it) {
+  if (B == 1) {                                              // (a grid of splits and heads)
+    it = {0, (int)blockIdx.y, (int)blockIdx.x, (int)pos[0] + 1, 0};
+    it.chunk = __builtin_amdgcn_readfirstlane(split_chunk32(it.len, nsplit, least));
+    return it.split * it.chunk < it.len;
+  }
+  int before = 0;
+  for (int b0 = 0; b0 < B; b0 += 64) {
+    const int lane = threadIdx.x & 63;
+    const int len = b0 + lane < B ? max((int)pos[b0 + lane] + 1, 0) : 0, chunk = split_chunk32(len, nsplit, least);
+    const int n = quotient(len + chunk - 1, chunk);
+    const int sum = before + scan64(n * hkv);
+    const unsigned long long m = __ballot(sum > id);
+    if (m) {
+      const int at = __builtin_ctzll(m), each = __builtin_amdgcn_readlane(n, at);
+      const int local = id - (__builtin_amdgcn_readlane(sum, at) - each * hkv);
+      it.b = b0 + at;
+      it.len = __builtin_amdgcn_readlane(len, at);
+      it.chunk = __builtin_amdgcn_readlane(chunk, at);
+      it.kh = __builtin_amdgcn_readfirstlane(quotient(local, each));
+      it.split = local - it.kh * each;
+      return true;
+    }
+    before = __builtin_amdgcn_readlane(sum, 63);
+  }
+  return false;
+}
 // x as the float it is rounded to: the compiler fuses no product with a sum across this
 __device__ __forceinline__ float rounded(float x) {
   asm("" : "+v"(x));
@@ -215,7 +265,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
                                                           bf16* __restrict__ kc, bf16* __restrict__ vc,
                                                           const int64_t* __restrict__ pos, float* __restrict__ opart,
                                                           float* __restrict__ mpart, float* __restrict__ lpart,
-                                                          int Smax, int hq, int hkv, int nsplit, float scale_log2) {
+                                                          int Smax, int B, int hq, int hkv, int nsplit, int least, float scale_log2) {
   constexpr int LDR = D + 8;          // padded LDS row (elements)
   constexpr int CH = D / 8;           // 16-B chunks per row
   constexpr int NS = D / 32;          // k-steps over the head dim
@@ -227,12 +277,11 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
   static_assert(4 * 16 * D * 4 <= 4 * VT * 2, "merge buffer aliases the V tiles");
 
   asm volatile("" ::"s"(q), "s"(knew), "s"(vnew), "s"(kc), "s"(vc), "s"(ldq), "s"(ldkn), "s"(ldvn));   // (all at once, not behind the length)
-  const int split = blockIdx.x, kh = blockIdx.y, b = blockIdx.z;
   const int G = hq / hkv;
-  const int len = (int)pos[b] + 1;
-  const int chunk = split_chunk32(len, nsplit);
+  SplitItem it;
+  if (!find_split(pos, B, hkv, nsplit, least, blockIdx.x, it)) return;
+  const int split = it.split, kh = it.kh, b = it.b, len = it.len, chunk = it.chunk;
   const int k0 = split * chunk, k1 = min(k0 + chunk, len);
-  if (k0 >= len) return;              // whole workgroup: empty split, never merged
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, li = lane & 15;
 
   const size_t rs = (size_t)hkv * D;
@@ -375,7 +424,7 @@ __global__ __launch_bounds__(D) void decode_attn_merge2_k(const float* __restric
                                                           const float* __restrict__ mpart,
                                                           const float* __restrict__ lpart,
                                                           const int64_t* __restrict__ pos, bf16* __restrict__ out,
-                                                          int hq, int nsplit) {
+                                                          int hq, int nsplit, int least) {
   extern __shared__ __attribute__((aligned(16))) float sc[];   // weight of each split, then its sum
   __shared__ float scratch[D / 64];
   const size_t h = blockIdx.x;  // b*hq + head
@@ -386,7 +435,7 @@ __global__ __launch_bounds__(D) void decode_attn_merge2_k(const float* __restric
   for (int j = 0; j < NP; ++j) v[j] = op[(size_t)min(j, nsplit - 1) * D];
   const float m0 = mpart[h * nsplit + min(d, nsplit - 1)], l0 = lpart[h * nsplit + min(d, nsplit - 1)];
   const int len = (int)pos[h / hq] + 1;
-  const int chunk = split_chunk32(len, nsplit);
+  const int chunk = split_chunk32(len, nsplit, least);
   const int nv = min(nsplit, (len + chunk - 1) / chunk);
   float m = d < nv ? m0 : -INFINITY;
   for (int s = d + D; s < nv; s += D) m = fmaxf(m, mpart[h * nsplit + s]);
@@ -586,6 +635,18 @@ void launch_decode_attention(const void* q, const void* kc, const void* vc, cons
 }
 
 
+// Fewest keys of a split.  The number of splits stands when a step is captured, for rows of any length; cut that finely a short row's
+// splits leave two or three of a workgroup's four waves idle and are more workgroups than the chip holds.  By rows x kv heads (the row's own
+// length and these alone decide how it is cut, not its neighbours').  µs, both launches, heads of 128, 32 query on 8, from memory, splits as
+// captured with the empty ones launched between the others -> at least 64 / 128 / 256 keys, the empty ones last: 12 rows of 474 to 1400 keys
+// 20.5 -> 20.1 / 15.6 / 18.2; 6 of 120 to 300 11.0 -> 8.9 / 9.5 / 11.6; 20 of 33 to 100 12.1 -> 9.5 / 9.8 / 9.8, of 644 to 1900 29.8 -> 30.4 / 29.6 /
+// 29.3; 32 of 314 to 1000 28.1 -> 27.2 / 25.1 / 27.2; 48 of 125 to 400 24.3 -> 23.0 / 20.2 / 22.3; 64 of 688 to 1700 68.8 -> 69.8 / 69.7 / 67.7, of 80 to 200
+// 23.1 -> 20.3 / 18.4 / 17.3.  One row of 937 keeps 32: 8.3, and 8.3 / 9.0 / 11.2.
+int split_least(int B, int hkv) {
+  const int pairs = B * hkv;
+  return B == 1 ? 32 : pairs < 64 ? 64 : pairs < 512 ? 128 : 256;
+}
+
 // v2: MFMA split-K decode attention with the KV append fused (see decode_attn_mfma_k)
 int decode_split_plan2(int B, int hkv, int max_len) {
   const int pairs = std::max(1, B * hkv);
@@ -596,15 +657,16 @@ int decode_split_plan2(int B, int hkv, int max_len) {
 void launch_decode_attention2(const void* q, int ldq, const void* knew, int ldkn, const void* vnew, int ldvn, void* kc,
                               void* vc, const int64_t* pos, float* opart, float* mpart, float* lpart, void* out, int B,
                               int Smax, int hq, int hkv, int d, int nsplit, float scale, hipStream_t st) {
-  dim3 grid(nsplit, hkv, B);
+  const dim3 grid = B == 1 ? dim3(nsplit, hkv) : dim3(nsplit * hkv * B);
+  const int least = split_least(B, hkv);
   const float sl2 = scale * 1.4426950408889634f;
 #define M(D_, NP_) \
-  decode_attn_merge2_k<D_, NP_><<<B * hq, D_, 2 * (std::max(nsplit, NP_) + 3 & ~3) * sizeof(float), st>>>(opart, mpart, lpart, pos, (bf16*)out, hq, nsplit)
+  decode_attn_merge2_k<D_, NP_><<<B * hq, D_, 2 * (std::max(nsplit, NP_) + 3 & ~3) * sizeof(float), st>>>(opart, mpart, lpart, pos, (bf16*)out, hq, nsplit, least)
 #define P(D_)                                                                                                          \
   decode_attn_mfma_k<D_><<<grid, 256, 0, st>>>((const bf16*)q, ldq, (const bf16*)knew, ldkn, (const bf16*)vnew, ldvn, \
-                                               (bf16*)kc, (bf16*)vc, pos, opart, mpart, lpart, Smax, hq, hkv, nsplit, \
+                                               (bf16*)kc, (bf16*)vc, pos, opart, mpart, lpart, Smax, B, hq, hkv, nsplit, least, \
                                                sl2);                                                                   \
-  if (nsplit > 8) M(D_, 32); else if (nsplit > 4) M(D_, 8); else M(D_, 4)
+  if (nsplit > 16) M(D_, 32); else if (nsplit > 8) M(D_, 16); else if (nsplit > 4) M(D_, 8); else M(D_, 4)
   if (d == 128) { P(128); } else { P(64); }
 #undef P
 #undef M

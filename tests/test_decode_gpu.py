@@ -144,6 +144,30 @@ def test_decode_attention_append_merge(native_ext, max_len, d):
     assert (o.float() - r).abs().max().item() < 3 * 2.0 ** -8 * vc.float().abs().max().item()
 
 
+@pytest.mark.parametrize("hkv,d", [(1, 128), (3, 64), (8, 128)])
+@pytest.mark.parametrize("B", [2, 20, 63, 64, 65, 130])
+def test_decode_attention_append_counts_the_splits_that_have_keys(native_ext, B, hkv, d):
+    """Rows whose keys end at, behind and in front of a shortest split (64, 128, 256), in batches on both sides of 64 rows and of each
+    shortest split; a row's bits are the same among other neighbours."""
+    torch.manual_seed(B + hkv)
+    hq, max_len = 2 * hkv, 700
+    ends = [0, 62, 63, 64, 126, 127, 128, 254, 255, 256, 699, 511, 512]
+    P = torch.tensor([ends[(i * 5) % len(ends)] for i in range(B)], device=DEV)
+    kc, vc = (torch.randn(B, max_len, hkv * d, device=DEV).to(torch.bfloat16) for _ in range(2))
+    q, k, v = (torch.randn(B, n * d, device=DEV).to(torch.bfloat16) for n in (hq, hkv, hkv))
+    o = native_ext.decode_attention_append(q, k, v, kc, vc, P, hq, hkv, d, max_len, 1 / math.sqrt(d))
+    rows = torch.arange(B, device=DEV)
+    assert torch.equal(kc[rows, P], k) and torch.equal(vc[rows, P], v)
+    r = decode_attention_reference(q.float(), kc.float(), vc.float(), (P + 1).int(), hq, hkv, d)
+    # weights and values in bf16: 2^-8 of the largest value for each, and the output's own rounding
+    assert (o.float() - r).abs().max().item() < 3 * 2.0 ** -8 * vc.float().abs().max().item()
+    keep = B // 2
+    other = torch.full_like(P, 300)
+    other[keep] = P[keep]
+    again = native_ext.decode_attention_append(q, k, v, kc, vc, other, hq, hkv, d, max_len, 1 / math.sqrt(d))
+    assert torch.equal(again[keep], o[keep])
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 33, 64])
 @pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 12288), (272, 192)])
 def test_gemm_skinny_matches_fp32(native_ext, M, N, K):
