@@ -8,6 +8,8 @@
 // Router scores, weights and the combine are float; expert products read the activation type and accumulate in float.
 #include "seq_common.h"
 
+#include <type_traits>
+
 using namespace lipa;
 
 constexpr int RPL = 4;   // router outputs per lane: experts + identity experts <= 64 * RPL
@@ -494,6 +496,147 @@ __global__ __launch_bounds__(256) void k_moe_pair_down(const T* __restrict__ a, 
   if (lane == 0) out[(size_t)t * W + c] = acc;
 }
 
+// ---- the same of a decode batch, bf16: an expert's rows are read once for all of its pairs, which share them on the matrix units, instead of once
+// a pair.  Every block finds the pairs of its expert by itself, so there is no sort.  What stays: sums and the experts' outputs are float, a
+// token's outputs are added in the order of its choices.  Bound by latency: ids, rows and weights are one round trip each, two launches.
+constexpr int FEW = 512;                        // pairs
+
+// The pairs of expert e in their order, in a wave's own place in LDS; their number.
+__device__ __forceinline__ int list_pairs(const int* __restrict__ idx, int P, int e, int lane, unsigned short* list) {
+  int v[FEW / 64], n = 0;
+#pragma unroll
+  for (int i = 0; i < FEW / 64; ++i) v[i] = idx[min(64 * i + lane, P - 1)];
+#pragma unroll
+  for (int i = 0; i < FEW / 64; ++i) {
+    const unsigned long long m = __ballot(64 * i + lane < P && v[i] == e);
+    if (m >> lane & 1) list[n + __popcll(m & ((1ull << lane) - 1))] = (unsigned short)(64 * i + lane);
+    n += __popcll(m);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  return __builtin_amdgcn_readfirstlane(n);
+}
+
+// A row of lanes' operands over S steps of 32 of the depth, all on their way at once.  (Steps past the end are the last one again, and left out.)
+template <int S>
+__device__ __forceinline__ void load_steps(const bf16* p, int steps, bf16x8 (&v)[S]) {
+#pragma unroll
+  for (int s = 0; s < S; ++s) v[s] = *reinterpret_cast<const bf16x8*>(p + 32 * min(s, steps - 1));
+}
+template <int S>
+__device__ __forceinline__ f32x4 multiply_steps(const bf16x8 (&a)[S], const bf16x8 (&x)[S], int steps, f32x4 acc) {
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], x[s], acc, 0, 0, 0);
+  return acc;
+}
+// f(tiles) for the tiles of 16 that `left` pairs fill, four at most
+template <typename F>
+__device__ __forceinline__ void few_tiles(int left, F f) {
+  if (left <= 16) f(std::integral_constant<int, 1>{});
+  else if (left <= 32) f(std::integral_constant<int, 2>{});
+  else if (left <= 48) f(std::integral_constant<int, 3>{});
+  else f(std::integral_constant<int, 4>{});
+}
+
+// stage 1: a block 16 hidden units of an expert, gate and up rows, a wave a quarter of the depth.  Its weights are on their way before it
+// knows its pairs, a tile's rows under the products of the tile before.
+template <int S>
+__global__ __launch_bounds__(256, 1) void k_moe_few_up(const bf16* __restrict__ h, int ldh, const bf16* __restrict__ wgu,
+                                                       const int* __restrict__ idx, bf16* __restrict__ a, int P, int top, int F, int W,
+                                                       float limit, int mode, const float* __restrict__ inw) {
+  __shared__ unsigned short list[4][FEW];
+  __shared__ f32x4 red[4][2][4][64];
+  const int e = blockIdx.y, r0 = blockIdx.x * 16, w = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, q = lane >> 4;
+  const int steps = W / 128, k0 = w * (W / 4) + 8 * q;
+  const bf16* wg = wgu + ((size_t)e * 2 * F + r0 + li) * W + k0;
+  bf16x8 gate[S], up[S], x[2][S];
+  load_steps<S>(wg, steps, gate);
+  load_steps<S>(wg + (size_t)F * W, steps, up);
+  const int n = list_pairs(idx, P, e, lane, list[w]);
+  for (int g0 = 0; g0 < n; g0 += 64)
+    few_tiles(n - g0, [&](auto tiles) {
+      constexpr int NT = decltype(tiles)::value;
+      const auto load = [&](int t) {
+        load_steps<S>(h + (size_t)(list[w][min(g0 + 16 * t + li, n - 1)] / top) * ldh + k0, steps, x[t & 1]);
+      };
+      load(0);
+      f32x4 acc[2][NT] = {};
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if (t + 1 < NT) load(t + 1);
+        acc[0][t] = multiply_steps<S>(gate, x[t & 1], steps, acc[0][t]);
+        acc[1][t] = multiply_steps<S>(up, x[t & 1], steps, acc[1][t]);
+      }
+      if (g0 > 0) __syncthreads();              // (the last sums are read)
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) red[w][r][t][lane] = acc[r][t];
+      __syncthreads();
+      const int at = g0 + 16 * w + li;          // wave w finishes tile w: hidden units 4 q .. 4 q + 3 of pair li
+      if (w >= NT || at >= n) return;
+      f32x4 g = red[0][0][w][lane], u = red[0][1][w][lane];
+#pragma unroll
+      for (int i = 1; i < 4; ++i) {
+        g += red[i][0][w][lane];
+        u += red[i][1][w][lane];
+      }
+      const int pair = list[w][at];
+      const float iw = inw != nullptr ? inw[pair] : 1.f;
+      bf16x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = (bf16)glu(iw * g[i], iw * u[i], limit, mode);
+      *reinterpret_cast<bf16x4*>(a + (size_t)pair * F + r0 + 4 * q) = o;
+    });
+}
+
+// stage 2: a block 16 output columns, a wave every eighth expert; the pairs' outputs stay float and meet in LDS
+template <int S>
+__global__ __launch_bounds__(512) void k_moe_few_down(const bf16* __restrict__ a, const bf16* __restrict__ wd, const int* __restrict__ idx,
+                                                      const float* __restrict__ wts, const bf16* __restrict__ h, int ldh,
+                                                      const bf16* __restrict__ shared, const float* __restrict__ sgate,
+                                                      float* __restrict__ out, int T_, int top, int E, int F, int W) {
+  constexpr int LDY = 20;
+  __shared__ unsigned short list[8][FEW];
+  __shared__ __attribute__((aligned(16))) float y[FEW * LDY];
+  const int c0 = blockIdx.x * 16, w = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, q = lane >> 4, P = T_ * top, steps = F / 32;
+  for (int e = w; e < E; e += 8) {
+    bf16x8 rows[S], x[2][S];
+    load_steps<S>(wd + ((size_t)e * W + c0 + li) * F + 8 * q, steps, rows);
+    const int n = list_pairs(idx, P, e, lane, list[w]);
+    for (int g0 = 0; g0 < n; g0 += 64)
+      few_tiles(n - g0, [&](auto tiles) {
+        constexpr int NT = decltype(tiles)::value;
+        int pair[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) pair[t] = list[w][min(g0 + 16 * t + li, n - 1)];
+        load_steps<S>(a + (size_t)pair[0] * F + 8 * q, steps, x[0]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          if (t + 1 < NT) load_steps<S>(a + (size_t)pair[t + 1] * F + 8 * q, steps, x[(t + 1) & 1]);
+          const f32x4 acc = multiply_steps<S>(rows, x[t & 1], steps, f32x4{0.f, 0.f, 0.f, 0.f});
+          *reinterpret_cast<f32x4*>(y + pair[t] * LDY + 4 * q) = acc;           // (pairs past the end repeat the last)
+        }
+      });
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the list is read)
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 4 * T_; i += 512) {
+    const int t = i >> 2, c = c0 + 4 * (i & 3);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    if (shared != nullptr) acc = load4(shared + (size_t)t * W + c) * (sgate != nullptr ? sigmoidf_(sgate[t]) : 1.f);
+    for (int j = 0; j < top; ++j) {
+      const int p = t * top + j, e = idx[p];
+      const float wt = wts != nullptr ? wts[p] : 1.f;
+      if (e >= E)
+        acc += load4(h + (size_t)t * ldh + c) * wt;
+      else if (e >= 0)
+        acc += *reinterpret_cast<const f32x4*>(y + p * LDY + 4 * (i & 3)) * wt;
+    }
+    *reinterpret_cast<f32x4*>(out + (size_t)t * W + c) = acc;
+  }
+}
+
 // sorted path: out[t, c] = sum_j w[t, j] * (e_j < E ? ys[pos[t, j], c] : h[t, c]) + shared[t, c]
 template <typename T>
 __global__ __launch_bounds__(256) void k_moe_combine(const T* __restrict__ ys, const long* __restrict__ pos,
@@ -634,10 +777,30 @@ void seq_route_fused(int code, const void* h, int ldh, const float* router, cons
   LIPA_CHECK_LAUNCH();
 }
 
+// Where a decode batch's experts are read once: operands that 16-byte loads take, at most 2048 deep (512 the second products), pairs that LDS holds.
+// us of a step in a captured graph, routing included, a wave a (pair, row) -> here, 8 experts: width 2048, F 384, top 2, 12 / 16 / 32 / 48 / 128 pairs 22.9 ->
+// 23.7 (not taken), 25.7 -> 24.1 (not taken), 37 -> 24, 47 -> 25, 87 -> 29; width 1024, F 448, 16 / 32 / 128 pairs 18.1 -> 19.1 (not taken), 25 -> 20, 54 -> 23; F 512, top 4,
+// width 2048, 12 / 16 / 64 / 256 26.0 -> 27.1 (not taken), 29.9 -> 28.0, 62 -> 29, 150 -> 37; width 1024, 16 / 32 / 256 18.6 -> 20.8 (not taken), 25.4 -> 21.7, 91 -> 29.
+// More experts have fewer pairs each to share their rows.
+bool seq_moe_few(int code, const void* h, int ldh, const void* wgu, const void* wd, const void* shared, int T_, int top, int E, int F, int W) {
+  const auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  const long P = (long)T_ * top;
+  return code == 0 && P <= FEW && P * F * W >= 14000000 && P >= 2 * E && E <= 16 && F % 32 == 0 && F <= 512 && W % 128 == 0 && W <= 2048 && ldh % 8 == 0 &&
+         aligned(h) && aligned(wgu) && aligned(wd) && aligned(shared);
+}
+
 void seq_moe_pairs(int code, const void* h, int ldh, const void* wgu, const void* wd, const int* idx, const float* wts,
                    const void* shared, const float* sgate, void* a, float* out, int T_, int top, int E, int F, int W,
                    float limit, int mode, int weight_input, hipStream_t st) {
   if (T_ == 0) return;
+  if (seq_moe_few(code, h, ldh, wgu, wd, shared, T_, top, E, F, W)) {
+    hipLaunchKernelGGL(W <= 1024 ? k_moe_few_up<8> : k_moe_few_up<16>, dim3(F / 16, E), dim3(256), 0, st, (const bf16*)h, ldh, (const bf16*)wgu, idx,
+                       (bf16*)a, T_ * top, top, F, W, limit, mode, weight_input ? wts : nullptr);
+    hipLaunchKernelGGL(F <= 256 ? k_moe_few_down<8> : k_moe_few_down<16>, dim3(W / 16), dim3(512), 0, st, (const bf16*)a, (const bf16*)wd, idx,
+                       weight_input ? nullptr : wts, (const bf16*)h, ldh, (const bf16*)shared, sgate, out, T_, top, E, F, W);
+    LIPA_CHECK_LAUNCH();
+    return;
+  }
   SEQ_DISPATCH_T(code, {
     hipLaunchKernelGGL(k_moe_pair_up<T>, dim3(T_ * top, (F + 3) / 4), dim3(256), 0, st, (const T*)h, ldh, (const T*)wgu,
                        idx, (T*)a, T_ * top, top, E, F, W, limit, mode, weight_input ? wts : nullptr);

@@ -52,6 +52,7 @@ void seq_route_fused(int, const void*, int, const float*, const float*, int*, fl
                      int, int, float*, int, hipStream_t);
 void seq_moe_pairs(int, const void*, int, const void*, const void*, const int*, const float*, const void*, const float*,
                    void*, float*, int, int, int, int, int, float, int, int, hipStream_t);
+bool seq_moe_few(int, const void*, int, const void*, const void*, const void*, int, int, int, int, int);
 bool seq_moe_tiles_ok(int, const void*, const void*, const void*, long, int, int, int, int);
 void seq_moe_tiles(const void*, const void*, const void*, const int*, const float*, int*, int*, long*, void*, void*, int, int, int,
                    int, int, float, int, hipStream_t);
@@ -1314,6 +1315,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("route_grouped", &route_grouped);
   m.def("route_fused", &route_fused);
   m.def("moe_pairs", &moe_pairs);
+  // whether a decode batch's experts are read once (bf16, operands that its loads take)
+  m.def("moe_few", [](int64_t T, int64_t top, int64_t E, int64_t F, int64_t W) {
+    return seq_moe_few(0, nullptr, (int)W, nullptr, nullptr, nullptr, (int)T, (int)top, (int)E, (int)F, (int)W);
+  });
   m.def("moe_tiles", &moe_tiles);
   m.def("moe_combine_sorted", &moe_combine_sorted);
   m.def("ff_act", &ff_act, py::arg("z"), py::arg("mode"), py::arg("limit"), py::arg("row_scale") = py::none());

@@ -183,3 +183,41 @@ def test_combine_rows_together(T, W, top, dtype):
         got = native_seq().moe_combine_sorted(ys, pos, idx, w, h, sh, E, g).double()
         bound = (top + 8) * 2.0 ** -23 * (base.abs() + terms.abs().sum(1))
         assert ((got - base - terms.sum(1)).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,top,E,F,W", [(33, 2, 3, 384, 2048), (8, 2, 8, 512, 2048), (17, 3, 8, 448, 1024), (64, 4, 8, 512, 1024), (128, 4, 16, 96, 640),
+                                         (512, 1, 1, 32, 896), (170, 3, 5, 480, 1920)])
+@pytest.mark.parametrize("act,weight_input", [("clipped", False), ("silu", False), ("silu", True)])
+def test_decode_batches_read_an_expert_once(T, top, E, F, W, act, weight_input):
+    """Pairs of an expert that fill no tile of 16, one to four and more than four; identity experts, choices of none, an expert chosen twice;
+    depths of few steps, of all and of a number that is no multiple of a load group."""
+    from llm_in_practise_amd.ops._native import native_seq
+    assert native_seq().moe_few(T, top, E, F, W) and not native_seq().moe_few(T, top, E, F, 4096) and not native_seq().moe_few(513, top, E, F, W)
+    g = torch.Generator().manual_seed(T + F)
+    h = torch.randn(T, W, generator=g).bfloat16().cuda()
+    gu, dn = ((torch.randn(*s, generator=g) * s[-1] ** -0.5).bfloat16().cuda() for s in ((E, 2, F, W), (E, W, F)))
+    idx, w = torch.randint(-1, E + 2, (T, top), generator=g).int().cuda(), torch.rand(T, top, generator=g).cuda()
+    shared, sg = torch.randn(T, W, generator=g).bfloat16().cuda(), torch.randn(T, generator=g).cuda()
+    if weight_input:
+        idx = idx.clamp(max=E - 1)
+    for extra in ((None, None), (shared, None), (shared, sg)):
+        got = M.moe_glu_experts(h, gu, dn, idx, w, 7.0, extra[0], True, act=act, shared_gate=extra[1], weight_input=weight_input)
+        want = torch.zeros(T, W, dtype=torch.float64, device="cuda")
+        if extra[0] is not None:
+            want += shared.double() * (1.0 if extra[1] is None else torch.sigmoid(sg.double())[:, None])
+        for j in range(top):
+            for e in range(E + 2):
+                rows = (idx[:, j] == e).nonzero()[:, 0]
+                x, wt = h[rows].double(), w[rows, j, None].double()
+                if e < E:
+                    gate, up = (x @ gu[e, i].double().t() * (wt if weight_input else 1.0) for i in (0, 1))
+                    if act == "silu":
+                        a = torch.nn.functional.silu(gate) * up
+                    else:
+                        gate, up = gate.clamp(max=7.0), up.clamp(-7.0, 7.0)
+                        a = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
+                    x = a.float().bfloat16().double() @ dn[e].double().t()
+                want[rows] += x * (1.0 if weight_input else wt)
+        # float sums of up to 2048 products; of the activations one in a few thousand is rounded to the other bf16 neighbour, 2^-8 of it
+        assert ((got.double() - want).norm() / want.norm()).item() < 2e-4
