@@ -277,9 +277,14 @@ __global__ __launch_bounds__(64 * NW) void k_route_fused(const T* __restrict__ h
   for (int e = threadIdx.x; e < n; e += 64 * NW) sz[e] = (part[e][0] + part[e][1]) + (part[e][2] + part[e][3]);
   __syncthreads();
   for (int e = threadIdx.x; e < extra; e += 64 * NW) xout[(size_t)t * extra + e] = sz[n - extra + e];
-  if (wv == 0)
-    route_wave(sz, corr, idx + (size_t)t * (top + always), wout + (size_t)t * (top + always), lane, n - extra, top, groups,
-               keep, scale, kind, always);
+  if (wv > 0) return;
+  const size_t at = (size_t)t * (top + always);
+  if (n - extra <= 16 && top + always <= 16) {             // (the same choices and weights; a chain of moves inside a row of 16 lanes)
+    const float z[1] = {lane < n - extra ? sz[lane] : 0.f};
+    if (lane < 16) route_lanes<16, 1>(z, corr, idx + at, wout + at, lane, n - extra, top, groups, keep, scale, kind, always);
+  } else {
+    route_wave(sz, corr, idx + at, wout + at, lane, n - extra, top, groups, keep, scale, kind, always);
+  }
 }
 
 // The same for prompts and up to 16 outputs: a block takes four tokens, a wave a quarter of their columns, so that a router row
@@ -501,11 +506,14 @@ __global__ __launch_bounds__(256) void k_moe_pair_down(const T* __restrict__ a, 
 // token's outputs are added in the order of its choices.  Bound by latency: ids, rows and weights are one round trip each, two launches.
 constexpr int FEW = 512;                        // pairs
 
-// The pairs of expert e in their order, in a wave's own place in LDS; their number.
-__device__ __forceinline__ int list_pairs(const int* __restrict__ idx, int P, int e, int lane, unsigned short* list) {
-  int v[FEW / 64], n = 0;
+__device__ __forceinline__ void load_ids(const int* __restrict__ idx, int P, int lane, int (&v)[FEW / 64]) {
 #pragma unroll
   for (int i = 0; i < FEW / 64; ++i) v[i] = idx[min(64 * i + lane, P - 1)];
+  __builtin_amdgcn_sched_barrier(0);            // (in front of the weights: loads come back in order)
+}
+// The pairs of expert e in their order, in a wave's own place in LDS; their number.
+__device__ __forceinline__ int list_pairs(const int (&v)[FEW / 64], int P, int e, int lane, unsigned short* list) {
+  int n = 0;
 #pragma unroll
   for (int i = 0; i < FEW / 64; ++i) {
     const unsigned long long m = __ballot(64 * i + lane < P && v[i] == e);
@@ -550,9 +558,12 @@ __global__ __launch_bounds__(256, 1) void k_moe_few_up(const bf16* __restrict__ 
   const int steps = W / 128, k0 = w * (W / 4) + 8 * q;
   const bf16* wg = wgu + ((size_t)e * 2 * F + r0 + li) * W + k0;
   bf16x8 gate[S], up[S], x[2][S];
+  int ids[FEW / 64];
+  load_ids(idx, P, lane, ids);
   load_steps<S>(wg, steps, gate);
   load_steps<S>(wg + (size_t)F * W, steps, up);
-  const int n = list_pairs(idx, P, e, lane, list[w]);
+  __builtin_amdgcn_sched_barrier(0);
+  const int n = list_pairs(ids, P, e, lane, list[w]);
   for (int g0 = 0; g0 < n; g0 += 64)
     few_tiles(n - g0, [&](auto tiles) {
       constexpr int NT = decltype(tiles)::value;
@@ -600,10 +611,25 @@ __global__ __launch_bounds__(512) void k_moe_few_down(const bf16* __restrict__ a
   __shared__ unsigned short list[8][FEW];
   __shared__ __attribute__((aligned(16))) float y[FEW * LDY];
   const int c0 = blockIdx.x * 16, w = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, q = lane >> 4, P = T_ * top, steps = F / 32;
+  __shared__ int sid[FEW];
+  __shared__ float swt[FEW];
+  // a thread's first four outputs: what stands beside the experts' is on its way from here on
+  const int i0 = min((int)threadIdx.x, 4 * T_ - 1);
+  const int id0 = idx[min((int)threadIdx.x, P - 1)];
+  const float wt0 = wts != nullptr ? wts[min((int)threadIdx.x, P - 1)] : 1.f;
+  f32x4 beside = {0.f, 0.f, 0.f, 0.f};
+  if (shared != nullptr) beside = load4(shared + (size_t)(i0 >> 2) * W + c0 + 4 * (i0 & 3));
+  int ids[FEW / 64];
+  load_ids(idx, P, lane, ids);
+  if ((int)threadIdx.x < P) {
+    sid[threadIdx.x] = id0;
+    swt[threadIdx.x] = wt0;
+  }
   for (int e = w; e < E; e += 8) {
     bf16x8 rows[S], x[2][S];
     load_steps<S>(wd + ((size_t)e * W + c0 + li) * F + 8 * q, steps, rows);
-    const int n = list_pairs(idx, P, e, lane, list[w]);
+    __builtin_amdgcn_sched_barrier(0);
+    const int n = list_pairs(ids, P, e, lane, list[w]);
     for (int g0 = 0; g0 < n; g0 += 64)
       few_tiles(n - g0, [&](auto tiles) {
         constexpr int NT = decltype(tiles)::value;
@@ -624,10 +650,10 @@ __global__ __launch_bounds__(512) void k_moe_few_down(const bf16* __restrict__ a
   for (int i = threadIdx.x; i < 4 * T_; i += 512) {
     const int t = i >> 2, c = c0 + 4 * (i & 3);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (shared != nullptr) acc = load4(shared + (size_t)t * W + c) * (sgate != nullptr ? sigmoidf_(sgate[t]) : 1.f);
+    if (shared != nullptr) acc = (i < 512 ? beside : load4(shared + (size_t)t * W + c)) * (sgate != nullptr ? sigmoidf_(sgate[t]) : 1.f);
     for (int j = 0; j < top; ++j) {
-      const int p = t * top + j, e = idx[p];
-      const float wt = wts != nullptr ? wts[p] : 1.f;
+      const int p = t * top + j, e = sid[p];
+      const float wt = swt[p];
       if (e >= E)
         acc += load4(h + (size_t)t * ldh + c) * wt;
       else if (e >= 0)
@@ -778,14 +804,16 @@ void seq_route_fused(int code, const void* h, int ldh, const float* router, cons
 }
 
 // Where a decode batch's experts are read once: operands that 16-byte loads take, at most 2048 deep (512 the second products), pairs that LDS holds.
-// us of a step in a captured graph, routing included, a wave a (pair, row) -> here, 8 experts: width 2048, F 384, top 2, 12 / 16 / 32 / 48 / 128 pairs 22.9 ->
-// 23.7 (not taken), 25.7 -> 24.1 (not taken), 37 -> 24, 47 -> 25, 87 -> 29; width 1024, F 448, 16 / 32 / 128 pairs 18.1 -> 19.1 (not taken), 25 -> 20, 54 -> 23; F 512, top 4,
-// width 2048, 12 / 16 / 64 / 256 26.0 -> 27.1 (not taken), 29.9 -> 28.0, 62 -> 29, 150 -> 37; width 1024, 16 / 32 / 256 18.6 -> 20.8 (not taken), 25.4 -> 21.7, 91 -> 29.
+// us of a step in a captured graph, routing included (1.0 to 1.7 us shorter on both sides by now), a wave a (pair, row) -> here, 8 experts: width 2048, F
+// 384, top 2, 12 / 16 / 32 / 48 / 128 pairs 22.9 -> 23.7 (not taken), 25.7 -> 24.1, 37 -> 24, 47 -> 25, 87 -> 29; width 1024, F 448, 16 / 32 / 128 pairs 18.1 ->
+// 19.1 (not taken), 25 -> 20, 54 -> 23; F 512, top 4, width 2048, 12 / 16 / 64 / 256 26.0 -> 27.1 (not taken), 29.9 -> 28.0, 62 -> 29, 150 -> 37; width 1024, 16 / 24
+// / 32 / 256 18.6 -> 20.8 (not taken), 23.3 -> 21.5, 25.4 -> 21.7, 91 -> 29.  With the ids' loads in front of the weights', and what stands beside the experts'
+// outputs on its way from the start, half a us less.
 // More experts have fewer pairs each to share their rows.
 bool seq_moe_few(int code, const void* h, int ldh, const void* wgu, const void* wd, const void* shared, int T_, int top, int E, int F, int W) {
   const auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   const long P = (long)T_ * top;
-  return code == 0 && P <= FEW && P * F * W >= 14000000 && P >= 2 * E && E <= 16 && F % 32 == 0 && F <= 512 && W % 128 == 0 && W <= 2048 && ldh % 8 == 0 &&
+  return code == 0 && P <= FEW && P * F * W >= 12500000 && P >= 2 * E && E <= 16 && F % 32 == 0 && F <= 512 && W % 128 == 0 && W <= 2048 && ldh % 8 == 0 &&
          aligned(h) && aligned(wgu) && aligned(wd) && aligned(shared);
 }
 
