@@ -25,6 +25,7 @@
 using namespace lipa;
 
 size_t seq_walk_floats(int, int, int, int, int, int, size_t);
+bool seq_walk_short(int, int, int, int, int, int);
 void seq_walk(bool, const void*, int, const void*, int, const void*, int, const GateArgs&, float*, float*, float*, float*, float*, float*, float*, size_t,
               int, int, int, int, int, const SeqDesc&, hipStream_t);
 
@@ -766,7 +767,7 @@ void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* 
 // Floats of workspace of the chunked form, or 0 where the token-by-token scan is the one to run: float activations, key sizes
 // that are no multiple of 32 or above 128, rows that 16-byte (q, k, the states S and N) or 8-byte (v) loads cannot take, and steps of
 // few tokens a sequence.  At most `most`: longer steps run in windows.
-size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const void* S,
+size_t seq_chunk_floats(int code, bool mlstm, const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const void* S,
                         const void* N, int T_, int B, int H, int dk, int dv, int longest, size_t most) {
   const auto fits = [](const void* p, int ld, int n) { return ld % n == 0 && ((uintptr_t)p & (2 * n - 1)) == 0; };
   if (code != 0 || dk % 32 != 0 || dk > 128 || dv % 4 != 0 || (long)H * dv >= 1l << 22 || std::max({ldq, ldk, ldv}) >= 1 << 22 ||
@@ -784,7 +785,8 @@ size_t seq_chunk_floats(int code, const void* q, int ldq, const void* k, int ldk
   if (pairs >= 256 && dk <= 64 && dv >= 128) least = std::max(least, 96l);
   if (pairs >= 1024 && (dk <= 64 || dv <= 32)) least = 192;
   if (pairs * dv >= 1l << 17 && dk <= 32) least = 256;
-  if (B == 0 || T_ < least * B) return 0;
+  if (B == 0) return 0;
+  if (T_ < least * B) return mlstm && seq_walk_short(T_, B, H, dk, dv, longest) ? seq_walk_floats(T_, B, H, dk, dv, longest, most) : 0;
   if (const size_t n = seq_walk_floats(T_, B, H, dk, dv, longest, most)) return n;      // (the state never leaves its block)
   const int sc = run_chunks(T_, B, H, dv);
   const size_t slots = run_plan(T_, B, H, dk, dv, sc, most).slots;

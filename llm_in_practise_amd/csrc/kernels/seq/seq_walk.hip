@@ -604,7 +604,7 @@ PiecePlan walk_plan(int T_, int B, int H, size_t most) { return plan_pieces(T_, 
 // space, 64 heads of 128 x 64: 512 34 -> 19, 4 x 512 63 -> 45, 8 x 1024 172 -> 143, 2 x 4096 162 -> 129, one of 4093 91 -> 92, of 9000 188 -> 186; 32
 // heads: 1000 33 -> 27, 12 x 700 108 -> 83, one of 4093 61 -> 89.  More columns a block: fewer blocks for the scores and splits, but longer turns (8 x 1024
 // of 128 x 192 with 16 / 32 / 48 columns 78 / 70 / 52, one prompt of 512 21 / 25 / 29; 8 x 512 of 64 x 96 25 / 21 / 24).
-int walk_tiles(int T_, int B, int H, int dk, int dv, int longest) {
+int walk_tiles(int T_, int B, int H, int dk, int dv, int longest, float* takes = nullptr) {
   if ((dk != 64 && dk != 128) || B == 0) return 0;
   constexpr float TURN_US[2][4] = {{2.1f, 2.9f, 3.5f, 4.4f}, {2.8f, 3.8f, 4.9f, 0.f}};
   const long pairs = (long)B * H, tiles = (dv + 15) / 16;
@@ -621,6 +621,7 @@ int walk_tiles(int T_, int B, int H, int dk, int dv, int longest) {
       nt = t;
     }
   }
+  if (takes != nullptr) *takes = best;
   return nt;
 }
 
@@ -662,6 +663,19 @@ void dispatch(const bf16* q, int ldq, const bf16* k, int ldk, const bf16* v, int
 }  // namespace
 
 int seq_walk_tiles(int T_, int B, int H, int dk, int dv, int longest) { return walk_tiles(T_, B, H, dk, dv, longest); }
+
+// Whether an mLSTM's prompts too short for chunks walk their tokens here and not one by one (lengths that are known).  That form takes 7 us and 0.38 a
+// token of the longest sequence (keys of 64: 5.5 and 0.3), or 0.14 ps a token, key channel and column where they fill the chip.  us, token by token ->
+// here: 8 heads of 128 x 192, one prompt of 12 / 16 / 20 / 32 / 63 tokens 13 (not taken), 13 -> 13, 17 -> 13, 20 -> 13, 34 -> 13, 8 of 20 / 40 / 63 19 -> 14, 27 -> 14, 37 ->
+// 15, 12 of 20 / 63 21 (not taken), 44 -> 21, 32 of 63 113 -> 36; of 64 x 96, 8 of 24 / 63 16 -> 13, 31 -> 13; 32 heads of 64 x 96, 32 prompts of 24 41 (53 here:
+// not taken).  Error against 64 bits of 20 to 63 tokens 1.6 to 2.6e-7 -> 0.9 to 1.4e-7.  (The state space would gain as much, 13 -> 11 us at 20 tokens, 30 -> 11 at
+// 63, but its outputs' error is 0.4e-7 token by token and 0.6 here.)
+bool seq_walk_short(int T_, int B, int H, int dk, int dv, int longest) {
+  float us = 0.f;
+  if (longest <= 0 || longest > T_ || walk_tiles(T_, B, H, dk, dv, longest, &us) == 0) return false;
+  const float full = 0.14e-6f * ((float)B * H * dv * dk) * T_ / B, chain = (dk == 64 ? 0.3f : 0.38f) * longest;
+  return us < 0.97f * ((dk == 64 ? 5.5f : 7.f) + std::max(chain, full));
+}
 
 // Floats of workspace for at most `most` (longer steps run in windows), or 0 where the state in chunks (seq_chunk.hip) is to run.  longest: tokens of
 // the longest sequence, 0 where the caller does not know.

@@ -105,7 +105,7 @@ void seq_delta_scan(int, const void*, int, const void*, int, const void*, int, c
 void seq_talk_attention(int, const void*, int, const void*, const void*, float*, float*, float*, const float*,
                         const void*, int, void*, int, int, int, int, int, int, float, const int*, const int*, int,
                         SeqDesc, hipStream_t);
-size_t seq_chunk_floats(int, const void*, int, const void*, int, const void*, int, const void*, const void*, int, int, int, int, int, int,
+size_t seq_chunk_floats(int, bool, const void*, int, const void*, int, const void*, int, const void*, const void*, int, int, int, int, int, int,
                         size_t);
 int seq_walk_tiles(int, int, int, int, int, int);
 void seq_chunk_ssd(const void*, int, const void*, int, const void*, int, const void*, int, const float*, const float*,
@@ -362,7 +362,7 @@ std::vector<Tensor> mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor ipre, Tensor
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H, dv}, S.options());
   auto den = at::empty({T, H}, S.options()), efl = at::empty({T, H}, S.options());
-  if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), S.data_ptr(),
+  if (const size_t n = seq_chunk_floats(code, true, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), S.data_ptr(),
                                         N.data_ptr(), (int)T, d.B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_chunk_mlstm(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), ipre.data_ptr<float>(),
@@ -479,7 +479,7 @@ Tensor ssd_scan(Tensor q, Tensor k, Tensor v, Tensor dtraw, Tensor dt_bias, Tens
   check_state(S, H, dv, dk);
   SeqDesc d = desc_of(desc, live, T);
   auto out = at::empty({T, H * dv}, S.options());
-  if (const size_t n = seq_chunk_floats(code, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), S.data_ptr(), nullptr,
+  if (const size_t n = seq_chunk_floats(code, false, q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), S.data_ptr(), nullptr,
                                         (int)T, d.B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most)) {
     auto ws = at::empty({(int64_t)n}, S.options());
     seq_chunk_ssd(q.data_ptr(), ld(q), k.data_ptr(), ld(k), v.data_ptr(), ld(v), dtraw.data_ptr(), ld(dtraw),
@@ -1333,17 +1333,17 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   // workspace of a step through the chunked ("ssd", "mlstm") or blocked ("delta", "gla") form, bf16 rows that its loads take; 0: token by token
   m.def("scan_floats", [](const std::string& op, int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most, int64_t longest) {
     if (op == "ssd" || op == "mlstm")
-      return (int64_t)seq_chunk_floats(0, nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most);
+      return (int64_t)seq_chunk_floats(0, op == "mlstm", nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)most);
     TORCH_CHECK(op == "delta" || op == "gla", "scan_floats: ssd, mlstm, delta or gla");
     return (int64_t)seq_block_floats(0, op == "delta", nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H,
                                      (int)dk, (int)dv, (int)longest, (size_t)most);
   }, py::arg("op"), py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("most") = MOST_WS, py::arg("longest") = 0);
   // columns of a block that walks the tokens with the state at hand ("ssd", "mlstm"), 0: chunks, or token by token
-  m.def("scan_walk", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t longest) {
-    if (seq_chunk_floats(0, nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)MOST_WS) == 0)
+  m.def("scan_walk", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t longest, const std::string& op) {
+    if (seq_chunk_floats(0, op == "mlstm", nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)MOST_WS) == 0)
       return 0;
     return 16 * seq_walk_tiles((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest);
-  });
+  }, py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("longest"), py::arg("op") = "ssd");
   m.def("delta_block", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most) {      // tokens of a block, 0: token by token
     if (seq_block_floats(0, true, nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, 0, (size_t)most) == 0) return 0;
     return seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, 0, (size_t)most) > 0 ? 32 : 16;

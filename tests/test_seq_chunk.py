@@ -822,6 +822,44 @@ def test_walk_with_the_state_at_hand(op, lens, H, dk, dv, cols, bad, whole):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,B,H,dk,dv,longest,walks", [
+    (12, 1, 8, 128, 192, 12, False), (20, 1, 8, 128, 192, 20, True), (63, 1, 8, 128, 192, 0, False), (160, 8, 8, 128, 192, 20, True),
+    (240, 12, 8, 128, 192, 20, False), (756, 12, 8, 128, 192, 63, True), (768, 32, 32, 64, 96, 24, False), (192, 8, 8, 64, 96, 24, True),
+    (63, 1, 8, 96, 96, 63, False)])
+def test_short_mlstm_prompts_walk_where_it_is_not_slower(T, B, H, dk, dv, longest, walks):
+    """Timed shapes on both sides of the choice between the walk and tokens one by one; lengths that are not known, keys that have no walk; and
+    the state space, which has none of it."""
+    from llm_in_practise_amd.ops._native import native_seq
+    ext = native_seq()
+    assert (ext.scan_walk(T, B, H, dk, dv, longest, "mlstm") > 0) == (ext.scan_floats("mlstm", T, B, H, dk, dv, longest=longest) > 0) == walks
+    assert ext.scan_walk(T, B, H, dk, dv, longest) == ext.scan_floats("ssd", T, B, H, dk, dv, longest=longest) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,H,dk,dv", [([20], 2, 128, 192), ([63], 3, 64, 96), ([48, 1, 30, 17, 63], 4, 128, 64), ([40, 33], 2, 64, 36)])
+def test_short_mlstm_prompts_walk_as_token_by_token(lens, H, dk, dv):
+    from llm_in_practise_amd.ops._native import native_seq
+    ext = native_seq()
+    g = torch.Generator().manual_seed(dk + dv)
+    T, B, longest = sum(lens), len(lens), max(lens)
+    assert ext.scan_walk(T, B, H, dk, dv, longest, "mlstm") > 0
+
+    def rand(*s, dt=torch.float32):
+        return torch.randn(*s, generator=g).to(dt).cuda()
+    q, k, v = (rand(T, H * n, dt=torch.bfloat16) for n in (dk, dk, dv))
+    i, f, a, b = 3 * rand(T, H), 3 * rand(T, H), rand(H), rand(H)
+    S0, N0, res = rand(B, H, dv, dk), rand(B, H, dk), []
+    for most in (1 << 28, 0):                             # (no room: token by token)
+        st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lens, [7 * (j % 2) for j in range(B)], "cuda")
+        st["S"].copy_(S0)
+        st["N"].copy_(N0)
+        st["M"].fill_(0.5)
+        out = ext.mlstm_scan(q, k, v, i, f, a, b + 3, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb.desc, sb.live, most=most, longest=longest)
+        res.append([*out, st["S"], st["N"], st["M"]])
+    _close(res[0], res[1], ("o", "den", "floor", "S", "N", "M"))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,B,H,dk,dv,longest,cols", [
     (4093, 1, 64, 128, 64, 4093, 0), (1000, 1, 64, 128, 64, 1000, 16), (2000, 4, 64, 128, 64, 512, 32), (7040, 8, 8, 128, 192, 1024, 48),
     (512, 1, 8, 64, 96, 512, 16), (2048, 1, 8, 64, 96, 2048, 0), (4096, 8, 8, 64, 96, 512, 32), (9060, 12, 8, 64, 96, 9000 - 640, 0),
