@@ -1,4 +1,4 @@
-// Generation-time kernels (SURVEY.md K16, K17): KV-cache decode attention and the fused
+// Generation-time kernels: KV-cache decode attention and the fused
 // logits → token sampler.
 //
 // decode attention ("flash-decoding" on CDNA4): one query token per sequence against its

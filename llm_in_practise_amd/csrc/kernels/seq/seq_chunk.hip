@@ -12,7 +12,8 @@
 // decays are summed in 64 bits and kept as two floats, so that the difference of two large sums is exact.
 //
 // Measured, token by token -> chunks: state space, one prompt of 4093 tokens, 64 heads of 128 x 64: 2350 -> 92 us (state 32, walk 9,
-// outputs 50); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 80 us (25, 11, 43).  Error against 64 bits
+// outputs 50); mLSTM, 8 prompts of 333 to 1024 tokens, 8 heads of 128 x 192: 649 -> 80 us (25, 11, 43;
+// they now walk in 50, seq_walk.hip).  Error against 64 bits
 // 1.6e-7 -> 0.9e-7 and 4.4e-7 -> 1.9e-7: fewer roundings stand between a token and the outputs far behind it.
 // The first case reads and writes 335 MB, 235 of them states and outputs, of which a copy moves 5 TB/s.  With every chunk's contribution
 // walked by itself (69 MB of states out, in, out and in), operands of the outputs loaded from memory rows as they are needed, an
