@@ -208,7 +208,9 @@ __device__ __forceinline__ int quotient(int a, int b) {
   q += (q + 1) * b <= a;
   return q;
 }
-__device__ __forceinline__ int split_chunk32(int len, int nsplit, int least) { return (max(quotient(len + nsplit - 1, nsplit), least) + 31) & ~31; }
+__device__ __forceinline__ int split_chunk32(int len, int nsplit) { return (max(quotient(len + nsplit - 1, nsplit), 1) + 31) & ~31; }
+// Splits of one tile or two that a workgroup takes side by side, a wave a tile
+__device__ __forceinline__ int splits_held(int chunk) { return chunk == 32 ? 4 : chunk == 64 ? 2 : 1; }
 template <int CTRL, int ROWS>
 __device__ __forceinline__ int plus_dpp(int v) { return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false); }
 __device__ __forceinline__ int scan64(int v) {               // sum over the lanes up to this one
@@ -219,23 +221,23 @@ __device__ __forceinline__ int scan64(int v) {               // sum over the lan
   v = plus_dpp<0x142, 0xA>(v);                               // row_bcast 15 into the rows 1 and 3, 31 into 2 and 3
   return plus_dpp<0x143, 0xC>(v);
 }
-// Item `id` of all (row, kv head, split of its keys) that hold keys: rows one after the other, of each the heads, of each the splits.  False past
-// the last one.  (Counted over the rows' lengths, 64 of them at a time; what a wave holds once is read into scalar registers, or every
+// Item `id` of all (row, kv head, the splits of its keys that a workgroup takes) that hold keys: rows one after the other, of each the heads, of each
+// the splits.  False past the last one.  (Counted over the rows' lengths, 64 of them at a time; what a wave holds once is read into scalar registers, or every
 // address behind it is a lane's own: 15.6 -> 17.7 us for 12 rows.)
 struct SplitItem {
-  int b, kh, split, len, chunk;
+  int b, kh, split, held, len, chunk;
 };
-__device__ __forceinline__ bool find_split(const int64_t* __restrict__ pos, int B, int hkv, int nsplit, int least, int id, SplitItem& it) {
-  if (B == 1) {                                              // (a grid of splits and heads)
-    it = {0, (int)blockIdx.y, (int)blockIdx.x, (int)pos[0] + 1, 0};
-    it.chunk = __builtin_amdgcn_readfirstlane(split_chunk32(it.len, nsplit, least));
+__device__ __forceinline__ bool find_split(const int64_t* __restrict__ pos, int B, int hkv, int nsplit, bool counted, int id, SplitItem& it) {
+  if (!counted) {                                            // (a grid of splits, heads and rows)
+    it = {(int)blockIdx.z, (int)blockIdx.y, (int)blockIdx.x, 1, (int)pos[blockIdx.z] + 1, 0};
+    it.chunk = __builtin_amdgcn_readfirstlane(split_chunk32(it.len, nsplit));
     return it.split * it.chunk < it.len;
   }
   int before = 0;
   for (int b0 = 0; b0 < B; b0 += 64) {
     const int lane = threadIdx.x & 63;
-    const int len = b0 + lane < B ? max((int)pos[b0 + lane] + 1, 0) : 0, chunk = split_chunk32(len, nsplit, least);
-    const int n = quotient(len + chunk - 1, chunk);
+    const int len = b0 + lane < B ? max((int)pos[b0 + lane] + 1, 0) : 0, chunk = split_chunk32(len, nsplit);
+    const int keys = chunk * splits_held(chunk), n = quotient(len + keys - 1, keys);
     const int sum = before + scan64(n * hkv);
     const unsigned long long m = __ballot(sum > id);
     if (m) {
@@ -245,7 +247,8 @@ __device__ __forceinline__ bool find_split(const int64_t* __restrict__ pos, int 
       it.len = __builtin_amdgcn_readlane(len, at);
       it.chunk = __builtin_amdgcn_readlane(chunk, at);
       it.kh = __builtin_amdgcn_readfirstlane(quotient(local, each));
-      it.split = local - it.kh * each;
+      it.held = splits_held(it.chunk);
+      it.split = (local - it.kh * each) * it.held;
       return true;
     }
     before = __builtin_amdgcn_readlane(sum, 63);
@@ -265,7 +268,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
                                                           bf16* __restrict__ kc, bf16* __restrict__ vc,
                                                           const int64_t* __restrict__ pos, float* __restrict__ opart,
                                                           float* __restrict__ mpart, float* __restrict__ lpart,
-                                                          int Smax, int B, int hq, int hkv, int nsplit, int least, float scale_log2) {
+                                                          int Smax, int B, int hq, int hkv, int nsplit, bool counted, float scale_log2) {
   constexpr int LDR = D + 8;          // padded LDS row (elements)
   constexpr int CH = D / 8;           // 16-B chunks per row
   constexpr int NS = D / 32;          // k-steps over the head dim
@@ -279,9 +282,9 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
   asm volatile("" ::"s"(q), "s"(knew), "s"(vnew), "s"(kc), "s"(vc), "s"(ldq), "s"(ldkn), "s"(ldvn));   // (all at once, not behind the length)
   const int G = hq / hkv;
   SplitItem it;
-  if (!find_split(pos, B, hkv, nsplit, least, blockIdx.x, it)) return;
-  const int split = it.split, kh = it.kh, b = it.b, len = it.len, chunk = it.chunk;
-  const int k0 = split * chunk, k1 = min(k0 + chunk, len);
+  if (!find_split(pos, B, hkv, nsplit, counted, blockIdx.x, it)) return;
+  const int split = it.split, held = it.held, kh = it.kh, b = it.b, len = it.len, chunk = it.chunk;
+  const int k0 = split * chunk, k1 = min(k0 + held * chunk, len);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, li = lane & 15;
 
   const size_t rs = (size_t)hkv * D;
@@ -395,22 +398,41 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_k(const bf16* __restrict
 #pragma unroll
     for (int r = 0; r < 4; ++r) sacc[(w * 16 + li) * D + 16 * dt + 4 * g + r] = acc[dt][r];
   __syncthreads();
-  for (int i = threadIdx.x; i < G * D; i += 256) {
-    const int hh = i / D, d = i % D;
-    const float M = fmaxf(fmaxf(sm[0][hh], sm[1][hh]), fmaxf(sm[2][hh], sm[3][hh]));
-    float L = 0.f, A = 0.f;
-#pragma unroll
-    for (int s2 = 0; s2 < 4; ++s2) {
-      const float c = __builtin_amdgcn_exp2f(sm[s2][hh] - M);   // -inf (idle wave) → 0
-      // (products are rounded before they are summed: a step's bits do not depend on what the compiler fuses)
-      L += rounded(sl[s2][hh] * c);
-      A += rounded(sacc[(s2 * 16 + hh) * D + d] * c);
-    }
+  const auto leave = [&](int hh, int d, int split, float M, float L, float A) {
     const size_t hrow = ((size_t)b * hq + kh * G + hh) * nsplit + split;
     opart[hrow * D + d] = A;
     if (d == 0) {
       mpart[hrow] = M * 0.6931471805599453f;
       lpart[hrow] = L;
+    }
+  };
+  // (-inf of an idle wave: a weight of 0; products are rounded before they are summed: a step's bits do not depend on what the compiler fuses)
+  if (held == 1) {
+    for (int i = threadIdx.x; i < G * D; i += 256) {
+      const int hh = i / D, d = i % D;
+      const float M = fmaxf(fmaxf(sm[0][hh], sm[1][hh]), fmaxf(sm[2][hh], sm[3][hh]));
+      float L = 0.f, A = 0.f;
+#pragma unroll
+      for (int s2 = 0; s2 < 4; ++s2) {
+        const float c = __builtin_amdgcn_exp2f(sm[s2][hh] - M);
+        L += rounded(sl[s2][hh] * c);
+        A += rounded(sacc[(s2 * 16 + hh) * D + d] * c);
+      }
+      leave(hh, d, split, M, L, A);
+    }
+  } else if (chunk == 32) {                                  // a wave a split
+    for (int i = threadIdx.x; i < held * G * D; i += 256) {
+      const int j = i / (G * D), hh = i / D - j * G, d = i % D;
+      if (k0 + 32 * j < len) leave(hh, d, split + j, sm[j][hh], sl[j][hh], sacc[(j * 16 + hh) * D + d]);
+    }
+  } else {                                                   // two
+    for (int i = threadIdx.x; i < 2 * G * D; i += 256) {
+      const int j = i >= G * D, hh = i / D - j * G, d = i % D;
+      const float ma = sm[2 * j][hh], mb = sm[2 * j + 1][hh], M = fmaxf(ma, mb);
+      const float ca = __builtin_amdgcn_exp2f(ma - M), cb = __builtin_amdgcn_exp2f(mb - M);
+      const float L = rounded(sl[2 * j][hh] * ca) + rounded(sl[2 * j + 1][hh] * cb);
+      const float A = rounded(sacc[(2 * j * 16 + hh) * D + d] * ca) + rounded(sacc[((2 * j + 1) * 16 + hh) * D + d] * cb);
+      if (k0 + 64 * j < len) leave(hh, d, split + j, M, L, A);
     }
   }
 }
@@ -424,7 +446,7 @@ __global__ __launch_bounds__(D) void decode_attn_merge2_k(const float* __restric
                                                           const float* __restrict__ mpart,
                                                           const float* __restrict__ lpart,
                                                           const int64_t* __restrict__ pos, bf16* __restrict__ out,
-                                                          int hq, int nsplit, int least) {
+                                                          int hq, int nsplit) {
   extern __shared__ __attribute__((aligned(16))) float sc[];   // weight of each split, then its sum
   __shared__ float scratch[D / 64];
   const size_t h = blockIdx.x;  // b*hq + head
@@ -435,7 +457,7 @@ __global__ __launch_bounds__(D) void decode_attn_merge2_k(const float* __restric
   for (int j = 0; j < NP; ++j) v[j] = op[(size_t)min(j, nsplit - 1) * D];
   const float m0 = mpart[h * nsplit + min(d, nsplit - 1)], l0 = lpart[h * nsplit + min(d, nsplit - 1)];
   const int len = (int)pos[h / hq] + 1;
-  const int chunk = split_chunk32(len, nsplit, least);
+  const int chunk = split_chunk32(len, nsplit);
   const int nv = min(nsplit, (len + chunk - 1) / chunk);
   float m = d < nv ? m0 : -INFINITY;
   for (int s = d + D; s < nv; s += D) m = fmaxf(m, mpart[h * nsplit + s]);
@@ -635,18 +657,6 @@ void launch_decode_attention(const void* q, const void* kc, const void* vc, cons
 }
 
 
-// Fewest keys of a split.  The number of splits stands when a step is captured, for rows of any length; cut that finely a short row's
-// splits leave two or three of a workgroup's four waves idle and are more workgroups than the chip holds.  By rows x kv heads (the row's own
-// length and these alone decide how it is cut, not its neighbours').  µs, both launches, heads of 128, 32 query on 8, from memory, splits as
-// captured with the empty ones launched between the others -> at least 64 / 128 / 256 keys, the empty ones last: 12 rows of 474 to 1400 keys
-// 20.5 -> 20.1 / 15.6 / 18.2; 6 of 120 to 300 11.0 -> 8.9 / 9.5 / 11.6; 20 of 33 to 100 12.1 -> 9.5 / 9.8 / 9.8, of 644 to 1900 29.8 -> 30.4 / 29.6 /
-// 29.3; 32 of 314 to 1000 28.1 -> 27.2 / 25.1 / 27.2; 48 of 125 to 400 24.3 -> 23.0 / 20.2 / 22.3; 64 of 688 to 1700 68.8 -> 69.8 / 69.7 / 67.7, of 80 to 200
-// 23.1 -> 20.3 / 18.4 / 17.3.  One row of 937 keeps 32: 8.3, and 8.3 / 9.0 / 11.2.
-int split_least(int B, int hkv) {
-  const int pairs = B * hkv;
-  return B == 1 ? 32 : pairs < 64 ? 64 : pairs < 512 ? 128 : 256;
-}
-
 // v2: MFMA split-K decode attention with the KV append fused (see decode_attn_mfma_k)
 int decode_split_plan2(int B, int hkv, int max_len) {
   const int pairs = std::max(1, B * hkv);
@@ -654,17 +664,24 @@ int decode_split_plan2(int B, int hkv, int max_len) {
   return std::min(ns, std::max(1, (max_len + 127) / 128));
 }
 
+// The number of splits stands when a step is captured, for rows of any length.  Cut that finely a short row's splits have one tile of 32 keys or
+// two, which leaves two or three of a workgroup's four waves idle, and are more workgroups than the chip holds: from 64 rows x kv heads on, a workgroup takes
+// four splits of one tile or two of two tiles, adds each of them up by itself in the order it has alone (the bits stay), and the empty ones are numbered last.
+// µs, both launches, heads of 128, 32 query on 8, from memory, a workgroup a split with the empty ones between the others -> here: 12 rows of 474 to 1400 keys 20.5 -> 17.5; 20 of
+// 33 to 100 12.1 -> 10.8, of 644 to 1900 29.4 -> 29.6; 32 of 314 to 1000 27.8 -> 25.4; 48 of 125 to 400 24.2 -> 21.2; 64 of 688 to 1700 68.8 -> 69.2, of 80 to 200 22.8 ->
+// 18.8.  Below, CUs are idle and a workgroup's own work counts: 4 rows of 562 to 1400 11.7 -> 12.3 (not taken).  Fewer and longer splits (12 rows 15.7) add in another
+// order, which an 8B model's logits show by 0.03, as much as their own rounding error.
 void launch_decode_attention2(const void* q, int ldq, const void* knew, int ldkn, const void* vnew, int ldvn, void* kc,
                               void* vc, const int64_t* pos, float* opart, float* mpart, float* lpart, void* out, int B,
                               int Smax, int hq, int hkv, int d, int nsplit, float scale, hipStream_t st) {
-  const dim3 grid = B == 1 ? dim3(nsplit, hkv) : dim3(nsplit * hkv * B);
-  const int least = split_least(B, hkv);
+  const bool counted = B * hkv >= 64;
+  const dim3 grid = counted ? dim3(nsplit * hkv * B) : dim3(nsplit, hkv, B);
   const float sl2 = scale * 1.4426950408889634f;
 #define M(D_, NP_) \
-  decode_attn_merge2_k<D_, NP_><<<B * hq, D_, 2 * (std::max(nsplit, NP_) + 3 & ~3) * sizeof(float), st>>>(opart, mpart, lpart, pos, (bf16*)out, hq, nsplit, least)
+  decode_attn_merge2_k<D_, NP_><<<B * hq, D_, 2 * (std::max(nsplit, NP_) + 3 & ~3) * sizeof(float), st>>>(opart, mpart, lpart, pos, (bf16*)out, hq, nsplit)
 #define P(D_)                                                                                                          \
   decode_attn_mfma_k<D_><<<grid, 256, 0, st>>>((const bf16*)q, ldq, (const bf16*)knew, ldkn, (const bf16*)vnew, ldvn, \
-                                               (bf16*)kc, (bf16*)vc, pos, opart, mpart, lpart, Smax, B, hq, hkv, nsplit, least, \
+                                               (bf16*)kc, (bf16*)vc, pos, opart, mpart, lpart, Smax, B, hq, hkv, nsplit, counted, \
                                                sl2);                                                                   \
   if (nsplit > 16) M(D_, 32); else if (nsplit > 8) M(D_, 16); else if (nsplit > 4) M(D_, 8); else M(D_, 4)
   if (d == 128) { P(128); } else { P(64); }

@@ -147,8 +147,8 @@ def test_decode_attention_append_merge(native_ext, max_len, d):
 @pytest.mark.parametrize("hkv,d", [(1, 128), (3, 64), (8, 128)])
 @pytest.mark.parametrize("B", [2, 20, 63, 64, 65, 130])
 def test_decode_attention_append_counts_the_splits_that_have_keys(native_ext, B, hkv, d):
-    """Rows whose keys end at, behind and in front of a shortest split (64, 128, 256), in batches on both sides of 64 rows and of each
-    shortest split; a row's bits are the same among other neighbours."""
+    """Rows whose keys end at, behind and in front of tiles and of the splits of one, two and more tiles that a workgroup takes four, two and one of, in
+    batches on both sides of 64 rows and of 64 rows x heads; a row's bits are the same among other neighbours."""
     torch.manual_seed(B + hkv)
     hq, max_len = 2 * hkv, 700
     ends = [0, 62, 63, 64, 126, 127, 128, 254, 255, 256, 699, 511, 512]
