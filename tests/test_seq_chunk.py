@@ -395,6 +395,32 @@ def test_parts_find_room_beside_the_blocks(op, dk):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("op,T,dk,most", [("delta", 6000, 64, 262144), ("delta", 3200, 128, 262144), ("gla", 6000, 64, 131072)])
+def test_parts_without_room_for_the_blocks(op, T, dk, most):
+    """Room for what the parts leave, but for no plan of the blocks they are made of: the step runs as it does with lengths that are not known."""
+    from llm_in_practise_amd.ops._native import native_seq
+    ext, H, dv, lens = native_seq(), 1, 16, [T - 120, 40, 40, 40]
+    floats = ext.scan_floats(op, T, 4, H, dk, dv, most=most)
+    assert ext.scan_parts(op, T, 4, H, dk, dv, longest=lens[0]) > 0 == ext.scan_parts(op, T, 4, H, dk, dv, longest=lens[0], most=most)
+    assert ext.scan_floats(op, T, 4, H, dk, dv, most=most, longest=lens[0]) == floats <= most
+    g = torch.Generator().manual_seed(T + dk)
+    P = torch.nn.functional.normalize(torch.randn(T, 2, dk, generator=g), dim=-1).flatten(1).bfloat16().cuda()
+    v, z, beta = torch.randn(T, dv, generator=g).bfloat16().cuda(), torch.rand(T, dk, generator=g).cuda() ** 0.02, torch.randn(T, H, generator=g).cuda()
+    zb, res = torch.zeros(dk, device="cuda"), []
+    for longest in (0, lens[0]):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, [0] * 4, "cuda")
+        st["S"].zero_()
+        if op == "delta":
+            o = ext.delta_scan(P[:, :dk], P[:, dk:], v, z, beta, st["S"], H, 1, sb.desc, sb.live, longest=longest, most=most)
+        else:
+            o = ext.gated_linear_scan(P[:, :dk], P[:, dk:], v, z, zb, 16.0, 1.0, st["S"], H, sb.desc, sb.live, longest=longest, most=most)
+        res.append((o, st["S"]))
+    assert torch.isfinite(res[0][0]).all() and res[0][0].abs().max() > 0
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("L,B,H,dk,dv,long", [
     (1000, 1, 8, 128, 128, True), (200, 1, 8, 128, 128, False), (300, 5, 6, 128, 128, True), (299, 5, 6, 128, 128, False),
     (2000, 4, 8, 128, 128, True), (2000, 5, 8, 128, 128, False), (400, 20, 16, 128, 64, True), (400, 20, 16, 128, 68, False),
