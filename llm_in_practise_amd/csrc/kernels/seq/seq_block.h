@@ -26,6 +26,8 @@ enum { WHOLE, ENDS, PARTS };
 
 // Part `id` of all that run, without a sequence's last one for `ends`; place: the sequence's first place.  (Counted, not bounded as the
 // pieces are: blocks of threads that find nothing to do leave others side by side on one CU, 84 us for 45.)
+// Parts and places are counted in the halves of an int: MOST_PARTS at most, T / len + B.
+constexpr int MOST_PARTS = (1 << 15) - 1;
 struct Part {
   int s, idx, place, t0, t1, end;
 };

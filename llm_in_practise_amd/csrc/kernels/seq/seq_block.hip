@@ -429,7 +429,8 @@ BlockPlan block_plan(bool delta, int T_, int B, int H, int dk, int dv, int longe
   if (delta || r.p.slots == 0 || r.p.count != 0) return r;
   if (const int blocks = part_blocks(T_, B, H, dk, dv, longest)) {
     const size_t more = (size_t)T_ / (blocks * BT) * H * part_floats(dk, dv);
-    if (r.floats + more <= most) r.blocks = blocks, r.floats += more;
+    // (16 parts of a sequence at most where none is longer than `longest`, which a caller may have wrong)
+    if (T_ / (blocks * BT) + B <= MOST_PARTS && r.floats + more <= most) r.blocks = blocks, r.floats += more;
   }
   return r;
 }

@@ -595,7 +595,7 @@ DeltaPlan plan_of(int T_, int B, int H, int dk, int dv, int longest, size_t most
   DeltaPlan r = {delta_plan(T_, B, H, dk, dv, most), 0, 0};
   r.floats = r.p.slots * slot_floats(H, dk, dv);
   if (r.p.slots == 0 || r.p.count != 0) return r;
-  if (const int blocks = part_blocks(T_, B, H, dk, dv, longest)) {
+  if (const int blocks = part_blocks(T_, B, H, dk, dv, longest)) {      // (6 blocks or more of 65535: no more than MOST_PARTS)
     const size_t more = (size_t)T_ / (blocks * LEN) * H * part_floats(dk, dv);
     if (r.floats + more <= most) r.blocks = blocks, r.floats += more;
   }

@@ -395,6 +395,22 @@ def test_parts_find_room_beside_the_blocks(op, dk):
 
 
 @pytest.mark.gpu
+def test_parts_that_can_be_counted():
+    """Parts are counted in 16 bits: a step that would have more, which takes a longest sequence that is not the longest, has none."""
+    from llm_in_practise_amd.ops._native import native_seq
+    ext = native_seq()
+    part = 16 * ext.scan_parts("gla", 1000, 1, 1, 64, 16, longest=1000)
+    assert part > 0
+    for T, parts in ((32766 * part, True), (32767 * part, False), (40000 * part, False), (65537 * part, False)):
+        floats = ext.scan_floats("gla", T, 1, 1, 64, 16, most=1 << 40)
+        assert (ext.scan_parts("gla", T, 1, 1, 64, 16, longest=1000, most=1 << 40) > 0) == parts
+        assert (ext.scan_floats("gla", T, 1, 1, 64, 16, most=1 << 40, longest=1000) > floats) == parts
+    # keys of the delta rule: what a plan holds is no more, whatever the caller says
+    assert ext.scan_parts("delta", 2_000_000, 1, 1, 64, 16, longest=1000, most=1 << 40) > 0
+    assert ext.scan_parts("delta", 2_100_000, 1, 1, 64, 16, longest=1000, most=1 << 40) == 0
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("op,T,dk,most", [("delta", 6000, 64, 262144), ("delta", 3200, 128, 262144), ("gla", 6000, 64, 131072)])
 def test_parts_without_room_for_the_blocks(op, T, dk, most):
     """Room for what the parts leave, but for no plan of the blocks they are made of: the step runs as it does with lengths that are not known."""
