@@ -593,8 +593,17 @@ __global__ __launch_bounds__(512, 2) void k_walk(const bf16* __restrict__ q, int
   walk_tiles(std::false_type{});
 }
 
-// floats of a piece's slot, for the larger of the two tables; 0.4 us a token in the token-by-token form
-size_t slot_floats(int H) { return (size_t)H * (6 + 8 * PT); }
+// Where the tables of `cells` (piece, head) stand, in floats.  The rows of 32 bytes come first: 16-byte loads and stores take them, and behind the
+// doubles of an odd number of cells they would be 8 bytes off.
+struct WalkPlaces {
+  size_t tab, loc, m0, end;
+};
+WalkPlaces walk_places(size_t cells) {
+  const size_t loc = cells * 8 * PT, m0 = loc + 4 * cells;
+  return {0, loc, m0, m0 + 2 * cells};
+}
+// floats of a piece's slot; 0.4 us a token in the token-by-token form
+size_t slot_floats(int H) { return walk_places(H).end; }
 PiecePlan walk_plan(int T_, int B, int H, size_t most) { return plan_pieces(T_, B, PT, slot_floats(H), most, 0.4f); }
 
 // Tiles of 16 columns a block, or 0 where the states in chunks (seq_chunk.hip) are ahead or the sizes have no form here.  A block takes `turn` us
@@ -629,10 +638,8 @@ template <int NK, int NT, bool MLSTM>
 void launch(const bf16* q, int ldq, const bf16* k, int ldk, const bf16* v, int ldv, const GateArgs& ga, float* S, float* N, float* M,
             float* out, float* den, float* efl, float* ws, size_t most, int H, int G, int dv, const SeqDesc& d, hipStream_t st) {
   const PiecePlan plan = walk_plan(d.Ttot, d.B, H, most);
-  WalkWs w;
-  w.loc = reinterpret_cast<double*>(ws);
-  w.m0 = w.loc + 2 * plan.slots * H;
-  w.tab = reinterpret_cast<float*>(w.m0 + plan.slots * H);
+  const WalkPlaces at = walk_places(plan.slots * H);
+  const WalkWs w = {reinterpret_cast<double*>(ws + at.loc), reinterpret_cast<double*>(ws + at.m0), ws + at.tab};
   for (int i = 0; i < plan.windows; ++i) {
     const Pieces pc = {PT, i * plan.count, plan.count};
     hipLaunchKernelGGL((k_walk_gates<MLSTM>), dim3((unsigned)plan.slots, (H + 3) / 4), dim3(256), 0, st, ga, w, M, H, pc, d);
@@ -661,6 +668,12 @@ void dispatch(const bf16* q, int ldq, const bf16* k, int ldk, const bf16* v, int
 }
 
 }  // namespace
+
+// the same, for checks: the three tables' places and the end
+void seq_walk_places(size_t cells, size_t* at) {
+  const WalkPlaces p = walk_places(cells);
+  at[0] = p.tab, at[1] = p.loc, at[2] = p.m0, at[3] = p.end;
+}
 
 int seq_walk_tiles(int T_, int B, int H, int dk, int dv, int longest) { return walk_tiles(T_, B, H, dk, dv, longest); }
 

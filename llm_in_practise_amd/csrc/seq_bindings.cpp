@@ -108,6 +108,7 @@ void seq_talk_attention(int, const void*, int, const void*, const void*, float*,
 size_t seq_chunk_floats(int, bool, const void*, int, const void*, int, const void*, int, const void*, const void*, int, int, int, int, int, int,
                         size_t);
 int seq_walk_tiles(int, int, int, int, int, int);
+void seq_walk_places(size_t, size_t*);
 void seq_chunk_ssd(const void*, int, const void*, int, const void*, int, const void*, int, const float*, const float*,
                    const float*, float*, float*, float*, size_t, int, int, int, int, int, SeqDesc, hipStream_t);
 void seq_chunk_mlstm(const void*, int, const void*, int, const void*, int, const float*, const float*, const float*,
@@ -1344,6 +1345,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       return 0;
     return 16 * seq_walk_tiles((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest);
   }, py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("longest"), py::arg("op") = "ssd");
+  // where its workspace for so many (piece, head) has the rows of the gates, the decays of the pieces and the states' units, and its end, in floats
+  m.def("walk_places", [](int64_t cells) {
+    std::vector<size_t> at(4);
+    seq_walk_places((size_t)cells, at.data());
+    return at;
+  });
   m.def("delta_block", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t most) {      // tokens of a block, 0: token by token
     if (seq_block_floats(0, true, nullptr, 8, nullptr, 8, nullptr, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, 0, (size_t)most) == 0) return 0;
     return seq_delta_floats((int)T, (int)B, (int)H, (int)dk, (int)dv, 0, (size_t)most) > 0 ? 32 : 16;

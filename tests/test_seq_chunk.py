@@ -864,6 +864,17 @@ def test_walk_with_the_state_at_hand(op, lens, H, dk, dv, cols, bad, whole):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("cells", [1, 2, 13 * 33, 64 * 8])
+def test_walk_tables_where_vector_loads_take_them(cells):
+    """Rows of 8 floats and pairs of doubles at multiples of 16 bytes, doubles at multiples of 8, each behind the one before, odd numbers of cells too."""
+    from llm_in_practise_amd.ops._native import native_seq
+    tab, loc, m0, end = native_seq().walk_places(cells)
+    assert tab % 4 == 0 and loc % 4 == 0 and m0 % 2 == 0
+    spans = sorted([(tab, 64 * 8), (loc, 2 * 2), (m0, 2)])
+    assert all(a + n * cells <= b for (a, n), b in zip(spans, [spans[1][0], spans[2][0], end]))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,B,H,dk,dv,longest,walks", [
     (12, 1, 8, 128, 192, 12, False), (20, 1, 8, 128, 192, 20, True), (63, 1, 8, 128, 192, 0, False), (160, 8, 8, 128, 192, 20, True),
     (240, 12, 8, 128, 192, 20, False), (756, 12, 8, 128, 192, 63, True), (768, 32, 32, 64, 96, 24, False), (192, 8, 8, 64, 96, 24, True),
