@@ -25,7 +25,7 @@
 
 using namespace lipa;
 
-size_t seq_walk_floats(int, int, int, int, int, int, size_t);
+size_t seq_walk_floats(bool, int, int, int, int, int, int, size_t);
 bool seq_walk_short(int, int, int, int, int, int);
 void seq_walk(bool, const void*, int, const void*, int, const void*, int, const GateArgs&, float*, float*, float*, float*, float*, float*, float*, size_t,
               int, int, int, int, int, const SeqDesc&, hipStream_t);
@@ -749,7 +749,7 @@ template <bool MLSTM>
 void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const GateArgs& ga, float* S, float* N,
                     float* M, float* out, float* den, float* efl, float* ws, size_t most, int H, int G, int dk, int dv,
                     int longest, SeqDesc d, hipStream_t st) {
-  if (seq_walk_floats(d.Ttot, d.B, H, dk, dv, longest, most) > 0)
+  if (seq_walk_floats(MLSTM, d.Ttot, d.B, H, dk, dv, longest, most) > 0)
     return seq_walk(MLSTM, q, ldq, k, ldk, v, ldv, ga, S, N, M, out, den, efl, ws, most, H, G, dk, dv, longest, d, st);
 #define CHUNK(NK_)                                                                                                          \
   chunk_launch<NK_, MLSTM>((const bf16*)q, ldq, (const bf16*)k, ldk, (const bf16*)v, ldv, ga, S, N, M, out, den, efl, ws, \
@@ -764,6 +764,8 @@ void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* 
 }
 
 }  // namespace
+
+int seq_run_chunks(int T_, int B, int H, int dv) { return run_chunks(T_, B, H, dv); }
 
 // Floats of workspace of the chunked form, or 0 where the token-by-token scan is the one to run: float activations, key sizes
 // that are no multiple of 32 or above 128, rows that 16-byte (q, k, the states S and N) or 8-byte (v) loads cannot take, and steps of
@@ -787,8 +789,8 @@ size_t seq_chunk_floats(int code, bool mlstm, const void* q, int ldq, const void
   if (pairs >= 1024 && (dk <= 64 || dv <= 32)) least = 192;
   if (pairs * dv >= 1l << 17 && dk <= 32) least = 256;
   if (B == 0) return 0;
-  if (T_ < least * B) return mlstm && seq_walk_short(T_, B, H, dk, dv, longest) ? seq_walk_floats(T_, B, H, dk, dv, longest, most) : 0;
-  if (const size_t n = seq_walk_floats(T_, B, H, dk, dv, longest, most)) return n;      // (the state never leaves its block)
+  if (T_ < least * B) return mlstm && seq_walk_short(T_, B, H, dk, dv, longest) ? seq_walk_floats(true, T_, B, H, dk, dv, longest, most) : 0;
+  if (const size_t n = seq_walk_floats(mlstm, T_, B, H, dk, dv, longest, most)) return n;      // (the state never leaves its block)
   const int sc = run_chunks(T_, B, H, dv);
   const size_t slots = run_plan(T_, B, H, dk, dv, sc, most).slots;
   return slots == 0 ? 0 : slots * run_floats(sc, H, dk, dv) + 4;

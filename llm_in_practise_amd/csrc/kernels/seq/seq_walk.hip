@@ -24,6 +24,8 @@
 
 using namespace lipa;
 
+int seq_run_chunks(int, int, int, int);
+
 namespace {
 
 constexpr int PT = 64;                  // tokens of a piece
@@ -606,25 +608,42 @@ WalkPlaces walk_places(size_t cells) {
 size_t slot_floats(int H) { return walk_places(H).end; }
 PiecePlan walk_plan(int T_, int B, int H, size_t most) { return plan_pieces(T_, B, PT, slot_floats(H), most, 0.4f); }
 
-// Tiles of 16 columns a block, or 0 where the states in chunks (seq_chunk.hip) are ahead or the sizes have no form here.  A block takes `turn` us
-// for 128 tokens and 3 around them, one runs on a CU, and the longest sequence's have to follow each other; the chunks' three launches go by their
-// blocks of 128 tokens and 64 columns alone.  Chunks -> here, us: mLSTM, 8 heads of 128 x 192: 80 tokens 21 -> 11, 512 28 -> 21, 2 x 512 31 -> 22,
-// 8 x 1024 89 -> 52, 48 x 128 99 -> 67, but one prompt of 2048 44 -> 58; of 64 x 96: 8 x 512 32 -> 21, 12 x 700 47 -> 32, one of 2048 32 -> 43; state
-// space, 64 heads of 128 x 64: 512 34 -> 19, 4 x 512 63 -> 45, 8 x 1024 172 -> 143, 2 x 4096 162 -> 129, one of 4093 91 -> 92, of 9000 188 -> 186; 32
-// heads: 1000 33 -> 27, 12 x 700 108 -> 83, one of 4093 61 -> 89.  More columns a block: fewer blocks for the scores and splits, but longer turns (8 x 1024
-// of 128 x 192 with 16 / 32 / 48 columns 78 / 70 / 52, one prompt of 512 21 / 25 / 29; 8 x 512 of 64 x 96 25 / 21 / 24).
-int walk_tiles(int T_, int B, int H, int dk, int dv, int longest, float* takes = nullptr) {
+// Tiles of 16 columns a block, or 0 where the states in chunks (seq_chunk.hip) are ahead or the sizes have no form here.
+//
+// Here a block takes `turn` us for 128 tokens, a seventh less where most CUs are idle, and one runs on a CU.  Up to 256 blocks the longest sequence's
+// turns are all of it.  More of them come in rounds, of blocks of the mean length; the longest sequence's last block may be in the last
+// round, so its turns beyond the mean stand behind all of them.  (Counted as if they ran beside the rounds, one long prompt among short ones was walked where
+// that takes up to 1.5 times as long: mLSTM, 8 heads of 64 x 160, six of 2517 tokens and 14 short ones 110 in chunks, 160 here.)  The chunks' three
+// launches go by their blocks of 128 tokens and 64 columns, in part by the columns that these have, and by the chunks of the longest sequence
+// in their second, in runs.
+// The constants are fitted to 3500 calls of both ops, 1 to 64 heads, 1 to 64 sequences, all of one length, ragged, or one or a few long ones among short
+// ones: chunks within 10 %, blocks of one round within 6.  It walks 1860 of them, in 0.70 of the chunks' time; 5 are slower than in chunks, by
+// 4 to 9 %.  (Before: 81 slower, by up to 47 %.)
+// Chunks -> here, us: mLSTM, 8 heads of 128 x 192: 80 tokens 21 -> 11, 512 28 -> 21, 2 x 512 31 -> 22, 8 x 1024 89 -> 52, 48 x 128 99 -> 67, but one
+// prompt of 2048 44 -> 58; of 64 x 96: 8 x 512 32 -> 21, 12 x 700 47 -> 32, one of 2048 32 -> 43; state space, 64 heads of 128 x 64: 512 34 -> 19, 4 x 512 63 ->
+// 45, 8 x 1024 172 -> 143, 2 x 4096 162 -> 129, one of 4093 91 -> 92; 32 heads: 1000 33 -> 27, 12 x 700 108 -> 83, one of 4093 61 -> 89.  More
+// columns a block: fewer blocks for the scores and splits, but longer turns (8 x 1024 of 128 x 192 with 16 / 32 / 48 columns 78 / 70 / 52, one prompt
+// of 512 21 / 25 / 29; 8 x 512 of 64 x 96 25 / 21 / 24).
+int walk_tiles(bool mlstm, int T_, int B, int H, int dk, int dv, int longest, float* takes = nullptr) {
   if ((dk != 64 && dk != 128) || B == 0) return 0;
-  constexpr float TURN_US[2][4] = {{2.1f, 2.9f, 3.5f, 4.4f}, {2.8f, 3.8f, 4.9f, 0.f}};
+  struct Cost {
+    float turn[4], launches, block, column, head;
+  };
+  constexpr Cost COST[2][2] = {{{{1.97f, 2.95f, 3.74f, 4.67f}, 17.f, 0.0135f, 0.011f, 0.003f}, {{2.77f, 3.94f, 5.02f, 0.f}, 20.f, 0.023f, 0.017f, 0.002f}},
+                               {{{2.51f, 3.38f, 3.9f, 4.8f}, 18.5f, 0.014f, 0.0125f, 0.007f}, {{3.31f, 4.37f, 5.3f, 0.f}, 22.f, 0.02f, 0.024f, 0.009f}}};
+  const Cost& cost = COST[mlstm][dk / 128];
   const long pairs = (long)B * H, tiles = (dv + 15) / 16;
   if (longest <= 0 || longest > T_) longest = T_ - (B - 1);                    // (not known: all but a token of each other sequence)
-  const long most = (longest + TURN - 1) / TURN, mean = (T_ / B + TURN - 1) / TURN;
-  const float chunks = 18.f + (dk == 64 ? 0.03f : 0.04f) * ((float)T_ / 128 + 0.5f * B) * H * ((dv + 63) / 64);
-  float best = 0.97f * chunks;
+  const int run = seq_run_chunks(T_, B, H, dv);
+  const float chunks = (cost.launches + 0.55f / run * longest / 128 +
+                        ((float)T_ / 128 + 0.5f * B) * H * (cost.block * ((dv + 63) / 64) + cost.column * dv / 64 + cost.head)) * (run == 4 ? 0.92f : 1.f);
+  const float most = 0.5f * ((longest + PT - 1) / PT), mean = std::min(most, (float)T_ / B / TURN + 0.25f);        // turns
+  float best = 0.93f * chunks;
   int nt = 0;
   for (int t = 1; t <= (dk == 64 ? 4 : 3) && t <= tiles; ++t) {
-    const long rounds = (pairs * ((tiles + t - 1) / t) + 255) / 256;
-    const float turn = TURN_US[dk / 128][t - 1], us = 6.f + std::max(3.f + most * turn, rounds * (3.f + mean * turn));
+    const long blocks = pairs * ((tiles + t - 1) / t);
+    const float turn = cost.turn[t - 1] * (0.87f + 0.13f * std::min(1.f, blocks / 256.f));
+    const float us = (mlstm ? 9.7f : 8.6f) + turn * (most + 0.25f) + (float)((blocks + 255) / 256 - 1) * (3.f + turn * (mean + 0.25f));
     if (us < best) {
       best = us;
       nt = t;
@@ -654,7 +673,7 @@ void dispatch(const bf16* q, int ldq, const bf16* k, int ldk, const bf16* v, int
               float* out, float* den, float* efl, float* ws, size_t most, int H, int G, int dk, int dv, int longest, const SeqDesc& d, hipStream_t st) {
 #define WALK(NK_, NT_) \
   return launch<NK_, NT_, MLSTM>(q, ldq, k, ldk, v, ldv, ga, S, N, M, out, den, efl, ws, most, H, G, dv, d, st)
-  const int nt = walk_tiles(d.Ttot, d.B, H, dk, dv, longest);
+  const int nt = walk_tiles(MLSTM, d.Ttot, d.B, H, dk, dv, longest);
   if (dk == 64) {
     if (nt == 1) WALK(2, 1);
     if (nt == 2) WALK(2, 2);
@@ -675,7 +694,7 @@ void seq_walk_places(size_t cells, size_t* at) {
   at[0] = p.tab, at[1] = p.loc, at[2] = p.m0, at[3] = p.end;
 }
 
-int seq_walk_tiles(int T_, int B, int H, int dk, int dv, int longest) { return walk_tiles(T_, B, H, dk, dv, longest); }
+int seq_walk_tiles(bool mlstm, int T_, int B, int H, int dk, int dv, int longest) { return walk_tiles(mlstm, T_, B, H, dk, dv, longest); }
 
 // Whether an mLSTM's prompts too short for chunks walk their tokens here and not one by one (lengths that are known).  That form takes 7 us and 0.38 a
 // token of the longest sequence (keys of 64: 5.5 and 0.3), or 0.14 ps a token, key channel and column where they fill the chip.  us, token by token ->
@@ -685,15 +704,15 @@ int seq_walk_tiles(int T_, int B, int H, int dk, int dv, int longest) { return w
 // 63, but its outputs' error is 0.4e-7 token by token and 0.6 here.)
 bool seq_walk_short(int T_, int B, int H, int dk, int dv, int longest) {
   float us = 0.f;
-  if (longest <= 0 || longest > T_ || walk_tiles(T_, B, H, dk, dv, longest, &us) == 0) return false;
+  if (longest <= 0 || longest > T_ || walk_tiles(true, T_, B, H, dk, dv, longest, &us) == 0) return false;
   const float full = 0.14e-6f * ((float)B * H * dv * dk) * T_ / B, chain = (dk == 64 ? 0.3f : 0.38f) * longest;
   return us < 0.97f * ((dk == 64 ? 5.5f : 7.f) + std::max(chain, full));
 }
 
 // Floats of workspace for at most `most` (longer steps run in windows), or 0 where the state in chunks (seq_chunk.hip) is to run.  longest: tokens of
 // the longest sequence, 0 where the caller does not know.
-size_t seq_walk_floats(int T_, int B, int H, int dk, int dv, int longest, size_t most) {
-  if (walk_tiles(T_, B, H, dk, dv, longest) == 0) return 0;
+size_t seq_walk_floats(bool mlstm, int T_, int B, int H, int dk, int dv, int longest, size_t most) {
+  if (walk_tiles(mlstm, T_, B, H, dk, dv, longest) == 0) return 0;
   return walk_plan(T_, B, H, most).slots * slot_floats(H);
 }
 

@@ -107,7 +107,7 @@ void seq_talk_attention(int, const void*, int, const void*, const void*, float*,
                         SeqDesc, hipStream_t);
 size_t seq_chunk_floats(int, bool, const void*, int, const void*, int, const void*, int, const void*, const void*, int, int, int, int, int, int,
                         size_t);
-int seq_walk_tiles(int, int, int, int, int, int);
+int seq_walk_tiles(bool, int, int, int, int, int, int);
 void seq_walk_places(size_t, size_t*);
 void seq_chunk_ssd(const void*, int, const void*, int, const void*, int, const void*, int, const float*, const float*,
                    const float*, float*, float*, float*, size_t, int, int, int, int, int, SeqDesc, hipStream_t);
@@ -1343,7 +1343,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("scan_walk", [](int64_t T, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t longest, const std::string& op) {
     if (seq_chunk_floats(0, op == "mlstm", nullptr, 8, nullptr, 8, nullptr, 8, nullptr, nullptr, (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest, (size_t)MOST_WS) == 0)
       return 0;
-    return 16 * seq_walk_tiles((int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest);
+    return 16 * seq_walk_tiles(op == "mlstm", (int)T, (int)B, (int)H, (int)dk, (int)dv, (int)longest);
   }, py::arg("T"), py::arg("B"), py::arg("H"), py::arg("dk"), py::arg("dv"), py::arg("longest"), py::arg("op") = "ssd");
   // where its workspace for so many (piece, head) has the rows of the gates, the decays of the pieces and the states' units, and its end, in floats
   m.def("walk_places", [](int64_t cells) {
