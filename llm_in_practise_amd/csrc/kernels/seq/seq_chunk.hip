@@ -767,6 +767,22 @@ void chunk_dispatch(const void* q, int ldq, const void* k, int ldk, const void* 
 
 int seq_run_chunks(int T_, int B, int H, int dv) { return run_chunks(T_, B, H, dv); }
 
+// Tokens a sequence from which on prompts run in chunks.
+// Three launches and a chunk of padding against 0.4 us a token (two heads a CU) in the token-by-token form: 64 tokens a
+// sequence are 21 / 32 / 96 us here and 30 / 36 / 148 us there (state space, 32 heads, 1 / 8 / 48 sequences), 48 are 21 / 32 / 94
+// and 24 / 29 / 118 us; mLSTM (8 heads of 128 x 192) at 64: 26 / 34 / 68 against 31 / 36 / 159 us.  The outputs walk the columns 32 at a
+// time, one after another: 512 of them 43 against 26 us at 64 tokens, even at 128 to 160.  Where (sequence, head) pairs fill the chip,
+// the padding counts, and with small keys the token form is the cheaper one for longer: 1024 pairs of 64 x 64 take 1.3 times its time at
+// 64 to 128 tokens, 0.94 at 192; 1024 of 32 x 128 1.2 at 192, 1.08 at 256, 0.92 at 512; 1024 of 128 x 64 are ahead from 64 on.
+long seq_chunk_least(int B, int H, int dk, int dv) {
+  const long pairs = (long)B * H;
+  long least = std::max(64, std::min(dv * 5 / 12, 192));
+  if (pairs >= 256 && dk <= 64 && dv >= 128) least = std::max(least, 96l);
+  if (pairs >= 1024 && (dk <= 64 || dv <= 32)) least = 192;
+  if (pairs * dv >= 1l << 17 && dk <= 32) least = 256;
+  return least;
+}
+
 // Floats of workspace of the chunked form, or 0 where the token-by-token scan is the one to run: float activations, key sizes
 // that are no multiple of 32 or above 128, rows that 16-byte (q, k, the states S and N) or 8-byte (v) loads cannot take, and steps of
 // few tokens a sequence.  At most `most`: longer steps run in windows.
@@ -777,19 +793,9 @@ size_t seq_chunk_floats(int code, bool mlstm, const void* q, int ldq, const void
       !fits(q, ldq, 8) || !fits(k, ldk, 8) || !fits(v, ldv, 4) ||
       !fits(S, 8, 8) || !fits(N, 8, 8))
     return 0;
-  // Three launches and a chunk of padding against 0.4 us a token (two heads a CU) in the token-by-token form: 64 tokens a
-  // sequence are 21 / 32 / 96 us here and 30 / 36 / 148 us there (state space, 32 heads, 1 / 8 / 48 sequences), 48 are 21 / 32 / 94
-  // and 24 / 29 / 118 us; mLSTM (8 heads of 128 x 192) at 64: 26 / 34 / 68 against 31 / 36 / 159 us.  The outputs walk the columns 32 at a
-  // time, one after another: 512 of them 43 against 26 us at 64 tokens, even at 128 to 160.  Where (sequence, head) pairs fill the chip,
-  // the padding counts, and with small keys the token form is the cheaper one for longer: 1024 pairs of 64 x 64 take 1.3 times its time at
-  // 64 to 128 tokens, 0.94 at 192; 1024 of 32 x 128 1.2 at 192, 1.08 at 256, 0.92 at 512; 1024 of 128 x 64 are ahead from 64 on.
-  const long pairs = (long)B * H;
-  long least = std::max(64, std::min(dv * 5 / 12, 192));
-  if (pairs >= 256 && dk <= 64 && dv >= 128) least = std::max(least, 96l);
-  if (pairs >= 1024 && (dk <= 64 || dv <= 32)) least = 192;
-  if (pairs * dv >= 1l << 17 && dk <= 32) least = 256;
   if (B == 0) return 0;
-  if (T_ < least * B) return mlstm && seq_walk_short(T_, B, H, dk, dv, longest) ? seq_walk_floats(true, T_, B, H, dk, dv, longest, most) : 0;
+  if (T_ < seq_chunk_least(B, H, dk, dv) * B)
+    return mlstm && seq_walk_short(T_, B, H, dk, dv, longest) ? seq_walk_floats(true, T_, B, H, dk, dv, longest, most) : 0;
   if (const size_t n = seq_walk_floats(mlstm, T_, B, H, dk, dv, longest, most)) return n;      // (the state never leaves its block)
   const int sc = run_chunks(T_, B, H, dv);
   const size_t slots = run_plan(T_, B, H, dk, dv, sc, most).slots;

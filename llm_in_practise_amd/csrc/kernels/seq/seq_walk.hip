@@ -25,6 +25,7 @@
 using namespace lipa;
 
 int seq_run_chunks(int, int, int, int);
+long seq_chunk_least(int, int, int, int);
 
 namespace {
 
@@ -608,17 +609,18 @@ WalkPlaces walk_places(size_t cells) {
 size_t slot_floats(int H) { return walk_places(H).end; }
 PiecePlan walk_plan(int T_, int B, int H, size_t most) { return plan_pieces(T_, B, PT, slot_floats(H), most, 0.4f); }
 
-// Tiles of 16 columns a block, or 0 where the states in chunks (seq_chunk.hip) are ahead or the sizes have no form here.
-//
-// Here a block takes `turn` us for 128 tokens, a seventh less where most CUs are idle, and one runs on a CU.  Up to 256 blocks the longest sequence's
-// turns are all of it.  More of them come in rounds, of blocks of the mean length; the longest sequence's last block may be in the last
-// round, so its turns beyond the mean stand behind all of them.  (Counted as if they ran beside the rounds, one long prompt among short ones was walked where
-// that takes up to 1.5 times as long: mLSTM, 8 heads of 64 x 160, six of 2517 tokens and 14 short ones 110 in chunks, 160 here.)  The chunks' three
-// launches go by their blocks of 128 tokens and 64 columns, in part by the columns that these have, and by the chunks of the longest sequence
-// in their second, in runs.
-// The constants are fitted to 3500 calls of both ops, 1 to 64 heads, 1 to 64 sequences, all of one length, ragged, or one or a few long ones among short
-// ones: chunks within 10 %, blocks of one round within 6.  It walks 1860 of them, in 0.70 of the chunks' time; 5 are slower than in chunks, by
-// 4 to 9 %.  (Before: 81 slower, by up to 47 %.)
+// Tiles of 16 columns a block, or 0 where the states in chunks (seq_chunk.hip) are ahead or the sizes have no form here.  Two estimates have to agree:
+//  * a block takes `turn` us for 128 tokens and 3 around them, one runs on a CU, and the longest sequence's have to follow each other beside the
+//    rounds of all blocks; the chunks' three launches go by their blocks of 128 tokens and 64 columns alone;
+//  * the longest sequence's last block may be in the last round, so its turns beyond the mean stand behind all rounds, where there is more than one; a
+//    turn is a seventh shorter where most CUs are idle; the chunks go by their blocks, the columns that these have, and the longest sequence's chunks in
+//    their second launch, in runs.
+// The first alone walks one or a few long prompts among short ones where that takes up to twice as long (mLSTM, 8 heads of 64 x 160, six of 2517 tokens
+// and 14 short ones 110 in chunks, 160 here).  The second is fitted to the chunks and every width of a block on 3600 calls, 1 to 64 heads, 1 to
+// 64 sequences, all of one length, ragged, or one or a few long ones among short ones in any place: chunks within 10 %, blocks of one round within
+// 6.  It does not know which place that is, nor how many heads share keys, so it only has to be within 5 % of agreeing.  Of 6370 calls the first one
+// walks 3770, 156 of them slower so; both together 3470, 26 of them slower, by 2 to 20 %.
+// Prompts that no chunks are there for (seq_walk_short) ask the first one alone.
 // Chunks -> here, us: mLSTM, 8 heads of 128 x 192: 80 tokens 21 -> 11, 512 28 -> 21, 2 x 512 31 -> 22, 8 x 1024 89 -> 52, 48 x 128 99 -> 67, but one
 // prompt of 2048 44 -> 58; of 64 x 96: 8 x 512 32 -> 21, 12 x 700 47 -> 32, one of 2048 32 -> 43; state space, 64 heads of 128 x 64: 512 34 -> 19, 4 x 512 63 ->
 // 45, 8 x 1024 172 -> 143, 2 x 4096 162 -> 129, one of 4093 91 -> 92; 32 heads: 1000 33 -> 27, 12 x 700 108 -> 83, one of 4093 61 -> 89.  More
@@ -626,6 +628,7 @@ PiecePlan walk_plan(int T_, int B, int H, size_t most) { return plan_pieces(T_, 
 // of 512 21 / 25 / 29; 8 x 512 of 64 x 96 25 / 21 / 24).
 int walk_tiles(bool mlstm, int T_, int B, int H, int dk, int dv, int longest, float* takes = nullptr) {
   if ((dk != 64 && dk != 128) || B == 0) return 0;
+  constexpr float TURN_US[2][4] = {{2.1f, 2.9f, 3.5f, 4.4f}, {2.8f, 3.8f, 4.9f, 0.f}};
   struct Cost {
     float turn[4], launches, block, column, head;
   };
@@ -634,22 +637,33 @@ int walk_tiles(bool mlstm, int T_, int B, int H, int dk, int dv, int longest, fl
   const Cost& cost = COST[mlstm][dk / 128];
   const long pairs = (long)B * H, tiles = (dv + 15) / 16;
   if (longest <= 0 || longest > T_) longest = T_ - (B - 1);                    // (not known: all but a token of each other sequence)
+  const bool chunked = T_ >= seq_chunk_least(B, H, dk, dv) * B;
+  const long most = (longest + TURN - 1) / TURN, mean = (T_ / B + TURN - 1) / TURN;
+  const float cells = ((float)T_ / 128 + 0.5f * B) * H, blocks64 = (dv + 63) / 64;
+  const float chunks = 18.f + (dk == 64 ? 0.03f : 0.04f) * cells * blocks64;
   const int run = seq_run_chunks(T_, B, H, dv);
-  const float chunks = (cost.launches + 0.55f / run * longest / 128 +
-                        ((float)T_ / 128 + 0.5f * B) * H * (cost.block * ((dv + 63) / 64) + cost.column * dv / 64 + cost.head)) * (run == 4 ? 0.92f : 1.f);
-  const float most = 0.5f * ((longest + PT - 1) / PT), mean = std::min(most, (float)T_ / B / TURN + 0.25f);        // turns
-  float best = 0.93f * chunks;
+  const float chunks2 = (cost.launches + 0.55f / run * longest / 128 + cells * (cost.block * blocks64 + cost.column * dv / 64 + cost.head)) *
+                        (run == 4 ? 0.92f : 1.f);
+  const float most2 = 0.5f * ((longest + PT - 1) / PT), mean2 = std::min(most2, (float)T_ / B / TURN + 0.25f);
+  float best = 3.f;
   int nt = 0;
   for (int t = 1; t <= (dk == 64 ? 4 : 3) && t <= tiles; ++t) {
-    const long blocks = pairs * ((tiles + t - 1) / t);
-    const float turn = cost.turn[t - 1] * (0.87f + 0.13f * std::min(1.f, blocks / 256.f));
-    const float us = (mlstm ? 9.7f : 8.6f) + turn * (most + 0.25f) + (float)((blocks + 255) / 256 - 1) * (3.f + turn * (mean + 0.25f));
-    if (us < best) {
-      best = us;
+    const long blocks = pairs * ((tiles + t - 1) / t), rounds = (blocks + 255) / 256;
+    const float turn = TURN_US[dk / 128][t - 1], us = 6.f + std::max(3.f + most * turn, rounds * (3.f + mean * turn));
+    float score = us / chunks;
+    if (score >= 0.97f) continue;
+    if (chunked) {
+      const float turn2 = cost.turn[t - 1] * (0.87f + 0.13f * std::min(1.f, blocks / 256.f));
+      const float late = ((mlstm ? 9.7f : 8.6f) + turn2 * (most2 + 0.25f) + (float)(rounds - 1) * (3.f + turn2 * (mean2 + 0.25f))) / chunks2;
+      if (late >= 1.05f) continue;
+      score += late;
+    }
+    if (score < best) {
+      best = score;
       nt = t;
+      if (takes != nullptr) *takes = us;
     }
   }
-  if (takes != nullptr) *takes = best;
   return nt;
 }
 
