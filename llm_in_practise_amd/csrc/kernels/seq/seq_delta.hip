@@ -563,16 +563,27 @@ PiecePlan delta_plan(int T_, int B, int H, int dk, int dv, size_t most) {
 // a step that leaves CUs idle; in parts the windows of all of them count: 1.42 us a window of the outputs' walk where a CU has one block,
 // 1.15 where it has two or more at once, 0.95 and 0.82 a window of the ends' (which bring 35 KB each, 7 to 10 TB/s out of the caches), 2 us
 // for each part in front of the last one's state and 8 for the launch and what stands in front of the first windows (keys of 128; of 64
-// three quarters).  The other sequences are taken to be of one length.  us, in one piece -> in parts, 4 heads of 128 x 128: 1000 tokens 62 -> 47,
-// 4093 198 -> 87, 9000 422 -> 170, 3000 + 1700 155 -> 103, 5000 and three of 40 240 -> 114 (400 33 -> 35, 4 x 2000 122 -> 121, 1000 + 700 + 500
-// + 600 + 800 67 -> 73: in one piece); 8 heads: 700 47 -> 43, 1000 61 -> 54, 1500 + 700 + 97 94 -> 87, 4093 209 -> 140, 9000 445 -> 295, 3000 +
-// 1700 167 -> 142 (4 x 2000 149 -> 206: in one piece).
+// three quarters).  The other sequences are taken to be of one length.
+// Where there are others, a second estimate can object: as many as can be are of the longest's length, or all of them have the parts that their
+// tokens make up; constants fitted to 930 timed calls of 1 to 64 heads and sequences with parts of up to nine lengths each (within 13 %).  Few long ones
+// among short ones have more parts than the first one counts: 8 heads of 128 x 16, eight of 1134 tokens and 16 short ones 122 in one piece, 163 in parts of 8
+// blocks.  Of 2450 calls 2080 ran in parts, 58 of them slower so, by up to a third; now 2010, 26 of them, by up to 18 %.
+// us, in one piece -> in parts, 4 heads of 128 x 128: 1000 tokens 62 -> 47, 4093 197 -> 88, 9000 422 -> 170, 3000 + 1700 155 -> 103, 5000 and three
+// of 40 240 -> 114 (400 33 -> 35, 4 x 2000 122 -> 121, 1000 + 700 + 500 + 600 + 800 67 -> 73: in one piece); 8 heads: 700 47 -> 43, 1000 61 -> 54, 1500 +
+// 700 + 97 92 -> 86 (four parts, two and one; in parts of 8 / 10 / 14 / 16 / 18 / 24 blocks for 12 97 / 91 / 93 / 89 / 93 / 89), 4093 208 -> 136,
+// 9000 445 -> 295, 3000 + 1700 167 -> 142 (4 x 2000 149 -> 206: in one piece).
 int part_blocks(int T_, int B, int H, int dk, int dv, int longest) {
   const int tiles = (dv + 15) / 16, units = dk / 16, top = (longest + LEN - 1) / LEN;
   if (longest > T_ || top < 2 || (long)B * H * tiles > 256) return 0;
-  const int rest = B > 1 ? ((T_ - longest) / (B - 1) + LEN - 1) / LEN : 0;
+  const int rest = B > 1 ? ((T_ - longest) / (B - 1) + LEN - 1) / LEN : 0, alike = std::min(B, T_ / longest);
   const auto cus = [](float n) { return ceilf(n / 256.f); };
   const float scale = dk == 64 ? 0.75f : 1.f;
+  struct Cost {
+    float piece, window, parts, walk, end, more, prep;
+  };
+  constexpr Cost COST[2] = {{12.9f, 0.92f, 19.6f, 0.73f, 0.44f, 1.f, 3.3f}, {15.2f, 1.35f, 25.8f, 1.55f, 0.67f, 2.f, 6.4f}};
+  const Cost& c = COST[dk / 128];
+  const float prep = ((float)T_ / LEN + 0.5f * B) * H / 256 * (c.prep + 0.8f * dv / 64);
   float best = 0.92f * (1.36f * scale * top + 4.f);
   int blocks = 0;
   for (int parts = 2; parts <= 12; ++parts) {
@@ -582,7 +593,18 @@ int part_blocks(int T_, int B, int H, int dk, int dv, int longest) {
     const float walk = cus((float)(n + (B - 1) * m) * H * tiles);
     const float ends = cus(H * ((float)tiles * (n - 1 + (B - 1) * std::max(m - 1, 0)) + (float)units * (n - 2 + (B - 1) * std::max(m - 2, 0))));
     const float us = scale * (L * ((walk > 1.f ? 1.15f * walk : 1.42f) + (ends > 1.f ? 0.82f * ends : 0.95f)) + 2.f * (n - 2)) + 8.f;
-    if (us < best) best = us, blocks = L;
+    if (us >= best) continue;
+    if (B > 1) {
+      const auto takes = [&](float walked, float ended, float transitions) {
+        const float w = walked * H * tiles / 256, e = H * (ended * tiles + transitions * units) / 256;
+        return c.parts + prep + L * (c.walk * std::max(1.f, w) + c.end * std::max(1.f, e)) + c.more * (n - 2);
+      };
+      const float others = std::max((float)(T_ - longest) / (LEN * L) - 0.5f * (B - 1), 0.f);        // their ends
+      if (std::max(takes(alike * n + B - alike, alike * (n - 1), alike * (n - 2)),
+                   takes(n + others + B - 1, n - 1 + others, n - 2 + std::max(others - (B - 1), 0.f))) >= 0.99f * (c.piece + prep + c.window * top))
+        continue;
+    }
+    best = us, blocks = L;
   }
   return blocks;
 }

@@ -395,6 +395,17 @@ def test_parts_find_room_beside_the_blocks(op, dk):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,B,H,dk,dv,longest,blocks", [
+    (10239, 24, 8, 128, 16, 1134, 0), (5073, 8, 32, 128, 16, 2446, 0), (16095, 32, 4, 128, 16, 1065, 0), (8000, 4, 4, 128, 128, 2000, 0),
+    (2297, 3, 8, 128, 128, 1500, 12), (700, 1, 8, 128, 128, 700, 8), (4093, 1, 8, 128, 128, 4093, 19), (5120, 4, 4, 128, 128, 5000, 32)])
+def test_delta_in_parts_only_where_it_is_not_slower(T, B, H, dk, dv, longest, blocks):
+    """Timed shapes, us in one piece / in parts: few long sequences among short ones that fill the chip (122 / 163, 269 / 306, 109 / 121) and long ones that
+    do (122 / 121) stay in one piece; (92 / 86, 47 / 43, 208 / 136, 240 / 114) do not."""
+    from llm_in_practise_amd.ops._native import native_seq
+    assert native_seq().scan_parts("delta", T, B, H, dk, dv, longest) == blocks
+
+
+@pytest.mark.gpu
 def test_parts_that_can_be_counted():
     """Parts are counted in 16 bits: a step that would have more, which takes a longest sequence that is not the longest, has none."""
     from llm_in_practise_amd.ops._native import native_seq
@@ -405,9 +416,9 @@ def test_parts_that_can_be_counted():
         floats = ext.scan_floats("gla", T, 1, 1, 64, 16, most=1 << 40)
         assert (ext.scan_parts("gla", T, 1, 1, 64, 16, longest=1000, most=1 << 40) > 0) == parts
         assert (ext.scan_floats("gla", T, 1, 1, 64, 16, most=1 << 40, longest=1000) > floats) == parts
-    # keys of the delta rule: what a plan holds is no more, whatever the caller says
-    assert ext.scan_parts("delta", 2_000_000, 1, 1, 64, 16, longest=1000, most=1 << 40) > 0
-    assert ext.scan_parts("delta", 2_100_000, 1, 1, 64, 16, longest=1000, most=1 << 40) == 0
+    # the delta rule: what a plan holds is no more, whatever the caller says
+    assert ext.scan_parts("delta", 2_000_000, 1, 1, 64, 16, longest=2_000_000, most=1 << 40) > 0
+    assert ext.scan_parts("delta", 2_100_000, 1, 1, 64, 16, longest=2_100_000, most=1 << 40) == 0
 
 
 @pytest.mark.gpu
