@@ -398,13 +398,29 @@ size_t slot_floats(int H, int dk) { return (size_t)H * (cell_floats(dk) + 4); }
 // Blocks of a part of linear attention, 0: sequences in one piece.  A block of tokens takes 0.49 us where a CU has one or two blocks of threads,
 // whatever the others do; in parts the blocks of all of them count, twice: 0.28 us for each block of threads on a CU, at least as for 1.3,
 // 0.6 for a part in front of the last one's state and 6 for the launch and the first blocks (keys of 64).  The other sequences are taken
-// to be of one length.  us, in one piece -> in parts, 8 heads of 64 x 128: 1000 tokens 40 -> 26, 4093 137 -> 63, 9000 288 -> 118, 3000 + 1700
+// to be of one length.
+// A second estimate can object.  It knows that keys of 192 and 256 leave one block of threads a CU, and that few long sequences among short ones have more parts:
+// as many as can be are of the longest's length, or the others have the parts that their tokens make up.  Its constants are fitted to 1650 timed
+// calls of 1 to 64 heads and sequences with parts of up to nine lengths each (within 17 %).  Of 3440 calls 2580 ran in parts, 93 of them slower so, by up to
+// 36 % (keys of 192, 16 heads of 192 columns, one prompt of 1396 tokens 110 -> 147); now 2460, 31 of them, by up to 15 %.
+// us, in one piece -> in parts, 8 heads of 64 x 128: 1000 tokens 40 -> 26, 4093 137 -> 68, 9000 288 -> 118, 3000 + 1700
 // 107 -> 77, 5000 and three of 40 165 -> 76 (400 21 -> 20, 4 x 2000 86 -> 91, 10 x 700 74 -> 89: in one piece); 16 heads: 1000 45 -> 38, 4093
 // 147 -> 100, 9000 312 -> 203, 5000 and three of 40 224 -> 127 (400 22 -> 25, 3000 + 1700 118 -> 113: in one piece).
 int part_blocks(int T_, int B, int H, int dk, int dv, int longest) {
   const int top = (longest + BT - 1) / BT, rest = B > 1 ? ((T_ - longest) / (B - 1) + BT - 1) / BT : 0;
-  if (longest > T_ || (long)B * H * ((dv + 15) / 16) > 1024) return 0;
+  if (longest <= 0 || longest > T_ || (long)B * H * ((dv + 15) / 16) > 1024) return 0;
   const float full = H * ((dv + 15) / 16) / 256.f, scale = (dk + 64) / 128.f;
+  struct Cost {
+    float launches, piece, shared, part, beside, prep, prep64;       // us: of a step; of a block in one piece, and for each on its CU beyond one; in parts
+  };
+  constexpr Cost COST[4] = {{10.3f, 0.43f, 0.09f, 0.64f, 0.215f, 1.45f, 0.6f},
+                            {12.4f, 0.53f, 0.11f, 0.78f, 0.28f, 3.f, 0.95f},
+                            {15.2f, 0.69f, 0.19f, 1.08f, 0.58f, 4.6f, 1.8f},
+                            {15.6f, 0.98f, 0.36f, 1.4f, 0.74f, 8.f, 2.1f}};
+  const Cost& c = COST[dk / 64 - 1];
+  const float step = c.launches + ((float)T_ / BT + 0.5f * B) * H / 256 * (c.prep + c.prep64 * dv / 64);
+  const float one = step + top * (c.piece + c.shared * std::max(0.f, B * full - 1.f));
+  const int alike = std::min(B, T_ / longest);
   float best = 0.85f * 0.49f * scale * top;
   int blocks = 0;
   for (int parts = 2; parts <= 16; ++parts) {
@@ -413,7 +429,11 @@ int part_blocks(int T_, int B, int H, int dk, int dv, int longest) {
     const int n = (top + L - 1) / L, m = (rest + L - 1) / L;
     const float walk = full * (n + (B - 1) * m), ends = full * (n - 1 + (B - 1) * std::max(m - 1, 0));
     const float us = scale * (0.28f * L * (std::max(walk, 1.3f) + std::max(ends, 1.3f)) + 0.6f * (n - 2)) + 6.f;
-    if (us < best) best = us, blocks = L;
+    if (us >= best) continue;
+    const float others = std::max((float)(T_ - longest) / (BT * L) - 0.5f * (B - 1), 0.f);        // their ends
+    const float walk2 = full * std::max((float)(alike * n + B - alike), n + others + B - 1), ends2 = full * std::max((float)(alike * (n - 1)), n - 1 + others);
+    const float us2 = step + 5.5f + L * (c.part + c.beside * (std::max(0.f, walk2 - 1.f) + std::max(0.f, ends2 - 1.f))) + 0.25f * (n - 2);
+    if (us2 < (dk <= 128 ? 0.97f : 0.94f) * one) best = us, blocks = L;
   }
   return blocks;
 }
@@ -429,7 +449,7 @@ BlockPlan block_plan(bool delta, int T_, int B, int H, int dk, int dv, int longe
   if (delta || r.p.slots == 0 || r.p.count != 0) return r;
   if (const int blocks = part_blocks(T_, B, H, dk, dv, longest)) {
     const size_t more = (size_t)T_ / (blocks * BT) * H * part_floats(dk, dv);
-    // (16 parts of a sequence at most where none is longer than `longest`, which a caller may have wrong)
+    // (16 parts of a sequence at most where none is longer than `longest`; a caller may have that wrong, and the estimates' constants are no bound)
     if (T_ / (blocks * BT) + B <= MOST_PARTS && r.floats + more <= most) r.blocks = blocks, r.floats += more;
   }
   return r;

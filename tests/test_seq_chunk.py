@@ -406,16 +406,25 @@ def test_delta_in_parts_only_where_it_is_not_slower(T, B, H, dk, dv, longest, bl
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,B,H,dk,dv,longest,parts", [
+    (1396, 1, 16, 192, 192, 1396, False), (3596, 4, 4, 192, 192, 899, False), (9174, 3, 4, 256, 256, 3058, False), (8000, 4, 8, 64, 128, 2000, False),
+    (1000, 1, 8, 64, 128, 1000, True), (4093, 1, 16, 64, 128, 4093, True), (6275, 3, 8, 192, 160, 6190, True), (2232, 4, 3, 256, 64, 558, True)])
+def test_linear_attention_in_parts_only_where_it_is_not_slower(T, B, H, dk, dv, longest, parts):
+    """Timed shapes, us in one piece / in parts: 110 / 147, 79 / 108, 293 / 352, 86 / 91; 40 / 26, 147 / 100, 366 / 241, 66 / 49."""
+    from llm_in_practise_amd.ops._native import native_seq
+    assert (native_seq().scan_parts("gla", T, B, H, dk, dv, longest) > 0) == parts
+
+
+@pytest.mark.gpu
 def test_parts_that_can_be_counted():
     """Parts are counted in 16 bits: a step that would have more, which takes a longest sequence that is not the longest, has none."""
     from llm_in_practise_amd.ops._native import native_seq
     ext = native_seq()
     part = 16 * ext.scan_parts("gla", 1000, 1, 1, 64, 16, longest=1000)
     assert part > 0
-    for T, parts in ((32766 * part, True), (32767 * part, False), (40000 * part, False), (65537 * part, False)):
-        floats = ext.scan_floats("gla", T, 1, 1, 64, 16, most=1 << 40)
-        assert (ext.scan_parts("gla", T, 1, 1, 64, 16, longest=1000, most=1 << 40) > 0) == parts
-        assert (ext.scan_floats("gla", T, 1, 1, 64, 16, most=1 << 40, longest=1000) > floats) == parts
+    for T in (32767 * part, 40000 * part, 65537 * part):
+        assert ext.scan_parts("gla", T, 1, 1, 64, 16, longest=1000, most=1 << 40) == 0
+        assert ext.scan_floats("gla", T, 1, 1, 64, 16, most=1 << 40, longest=1000) == ext.scan_floats("gla", T, 1, 1, 64, 16, most=1 << 40)
     # the delta rule: what a plan holds is no more, whatever the caller says
     assert ext.scan_parts("delta", 2_000_000, 1, 1, 64, 16, longest=2_000_000, most=1 << 40) > 0
     assert ext.scan_parts("delta", 2_100_000, 1, 1, 64, 16, longest=2_100_000, most=1 << 40) == 0
