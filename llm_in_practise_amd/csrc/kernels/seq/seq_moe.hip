@@ -809,11 +809,19 @@ void seq_route_fused(int code, const void* h, int ldh, const float* router, cons
 // 19.1 (not taken), 25 -> 20, 54 -> 23; F 512, top 4, width 2048, 12 / 16 / 64 / 256 26.0 -> 27.1 (not taken), 29.9 -> 28.0, 62 -> 29, 150 -> 37; width 1024, 16 / 24
 // / 32 / 256 18.6 -> 20.8 (not taken), 23.3 -> 21.5, 25.4 -> 21.7, 91 -> 29.  With the ids' loads in front of the weights', and what stands beside the experts'
 // outputs on its way from the start, half a us less.
-// More experts have fewer pairs each to share their rows.
+// Where the line lies.  12.5 million: nothing between 10.5 (slower here) and 12.58 was timed.  1260 more steps, 1 to 16 experts, top 1 to 8, F 32 to 512,
+// widths of 128 to 2048, weights from memory, experts alone, routed evenly: up to 10 experts all are ahead by then, whatever the depths (8 experts 1.05 to
+// 12 times), but a single one of less than 640 columns (0.93).  With more, an expert's few pairs do not pay for blocks that fill the chip twice:
+// 16 experts, F 512, width 1024, top 4, 32 pairs 20.7 -> 22.9, 36 26.5 -> 22.9; width 768 32 / 36 pairs 18.7 -> 21.6, 21.6 -> 21.9; F 448, width 640, 44 / 48
+// 20.9 -> 22.0, 21.6 -> 22.3; F 384, width 1536, 32 / 40 / 48 26.7 -> 29.6, 29.0 -> 29.8, 34.7 -> 30.1; width 2048, 32 33.0 -> 31.7; up to F 256 always
+// ahead.  Taken here: 1160 of the 1260, none slower by more than 1 %.  (Where all tokens choose the same experts the other form reads no others'
+// rows: of 500 such steps 33 are slower here, by up to 13 %.)
 bool seq_moe_few(int code, const void* h, int ldh, const void* wgu, const void* wd, const void* shared, int T_, int top, int E, int F, int W) {
   const auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  const long P = (long)T_ * top;
-  return code == 0 && P <= FEW && P * F * W >= 12500000 && P >= 2 * E && E <= 16 && F % 32 == 0 && F <= 512 && W % 128 == 0 && W <= 2048 && ldh % 8 == 0 &&
+  const long P = (long)T_ * top, work = P * F * W;
+  const bool many = E > 10 && F > 256 && W <= 1536;
+  return code == 0 && P <= FEW && work >= 12500000 && P >= 2 * E && E <= 16 && (E > 1 || W >= 640) &&
+         (!many || (W <= 1024 ? P > 32 && work >= 1000000l * E : P >= 3 * E)) && F % 32 == 0 && F <= 512 && W % 128 == 0 && W <= 2048 && ldh % 8 == 0 &&
          aligned(h) && aligned(wgu) && aligned(wd) && aligned(shared);
 }
 

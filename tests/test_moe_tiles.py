@@ -221,3 +221,15 @@ def test_decode_batches_read_an_expert_once(T, top, E, F, W, act, weight_input):
                 want[rows] += x * (1.0 if weight_input else wt)
         # float sums of up to 2048 products; of the activations one in a few thousand is rounded to the other bf16 neighbour, 2^-8 of it
         assert ((got.double() - want).norm() / want.norm()).item() < 2e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,top,E,F,W,few", [
+    (8, 4, 16, 512, 1024, False), (9, 4, 16, 512, 1024, True), (12, 4, 16, 448, 640, False), (8, 4, 16, 384, 1536, False), (12, 4, 16, 384, 1536, True),
+    (8, 4, 16, 384, 2048, True), (12, 4, 16, 256, 1024, True), (6, 4, 12, 384, 1536, False), (6, 4, 9, 384, 1536, True), (8, 2, 8, 384, 2048, True),
+    (7, 2, 8, 384, 2048, False), (512, 1, 1, 64, 512, False), (204, 1, 1, 96, 640, True), (40, 2, 17, 512, 2048, False)])
+def test_an_expert_is_read_once_only_where_it_is_not_slower(T, top, E, F, W, few):
+    """Timed steps on both sides (in us, a wave a pair / an expert once: 20.7 / 22.9, 26.5 / 22.9, 21.6 / 22.3, 26.7 / 29.6, 34.7 / 30.1, 33.0 / 31.7, 21.8 / 15.1,
+    23.8 / 26.4, 23.8 / 18.5, 18.7 / 17.6; 53.9 / 57.7 and 34.5 / 26.9 for a single one), a line nothing was timed at, too many experts."""
+    from llm_in_practise_amd.ops._native import native_seq
+    assert native_seq().moe_few(T, top, E, F, W) == few
