@@ -51,6 +51,7 @@ bool skinny_norms(int, int, bool);
 void launch_rows_swiglu(const void*, int, const void*, void*, int, int, int, hipStream_t);
 void launch_rows_parts(const void*, int, const void*, const void*, void*, float*, int, int, int, int, hipStream_t);
 bool parts_norm_ok(int);
+bool parts_norm_ahead(int, int);
 void launch_parts_norm(const float*, int, const void*, const void*, void*, void*, int, int, float, hipStream_t);
 void launch_gemm_skinny(const void*, int, const void*, const void*, void*, int, int, int, bool, const void*, float, hipStream_t);
 bool w4mm_supported(int, int, int, int);
@@ -789,12 +790,12 @@ Tensor w4g(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, optional<T
 }
 
 // A W4A16 product whose sums of K's slices go through memory, their sum with the residual and its RMSNorm: (y, norm(y)); none where one launch
-// holds all of K, or w4g takes it in one slice.  few: as w4mm runs it, else as w4g does.
+// holds all of K, w4g takes it in one slice, or two launches sum and norm so many faster.  few: as w4mm runs it, else as w4g does.
 std::vector<Tensor> w4_parts_norm(Tensor x, Tensor codes, Tensor sc2, int64_t N, int64_t gs, bool few, Tensor residual, Tensor norm, double eps) {
   check_w4mm(x, codes, sc2, N, gs);
   const int64_t M = x.size(0), K = x.size(1);
   const int nb = w4mm_nkb((int)M, (int)N, (int)K), s = few ? (int)(K / (128 * nb)) : w4g_splits((int)M, (int)N, (int)K);
-  if (s <= 1 || (few && w4row_serves((int)M, (int)N, (int)K, nb, false))) return {};
+  if (s <= 1 || (few && w4row_serves((int)M, (int)N, (int)K, nb, false)) || !parts_norm_ahead((int)N, s)) return {};
   TORCH_CHECK(few || w4g_supported((int)M, (int)N, (int)K, (int)gs), "w4g: M<=64, N%128, K%128, gs%128");
   check_parts_norm(x, residual, norm, N);
   Tensor y = at::empty({M, N}, x.options()), yn = at::empty({M, N}, x.options()), part = at::empty({s, M, N}, x.options().dtype(at::kFloat));

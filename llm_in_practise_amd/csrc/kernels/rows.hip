@@ -216,6 +216,14 @@ __global__ __launch_bounds__(1024) void parts_norm_k(const float* __restrict__ p
 // Whether parts_norm_k takes rows of N: a thread eight columns, whole waves
 bool parts_norm_ok(int N) { return N % 512 == 0 && N <= 8192; }
 
+// Whether parts_norm_k is ahead of the sum's own launch and the norm's: a row's parts all come through one CU here, where the sum spreads them over the chip.
+// Of W4A16 products of 5 to 64 rows (N 512 to 8192, K 1024 to 25600, 3 to 100 slices; the product included) the two launches -> this one, µs at 8 rows:
+// 1024 × 4096 (16 slices) 9.8 → 8.6, 2560 × 9728 (38) 16.7 → 15.8, 1536 × 12288 (48) 16.6 → 15.8, at 17 rows 4096 × 12288 (24) 24.4 → 24.3; not taken: 4096 × 19456
+// (38) 0.92 times as fast, 5120 × 9728 (19) 20.1 → 20.7, 8192 × 5120 (10) 0.93 times, 8192 × 12288 (24) 27.0 → 31.3, 1024 × 17408 (68, a long chain) 0.97 times.  Past
+// 4096 columns a row has more than eight waves to bring its parts through.  Of 881 such products 583 are taken, none slower by more than 1.5 %; 221 of
+// all were, by up to a third.  (bf16 products have four parts: 1.04 and more at every size.)
+bool parts_norm_ahead(int N, int S) { return S <= 48 && (long)S * N <= (N <= 4096 ? 98304 : 65536); }
+
 // y [M, N] = sum of S parts + res, yn = its RMSNorm with weight w
 void launch_parts_norm(const float* part, int S, const void* res, const void* w, void* y, void* yn, int M, int N, float eps, hipStream_t st) {
   const int ch = N % 1024 ? 0 : N / 1024;                  // (the norm's kernel gives these widths two waves a row, others one)

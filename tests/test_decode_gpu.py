@@ -481,6 +481,22 @@ def test_parts_and_the_norm_behind_them(native_ext, M, N, K):
     assert not native_ext.parts_norm_serves(N + 16) and not native_ext.parts_norm_serves(8704)
 
 
+@pytest.mark.parametrize("M,N,K,served", [(8, 1536, 12288, True), (8, 1024, 17408, False), (17, 4096, 12288, True), (17, 4096, 13824, False),
+                                          (8, 5120, 9728, False), (17, 5120, 5120, True), (17, 8192, 5120, False), (40, 8192, 5120, True)])
+def test_slices_are_summed_beside_the_norm_only_where_it_is_not_slower(native_ext, M, N, K, served):
+    """Sizes on both sides of what one CU brings of a row's slices in the time of two launches, and of the longest chain."""
+    from llm_in_practise_amd.ops.norm import rms_norm
+    from llm_in_practise_amd.quant.int4 import int4_linear, int4_normed, quantize_rtn
+    torch.manual_seed(N + M)
+    x, res, nw = torch.randn(M, K, device=DEV).bfloat16(), torch.randn(M, N, device=DEV).bfloat16(), torch.randn(N, device=DEV).bfloat16()
+    w4 = quantize_rtn((torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16(), 128)
+    got = int4_normed(x, w4, res, nw, 1e-6)
+    assert (got is not None) == served
+    if served:
+        want = int4_linear(x, w4, None, res)
+        assert torch.equal(got[0], want) and torch.equal(got[1], rms_norm(want, nw, 1e-6))
+
+
 @pytest.mark.parametrize("rows", [5, 17, 33, 64])
 @pytest.mark.parametrize("weights", ["bf16", "int4"])
 def test_decode_steps_norm_rows_where_parts_are_added_up(native_ext, monkeypatch, rows, weights):
