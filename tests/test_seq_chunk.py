@@ -216,6 +216,108 @@ def test_mlstm_token_that_is_no_number(name, value, t):
     _planted(run, inputs, name, t, 1, value, lens)
 
 
+def _in_chunks(op, lens, H, dk, dv):
+    """The step runs in chunks: not walked with the state at hand, not token by token."""
+    from llm_in_practise_amd.ops._native import native_seq
+    shape = (sum(lens), len(lens), H, dk, dv)
+    return native_seq().scan_walk(*shape, max(lens), op) == 0 < native_seq().scan_floats(op, *shape, longest=max(lens))
+
+
+# keys that have no walk, long sequences; one, two and four chunks a run
+CHUNK_LENS = [([120, 264], 2, 1, 96, 40), ([64, 1500], 4, 2, 128, 40), ([3000, 1100], 16, 2, 128, 64), ([1100, 6000], 16, 4, 64, 128)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,value", [("v", float("inf")), ("k", float("-inf")), ("k", float("nan")), ("q", float("nan")), ("q", float("inf")),
+                                        ("dt", float("nan")), ("dt", float("inf"))])
+@pytest.mark.parametrize("lens,H,G,dk,dv", CHUNK_LENS)
+@pytest.mark.parametrize("at", [0, 131, 255])
+def test_ssd_chunks_with_a_token_that_is_no_number(name, value, lens, H, G, dk, dv, at):
+    assert _in_chunks("ssd", lens, H, dk, dv)
+    g = torch.Generator().manual_seed(at)
+    T = sum(lens)
+    inputs = {n: torch.randn(T, w, generator=g).bfloat16().cuda() for n, w in (("q", G * dk), ("k", G * dk), ("v", H * dv), ("dt", H))}
+    dtb, a_log, skip = (torch.randn(H, generator=g).cuda() for _ in range(3))
+
+    def run(x):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, [0, 5], "cuda")
+        st["S"].fill_(0.5)
+        return (R.ssd_scan(x["q"], x["k"], x["v"], x["dt"], dtb, a_log, skip, st["S"], H, G, sb).view(T, H, dv),)
+    _planted(run, inputs, name, lens[0] + at, 1, value, lens)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,value", [("v", float("-inf")), ("k", float("inf")), ("k", float("nan")), ("q", float("nan")), ("i", float("nan")),
+                                        ("f", float("nan"))])
+@pytest.mark.parametrize("lens,H,G,dk,dv", CHUNK_LENS)
+@pytest.mark.parametrize("at", [1, 128, 250])
+def test_mlstm_chunks_with_a_token_that_is_no_number(name, value, lens, H, G, dk, dv, at):
+    assert _in_chunks("mlstm", lens, H, dk, dv)
+    g = torch.Generator().manual_seed(at)
+    T = sum(lens)
+    inputs = {n: torch.randn(T, H * w, generator=g).bfloat16().cuda() for n, w in (("q", dk), ("k", dk), ("v", dv))}
+    inputs |= {n: 2 * torch.randn(T, H, generator=g).cuda() for n in "if"}
+    ib, fb = torch.randn(H, generator=g).cuda(), (torch.randn(H, generator=g) + 3).cuda()
+
+    def run(x):
+        st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lens, [9, 0], "cuda")
+        for s in st.values():
+            s.fill_(0.25)
+        return R.mlstm_scan(x["q"], x["k"], x["v"], x["i"], x["f"], ib, fb, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb)
+    _planted(run, inputs, name, lens[0] + at, 1, value, lens)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,starts", [([40, 1500], [0, 0]), ([1411, 1, 128], [3, 0, 9])])
+@pytest.mark.parametrize("H,G,dk,dv", [(4, 2, 128, 64), (6, 1, 128, 36), (4, 2, 64, 64)])
+def test_ssd_chunks_of_long_sequences(lens, starts, H, G, dk, dv):
+    """Keys of 64 and 128 that several heads share, sequences long enough to be left to the chunks, against the token-by-token reference."""
+    assert _in_chunks("ssd", lens, H, dk, dv)
+    g = torch.Generator().manual_seed(dk + dv + len(lens))
+    T = sum(lens)
+    xbc = torch.randn(T, H * dv + 2 * G * dk, generator=g).bfloat16()
+    dt, dtb = torch.randn(T, H, generator=g).bfloat16(), torch.randn(H, generator=g) - 2
+    a_log, skip = torch.randn(H, generator=g), torch.randn(H, generator=g)
+    S0 = 0.3 * torch.randn(len(lens), H, dv, dk, generator=g)
+    res = []
+    for dev in ("cpu", "cuda"):
+        st, sb = _batch({"S": ((H, dv, dk), "f32")}, lens, starts, dev)
+        st["S"].copy_(S0)
+        x, p = xbc.to(dev), [t.to(dev) for t in (dt, dtb, a_log, skip)]
+        y = R.ssd_scan(x[:, H * dv + G * dk:], x[:, H * dv:H * dv + G * dk], x[:, :H * dv], *p, st["S"], H, G, sb)
+        res.append((y.view(T, H, dv), st["S"]))
+    _close(res[1], res[0], ("y", "state"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["ssd", "mlstm"])
+@pytest.mark.parametrize("H,dk,dv", [(2, 128, 32), (3, 96, 20)])
+def test_idle_sequences_keep_their_state_in_chunks(op, H, dk, dv):
+    lens = [130, 2000, 70]
+    assert _in_chunks(op, lens, H, dk, dv)
+    g = torch.Generator().manual_seed(0)
+    T = sum(lens)
+    q, k, v = (torch.randn(T, H * n, generator=g).bfloat16().cuda() for n in (dk, dk, dv))
+    i, f = (torch.randn(T, H, generator=g).cuda() for _ in "if")
+    a, b, skip = (torch.randn(H, generator=g).cuda() for _ in range(3))
+    out = []
+    for live in (None, [1, 0, 1]):
+        st, sb = _batch({"S": ((H, dv, dk), "f32"), "N": ((H, dk), "f32"), "M": ((H,), "f32")}, lens, [0, 3, 8], "cuda", live)
+        for x in st.values():
+            x.fill_(7.0)
+        if op == "ssd":
+            y = [R.ssd_scan(q, k, v, i.bfloat16(), a - 3, b, skip, st["S"], H, H, sb)]
+        else:
+            y = R.mlstm_scan(q, k, v, i, f, a, b + 3, 15.0, dk ** -0.5, st["S"], st["N"], st["M"], H, sb)
+        out.append(([x for x in y], [st["S"]] if op == "ssd" else list(st.values())))
+    for x in out[1][1]:
+        assert (x[1] == 7.0).all()                      # slot 1 belongs to sequence 1
+    for x, y in zip(out[0][1], out[1][1]):
+        assert torch.equal(x[[0, 2]], y[[0, 2]])
+    for x, y in zip(out[0][0], out[1][0]):
+        assert torch.equal(x[:130], y[:130]) and torch.equal(x[2130:], y[2130:])
+
+
 BLOCK_LENS = [([32], [0]), ([31], [3]), ([48, 15, 1, 128, 65, 33], [0, 0, 9, 5, 0, 0]), ([100, 47], [512, 0])]
 
 
