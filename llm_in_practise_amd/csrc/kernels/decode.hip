@@ -669,8 +669,10 @@ int decode_split_plan2(int B, int hkv, int max_len) {
 // four splits of one tile or two of two tiles, adds each of them up by itself in the order it has alone (the bits stay), and the empty ones are numbered last.
 // µs, both launches, heads of 128, 32 query on 8, from memory, a workgroup a split with the empty ones between the others -> here: 12 rows of 474 to 1400 keys 20.5 -> 17.5; 20 of
 // 33 to 100 12.1 -> 10.8, of 644 to 1900 29.4 -> 29.6; 32 of 314 to 1000 27.8 -> 25.4; 48 of 125 to 400 24.2 -> 21.2; 64 of 688 to 1700 68.8 -> 69.2, of 80 to 200 22.8 ->
-// 18.8.  Below, CUs are idle and a workgroup's own work counts: 4 rows of 562 to 1400 11.7 -> 12.3 (not taken).  Fewer and longer splits (12 rows 15.7) add in another
-// order, which an 8B model's logits show by 0.03, as much as their own rounding error.
+// 18.8.  At the line, 8 rows of 8 heads: 22 to 40 keys 12.8 -> 8.2, 40 to 100 12.9 -> 9.5, 160 to 400 13.6 -> 10.7, 402 to 1000 14.8 -> 13.3, 610 to 1400 15.7 -> 14.7, 804 to 2000 17.0 ->
+// 16.5; 64 rows of one head 14.6 -> 9.6, 17.1 -> 15.7 (305 to 1000), 18.1 -> 16.7 (611 to 2000).  What it costs to find a split shows where all rows fill the cache: all of 2000 keys 19.3 ->
+// 19.8 and 20.0 -> 20.7, 12 rows of 8 heads 24.9 -> 26.0.  Below, CUs are idle and a workgroup's own work counts: 4 rows of 562 to 1400 11.7 -> 12.3 (not taken).  Fewer and longer splits
+// (12 rows 15.7) add in another order, which an 8B model's logits show by 0.03, as much as their own rounding error.
 void launch_decode_attention2(const void* q, int ldq, const void* knew, int ldkn, const void* vnew, int ldvn, void* kc,
                               void* vc, const int64_t* pos, float* opart, float* mpart, float* lpart, void* out, int B,
                               int Smax, int hq, int hkv, int d, int nsplit, float scale, hipStream_t st) {

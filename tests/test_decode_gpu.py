@@ -168,6 +168,27 @@ def test_decode_attention_append_counts_the_splits_that_have_keys(native_ext, B,
     assert torch.equal(again[keep], o[keep])
 
 
+@pytest.mark.parametrize("B,hkv,d", [(8, 8, 128), (11, 8, 128), (16, 4, 64), (22, 3, 128), (66, 1, 64)])
+@pytest.mark.parametrize("max_len", [128, 500, 700, 1000])
+def test_decode_attention_append_bits_of_counted_splits(native_ext, B, hkv, d, max_len):
+    """From 64 rows x heads on a workgroup takes several short splits: the bits are those of a workgroup a split, which fewer rows with as many
+    splits (one of every 128 keys on either side) have."""
+    torch.manual_seed(B + max_len)
+    hq = 4 * hkv
+    ends = [0, 5, 31, 32, 33, 62, 63, 64, 95, 126, 127, 128, 191, 255, 256, 257, 383, 499, 511, 512, 699, 767, 999]
+    ends = [e for e in ends if e < max_len]
+    P = torch.tensor([ends[(i * 7) % len(ends)] for i in range(B - 1)] + [max_len - 1], device=DEV)
+    kc, vc = (torch.randn(B, max_len, hkv * d, device=DEV).to(torch.bfloat16) for _ in range(2))
+    q, k, v = (torch.randn(B, n * d, device=DEV).to(torch.bfloat16) for n in (hq, hkv, hkv))
+    K2, V2 = kc.clone(), vc.clone()
+    got = native_ext.decode_attention_append(q, k, v, kc, vc, P, hq, hkv, d, max_len, d ** -0.5)
+    n = 63 // hkv                                           # rows of a call below 64 rows x heads
+    assert B * hkv >= 64 > n * hkv
+    want = torch.cat([native_ext.decode_attention_append(*(t[i:i + n] for t in (q, k, v)), K2[i:i + n], V2[i:i + n], P[i:i + n], hq, hkv, d, max_len,
+                                                         d ** -0.5) for i in range(0, B, n)])
+    assert torch.equal(got, want) and torch.equal(kc, K2) and torch.equal(vc, V2)
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 33, 64])
 @pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 12288), (272, 192)])
 def test_gemm_skinny_matches_fp32(native_ext, M, N, K):
