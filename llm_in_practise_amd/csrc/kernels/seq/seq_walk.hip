@@ -618,8 +618,8 @@ PiecePlan walk_plan(int T_, int B, int H, size_t most) { return plan_pieces(T_, 
 // The first alone walks one or a few long prompts among short ones where that takes up to twice as long (mLSTM, 8 heads of 64 x 160, six of 2517 tokens
 // and 14 short ones 110 in chunks, 160 here).  The second is fitted to the chunks and every width of a block on 3600 calls, 1 to 64 heads, 1 to
 // 64 sequences, all of one length, ragged, or one or a few long ones among short ones in any place: chunks within 10 %, blocks of one round within
-// 6.  It does not know which place that is, nor how many heads share keys, so it only has to be within 5 % of agreeing.  Of 6370 calls the first one
-// walks 3770, 156 of them slower so; both together 3470, 26 of them slower, by 2 to 20 %.
+// 6.  It does not know which place that is, nor how many heads share keys, so it only has to be within 5 % of agreeing (state space, where heads do, 10).  Of 6370
+// calls the first one walks 3770, 156 of them slower so; both together 3490, 29 of them slower, by 2 to 25 %.
 // Prompts that no chunks are there for (seq_walk_short) ask the first one alone.
 // Chunks -> here, us: mLSTM, 8 heads of 128 x 192: 80 tokens 21 -> 11, 512 28 -> 21, 2 x 512 31 -> 22, 8 x 1024 89 -> 52, 48 x 128 99 -> 67, but one
 // prompt of 2048 44 -> 58; of 64 x 96: 8 x 512 32 -> 21, 12 x 700 47 -> 32, one of 2048 32 -> 43; state space, 64 heads of 128 x 64: 512 34 -> 19, 4 x 512 63 ->
@@ -655,7 +655,7 @@ int walk_tiles(bool mlstm, int T_, int B, int H, int dk, int dv, int longest, fl
     if (chunked) {
       const float turn2 = cost.turn[t - 1] * (0.87f + 0.13f * std::min(1.f, blocks / 256.f));
       const float late = ((mlstm ? 9.7f : 8.6f) + turn2 * (most2 + 0.25f) + (float)(rounds - 1) * (3.f + turn2 * (mean2 + 0.25f))) / chunks2;
-      if (late >= 1.05f) continue;
+      if (late >= (mlstm ? 1.05f : 1.1f)) continue;
       score += late;
     }
     if (score < best) {
