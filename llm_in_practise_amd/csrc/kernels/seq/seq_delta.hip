@@ -12,7 +12,8 @@
 //
 // Measured, blocks of 16 -> of 32 tokens: three sequences of 1500, 700 and 97 tokens, 8 heads of 128 x 128: 112 -> 90 us (26 for the first
 // kernel - 32 with two blocks a CU and rows that left four bytes a lane - and 64 for the walk, which is bound by the longest sequence's
-// chain: 1.3 us a block of 32, 0.7 of them products of a wave on the float matrix unit; 0.94 us a block of 16; in two parts 25 and 40, 84 us in all).  Error against 64 bits of
+// chain: 1.3 us a block of 32, 0.7 of them products of a wave on the float matrix unit; 0.94 us a block of 16; with the 1500 tokens in four parts and the 700 in two,
+// 25 for the ends and 40 for the parts, 84 us in all).  Error against 64 bits of
 // outputs, blocks of 16 -> 32: 3.2 -> 2.6e-7 where decays are next to 1, 1.6 -> 1.55 at 0.95, 1.25 -> 1.28 at 0.8, 1.08 -> 1.10 at 0.4:
 // the state and a tile's sums are added up by themselves and rounded once at the size of what they are added to.
 #include "seq_block.h"

@@ -811,7 +811,7 @@ void seq_route_fused(int code, const void* h, int ldh, const float* router, cons
 // outputs on its way from the start, half a us less.
 // Where the line lies.  12.5 million: nothing between 10.5 (slower here) and 12.58 was timed.  1260 more steps, 1 to 16 experts, top 1 to 8, F 32 to 512,
 // widths of 128 to 2048, weights from memory, experts alone, routed evenly: up to 10 experts all are ahead by then, whatever the depths (8 experts 1.05 to
-// 12 times), but a single one of less than 640 columns (0.93).  With more, an expert's few pairs do not pay for blocks that fill the chip twice:
+// 9 times), but a single one of less than 640 columns (0.93).  With more, an expert's few pairs do not pay for blocks that fill the chip twice:
 // 16 experts, F 512, width 1024, top 4, 32 pairs 20.7 -> 22.9, 36 26.5 -> 22.9; width 768 32 / 36 pairs 18.7 -> 21.6, 21.6 -> 21.9; F 448, width 640, 44 / 48
 // 20.9 -> 22.0, 21.6 -> 22.3; F 384, width 1536, 32 / 40 / 48 26.7 -> 29.6, 29.0 -> 29.8, 34.7 -> 30.1; width 2048, 32 33.0 -> 31.7; up to F 256 always
 // ahead.  Taken here: 1160 of the 1260, none slower by more than 1 %.  (Where all tokens choose the same experts the other form reads no others'
